@@ -266,3 +266,19 @@ def test_experts(dtype, T, E, top, ff, width):
     y = ops.experts(x.to(DEV), ids.to(DEV), ops.pack_matrix(up).contiguous().to(DEV), ops.pack_matrix(down).contiguous().to(DEV), width).view(T, top, width)
     want = torch.stack([torch.stack([ref.expert(x[t].double()[:width], up[e].double()[:ff, :width], down[e].double()[:width, :ff]) for e in ids[t].tolist()]) for t in range(T)])
     close(y, want, 2e-6 if dtype == torch.float32 else 1.2e-2)
+
+
+def test_experts_with_row_counts_at_the_edges_of_tiles():
+    """Prompt-sized products (row tiles of 256, blocks of 32 of which only those with rows are multiplied): experts with no row, one
+    row, one short of a block or a tile, exactly one, one more, and both kinds of tiles at once."""
+    counts = [0, 1, 31, 32, 33, 255, 256, 257, 512, 545]
+    E, top, ff, width, T = len(counts), 1, 64, 64, sum(counts)
+    assert T >= 96 * E
+    x = rnd(T, width, seed=1, dtype=torch.bfloat16)
+    up, down = (rnd(E, ff, width, seed=2) * width ** -0.5).to(torch.bfloat16), (rnd(E, width, ff, seed=3) * ff ** -0.5).to(torch.bfloat16)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=torch.Generator().manual_seed(4))]
+    y = ops.experts(x.to(DEV), ids[:, None].int().to(DEV), ops.pack_matrix(up).contiguous().to(DEV), ops.pack_matrix(down).contiguous().to(DEV), width)
+    want = torch.empty(T, width, dtype=torch.float64)
+    for e in range(E):
+        want[ids == e] = ref.expert(x[ids == e].double(), up[e].double(), down[e].double())
+    close(y, want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each: 2^-8 of the largest each, and slack for their spread

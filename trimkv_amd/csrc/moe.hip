@@ -76,34 +76,40 @@ __global__ __launch_bounds__(256) void route_kernel(const float* z, const float*
 
 // One workgroup orders all rows (a step's few thousand, or a prompt's tens of thousands): counts, offsets and scatter in LDS.
 __global__ __launch_bounds__(1024) void plan_kernel(const int32_t* ids, int rows, int E, int tile, int32_t* order, int32_t* offsets, int32_t* tiles) {
-    extern __shared__ int32_t pl[];               // cursor [E], tile cursor [E]
-    int32_t* cursor = pl; int32_t* tcur = pl + E;
+    extern __shared__ int32_t pl[];               // cursor [E], tile cursor [E], cursor of the last tile if it is not full [E]
+    int32_t* cursor = pl; int32_t* tcur = pl + E; int32_t* tlast = tcur + E;
+    const bool apart = tile >= 256;               // tiles of the matrix-bound kernel: those that are not full come last, so that the launch ends on short ones
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += 1024) cursor[e] = 0;
     __syncthreads();
     for (int i = tid; i < rows; i += 1024) atomicAdd(&cursor[ids[i]], 1);
     __syncthreads();
     if (tid < 64) {                               // exclusive sums over experts, 64 at a time
-        int base = 0, tbase = 0;
+        int base = 0, tbase = 0, lbase = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + tid, c = e < E ? cursor[e] : 0, nt = (c + tile - 1) / tile;
-            int s = c, ts = nt;
+            const int e = e0 + tid, c = e < E ? cursor[e] : 0, nt = apart ? c / tile : (c + tile - 1) / tile, nl = apart && c % tile ? 1 : 0;
+            int s = c, ts = nt, ls = nl;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(s, d, 64), to = __shfl_up(ts, d, 64);
-                if (tid >= d) { s += o; ts += to; }
+                const int o = __shfl_up(s, d, 64), to = __shfl_up(ts, d, 64), lo = __shfl_up(ls, d, 64);
+                if (tid >= d) { s += o; ts += to; ls += lo; }
             }
-            if (e < E) { offsets[e] = base + s - c; cursor[e] = base + s - c; tcur[e] = tbase + ts - nt; }
+            if (e < E) { offsets[e] = base + s - c; cursor[e] = base + s - c; tcur[e] = tbase + ts - nt; tlast[e] = lbase + ls - nl; }
             base += __shfl(s, 63, 64);
             tbase += __shfl(ts, 63, 64);
+            lbase += __shfl(ls, 63, 64);
         }
-        if (tid == 0) { offsets[E] = base; tiles[0] = tbase; }
+        if (tid == 0) { offsets[E] = base; tiles[0] = tbase + lbase; pl[3 * E] = tbase; }
     }
     __syncthreads();
     // tiles[1 + 2 i] = expert, tiles[2 + 2 i] = first row of tile i
     for (int e = tid; e < E; e += 1024) {
         const int first = cursor[e], c = (e + 1 < E ? cursor[e + 1] : rows) - first;
-        for (int x = 0; x * tile < c; ++x) { tiles[1 + 2 * (tcur[e] + x)] = e; tiles[2 + 2 * (tcur[e] + x)] = first + x * tile; }
+        for (int x = 0; x * tile < c; ++x) {
+            const int i = apart && (x + 1) * tile > c ? pl[3 * E] + tlast[e] : tcur[e] + x;
+            tiles[1 + 2 * i] = e;
+            tiles[2 + 2 * i] = first + x * tile;
+        }
     }
     __syncthreads();
     for (int i = tid; i < rows; i += 1024) order[atomicAdd(&cursor[ids[i]], 1)] = i;
@@ -211,28 +217,34 @@ __global__ __launch_bounds__(KS * 64) void grouped_skinny_kernel(GroupedArgs a) 
 }
 
 // bf16, many rows per expert (prompts): WM YT x 32 rows by WN XT x 32 outputs per workgroup of WM WN wavefronts, each XT x YT
-// tiles of 32x32x16 MFMAs.  Steps of 32 k rotate through four LDS buffers filled by LDS-direct loads, three steps ahead: the
+// tiles of 32x32x16 MFMAs.  Steps of 32 k rotate through five LDS buffers filled by LDS-direct loads, four steps ahead: the
 // weights lane-linear as they lie in memory, token rows gathered, the 16-byte piece c of row r at c ^ ((r / 4) % 4), so that
 // the rows of a fragment read fall on different banks.
+// What bounds it is the way of the operands into LDS, not the matrix cores (busy 66 % of a compute unit's time): with the loads
+// taken out the two products of 8192 tokens x 4 of 32 experts (4096 x 4608) take 1.93 ms, with loads that always hit 2.28 ms, as
+// it is 2.64 ms.  Reads and requests one by one between the products, four steps ahead, rows that are not there not multiplied
+// and equal shares for the XCDs: 2.76 -> 2.64 ms.  Two buffers of 64 k were slower (2.88 ms), four wavefronts of 128 x 128 outputs
+// the same.
 template <bool UP, int XT, int YT, int WN, int WM>
 __global__ __launch_bounds__(WN * WM * 64) void grouped_big_kernel(GroupedArgs a, int n_tiles) {
     constexpr int THREADS = WN * WM * 64, TM = WM * YT * 32, TN = WN * XT * 32, RL = THREADS / 4, XB = TM * 64, BUF = (TM + TN) * 64;
-    constexpr int XL = TM / RL, WL = TN / 16 / (WN * WM);
+    constexpr int XL = TM / RL, WL = TN / 16 / (WN * WM), AHEAD = 4;
     static_assert(TM % RL == 0 && TN / 16 % (WN * WM) == 0, "whole loads");
     extern __shared__ __attribute__((aligned(16))) char gb_lds[];
     HY_LDS char* const lds3 = (HY_LDS char*)gb_lds;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds3;
-    // an XCD takes a contiguous share of the row tiles and walks it in blocks of 4 row tiles x all outputs: the rows and the
-    // weights that neighbouring workgroups read stay in its L2
-    const int total = a.tiles[0], share = (total + 7) / 8, turn = blockIdx.x >> 3;
-    const int blk = turn / (4 * n_tiles), in = turn - blk * 4 * n_tiles;
-    const int first = blk * 4, rows_here = min(4, share - first);
-    if (rows_here <= 0) return;
-    const int nt = in / rows_here, rt = (blockIdx.x & 7) * share + first + in % rows_here;
-    if (nt >= n_tiles || rt >= total) return;
+    // The tiles in blocks of 4 row tiles x all outputs, row tiles fastest, cut into eight equal runs, one for each XCD: the rows
+    // and the weights that neighbouring workgroups read stay in its L2.
+    const int total = a.tiles[0], share = (total * n_tiles + 7) / 8, turn = blockIdx.x >> 3, at = (blockIdx.x & 7) * share + turn;
+    if (turn >= share || at >= total * n_tiles) return;
+    const int blk = at / (4 * n_tiles), in = at - blk * 4 * n_tiles, high = min(4, total - 4 * blk);
+    const int nt = in / high, rt = 4 * blk + in % high;
     const int e = a.tiles[1 + 2 * rt], m0 = a.tiles[2 + 2 * rt], mend = a.offsets[e + 1], n0 = nt * TN;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 31, hl = lane >> 5;
-    const int wm = w % WM, wn = w / WM, kb16 = a.kp >> 4;
+    // Wavefronts of one wn share a SIMD and take turns on the tile's blocks of 32 rows, of which only those with rows are
+    // multiplied: the last tile of an expert costs what it holds.
+    const int wn = w % WN, wm = w / WN, kb16 = a.kp >> 4;
+    const int blocks = __builtin_amdgcn_readfirstlane((min(mend - m0, TM) + 31) / 32), mine = (blocks - wm + WM - 1) / WM;
     const uint16_t* xp[XL]; const char* wp[WL];
     const int lrow = tid >> 2, piece = ((tid & 3) ^ ((lrow >> 2) & 3)) * 8;       // RL is a multiple of 16: one swizzle for all loads
 #pragma unroll
@@ -247,13 +259,12 @@ __global__ __launch_bounds__(WN * WM * 64) void grouped_big_kernel(GroupedArgs a
     }
     const uint32_t woff = lane * 16;
     const int steps = a.kp / 32;
-    auto request = [&](int s, int buf) __attribute__((always_inline)) {
+    // load i of step s, of the wavefront's XL + WL of them
+    auto request = [&](int s, int buf, int i) __attribute__((always_inline)) {
         const int sc = min(s, steps - 1);                                         // past the end: re-read, never used
         const uint32_t dst = lds0 + buf * BUF;
-#pragma unroll
-        for (int x = 0; x < XL; ++x) load_to_lds16(xp[x] + sc * 32, dst + x * RL * 64 + w * 1024);
-#pragma unroll
-        for (int x = 0; x < WL; ++x) load_to_lds16_at(wp[x] + (int64_t)sc * 2048, woff, dst + XB + (w * WL + x) * 1024);
+        if (i < XL) load_to_lds16(xp[i] + sc * 32, dst + i * RL * 64 + w * 1024);
+        else load_to_lds16_at(wp[i - XL] + (int64_t)sc * 2048, woff, dst + XB + (w * WL + i - XL) * 1024);
     };
     hy_f32x16 acc[XT][YT];
 #pragma unroll
@@ -263,37 +274,60 @@ __global__ __launch_bounds__(WN * WM * 64) void grouped_big_kernel(GroupedArgs a
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.0f;
     const int sw = (j >> 2) & 3;
-    HY_LDS char* const xr = lds3 + (wm * YT * 32 + j) * 64;
+    HY_LDS char* const xr = lds3 + (wm * 32 + j) * 64;            // of block wm + WM y: + y WM 2048
     HY_LDS char* const wr = lds3 + XB + wn * XT * 2048 + lane * 16;
-    request(0, 0);
-    request(1, 1);
-    request(2, 2);
-    for (int s = 0; s < steps; ++s) {
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * (XL + WL)) : "memory");     // step s is here; two more are on their way
-        __syncthreads();
-        request(s + 3, (s + 3) & 3);
-        const int off = (s & 3) * BUF;
-        hy_bf16x8 xf[2][YT], wf[2][XT];
+    constexpr int N = XL + WL;
+    // The first half of a step is in registers when the step begins; its products run behind the reads of the second half and
+    // the requests of step s + AHEAD, the second half's products behind the reads of the next step's first half.  The wavefronts
+    // meet where step s + 1 has landed everywhere and nobody reads step s - 1, whose buffer is requested anew, any more.
+    auto walk = [&](auto count) __attribute__((always_inline)) {
+        constexpr int YC = decltype(count)::value;    // blocks of rows of this wavefront
+        hy_bf16x8 xf[2][YC + 1], wf[2][XT];
+        auto fetch = [&](int ks, int buf, int i) __attribute__((always_inline)) { // operand i of half a step (16 of its 32 k)
+            const int off = buf * BUF;
+            if (i < YC) xf[ks][i] = *(const HY_LDS hy_bf16x8*)(xr + off + i * WM * 2048 + (((2 * ks + hl) ^ sw) << 4));
+            else if (YC && i < YC + XT) wf[ks][i - YC] = *(const HY_LDS hy_bf16x8*)(wr + off + (i - YC) * 2048 + ks * 1024);
+        };
+        auto multiply = [&](int ks, int i) __attribute__((always_inline)) {
+            if (i < XT * YC) acc[i / max(YC, 1)][i % max(YC, 1)] = mfma32(wf[ks][i / max(YC, 1)], xf[ks][i % max(YC, 1)], acc[i / max(YC, 1)][i % max(YC, 1)]);
+        };
+        constexpr int SLOTS = XT * YC > XT + YC ? XT * YC : XT + YC;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int po = off + (((2 * ks + hl) ^ sw) << 4);
+        for (int i = 0; i < XT + YC; ++i) fetch(0, 0, i);
+        int buf = 0, next = 1, last = AHEAD;          // of step s, s + 1 and s + AHEAD
+        for (int s = 0; s < steps; ++s) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((AHEAD - 2) * N) : "memory");
 #pragma unroll
-            for (int y = 0; y < YT; ++y) xf[ks][y] = *(const HY_LDS hy_bf16x8*)(xr + y * 2048 + po);
+            for (int i = 0; i < 2 * SLOTS; ++i) {
+                multiply(i / SLOTS, i % SLOTS);
+                if (i < SLOTS) fetch(1, buf, i); else fetch(0, next, i - SLOTS);
+                // the requests are spread over the step: in one burst they queue up in front of the L1 and the products wait
 #pragma unroll
-            for (int x = 0; x < XT; ++x) wf[ks][x] = *(const HY_LDS hy_bf16x8*)(wr + off + x * 2048 + ks * 1024);
+                for (int x = i * N / (2 * SLOTS); x < (i + 1) * N / (2 * SLOTS); ++x) request(s + AHEAD, last, x);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            buf = next;
+            next = next == AHEAD ? 0 : next + 1;
+            last = last == AHEAD ? 0 : last + 1;
         }
+    };
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+    for (int p = 0; p < AHEAD; ++p)
 #pragma unroll
-            for (int x = 0; x < XT; ++x)
-#pragma unroll
-                for (int y = 0; y < YT; ++y) acc[x][y] = mfma32(wf[ks][x], xf[ks][y], acc[x][y]);
-    }
+        for (int i = 0; i < N; ++i) request(p, p, i);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"((AHEAD - 1) * N) : "memory");
+    __syncthreads();
+    static_assert(YT == 4, "one walk for every number of blocks");
+    if (mine == 4) walk(std::integral_constant<int, 4>{});
+    else if (mine == 3) walk(std::integral_constant<int, 3>{});
+    else if (mine == 2) walk(std::integral_constant<int, 2>{});
+    else if (mine == 1) walk(std::integral_constant<int, 1>{});
+    else walk(std::integral_constant<int, 0>{});
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup has gone
-    // acc[x][y]: outputs n0 + (wn XT + x) 32 + 8 (v / 4) + 4 hl + v % 4 of row m0 + (wm YT + y) 32 + j
+    // acc[x][y]: outputs n0 + (wn XT + x) 32 + 8 (v / 4) + 4 hl + v % 4 of row m0 + (wm + WM y) 32 + j
 #pragma unroll
     for (int y = 0; y < YT; ++y) {
-        const int i = m0 + (wm * YT + y) * 32 + j;
+        const int i = m0 + (wm + WM * y) * 32 + j;
         if (i >= mend) continue;
         uint16_t* yr = (uint16_t*)a.y + (UP ? (int64_t)i : (int64_t)a.order[i]) * a.ys;
 #pragma unroll
@@ -306,7 +340,7 @@ __global__ __launch_bounds__(WN * WM * 64) void grouped_big_kernel(GroupedArgs a
 
 template <bool UP, int XT, int YT, int WN, int WM>
 static int launch_big(const GroupedArgs& a, int most, hipStream_t s) {
-    constexpr int LDS = 4 * (WM * YT + WN * XT) * 32 * 64;
+    constexpr int LDS = 5 * (WM * YT + WN * XT) * 32 * 64;
     static bool opted_in[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
@@ -315,7 +349,7 @@ static int launch_big(const GroupedArgs& a, int most, hipStream_t s) {
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) opted_in[dev] = true;
     }
-    const int n_tiles = (a.np + WN * XT * 32 - 1) / (WN * XT * 32), blocks = 8 * (((most + 7) / 8 + 3) / 4) * 4 * n_tiles;
+    const int n_tiles = (a.np + WN * XT * 32 - 1) / (WN * XT * 32), blocks = 8 * ((most * n_tiles + 7) / 8);
     hipLaunchKernelGGL((grouped_big_kernel<UP, XT, YT, WN, WM>), dim3(blocks), dim3(WN * WM * 64), LDS, s, a, n_tiles);
     return 0;
 }
@@ -348,7 +382,7 @@ extern "C" int trimkv_moe_plan(const int32_t* ids, int rows, int experts, int ti
     const char* fn = "trimkv_moe_plan";
     if (!ids || !order || !offsets || !tiles) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (rows <= 0 || experts <= 0 || experts > ROUTE_MAX_E || tile <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: bad sizes rows=%d experts=%d tile=%d", fn, rows, experts, tile);
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 2 * experts * sizeof(int32_t), (hipStream_t)stream, ids, rows, experts, tile, order, offsets, tiles);
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), (3 * experts + 1) * sizeof(int32_t), (hipStream_t)stream, ids, rows, experts, tile, order, offsets, tiles);
     return launch_status(fn);
 }
 
