@@ -282,3 +282,37 @@ def test_experts_with_row_counts_at_the_edges_of_tiles():
     for e in range(E):
         want[ids == e] = ref.expert(x[ids == e].double(), up[e].double(), down[e].double())
     close(y, want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each: 2^-8 of the largest each, and slack for their spread
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [3, 37, 64, 129])
+def test_values_that_are_not_finite_stay_out_of_rows_that_do_not_see_them(bad, at):
+    """fp32 prompts take tiles of keys (and chunks of tokens) at a time: a value that is masked for a row is multiplied by zero
+    there and must not turn the row into NaN.  Rows in front of the token are as if it were harmless; in the window's case
+    those behind it, too."""
+    n, s, m = 150, ops.WindowSpec(4, 2, 24, 40, 20, 3, 0.3), ops.MlstmSpec(2, 40, 72, 9.0)
+    outs = []
+    for value in (1.0, bad):
+        sizes = [s.heads * s.dim, s.kv_heads * s.dim, s.kv_heads * s.vdim, s.heads * s.vdim]
+        offs = [0, sizes[0], sum(sizes[:2]), sum(sizes[:3])]
+        proj = rnd(n, sum(sizes), seed=1)
+        proj[at, offs[2]] = value
+        cache = HybridCache([s], torch.float32, DEV, num_slots=1)
+        batch = cache.batch([n], cache.allocate(1))
+        ones = [torch.ones(k, device=DEV) for k in sizes[:2]]
+        a = ops.window_attention(proj.to(DEV), offs, *ones, 1e-5, s, cache.layers_state[0], batch)
+        sizes = [m.heads * m.dim] * 2 + [m.heads * m.vdim] * 2
+        offs = [0, sizes[0], sum(sizes[:2]), sum(sizes[:3])]
+        proj = rnd(n, sum(sizes), seed=2)
+        proj[at, offs[2]] = value
+        cache = HybridCache([m], torch.float32, DEV, num_slots=1)
+        batch = cache.batch([n], cache.allocate(1))
+        gates, z = rnd(n, 2 * m.heads, seed=3).to(DEV), torch.zeros(m.heads, device=DEV)
+        r = ops.mlstm(proj.to(DEV), offs, gates, z, z + 3, torch.ones(m.heads * m.vdim, device=DEV), 1e-5, m, cache.layers_state[0], batch)
+        outs.append((a.cpu(), r.cpu()))
+    (a, r), (ab, rb) = outs
+    sees = torch.tensor([t >= at and (t - at < s.window or at < s.keep_first) for t in range(n)])
+    assert (ab[~sees] - a[~sees]).abs().max() <= 1e-6        # the same sums in the same or another order of 64 keys at most
+    assert not ab[sees][:, 0].isfinite().any()
+    assert (rb[:at] - r[:at]).abs().max() <= 1e-5
+    assert not rb[at:, 0].isfinite().any()

@@ -64,6 +64,13 @@ typedef uint32_t hy_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t hy_u32x4 __attribute__((ext_vector_type(4)));
 #define HY_LDS __attribute__((address_space(3)))
 
+// neither infinite nor NaN, by the bits (a file may be compiled without NaNs)
+__device__ __forceinline__ bool finite_bits(uint32_t x) { return (x & 0x7f800000u) != 0x7f800000u; }
+__device__ __forceinline__ bool finite_bits(hy_u32x4 x) { return finite_bits(x[0]) && finite_bits(x[1]) && finite_bits(x[2]) && finite_bits(x[3]); }
+
+// v or zeros, without a branch
+__device__ __forceinline__ hy_u32x4 kept4(hy_u32x4 v, bool keep) { return hy_u32x4{keep ? v[0] : 0u, keep ? v[1] : 0u, keep ? v[2] : 0u, keep ? v[3] : 0u}; }
+
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     const hy_f32x2 f = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, hy_bf16x2));
@@ -84,6 +91,7 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t (&out)[TERMS])
 }
 
 __device__ __forceinline__ hy_f32x4 mfma16(hy_bf16x8 a, hy_bf16x8 b, hy_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ hy_f32x4 mfma16_f32(float a, float b, hy_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ hy_f32x16 mfma32(hy_bf16x8 a, hy_bf16x8 b, hy_f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 
 // One LDS-direct load of 16 bytes per lane: lane l's bytes land at lds_addr + 16 l (lds_addr wavefront-uniform).  The compiler

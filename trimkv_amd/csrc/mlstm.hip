@@ -8,8 +8,9 @@
 // a head while S is split over workgroups by value columns, so a step reads (n, m) from the copy of the parity of the
 // slot's step count and writes the other one.  A slot whose token count is 0 starts from the zero state whatever it holds.
 //
-//   mlstm_recurrent_kernel  token by token; decode, and any portion in fp32
+//   mlstm_recurrent_kernel  token by token: decode, and what the other two do not take
 //   mlstm_chunk_kernel      prompts in bf16 on the matrix cores, 64 tokens at a time
+//   mlstm_chunk_f32_kernel  the same in fp32
 #include "hybrid.hip.h"
 #include <type_traits>
 
@@ -484,6 +485,262 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
     if (e == 0) out[a.D] = m * LN2;
 }
 
+// ---- fp32 portions: TC tokens at a time on the matrix cores' fp32 products ---------------------------
+// The equations of the bf16 kernel with everything in fp32; the running sums of gates, their maxima and m are kept in double
+// inside a chunk, so that an exponent, a difference of two long sums, is as exact as the sequential recurrence's.  A workgroup
+// owns 64 value columns of one head, a wavefront 16, whose part of S stays in the accumulators of 16x16x4 MFMAs: with g = lane / 16,
+// A and B hold k = g of row / column lane % 16, register r of C row 4 g + r.  Sums over features and over tokens run in the order
+// 16 x + 4 g + r, in which the accumulators of S are an operand as they are and an A operand is four consecutive floats in LDS.
+// LDS rows are a multiple of 16 plus 4 floats apart, so that reads along rows and down columns fall on different banks.
+//
+// Bound by the serial chain of chunks (16 us each at 128 features, 6 us of which are products).  300 + 511 tokens of 8 heads of
+// 128 x 256: 129 us; token by token 1314 us (2.6 us a token).
+// A value that is not finite must not reach earlier tokens of its chunk through 0 x inf: such chunks take the products of the
+// diagonal blocks one token at a time.
+template <int DT, int TC>
+struct F32Cfg {
+    static constexpr int LD = DT + 4, LV = 68, LW = TC + 4;
+    static constexpr int Q0 = 0, K0 = Q0 + TC * LD, V0 = K0 + TC * LD, W0 = V0 + TC * LV, N0 = W0 + TC * LW;      // in floats
+    static constexpr int G0 = (N0 + DT + 3 * TC + 8 + 1) / 2 * 2, LDS = (G0 + 2 * (2 * TC + 4)) * 4;                // G0: doubles from there on
+};
+__device__ __forceinline__ double shfl_up_d(double v, int d) {
+    const long long x = __double_as_longlong(v);
+    const int lo = __shfl_up((int)(x & 0xffffffffll), d, 64), hi = __shfl_up((int)(x >> 32), d, 64);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+template <int DT, int TC>
+__global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
+    using C = F32Cfg<DT, TC>;
+    constexpr int DB = DT / 16, TB = TC / 16, LD = C::LD, LV = C::LV, LW = C::LW, QL = TC * DT / 1024, VL = TC * 64 / 1024;
+    extern __shared__ __attribute__((aligned(16))) float cf_lds[];
+    float* const q = cf_lds + C::Q0; float* const k = cf_lds + C::K0; float* const v = cf_lds + C::V0; float* const wt = cf_lds + C::W0;
+    float* const n = cf_lds + C::N0; float* const carry = n + DT; float* const end = carry + TC; float* const den = end + TC;   // exp(m_0 - M_t), exp(d_s - M_C), 1 / denominator
+    int* const odd = (int*)(den + TC);                // chunk + 1 whose values were not all finite
+    double* const gD = (double*)(cf_lds + C::G0); double* const gM = gD + TC; double* const gm = gM + TC;           // d_s, M_t; m_0 and F_C
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    const int h = blockIdx.y, b = blockIdx.z, col0 = blockIdx.x * 64, col = col0 + w * 16 + c;
+    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, slot = a.slots[b];
+    const bool fresh = a.seen[2 * slot] == 0;
+    const int parity = a.seen[2 * slot + 1] & 1;
+    const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
+    const float* nm_in = a.nm + parity * copy + at;
+    float* Sp = a.S + ((int64_t)slot * a.H + h) * a.D * a.Dv;
+    hy_u32x4 qn[QL], kn[QL], vn[VL];
+    float zi, zf;                                     // raw gates, lane = token
+    auto fetch = [&](int ch) __attribute__((always_inline)) {
+        const float* gp = a.gates + (int64_t)(t0 + min(ch * TC + lane, len - 1)) * 2 * a.H + h;
+        zi = gp[0];
+        zf = gp[a.H];
+#pragma unroll
+        for (int x = 0; x < QL; ++x) {
+            const int p = x * 256 + tid, r = p / (DT / 4), e = (p % (DT / 4)) * 4;
+            const float* row = (const float*)a.p + (int64_t)(t0 + min(ch * TC + r, len - 1)) * a.p_stride + h * a.D;
+            // loads are unconditional (a load under a branch is waited for on the spot); what is not there becomes zero
+            qn[x] = *(const hy_u32x4*)(row + a.q_off + min(e, a.D - 4));
+            kn[x] = *(const hy_u32x4*)(row + a.k_off + min(e, a.D - 4));
+        }
+#pragma unroll
+        for (int x = 0; x < VL; ++x) {
+            const int p = x * 256 + tid, r = p >> 4, e = (p & 15) * 4;
+            vn[x] = *(const hy_u32x4*)((const float*)a.p + (int64_t)(t0 + min(ch * TC + r, len - 1)) * a.p_stride + a.v_off + h * a.Dv + min(col0 + e, a.Dv - 4));
+        }
+    };
+    fetch(0);
+    hy_f32x4 S[DB];
+#pragma unroll
+    for (int x = 0; x < DB; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int d = 16 * x + 4 * g + r;
+            const float old = Sp[(int64_t)min(d, a.D - 1) * a.Dv + min(col, a.Dv - 1)];
+            S[x][r] = fresh || d >= a.D || col >= a.Dv ? 0.0f : old;
+        }
+    for (int d = tid; d < DT; d += 256) n[d] = fresh || d >= a.D ? 0.0f : nm_in[d];
+    if (tid == 0) { *odd = 0; gm[0] = fresh ? 0.0 : (double)nm_in[a.D]; }
+    const float ib = a.ib[h], fb = a.fb[h];
+    const int nchunks = (len + TC - 1) / TC;
+    for (int ch = 0; ch < nchunks; ++ch) {
+        const int base = ch * TC, rows = min(TC, len - base);
+        __syncthreads();                              // the last chunk is done with
+        bool fine = true;
+#pragma unroll
+        for (int x = 0; x < QL; ++x) {
+            const int p = x * 256 + tid, r = p / (DT / 4), e = (p % (DT / 4)) * 4;
+            const float4 qq = __builtin_bit_cast(float4, kept4(qn[x], e < a.D));
+            *(float4*)(q + r * LD + e) = make_float4(qq.x * a.qscale, qq.y * a.qscale, qq.z * a.qscale, qq.w * a.qscale);
+            *(hy_u32x4*)(k + r * LD + e) = kept4(kn[x], e < a.D && r < rows);
+        }
+#pragma unroll
+        for (int x = 0; x < VL; ++x) {
+            const int p = x * 256 + tid, r = p >> 4, e = (p & 15) * 4;
+            const hy_u32x4 vv = kept4(vn[x], col0 + e < a.Dv && r < rows);
+            *(hy_u32x4*)(v + r * LV + e) = vv;
+            fine = fine && finite_bits(vv);
+        }
+        if (!fine) *odd = ch + 1;
+        if (w == 0) {                                 // lane = token; lanes past TC (TC = 32) repeat the end
+            const bool in = lane < rows;
+            const double li = in ? (double)log_input_gate(zi + ib, a.cap) : -1.0e300;
+            double F = in ? (double)log_forget_gate(zf + fb, a.cap) : 0.0;
+            const double m0 = gm[0];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) { const double o = shfl_up_d(F, d); if (lane >= d) F += o; }
+            const double ds = li - F;
+            double M = fmax(ds, m0);
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) { const double o = shfl_up_d(M, d); if (lane >= d) M = fmax(M, o); }
+            if (lane < TC) {
+                gD[lane] = ds;
+                gM[lane] = M;
+                carry[lane] = expf((float)(m0 - M));
+                den[lane] = expf((float)(-(F + M)));  // exp(-m_t)
+            }
+            if (lane == TC - 1) gm[1] = F;
+        }
+        __syncthreads();
+        if (ch + 1 < nchunks) fetch(ch + 1);
+        const double MC = gM[TC - 1];
+        // weighted scores of the blocks s <= t, transposed: column t, rows s
+        for (int x = w; x < TB * (TB + 1) / 2; x += 4) {
+            int tb = 0, sb = x;
+            while (sb > tb) { ++tb; sb -= tb; }
+            hy_f32x4 p = {0.f, 0.f, 0.f, 0.f};
+            const float* kr = k + (sb * 16 + c) * LD + 4 * g; const float* qr = q + (tb * 16 + c) * LD + 4 * g;
+#pragma unroll
+            for (int y = 0; y < DB; ++y) {
+                const float4 kf = *(const float4*)(kr + 16 * y), qf = *(const float4*)(qr + 16 * y);
+                p = mfma16_f32(kf.x, qf.x, p);
+                p = mfma16_f32(kf.y, qf.y, p);
+                p = mfma16_f32(kf.z, qf.z, p);
+                p = mfma16_f32(kf.w, qf.w, p);
+            }
+            const int t = tb * 16 + c, s = sb * 16 + 4 * g;
+            const double M = gM[t];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[r] = s + r <= t ? p[r] * expf((float)(gD[s + r] - M)) : 0.0f;
+            *(hy_f32x4*)(wt + t * LW + s) = p;
+        }
+        if (tid >= 256 - TC) end[tid - (256 - TC)] = expf((float)(gD[tid - (256 - TC)] - MC));
+        __syncthreads();
+        {                                             // n.q of every token: 256 / TC threads share one
+            constexpr int SH = 256 / TC;
+            const int t = tid / SH, x = tid % SH;
+            float old = 0.0f, own = 0.0f;
+            for (int d = 4 * x; d < DT; d += 4 * SH) {
+                const float4 qq = *(const float4*)(q + t * LD + d), nn = *(const float4*)(n + d);
+                old += qq.x * nn.x + qq.y * nn.y + qq.z * nn.z + qq.w * nn.w;
+            }
+            for (int s = x; s <= t; s += SH) own += wt[t * LW + s];
+#pragma unroll
+            for (int d = 1; d < SH; d <<= 1) { old += __shfl_xor(old, d, 64); own += __shfl_xor(own, d, 64); }
+            if (x == 0) den[t] = 1.0f / (fmaxf(fabsf(own + carry[t] * old), den[t]) + 1e-6f);
+        }
+        hy_f32x4 o[TB];
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {             // S_0^T q
+            o[tb] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
+            const float* qr = q + (tb * 16 + c) * LD + 4 * g;
+#pragma unroll
+            for (int x = 0; x < DB; ++x) {
+                const float4 f = *(const float4*)(qr + 16 * x);
+                o[tb] = mfma16_f32(f.x, S[x][0], o[tb]);
+                o[tb] = mfma16_f32(f.y, S[x][1], o[tb]);
+                o[tb] = mfma16_f32(f.z, S[x][2], o[tb]);
+                o[tb] = mfma16_f32(f.w, S[x][3], o[tb]);
+            }
+            const float4 f = *(const float4*)(carry + tb * 16 + 4 * g);
+            o[tb][0] *= f.x; o[tb][1] *= f.y; o[tb][2] *= f.z; o[tb][3] *= f.w;
+        }
+        const float keep = expf((float)(gm[0] - MC));
+#pragma unroll
+        for (int x = 0; x < DB; ++x) S[x] *= keep;
+        const bool plain = *odd != ch + 1;
+#pragma unroll
+        for (int sb = 0; sb < TB; ++sb) {
+            const float4 e = *(const float4*)(end + sb * 16 + 4 * g);
+            const float ee[4] = {e.x, e.y, e.z, e.w};
+            float vv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) vv[r] = v[(sb * 16 + 4 * g + r) * LV + w * 16 + c];
+#pragma unroll
+            for (int tb = sb; tb < TB; ++tb) {
+                if (tb > sb || plain) {
+                    const float4 f = *(const float4*)(wt + (tb * 16 + c) * LW + sb * 16 + 4 * g);
+                    o[tb] = mfma16_f32(f.x, vv[0], o[tb]);
+                    o[tb] = mfma16_f32(f.y, vv[1], o[tb]);
+                    o[tb] = mfma16_f32(f.z, vv[2], o[tb]);
+                    o[tb] = mfma16_f32(f.w, vv[3], o[tb]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll 1
+                        for (int s = 0; s <= 4 * g + r; ++s) o[tb][r] += wt[(tb * 16 + 4 * g + r) * LW + sb * 16 + s] * v[(sb * 16 + s) * LV + w * 16 + c];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float f = vv[r] * ee[r];
+                const float* kr = k + (sb * 16 + 4 * g + r) * LD + c;
+#pragma unroll
+                for (int x = 0; x < DB; ++x) S[x] = mfma16_f32(kr[16 * x], f, S[x]);
+            }
+        }
+        __syncthreads();                              // denominators are there, n.q has been taken
+        for (int d = tid; d < DT; d += 256) {
+            float x = n[d] * keep;
+            for (int s = 0; s < rows; ++s) x += end[s] * k[s * LD + d];
+            n[d] = x;
+        }
+        if (col < a.Dv) {
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = tb * 16 + 4 * g + r;
+                    if (t < rows) ((float*)a.o)[((int64_t)(t0 + base + t) * a.H + h) * a.Dv + col] = o[tb][r] * den[t];
+                }
+        }
+        if (tid == 0) gm[0] = gm[1] + MC;             // read again behind the next barrier
+    }
+    __syncthreads();
+    if (col < a.Dv) {
+#pragma unroll
+        for (int x = 0; x < DB; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int d = 16 * x + 4 * g + r;
+                if (d < a.D) Sp[(int64_t)d * a.Dv + col] = S[x][r];
+            }
+    }
+    if (blockIdx.x == 0) {
+        float* nm_out = a.nm + (1 - parity) * copy + at;
+        for (int d = tid; d < a.D; d += 256) nm_out[d] = n[d];
+        if (tid == 0) nm_out[a.D] = (float)gm[0];
+    }
+}
+
+template <int DT, int TC>
+static int launch_chunk_f32(const MlstmArgs& a, int batch, hipStream_t s) {
+    constexpr int LDS = F32Cfg<DT, TC>::LDS;
+    static bool opted_in[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+    if (dev < 0 || !opted_in[dev]) {
+        hipError_t e = hipFuncSetAttribute((const void*)mlstm_chunk_f32_kernel<DT, TC>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        if (e != hipSuccess) return (int)e;
+        if (dev >= 0) opted_in[dev] = true;
+    }
+    hipLaunchKernelGGL((mlstm_chunk_f32_kernel<DT, TC>), dim3((a.Dv + 63) / 64, a.H, batch), dim3(256), LDS, s, a);
+    return 0;
+}
+// Portions of a few tokens stay with the token-by-token kernel: a chunk costs 16 us however few tokens it holds, a token 2.6 us.
+constexpr int F32_CHUNK_FROM = 8;
+static bool chunk_f32_fits(const MlstmArgs& a, int dtype, int max_len) {
+    return dtype == TRIMKV_F32 && max_len >= F32_CHUNK_FROM && a.D <= 256 && a.D % 4 == 0 && a.Dv % 4 == 0 && a.p_stride % 4 == 0 && (a.q_off | a.k_off | a.v_off) % 4 == 0 &&
+           !((uintptr_t)a.p & 15);
+}
+
 template <int DKT, int MODE, bool FULL>
 static int launch_chunk(const ChunkArgs& c, dim3 grid, hipStream_t s) {
     static bool opted_in[64] = {};
@@ -557,6 +814,11 @@ extern "C" int trimkv_mlstm(const void* proj, int64_t proj_stride, int q_off, in
         else if (dim == 64) rc = launch_chunked<2, true>(c, batch, s);
         else rc = dim <= 32 ? launch_chunked<1, false>(c, batch, s) : dim < 64 ? launch_chunked<2, false>(c, batch, s) : dim < 128 ? launch_chunked<4, false>(c, batch, s)
                                                                                                                      : launch_chunked<8, false>(c, batch, s);
+        if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
+        return launch_status(fn);
+    }
+    if (chunk_f32_fits(a, dtype, max_len)) {
+        const int rc = dim <= 64 ? launch_chunk_f32<64, 64>(a, batch, s) : dim <= 128 ? launch_chunk_f32<128, 64>(a, batch, s) : launch_chunk_f32<256, 32>(a, batch, s);
         if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
         return launch_status(fn);
     }

@@ -2,7 +2,8 @@
 //
 //   window_prefill_kernel  on the matrix cores (bf16): keys are the ring (what earlier portions left) and then the portion's own
 //                          rows; tiles that no query of the workgroup sees are skipped
-//   window_rows_kernel     the same for fp32 and for head sizes beyond the tiles: one wavefront per query
+//   window_prefill_f32_kernel  the same in fp32
+//   window_rows_kernel     head sizes beyond the tiles: one wavefront per query
 //
 // In the prefill kernel the probabilities enter the second product as two bf16 terms each (17 bits).
 #include "window.hip.h"
@@ -63,6 +64,180 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowArgs a) {
         const int d = c * 64 + lane;
         if (d < a.Dv) st(o + d, acc[c] * inv * window_gate<T>(a, t0 + t, h, d));
     }
+}
+
+// ---- fp32 prompts on the matrix cores --------------------------------------------------------------
+// A workgroup owns 64 rows (consecutive query times x the query heads of one KV head), 16 per wavefront, and walks tiles of 64
+// keys.  Both products run on 16x16x4 fp32 MFMAs, transposed: S^T = K . Q^T, O^T += V^T . P^T, so a row is a column of the
+// accumulators (lane % 16) and the probabilities a lane holds behind the first product are its operand of the second.  With
+// g = lane / 16, A and B hold k = g of row / column lane % 16 and register r of C row 4 g + r; the sums take features in the order
+// 16 x + 4 g + r and keys likewise, so that a lane reads four consecutive floats of K.  LDS rows are DT + 4 floats apart: reads of
+// either product fall on different banks.  The next tile waits in registers.
+//
+// Bound by the matrix cores' fp32 rate (a sixteenth of bf16) and, for short prompts, by the few workgroups there are.  300 + 511
+// tokens, 16 heads of 128 (8 KV heads): 70 us; a wavefront per query row, which this replaces for head sizes up to 128, took
+// 1060 us there, bound by its row-wise loads.
+// NaNs and infinities of keys that a row does not see must not reach it through 0 x inf: tiles with such values in V take their
+// second product one key at a time.
+template <int DT>
+__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
+    constexpr int LD = DT + 4, DB = DT / 16, PIECES = DT / 4, LOADS = 64 * PIECES / 256;
+    extern __shared__ __attribute__((aligned(16))) char wf_lds[];
+    float* const kt = (float*)wf_lds; float* const vt = kt + 64 * LD;
+    int* const where = (int*)(vt + 64 * LD);          // position of every key of the tile; past the end: beyond all queries
+    int* const odd = where + 64;                      // number of tiles + 1 whose V held something that is not finite
+    const int b = blockIdx.y / a.G, g = blockIdx.y % a.G, slot = a.slots[b];
+    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, per = a.H / a.G, bt = 64 / per;
+    // later times first: they walk the most tiles
+    const int first = ((int)gridDim.x - 1 - (int)blockIdx.x) * bt;
+    if (first >= len) return;                         // workgroup-uniform, before any barrier
+    const int past = a.seen[2 * slot], cap = a.keep + a.size, nring = min(past, cap), last = min(first + bt, len) - 1;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, gr = lane >> 4;
+    const int row = w * 16 + c, t = min(first + row / per, last), h = g * per + row % per, i = past + t;
+    const bool live = row < bt * per && first + row / per < len;
+    const float* rk = (const float*)a.rk + ((int64_t)slot * a.G + g) * cap * a.Dp;
+    const float* rv = (const float*)a.rv + ((int64_t)slot * a.G + g) * cap * a.Dvp;
+    const float* pk = (const float*)a.k + ((int64_t)t0 * a.G + g) * a.Dp;
+    const float* pv = (const float*)a.v + ((int64_t)t0 * a.G + g) * a.Dvp;
+    float4 q[DB];
+    {
+        const float* qr = (const float*)a.q + ((int64_t)(t0 + t) * a.H + h) * a.Dp;
+#pragma unroll
+        for (int x = 0; x < DB; ++x) q[x] = *(const float4*)(qr + min(16 * x + 4 * gr, a.Dp - 4));
+#pragma unroll
+        for (int x = 0; x < DB; ++x) q[x] = __builtin_bit_cast(float4, kept4(__builtin_bit_cast(hy_u32x4, q[x]), 16 * x + 4 * gr < a.Dp));
+    }
+    // keys in the order ring, portion; a portion's tile that no row sees is skipped
+    const int nkeys = nring + last + 1, ntiles = (nkeys + 63) / 64;
+    auto next_tile = [&](int x) {
+        for (; x < ntiles; ++x) {
+            const int lo = past + x * 64 - nring, hi = lo + 63;      // positions, if the tile is all portion
+            if (x * 64 < nring || hi > past + first - a.size || lo < a.keep) break;
+        }
+        return x;
+    };
+    hy_u32x4 kn[LOADS], vn[LOADS];
+    int where_n = 0;
+    auto fetch = [&](int x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int y = 0; y < LOADS; ++y) {
+            const int p = y * 256 + tid, r = p / PIECES, e = (p % PIECES) * 4, key = x * 64 + r;
+            // loads are unconditional (a load under a branch is waited for on the spot); what is not there becomes zero
+            const int kc = min(key, nkeys - 1), ek = min(e, a.Dp - 4), ev = min(e, a.Dvp - 4);
+            const bool ring = kc < nring;
+            const int64_t at = ring ? kc : (int64_t)(kc - nring) * a.G;
+            kn[y] = *(const hy_u32x4*)((ring ? rk : pk) + at * a.Dp + ek);
+            vn[y] = *(const hy_u32x4*)((ring ? rv : pv) + at * a.Dvp + ev);
+        }
+        const int key = x * 64 + (tid & 63);
+        where_n = key >= nkeys ? 0x7fffffff : key < nring ? ring_position(key, past, a.keep, a.size) : past + key - nring;
+    };
+    hy_f32x4 o[DB];
+#pragma unroll
+    for (int x = 0; x < DB; ++x) o[x] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = WA_NEG, l = 0.0f;
+    if (tid == 0) *odd = 0;
+    int tile = next_tile(0);
+    if (tile < ntiles) fetch(tile);
+    while (tile < ntiles) {
+        __syncthreads();                              // the last tile is done with
+        bool fine = true;
+#pragma unroll
+        for (int y = 0; y < LOADS; ++y) {
+            const int p = y * 256 + tid, r = p / PIECES, e = (p % PIECES) * 4;
+            const bool in = tile * 64 + r < nkeys;
+            const hy_u32x4 vv = kept4(vn[y], in && e < a.Dvp);
+            *(hy_u32x4*)(kt + r * LD + e) = kept4(kn[y], in && e < a.Dp);
+            *(hy_u32x4*)(vt + r * LD + e) = vv;
+            fine = fine && finite_bits(vv);
+        }
+        if (tid < 64) where[tid] = where_n;
+        if (!fine) *odd = tile + 1;
+        __syncthreads();
+        const int now = tile;
+        tile = next_tile(tile + 1);
+        if (tile < ntiles) fetch(tile);
+        hy_f32x4 s[4];
+        float top = WA_NEG;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            s[kb] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
+            const float* kr = kt + (kb * 16 + c) * LD + 4 * gr;
+#pragma unroll
+            for (int x = 0; x < DB; ++x) {
+                const float4 f = *(const float4*)(kr + 16 * x);
+                s[kb] = mfma16_f32(f.x, q[x].x, s[kb]);
+                s[kb] = mfma16_f32(f.y, q[x].y, s[kb]);
+                s[kb] = mfma16_f32(f.z, q[x].z, s[kb]);
+                s[kb] = mfma16_f32(f.w, q[x].w, s[kb]);
+            }
+            const int4 at = *(const int4*)(where + kb * 16 + 4 * gr);
+            const int pos[4] = {at.x, at.y, at.z, at.w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                s[kb][r] = pos[r] <= i && (i - pos[r] < a.size || pos[r] < a.keep) ? s[kb][r] * a.scale_log2 : -INFINITY;
+                top = fmaxf(top, s[kb][r]);
+            }
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float mn = fmaxf(m, top), alpha = exp2f(m - mn);
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { s[kb][r] = exp2f(s[kb][r] - mn); l += s[kb][r]; }
+#pragma unroll
+        for (int x = 0; x < DB; ++x) o[x] *= alpha;
+        if (*odd != now + 1) {
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float* vr = vt + (kb * 16 + 4 * gr + r) * LD + c;
+#pragma unroll
+                    for (int x = 0; x < DB; ++x) o[x] = mfma16_f32(vr[16 * x], s[kb][r], o[x]);
+                }
+        } else {                                      // workgroup-uniform: the keys' place takes the probabilities
+            __syncthreads();
+            float* const ps = kt + w * 1024;          // [key][row]
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ps[(kb * 16 + 4 * gr + r) * 16 + c] = s[kb][r];
+            __syncthreads();
+#pragma unroll 1
+            for (int key = 0; key < 64; ++key) {
+                const float p = ps[key * 16 + c];
+#pragma unroll
+                for (int x = 0; x < DB; ++x) {
+                    const float4 f = *(const float4*)(vt + key * LD + 16 * x + 4 * gr);
+                    o[x][0] += p == 0.0f ? 0.0f : p * f.x;
+                    o[x][1] += p == 0.0f ? 0.0f : p * f.y;
+                    o[x][2] += p == 0.0f ? 0.0f : p * f.z;
+                    o[x][3] += p == 0.0f ? 0.0f : p * f.w;
+                }
+            }
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (!live) return;
+    const float inv = 1.0f / (l + window_sink(a, m));
+    float* out = (float*)a.out + ((int64_t)(t0 + t) * a.H + h) * a.Dv;
+    float gate[DB][4];
+#pragma unroll
+    for (int x = 0; x < DB; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gate[x][r] = window_gate<float>(a, t0 + t, h, min(16 * x + 4 * gr + r, a.Dv - 1));
+#pragma unroll
+    for (int x = 0; x < DB; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int d = 16 * x + 4 * gr + r;
+            if (d < a.Dv) out[d] = o[x][r] * inv * gate[x][r];
+        }
 }
 
 // ---- prompts on the matrix cores -------------------------------------------------------------------
@@ -338,6 +513,22 @@ static int launch_window_prefill(const WindowArgs& a, int batch, int max_len, hi
     return 0;
 }
 
+template <int DT>
+static int launch_window_prefill_f32(const WindowArgs& a, int batch, int max_len, hipStream_t s) {
+    constexpr int LDS = (2 * 64 * (DT + 4) + 64 + 4) * 4;
+    static bool opted_in[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+    if (dev < 0 || !opted_in[dev]) {
+        hipError_t e = hipFuncSetAttribute((const void*)window_prefill_f32_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        if (e != hipSuccess) return (int)e;
+        if (dev >= 0) opted_in[dev] = true;
+    }
+    const int bt = 64 / (a.H / a.G);
+    hipLaunchKernelGGL((window_prefill_f32_kernel<DT>), dim3((max_len + bt - 1) / bt, batch * a.G), dim3(256), LDS, s, a);
+    return 0;
+}
+
 }  // namespace trimkv
 
 using namespace trimkv;
@@ -361,6 +552,11 @@ extern "C" int trimkv_window_prefill(const void* q, const void* k, const void* v
         a.vec = vdim % 4 == 0 && !((uintptr_t)out & 7) && (head_gate || (gate_stride % 4 == 0 && !((uintptr_t)gate & 7)));
         const int rc = big <= 64 ? launch_window_prefill<64>(a, batch, max_len, s) : big <= 96 ? launch_window_prefill<128, 96>(a, batch, max_len, s) : big <= 128 ? launch_window_prefill<128>(a, batch, max_len, s)
                                                                                                : launch_window_prefill<256>(a, batch, max_len, s);
+        if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
+        return launch_status(fn);
+    }
+    if (dtype == TRIMKV_F32 && big <= 128 && per <= 64 && aligned) {
+        const int rc = big <= 64 ? launch_window_prefill_f32<64>(a, batch, max_len, s) : launch_window_prefill_f32<128>(a, batch, max_len, s);
         if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
         return launch_status(fn);
     }
