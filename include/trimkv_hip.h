@@ -295,6 +295,19 @@ int trimkv_evict_listed(const trimkv_layer_slabs* layers, int nlayers, int nseg,
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * trimkv_evict_split -- trimkv_evict_layers (work = NULL) or trimkv_evict_listed with the rows of a segment moved by several
+ * workgroups, in three launches: for few, long segments, of which one workgroup each leaves most of the chip idle.  spill: the
+ * most rows that any segment loses (512 or more: any number); a segment that loses more is moved by one workgroup all the same.
+ * head_dim 64, 96 or 128, max_len <= 32768.  workspace: trimkv_evict_split_workspace(number of pairs, ...) bytes, 16-byte aligned;
+ * pairs = nwork, or nlayers * nseg.  The query index is an argument or per layer in the table.  Same results.
+ */
+size_t trimkv_evict_split_workspace(int npairs, int max_len, int head_dim, int spill);
+int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                       int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                       int strategy, int rounding, int sliding_window, int max_len, int spill,
+                       const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * trimkv_compact_threshold_layers -- trimkv_compact_threshold for nlayers layers in one launch
  * (the per-layer rebuild loops at cache_utils.py:466-482, 912-943).  thr_key / tie_take are
  * [ngroups] shared by all layers (thr_layer_stride = 0: one budget across layers) or

@@ -1,0 +1,89 @@
+"""Evictions whose rows are moved by several workgroups per segment (trimkv_evict_split) against a plain gather: patterns whose
+shifts are the smallest and the largest, rows on both sides of a chunk's end, chunks that lose everything, work lists, segments
+that lose more rows than the workspace was sized for, and every row size and log-beta type."""
+import numpy as np
+import pytest
+import torch
+
+from trimkv_amd import BatchedDynamicBudgetTrimKVCache, TrimKVCache, _lib
+import trimkv_amd.cache_utils as cache_utils
+from tests.gpu_util import DEV
+from tests.test_gpu_evict_patterns import _patterns
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def always_split(monkeypatch):
+    calls = []
+    monkeypatch.setattr(cache_utils, "split_evict", lambda *a: calls.append(a) or True)
+    return calls
+
+
+def _filled(cls, layers, B, H, n, D, kv_dtype, lb_dtype, keep):
+    """A cache whose segments keep exactly the rows ``keep`` when cut to keep.size rows; returns it and its contents."""
+    gen = torch.Generator().manual_seed(n + D)
+    cache, held = cls(), []
+    for l in range(layers):
+        k, v = (torch.randn(B, H, n, D, generator=gen).to(kv_dtype) for _ in range(2))
+        lb = torch.full((B, H, n), -5.0)
+        lb[:, :, torch.from_numpy(keep)] = -1e-7 * (1.0 + torch.rand(B, H, keep.size, generator=gen))
+        lb = lb.to(lb_dtype)
+        cache.update(k.to(DEV), v.to(DEV), lb.to(DEV), torch.arange(n, device=DEV), l)
+        held.append((k, v, lb))
+    return cache, held
+
+
+def _check(cache, held, rows, what):
+    for l, (k, v, lb) in enumerate(held):
+        s = cache._slabs[l]
+        m = rows.size
+        assert (s.seg_len.cpu() == m).all(), what
+        for got, want in ((s.k, k), (s.v, v), (s.lb, lb)):
+            want = want.flatten(0, 1)[:, torch.from_numpy(rows)]
+            assert torch.equal(got[:, :m].cpu(), want), what
+        assert torch.equal(s.pos[:, :m].cpu(), torch.from_numpy(rows).expand(s.nseg, m)), what
+
+
+@pytest.mark.parametrize("D,kv_dtype,lb_dtype", [(128, torch.bfloat16, torch.float32), (96, torch.float16, torch.float32), (64, torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("n,M", [(4224, 4096), (5000, 4999), (3000, 1025), (2600, 1024), (2049, 1537), (9000, 3000), (2100, 1)])
+def test_patterns(n, M, D, kv_dtype, lb_dtype, always_split):
+    for name, keep in _patterns(n, M):
+        keep = np.asarray(keep)
+        if keep.size != M:
+            continue
+        cache, held = _filled(TrimKVCache, 2 if D == 128 else 1, 1, 3, n, D, kv_dtype, lb_dtype, keep)
+        cache.compress("alpha", memory_size=M, buffer_size=n - M)
+        _check(cache, held, keep, name)
+    assert always_split
+
+
+@pytest.mark.parametrize("spill", [4, 130, 512])
+def test_segments_that_lose_more_than_the_workspace_was_sized_for(spill, always_split):
+    n, M = 3300, 3100          # 200 rows lost: more than 4 and 130 (moved whole), less than 512
+    keep = np.sort(np.random.default_rng(1).choice(n, size=M, replace=False))
+    cache, held = _filled(TrimKVCache, 2, 2, 2, n, 128, torch.bfloat16, torch.float32, keep)
+    cache._evict_layers([0, 1], M, None, 0, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST, 0, n + 1, spill=spill)
+    _check(cache, held, keep, f"spill {spill}")
+
+
+def test_work_list_with_budgets_of_its_own_against_one_workgroup_per_segment(monkeypatch):
+    """Budgets from one row to all but one, a few segments due: the listed split against trimkv_evict_listed."""
+    B, H, n, L = 2, 4, 4000, 2
+    budgets = np.array([[n, 3900, n, 1, n, n, 2000, n], [n, n, 1030, n, 3999, n, n, 520]])
+    states = []
+    for split in (False, True):
+        monkeypatch.setattr(cache_utils, "split_evict", lambda *a, split=split: split)
+        gen = torch.Generator().manual_seed(5)
+        cache = BatchedDynamicBudgetTrimKVCache()
+        for l in range(L):
+            k, v = (torch.randn(B, H, n, 128, generator=gen).to(torch.bfloat16).to(DEV) for _ in range(2))
+            cache.update(k, v, (-torch.rand(B, H, n, generator=gen) - 0.01).to(DEV), torch.arange(n, device=DEV), l)
+        cache.set_budgets(budgets)
+        cache.evict_to_budgets(buffer_size=0)
+        states.append([(t.cpu() for t in (cache.key_cache[l], cache.value_cache[l], cache.retention_weights[l], cache.kv_positions[l], cache.head_lens[l], cache.cu_seqlens_k[l]))
+                       for l in range(L)])
+    for a, b in zip(*states):
+        for x, y in zip(a, b):
+            assert torch.equal(x, y)
+    assert [int(t) for t in cache.head_lens[0]] == budgets[0].tolist()

@@ -86,6 +86,18 @@ class LazyLogBeta:
         return out.transpose(1, 2) if self.transposed else out
 
 
+def split_evict(longest: int, rows: int, spill: int, head_dim: int) -> bool:
+    """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split``): ``rows`` due rows
+    in all, the longest segment of ``longest``, none losing more than ``spill``.  One workgroup per segment takes about
+    15 us + 18 ns a row of the longest one; three launches and the detour of the rows that cross a chunk's end take about 30 us
+    + 0.25 ns a row (0.4 ns when most rows cross).  Measured, whole -> split, segments of 128 features that lose 128 rows:
+    8 x 8320 167 -> 60 us, 32 x 8320 196 -> 107, 64 x 4224 117 -> 98, 64 x 2176 63 -> 66, 128 x 8320 253 -> 270; losing 4096:
+    8 x 12288 181 -> 89, 32 x 12288 207 -> 156, 64 x 12288 240 -> 257.  Not while a graph is captured: the launches' table may be
+    uploaded for the first time."""
+    return (2048 <= longest <= 32768 and head_dim in (64, 96, 128) and rows * (5 if spill < 512 else 8) < 360 * longest - 300000
+            and not torch.cuda.is_current_stream_capturing())
+
+
 class _Slab:
     """Device storage of one layer."""
 
@@ -178,7 +190,7 @@ class _SlabBacked(_CacheBase):
     def _workspace(self, nbytes: int, device) -> Optional[torch.Tensor]:
         if nbytes <= 0:
             return None
-        key = ("evict", str(device))
+        key = ("evict", str(device), _lib.current_stream(device))     # a buffer's launches are in the order of its stream
         ws = self._ws.get(key)
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -355,12 +367,14 @@ class _SlabBacked(_CacheBase):
         return torch.from_numpy(arr.view(np.uint8)).to(self._slabs[layers[0]].k.device)
 
     def _evict_layers(self, layers: List[int], keep: int, keep_per_seg, slack: int, strategy_code: int,
-                      rounding: int, sliding_window: int, q_idx, work: Optional[np.ndarray] = None) -> None:
+                      rounding: int, sliding_window: int, q_idx, work: Optional[np.ndarray] = None, spill: int = 512,
+                      due: Optional[Tuple[int, int]] = None) -> None:
         """``trimkv_evict_layers`` over ``layers`` (all of one shape): one launch of nseg x len(layers) workgroups.
         ``q_idx``: the query index, one int or one per layer.  ``keep_per_seg``: None, a host array (uploaded) or a device
         int32 tensor, ``[nseg]`` or ``[len(layers), nseg]``.  ``work``: host int32 array of ``index in layers * nseg +
         segment``: only these pairs get a workgroup (``trimkv_evict_listed``); it reaches the device through pinned memory
-        in stream order."""
+        in stream order.  ``spill``: the most rows a segment loses, where the caller knows (512: any number); ``due``: rows of the longest segment
+        that is due, and of all that are."""
         s0 = self._slabs[layers[0]]
         dev = s0.k.device
         max_len = max(self._slabs[l].max_len for l in layers)
@@ -377,9 +391,18 @@ class _SlabBacked(_CacheBase):
                 kdev = torch.from_numpy(np.ascontiguousarray(keep_per_seg, dtype=np.int32)).to(dev)
             stride = 0 if kdev.dim() == 1 else s0.nseg
         lib = _lib.load()
+        pairs = len(layers) * s0.nseg if work is None else int(work.size)
+        wdev = None if work is None else self._upload_work(work, len(layers) * s0.nseg, dev)
+        if split_evict(*(due or (max_len, pairs * max_len)), spill, s0.D) and max_len <= 32768:
+            ws = self._workspace(lib.trimkv_evict_split_workspace(pairs, max_len, s0.D, spill), dev)
+            rc = lib.trimkv_evict_split(table.data_ptr(), len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype),
+                                        int(keep), _lib.ptr(kdev), stride, int(slack), q_all, strategy_code, rounding, int(sliding_window),
+                                        max_len, spill, _lib.ptr(wdev), 0 if work is None else pairs, ws.data_ptr(), ws.numel(), _lib.current_stream(dev))
+            _lib.check(rc, "trimkv_evict_split")
+            self._keepalive_layers = (table, kdev)
+            return
         ws = self._workspace(len(layers) * lib.trimkv_evict_workspace(s0.nseg, max_len), dev)
         if work is not None:
-            wdev = self._upload_work(work, len(layers) * s0.nseg, dev)
             rc = lib.trimkv_evict_listed(table.data_ptr(), len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype),
                                          int(keep), _lib.ptr(kdev), stride, int(slack), q_all, None, strategy_code, rounding, int(sliding_window),
                                          max_len, wdev.data_ptr(), int(work.size), _lib.ptr(ws), 0 if ws is None else ws.numel(),
@@ -667,9 +690,12 @@ class TrimKVCache(_SlabBacked):
             return self._compress_on_device(strategy, memory_size, buffer_size, skip_layers, num_layers)
         self._budget_hint = memory_size + buffer_size
         todo = [l for l in range(skip_layers, num_layers) if memory_size + buffer_size <= self.get_cache_length(l)]
-        if len(todo) > 1 and self._layers_alike(todo):   # the usual case: every layer is due at the same step -> one launch
+        lost = min(512, max(1, max((self._slabs[l].max_len for l in todo), default=0) - memory_size))
+        first = self._slabs[todo[0]] if todo else None
+        # the usual case: every layer is due at the same step -> one launch
+        if len(todo) > 1 and self._layers_alike(todo) or len(todo) == 1 and split_evict(first.max_len, first.nseg * first.max_len, lost, first.D):
             self._evict_layers(todo, memory_size, None, 0, self._dense_strategy_code(strategy), _lib.ROUND_UPCAST,
-                               self.sliding_window_size, [self.get_seq_length(l) + 1 for l in todo])
+                               self.sliding_window_size, [self.get_seq_length(l) + 1 for l in todo], spill=lost)
             for l in todo:
                 self._slabs[l].lens[:] = memory_size
                 self._slabs[l].max_len = memory_size
@@ -1265,7 +1291,9 @@ class _RaggedCache(_SlabBacked):
             # (layer, segment) costs about 0.1 ms in dispatch alone when nearly all of them have nothing to do.
             ndue = int(hit_all.sum())
             work = np.flatnonzero(hit_all).astype(np.int32) if ndue * 4 < hit_all.size else None
-            self._evict_layers(every, 0, keep, buffer_size, code, _lib.ROUND_NATIVE, 0, q_idx, work=work)
+            due_lens = lens_all[hit_all]
+            self._evict_layers(every, 0, keep, buffer_size, code, _lib.ROUND_NATIVE, 0, q_idx, work=work,
+                               spill=min(512, int((lens_all - kh_all)[hit_all].max())), due=(int(due_lens.max()), int(due_lens.sum())))
             t = self._device_tables(every)
             rc = lib.trimkv_build_cu_seqlens_layers(t["len"].data_ptr(), t["cu"].data_ptr(), len(every), self._slabs[every[0]].nseg,
                                                     _lib.current_stream(dev))

@@ -8,6 +8,7 @@
 // moved tile by tile inside the slab (destination row <= source row, so a tile is read in full
 // before it is written).
 #include "common.hip.h"
+#include <type_traits>
 
 namespace trimkv {
 
@@ -304,20 +305,18 @@ struct EvictArgs {
     const int64_t* q_idx_dev; int64_t q_idx_all;
     // listed launch: workgroup i works on entry work[i] = layer * nseg + segment instead of (blockIdx.y, blockIdx.x)
     const int32_t* work; int nlayers;
+    // rows moved by launches of their own (trimkv_evict_split): per pair {rows kept, first row that moves, -, -}, the list of kept
+    // rows, and room for split_spill rows per chunk
+    int4* split_head; uint32_t* split_idx; char* split_stash; int split_stride, split_chunks, split_spill;
 };
 
-// blockIdx.y (or the work list) selects a layer: its slab addresses, capacity and query index replace the scalar fields,
-// and the per-layer parts of the other arrays are stepped to.  Returns the workgroup's segment, -1 for a list entry that
-// names no (layer, segment) of this launch.
-__device__ __forceinline__ int select_layer(EvictArgs& a) {
-    if (!a.layers) return blockIdx.x;
-    int layer = blockIdx.y, seg = blockIdx.x;
-    if (a.work) {
-        const int item = a.work[blockIdx.x];
-        if (item < 0 || item >= a.nlayers * a.nseg) return -1;
-        layer = item / a.nseg;
-        seg = item - layer * a.nseg;
-    }
+// The layer of pair `pair` (an entry of the work list, or layer * nseg + segment): its slab addresses, capacity and query index
+// replace the scalar fields, and the per-layer parts of the other arrays are stepped to.  Returns the segment, -1 for a list
+// entry that names no (layer, segment) of this launch.
+__device__ __forceinline__ int select_pair(EvictArgs& a, int pair) {
+    const int item = a.work ? a.work[pair] : pair;
+    if (item < 0 || item >= a.nlayers * a.nseg) return -1;
+    const int layer = item / a.nseg, seg = item - layer * a.nseg;
     const trimkv_layer_slabs L = a.layers[layer];
     a.k_slab = (char*)L.k_slab; a.v_slab = (char*)L.v_slab; a.lb_slab = (char*)L.lb_slab; a.pos_slab = L.pos_slab; a.seg_len = L.seg_len;
     a.q_idx = a.q_idx_dev ? *a.q_idx_dev : (a.q_idx_all > 0 ? a.q_idx_all : L.q_idx);
@@ -327,6 +326,115 @@ __device__ __forceinline__ int select_layer(EvictArgs& a) {
     if (a.thr_key) { a.thr_key += (int64_t)layer * a.thr_layer_stride; a.tie_take += (int64_t)layer * a.thr_layer_stride; }
     if (a.ws_keys) a.ws_keys += (int64_t)layer * a.nseg * a.ws_stride;
     return seg;
+}
+__device__ __forceinline__ int pair_of_block(const EvictArgs& a) { return a.work ? blockIdx.x : blockIdx.y * gridDim.x + blockIdx.x; }
+
+// ---- rows moved by several workgroups per segment ----------------------------------------------
+// With few segments in a launch most of the chip idles while one workgroup moves a long segment (84 GB/s: 8192 rows of 128
+// features in 100 us, behind 15 us of selection; in three launches 8 such segments take 60 instead of 167 us, and the
+// evictions between the token steps of 256 heads with lognormal budgets up to 8192 rows 53 instead of 107 us).  Then the launch that selects only leaves the list of kept rows, and the
+// destination rows are dealt out in chunks of SPLIT_ROWS.  A chunk's sources lie at or behind its destinations: those
+// inside its own rows nobody else touches; those behind them (the last ones of the chunk, no more than were evicted) are
+// copied aside by split_stash_kernel before split_move_kernel overwrites anything.  The order between the two is the order
+// of launches: nothing waits inside a launch.
+constexpr int SPLIT_ROWS = 512, SPLIT_FROM = 1024;      // rows per chunk; segments with fewer rows to move stay whole
+
+__device__ __forceinline__ int64_t split_stash_bytes(const EvictArgs& a) { return (int64_t)a.split_spill * (2 * a.row_bytes + 12); }
+// first row of lo .. hi - 1 whose source is `end` or behind it (sources ascend)
+__device__ __forceinline__ int first_spilled(const uint32_t* idx, int lo, int hi, int end) {
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((int)idx[mid] >= end) hi = mid; else lo = mid + 1;
+    }
+    return lo;
+}
+
+// blockIdx: chunk, pair, 0 = keys / 1 = values and metadata
+template <int PPR>      // 16-byte pieces per row
+__global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a) {
+    const int chunk = blockIdx.x, pair = blockIdx.y;
+    const int4 head = a.split_head[pair];
+    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
+    if (lo >= hi) return;
+    const int seg = select_pair(a, pair);
+    const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
+    const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS), m = hi - from;
+    if (seg < 0 || m <= 0) return;
+    char* stash = a.split_stash + ((int64_t)pair * a.split_chunks + chunk) * split_stash_bytes(a);
+    const char* src = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
+    char* dst = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
+    for (int base = 0; base < m * PPR; base += 8 * 256) {
+        uint4 t[8];
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            const int q = min(base + p * 256 + (int)threadIdx.x, m * PPR - 1);
+            t[p] = load_stream(src + (int64_t)idx[from + q / PPR] * a.row_bytes + (q % PPR) * 16);
+        }
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            const int q = base + p * 256 + (int)threadIdx.x;
+            if (q < m * PPR) *(uint4*)(dst + (int64_t)q * 16) = t[p];
+        }
+    }
+    if (blockIdx.z) {
+        int64_t* pos = (int64_t*)(stash + (int64_t)a.split_spill * 2 * a.row_bytes);
+        uint32_t* lb = (uint32_t*)(pos + a.split_spill);
+        const int lb_bytes = a.lb_dtype == TRIMKV_F32 ? 4 : 2;
+        const char* lbseg = a.lb_slab + (int64_t)seg * a.cap * lb_bytes;
+        const int64_t* posseg = a.pos_slab + (int64_t)seg * a.cap;
+        for (int r = threadIdx.x; r < m; r += 256) {
+            const int s = (int)idx[from + r];
+            pos[r] = posseg[s];
+            lb[r] = lb_bytes == 4 ? ((const uint32_t*)lbseg)[s] : (uint32_t)((const uint16_t*)lbseg)[s];
+        }
+    }
+}
+
+template <int PPR>
+__global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a) {
+    const int chunk = blockIdx.x, pair = blockIdx.y, tid = threadIdx.x;
+    const int4 head = a.split_head[pair];
+    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
+    if (lo >= hi) return;
+    const int seg = select_pair(a, pair);
+    if (seg < 0) return;
+    const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
+    const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS);
+    const char* stash = a.split_stash + ((int64_t)pair * a.split_chunks + chunk) * split_stash_bytes(a);
+    const char* kept = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
+    char* rows = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
+    uint4 t[PPR];
+#pragma unroll
+    for (int p = 0; p < PPR; ++p) {
+        const int q = p * SPLIT_ROWS + tid, r = min(lo + q / PPR, hi - 1), c = (q % PPR) * 16;
+        t[p] = load_stream(r < from ? rows + (int64_t)idx[r] * a.row_bytes + c : kept + (int64_t)(r - from) * a.row_bytes + c);
+    }
+    const int lb_bytes = a.lb_dtype == TRIMKV_F32 ? 4 : 2, r = min(lo + tid, hi - 1);
+    char* lbseg = a.lb_slab + (int64_t)seg * a.cap * lb_bytes;
+    int64_t* posseg = a.pos_slab + (int64_t)seg * a.cap;
+    int64_t pos = 0;
+    uint32_t lb = 0;
+    if (blockIdx.z) {
+        const int64_t* kpos = (const int64_t*)(stash + (int64_t)a.split_spill * 2 * a.row_bytes);
+        const int s = (int)idx[r];
+        pos = r < from ? posseg[s] : kpos[r - from];
+        lb = r >= from ? ((const uint32_t*)(kpos + a.split_spill))[r - from] : lb_bytes == 4 ? ((const uint32_t*)lbseg)[s] : (uint32_t)((const uint16_t*)lbseg)[s];
+    }
+#pragma unroll
+    for (int p = 0; p < PPR; ++p) land(t[p]);
+    land(pos);
+    land(lb);
+    __syncthreads();                                  // the chunk's rows are in registers: they may be overwritten
+#pragma unroll
+    for (int p = 0; p < PPR; ++p) {
+        const int q = p * SPLIT_ROWS + tid, row = lo + q / PPR;
+        if (row < hi) store_stream(rows + (int64_t)row * a.row_bytes + (q % PPR) * 16, t[p]);
+    }
+    if (blockIdx.z && lo + tid < hi) {
+        posseg[r] = pos;
+        if (lb_bytes == 4) ((uint32_t*)lbseg)[r] = lb;
+        else ((uint16_t*)lbseg)[r] = (uint16_t)lb;
+    }
 }
 
 // SELECT = true: find the cut inside the segment (trimkv_evict).
@@ -338,7 +446,8 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a) {
     __shared__ uint32_t scratch[EV_THREADS / 64 + 4];
     __shared__ int first_evicted;
 
-    const int seg = select_layer(a);
+    if (SELECT && a.split_head && threadIdx.x == 0) a.split_head[pair_of_block(a)] = make_int4(0, 0, 0, 0);   // nothing left to move, unless said otherwise below
+    const int seg = a.layers ? select_pair(a, pair_of_block(a)) : blockIdx.x;
     if (seg < 0) return;
     const int n = a.seg_len[seg];
     // nothing cached, a corrupt length, or more rows than the caller's bound (which sized the key array): touch nothing
@@ -383,7 +492,11 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a) {
         for (int r = threadIdx.x; r < kept && r < a.kept_stride; r += EV_THREADS)
             a.kept_idx[(int64_t)seg * a.kept_stride + r] = (int32_t)keys[r];
     }
-    if (first_moved < kept)
+    if (SELECT && a.split_head && kept - first_moved >= SPLIT_FROM && (n - kept <= a.split_spill || a.split_spill >= SPLIT_ROWS)) {
+        const int pair = pair_of_block(a);
+        for (int r = threadIdx.x; r < kept; r += EV_THREADS) a.split_idx[(int64_t)pair * a.split_stride + r] = keys[r];
+        if (threadIdx.x == 0) a.split_head[pair] = make_int4(kept, first_moved, 0, 0);
+    } else if (first_moved < kept)
         move_segment(kseg, vseg, lbseg, posseg, keys, kept, first_moved, a.row_bytes, a.lpr_shift, lb_bytes);
     if (threadIdx.x == 0) a.seg_len[seg] = kept;
 }
@@ -828,7 +941,8 @@ static int check_layer_args(const char* fn, const trimkv_layer_slabs* layers, in
     return TRIMKV_OK;
 }
 
-static int evict_layers_common(const char* fn, const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+// a: empty, or with the fields of trimkv_evict_split
+static int evict_layers_common(const char* fn, EvictArgs& a, const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
                                int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack,
                                int64_t q_idx, const int64_t* q_idx_dev,
                                int strategy, int rounding, int sliding_window, int max_len,
@@ -842,7 +956,6 @@ static int evict_layers_common(const char* fn, const trimkv_layer_slabs* layers,
         return fail(TRIMKV_ERR_SHAPE, "%s: keep_layer_stride must be 0 or nseg (got %d)", fn, keep_layer_stride);
     if (strategy != TRIMKV_SCORE_ALPHA && strategy != TRIMKV_SCORE_KNORM_ALPHA) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: unknown strategy %d", fn, strategy);
     if (rounding != TRIMKV_ROUND_UPCAST && rounding != TRIMKV_ROUND_NATIVE) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: unknown rounding %d", fn, rounding);
-    EvictArgs a = {};
     a.layers = layers; a.keep_layer_stride = keep_layer_stride; a.q_idx_all = q_idx; a.q_idx_dev = q_idx_dev;
     a.nseg = nseg; a.row_bytes = head_dim * 2; a.lpr_shift = lpr_shift; a.kv_dtype = kv_dtype; a.lb_dtype = lb_dtype;
     a.keep = keep; a.keep_per_seg = keep_per_seg; a.slack = slack < 0 ? 0 : slack;
@@ -857,7 +970,8 @@ extern "C" int trimkv_evict_layers(const trimkv_layer_slabs* layers, int nlayers
                                    int64_t q_idx, const int64_t* q_idx_dev,
                                    int strategy, int rounding, int sliding_window, int max_len,
                                    void* workspace, size_t workspace_bytes, void* stream) {
-    return evict_layers_common("trimkv_evict_layers", layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride,
+    EvictArgs a = {};
+    return evict_layers_common("trimkv_evict_layers", a, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride,
                                slack, q_idx, q_idx_dev, strategy, rounding, sliding_window, max_len, nullptr, 0, workspace, workspace_bytes, stream);
 }
 
@@ -871,8 +985,57 @@ extern "C" int trimkv_evict_listed(const trimkv_layer_slabs* layers, int nlayers
     if (nwork == 0) return TRIMKV_OK;
     if (!work) return fail(TRIMKV_ERR_NULL, "%s: null work list", fn);
     if (nwork < 0) return fail(TRIMKV_ERR_SHAPE, "%s: nwork=%d", fn, nwork);
-    return evict_layers_common(fn, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride,
+    EvictArgs a = {};
+    return evict_layers_common(fn, a, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride,
                                slack, q_idx, q_idx_dev, strategy, rounding, sliding_window, max_len, work, nwork, workspace, workspace_bytes, stream);
+}
+
+// workspace of trimkv_evict_split: heads, lists of kept rows, stashes
+struct SplitSizes { int chunks, spill; size_t idx, stash, total; };
+static SplitSizes split_sizes(int npairs, int max_len, int row_bytes, int spill) {
+    SplitSizes z;
+    z.chunks = (max_len + SPLIT_ROWS - 1) / SPLIT_ROWS;
+    z.spill = ((spill < SPLIT_ROWS ? spill : SPLIT_ROWS) + 3) / 4 * 4;      // rows of 12 bytes of metadata stay 16-byte aligned
+    z.idx = (size_t)npairs * sizeof(int4);
+    z.stash = (z.idx + (size_t)npairs * max_len * 4 + 255) / 256 * 256;
+    z.total = z.stash + (size_t)npairs * z.chunks * z.spill * (2 * row_bytes + 12);
+    return z;
+}
+
+extern "C" size_t trimkv_evict_split_workspace(int npairs, int max_len, int head_dim, int spill) {
+    if (npairs <= 0 || max_len <= 0 || head_dim <= 0 || spill <= 0) return 0;
+    return split_sizes(npairs, max_len, head_dim * 2, spill).total;
+}
+
+extern "C" int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                                  int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                                  int strategy, int rounding, int sliding_window, int max_len, int spill,
+                                  const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "trimkv_evict_split";
+    if (work && nwork == 0) return TRIMKV_OK;
+    if (nwork < 0 || spill <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: nwork=%d spill=%d", fn, nwork, spill);
+    if (head_dim != 64 && head_dim != 96 && head_dim != 128) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: head_dim %d (64, 96 or 128)", fn, head_dim);
+    if (max_len <= 0 || (size_t)max_len * 4 > (size_t)EV_LDS_KEY_BYTES) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: max_len %d (up to %d)", fn, max_len, EV_LDS_KEY_BYTES / 4);
+    const int64_t pairs = work ? nwork : (int64_t)nlayers * nseg;
+    if (pairs <= 0 || pairs > 65535) return fail(TRIMKV_ERR_SHAPE, "%s: %lld (layer, segment) pairs", fn, (long long)pairs);
+    const SplitSizes z = split_sizes((int)pairs, max_len, head_dim * 2, spill);
+    if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < z.total)
+        return fail(TRIMKV_ERR_WORKSPACE, "%s: aligned workspace of %zu bytes needed, got %zu", fn, z.total, workspace_bytes);
+    EvictArgs a{};
+    a.split_head = (int4*)workspace; a.split_idx = (uint32_t*)((char*)workspace + z.idx); a.split_stash = (char*)workspace + z.stash;
+    a.split_stride = max_len; a.split_chunks = z.chunks; a.split_spill = z.spill;
+    if (int rc = evict_layers_common(fn, a, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, nullptr, strategy,
+                                     rounding, sliding_window, max_len, work, nwork, nullptr, 0, stream)) return rc;
+    const dim3 grid(z.chunks, (unsigned)pairs, 2);
+    hipStream_t st = (hipStream_t)stream;
+    auto go = [&](auto ppr) {
+        hipLaunchKernelGGL((split_stash_kernel<decltype(ppr)::value>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((split_move_kernel<decltype(ppr)::value>), grid, dim3(SPLIT_ROWS), 0, st, a);
+    };
+    if (head_dim == 128) go(std::integral_constant<int, 16>{});
+    else if (head_dim == 96) go(std::integral_constant<int, 12>{});
+    else go(std::integral_constant<int, 8>{});
+    return launch_status(fn);
 }
 
 extern "C" int trimkv_compact_threshold_layers(const trimkv_layer_slabs* layers, int nlayers, int nseg, int segs_per_group, int head_dim,
