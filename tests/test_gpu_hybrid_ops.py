@@ -316,3 +316,11 @@ def test_values_that_are_not_finite_stay_out_of_rows_that_do_not_see_them(bad, a
     assert not ab[sees][:, 0].isfinite().any()
     assert (rb[:at] - r[:at]).abs().max() <= 1e-5
     assert not rb[at:, 0].isfinite().any()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_decode_of_sequences_with_fewer_rows_than_the_batch_is_split_for(dtype):
+    """A window of 1520 rows is split over twelve workgroups (127 rows each): sequences that fill one row, one share, one share and a
+    row, some, and all of them, decoded side by side."""
+    spec = ops.WindowSpec(2, 1, 64, 64, 1500, 20, 0.15)
+    run_window(spec, dtype, [4, 128, 129, 400, 1600], [[1] * 4, [125, 1, 1, 1], [126, 1, 1, 1], [397, 1, 1, 1], [1597, 1, 1, 1]])

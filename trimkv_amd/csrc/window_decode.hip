@@ -44,7 +44,9 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
     extern __shared__ float lds[];                  // [WAVES][GQ][L * 8 + 2]
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int per = a.H / a.G, passes = (per + GQ - 1) / GQ;
-    const int split = blockIdx.x, g = blockIdx.y / passes, h0 = (blockIdx.y % passes) * GQ, b = blockIdx.z;
+    // heads on the fast axis: workgroups go to the eight XCDs in turn, and with the splits there the XCDs of the later ones, which
+    // short sequences do not have, would idle
+    const int split = blockIdx.z, g = blockIdx.x / passes, h0 = (blockIdx.x % passes) * GQ, b = blockIdx.y;
     const int nh = min(GQ, per - h0);
     const int slot = a.slots[b], cap = a.keep + a.size;
     const int n = min(a.seen[2 * slot] + 1, cap);
@@ -60,6 +62,7 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
 #pragma unroll
         for (int y = 0; y < 8; ++y) q[x][y] = kin ? q[x][y] * a.scale_log2 : 0.0f;
     }
+    if (r0 >= n) return;                            // a short sequence has fewer shares; the combination knows (q is on its way by now)
     float m[GQ], l[GQ], acc[GQ][8];
 #pragma unroll
     for (int x = 0; x < GQ; ++x) {
@@ -166,7 +169,11 @@ __global__ __launch_bounds__(256) void window_combine_kernel(WindowArgs a) {
     const int64_t b = bh / a.H;
     const int h = (int)(bh - b * a.H), tid = threadIdx.x, row = a.Dv + 2;
     const float* w = a.ws + bh * a.splits * row;
-    const float m = tid < a.splits ? w[tid * row + a.Dv] : WA_NEG, l = tid < a.splits ? w[tid * row + a.Dv + 1] : 0.0f;
+    // everything is requested before the number of shares is known
+    float m = w[min(tid, a.splits - 1) * row + a.Dv], l = w[min(tid, a.splits - 1) * row + a.Dv + 1];
+    const int shares = min(a.splits, (min(a.seen[2 * a.slots[b]] + 1, a.keep + a.size) + a.chunk - 1) / a.chunk);
+    m = tid < shares ? m : WA_NEG;
+    l = tid < shares ? l : 0.0f;
     const float wm = wave_max_f(m);
     if ((tid & 63) == 0) part[tid >> 6] = wm;
     __syncthreads();
@@ -179,7 +186,7 @@ __global__ __launch_bounds__(256) void window_combine_kernel(WindowArgs a) {
     for (int d = tid; d < a.Dv; d += 256) {
         float num = 0.0f;
 #pragma unroll 8
-        for (int s = 0; s < a.splits; ++s) num += w[s * row + d] * f[s];
+        for (int s = 0; s < shares; ++s) num += w[s * row + d] * f[s];
         st((T*)a.out + bh * a.Dv + d, num * window_gate<T>(a, b, h, d));
     }
 }
@@ -190,7 +197,7 @@ static void launch_window_decode(const WindowArgs& a, int batch, hipStream_t s) 
     auto go = [&](auto gq) {
         constexpr int GQ = decltype(gq)::value;
         const int passes = (per + GQ - 1) / GQ;
-        hipLaunchKernelGGL((window_decode_kernel<T, L, GQ>), dim3(a.splits, a.G * passes, batch), dim3(256), 4 * GQ * (L * 8 + 2) * sizeof(float), s, a);
+        hipLaunchKernelGGL((window_decode_kernel<T, L, GQ>), dim3(a.G * passes, batch, a.splits), dim3(256), 4 * GQ * (L * 8 + 2) * sizeof(float), s, a);
     };
     if (per == 1) go(std::integral_constant<int, 1>{});
     else if (per == 2) go(std::integral_constant<int, 2>{});
@@ -202,12 +209,18 @@ static void launch_window_decode(const WindowArgs& a, int batch, hipStream_t s) 
 
 using namespace trimkv;
 
+constexpr int SHARE_ROWS = 1024;
+
 extern "C" int trimkv_window_decode_splits(int batch, int kv_heads, int capacity) {
     if (batch <= 0 || kv_heads <= 0 || capacity <= 0) return 1;
-    // enough workgroups to fill the chip, at least 128 rows for each
+    // Enough workgroups to fill the chip, at least 128 rows for each and no more than 1024: a batch's sequences differ in length, and
+    // the launch ends with the workgroup that has the most rows.  64 sequences of 256 .. 4096 rows x 8 heads of 128, a step of the
+    // two-layer decoder: 370 us with the splits on the fast axis of the grid, 347 with the heads there, 341 with 512 rows at most,
+    // which costs 64 full windows of 4096 rows 2 - 4 % (207 us).
     const int64_t pairs = (int64_t)batch * kv_heads;
     int64_t s = (2048 + pairs - 1) / pairs;
-    const int most = (capacity + 127) / 128;
+    const int most = (capacity + 127) / 128, least = (capacity + SHARE_ROWS - 1) / SHARE_ROWS;
+    s = s < least ? least : s;
     s = s < 1 ? 1 : s > most ? most : s;
     return (int)(s > 256 ? 256 : s);
 }
