@@ -459,6 +459,21 @@ int trimkv_append_attend_uniform(const void* q, void* out,
                                  const int64_t* pos_new, int64_t pos_stride_b, int64_t pos_stride_h,
                                  float scale, int len_before, int pieces_per_segment,
                                  void* workspace, size_t workspace_bytes, void* stream);
+/* The arguments of trimkv_append_attend_uniform (pieces = NULL) or trimkv_append_attend_pieces as one block: a caller that makes
+ * the same call for every layer and step fills in the second part only.  Layout: 64-bit fields throughout. */
+typedef struct trimkv_append_step {
+    void* k_slab; void* v_slab; void* lb_slab; int64_t* pos_slab; int32_t* seg_len; int32_t* cu_seqlens;
+    int64_t nseg, kv_heads, cap, head_dim, kv_dtype, lb_dtype;
+    const void* q; void* out;
+    const void* k_new; const void* v_new; int64_t kv_stride_b, kv_stride_h;
+    const void* lb_new; int64_t lb_stride_b, lb_stride_h;
+    const int64_t* pos_new; int64_t pos_stride_b, pos_stride_h;
+    int64_t group; double scale;
+    int64_t len;                  /* uniform: rows before the append; pieces: max_len */
+    int64_t count;                /* uniform: pieces per segment; pieces: entries of the list */
+    const int32_t* pieces; void* workspace; int64_t workspace_bytes;
+} trimkv_append_step;
+int trimkv_append_attend_step(const trimkv_append_step* step, void* stream);
 int trimkv_append_attend_uniform_gated(const void* q, void* out,
                                        void* k_slab, void* v_slab, void* lb_slab, int64_t* pos_slab, int32_t* seg_len, int32_t* cu_seqlens,
                                        int nseg, int kv_heads, int cap, int head_dim, int group, int kv_dtype, int lb_dtype,

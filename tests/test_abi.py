@@ -153,3 +153,22 @@ def test_registry_keys_and_lazy_log_beta():
     assert lz.shape == (2, 3, 4) and lz.transpose(1, 2).shape == (2, 4, 3) and lz.dim() == 3
     m = lz.transpose(1, 2).materialize()
     assert m.shape == (2, 4, 3) and torch.allclose(m, torch.nn.functional.logsigmoid(torch.tensor(10.0)).expand(2, 4, 3))
+
+
+def test_argument_blocks_and_split_evictions_refuse_what_the_plain_entry_points_refuse():
+    import ctypes
+    from trimkv_amd.cache_utils import _Slab
+    lib = _lib.load()
+    assert _Slab._STEP_FIXED.size + _Slab._STEP.size == 31 * 8        # struct trimkv_append_step
+    assert lib.trimkv_append_attend_step(None, None) == -1
+    block = ctypes.create_string_buffer(31 * 8)                       # all null
+    assert lib.trimkv_append_attend_step(ctypes.addressof(block), None) < 0
+    one = 256
+    split = lambda nwork=0, work=None, D=128, max_len=4096, spill=128, ws=one, nbytes=1 << 30, nl=2: lib.trimkv_evict_split(
+        one, nl, 4, D, _lib.BF16, _lib.F32, 8, None, 0, 0, 100, 0, 0, 0, max_len, spill, work, nwork, ws, nbytes, None)
+    assert split(nwork=0, work=one) == 0                              # an empty list launches nothing
+    assert split(nwork=-1, work=one) == -2 and split(spill=0) == -2 and split(nl=0) == -2
+    need = lib.trimkv_evict_split_workspace(8, 4096, 128, 128)
+    assert split(nbytes=need - 1) == split(ws=None) == split(ws=one + 8) < 0
+    assert split(D=80) == split(max_len=32769) < 0
+    assert need >= 8 * (16 + 4096 * 4 + 8 * 128 * (2 * 256 + 12)) and lib.trimkv_evict_split_workspace(0, 4096, 128, 128) == 0

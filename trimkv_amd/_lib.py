@@ -75,6 +75,7 @@ SIGNATURES = {
     "trimkv_decode_attn_uniform": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _f, _i, _i, _p, _sz, _p]),
     "trimkv_append_attend_uniform": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _i64,
                                           _p, _i64, _i64, _p, _i64, _i64, _f, _i, _i, _p, _sz, _p]),
+    "trimkv_append_attend_step": (_i, [_p, _p]),
     "trimkv_append_attend_uniform_gated": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _i64,
                                                 _p, _i, _p, _p, _i64, _i64, _f, _i, _i, _p, _sz, _p]),
     "trimkv_plan_attn_pieces": (_i, [_p, _i, _i, _i, _p, _i]),
@@ -185,11 +186,14 @@ def ptr(t) -> int:
     return None if t is None else t.data_ptr()
 
 
+_raw_stream = None
+
+
 def current_stream(device) -> int:
     """Raw hipStream_t of torch's current stream on ``device`` (the fast C accessor when torch has it)."""
+    global _raw_stream
     import torch
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        idx = device.index if isinstance(device, torch.device) else torch.device(device).index
-        return raw(torch.cuda.current_device() if idx is None else idx)
-    return torch.cuda.current_stream(device).cuda_stream
+    if _raw_stream is None:
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+    idx = device.index if isinstance(device, torch.device) else torch.device(device).index
+    return _raw_stream(torch.cuda.current_device() if idx is None else idx)

@@ -156,9 +156,12 @@ def append_attend(slab, query: torch.Tensor, group: int, scale: float, chunk: in
     gated = not torch.is_tensor(slab.pending[3])
     if uniform_pps > 0:      # a dense cache: every segment holds max_len - 1 rows before this token; length and cut are launch arguments
         ws = _workspace_zeroed(query.device, lib.trimkv_decode_attn_pieces_workspace(nseg * uniform_pps, group), st) if uniform_pps > 1 else None
-        fn = lib.trimkv_append_attend_uniform_gated if gated else lib.trimkv_append_attend_uniform
-        rc = fn(query.data_ptr(), out.data_ptr(), *slab.ptrs, nseg, slab.H, slab.cap, d, group, *slab.codes, *slab.pending[0], scale,
-                slab.max_len - 1, uniform_pps, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), st)
+        wp, wn = (0, 0) if ws is None else (ws.data_ptr(), ws.numel())
+        if gated:
+            rc = lib.trimkv_append_attend_uniform_gated(query.data_ptr(), out.data_ptr(), *slab.ptrs, nseg, slab.H, slab.cap, d, group, *slab.codes, *slab.pending[0], scale,
+                                                        slab.max_len - 1, uniform_pps, wp, wn, st)
+        else:      # one block of arguments instead of 34: the call is made for every layer of every step
+            rc = lib.trimkv_append_attend_step(slab.step_args(query.data_ptr(), out.data_ptr(), slab.pending[0], group, scale, slab.max_len - 1, uniform_pps, 0, wp, wn), st)
         if rc:
             _lib.check(rc, "trimkv_append_attend_uniform_gated" if gated else "trimkv_append_attend_uniform")
         slab.pending = None
@@ -166,9 +169,13 @@ def append_attend(slab, query: torch.Tensor, group: int, scale: float, chunk: in
     if pieces is not None:   # ragged lengths: one launch over the (segment, piece) list, merged inside it
         plist, npieces = pieces
         ws = _workspace_zeroed(query.device, lib.trimkv_decode_attn_pieces_workspace(npieces, group), st)
-        fn = lib.trimkv_append_attend_pieces_gated if gated else lib.trimkv_append_attend_pieces
-        rc = fn(query.data_ptr(), out.data_ptr(), *slab.ptrs, plist.data_ptr(), npieces, nseg, slab.H, slab.cap, d, group, *slab.codes,
-                *slab.pending[0], scale, bound if bound > 0 else slab.max_len, ws.data_ptr(), ws.numel(), st)
+        most = bound if bound > 0 else slab.max_len
+        if gated:
+            rc = lib.trimkv_append_attend_pieces_gated(query.data_ptr(), out.data_ptr(), *slab.ptrs, plist.data_ptr(), npieces, nseg, slab.H, slab.cap, d, group, *slab.codes,
+                                                       *slab.pending[0], scale, most, ws.data_ptr(), ws.numel(), st)
+        else:
+            rc = lib.trimkv_append_attend_step(slab.step_args(query.data_ptr(), out.data_ptr(), slab.pending[0], group, scale, most, npieces, plist.data_ptr(),
+                                                              ws.data_ptr(), ws.numel()), st)
         if rc:
             _lib.check(rc, "trimkv_append_attend_pieces_gated" if gated else "trimkv_append_attend_pieces")
         slab.pending = None
@@ -311,6 +318,21 @@ def _dense_torch_attention(query, key, value, attention_mask, scale: float, caus
     return torch.matmul(w.to(query.dtype), v).transpose(1, 2).contiguous()
 
 
+def _decode_step(query: torch.Tensor, key: torch.Tensor, slab, scaling: Optional[float]) -> Optional[torch.Tensor]:
+    """The usual decode step of a dense cache (one query row per sequence, the layer's append deferred to this call, nothing masked)
+    without the general path's questions: the call costs the host about half.  None: not that case."""
+    B, Hq, Q, D = query.shape
+    H = slab.H
+    G = Hq // H
+    if (Q != 1 or G > _MAX_GROUP or Hq != G * H or B != slab.B or D != slab.D or slab.pending is None or slab.cu is not None or not query.is_cuda
+            or query.dtype != slab.k.dtype or key.data_ptr() != slab.ptrs[0] or key.shape[2] != slab.max_len):
+        return None
+    q2 = query.reshape(B * Hq, D)
+    if not q2.is_contiguous():
+        q2 = q2.contiguous()
+    return append_attend(slab, q2, G, D ** -0.5 if scaling is None else scaling, uniform_pps=_uniform_cut(B * H, slab.max_len)).view(B, 1, Hq, D)
+
+
 def dense_attention_forward(module: nn.Module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
                             attention_mask: Optional[torch.Tensor] = None, scaling: Optional[float] = None,
                             dropout: float = 0.0, flash_attn_kwargs: Optional[dict] = None, sliding_window: Optional[int] = None,
@@ -324,6 +346,12 @@ def dense_attention_forward(module: nn.Module, query: torch.Tensor, key: torch.T
     ``dropout`` > 0 drops probabilities; ``softcap`` caps the scores.  At Q_LEN == 1 a window is a first attended row per
     segment and runs on the kernel, causality changes nothing; a window or ``is_causal=False`` on a query block, dropout
     and softcap run on torch ops and say so (``slow_path``)."""
+    kw = flash_attn_kwargs
+    if (kw and "pending_append" in kw and attention_mask is None and sliding_window is None and softcap is None and not dropout and not dense_chunk
+            and "lengths_on_device" not in kw):
+        out = _decode_step(query, key, kw["pending_append"][1], scaling)     # a decode step whose append rides along
+        if out is not None:
+            return out, None, None
     B, Hq, Q, D = query.shape
     Hkv, n = key.shape[1], key.shape[2]
     G = Hq // Hkv

@@ -17,7 +17,9 @@ There is no CPU path: tensors must live on the GPU and the library must be built
 """
 from __future__ import annotations
 
+import ctypes
 import math
+import struct
 from typing import Any, Dict, Iterable, List, Optional, Tuple
 
 import numpy as np
@@ -102,7 +104,8 @@ class _Slab:
     """Device storage of one layer."""
 
     __slots__ = ("k", "v", "lb", "pos", "seg_len", "cu", "B", "H", "D", "cap", "lens", "max_len", "k4", "v4", "lb3", "pos3", "ptrs", "order",
-                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host")
+                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host", "row_shape", "views", "step",
+                 "seg_start")
 
     def __init__(self, B, H, D, cap, kv_dtype, lb_dtype, device, ragged: bool):
         nseg = B * H
@@ -133,6 +136,43 @@ class _Slab:
         self.ptrs = (self.k.data_ptr(), self.v.data_ptr(), self.lb.data_ptr(), self.pos.data_ptr(), self.seg_len.data_ptr(),
                      None if self.cu is None else self.cu.data_ptr())
         self.codes = (_lib.dtype_code(self.k.dtype), _lib.dtype_code(self.lb.dtype))
+        self.row_shape = (B, H, 1, D)
+        self.views = {}
+        self.seg_start = None
+        self.step = None
+
+    # struct trimkv_append_step: what stays while the storage does not move, then what a step brings
+    _STEP_FIXED, _STEP = struct.Struct("12q"), struct.Struct("13qd5q")
+
+    def step_args(self, q: int, out: int, new: tuple, group: int, scale: float, rows: int, count: int, pieces: int, ws: int, ws_bytes: int) -> int:
+        """Address of a filled-in ``trimkv_append_step`` of this layer (valid until the next call)."""
+        buf = self.step
+        if buf is None:
+            buf = self.step = ctypes.create_string_buffer(self._STEP_FIXED.size + self._STEP.size)
+            k, v, lb, pos, seg_len, cu = self.ptrs
+            self._STEP_FIXED.pack_into(buf, 0, k, v, lb, pos, seg_len, cu or 0, self.nseg, self.H, self.cap, self.D, *self.codes)
+        self._STEP.pack_into(buf, self._STEP_FIXED.size, q, out, *new, group, scale, rows, count, pieces, ws, ws_bytes)
+        return ctypes.addressof(buf)
+
+    def rows(self, n: int):
+        """The first ``n`` rows of K, V, log beta and positions as [B,Hkv,n,...] views.  A decode step hands them out per layer and
+        the lengths of an eviction cycle come again, so the views are kept (four of them cost 5 us to make); they go when
+        storage moves, and views made under inference mode stay apart from others."""
+        key = (n, torch.is_inference_mode_enabled())
+        got = self.views.get(key)
+        if got is None or got[0].requires_grad or got[1].requires_grad:
+            if len(self.views) >= 1024:
+                self.views.clear()
+            got = self.views[key] = (self.k4.narrow(2, 0, n), self.v4.narrow(2, 0, n), self.lb3.narrow(2, 0, n), self.pos3.narrow(2, 0, n))
+        return got
+
+    def flat(self):
+        """K, V, log beta and positions with the segments one behind the other, [nseg * cap, ...] (kept like ``rows``)."""
+        key = ("flat", torch.is_inference_mode_enabled())
+        got = self.views.get(key)
+        if got is None or got[0].requires_grad or got[1].requires_grad:
+            got = self.views[key] = (self.k.view(-1, self.D), self.v.view(-1, self.D), self.lb.view(-1, 1), self.pos.view(-1, 1))
+        return got
 
     @property
     def nseg(self) -> int:
@@ -215,10 +255,11 @@ class _SlabBacked(_CacheBase):
         lazy = isinstance(lb, LazyLogBeta)
         if not k.is_cuda or not (lazy or lb.is_cuda):
             return False
-        B, H, D = slab.B, slab.H, slab.D
-        if tuple(k.shape) != (B, H, 1, D) or v.shape != k.shape or v.dtype != k.dtype or k.dtype != slab.k.dtype:
+        B, H = slab.B, slab.H
+        dt = k.dtype
+        if k.shape != slab.row_shape or v.shape != slab.row_shape or v.dtype != dt or dt != slab.k.dtype:
             return False
-        if tuple(lb.shape) != (B, H, 1) or lb.dtype != slab.lb.dtype:
+        if lb.shape != slab.row_shape[:3] or lb.dtype != slab.lb.dtype:
             return False
         if lazy:
             # the gate's partial sums [slices, B, Hkv]: the attention launch finishes them (trimkv_append_attend_gated),
@@ -228,9 +269,11 @@ class _SlabBacked(_CacheBase):
                 return False
             lb_args = (part.data_ptr(), part.shape[0], lb.bias_f32.data_ptr())
         else:
-            lb_args = (lb.data_ptr(), lb.stride(0), lb.stride(1))
+            ls = lb.stride()
+            lb_args = (lb.data_ptr(), ls[0], ls[1])
         ks, vs = k.stride(), v.stride()   # the stride over the single new token does not matter
-        if ks[3] != 1 or (ks[0] | ks[1]) % 8 or (vs[0], vs[1], vs[3]) != (ks[0], ks[1], ks[3]) or (k.data_ptr() | v.data_ptr()) % 16:
+        kp, vp = k.data_ptr(), v.data_ptr()
+        if ks[3] != 1 or (ks[0] | ks[1]) % 8 or vs[0] != ks[0] or vs[1] != ks[1] or vs[3] != 1 or (kp | vp) % 16:
             return False
         if pos.dtype != torch.int64 or pos.device != k.device:
             return False
@@ -245,11 +288,10 @@ class _SlabBacked(_CacheBase):
         # [0]: what trimkv_append_attend(_gated) needs of the new row (addresses, element strides over batch and head; for a
         # lazy log beta the partial sums, their slice count and the bias); [1:]: the tensors themselves, kept alive and
         # used by _flush
-        slab.pending = ((k.data_ptr(), v.data_ptr(), ks[0], ks[1], *lb_args, pos.data_ptr(), ps[0], ps[1]),
-                        k, v, lb, pos)
+        slab.pending = ((kp, vp, ks[0], ks[1], *lb_args, pos.data_ptr(), ps[0], ps[1]), k, v, lb, pos)
         slab.lens += 1
         slab.max_len += 1
-        slab.total += slab.lens.size
+        slab.total += B * H
         return True
 
     def _flush(self, slab: Optional[_Slab]) -> None:
@@ -618,8 +660,7 @@ class TrimKVCache(_SlabBacked):
             return (self.key_cache[layer], self.value_cache[layer], self.retention_weights[layer], self.kv_positions[layer])
         if flush and s.pending is not None:
             self._flush(s)
-        n = s.max_len
-        return (s.k4.narrow(2, 0, n), s.v4.narrow(2, 0, n), s.lb3.narrow(2, 0, n), s.pos3.narrow(2, 0, n))
+        return s.rows(s.max_len)
 
     def __getitem__(self, layer_idx: int):
         if layer_idx < len(self):
@@ -968,8 +1009,7 @@ class _RaggedCache(_SlabBacked):
             # head_lens / cu_seqlens_k still hold the values before this token: the attention call that receives this
             # dictionary appends the row and advances them in the same launch
             kw["pending_append"] = (self, slab)
-        flat = (slab.k.view(-1, slab.D), slab.v.view(-1, slab.D), slab.lb.view(-1, 1), slab.pos.view(-1, 1))
-        return flat, kw
+        return slab.flat(), kw
 
     def _piece_list(self, slab: _Slab):
         """The decode-attention launch of a ragged layer as a list of (segment, piece) workgroups, see
@@ -1013,12 +1053,14 @@ class _RaggedCache(_SlabBacked):
         return slab.pieces
 
     def _seg_start(self, slab: _Slab) -> torch.Tensor:
-        key = ("seg_start", slab.nseg, slab.cap, str(slab.k.device))
-        t = self._tables.get(key)
-        if t is None:
-            t = torch.arange(slab.nseg, dtype=torch.int32, device=slab.k.device) * slab.cap
-            self._tables[key] = t
-        return t
+        if slab.seg_start is None:
+            key = ("seg_start", slab.nseg, slab.cap, str(slab.k.device))
+            t = self._tables.get(key)
+            if t is None:
+                t = torch.arange(slab.nseg, dtype=torch.int32, device=slab.k.device) * slab.cap
+                self._tables[key] = t
+            slab.seg_start = t
+        return slab.seg_start
 
     # ---- selection plumbing ----------------------------------------------------------------
     @staticmethod

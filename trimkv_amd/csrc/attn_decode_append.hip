@@ -61,3 +61,16 @@ extern "C" int trimkv_append_attend_uniform(const void* q, void* out,
     else launch_pieces_append(a, npieces, group, head_dim, kv_dtype, (hipStream_t)stream);
     return launch_status(fn);
 }
+
+static_assert(sizeof(trimkv_append_step) == 31 * 8, "64-bit fields without gaps");
+extern "C" int trimkv_append_attend_step(const trimkv_append_step* s, void* stream) {
+    if (!s) return fail(TRIMKV_ERR_NULL, "trimkv_append_attend_step: null arguments");
+    const int nseg = (int)s->nseg, heads = (int)s->kv_heads, cap = (int)s->cap, dim = (int)s->head_dim, group = (int)s->group, kv = (int)s->kv_dtype, lb = (int)s->lb_dtype;
+    if (s->pieces)
+        return trimkv_append_attend_pieces(s->q, s->out, s->k_slab, s->v_slab, s->lb_slab, s->pos_slab, s->seg_len, s->cu_seqlens, s->pieces, (int)s->count, nseg, heads, cap, dim,
+                                           group, kv, lb, s->k_new, s->v_new, s->kv_stride_b, s->kv_stride_h, s->lb_new, s->lb_stride_b, s->lb_stride_h, s->pos_new,
+                                           s->pos_stride_b, s->pos_stride_h, (float)s->scale, (int)s->len, s->workspace, (size_t)s->workspace_bytes, stream);
+    return trimkv_append_attend_uniform(s->q, s->out, s->k_slab, s->v_slab, s->lb_slab, s->pos_slab, s->seg_len, s->cu_seqlens, nseg, heads, cap, dim, group, kv, lb, s->k_new,
+                                        s->v_new, s->kv_stride_b, s->kv_stride_h, s->lb_new, s->lb_stride_b, s->lb_stride_h, s->pos_new, s->pos_stride_b, s->pos_stride_h,
+                                        (float)s->scale, (int)s->len, (int)s->count, s->workspace, (size_t)s->workspace_bytes, stream);
+}
