@@ -585,6 +585,22 @@ int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, i
                         int max_len, void* stream);
 
 /*
+ * trimkv_prefill_attn_split -- trimkv_prefill_attn with the keys of a query tile (256 / group query times of a segment)
+ * divided among workgroups that take split_tiles * 64 keys each; their unfinished outputs, exponent references and row sums
+ * (fp32) are merged by a second launch.  Same operands and results (up to the rounding of the merge).
+ * `workspace`: at least trimkv_prefill_split_workspace(...) bytes, 16-byte aligned, contents of no meaning before and after.
+ * trimkv_prefill_split_tiles: the split_tiles at which this is expected to be faster than one workgroup per query tile, or 0
+ * where it is not (uneven: the segments' lengths differ and max_len is that of the longest).
+ * Returns TRIMKV_OK or a negative trimkv_status (as trimkv_prefill_attn; split_tiles <= 0 or a workspace that is too small).
+ */
+int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven);
+int64_t trimkv_prefill_split_workspace(int batch, int kv_heads, int group, int q_len, int max_len, int split_tiles);
+int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+                              const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
+                              int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
+                              int max_len, int split_tiles, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * trimkv_rmsnorm / trimkv_qk_norm_rope / trimkv_silu_mul -- the element-wise work of a decoder layer around the cache
  * path, one launch each (a module-by-module decoder issues 5-16 small launches for each, and a decode step is bound
  * by their number).  dtype: TRIMKV_BF16 or TRIMKV_F16; every intermediate is rounded where the torch modules round it.

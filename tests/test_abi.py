@@ -172,3 +172,13 @@ def test_argument_blocks_and_split_evictions_refuse_what_the_plain_entry_points_
     assert split(nbytes=need - 1) == split(ws=None) == split(ws=one + 8) < 0
     assert split(D=80) == split(max_len=32769) < 0
     assert need >= 8 * (16 + 4096 * 4 + 8 * 128 * (2 * 256 + 12)) and lib.trimkv_evict_split_workspace(0, 4096, 128, 128) == 0
+    divided = lambda tiles=8, ws=one, nbytes=1 << 30, n=4096, D=128: lib.trimkv_prefill_attn_split(
+        one, 1 << 20, 1 << 15, 128, one, one, one, None, None, 1, 8, 2, 256, n, D, _lib.BF16, 0.1, n, tiles, ws, nbytes, None)
+    need = lib.trimkv_prefill_split_workspace(1, 8, 2, 256, 4096, 8)
+    assert need == 8 * 2 * 8 * 256 * 130 * 4 and lib.trimkv_prefill_split_workspace(1, 8, 2, 256, 4096, 0) == 0
+    assert divided(nbytes=need - 1) == divided(ws=None) == divided(ws=one + 8) < 0
+    assert divided(tiles=0) == divided(n=0) == -2 and divided(D=80) < 0
+    rule = lambda batch, heads, group, q_len, n, uneven=0: lib.trimkv_prefill_split_tiles(batch, heads, group, q_len, n, uneven)
+    assert rule(1, 8, 2, 63, 65536) == 0 and rule(4, 64, 1, 256, 8192) == 0     # short chunks; as many query tiles as CUs
+    assert rule(1, 8, 4, 512, 4096) == 16 and rule(1, 8, 4, 1280, 8192) == 0 and rule(1, 8, 4, 1280, 8192, 1) == 43
+    assert all(rule(1, 8, 4, 64 * q, n) * 32 >= (n + 63) // 64 or rule(1, 8, 4, 64 * q, n) == 0 for q in range(1, 40) for n in (64, 1000, 50000))

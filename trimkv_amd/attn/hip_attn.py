@@ -18,6 +18,7 @@ ragged entry points ignore ``attention_mask`` and ``scaling`` (flash_attn.py:15,
 """
 from __future__ import annotations
 
+import functools
 import os
 import warnings
 from typing import Dict, Optional, Tuple
@@ -211,6 +212,14 @@ def _take_pending(kw: Optional[dict], query: torch.Tensor, key: torch.Tensor, gr
     return None
 
 
+@functools.lru_cache(maxsize=1024)
+def _prefill_split(batch: int, kv_heads: int, group: int, q_len: int, max_len: int, uneven: bool) -> Tuple[int, int]:
+    """(64-key tiles per workgroup, workspace bytes) of a chunk's attention; (0, 0): a query tile's keys stay together."""
+    lib = _lib.load()
+    tiles = lib.trimkv_prefill_split_tiles(batch, kv_heads, group, q_len, max_len, uneven)
+    return tiles, lib.trimkv_prefill_split_workspace(batch, kv_heads, group, q_len, max_len, tiles)
+
+
 def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.Tensor, batch: int, kv_heads: int, group: int,
                       seg_len: Optional[torch.Tensor], seg_start: Optional[torch.Tensor], cap: int, max_len: int,
                       scale: float) -> torch.Tensor:
@@ -231,11 +240,20 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
     if query.stride(3) != 1 or any(s % 8 for s in query.stride()[:3]) or query.data_ptr() % 16:
         query = query.contiguous()
     out = torch.empty(B, Q, Hq, D, dtype=query.dtype, device=query.device)
-    rc = lib.trimkv_prefill_attn(query.data_ptr(), query.stride(0), query.stride(1), query.stride(2), out.data_ptr(),
-                                 k_rows.data_ptr(), v_rows.data_ptr(), _lib.ptr(seg_len), _lib.ptr(seg_start),
-                                 batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len,
-                                 _lib.current_stream(query.device))
-    _lib.check(rc, "trimkv_prefill_attn")
+    args = (query.data_ptr(), query.stride(0), query.stride(1), query.stride(2), out.data_ptr(),
+            k_rows.data_ptr(), v_rows.data_ptr(), _lib.ptr(seg_len), _lib.ptr(seg_start),
+            batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len)
+    stream = _lib.current_stream(query.device)
+    tiles, need = _prefill_split(batch, kv_heads, group, Q, max_len, seg_start is not None)
+    if tiles:   # few query tiles: their keys divided among several workgroups
+        try:
+            work = torch.empty(need, dtype=torch.uint8, device=query.device)
+        except torch.OutOfMemoryError:
+            work = None
+        if work is not None:
+            _lib.check(lib.trimkv_prefill_attn_split(*args, tiles, work.data_ptr(), need, stream), "trimkv_prefill_attn_split")
+            return out
+    _lib.check(lib.trimkv_prefill_attn(*args, stream), "trimkv_prefill_attn")
     return out
 
 

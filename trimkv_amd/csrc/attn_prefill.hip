@@ -47,6 +47,7 @@ struct PrefillArgs {
     int kv_heads, group, q_len, cap, max_len;
     int hd;                                         // real head_dim: rows of K, V, q and out hold hd elements
     float scale_log2;
+    int split_tiles; float* part; float* part_ml;   // keys split over workgroups: tiles of keys apiece, unfinished outputs, their references and sums
 };
 
 template <int G>
@@ -308,7 +309,9 @@ __device__ __forceinline__ void pf2_load_to_lds(const char* sbase, uint32_t voff
                  : "=&s"(saved) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 
-template <bool F16>
+// SPLIT: blockIdx.z takes split_tiles tiles of the keys.  Where a query tile has more than that, its workgroups leave unnormalised
+// outputs with their exponent references and row sums (fp32) for prefill_merge_kernel; else the one workgroup writes the result.
+template <bool F16, bool SPLIT>
 __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(16))) char pf2_lds[];
     PF_LDS3 char* const lds3 = (PF_LDS3 char*)pf2_lds;
@@ -378,7 +381,10 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     for (int v = 0; v < 16; ++v) negm[v] = 0.0f;
 
     const int t_last = min(Q - 1, t_wg0 + BT - 1);
-    const int k_end = max(0, min(n, n - Q + t_last + 1));     // keys the workgroup visits
+    const int k_end = max(0, min(n, n - Q + t_last + 1));     // keys the query tile sees
+    const int all_tiles = (k_end + PF2_BN - 1) / PF2_BN;
+    const int t_first = SPLIT ? (int)blockIdx.z * a.split_tiles : 0;   // the workgroup's first tile of keys
+    if (SPLIT && t_first > 0 && t_first >= all_tiles) return;
     const int vis_j = n - Q + t_q;                            // last key this lane's query sees
     const int vis_lo = n - Q + t_w_first;                     // ... the wavefront's first query
     const int last_row = max(n - 1, 0);
@@ -396,7 +402,7 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     const uint32_t st_koff = (uint32_t)st_row * row_bytes + st_kcol;     // offsets inside a tile whose 64 rows all exist
     const uint32_t st_voff = (uint32_t)st_row * row_bytes + st_vcol;
     auto request_tile = [&](int tt, int buf) __attribute__((always_inline)) {
-        const int kbase = tt * PF2_BN;
+        const int kbase = (t_first + tt) * PF2_BN;
         const uint32_t dk = lds0 + buf * PF2_TILE + w * 1024, dv = dk + PF2_VBASE;
         if (kbase + PF2_BN <= n) {   // wave-uniform; the tile's base goes into the scalar base address
             const char* kt = kseg + (uint32_t)kbase * row_bytes;
@@ -455,12 +461,13 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     auto prepare = [&](pf_f32x16& s, int blk, float tmax, auto first_c) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first_c)::value;
         if (FIRST) tmax = max16(s);
-        if (blk * 32 + 31 > vis_lo) {   // wave-uniform: some query of the wavefront does not see the whole block
+        const int key0 = (blk + 2 * t_first) * 32;
+        if (key0 + 31 > vis_lo) {   // wave-uniform: some query of the wavefront does not see the whole block
             // (the empty volatile statement keeps this a branch: as 48 speculated selects it would run for every block)
             asm volatile("" ::: );
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int key = blk * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
+                const int key = key0 + 8 * (v >> 2) + 4 * hl + (v & 3);
                 s[v] = key <= vis_j ? s[v] : PF_NEG;
             }
             tmax = max16(s);
@@ -567,7 +574,7 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     // of block b + 1 and then P.V of block b.  Every wavefront walks all blocks of the workgroup's tiles: the blocks that
     // lie wholly above a wavefront's diagonal (at most two of up to several hundred, the workgroup spans BT query times)
     // are masked like the diagonal ones and contribute zeros, which keeps the loop free of per-wavefront branches.
-    const int ntiles = (k_end + PF2_BN - 1) / PF2_BN;
+    const int ntiles = SPLIT ? min(all_tiles - t_first, a.split_tiles) : all_tiles;
     if (ntiles > 0) {
         pf_f32x16 s_a, s_b;   // scores of the current and of the next block, roles swapping every step
         pf_bf16x8 pre[PF2_PD];
@@ -617,6 +624,17 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
 
     // the two halves of a query hold disjoint keys: add their sums, then normalise and store
     l_run += __shfl_xor(l_run, 32, 64);
+    if (SPLIT && all_tiles > a.split_tiles) {
+        const int64_t wg = ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile;
+        if (hl == 0) *(float2*)(a.part_ml + (wg * (PF2_WAVES * 32) + r) * 2) = make_float2(m_ref, l_run);
+        float4* po = (float4*)a.part + (wg * PF2_WAVES + w) * (16 * 64) + lane;   // in register order: 1 KB per store
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                po[(db * 4 + c) * 64] = make_float4(o[db][4 * c], o[db][4 * c + 1], o[db][4 * c + 2], o[db][4 * c + 3]);
+        return;
+    }
     if (q_ok) {
         const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
         char* orow = (char*)(a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + (h * G + g)) * a.hd);
@@ -632,6 +650,80 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     }
 }
 
+// The shares of the keys put together: one wavefront per (query tile, 32 of its rows, 32 features), lanes as they wrote.
+// A share that a row saw nothing of has sum 0 and a reference of no meaning: it is left out.
+template <bool F16>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+    const int seg = blockIdx.y, tile = (int)blockIdx.x >> 3, w = (int)blockIdx.x & 7, tiles = (int)gridDim.x >> 3;
+    const int b = seg / a.kv_heads, h = seg - b * a.kv_heads;
+    int n = a.seg_len ? a.seg_len[seg] : a.max_len;
+    n = max(0, min(n, a.max_len));
+    const int db = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, hl = lane >> 5;
+    const int G = a.group, Q = a.q_len, BT = (PF2_WAVES * 32) / G;
+    const int t_last = min(Q - 1, tile * BT + BT - 1);
+    const int all_tiles = (max(0, min(n, n - Q + t_last + 1)) + PF2_BN - 1) / PF2_BN;
+    if (all_tiles <= a.split_tiles) return;   // one share: its workgroup wrote the result
+    const int shares = (all_tiles + a.split_tiles - 1) / a.split_tiles;
+    const int r = w * 32 + j, g = r % G, t_q = tile * BT + r / G;
+    if (r >= BT * G || t_q >= Q) return;
+    const int64_t wg = (int64_t)seg * tiles + tile, per_share = (int64_t)gridDim.y * tiles;
+    const float2* ml = (const float2*)a.part_ml + wg * (PF2_WAVES * 32) + r;
+    const float4* po = (const float4*)a.part + (wg * PF2_WAVES + w) * (16 * 64) + db * (4 * 64) + lane;
+    float m = -3.0e38f;
+    for (int z = 0; z < shares; ++z) {
+        const float2 x = ml[z * per_share * (PF2_WAVES * 32)];
+        if ((__float_as_uint(x.y) << 1) != 0) m = __builtin_fmaxf(m, x.x);
+    }
+    float l = 0.0f;
+    float4 o[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 2
+    for (int z = 0; z < shares; ++z) {
+        const float2 x = ml[z * per_share * (PF2_WAVES * 32)];
+        float4 v[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = po[z * per_share * (PF2_WAVES * 16 * 64) + c * 64];
+        const float f = (__float_as_uint(x.y) << 1) != 0 ? __builtin_amdgcn_exp2f(x.x - m) : 0.0f;
+        l += x.y * f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { o[c].x += v[c].x * f; o[c].y += v[c].y * f; o[c].z += v[c].z * f; o[c].w += v[c].w * f; }
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    char* orow = (char*)(a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + (h * G + g)) * a.hd);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int d = db * 32 + 8 * c + 4 * hl;
+        if (d < a.hd) *(uint2*)(orow + d * 2) = make_uint2(pack_kv<F16>(o[c].x * inv, o[c].y * inv), pack_kv<F16>(o[c].z * inv, o[c].w * inv));
+    }
+}
+
+constexpr int PF2_PART = PF2_WAVES * 32 * (PF_D + 2) * 4;   // bytes that one workgroup leaves for the merge
+
+// > 64 KB of dynamic LDS needs the attribute once per device (the flag is only ever set, so a race repeats the call at worst)
+template <bool F16, bool SPLIT>
+static int opt_in_lds() {
+    static bool done[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+    if (dev < 0 || !done[dev]) {
+        hipError_t e = hipFuncSetAttribute((const void*)prefill_attn_kernel<F16, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, PF2_LDS);
+        if (e != hipSuccess) return (int)e;
+        if (dev >= 0) done[dev] = true;
+    }
+    return 0;
+}
+
+template <bool F16>
+static int launch_prefill_split(const PrefillArgs& a, int nseg, hipStream_t st) {
+    if (int rc = opt_in_lds<F16, true>()) return rc;
+    const int bt = (PF2_WAVES * 32) / a.group, tiles = (a.q_len + bt - 1) / bt;
+    const int key_tiles = (a.max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + a.split_tiles - 1) / a.split_tiles;
+    hipLaunchKernelGGL((prefill_attn_kernel<F16, true>), dim3(tiles, nseg, shares), dim3(PF2_THREADS), PF2_LDS, st, a);
+    hipLaunchKernelGGL(prefill_merge_kernel<F16>, dim3(tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
+    return 0;
+}
+
 template <int G, bool F16>
 static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
     // short chunks: 16 queries per wavefront waste fewer MFMA columns
@@ -641,17 +733,9 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
         hipLaunchKernelGGL((prefill_small_kernel<G, F16>), dim3(tiles, nseg), dim3(C::THREADS), 0, st, a);
         return 0;
     }
-    // > 64 KB of dynamic LDS needs the attribute once per device (the flag is only ever set, so a race repeats the call at worst)
-    static bool lds_opted_in[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
-    if (dev < 0 || !lds_opted_in[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)prefill_attn_kernel<F16>, hipFuncAttributeMaxDynamicSharedMemorySize, PF2_LDS);
-        if (e != hipSuccess) return (int)e;
-        if (dev >= 0) lds_opted_in[dev] = true;
-    }
+    if (int rc = opt_in_lds<F16, false>()) return rc;
     const int bt = (PF2_WAVES * 32) / G;
-    hipLaunchKernelGGL(prefill_attn_kernel<F16>, dim3((a.q_len + bt - 1) / bt, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<F16, false>), dim3((a.q_len + bt - 1) / bt, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
     return 0;
 }
 
@@ -659,11 +743,11 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
 
 using namespace trimkv;
 
-extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+// Checks what both entry points take, and fills the arguments.
+static int prefill_args(const char* fn, PrefillArgs& a, const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
                                    const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
                                    int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
-                                   int max_len, void* stream) {
-    const char* fn = "trimkv_prefill_attn";
+                                   int max_len) {
     if (!q || !out || !k_slab || !v_slab) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (dtype != TRIMKV_BF16 && dtype != TRIMKV_F16) return fail(TRIMKV_ERR_DTYPE, "%s: K/V/q must be bf16 or fp16 (dtype=%d)", fn, dtype);
     if (head_dim != 128 && head_dim != 96 && head_dim != 64) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: head_dim must be 64, 96 or 128 (got %d)", fn, head_dim);
@@ -675,23 +759,91 @@ extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_
     if (!seg_start && max_len > cap) return fail(TRIMKV_ERR_CAPACITY, "%s: max_len %d exceeds capacity %d", fn, max_len, cap);
     if (((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_slab | (uintptr_t)v_slab) & 15 || ((q_stride_b | q_stride_h | q_stride_t) & 7))
         return fail(TRIMKV_ERR_SHAPE, "%s: q/out/K/V must be 16-byte aligned and q strides multiples of 8 elements", fn);
-    PrefillArgs a;
     a.q = (const uint16_t*)q; a.q_sb = q_stride_b; a.q_sh = q_stride_h; a.q_st = q_stride_t; a.out = (uint16_t*)out;
     a.k = (const char*)k_slab; a.v = (const char*)v_slab; a.seg_len = seg_len; a.seg_start = seg_start;
     a.kv_heads = kv_heads; a.group = group; a.q_len = q_len; a.cap = cap; a.max_len = max_len; a.hd = head_dim; a.scale_log2 = scale * 1.4426950408889634f;
+    a.split_tiles = 0; a.part = nullptr; a.part_ml = nullptr;
+    return 0;
+}
+
+extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+                                   const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
+                                   int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
+                                   int max_len, void* stream) {
+    const char* fn = "trimkv_prefill_attn";
+    PrefillArgs a;
+    if (int bad = prefill_args(fn, a, q, q_stride_b, q_stride_h, q_stride_t, out, k_slab, v_slab, seg_len, seg_start, batch, kv_heads,
+                               group, q_len, cap, head_dim, dtype, scale, max_len)) return bad;
+    const int nseg = batch * kv_heads;
     hipStream_t st = (hipStream_t)stream;
     const bool f16 = dtype == TRIMKV_F16;
     int rc = 0;
     switch (group) {
-        case 1: rc = f16 ? launch_prefill<1, true>(a, (int)nseg, st) : launch_prefill<1, false>(a, (int)nseg, st); break;
-        case 2: rc = f16 ? launch_prefill<2, true>(a, (int)nseg, st) : launch_prefill<2, false>(a, (int)nseg, st); break;
-        case 3: rc = f16 ? launch_prefill<3, true>(a, (int)nseg, st) : launch_prefill<3, false>(a, (int)nseg, st); break;
-        case 4: rc = f16 ? launch_prefill<4, true>(a, (int)nseg, st) : launch_prefill<4, false>(a, (int)nseg, st); break;
-        case 5: rc = f16 ? launch_prefill<5, true>(a, (int)nseg, st) : launch_prefill<5, false>(a, (int)nseg, st); break;
-        case 6: rc = f16 ? launch_prefill<6, true>(a, (int)nseg, st) : launch_prefill<6, false>(a, (int)nseg, st); break;
-        case 7: rc = f16 ? launch_prefill<7, true>(a, (int)nseg, st) : launch_prefill<7, false>(a, (int)nseg, st); break;
-        default: rc = f16 ? launch_prefill<8, true>(a, (int)nseg, st) : launch_prefill<8, false>(a, (int)nseg, st); break;
+        case 1: rc = f16 ? launch_prefill<1, true>(a, nseg, st) : launch_prefill<1, false>(a, nseg, st); break;
+        case 2: rc = f16 ? launch_prefill<2, true>(a, nseg, st) : launch_prefill<2, false>(a, nseg, st); break;
+        case 3: rc = f16 ? launch_prefill<3, true>(a, nseg, st) : launch_prefill<3, false>(a, nseg, st); break;
+        case 4: rc = f16 ? launch_prefill<4, true>(a, nseg, st) : launch_prefill<4, false>(a, nseg, st); break;
+        case 5: rc = f16 ? launch_prefill<5, true>(a, nseg, st) : launch_prefill<5, false>(a, nseg, st); break;
+        case 6: rc = f16 ? launch_prefill<6, true>(a, nseg, st) : launch_prefill<6, false>(a, nseg, st); break;
+        case 7: rc = f16 ? launch_prefill<7, true>(a, nseg, st) : launch_prefill<7, false>(a, nseg, st); break;
+        default: rc = f16 ? launch_prefill<8, true>(a, nseg, st) : launch_prefill<8, false>(a, nseg, st); break;
     }
+    if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
+    return launch_status(fn);
+}
+
+// ---- keys of a query tile split over several workgroups ----
+// A query tile (256 / group times of one segment) is one workgroup, and a CU holds one: a chunk of few segments leaves CUs idle
+// for as long as its longest segment takes (1.15 us per 64 keys).  Up to 128 query tiles the keys go to S workgroups of a query
+// tile, all of them on the chip at once (tiles * S <= 256).  What S costs was fitted to tiles 8 .. 128, 512 .. 65536 keys: 3 us
+// for the merge's launch, 0.8 us per share that a row's merge walks, 0.045 us per workgroup for its 130 KB written and read.
+// Measured (us, D 128, whole -> split): 8 tiles of 2048 keys 44 -> 21, of 8192 keys 150 -> 31; 32 of 4096 79 -> 35; 56 of 2954
+// 64 -> 37; 96 of 4096 80 -> 57; 128 of 8192 155 -> 107; left whole: 96 of 2048 44 -> 40, of 1024 27 -> 30, 40 of 1024 27 -> 25.
+// Between 128 and 256 tiles of like length the chip's rate gains nothing from more workgroups (168 tiles of 2954 keys: 68 -> 77);
+// of unlike segments the longest one holds up the rest, and three shares let the others' CUs help: 168 .. 224 tiles, lengths
+// uniform up to 4096 keys 80 -> 74 .. 85 -> 83, to 10000 keys 188 -> 166 .. 197 -> 170; up to 3000 keys 63 -> 70, hence the line.
+extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
+    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len < 64 || max_len <= 0) return 0;
+    const int64_t bt = (PF2_WAVES * 32) / group, items = (q_len + bt - 1) / bt * batch * kv_heads;
+    const int64_t key_tiles = ((int64_t)max_len + PF2_BN - 1) / PF2_BN;
+    if (items >= 256) return 0;
+    if (items > 128) return uneven && key_tiles >= 64 ? (int)((key_tiles + 2) / 3) : 0;
+    float best = 1.15f * (float)key_tiles - 8.0f;   // below that the second launch costs a caller whose queue runs dry as much
+    int64_t take = 0;
+    for (int64_t s = 2; s <= 32 && items * s <= 256; ++s) {
+        const int64_t each = (key_tiles + s - 1) / s;
+        const float us = 1.15f * (float)each + 3.0f + (0.8f + 0.045f * (float)items) * (float)s;
+        if (us < best) { best = us; take = each; }
+    }
+    return (int)take;
+}
+
+extern "C" int64_t trimkv_prefill_split_workspace(int batch, int kv_heads, int group, int q_len, int max_len, int split_tiles) {
+    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0 || split_tiles <= 0) return 0;
+    const int64_t bt = (PF2_WAVES * 32) / group, tiles = (q_len + bt - 1) / bt;
+    const int64_t key_tiles = ((int64_t)max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + split_tiles - 1) / split_tiles;
+    return tiles * batch * kv_heads * shares * PF2_PART;
+}
+
+extern "C" int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+                                         const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
+                                         int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
+                                         int max_len, int split_tiles, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "trimkv_prefill_attn_split";
+    PrefillArgs a;
+    if (int bad = prefill_args(fn, a, q, q_stride_b, q_stride_h, q_stride_t, out, k_slab, v_slab, seg_len, seg_start, batch, kv_heads,
+                               group, q_len, cap, head_dim, dtype, scale, max_len)) return bad;
+    if (split_tiles <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: split_tiles must be positive (got %d)", fn, split_tiles);
+    const int64_t need = trimkv_prefill_split_workspace(batch, kv_heads, group, q_len, max_len, split_tiles);
+    const int64_t shares = (((int64_t)max_len + PF2_BN - 1) / PF2_BN + split_tiles - 1) / split_tiles;
+    if (shares > 65535) return fail(TRIMKV_ERR_SHAPE, "%s: %lld shares of the keys exceed the grid limit 65535", fn, (long long)shares);
+    if (!workspace || workspace_bytes < need || (uintptr_t)workspace & 15)
+        return fail(TRIMKV_ERR_CAPACITY, "%s: needs a 16-byte aligned workspace of %lld bytes (got %lld)", fn, (long long)need, (long long)workspace_bytes);
+    a.split_tiles = split_tiles;
+    a.part = (float*)workspace;
+    a.part_ml = (float*)workspace + need / PF2_PART * (PF2_WAVES * 32 * PF_D);
+    hipStream_t st = (hipStream_t)stream;
+    const int rc = dtype == TRIMKV_F16 ? launch_prefill_split<true>(a, batch * kv_heads, st) : launch_prefill_split<false>(a, batch * kv_heads, st);
     if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
     return launch_status(fn);
 }
