@@ -308,6 +308,16 @@ int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, 
                        const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * trimkv_evict_host_layers -- trimkv_evict_layers (spill = 0) or trimkv_evict_split (spill > 0) over up to 48 layers whose table
+ * is in HOST memory: it travels in the launches' arguments, so that slabs which have just moved need no upload.  Read before the
+ * call returns.  Other arguments, workspace and results as there.
+ */
+int trimkv_evict_host_layers(const trimkv_layer_slabs* host_layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                             int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                             int strategy, int rounding, int sliding_window, int max_len, int spill,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * trimkv_compact_threshold_layers -- trimkv_compact_threshold for nlayers layers in one launch
  * (the per-layer rebuild loops at cache_utils.py:466-482, 912-943).  thr_key / tie_take are
  * [ngroups] shared by all layers (thr_layer_stride = 0: one budget across layers) or

@@ -172,6 +172,10 @@ def test_argument_blocks_and_split_evictions_refuse_what_the_plain_entry_points_
     assert split(nbytes=need - 1) == split(ws=None) == split(ws=one + 8) < 0
     assert split(D=80) == split(max_len=32769) < 0
     assert need >= 8 * (16 + 4096 * 4 + 8 * 128 * (2 * 256 + 12)) and lib.trimkv_evict_split_workspace(0, 4096, 128, 128) == 0
+    table = bytearray(2 * 56)                                         # read on the host: null slabs are refused before any launch
+    host = lambda nl=2, spill=128, at=ctypes.addressof((ctypes.c_char * 112).from_buffer(table)): lib.trimkv_evict_host_layers(
+        at, nl, 4, 128, _lib.BF16, _lib.F32, 8, None, 0, 0, 100, 0, 0, 0, 4096, spill, one, 1 << 30, None)
+    assert host() == host(spill=0) == host(at=None) < 0 and host(nl=49) == host(nl=0) == host(spill=-1) == -2
     divided = lambda tiles=8, ws=one, nbytes=1 << 30, n=4096, D=128: lib.trimkv_prefill_attn_split(
         one, 1 << 20, 1 << 15, 128, one, one, one, None, None, 1, 8, 2, 256, n, D, _lib.BF16, 0.1, n, tiles, ws, nbytes, None)
     need = lib.trimkv_prefill_split_workspace(1, 8, 2, 256, 4096, 8)

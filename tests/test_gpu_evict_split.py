@@ -87,3 +87,18 @@ def test_work_list_with_budgets_of_its_own_against_one_workgroup_per_segment(mon
         for x, y in zip(a, b):
             assert torch.equal(x, y)
     assert [int(t) for t in cache.head_lens[0]] == budgets[0].tolist()
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("layers", [3, 48, 49])
+def test_layers_in_the_arguments_and_in_a_device_table(layers, split, monkeypatch):
+    """Up to 48 layers travel with the launch, more in a device table; one query index for all, or one per layer."""
+    monkeypatch.setattr(cache_utils, "split_evict", lambda *a: split)
+    n, M = 2200, 2000
+    keep = np.sort(np.random.default_rng(layers).choice(n, size=M, replace=False))
+    for qs in (n + 1, [n + 1 + l for l in range(layers)]):
+        cache, held = _filled(TrimKVCache, layers, 1, 1, n, 64, torch.bfloat16, torch.float32, keep)
+        every = list(range(layers))
+        cache._evict_layers(every, M, None, 0, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST, 0, qs)
+        _check(cache, held, keep, f"{layers} layers")
+        assert (("host", *every) in cache._table_cache) == (layers <= 48)

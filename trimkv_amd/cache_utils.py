@@ -88,15 +88,16 @@ class LazyLogBeta:
         return out.transpose(1, 2) if self.transposed else out
 
 
-def split_evict(longest: int, rows: int, spill: int, head_dim: int) -> bool:
+def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -> bool:
     """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split``): ``rows`` due rows
-    in all, the longest segment of ``longest``, none losing more than ``spill``.  One workgroup per segment takes about
+    in all, the longest segment of ``longest``, at most ``kept`` of a segment's left, none losing more than ``spill``.  One workgroup per segment takes about
     15 us + 18 ns a row of the longest one; three launches and the detour of the rows that cross a chunk's end take about 30 us
     + 0.25 ns a row (0.4 ns when most rows cross).  Measured, whole -> split, segments of 128 features that lose 128 rows:
     8 x 8320 167 -> 60 us, 32 x 8320 196 -> 107, 64 x 4224 117 -> 98, 64 x 2176 63 -> 66, 128 x 8320 253 -> 270; losing 4096:
-    8 x 12288 181 -> 89, 32 x 12288 207 -> 156, 64 x 12288 240 -> 257.  Not while a graph is captured: the launches' table may be
-    uploaded for the first time."""
-    return (2048 <= longest <= 32768 and head_dim in (64, 96, 128) and rows * (5 if spill < 512 else 8) < 360 * longest - 300000
+    8 x 12288 181 -> 89, 32 x 12288 207 -> 156, 64 x 12288 240 -> 257; of few kept rows one workgroup is done as soon: 16 segments of
+    4100 cut to 1100 58 -> 67, of 6945 cut to 4043 102 -> 74.  Not while a graph is captured: the launches' table may be uploaded
+    for the first time."""
+    return (2048 <= kept and longest <= 32768 and head_dim in (64, 96, 128) and rows * (5 if spill < 512 else 8) < 360 * longest - 300000
             and not torch.cuda.is_current_stream_capturing())
 
 
@@ -399,6 +400,18 @@ class _SlabBacked(_CacheBase):
         self._table_cache[key] = ([s.ptrs for s in slabs], [s.cap for s in slabs], tables)
         return tables
 
+    def _host_table(self, layers: List[int]) -> np.ndarray:
+        """The ``trimkv_layer_slabs`` of ``layers`` on the host, for the launches that carry them in their arguments: slabs that
+        have just moved need no upload.  Kept while no slab of the set moves, like the device tables."""
+        key, slabs = ("host", *layers), [self._slabs[l] for l in layers]
+        hit = self._table_cache.get(key)
+        if hit is None or hit[1] != [s.cap for s in slabs] or not all(a is s.ptrs for a, s in zip(hit[0], slabs)):
+            arr = np.zeros(len(layers), dtype=self._LAYER_DT)
+            for i, s in enumerate(slabs):
+                arr[i] = (s.ptrs[0], s.ptrs[1], s.ptrs[2], s.ptrs[3], s.ptrs[4], 0, s.cap, 0)
+            hit = self._table_cache[key] = ([s.ptrs for s in slabs], [s.cap for s in slabs], arr)
+        return hit[2]
+
     def _layer_table_with_q(self, layers: List[int], q_of_layer) -> torch.Tensor:
         """A one-off ``trimkv_layer_slabs`` table that carries a different query index per layer (layers that have seen
         different numbers of tokens); uploaded for this launch."""
@@ -410,18 +423,25 @@ class _SlabBacked(_CacheBase):
 
     def _evict_layers(self, layers: List[int], keep: int, keep_per_seg, slack: int, strategy_code: int,
                       rounding: int, sliding_window: int, q_idx, work: Optional[np.ndarray] = None, spill: int = 512,
-                      due: Optional[Tuple[int, int]] = None) -> None:
+                      due: Optional[Tuple[int, int, int]] = None) -> None:
         """``trimkv_evict_layers`` over ``layers`` (all of one shape): one launch of nseg x len(layers) workgroups.
         ``q_idx``: the query index, one int or one per layer.  ``keep_per_seg``: None, a host array (uploaded) or a device
         int32 tensor, ``[nseg]`` or ``[len(layers), nseg]``.  ``work``: host int32 array of ``index in layers * nseg +
         segment``: only these pairs get a workgroup (``trimkv_evict_listed``); it reaches the device through pinned memory
         in stream order.  ``spill``: the most rows a segment loses, where the caller knows (512: any number); ``due``: rows of the longest segment
-        that is due, and of all that are."""
+        that is due, of all that are, and the most that one of them keeps."""
         s0 = self._slabs[layers[0]]
         dev = s0.k.device
         max_len = max(self._slabs[l].max_len for l in layers)
         qs = [int(q_idx)] * len(layers) if np.isscalar(q_idx) else [int(q) for q in q_idx]
-        if all(q == qs[0] for q in qs) and qs[0] > 0:
+        one_q = all(q == qs[0] for q in qs) and qs[0] > 0
+        on_host = work is None and len(layers) <= 48 and not torch.cuda.is_current_stream_capturing()
+        if on_host:
+            table, q_all = self._host_table(layers), qs[0] if one_q else 0
+            if not one_q:
+                table = table.copy()
+                table["q"] = qs
+        elif one_q:
             table, q_all = self._device_tables(layers)["slabs"], qs[0]
         else:
             table, q_all = self._layer_table_with_q(layers, qs), 0
@@ -435,13 +455,18 @@ class _SlabBacked(_CacheBase):
         lib = _lib.load()
         pairs = len(layers) * s0.nseg if work is None else int(work.size)
         wdev = None if work is None else self._upload_work(work, len(layers) * s0.nseg, dev)
-        if split_evict(*(due or (max_len, pairs * max_len)), spill, s0.D) and max_len <= 32768:
-            ws = self._workspace(lib.trimkv_evict_split_workspace(pairs, max_len, s0.D, spill), dev)
-            rc = lib.trimkv_evict_split(table.data_ptr(), len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype),
-                                        int(keep), _lib.ptr(kdev), stride, int(slack), q_all, strategy_code, rounding, int(sliding_window),
-                                        max_len, spill, _lib.ptr(wdev), 0 if work is None else pairs, ws.data_ptr(), ws.numel(), _lib.current_stream(dev))
-            _lib.check(rc, "trimkv_evict_split")
-            self._keepalive_layers = (table, kdev)
+        split = split_evict(*(due or (max_len, pairs * max_len, max_len if kdev is not None else keep)), spill, s0.D) and max_len <= 32768
+        if on_host or split:
+            ws = self._workspace(lib.trimkv_evict_split_workspace(pairs, max_len, s0.D, spill) if split
+                                 else len(layers) * lib.trimkv_evict_workspace(s0.nseg, max_len), dev)
+            shape = (len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype), int(keep), _lib.ptr(kdev), stride, int(slack), q_all,
+                     strategy_code, rounding, int(sliding_window), max_len)
+            room = (_lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.current_stream(dev))
+            if on_host:
+                _lib.check(lib.trimkv_evict_host_layers(table.ctypes.data, *shape, spill if split else 0, *room), "trimkv_evict_host_layers")
+            else:
+                _lib.check(lib.trimkv_evict_split(table.data_ptr(), *shape, spill, _lib.ptr(wdev), 0 if work is None else pairs, *room), "trimkv_evict_split")
+            self._keepalive_layers = (table, kdev)   # read asynchronously by the launch
             return
         ws = self._workspace(len(layers) * lib.trimkv_evict_workspace(s0.nseg, max_len), dev)
         if work is not None:
@@ -734,7 +759,7 @@ class TrimKVCache(_SlabBacked):
         lost = min(512, max(1, max((self._slabs[l].max_len for l in todo), default=0) - memory_size))
         first = self._slabs[todo[0]] if todo else None
         # the usual case: every layer is due at the same step -> one launch
-        if len(todo) > 1 and self._layers_alike(todo) or len(todo) == 1 and split_evict(first.max_len, first.nseg * first.max_len, lost, first.D):
+        if len(todo) > 1 and self._layers_alike(todo) or len(todo) == 1 and split_evict(first.max_len, first.nseg * first.max_len, memory_size, lost, first.D):
             self._evict_layers(todo, memory_size, None, 0, self._dense_strategy_code(strategy), _lib.ROUND_UPCAST,
                                self.sliding_window_size, [self.get_seq_length(l) + 1 for l in todo], spill=lost)
             for l in todo:
@@ -1335,7 +1360,7 @@ class _RaggedCache(_SlabBacked):
             work = np.flatnonzero(hit_all).astype(np.int32) if ndue * 4 < hit_all.size else None
             due_lens = lens_all[hit_all]
             self._evict_layers(every, 0, keep, buffer_size, code, _lib.ROUND_NATIVE, 0, q_idx, work=work,
-                               spill=min(512, int((lens_all - kh_all)[hit_all].max())), due=(int(due_lens.max()), int(due_lens.sum())))
+                               spill=min(512, int((lens_all - kh_all)[hit_all].max())), due=(int(due_lens.max()), int(due_lens.sum()), int(np.broadcast_to(kh_all, lens_all.shape)[hit_all].max())))
             t = self._device_tables(every)
             rc = lib.trimkv_build_cu_seqlens_layers(t["len"].data_ptr(), t["cu"].data_ptr(), len(every), self._slabs[every[0]].nseg,
                                                     _lib.current_stream(dev))

@@ -310,14 +310,24 @@ struct EvictArgs {
     int4* split_head; uint32_t* split_idx; char* split_stash; int split_stride, split_chunks, split_spill;
 };
 
+// The slabs of the layers of a launch: in a device table (EvictArgs::layers, N = 0) or in the launch's own arguments.  A table
+// has to be uploaded whenever a slab moved, with a wait for everything queued before: a chunk of 3213 tokens on a budget of 557,
+// whose slab grows and shrinks every time, took 363 us with it and 183 without.
+constexpr int HOST_LAYERS = 48;   // 2688 bytes of the 4 KB of arguments
+template <int N> struct SlabTable { trimkv_layer_slabs at[N]; };
+template <> struct SlabTable<0> {};
+
 // The layer of pair `pair` (an entry of the work list, or layer * nseg + segment): its slab addresses, capacity and query index
 // replace the scalar fields, and the per-layer parts of the other arrays are stepped to.  Returns the segment, -1 for a list
 // entry that names no (layer, segment) of this launch.
-__device__ __forceinline__ int select_pair(EvictArgs& a, int pair) {
+template <int N>
+__device__ __forceinline__ int select_pair(EvictArgs& a, const SlabTable<N>& t, int pair) {
     const int item = a.work ? a.work[pair] : pair;
     if (item < 0 || item >= a.nlayers * a.nseg) return -1;
     const int layer = item / a.nseg, seg = item - layer * a.nseg;
-    const trimkv_layer_slabs L = a.layers[layer];
+    trimkv_layer_slabs L;
+    if constexpr (N > 0) L = t.at[layer];
+    else L = a.layers[layer];
     a.k_slab = (char*)L.k_slab; a.v_slab = (char*)L.v_slab; a.lb_slab = (char*)L.lb_slab; a.pos_slab = L.pos_slab; a.seg_len = L.seg_len;
     a.q_idx = a.q_idx_dev ? *a.q_idx_dev : (a.q_idx_all > 0 ? a.q_idx_all : L.q_idx);
     a.cap = L.cap;
@@ -350,13 +360,13 @@ __device__ __forceinline__ int first_spilled(const uint32_t* idx, int lo, int hi
 }
 
 // blockIdx: chunk, pair, 0 = keys / 1 = values and metadata
-template <int PPR>      // 16-byte pieces per row
-__global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a) {
+template <int PPR, int N>      // 16-byte pieces per row; layers in the arguments
+__global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const SlabTable<N> table) {
     const int chunk = blockIdx.x, pair = blockIdx.y;
     const int4 head = a.split_head[pair];
     const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
     if (lo >= hi) return;
-    const int seg = select_pair(a, pair);
+    const int seg = select_pair(a, table, pair);
     const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
     const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS), m = hi - from;
     if (seg < 0 || m <= 0) return;
@@ -390,13 +400,13 @@ __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a) {
     }
 }
 
-template <int PPR>
-__global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a) {
+template <int PPR, int N>
+__global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a, const SlabTable<N> table) {
     const int chunk = blockIdx.x, pair = blockIdx.y, tid = threadIdx.x;
     const int4 head = a.split_head[pair];
     const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
     if (lo >= hi) return;
-    const int seg = select_pair(a, pair);
+    const int seg = select_pair(a, table, pair);
     if (seg < 0) return;
     const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
     const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS);
@@ -439,15 +449,15 @@ __global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a) {
 
 // SELECT = true: find the cut inside the segment (trimkv_evict).
 // SELECT = false: the cut comes from thr_key/tie_take/tie_base (trimkv_compact_threshold).
-template <bool LDS_KEYS, bool SELECT>
-__global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a) {
+template <bool LDS_KEYS, bool SELECT, int N>
+__global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const SlabTable<N> table) {
     extern __shared__ uint32_t lds_keys[];
     __shared__ uint32_t hist[256];
     __shared__ uint32_t scratch[EV_THREADS / 64 + 4];
     __shared__ int first_evicted;
 
     if (SELECT && a.split_head && threadIdx.x == 0) a.split_head[pair_of_block(a)] = make_int4(0, 0, 0, 0);   // nothing left to move, unless said otherwise below
-    const int seg = a.layers ? select_pair(a, pair_of_block(a)) : blockIdx.x;
+    const int seg = N > 0 || a.layers ? select_pair(a, table, pair_of_block(a)) : blockIdx.x;
     if (seg < 0) return;
     const int n = a.seg_len[seg];
     // nothing cached, a corrupt length, or more rows than the caller's bound (which sized the key array): touch nothing
@@ -834,8 +844,9 @@ static int lpr_shift_of(int row_bytes) {
     return s;
 }
 
-template <bool SELECT>
-static int launch_evict(const char* fn, EvictArgs& a, int max_len, void* workspace, size_t workspace_bytes, hipStream_t st, int nlayers = 1, int nwork = 0) {
+template <bool SELECT, int N = 0>
+static int launch_evict(const char* fn, EvictArgs& a, int max_len, void* workspace, size_t workspace_bytes, hipStream_t st, int nlayers = 1, int nwork = 0,
+                        const SlabTable<N>& table = SlabTable<N>{}) {
     const size_t key_bytes = (size_t)max_len * 4;
     a.max_len = max_len;
     a.nlayers = nlayers;
@@ -847,18 +858,18 @@ static int launch_evict(const char* fn, EvictArgs& a, int max_len, void* workspa
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
         if (dev < 0 || !attr_set[dev]) {
-            hipError_t e = hipFuncSetAttribute((const void*)evict_kernel<true, SELECT>, hipFuncAttributeMaxDynamicSharedMemorySize, EV_LDS_KEY_BYTES);
+            hipError_t e = hipFuncSetAttribute((const void*)evict_kernel<true, SELECT, N>, hipFuncAttributeMaxDynamicSharedMemorySize, EV_LDS_KEY_BYTES);
             if (e != hipSuccess) return fail((int)e, "%s: hipFuncSetAttribute: %s", fn, hipGetErrorString(e));
             if (dev >= 0) attr_set[dev] = true;
         }
-        hipLaunchKernelGGL((evict_kernel<true, SELECT>), grid, dim3(EV_THREADS), key_bytes, st, a);
+        hipLaunchKernelGGL((evict_kernel<true, SELECT, N>), grid, dim3(EV_THREADS), key_bytes, st, a, table);
     } else {
         const size_t need = (size_t)nlayers * a.nseg * max_len * 4;
         if (!workspace || workspace_bytes < need)
             return fail(TRIMKV_ERR_WORKSPACE, "%s: workspace of %zu bytes needed for max_len=%d, got %zu", fn, need, max_len, workspace_bytes);
         a.ws_keys = (uint32_t*)workspace;
         a.ws_stride = max_len;
-        hipLaunchKernelGGL((evict_kernel<false, SELECT>), grid, dim3(EV_THREADS), 0, st, a);
+        hipLaunchKernelGGL((evict_kernel<false, SELECT, N>), grid, dim3(EV_THREADS), 0, st, a, table);
     }
     return launch_status(fn);
 }
@@ -941,13 +952,14 @@ static int check_layer_args(const char* fn, const trimkv_layer_slabs* layers, in
     return TRIMKV_OK;
 }
 
-// a: empty, or with the fields of trimkv_evict_split
+// a: empty, or with the fields of trimkv_evict_split; table: the layers' slabs where they are arguments of the launch
+template <int N = 0>
 static int evict_layers_common(const char* fn, EvictArgs& a, const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
                                int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack,
                                int64_t q_idx, const int64_t* q_idx_dev,
                                int strategy, int rounding, int sliding_window, int max_len,
                                const int32_t* work, int nwork,
-                               void* workspace, size_t workspace_bytes, void* stream) {
+                               void* workspace, size_t workspace_bytes, void* stream, const SlabTable<N>& table = SlabTable<N>{}) {
     int lpr_shift;
     int rc = check_layer_args(fn, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, max_len, &lpr_shift);
     if (rc) return rc;
@@ -962,7 +974,7 @@ static int evict_layers_common(const char* fn, EvictArgs& a, const trimkv_layer_
     a.strategy = strategy; a.rounding = rounding; a.sliding_window = sliding_window < 0 ? 0 : sliding_window;
     a.segs_per_group = 1;
     a.work = work;
-    return launch_evict<true>(fn, a, max_len, workspace, workspace_bytes, (hipStream_t)stream, nlayers, nwork);
+    return launch_evict<true>(fn, a, max_len, workspace, workspace_bytes, (hipStream_t)stream, nlayers, nwork, table);
 }
 
 extern "C" int trimkv_evict_layers(const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
@@ -1007,11 +1019,11 @@ extern "C" size_t trimkv_evict_split_workspace(int npairs, int max_len, int head
     return split_sizes(npairs, max_len, head_dim * 2, spill).total;
 }
 
-extern "C" int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+template <int N = 0>
+static int evict_split_common(const char* fn, const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
                                   int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
                                   int strategy, int rounding, int sliding_window, int max_len, int spill,
-                                  const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream) {
-    const char* fn = "trimkv_evict_split";
+                                  const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream, const SlabTable<N>& table = SlabTable<N>{}) {
     if (work && nwork == 0) return TRIMKV_OK;
     if (nwork < 0 || spill <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: nwork=%d spill=%d", fn, nwork, spill);
     if (head_dim != 64 && head_dim != 96 && head_dim != 128) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: head_dim %d (64, 96 or 128)", fn, head_dim);
@@ -1025,17 +1037,45 @@ extern "C" int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers,
     a.split_head = (int4*)workspace; a.split_idx = (uint32_t*)((char*)workspace + z.idx); a.split_stash = (char*)workspace + z.stash;
     a.split_stride = max_len; a.split_chunks = z.chunks; a.split_spill = z.spill;
     if (int rc = evict_layers_common(fn, a, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, nullptr, strategy,
-                                     rounding, sliding_window, max_len, work, nwork, nullptr, 0, stream)) return rc;
+                                     rounding, sliding_window, max_len, work, nwork, nullptr, 0, stream, table)) return rc;
     const dim3 grid(z.chunks, (unsigned)pairs, 2);
     hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto ppr) {
-        hipLaunchKernelGGL((split_stash_kernel<decltype(ppr)::value>), grid, dim3(256), 0, st, a);
-        hipLaunchKernelGGL((split_move_kernel<decltype(ppr)::value>), grid, dim3(SPLIT_ROWS), 0, st, a);
+        hipLaunchKernelGGL((split_stash_kernel<decltype(ppr)::value, N>), grid, dim3(256), 0, st, a, table);
+        hipLaunchKernelGGL((split_move_kernel<decltype(ppr)::value, N>), grid, dim3(SPLIT_ROWS), 0, st, a, table);
     };
     if (head_dim == 128) go(std::integral_constant<int, 16>{});
     else if (head_dim == 96) go(std::integral_constant<int, 12>{});
     else go(std::integral_constant<int, 8>{});
     return launch_status(fn);
+}
+
+extern "C" int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                                  int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                                  int strategy, int rounding, int sliding_window, int max_len, int spill,
+                                  const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream) {
+    return evict_split_common("trimkv_evict_split", layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx,
+                              strategy, rounding, sliding_window, max_len, spill, work, nwork, workspace, workspace_bytes, stream);
+}
+
+extern "C" int trimkv_evict_host_layers(const trimkv_layer_slabs* host_layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                                        int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                                        int strategy, int rounding, int sliding_window, int max_len, int spill,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "trimkv_evict_host_layers";
+    if (!host_layers) return fail(TRIMKV_ERR_NULL, "%s: null layer table", fn);
+    if (nlayers <= 0 || nlayers > HOST_LAYERS || spill < 0) return fail(TRIMKV_ERR_SHAPE, "%s: nlayers=%d (up to %d) spill=%d", fn, nlayers, HOST_LAYERS, spill);
+    SlabTable<HOST_LAYERS> table{};
+    for (int l = 0; l < nlayers; ++l) {
+        const trimkv_layer_slabs& s = table.at[l] = host_layers[l];
+        int lpr_shift;
+        if (int rc = check_slab_args(fn, s.k_slab, s.v_slab, s.lb_slab, s.pos_slab, s.seg_len, nseg, s.cap < max_len ? max_len : s.cap, head_dim, kv_dtype, lb_dtype, max_len, &lpr_shift)) return rc;   // rows past a layer's capacity: that segment is left alone
+    }
+    if (spill > 0) return evict_split_common(fn, host_layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, strategy,
+                                             rounding, sliding_window, max_len, spill, nullptr, 0, workspace, workspace_bytes, stream, table);
+    EvictArgs a = {};
+    return evict_layers_common(fn, a, host_layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, nullptr,
+                               strategy, rounding, sliding_window, max_len, nullptr, 0, workspace, workspace_bytes, stream, table);
 }
 
 extern "C" int trimkv_compact_threshold_layers(const trimkv_layer_slabs* layers, int nlayers, int nseg, int segs_per_group, int head_dim,
