@@ -231,6 +231,18 @@ int trimkv_group_threshold_wide(const void* const* lb_slabs, const int64_t* cons
                                 void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * trimkv_group_threshold_wide_each_layer -- trimkv_group_threshold_each_layer spread over workgroups in the same way.
+ * workspace: nlayers * trimkv_group_threshold_workspace(1, nseg, segs_per_group) bytes, 4-byte aligned.
+ */
+int trimkv_group_threshold_wide_each_layer(const void* const* lb_slabs, const int64_t* const* pos_slabs,
+                                const void* const* k_slabs, const int32_t* const* seg_lens,
+                                int nlayers, int nseg, int segs_per_group, int cap, int head_dim,
+                                int kv_dtype, int lb_dtype, int64_t budget, int use_threshold, float threshold_score,
+                                int64_t q_idx, int strategy, int rounding,
+                                uint32_t* thr_key, int32_t* tie_take, int32_t* tie_base, int32_t* new_len, int32_t* first_kept,
+                                void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * trimkv_compact_threshold -- in-place compaction of one layer against group thresholds:
  * keeps token i of segment seg iff key_i > thr_key[g] or (key_i == thr_key[g] and its rank
  * among equal keys, tie_base[seg] + rank inside the segment, is < tie_take[g]); g =

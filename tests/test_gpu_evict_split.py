@@ -102,3 +102,34 @@ def test_layers_in_the_arguments_and_in_a_device_table(layers, split, monkeypatc
         cache._evict_layers(every, M, None, 0, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST, 0, qs)
         _check(cache, held, keep, f"{layers} layers")
         assert (("host", *every) in cache._table_cache) == (layers <= 48)
+
+
+@pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
+@pytest.mark.parametrize("budget", [0, 1, 700, 10 ** 6])
+def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(budget, lb_dtype, strategy):
+    """Ties by the hundred, empty segments, lengths around the 256 and 1024 rows a workgroup reads at a time."""
+    lib, gen = _lib.load(), torch.Generator().manual_seed(budget % 97)
+    L, B, H, cap, D = 3, 2, 4, 1300, 64
+    nseg = B * H
+    lens = torch.tensor([[0, 1, 255, 256, 257, 1023, 1024, 1025], [1300, 1300, 64, 65, 0, 0, 0, 0], [5, 900, 1281, 1279, 3, 1, 2, 700]], dtype=torch.int32)
+    lb = [(-torch.randint(1, 6, (nseg, cap), generator=gen) / 8.0).to(lb_dtype).to(DEV) for _ in range(L)]
+    pos = [torch.arange(cap, device=DEV).div(3, rounding_mode="floor").repeat(nseg, 1).contiguous() for _ in range(L)]
+    k = [torch.randn(nseg, cap, D, generator=gen).to(torch.bfloat16).to(DEV) for _ in range(L)]
+    ln = [lens[l].clone().to(DEV) for l in range(L)]
+    tables = [torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64, device=DEV) for ts in (lb, pos, k, ln)]
+    stream, code = _lib.current_stream(torch.device(DEV)), _lib.SCORE_ALPHA if strategy == "alpha" else _lib.SCORE_KNORM_ALPHA
+    results = []
+    for wide in (False, True):
+        out = [torch.full((L, B), -1, dtype=torch.int32, device=DEV) for _ in range(2)] + [torch.full((L, nseg), -1, dtype=torch.int32, device=DEV) for _ in range(3)]
+        args = (*(t.data_ptr() for t in tables), L, nseg, H, cap, D, _lib.BF16, _lib.dtype_code(lb_dtype), budget, 0, 0.0, cap + 5, code, _lib.ROUND_NATIVE,
+                *(t.data_ptr() for t in out))
+        if wide:
+            ws = torch.full((L * lib.trimkv_group_threshold_workspace(1, nseg, H),), 255, dtype=torch.uint8, device=DEV)
+            _lib.check(lib.trimkv_group_threshold_wide_each_layer(*args, ws.data_ptr(), ws.numel(), stream), "wide")
+        else:
+            _lib.check(lib.trimkv_group_threshold_each_layer(*args, stream), "single")
+        results.append([t.cpu() for t in out])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    want = lens.view(L, B, H).sum(-1).clamp(max=budget)
+    assert torch.equal(results[0][3].view(L, B, H).sum(-1).int(), want.int())

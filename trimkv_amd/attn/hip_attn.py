@@ -237,10 +237,12 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
                                      seg_start, cap, max_len, scale)
             out[:, :, :, a:a + g1] = part.view(B, Q, kv_heads, g1, D)
         return out.view(B, Q, Hq, D)
-    if query.stride(3) != 1 or any(s % 8 for s in query.stride()[:3]) or query.data_ptr() % 16:
+    sb, sh, st, sd = query.stride()
+    if sd != 1 or (sb | sh | st) % 8 or query.data_ptr() % 16:
         query = query.contiguous()
+        sb, sh, st, _ = query.stride()
     out = torch.empty(B, Q, Hq, D, dtype=query.dtype, device=query.device)
-    args = (query.data_ptr(), query.stride(0), query.stride(1), query.stride(2), out.data_ptr(),
+    args = (query.data_ptr(), sb, sh, st, out.data_ptr(),
             k_rows.data_ptr(), v_rows.data_ptr(), _lib.ptr(seg_len), _lib.ptr(seg_start),
             batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len)
     stream = _lib.current_stream(query.device)

@@ -101,6 +101,14 @@ def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -
             and not torch.cuda.is_current_stream_capturing())
 
 
+def wide_group(segs: int, longest: int) -> bool:
+    """Whether a budget that one layer's ``segs`` segments share is selected by a workgroup per segment (seven launches) instead of
+    one in all, which reads them one after the other, five times over.  Measured, one -> wide, layers x groups of 8 segments: 5 x 2
+    of 2400 rows 99 -> 36 us, of 600 64 -> 27, 36 x 8 of 2400 234 -> 101, 36 x 1 of 300 73 -> 27; below the line the launches cost a
+    caller that is not ahead of the device what they save."""
+    return segs * longest >= 8192
+
+
 class _Slab:
     """Device storage of one layer."""
 
@@ -394,9 +402,12 @@ class _SlabBacked(_CacheBase):
         arr = np.zeros(len(layers), dtype=self._LAYER_DT)
         for i, s in enumerate(slabs):
             arr[i] = (s.ptrs[0], s.ptrs[1], s.ptrs[2], s.ptrs[3], s.ptrs[4], 0, s.cap, 0)
-        tables = {"slabs": torch.from_numpy(arr.view(np.uint8)).to(dev)}
-        for name, idx in (("k", 0), ("lb", 2), ("pos", 3), ("len", 4)) + ((("cu", 5),) if slabs[0].cu is not None else ()):
-            tables[name] = torch.tensor([s.ptrs[idx] for s in slabs], dtype=torch.int64).to(dev)
+        names = (("k", 0), ("lb", 2), ("pos", 3), ("len", 4)) + ((("cu", 5),) if slabs[0].cu is not None else ())
+        words = np.concatenate([arr.view(np.int64)] + [np.array([s.ptrs[idx] for s in slabs], dtype=np.int64) for _, idx in names])
+        on_dev, n, at = torch.from_numpy(words).to(dev), len(layers), arr.nbytes // 8     # one copy: each waits for the device
+        tables = {"slabs": on_dev[:at].view(torch.uint8)}
+        for i, (name, _) in enumerate(names):
+            tables[name] = on_dev[at + i * n:at + (i + 1) * n]
         self._table_cache[key] = ([s.ptrs for s in slabs], [s.cap for s in slabs], tables)
         return tables
 
@@ -756,10 +767,12 @@ class TrimKVCache(_SlabBacked):
             return self._compress_on_device(strategy, memory_size, buffer_size, skip_layers, num_layers)
         self._budget_hint = memory_size + buffer_size
         todo = [l for l in range(skip_layers, num_layers) if memory_size + buffer_size <= self.get_cache_length(l)]
-        lost = min(512, max(1, max((self._slabs[l].max_len for l in todo), default=0) - memory_size))
-        first = self._slabs[todo[0]] if todo else None
-        # the usual case: every layer is due at the same step -> one launch
-        if len(todo) > 1 and self._layers_alike(todo) or len(todo) == 1 and split_evict(first.max_len, first.nseg * first.max_len, memory_size, lost, first.D):
+        layered = len(todo) > 1 and self._layers_alike(todo)   # the usual case: every layer is due at the same step -> one launch
+        if len(todo) == 1:
+            first = self._slabs[todo[0]]
+            layered = split_evict(first.max_len, first.nseg * first.max_len, memory_size, max(1, first.max_len - memory_size), first.D)
+        if layered:
+            lost = min(512, max(1, max(self._slabs[l].max_len for l in todo) - memory_size))
             self._evict_layers(todo, memory_size, None, 0, self._dense_strategy_code(strategy), _lib.ROUND_UPCAST,
                                self.sliding_window_size, [self.get_seq_length(l) + 1 for l in todo], spill=lost)
             for l in todo:
@@ -1164,12 +1177,15 @@ class _RaggedCache(_SlabBacked):
         tie_base = torch.empty(L, nseg, dtype=torch.int32, device=dev)
         new_len = torch.empty(L, nseg, dtype=torch.int32, device=dev)
         t = self._device_tables(layers)
-        rc = _lib.load().trimkv_group_threshold_each_layer(
-            t["lb"].data_ptr(), t["pos"].data_ptr(), t["k"].data_ptr(), t["len"].data_ptr(), L, nseg, segs_per_group, s0.cap, s0.D,
-            _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype), int(budget), 0, 0.0, self.get_seq_length() + 1,
-            self._strategy_code(strategy), _lib.ROUND_NATIVE, thr.data_ptr(), take.data_ptr(), tie_base.data_ptr(), new_len.data_ptr(), None,
-            _lib.current_stream(dev))
-        _lib.check(rc, "trimkv_group_threshold_each_layer")
+        lib, stream = _lib.load(), _lib.current_stream(dev)
+        args = (t["lb"].data_ptr(), t["pos"].data_ptr(), t["k"].data_ptr(), t["len"].data_ptr(), L, nseg, segs_per_group, s0.cap, s0.D,
+                _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype), int(budget), 0, 0.0, self.get_seq_length() + 1,
+                self._strategy_code(strategy), _lib.ROUND_NATIVE, thr.data_ptr(), take.data_ptr(), tie_base.data_ptr(), new_len.data_ptr(), None)
+        if wide_group(segs_per_group, max(s.max_len for s in slabs)):
+            ws = self._workspace(L * lib.trimkv_group_threshold_workspace(1, nseg, segs_per_group), dev)
+            _lib.check(lib.trimkv_group_threshold_wide_each_layer(*args, ws.data_ptr(), ws.numel(), stream), "trimkv_group_threshold_wide_each_layer")
+        else:
+            _lib.check(lib.trimkv_group_threshold_each_layer(*args, stream), "trimkv_group_threshold_each_layer")
         return thr, take, tie_base, new_len
 
     def _compact(self, layer: int, segs_per_group: int, thr, take, tie_base_l, strategy: str) -> None:

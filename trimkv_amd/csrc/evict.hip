@@ -73,10 +73,9 @@ __device__ __forceinline__ float knorm_terms_of_wave(const ScoreArgs& s, int bas
 
 // Order-preserving key of token i's score; n = segment length (for the sliding window); knorm = the token's log ||k||
 // (read only by the knorm strategy).
-__device__ __forceinline__ uint32_t score_key(const ScoreArgs& s, int i, int n, float knorm) {
+__device__ __forceinline__ uint32_t score_key(const ScoreArgs& s, int i, int n, float lb, int64_t pos, float knorm) {
     if (s.sliding_window > 0 && i >= n - s.sliding_window) return float_key(__builtin_inff());
-    const float lb = load_as_f32(s.lb, i, s.lb_dtype);
-    const float age = (float)(s.q_idx - s.pos[i]);  // int64 -> fp32, round to nearest even
+    const float age = (float)(s.q_idx - pos);  // int64 -> fp32, round to nearest even
     float sc;
     if (s.rounding == TRIMKV_ROUND_NATIVE && s.lb_dtype != TRIMKV_F32) {
         sc = round_to_dtype(__fmul_rn(round_to_dtype(age, s.lb_dtype), lb), s.lb_dtype);
@@ -89,14 +88,33 @@ __device__ __forceinline__ uint32_t score_key(const ScoreArgs& s, int i, int n, 
 }
 
 // f(i, key) for every token i of the segment that this thread owns (i = threadIdx.x, + THREADS, ...).  Whole wavefronts
-// walk the segment together (the loop bound is wave-uniform), because the knorm term is computed by the wavefront.
-template <int THREADS, class F>
+// walk the segment together (the loop bound is wave-uniform), because the knorm term is computed by the wavefront.  The loads of
+// U tokens are in flight at a time: one after the other they were most of a launch's time (1 where registers are short).
+template <int THREADS, int U, class F>
 __device__ __forceinline__ void for_each_key(const ScoreArgs& s, int n, F&& f) {
     const int lane = threadIdx.x & 63;
-    for (int base = (int)(threadIdx.x & ~63u); base < n; base += THREADS) {
-        const float knorm = s.strategy == TRIMKV_SCORE_KNORM_ALPHA ? knorm_terms_of_wave(s, base, n) : 0.0f;
-        const int i = base + lane;
-        if (i < n) f(i, score_key(s, i, n, knorm));
+    for (int base = (int)(threadIdx.x & ~63u); base < n; base += U * THREADS) {
+        float lb[U];
+        int64_t pos[U];
+        if (s.lb_dtype == TRIMKV_F32) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) lb[u] = ((const float*)s.lb)[min(base + u * THREADS + lane, n - 1)];
+        } else {
+            uint16_t raw[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) raw[u] = ((const uint16_t*)s.lb)[min(base + u * THREADS + lane, n - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u) lb[u] = s.lb_dtype == TRIMKV_BF16 ? __uint_as_float((uint32_t)raw[u] << 16) : f16_bits_to_f32(raw[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) pos[u] = s.pos[min(base + u * THREADS + lane, n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int from = base + u * THREADS, i = from + lane;
+            if (from >= n) break;
+            const float knorm = s.strategy == TRIMKV_SCORE_KNORM_ALPHA ? knorm_terms_of_wave(s, from, n) : 0.0f;
+            if (i < n) f(i, score_key(s, i, n, lb[u], pos[u], knorm));
+        }
     }
 }
 
@@ -483,7 +501,7 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
     ScoreArgs s;
     s.lb = lbseg; s.pos = posseg; s.k = kseg; s.lb_dtype = a.lb_dtype; s.kv_dtype = a.kv_dtype; s.row_bytes = a.row_bytes;
     s.strategy = a.strategy; s.rounding = a.rounding; s.sliding_window = a.sliding_window; s.q_idx = a.q_idx;
-    for_each_key<EV_THREADS>(s, n, [&](int i, uint32_t key) { keys[i] = key; });
+    for_each_key<EV_THREADS, 4>(s, n, [&](int i, uint32_t key) { keys[i] = key; });
     __syncthreads();
 
     uint32_t thr;
@@ -587,7 +605,7 @@ __global__ __launch_bounds__(GT_THREADS) void group_threshold_kernel(GroupArgs a
                     for (int s = 0; s < a.segs_per_group; ++s) {
                         const int n = max(0, min(a.seg_lens[l][seg0 + s], a.cap));
                         const ScoreArgs sa = group_segment(a, l, seg0 + s);
-                        for_each_key<GT_THREADS>(sa, n, [&](int, uint32_t key) {
+                        for_each_key<GT_THREADS, 1>(sa, n, [&](int, uint32_t key) {
                             if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1ull);
                         });
                     }
@@ -619,7 +637,7 @@ __global__ __launch_bounds__(GT_THREADS) void group_threshold_kernel(GroupArgs a
             const ScoreArgs sa = group_segment(a, l, seg0 + s);
             uint64_t cnt = 0;  // low 32 bits: greater, high 32 bits: equal
             uint32_t key0 = 0;  // thread 0 owns row 0
-            for_each_key<GT_THREADS>(sa, n, [&](int i, uint32_t key) {
+            for_each_key<GT_THREADS, 1>(sa, n, [&](int i, uint32_t key) {
                 cnt += (key > thr ? 1ull : 0ull) + (key == thr ? (1ull << 32) : 0ull);
                 if (i == 0) key0 = key;
             });
@@ -643,9 +661,9 @@ __global__ __launch_bounds__(GT_THREADS) void group_threshold_kernel(GroupArgs a
 // ---- the same selection spread over many workgroups (large groups: one sequence over all layers, ...) -----------
 // One workgroup per (layer, segment).  Four histogram launches (one per key byte, most significant first) add into a
 // per-group global histogram; every workgroup re-derives the digits chosen so far from the earlier histograms (a
-// 256-bin walk, cheap) before it bins its own segment.  A count launch then classifies every segment's tokens against
+// scan of 256 bins) before it bins its own segment.  A count launch then classifies every segment's tokens against
 // the cut, and a scan launch (one workgroup per group) turns the per-segment counts into new_len / tie_base in
-// (layer, segment) order.  Kernel boundaries are the only synchronisation.
+// (layer, segment) order.  Kernel boundaries are the only synchronisation.  per_layer: a group per layer, its cut at layer * groups + group.
 constexpr int GW_THREADS = 256;
 struct WideArgs {
     GroupArgs g;
@@ -653,74 +671,68 @@ struct WideArgs {
     uint32_t* cnt;    // [nlayers][nseg][3]: tokens above the cut, tokens equal to it, row 0 (bit 0: above, bit 1: equal)
 };
 
-// digit and remaining rank chosen in a pass, from that pass's 256-bin histogram (in LDS), largest bin first
-__device__ __forceinline__ void walk_bins(const uint32_t* h, uint64_t remaining, uint32_t& digit, uint64_t& left) {
-    uint64_t acc = 0;
-    int b = 255;
-    for (; b > 0; --b) {
-        if (acc + h[b] >= remaining) break;
-        acc += h[b];
-    }
-    digit = (uint32_t)b;
-    left = remaining - acc;
-}
-
-// prefix (digits of passes 0..npass-1) and remaining rank for group g; *total = tokens in the group.  All threads call.
-__device__ __forceinline__ void wide_prefix(const WideArgs& w, int g, int npass, uint32_t* lh, uint32_t* sh_digit,
-                                            unsigned long long* sh_left, uint32_t& prefix, uint64_t& remaining, uint64_t& total) {
+// Prefix (digits of passes 0..npass-1) and remaining rank for group g; *total = tokens in the group.  All threads call: thread t
+// looks at bin 255 - t, a scan walks the bins from the largest down (one thread alone took 8 us a pass for it).
+__device__ __forceinline__ void wide_prefix(const WideArgs& w, int g, int npass, unsigned long long* sh, uint32_t& prefix,
+                                            uint64_t& remaining, uint64_t& total) {
+    static_assert(GW_THREADS == 256, "a thread per bin");
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    uint32_t h[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) h[q] = q < npass ? w.hist[((int64_t)g * 4 + q) * 256 + 255 - t] : 0u;
     prefix = 0;
     remaining = (uint64_t)max((int64_t)0, w.g.budget);
     total = 0;
-    for (int q = 0; q < npass; ++q) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (q >= npass) break;
+        unsigned long long upto = h[q];                    // tokens in this bin and in the larger ones
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned long long o = __shfl_up(upto, d, 64);
+            if (lane >= d) upto += o;
+        }
+        if (lane == 63) sh[wave] = upto;
         __syncthreads();
-        lh[threadIdx.x] = w.hist[((int64_t)g * 4 + q) * 256 + threadIdx.x];
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (q == 0) {
-                uint64_t t = 0;
-                for (int b = 0; b < 256; ++b) t += lh[b];
-                sh_left[1] = t;
-            }
-            uint32_t d;
-            uint64_t left;
-            walk_bins(lh, remaining, d, left);
-            *sh_digit = d;
-            sh_left[0] = left;
+        for (int x = 0; x < wave; ++x) upto += sh[x];
+        if (q == 0) total = sh[0] + sh[1] + sh[2] + sh[3];
+        const unsigned long long before = upto - h[q];
+        // the first bin that reaches the rank (the smallest one if none does)
+        if ((t == 0 || before < remaining) && (t == 255 || upto >= remaining)) {
+            sh[4] = 255 - t;
+            sh[5] = remaining - before;
         }
         __syncthreads();
-        prefix |= *sh_digit << (24 - 8 * q);
-        remaining = sh_left[0];
-        if (q == 0) total = sh_left[1];
+        prefix |= (uint32_t)sh[4] << (24 - 8 * q);
+        remaining = sh[5];
     }
     __syncthreads();
 }
 
 __global__ __launch_bounds__(GW_THREADS) void group_hist_kernel(WideArgs w, int pass) {
     __shared__ uint32_t lh[256];
-    __shared__ uint32_t sh_digit;
-    __shared__ unsigned long long sh_left[2];
+    __shared__ unsigned long long sh[6];
     const GroupArgs& a = w.g;
     const int s = blockIdx.x, l = blockIdx.y, g = blockIdx.z;
-    const int seg = g * a.segs_per_group + s;
+    const int seg = g * a.segs_per_group + s, cut = a.per_layer ? l * (int)gridDim.z + g : g;
     uint32_t prefix;
     uint64_t remaining, total;
-    wide_prefix(w, g, pass, lh, &sh_digit, sh_left, prefix, remaining, total);
+    wide_prefix(w, cut, pass, sh, prefix, remaining, total);
     const int shift = 24 - 8 * pass;
     const uint32_t hi_mask = pass == 0 ? 0u : (0xffffffffu << (shift + 8));
     lh[threadIdx.x] = 0;
     __syncthreads();
     const int n = max(0, min(a.seg_lens[l][seg], a.cap));
     const ScoreArgs sa = group_segment(a, l, seg);
-    for_each_key<GW_THREADS>(sa, n, [&](int, uint32_t key) {
+    for_each_key<GW_THREADS, 4>(sa, n, [&](int, uint32_t key) {
         if ((key & hi_mask) == prefix) atomicAdd(&lh[(key >> shift) & 255u], 1u);
     });
     __syncthreads();
-    if (lh[threadIdx.x]) atomicAdd(&w.hist[((int64_t)g * 4 + pass) * 256 + threadIdx.x], lh[threadIdx.x]);
+    if (lh[threadIdx.x]) atomicAdd(&w.hist[((int64_t)cut * 4 + pass) * 256 + threadIdx.x], lh[threadIdx.x]);
 }
 
 // cut of group g: from the threshold, or from the four histograms (with the keep-all / keep-nothing cases)
-__device__ __forceinline__ void wide_cut(const WideArgs& w, int g, uint32_t* lh, uint32_t* sh_digit, unsigned long long* sh_left,
-                                         uint32_t& thr, int64_t& take) {
+__device__ __forceinline__ void wide_cut(const WideArgs& w, int g, unsigned long long* sh, uint32_t& thr, int64_t& take) {
     const GroupArgs& a = w.g;
     if (a.use_threshold) {
         thr = float_key(a.threshold_score);
@@ -729,7 +741,7 @@ __device__ __forceinline__ void wide_cut(const WideArgs& w, int g, uint32_t* lh,
     }
     uint32_t prefix;
     uint64_t remaining, total;
-    wide_prefix(w, g, 4, lh, sh_digit, sh_left, prefix, remaining, total);
+    wide_prefix(w, g, 4, sh, prefix, remaining, total);
     const uint64_t budget = (uint64_t)max((int64_t)0, a.budget);
     if (budget >= total) { thr = 0u; take = INT32_MAX; }
     else if (budget == 0) { thr = 0xffffffffu; take = 0; }
@@ -737,21 +749,19 @@ __device__ __forceinline__ void wide_cut(const WideArgs& w, int g, uint32_t* lh,
 }
 
 __global__ __launch_bounds__(GW_THREADS) void group_count_kernel(WideArgs w) {
-    __shared__ uint32_t lh[256];
-    __shared__ uint32_t sh_digit;
-    __shared__ unsigned long long sh_left[2];
+    __shared__ unsigned long long sh[6];
     __shared__ uint64_t red[GW_THREADS / 64];
     const GroupArgs& a = w.g;
     const int s = blockIdx.x, l = blockIdx.y, g = blockIdx.z;
-    const int seg = g * a.segs_per_group + s;
+    const int seg = g * a.segs_per_group + s, cut = a.per_layer ? l * (int)gridDim.z + g : g;
     uint32_t thr;
     int64_t take;
-    wide_cut(w, g, lh, &sh_digit, sh_left, thr, take);
+    wide_cut(w, cut, sh, thr, take);
     const int n = max(0, min(a.seg_lens[l][seg], a.cap));
     const ScoreArgs sa = group_segment(a, l, seg);
     uint64_t cnt = 0;  // low 32 bits: greater, high 32 bits: equal
     uint32_t row0 = 0;  // thread 0 owns row 0
-    for_each_key<GW_THREADS>(sa, n, [&](int i, uint32_t key) {
+    for_each_key<GW_THREADS, 4>(sa, n, [&](int i, uint32_t key) {
         cnt += (key > thr ? 1ull : 0ull) + (key == thr ? (1ull << 32) : 0ull);
         if (i == 0) row0 = (key > thr ? 1u : 0u) | (key == thr ? 2u : 0u);
     });
@@ -765,9 +775,9 @@ __global__ __launch_bounds__(GW_THREADS) void group_count_kernel(WideArgs w) {
         w.cnt[e] = (uint32_t)(t & 0xffffffffull);
         w.cnt[e + 1] = (uint32_t)(t >> 32);
         w.cnt[e + 2] = row0;
-        if (s == 0 && l == 0) {
-            a.thr_key[g] = thr;
-            a.tie_take[g] = (int32_t)min(take, (int64_t)INT32_MAX);
+        if (s == 0 && (l == 0 || a.per_layer)) {
+            a.thr_key[cut] = thr;
+            a.tie_take[cut] = (int32_t)min(take, (int64_t)INT32_MAX);
         }
     }
 }
@@ -778,9 +788,9 @@ __global__ __launch_bounds__(GW_THREADS) void group_scan_kernel(WideArgs w) {
     uint32_t row0 = 0;
     __shared__ long long carry;
     const GroupArgs& a = w.g;
-    const int g = blockIdx.x;
-    const int64_t take = a.tie_take[g];   // written by the count launch
-    const int entries = a.nlayers * a.segs_per_group;   // (layer, segment) pairs of the group, in tie order
+    const int g = blockIdx.x, l0 = blockIdx.y;          // one budget per (layer, group): blockIdx.y = layer
+    const int64_t take = a.tie_take[l0 * (int)gridDim.x + g];   // written by the count launch
+    const int entries = (a.per_layer ? 1 : a.nlayers) * a.segs_per_group;   // (layer, segment) pairs of the group, in tie order
     if (threadIdx.x == 0) carry = 0;
     for (int e0 = 0; e0 < entries; e0 += GW_THREADS) {
         __syncthreads();
@@ -788,7 +798,7 @@ __global__ __launch_bounds__(GW_THREADS) void group_scan_kernel(WideArgs w) {
         int64_t idx = 0;
         if (e < entries) {
             const int l = e / a.segs_per_group, s = e - l * a.segs_per_group;
-            idx = (int64_t)l * a.nseg + g * a.segs_per_group + s;
+            idx = (int64_t)(l0 + l) * a.nseg + g * a.segs_per_group + s;
             gt_l[threadIdx.x] = w.cnt[idx * 3];
             eq_l[threadIdx.x] = w.cnt[idx * 3 + 1];
             row0 = w.cnt[idx * 3 + 2];
@@ -1146,14 +1156,13 @@ extern "C" size_t trimkv_group_threshold_workspace(int nlayers, int nseg, int se
     return ((size_t)(nseg / segs_per_group) * 4 * 256 + (size_t)nlayers * nseg * 3) * sizeof(uint32_t);
 }
 
-extern "C" int trimkv_group_threshold_wide(const void* const* lb_slabs, const int64_t* const* pos_slabs,
-                                           const void* const* k_slabs, const int32_t* const* seg_lens,
-                                           int nlayers, int nseg, int segs_per_group, int cap, int head_dim,
-                                           int kv_dtype, int lb_dtype, int64_t budget, int use_threshold, float threshold_score,
-                                           int64_t q_idx, int strategy, int rounding,
-                                           uint32_t* thr_key, int32_t* tie_take, int32_t* tie_base, int32_t* new_len, int32_t* first_kept,
-                                           void* workspace, size_t workspace_bytes, void* stream) {
-    const char* fn = "trimkv_group_threshold_wide";
+static int group_threshold_wide_common(const char* fn, int per_layer, const void* const* lb_slabs, const int64_t* const* pos_slabs,
+                                       const void* const* k_slabs, const int32_t* const* seg_lens,
+                                       int nlayers, int nseg, int segs_per_group, int cap, int head_dim,
+                                       int kv_dtype, int lb_dtype, int64_t budget, int use_threshold, float threshold_score,
+                                       int64_t q_idx, int strategy, int rounding,
+                                       uint32_t* thr_key, int32_t* tie_take, int32_t* tie_base, int32_t* new_len, int32_t* first_kept,
+                                       void* stream, void* workspace, size_t workspace_bytes) {
     if (!lb_slabs || !pos_slabs || !seg_lens || !thr_key || !tie_take || !tie_base || !new_len) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (strategy == TRIMKV_SCORE_KNORM_ALPHA && !k_slabs) return fail(TRIMKV_ERR_NULL, "%s: knorm_alpha needs k_slabs", fn);
     if (strategy != TRIMKV_SCORE_ALPHA && strategy != TRIMKV_SCORE_KNORM_ALPHA) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: unknown strategy %d", fn, strategy);
@@ -1165,7 +1174,8 @@ extern "C" int trimkv_group_threshold_wide(const void* const* lb_slabs, const in
         return fail(TRIMKV_ERR_UNSUPPORTED, "%s: knorm_alpha needs head_dim to be a multiple of 8, at most 512 (got %d)", fn, head_dim);
     const int ngroups = nseg / segs_per_group;
     if (nlayers > 65535 || ngroups > 65535) return fail(TRIMKV_ERR_SHAPE, "%s: nlayers=%d or groups=%d exceeds the grid limit 65535", fn, nlayers, ngroups);
-    const size_t need = trimkv_group_threshold_workspace(nlayers, nseg, segs_per_group);
+    const int cuts = per_layer ? nlayers * ngroups : ngroups;
+    const size_t need = ((size_t)cuts * 4 * 256 + (size_t)nlayers * nseg * 3) * sizeof(uint32_t);
     if (!workspace || workspace_bytes < need) return fail(TRIMKV_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, got %zu", fn, need, workspace_bytes);
     if ((uintptr_t)workspace & 3) return fail(TRIMKV_ERR_SHAPE, "%s: workspace must be 4-byte aligned", fn);
     WideArgs w;
@@ -1174,19 +1184,33 @@ extern "C" int trimkv_group_threshold_wide(const void* const* lb_slabs, const in
     a.nlayers = nlayers; a.nseg = nseg; a.segs_per_group = segs_per_group; a.cap = cap; a.row_bytes = head_dim * 2;
     a.kv_dtype = kv_dtype; a.lb_dtype = lb_dtype; a.budget = budget; a.use_threshold = use_threshold; a.threshold_score = threshold_score;
     a.q_idx = q_idx; a.strategy = strategy; a.rounding = rounding;
-    a.thr_key = thr_key; a.tie_take = tie_take; a.tie_base = tie_base; a.new_len = new_len; a.first_kept = first_kept; a.per_layer = 0;
+    a.thr_key = thr_key; a.tie_take = tie_take; a.tie_base = tie_base; a.new_len = new_len; a.first_kept = first_kept; a.per_layer = per_layer;
     w.hist = (uint32_t*)workspace;
-    w.cnt = w.hist + (size_t)ngroups * 4 * 256;
+    w.cnt = w.hist + (size_t)cuts * 4 * 256;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid(segs_per_group, nlayers, ngroups);
     if (!use_threshold) {
-        const int64_t nh = (int64_t)ngroups * 4 * 256;
+        const int64_t nh = (int64_t)cuts * 4 * 256;
         hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, w.hist, nh, 0u);
         for (int pass = 0; pass < 4; ++pass) hipLaunchKernelGGL(group_hist_kernel, grid, dim3(GW_THREADS), 0, st, w, pass);
     }
     hipLaunchKernelGGL(group_count_kernel, grid, dim3(GW_THREADS), 0, st, w);
-    hipLaunchKernelGGL(group_scan_kernel, dim3(ngroups), dim3(GW_THREADS), 0, st, w);
+    hipLaunchKernelGGL(group_scan_kernel, dim3(ngroups, per_layer ? nlayers : 1), dim3(GW_THREADS), 0, st, w);
     return launch_status(fn);
+}
+
+#define TRIMKV_GROUP_WIDE_PARAMS const void* const* lb_slabs, const int64_t* const* pos_slabs, const void* const* k_slabs, \
+    const int32_t* const* seg_lens, int nlayers, int nseg, int segs_per_group, int cap, int head_dim, int kv_dtype, int lb_dtype, \
+    int64_t budget, int use_threshold, float threshold_score, int64_t q_idx, int strategy, int rounding, \
+    uint32_t* thr_key, int32_t* tie_take, int32_t* tie_base, int32_t* new_len, int32_t* first_kept, \
+    void* workspace, size_t workspace_bytes, void* stream
+
+extern "C" int trimkv_group_threshold_wide(TRIMKV_GROUP_WIDE_PARAMS) {
+    return group_threshold_wide_common("trimkv_group_threshold_wide", 0, TRIMKV_GROUP_ARGS, workspace, workspace_bytes);
+}
+
+extern "C" int trimkv_group_threshold_wide_each_layer(TRIMKV_GROUP_WIDE_PARAMS) {
+    return group_threshold_wide_common("trimkv_group_threshold_wide_each_layer", 1, TRIMKV_GROUP_ARGS, workspace, workspace_bytes);
 }
 
 extern "C" int trimkv_build_cu_seqlens(const int32_t* seg_len, int nseg, int32_t* cu_seqlens, void* stream) {
