@@ -239,7 +239,7 @@ def timed_checked_eviction(cache, c, layers_to_check):
         ties += int(tie.sum())
         mismatches += int((~same & ~tie).sum())
     return ms, {"evicted_layers_checked": list(snaps), "evicted_segments_checked": checked, "retained_index_mismatches": mismatches,
-                "boundary_tie_rows": ties, "launch": "all layers in one trimkv_evict_layers launch"}
+                "boundary_tie_rows": ties, "launch": "all layers in one launch"}
 
 
 def prefill_main(args):
