@@ -183,6 +183,6 @@ def test_argument_blocks_and_split_evictions_refuse_what_the_plain_entry_points_
     assert divided(nbytes=need - 1) == divided(ws=None) == divided(ws=one + 8) < 0
     assert divided(tiles=0) == divided(n=0) == -2 and divided(D=80) < 0
     rule = lambda batch, heads, group, q_len, n, uneven=0: lib.trimkv_prefill_split_tiles(batch, heads, group, q_len, n, uneven)
-    assert rule(1, 8, 2, 63, 65536) == 0 and rule(4, 64, 1, 256, 8192) == 0     # short chunks; as many query tiles as CUs
+    assert rule(64, 8, 2, 63, 65536) == 0 and rule(4, 64, 1, 256, 8192) == 0    # as many query tiles as CUs
     assert rule(1, 8, 4, 512, 4096) == 16 and rule(1, 8, 4, 1280, 8192) == 0 and rule(1, 8, 4, 1280, 8192, 1) == 43
     assert all(rule(1, 8, 4, 64 * q, n) * 32 >= (n + 63) // 64 or rule(1, 8, 4, 64 * q, n) == 0 for q in range(1, 40) for n in (64, 1000, 50000))

@@ -15,6 +15,10 @@ pytestmark = pytest.mark.gpu
     (3, 96, torch.float16, 64, [64, 65, 127, 640], (1, 3)),                # the shortest chunk; padded rows of a query tile
     (5, 64, torch.bfloat16, 130, [191, 192, 193, 1500], (2, 8)),           # lengths around a tile of 64 keys
     (8, 128, torch.bfloat16, 77, [2000, 77, 1999, 400], (5, 32)),
+    (1, 128, torch.bfloat16, 63, [63, 1025, 0, 30], (1, 3, 17)),           # short chunks
+    (2, 96, torch.float16, 33, [64, 129, 500, 700], (1, 5)),
+    (3, 64, torch.bfloat16, 2, [1, 64, 65, 900], (1, 2)),
+    (8, 128, torch.bfloat16, 17, [800, 17, 16, 400], (4, 13)),
 ])
 def test_divided_keys_match_the_whole_and_the_oracle(G, D, dtype, Q, lens, shares_of):
     """The two kernels round P to 16 bits against different references: u Sum p |v| on either side, the row sums the same
@@ -53,7 +57,7 @@ def test_divided_keys_match_the_whole_and_the_oracle(G, D, dtype, Q, lens, share
         assert ok, (tiles, err)
 
 
-@pytest.mark.parametrize("B,H,G,Q,n", [(1, 2, 4, 300, 3000), (1, 1, 2, 128, 8200), (2, 8, 2, 640, 2100)])
+@pytest.mark.parametrize("B,H,G,Q,n", [(1, 2, 4, 300, 3000), (1, 1, 2, 128, 8200), (2, 8, 2, 640, 2100), (1, 8, 4, 50, 3000)])
 def test_the_rule_divides_few_query_tiles_and_the_public_call_follows_it(B, H, G, Q, n):
     from trimkv_amd import _lib
     from trimkv_amd.attn.hip_attn import prefill_attention

@@ -95,7 +95,8 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, b);
 }
 
-template <int G, bool F16>
+// SPLIT: blockIdx.z takes split_tiles * 64 keys (see prefill_attn_kernel); the unfinished rows lie one behind the other, 128 floats each
+template <int G, bool F16, bool SPLIT>
 __global__ __launch_bounds__(SmallCfg<G>::THREADS) void prefill_small_kernel(PrefillArgs a) {
     using C = SmallCfg<G>;
     __shared__ __attribute__((aligned(16))) char lds_k[PF_BN * PF_ROW];
@@ -134,7 +135,10 @@ __global__ __launch_bounds__(SmallCfg<G>::THREADS) void prefill_small_kernel(Pre
 
     // keys the workgroup has to visit: everything its last query may see
     const int t_last = min(Q - 1, t_wg0 + C::BT - 1);
-    const int k_end = max(0, min(n, n - Q + t_last + 1));
+    const int all_keys = max(0, min(n, n - Q + t_last + 1));
+    const int k_first = SPLIT ? (int)blockIdx.z * a.split_tiles * 64 : 0;
+    if (SPLIT && k_first > 0 && k_first >= all_keys) return;
+    const int k_end = SPLIT ? min(all_keys, k_first + a.split_tiles * 64) : all_keys;
     const int vis_j = n - Q + t_q;              // last key visible to this lane's query
     const int vis_wave_max = n - Q + min(Q - 1, t_wg0 + tt * 16 + 15);
 
@@ -163,8 +167,8 @@ __global__ __launch_bounds__(SmallCfg<G>::THREADS) void prefill_small_kernel(Pre
         }
     };
 
-    if (k_end > 0) fetch(0);
-    for (int kbase = 0; kbase < k_end; kbase += PF_BN) {
+    if (k_end > k_first) fetch(k_first);
+    for (int kbase = k_first; kbase < k_end; kbase += PF_BN) {
         __syncthreads();   // everyone is done reading the previous tile
         publish();
         __syncthreads();   // the tile is visible
@@ -245,6 +249,16 @@ __global__ __launch_bounds__(SmallCfg<G>::THREADS) void prefill_small_kernel(Pre
     // the four row groups of a query hold disjoint keys: add their sums, then normalise and store
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
+    if (SPLIT && all_keys > a.split_tiles * 64) {
+        const int64_t row = ((((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile) * C::WAVES + w) * 16 + j;
+        if (ig == 0) *(float2*)(a.part_ml + row * 2) = make_float2(m_run, l_run);
+        float* po = a.part + row * PF_D + 8 * ig;
+#pragma unroll
+        for (int pb = 0; pb < 4; ++pb)
+#pragma unroll
+            for (int v = 0; v < 4; v += 2) *(float4*)(po + pb * 32 + 2 * v) = make_float4(oe[pb][v], oo[pb][v], oe[pb][v + 1], oo[pb][v + 1]);
+        return;
+    }
     if (q_ok) {
         const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
         uint32_t* orow = (uint32_t*)(a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + (h * G + g)) * a.hd);
@@ -257,6 +271,43 @@ __global__ __launch_bounds__(SmallCfg<G>::THREADS) void prefill_small_kernel(Pre
     }
 }
 
+
+// The shares of the keys put together: a workgroup per wavefront of prefill_small_kernel (16 rows), 8 features per thread.  A share
+// that a row saw nothing of has sum 0 and is left out.
+template <int G, bool F16>
+__global__ __launch_bounds__(256) void prefill_small_merge_kernel(PrefillArgs a) {
+    using C = SmallCfg<G>;
+    const int seg = blockIdx.y, tile = (int)blockIdx.x / C::WAVES, w = (int)blockIdx.x % C::WAVES, tiles = (int)gridDim.x / C::WAVES;
+    const int b = seg / a.kv_heads, h = seg - b * a.kv_heads, Q = a.q_len;
+    int n = a.seg_len ? a.seg_len[seg] : a.max_len;
+    n = max(0, min(n, a.max_len));
+    const int all_keys = max(0, min(n, n - Q + min(Q - 1, tile * C::BT + C::BT - 1) + 1));
+    const int share = a.split_tiles * 64, shares = (all_keys + share - 1) / share;
+    if (shares <= 1) return;                     // one share: its workgroup wrote the result
+    const int j = threadIdx.x >> 4, d = (threadIdx.x & 15) * 8, t_q = tile * C::BT + w / G * 16 + j;
+    if (t_q >= Q || d >= a.hd) return;
+    const int64_t row = (((int64_t)seg * tiles + tile) * C::WAVES + w) * 16 + j, per_share = (int64_t)gridDim.y * gridDim.x * 16;
+    float m = -3.0e38f;
+    for (int z = 0; z < shares; ++z) {
+        const float2 x = *(const float2*)(a.part_ml + (row + z * per_share) * 2);
+        if ((__float_as_uint(x.y) << 1) != 0) m = __builtin_fmaxf(m, x.x);
+    }
+    float l = 0.0f, o[8] = {};
+#pragma unroll 4
+    for (int z = 0; z < shares; ++z) {
+        const float2 x = *(const float2*)(a.part_ml + (row + z * per_share) * 2);
+        const float* po = a.part + (row + z * per_share) * PF_D + d;
+        const float4 lo = *(const float4*)po, hi = *(const float4*)(po + 4);
+        const float f = (__float_as_uint(x.y) << 1) != 0 ? __builtin_amdgcn_exp2f(x.x - m) : 0.0f;
+        l += x.y * f;
+        o[0] += lo.x * f; o[1] += lo.y * f; o[2] += lo.z * f; o[3] += lo.w * f;
+        o[4] += hi.x * f; o[5] += hi.y * f; o[6] += hi.z * f; o[7] += hi.w * f;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    uint16_t* out = a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + h * G + w % G) * a.hd + d;
+    *(uint4*)out = make_uint4(pack_kv<F16>(o[0] * inv, o[1] * inv), pack_kv<F16>(o[2] * inv, o[3] * inv),
+                              pack_kv<F16>(o[4] * inv, o[5] * inv), pack_kv<F16>(o[6] * inv, o[7] * inv));
+}
 
 // ---------------------------------------------------------------------------------------------
 // Large-chunk kernel: 32 queries per wavefront, 64-key tiles, v_mfma_f32_32x32x16_bf16.
@@ -698,7 +749,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     }
 }
 
-constexpr int PF2_PART = PF2_WAVES * 32 * (PF_D + 2) * 4;   // bytes that one workgroup leaves for the merge
+constexpr int PF_PART_ROW = (PF_D + 2) * 4;   // bytes that a row of a workgroup leaves for the merge
 
 // > 64 KB of dynamic LDS needs the attribute once per device (the flag is only ever set, so a race repeats the call at worst)
 template <bool F16, bool SPLIT>
@@ -714,8 +765,35 @@ static int opt_in_lds() {
     return 0;
 }
 
+// query tiles of a chunk and rows of each
+static void query_tiles(int group, int q_len, int64_t* tiles, int64_t* rows) {
+    const int tt = group >= 3 ? 1 : 4 / group;               // SmallCfg
+    const int bt = q_len < 64 ? 16 * tt : (PF2_WAVES * 32) / group;
+    *tiles = (q_len + bt - 1) / bt;
+    *rows = q_len < 64 ? group * tt * 16 : PF2_WAVES * 32;
+}
+
 template <bool F16>
 static int launch_prefill_split(const PrefillArgs& a, int nseg, hipStream_t st) {
+    if (a.q_len < 64) {
+        auto go = [&](auto g) {
+            using C = SmallCfg<decltype(g)::value>;
+            const int tiles = (a.q_len + C::BT - 1) / C::BT, share = a.split_tiles * 64;
+            hipLaunchKernelGGL((prefill_small_kernel<decltype(g)::value, F16, true>), dim3(tiles, nseg, (a.max_len + share - 1) / share), dim3(C::THREADS), 0, st, a);
+            hipLaunchKernelGGL((prefill_small_merge_kernel<decltype(g)::value, F16>), dim3(tiles * C::WAVES, nseg), dim3(256), 0, st, a);
+        };
+        switch (a.group) {
+            case 1: go(std::integral_constant<int, 1>{}); break;
+            case 2: go(std::integral_constant<int, 2>{}); break;
+            case 3: go(std::integral_constant<int, 3>{}); break;
+            case 4: go(std::integral_constant<int, 4>{}); break;
+            case 5: go(std::integral_constant<int, 5>{}); break;
+            case 6: go(std::integral_constant<int, 6>{}); break;
+            case 7: go(std::integral_constant<int, 7>{}); break;
+            default: go(std::integral_constant<int, 8>{}); break;
+        }
+        return 0;
+    }
     if (int rc = opt_in_lds<F16, true>()) return rc;
     const int bt = (PF2_WAVES * 32) / a.group, tiles = (a.q_len + bt - 1) / bt;
     const int key_tiles = (a.max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + a.split_tiles - 1) / a.split_tiles;
@@ -730,7 +808,7 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
     if (a.q_len < 64) {
         using C = SmallCfg<G>;
         const int tiles = (a.q_len + C::BT - 1) / C::BT;
-        hipLaunchKernelGGL((prefill_small_kernel<G, F16>), dim3(tiles, nseg), dim3(C::THREADS), 0, st, a);
+        hipLaunchKernelGGL((prefill_small_kernel<G, F16, false>), dim3(tiles, nseg), dim3(C::THREADS), 0, st, a);
         return 0;
     }
     if (int rc = opt_in_lds<F16, false>()) return rc;
@@ -803,9 +881,24 @@ extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_
 // of unlike segments the longest one holds up the rest, and three shares let the others' CUs help: 168 .. 224 tiles, lengths
 // uniform up to 4096 keys 80 -> 74 .. 85 -> 83, to 10000 keys 188 -> 166 .. 197 -> 170; up to 3000 keys 63 -> 70, hence the line.
 extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
-    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len < 64 || max_len <= 0) return 0;
-    const int64_t bt = (PF2_WAVES * 32) / group, items = (q_len + bt - 1) / bt * batch * kv_heads;
+    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0) return 0;
+    int64_t tiles, rows;
+    query_tiles(group, q_len, &tiles, &rows);
+    const int64_t items = tiles * batch * kv_heads;
     const int64_t key_tiles = ((int64_t)max_len + PF2_BN - 1) / PF2_BN;
+    if (q_len < 64) {
+        // Short chunks: a workgroup walks 64 keys in 2.2 us, two or more fit on a CU.  Whole -> split, us: 8 query tiles of 2048 keys
+        // 72 -> 19, of 8192 278 -> 32; 32 of 2048 72 -> 20, of 8192 281 -> 40; 128 of 2048 73 -> 34, of 8192 281 -> 104; left whole:
+        // 512 keys (20 -> 13 for a second launch), 512 query tiles (2048 keys 99 -> 109).
+        float best = 2.2f * (float)key_tiles - 8.0f;
+        int64_t take = 0;
+        for (int64_t s = 2; s <= 32 && items * s <= 512; ++s) {
+            const int64_t each = (key_tiles + s - 1) / s;
+            const float us = 2.2f * (float)each + 3.0f + (0.8f + 0.02f * (float)items) * (float)s;
+            if (us < best) { best = us; take = each; }
+        }
+        return (int)take;
+    }
     if (items >= 256) return 0;
     if (items > 128) return uneven && key_tiles >= 64 ? (int)((key_tiles + 2) / 3) : 0;
     float best = 1.15f * (float)key_tiles - 8.0f;   // below that the second launch costs a caller whose queue runs dry as much
@@ -820,9 +913,10 @@ extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, in
 
 extern "C" int64_t trimkv_prefill_split_workspace(int batch, int kv_heads, int group, int q_len, int max_len, int split_tiles) {
     if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0 || split_tiles <= 0) return 0;
-    const int64_t bt = (PF2_WAVES * 32) / group, tiles = (q_len + bt - 1) / bt;
+    int64_t tiles, rows;
+    query_tiles(group, q_len, &tiles, &rows);
     const int64_t key_tiles = ((int64_t)max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + split_tiles - 1) / split_tiles;
-    return tiles * batch * kv_heads * shares * PF2_PART;
+    return tiles * batch * kv_heads * shares * rows * PF_PART_ROW;
 }
 
 extern "C" int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
@@ -841,7 +935,7 @@ extern "C" int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int6
         return fail(TRIMKV_ERR_CAPACITY, "%s: needs a 16-byte aligned workspace of %lld bytes (got %lld)", fn, (long long)need, (long long)workspace_bytes);
     a.split_tiles = split_tiles;
     a.part = (float*)workspace;
-    a.part_ml = (float*)workspace + need / PF2_PART * (PF2_WAVES * 32 * PF_D);
+    a.part_ml = (float*)workspace + need / PF_PART_ROW * PF_D;
     hipStream_t st = (hipStream_t)stream;
     const int rc = dtype == TRIMKV_F16 ? launch_prefill_split<true>(a, batch * kv_heads, st) : launch_prefill_split<false>(a, batch * kv_heads, st);
     if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
