@@ -320,6 +320,21 @@ int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers, int nseg, 
                        const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * trimkv_evict_split_rooms -- trimkv_evict_split with scratch for the rows that the pairs keep instead of max_len rows each, in
+ * chunks of 512 kept rows: most_chunks (up to 64) for every pair or, with first_chunk (device, [pairs + 1]), the chunks
+ * first_chunk[i] .. first_chunk[i + 1] - 1 of total_chunks for pair i, most_chunks of them at most.  A segment that keeps more rows
+ * than its chunks hold is moved by one workgroup.  on_host: the table of up to 48 layers is in host memory, as in
+ * trimkv_evict_host_layers.  workspace: trimkv_evict_split_rooms_workspace(pairs, total_chunks, ...) bytes, 16-byte aligned;
+ * without first_chunk total_chunks = pairs * most_chunks.
+ */
+size_t trimkv_evict_split_rooms_workspace(int npairs, int total_chunks, int head_dim, int spill);
+int trimkv_evict_split_rooms(const trimkv_layer_slabs* layers, int on_host, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                             int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                             int strategy, int rounding, int sliding_window, int max_len, int spill,
+                             const int32_t* work, int nwork, const int32_t* first_chunk, int total_chunks, int most_chunks,
+                             void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * trimkv_evict_host_layers -- trimkv_evict_layers (spill = 0) or trimkv_evict_split (spill > 0) over up to 48 layers whose table
  * is in HOST memory: it travels in the launches' arguments, so that slabs which have just moved need no upload.  Read before the
  * call returns.  Other arguments, workspace and results as there.

@@ -186,3 +186,19 @@ def test_argument_blocks_and_split_evictions_refuse_what_the_plain_entry_points_
     assert rule(64, 8, 2, 63, 65536) == 0 and rule(4, 64, 1, 256, 8192) == 0    # as many query tiles as CUs
     assert rule(1, 8, 4, 512, 4096) == 16 and rule(1, 8, 4, 1280, 8192) == 0 and rule(1, 8, 4, 1280, 8192, 1) == 43
     assert all(rule(1, 8, 4, 64 * q, n) * 32 >= (n + 63) // 64 or rule(1, 8, 4, 64 * q, n) == 0 for q in range(1, 40) for n in (64, 1000, 50000))
+
+
+def test_split_evictions_with_room_for_what_is_kept():
+    """The scratch counts chunks of 512 kept rows; what the call cannot carry out is refused before any launch."""
+    lib, one = _lib.load(), 256
+    per_chunk = 512 * 4 + 128 * (2 * 256 + 12)
+    need = lib.trimkv_evict_split_rooms_workspace(8, 20, 128, 128)
+    assert 20 * per_chunk <= need <= 20 * per_chunk + 8 * 16 + 256
+    assert lib.trimkv_evict_split_rooms_workspace(8, 0, 128, 128) == lib.trimkv_evict_split_rooms_workspace(0, 8, 128, 128) == 0
+    call = lambda nwork=8, work=one, first=one, total=20, most=8, D=128, max_len=4096, spill=128, ws=one, nbytes=1 << 30, on_host=0, at=one, nl=2: lib.trimkv_evict_split_rooms(
+        at, on_host, nl, 4, D, _lib.BF16, _lib.F32, 8, None, 0, 0, 100, 0, 0, 0, max_len, spill, work, nwork, first, total, most, ws, nbytes, None)
+    assert call(nwork=0) == 0
+    assert call(most=0) == call(most=65) == call(most=21) == call(nwork=-1) == call(spill=0) == call(nl=0) == -2
+    assert call(nbytes=need - 1) == call(ws=None) == call(ws=one + 8) < 0
+    assert call(work=None, nwork=0, first=None, total=0, nbytes=lib.trimkv_evict_split_rooms_workspace(8, 64, 128, 128) - 1) < 0
+    assert call(D=80) == call(max_len=32769) < 0 and call(at=None, on_host=1) < 0 and call(on_host=1, nl=49) == -2

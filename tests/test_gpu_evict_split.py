@@ -133,3 +133,86 @@ def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(bud
         assert torch.equal(a, b)
     want = lens.view(L, B, H).sum(-1).clamp(max=budget)
     assert torch.equal(results[0][3].view(L, B, H).sum(-1).int(), want.int())
+
+
+def _uneven(split, monkeypatch):
+    """192 segments with lognormal budgets of 1 to 7600 rows, filled, cut, and 700 tokens later due again."""
+    monkeypatch.setattr(cache_utils, "split_evict", lambda *a: False)
+    L, B, H, n = 6, 4, 8, 7600
+    budgets = np.exp(np.random.default_rng(3).normal(np.log(800.0), 1.0, (L, B * H))).clip(1, n).astype(np.int64)
+    budgets[0, 0] = n
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    cache, seen = BatchedDynamicBudgetTrimKVCache(), 0
+    for more in (n + 1, 700):
+        for l in range(L):
+            k, v = (torch.randn(B, H, more, 128, generator=gen, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+            lb = -torch.rand(B, H, more, generator=gen, device=DEV) - 0.01
+            cache.update(k, v, lb, torch.arange(seen, seen + more, device=DEV), l)
+        seen += more
+        cache.set_budgets(budgets)
+        if more == 700:
+            monkeypatch.setattr(cache_utils, "split_evict", lambda *a: split)
+            del k, v, lb
+            torch.cuda.synchronize()
+            before = torch.cuda.memory_allocated()
+            torch.cuda.reset_peak_memory_stats()
+        cache.evict_to_budgets(buffer_size=0)
+    torch.cuda.synchronize()
+    peak, after = torch.cuda.max_memory_allocated() - before, torch.cuda.memory_allocated() - before
+    held = [tuple(t.cpu() for t in (s.seg_len, s.cu)) + tuple(torch.cat([t[i, :int(m)] for i, m in enumerate(s.lens)]).cpu() for t in (s.k, s.v, s.lb, s.pos))
+            for s in cache._slabs]
+    assert all((s.lens == budgets[l]).all() for l, s in enumerate(cache._slabs))
+    return held, peak, after, cache.memory_bytes()
+
+
+def test_scratch_is_sized_by_what_the_due_segments_keep_and_given_back(monkeypatch):
+    """Segments of unlike budgets: the scratch follows the rows that they keep, not the longest of them times their number, and
+    nothing but work lists (a few KB) outlives the launches."""
+    want, _, _, _ = _uneven(False, monkeypatch)
+    got, peak, after, cache_bytes = _uneven(True, monkeypatch)
+    for a, b in zip(want, got):
+        assert all(torch.equal(x, y) for x, y in zip(a, b))
+    assert 1 << 20 < peak < cache_bytes / 6, (peak, cache_bytes)
+    assert after < 1 << 20
+
+
+@pytest.mark.parametrize("how", ["limit", "out of memory"])
+def test_without_room_for_scratch_a_workgroup_moves_each_segment(how, monkeypatch, always_split):
+    n, M = 4224, 4096
+    keep = np.sort(np.random.default_rng(2).choice(n, size=M, replace=False))
+    cache, held = _filled(TrimKVCache, 2, 1, 3, n, 128, torch.bfloat16, torch.float32, keep)
+    if how == "limit":
+        monkeypatch.setattr(cache_utils, "SPLIT_SCRATCH", 1 << 20)
+    else:
+        empty, refused = torch.empty, []
+
+        def short(*a, **kw):
+            if kw.get("dtype") == torch.uint8:
+                refused.append(a)
+                raise torch.OutOfMemoryError("no memory")
+            return empty(*a, **kw)
+        monkeypatch.setattr(torch, "empty", short)
+    cache.compress("alpha", memory_size=M, buffer_size=n - M)
+    monkeypatch.undo()
+    assert how == "limit" or refused
+    _check(cache, held, keep, how)
+
+
+@pytest.mark.parametrize("on_host", [0, 1])
+def test_pairs_with_chunks_of_their_own(on_host):
+    """A pair with just enough chunks, one with one too few, one with none, and lists that name chunks past the workspace's: those
+    that do not fit are moved by one workgroup, nothing is written behind the workspace."""
+    lib, n, M = _lib.load(), 3300, 3100                       # seven chunks of 512 kept rows
+    keep = np.sort(np.random.default_rng(6).choice(n, size=M, replace=False))
+    for first in ([0, 7, 13, 13, 20], [0, 0, 7, 21, 28], [-1, 7, 14, 20, 27], [0, 7, 14, 10 ** 9, 10 ** 9 + 7]):
+        cache, held = _filled(TrimKVCache, 2, 1, 2, n, 128, torch.bfloat16, torch.float32, keep)
+        total = 28
+        need = lib.trimkv_evict_split_rooms_workspace(4, total, 128, 200)
+        ws = torch.full((need + 4096,), 9, dtype=torch.uint8, device=DEV)
+        lists = torch.tensor([3, 0, 2, 1] + first, dtype=torch.int32, device=DEV)
+        table = cache._host_table([0, 1])
+        at = table.ctypes.data if on_host else cache._device_tables([0, 1])["slabs"].data_ptr()
+        _lib.check(lib.trimkv_evict_split_rooms(at, on_host, 2, 2, 128, _lib.BF16, _lib.F32, M, None, 0, 0, n + 1, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST, 0, n, 200,
+                                                lists.data_ptr(), 4, lists.data_ptr() + 16, total, 7, ws.data_ptr(), need, _lib.current_stream(ws.device)), "rooms")
+        assert (ws[need:] == 9).all()
+        _check(cache, held, keep, str(first))

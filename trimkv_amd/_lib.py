@@ -58,6 +58,8 @@ SIGNATURES = {
     "trimkv_evict_layers": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _p, _i, _i, _i, _i, _p, _sz, _p]),
     "trimkv_evict_split_workspace": (_sz, [_i, _i, _i, _i]),
     "trimkv_evict_split": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _i, _i, _i, _i, _i, _p, _i, _p, _sz, _p]),
+    "trimkv_evict_split_rooms_workspace": (_sz, [_i, _i, _i, _i]),
+    "trimkv_evict_split_rooms": (_i, [_p, _i, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _i, _i, _i, _i, _i, _p, _i, _p, _i, _i, _p, _sz, _p]),
     "trimkv_evict_host_layers": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _i, _i, _i, _i, _i, _p, _sz, _p]),
     "trimkv_evict_listed": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _p, _i, _i, _i, _i, _p, _i, _p, _sz, _p]),
     "trimkv_compact_threshold_layers": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _i, _p, _i64, _i, _i, _i, _p, _sz, _p]),

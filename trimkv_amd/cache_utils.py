@@ -88,6 +88,10 @@ class LazyLogBeta:
         return out.transpose(1, 2) if self.transposed else out
 
 
+SPLIT_SCRATCH = 256 << 20   # most bytes that a split eviction takes for the length of its launches
+_SPLIT_ROWS = 512           # kept rows per chunk (SPLIT_ROWS of csrc/evict.hip)
+
+
 def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -> bool:
     """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split``): ``rows`` due rows
     in all, the longest segment of ``longest``, at most ``kept`` of a segment's left, none losing more than ``spill``.  One workgroup per segment takes about
@@ -433,20 +437,31 @@ class _SlabBacked(_CacheBase):
         return torch.from_numpy(arr.view(np.uint8)).to(self._slabs[layers[0]].k.device)
 
     def _evict_layers(self, layers: List[int], keep: int, keep_per_seg, slack: int, strategy_code: int,
-                      rounding: int, sliding_window: int, q_idx, work: Optional[np.ndarray] = None, spill: int = 512,
-                      due: Optional[Tuple[int, int, int]] = None) -> None:
-        """``trimkv_evict_layers`` over ``layers`` (all of one shape): one launch of nseg x len(layers) workgroups.
+                      rounding: int, sliding_window: int, q_idx, due: Optional[Tuple[np.ndarray, np.ndarray, np.ndarray]] = None,
+                      spill: int = 512) -> None:
+        """``trimkv_evict_layers`` over ``layers`` (all of one shape): one launch of nseg x len(layers) workgroups, or the three
+        launches of the split eviction (``split_evict``).
         ``q_idx``: the query index, one int or one per layer.  ``keep_per_seg``: None, a host array (uploaded) or a device
-        int32 tensor, ``[nseg]`` or ``[len(layers), nseg]``.  ``work``: host int32 array of ``index in layers * nseg +
-        segment``: only these pairs get a workgroup (``trimkv_evict_listed``); it reaches the device through pinned memory
-        in stream order.  ``spill``: the most rows a segment loses, where the caller knows (512: any number); ``due``: rows of the longest segment
-        that is due, of all that are, and the most that one of them keeps."""
+        int32 tensor, ``[nseg]`` or ``[len(layers), nseg]``.  ``due``: where the caller knows which segments are, host arrays of their
+        pairs (``index in layers * nseg + segment``), their rows and the rows they keep; when these are few, only they get a
+        workgroup (``trimkv_evict_listed``).  ``spill``: the most rows a segment loses, where the caller knows (512: any number)."""
         s0 = self._slabs[layers[0]]
         dev = s0.k.device
         max_len = max(self._slabs[l].max_len for l in layers)
+        every = len(layers) * s0.nseg
         qs = [int(q_idx)] * len(layers) if np.isscalar(q_idx) else [int(q) for q in q_idx]
         one_q = all(q == qs[0] for q in qs) and qs[0] > 0
-        on_host = work is None and len(layers) <= 48 and not torch.cuda.is_current_stream_capturing()
+        kdev, stride = None, 0
+        if keep_per_seg is not None:
+            if torch.is_tensor(keep_per_seg):
+                kdev = keep_per_seg.to(device=dev, dtype=torch.int32).contiguous()
+            else:
+                kdev = torch.from_numpy(np.ascontiguousarray(keep_per_seg, dtype=np.int32)).to(dev)
+            stride = 0 if kdev.dim() == 1 else s0.nseg
+        lib = _lib.load()
+        room = self._split_scratch(layers, None if kdev is not None else int(keep), due, max_len, spill)
+        work = due[0] if due is not None and due[0].size * 4 < every and room is None else None
+        on_host = len(layers) <= 48 and work is None and not torch.cuda.is_current_stream_capturing()
         if on_host:
             table, q_all = self._host_table(layers), qs[0] if one_q else 0
             if not one_q:
@@ -456,42 +471,61 @@ class _SlabBacked(_CacheBase):
             table, q_all = self._device_tables(layers)["slabs"], qs[0]
         else:
             table, q_all = self._layer_table_with_q(layers, qs), 0
-        kdev, stride = None, 0
-        if keep_per_seg is not None:
-            if torch.is_tensor(keep_per_seg):
-                kdev = keep_per_seg.to(device=dev, dtype=torch.int32).contiguous()
-            else:
-                kdev = torch.from_numpy(np.ascontiguousarray(keep_per_seg, dtype=np.int32)).to(dev)
-            stride = 0 if kdev.dim() == 1 else s0.nseg
-        lib = _lib.load()
-        pairs = len(layers) * s0.nseg if work is None else int(work.size)
-        wdev = None if work is None else self._upload_work(work, len(layers) * s0.nseg, dev)
-        split = split_evict(*(due or (max_len, pairs * max_len, max_len if kdev is not None else keep)), spill, s0.D) and max_len <= 32768
-        if on_host or split:
-            ws = self._workspace(lib.trimkv_evict_split_workspace(pairs, max_len, s0.D, spill) if split
-                                 else len(layers) * lib.trimkv_evict_workspace(s0.nseg, max_len), dev)
-            shape = (len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype), int(keep), _lib.ptr(kdev), stride, int(slack), q_all,
-                     strategy_code, rounding, int(sliding_window), max_len)
-            room = (_lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.current_stream(dev))
-            if on_host:
-                _lib.check(lib.trimkv_evict_host_layers(table.ctypes.data, *shape, spill if split else 0, *room), "trimkv_evict_host_layers")
-            else:
-                _lib.check(lib.trimkv_evict_split(table.data_ptr(), *shape, spill, _lib.ptr(wdev), 0 if work is None else pairs, *room), "trimkv_evict_split")
-            self._keepalive_layers = (table, kdev)   # read asynchronously by the launch
+        at = table.ctypes.data if on_host else table.data_ptr()
+        shape = (len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype), int(keep), _lib.ptr(kdev), stride, int(slack), q_all)
+        how = (strategy_code, rounding, int(sliding_window), max_len)
+        stream = _lib.current_stream(dev)
+        self._keepalive_layers = (table, kdev)   # read asynchronously by the launch
+        if room is not None:
+            scratch, pairs, first, most = room
+            wdev = None if pairs is None else self._upload_work(np.concatenate([pairs, first]), 2 * every + 1, dev)
+            lists = (None, 0, None, 0) if pairs is None else (wdev.data_ptr(), pairs.size, wdev.data_ptr() + 4 * pairs.size, int(first[-1]))
+            _lib.check(lib.trimkv_evict_split_rooms(at, int(on_host), *shape, *how, spill, *lists, most, scratch.data_ptr(), scratch.numel(), stream),
+                       "trimkv_evict_split_rooms")
             return
         ws = self._workspace(len(layers) * lib.trimkv_evict_workspace(s0.nseg, max_len), dev)
-        if work is not None:
-            rc = lib.trimkv_evict_listed(table.data_ptr(), len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype),
-                                         int(keep), _lib.ptr(kdev), stride, int(slack), q_all, None, strategy_code, rounding, int(sliding_window),
-                                         max_len, wdev.data_ptr(), int(work.size), _lib.ptr(ws), 0 if ws is None else ws.numel(),
-                                         _lib.current_stream(dev))
-            _lib.check(rc, "trimkv_evict_listed")
+        keys = (_lib.ptr(ws), 0 if ws is None else ws.numel(), stream)
+        if on_host:
+            _lib.check(lib.trimkv_evict_host_layers(at, *shape, *how, 0, *keys), "trimkv_evict_host_layers")
+        elif work is not None:
+            wdev = self._upload_work(work, 2 * every + 1, dev)
+            _lib.check(lib.trimkv_evict_listed(at, *shape, None, *how, wdev.data_ptr(), int(work.size), *keys), "trimkv_evict_listed")
         else:
-            rc = lib.trimkv_evict_layers(table.data_ptr(), len(layers), s0.nseg, s0.D, _lib.dtype_code(s0.k.dtype), _lib.dtype_code(s0.lb.dtype),
-                                         int(keep), _lib.ptr(kdev), stride, int(slack), q_all, None, strategy_code, rounding, int(sliding_window),
-                                         max_len, _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.current_stream(dev))
-            _lib.check(rc, "trimkv_evict_layers")
-        self._keepalive_layers = (table, kdev)   # read asynchronously by the launch
+            _lib.check(lib.trimkv_evict_layers(at, *shape, None, *how, *keys), "trimkv_evict_layers")
+
+    def _split_scratch(self, layers: List[int], keep: Optional[int], due, max_len: int, spill: int):
+        """None, or what a split eviction takes: (scratch, pairs, first chunk of each and their number behind the last, most chunks
+        of one); pairs and first chunks None: all pairs, each with room for ``keep`` rows.  The scratch holds what the chunks of the
+        pairs that are due leave aside, 524 bytes at most for a kept row of 128 features.  It goes back to the allocator behind the
+        launches; where it would be more than ``SPLIT_SCRATCH`` bytes, or memory has run out, one workgroup per segment needs none."""
+        s0 = self._slabs[layers[0]]
+        every = len(layers) * s0.nseg
+        if max_len > 32768:
+            return None
+        if due is None and keep is not None:         # a dense cache: all pairs, alike
+            if not split_evict(max_len, every * max_len, keep, spill, s0.D):
+                return None
+            pairs, first, most = None, None, max(1, -(-min(keep, max_len) // _SPLIT_ROWS))
+            total, count = every * most, every
+        else:
+            if due is None:                          # budgets that are on the device only: a segment keeps what it holds at most
+                lens = np.concatenate([self._slabs[l].lens for l in layers])
+                due = (np.arange(every), lens, lens)
+            pairs, rows, kept = due
+            if not split_evict(int(rows.max()), int(rows.sum()), int(kept.max()), spill, s0.D):
+                return None
+            chunks = np.where(kept >= 1024, -(-kept // _SPLIT_ROWS), 0)      # with fewer rows than that the kernel does not split
+            first = np.concatenate([[0], np.cumsum(chunks)])
+            most, total, count = int(chunks.max()), int(first[-1]), int(pairs.size)
+            if total == 0:
+                return None
+        nbytes = _lib.load().trimkv_evict_split_rooms_workspace(count, total, s0.D, spill)
+        if nbytes > SPLIT_SCRATCH or count > 65535:
+            return None
+        try:
+            return torch.empty(nbytes, dtype=torch.uint8, device=s0.k.device), pairs, first, most
+        except torch.OutOfMemoryError:
+            return None
 
     def _upload_work(self, work: np.ndarray, room: int, dev) -> torch.Tensor:
         """A host int32 list on the device without a synchronisation: four pinned staging buffers take turns (an event per
@@ -1372,11 +1406,9 @@ class _RaggedCache(_SlabBacked):
                 self._budgets_dev[key] = keep
             # With few segments due, only those get a workgroup (their list is uploaded in stream order): a launch over every
             # (layer, segment) costs about 0.1 ms in dispatch alone when nearly all of them have nothing to do.
-            ndue = int(hit_all.sum())
-            work = np.flatnonzero(hit_all).astype(np.int32) if ndue * 4 < hit_all.size else None
-            due_lens = lens_all[hit_all]
-            self._evict_layers(every, 0, keep, buffer_size, code, _lib.ROUND_NATIVE, 0, q_idx, work=work,
-                               spill=min(512, int((lens_all - kh_all)[hit_all].max())), due=(int(due_lens.max()), int(due_lens.sum()), int(np.broadcast_to(kh_all, lens_all.shape)[hit_all].max())))
+            kept = np.broadcast_to(kh_all, lens_all.shape)[hit_all]
+            self._evict_layers(every, 0, keep, buffer_size, code, _lib.ROUND_NATIVE, 0, q_idx, due=(np.flatnonzero(hit_all), lens_all[hit_all], kept),
+                               spill=min(512, int((lens_all[hit_all] - kept).max())))
             t = self._device_tables(every)
             rc = lib.trimkv_build_cu_seqlens_layers(t["len"].data_ptr(), t["cu"].data_ptr(), len(every), self._slabs[every[0]].nseg,
                                                     _lib.current_stream(dev))

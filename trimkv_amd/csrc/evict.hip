@@ -323,9 +323,10 @@ struct EvictArgs {
     const int64_t* q_idx_dev; int64_t q_idx_all;
     // listed launch: workgroup i works on entry work[i] = layer * nseg + segment instead of (blockIdx.y, blockIdx.x)
     const int32_t* work; int nlayers;
-    // rows moved by launches of their own (trimkv_evict_split): per pair {rows kept, first row that moves, -, -}, the list of kept
-    // rows, and room for split_spill rows per chunk
-    int4* split_head; uint32_t* split_idx; char* split_stash; int split_stride, split_chunks, split_spill;
+    // rows moved by launches of their own (trimkv_evict_split): per pair {rows kept, first row that moves, its first chunk, -}, and
+    // per chunk of the scratch the list of its kept rows and room for split_spill rows.  A pair has split_chunks chunks, or those
+    // from split_first[pair] to split_first[pair + 1] - 1 of split_total, split_chunks of them at most
+    int4* split_head; uint32_t* split_idx; char* split_stash; const int32_t* split_first; int split_total, split_chunks, split_spill;
 };
 
 // The slabs of the layers of a launch: in a device table (EvictArgs::layers, N = 0) or in the launch's own arguments.  A table
@@ -368,6 +369,12 @@ __device__ __forceinline__ int pair_of_block(const EvictArgs& a) { return a.work
 constexpr int SPLIT_ROWS = 512, SPLIT_FROM = 1024;      // rows per chunk; segments with fewer rows to move stay whole
 
 __device__ __forceinline__ int64_t split_stash_bytes(const EvictArgs& a) { return (int64_t)a.split_spill * (2 * a.row_bytes + 12); }
+// the pair's first chunk of the scratch and how many it has there (none if the list says what cannot be)
+__device__ __forceinline__ int2 split_room(const EvictArgs& a, int pair) {
+    if (!a.split_first) return make_int2(pair * a.split_chunks, a.split_chunks);
+    const int at = a.split_first[pair], end = a.split_first[pair + 1];
+    return at < 0 || end > a.split_total ? make_int2(0, 0) : make_int2(at, min(end - at, a.split_chunks));
+}
 // first row of lo .. hi - 1 whose source is `end` or behind it (sources ascend)
 __device__ __forceinline__ int first_spilled(const uint32_t* idx, int lo, int hi, int end) {
     while (lo < hi) {
@@ -385,10 +392,10 @@ __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const Sla
     const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
     if (lo >= hi) return;
     const int seg = select_pair(a, table, pair);
-    const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
+    const uint32_t* idx = a.split_idx + (int64_t)head.z * SPLIT_ROWS;
     const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS), m = hi - from;
     if (seg < 0 || m <= 0) return;
-    char* stash = a.split_stash + ((int64_t)pair * a.split_chunks + chunk) * split_stash_bytes(a);
+    char* stash = a.split_stash + (int64_t)(head.z + chunk) * split_stash_bytes(a);
     const char* src = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
     char* dst = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
     for (int base = 0; base < m * PPR; base += 8 * 256) {
@@ -426,9 +433,9 @@ __global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a, con
     if (lo >= hi) return;
     const int seg = select_pair(a, table, pair);
     if (seg < 0) return;
-    const uint32_t* idx = a.split_idx + (int64_t)pair * a.split_stride;
+    const uint32_t* idx = a.split_idx + (int64_t)head.z * SPLIT_ROWS;
     const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS);
-    const char* stash = a.split_stash + ((int64_t)pair * a.split_chunks + chunk) * split_stash_bytes(a);
+    const char* stash = a.split_stash + (int64_t)(head.z + chunk) * split_stash_bytes(a);
     const char* kept = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
     char* rows = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
     uint4 t[PPR];
@@ -520,10 +527,12 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
         for (int r = threadIdx.x; r < kept && r < a.kept_stride; r += EV_THREADS)
             a.kept_idx[(int64_t)seg * a.kept_stride + r] = (int32_t)keys[r];
     }
-    if (SELECT && a.split_head && kept - first_moved >= SPLIT_FROM && (n - kept <= a.split_spill || a.split_spill >= SPLIT_ROWS)) {
-        const int pair = pair_of_block(a);
-        for (int r = threadIdx.x; r < kept; r += EV_THREADS) a.split_idx[(int64_t)pair * a.split_stride + r] = keys[r];
-        if (threadIdx.x == 0) a.split_head[pair] = make_int4(kept, first_moved, 0, 0);
+    // workgroup-uniform: few rows to move, more lost than a chunk has room for, or more kept than the pair has chunks: moved here
+    int2 room = make_int2(0, 0);
+    if (SELECT && a.split_head && kept - first_moved >= SPLIT_FROM && (n - kept <= a.split_spill || a.split_spill >= SPLIT_ROWS)) room = split_room(a, pair_of_block(a));
+    if (SELECT && (kept + SPLIT_ROWS - 1) / SPLIT_ROWS <= room.y) {
+        for (int r = threadIdx.x; r < kept; r += EV_THREADS) a.split_idx[(int64_t)room.x * SPLIT_ROWS + r] = keys[r];
+        if (threadIdx.x == 0) a.split_head[pair_of_block(a)] = make_int4(kept, first_moved, room.x, 0);
     } else if (first_moved < kept)
         move_segment(kseg, vseg, lbseg, posseg, keys, kept, first_moved, a.row_bytes, a.lpr_shift, lb_bytes);
     if (threadIdx.x == 0) a.seg_len[seg] = kept;
@@ -1013,42 +1022,49 @@ extern "C" int trimkv_evict_listed(const trimkv_layer_slabs* layers, int nlayers
 }
 
 // workspace of trimkv_evict_split: heads, lists of kept rows, stashes
-struct SplitSizes { int chunks, spill; size_t idx, stash, total; };
-static SplitSizes split_sizes(int npairs, int max_len, int row_bytes, int spill) {
+struct SplitSizes { int spill; size_t idx, stash, total; };
+static int split_chunks_of(int rows) { return (rows + SPLIT_ROWS - 1) / SPLIT_ROWS; }
+static SplitSizes split_sizes(int npairs, int64_t chunks, int row_bytes, int spill) {
     SplitSizes z;
-    z.chunks = (max_len + SPLIT_ROWS - 1) / SPLIT_ROWS;
     z.spill = ((spill < SPLIT_ROWS ? spill : SPLIT_ROWS) + 3) / 4 * 4;      // rows of 12 bytes of metadata stay 16-byte aligned
     z.idx = (size_t)npairs * sizeof(int4);
-    z.stash = (z.idx + (size_t)npairs * max_len * 4 + 255) / 256 * 256;
-    z.total = z.stash + (size_t)npairs * z.chunks * z.spill * (2 * row_bytes + 12);
+    z.stash = (z.idx + (size_t)chunks * SPLIT_ROWS * 4 + 255) / 256 * 256;
+    z.total = z.stash + (size_t)chunks * z.spill * (2 * row_bytes + 12);
     return z;
 }
 
-extern "C" size_t trimkv_evict_split_workspace(int npairs, int max_len, int head_dim, int spill) {
-    if (npairs <= 0 || max_len <= 0 || head_dim <= 0 || spill <= 0) return 0;
-    return split_sizes(npairs, max_len, head_dim * 2, spill).total;
+extern "C" size_t trimkv_evict_split_workspace(int npairs, int rows, int head_dim, int spill) {
+    if (npairs <= 0 || rows <= 0 || head_dim <= 0 || spill <= 0) return 0;
+    return split_sizes(npairs, (int64_t)npairs * split_chunks_of(rows), head_dim * 2, spill).total;
+}
+extern "C" size_t trimkv_evict_split_rooms_workspace(int npairs, int total_chunks, int head_dim, int spill) {
+    if (npairs <= 0 || total_chunks <= 0 || head_dim <= 0 || spill <= 0) return 0;
+    return split_sizes(npairs, total_chunks, head_dim * 2, spill).total;
 }
 
+// What the three split entry points share.  first_chunk = NULL: most_chunks for every pair.
 template <int N = 0>
 static int evict_split_common(const char* fn, const trimkv_layer_slabs* layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
                                   int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
                                   int strategy, int rounding, int sliding_window, int max_len, int spill,
-                                  const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream, const SlabTable<N>& table = SlabTable<N>{}) {
+                                  const int32_t* work, int nwork, const int32_t* first_chunk, int total_chunks, int most_chunks,
+                                  void* workspace, size_t workspace_bytes, void* stream, const SlabTable<N>& table = SlabTable<N>{}) {
     if (work && nwork == 0) return TRIMKV_OK;
     if (nwork < 0 || spill <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: nwork=%d spill=%d", fn, nwork, spill);
     if (head_dim != 64 && head_dim != 96 && head_dim != 128) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: head_dim %d (64, 96 or 128)", fn, head_dim);
     if (max_len <= 0 || (size_t)max_len * 4 > (size_t)EV_LDS_KEY_BYTES) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: max_len %d (up to %d)", fn, max_len, EV_LDS_KEY_BYTES / 4);
     const int64_t pairs = work ? nwork : (int64_t)nlayers * nseg;
     if (pairs <= 0 || pairs > 65535) return fail(TRIMKV_ERR_SHAPE, "%s: %lld (layer, segment) pairs", fn, (long long)pairs);
-    const SplitSizes z = split_sizes((int)pairs, max_len, head_dim * 2, spill);
+    if (!first_chunk) total_chunks = (int)pairs * most_chunks;      // 65535 pairs of 64 chunks at most
+    const SplitSizes z = split_sizes((int)pairs, total_chunks, head_dim * 2, spill);
     if (!workspace || ((uintptr_t)workspace & 15) || workspace_bytes < z.total)
         return fail(TRIMKV_ERR_WORKSPACE, "%s: aligned workspace of %zu bytes needed, got %zu", fn, z.total, workspace_bytes);
     EvictArgs a{};
     a.split_head = (int4*)workspace; a.split_idx = (uint32_t*)((char*)workspace + z.idx); a.split_stash = (char*)workspace + z.stash;
-    a.split_stride = max_len; a.split_chunks = z.chunks; a.split_spill = z.spill;
+    a.split_first = first_chunk; a.split_total = total_chunks; a.split_chunks = most_chunks; a.split_spill = z.spill;
     if (int rc = evict_layers_common(fn, a, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, nullptr, strategy,
                                      rounding, sliding_window, max_len, work, nwork, nullptr, 0, stream, table)) return rc;
-    const dim3 grid(z.chunks, (unsigned)pairs, 2);
+    const dim3 grid(most_chunks, (unsigned)pairs, 2);
     hipStream_t st = (hipStream_t)stream;
     auto go = [&](auto ppr) {
         hipLaunchKernelGGL((split_stash_kernel<decltype(ppr)::value, N>), grid, dim3(256), 0, st, a, table);
@@ -1065,7 +1081,38 @@ extern "C" int trimkv_evict_split(const trimkv_layer_slabs* layers, int nlayers,
                                   int strategy, int rounding, int sliding_window, int max_len, int spill,
                                   const int32_t* work, int nwork, void* workspace, size_t workspace_bytes, void* stream) {
     return evict_split_common("trimkv_evict_split", layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx,
-                              strategy, rounding, sliding_window, max_len, spill, work, nwork, workspace, workspace_bytes, stream);
+                              strategy, rounding, sliding_window, max_len, spill, work, nwork, nullptr, 0, split_chunks_of(max_len), workspace, workspace_bytes, stream);
+}
+
+// The table in HOST memory, checked and copied into the launches' arguments.
+static int host_table(const char* fn, SlabTable<HOST_LAYERS>& table, const trimkv_layer_slabs* host_layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype, int max_len) {
+    if (!host_layers) return fail(TRIMKV_ERR_NULL, "%s: null layer table", fn);
+    if (nlayers <= 0 || nlayers > HOST_LAYERS) return fail(TRIMKV_ERR_SHAPE, "%s: nlayers=%d (up to %d)", fn, nlayers, HOST_LAYERS);
+    for (int l = 0; l < nlayers; ++l) {
+        const trimkv_layer_slabs& s = table.at[l] = host_layers[l];
+        int lpr_shift;
+        // a layer of less capacity than max_len is taken: the kernel leaves segments with more rows than their layer can hold alone
+        if (int rc = check_slab_args(fn, s.k_slab, s.v_slab, s.lb_slab, s.pos_slab, s.seg_len, nseg, s.cap < max_len ? max_len : s.cap, head_dim, kv_dtype, lb_dtype, max_len, &lpr_shift)) return rc;
+    }
+    return TRIMKV_OK;
+}
+
+extern "C" int trimkv_evict_split_rooms(const trimkv_layer_slabs* layers, int on_host, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
+                                        int keep, const int32_t* keep_per_seg, int keep_layer_stride, int slack, int64_t q_idx,
+                                        int strategy, int rounding, int sliding_window, int max_len, int spill,
+                                        const int32_t* work, int nwork, const int32_t* first_chunk, int total_chunks, int most_chunks,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "trimkv_evict_split_rooms";
+    if (most_chunks <= 0 || most_chunks > EV_LDS_KEY_BYTES / 4 / SPLIT_ROWS || (first_chunk && most_chunks > total_chunks))
+        return fail(TRIMKV_ERR_SHAPE, "%s: total_chunks=%d most_chunks=%d", fn, total_chunks, most_chunks);
+    auto go = [&](const auto& table) {
+        return evict_split_common(fn, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, strategy, rounding, sliding_window,
+                                  max_len, spill, work, nwork, first_chunk, total_chunks, most_chunks, workspace, workspace_bytes, stream, table);
+    };
+    if (!on_host) return go(SlabTable<0>{});
+    SlabTable<HOST_LAYERS> table{};
+    if (int rc = host_table(fn, table, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, max_len)) return rc;
+    return go(table);
 }
 
 extern "C" int trimkv_evict_host_layers(const trimkv_layer_slabs* host_layers, int nlayers, int nseg, int head_dim, int kv_dtype, int lb_dtype,
@@ -1073,16 +1120,11 @@ extern "C" int trimkv_evict_host_layers(const trimkv_layer_slabs* host_layers, i
                                         int strategy, int rounding, int sliding_window, int max_len, int spill,
                                         void* workspace, size_t workspace_bytes, void* stream) {
     const char* fn = "trimkv_evict_host_layers";
-    if (!host_layers) return fail(TRIMKV_ERR_NULL, "%s: null layer table", fn);
-    if (nlayers <= 0 || nlayers > HOST_LAYERS || spill < 0) return fail(TRIMKV_ERR_SHAPE, "%s: nlayers=%d (up to %d) spill=%d", fn, nlayers, HOST_LAYERS, spill);
+    if (spill < 0) return fail(TRIMKV_ERR_SHAPE, "%s: spill=%d", fn, spill);
     SlabTable<HOST_LAYERS> table{};
-    for (int l = 0; l < nlayers; ++l) {
-        const trimkv_layer_slabs& s = table.at[l] = host_layers[l];
-        int lpr_shift;
-        if (int rc = check_slab_args(fn, s.k_slab, s.v_slab, s.lb_slab, s.pos_slab, s.seg_len, nseg, s.cap < max_len ? max_len : s.cap, head_dim, kv_dtype, lb_dtype, max_len, &lpr_shift)) return rc;   // rows past a layer's capacity: that segment is left alone
-    }
+    if (int rc = host_table(fn, table, host_layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, max_len)) return rc;
     if (spill > 0) return evict_split_common(fn, host_layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, strategy,
-                                             rounding, sliding_window, max_len, spill, nullptr, 0, workspace, workspace_bytes, stream, table);
+                                             rounding, sliding_window, max_len, spill, nullptr, 0, nullptr, 0, split_chunks_of(max_len), workspace, workspace_bytes, stream, table);
     EvictArgs a = {};
     return evict_layers_common(fn, a, host_layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, keep, keep_per_seg, keep_layer_stride, slack, q_idx, nullptr,
                                strategy, rounding, sliding_window, max_len, nullptr, 0, workspace, workspace_bytes, stream, table);
