@@ -230,3 +230,58 @@ def test_c_abi_append_attend_other_shapes_full_slabs_and_cu(D, dtype, lb_dtype, 
             ref = p @ vs
             err = (got.view(nseg, G, D)[seg].float() - ref).abs()
             assert bool((err <= 2e-2 + 1e-2 * ref.abs()).all()), (seg, float(err.max()))
+
+
+@pytest.mark.parametrize("cls", ["TrimKVCache", "BatchedDynamicBudgetTrimKVCache"])
+@pytest.mark.parametrize("inference", [False, True])
+def test_tensors_that_update_returns_are_the_callers_own(cls, inference):
+    """What a caller does to the shape of the returned tensors, or whether they require grad, neither reaches a later caller at
+    the same length nor a tensor of that length handed out before; after growth and batch selection the views are of the new
+    storage."""
+    import trimkv_amd
+    dense = cls == "TrimKVCache"
+    B, H, M, buf = 2, 2, 40, 4
+    gen = torch.Generator().manual_seed(1)
+    cache = getattr(trimkv_amd, cls)()
+
+    def add(S, at):
+        k, v = draw_kv(gen, B, H, S)
+        return cache.update(k.to(DEV), v.to(DEV), draw_log_beta(gen, B, H, S).to(DEV), torch.arange(at, at + S).to(DEV), 0)
+
+    def check(got):
+        s = cache._slabs[0]
+        n = s.max_len
+        want = [(s.k, (B, H, n, 128)), (s.v, (B, H, n, 128)), (s.lb, (B, H, n)), (s.pos, (B, H, n))] if dense else \
+            [(t, (s.nseg * s.cap, d)) for t, d in ((s.k, 128), (s.v, 128), (s.lb, 1), (s.pos, 1))]
+        for t, (base, shape) in zip(got, want):
+            assert tuple(t.shape) == shape and t.data_ptr() == base.data_ptr() and not t.requires_grad
+            assert torch.equal(t, base.view(B, H, s.cap, -1)[:, :, :n].reshape(shape) if dense else base.view(shape))
+
+    with torch.inference_mode(inference):
+        check(add(M, 0)[:4])
+        at, kept = M, {}
+        for cycle in range(3):
+            for _ in range(buf):
+                got = add(1, at)[:4]
+                at += 1
+                check(got)
+                n = cache._slabs[0].max_len
+                for i, t in enumerate(got):
+                    assert all(t is not o for o, _ in kept.get((n, i), ()))
+                    if t.is_floating_point() and not inference and cycle != 1:
+                        t.requires_grad_()
+                    else:
+                        t.unsqueeze_(0).transpose_(0, 1)
+                    kept.setdefault((n, i), []).append((t, tuple(t.shape)))
+                for t, shape in (x for xs in kept.values() for x in xs):
+                    assert tuple(t.shape) == shape
+            if dense:
+                cache.compress("alpha", memory_size=M, buffer_size=buf)
+            else:
+                cache.set_budgets(np.full(B * H, M))
+                cache.evict_to_budgets(buffer_size=0)
+        check(add(900, at)[:4])                                  # growth
+        if dense:
+            cache.batch_select_indices(torch.tensor([1, 0]))
+            check(cache[0])
+    check(add(1, at + 900)[:4])

@@ -117,7 +117,7 @@ class _Slab:
     """Device storage of one layer."""
 
     __slots__ = ("k", "v", "lb", "pos", "seg_len", "cu", "B", "H", "D", "cap", "lens", "max_len", "k4", "v4", "lb3", "pos3", "ptrs", "order",
-                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host", "row_shape", "views", "step",
+                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host", "row_shape", "strides", "step",
                  "seg_start")
 
     def __init__(self, B, H, D, cap, kv_dtype, lb_dtype, device, ragged: bool):
@@ -141,8 +141,7 @@ class _Slab:
         self._refresh_views()
 
     def _refresh_views(self) -> None:
-        """[B,Hkv,cap,...] views of the slabs and their addresses, rebuilt only when storage changes: the per-step
-        views handed to callers are one narrow() of these."""
+        """[B,Hkv,cap,...] views of the slabs, their strides and addresses, rebuilt only when storage changes."""
         B, H, cap, D = self.B, self.H, self.cap, self.D
         self.k4, self.v4 = self.k.view(B, H, cap, D), self.v.view(B, H, cap, D)
         self.lb3, self.pos3 = self.lb.view(B, H, cap), self.pos.view(B, H, cap)
@@ -150,7 +149,7 @@ class _Slab:
                      None if self.cu is None else self.cu.data_ptr())
         self.codes = (_lib.dtype_code(self.k.dtype), _lib.dtype_code(self.lb.dtype))
         self.row_shape = (B, H, 1, D)
-        self.views = {}
+        self.strides = (self.k4.stride(), self.lb3.stride())
         self.seg_start = None
         self.step = None
 
@@ -168,24 +167,15 @@ class _Slab:
         return ctypes.addressof(buf)
 
     def rows(self, n: int):
-        """The first ``n`` rows of K, V, log beta and positions as [B,Hkv,n,...] views.  A decode step hands them out per layer and
-        the lengths of an eviction cycle come again, so the views are kept (four of them cost 5 us to make); they go when
-        storage moves, and views made under inference mode stay apart from others."""
-        key = (n, torch.is_inference_mode_enabled())
-        got = self.views.get(key)
-        if got is None or got[0].requires_grad or got[1].requires_grad:
-            if len(self.views) >= 1024:
-                self.views.clear()
-            got = self.views[key] = (self.k4.narrow(2, 0, n), self.v4.narrow(2, 0, n), self.lb3.narrow(2, 0, n), self.pos3.narrow(2, 0, n))
-        return got
+        """The first ``n`` rows of K, V, log beta and positions as [B,Hkv,n,...] views, new objects for every caller (as_strided:
+        a decode step makes four per layer, 0.67 us each against 1.03 by narrow)."""
+        B, H, (s4, s3) = self.B, self.H, self.strides
+        four, three = (B, H, n, self.D), (B, H, n)
+        return self.k.as_strided(four, s4), self.v.as_strided(four, s4), self.lb.as_strided(three, s3), self.pos.as_strided(three, s3)
 
     def flat(self):
-        """K, V, log beta and positions with the segments one behind the other, [nseg * cap, ...] (kept like ``rows``)."""
-        key = ("flat", torch.is_inference_mode_enabled())
-        got = self.views.get(key)
-        if got is None or got[0].requires_grad or got[1].requires_grad:
-            got = self.views[key] = (self.k.view(-1, self.D), self.v.view(-1, self.D), self.lb.view(-1, 1), self.pos.view(-1, 1))
-        return got
+        """K, V, log beta and positions with the segments one behind the other, [nseg * cap, ...]."""
+        return self.k.view(-1, self.D), self.v.view(-1, self.D), self.lb.view(-1, 1), self.pos.view(-1, 1)
 
     @property
     def nseg(self) -> int:
