@@ -202,3 +202,14 @@ def test_split_evictions_with_room_for_what_is_kept():
     assert call(nbytes=need - 1) == call(ws=None) == call(ws=one + 8) < 0
     assert call(work=None, nwork=0, first=None, total=0, nbytes=lib.trimkv_evict_split_rooms_workspace(8, 64, 128, 128) - 1) < 0
     assert call(D=80) == call(max_len=32769) < 0 and call(at=None, on_host=1) < 0 and call(on_host=1, nl=49) == -2
+
+
+def test_keys_are_divided_for_many_query_tiles_only_where_lengths_differ_much():
+    """129 to 224 query tiles: the segments' mean length decides, 0 (alike) never divides; fewer tiles do not ask for it."""
+    rule = lambda tiles, n, uneven: _lib.load().trimkv_prefill_split_tiles(1, 8, 4, 64 * tiles // 8, n, uneven)
+    for n in (4096, 8192, 10240):
+        assert rule(168, n, 0) == rule(168, n, 76) == rule(168, n, 100) == 0 and rule(168, n, 75) == rule(168, n, 1) == (n // 64 + 2) // 3
+        assert rule(176, n, 0) == rule(176, n, 56) == 0 and rule(176, n, 55) == rule(224, n, 1) == (n // 64 + 2) // 3
+        assert rule(232, n, 1) == rule(248, n, 40) == 0
+        assert rule(64, n, 0) == rule(64, n, 30) > 0
+    assert rule(168, 4032, 1) == rule(176, 10304, 1) == 0 and rule(168, 10304, 1) > 0

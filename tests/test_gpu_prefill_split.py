@@ -69,3 +69,30 @@ def test_the_rule_divides_few_query_tiles_and_the_public_call_follows_it(B, H, G
     out = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), B, H, G, None, None, n, n, 128 ** -0.5)
     ok, err = attn_close(out, ragged_attention(q, k, v, cu, H))
     assert ok, err
+
+
+def test_the_rule_hears_how_uneven_the_segments_are(monkeypatch):
+    """A ragged cache of equal lengths is no uneven one; after budgets have been applied the mean length says how uneven it is.
+    Rows that come packed without their number count as alike."""
+    from trimkv_amd import BatchedDynamicBudgetTrimKVCache, get_attention_interface
+    from trimkv_amd.attn import hip_attn
+    heard, plain = [], hip_attn._prefill_split
+    monkeypatch.setattr(hip_attn, "_prefill_split", lambda *a: heard.append(a[-1]) or plain(*a))
+    attend, gen = get_attention_interface("db_attn_flash_batched"), torch.Generator().manual_seed(0)
+    B, H, Q, n = 1, 4, 70, 400
+    cache = BatchedDynamicBudgetTrimKVCache()
+
+    def chunk(S, at, **how):
+        k, v = (torch.randn(B, H, S, 128, generator=gen).to(torch.bfloat16).to(DEV) for _ in range(2))
+        keys, values, _, _, kw = cache.update(k, v, -torch.rand(B, H, S, generator=gen).to(DEV) - 0.01, torch.arange(at, at + S).to(DEV), 0, how)
+        q = torch.randn(B, 2 * H, S, 128, generator=gen).to(torch.bfloat16).to(DEV)
+        attend(None, q, keys, values, None, flash_attn_kwargs=kw)
+        return q, keys, values, kw
+    chunk(n, 0)
+    cache.set_budgets(np.array([400, 100, 100, 200]))
+    cache.evict_to_budgets()
+    chunk(Q, n)                                       # 470, 170, 170, 270: 57 % of 470 in the mean
+    q, keys, values, kw = chunk(Q, n + Q, packed=True)
+    del kw["rows"]
+    attend(None, q, keys, values, None, flash_attn_kwargs=kw)
+    assert heard == [0, 57, 62, 0]

@@ -213,8 +213,9 @@ def _take_pending(kw: Optional[dict], query: torch.Tensor, key: torch.Tensor, gr
 
 
 @functools.lru_cache(maxsize=1024)
-def _prefill_split(batch: int, kv_heads: int, group: int, q_len: int, max_len: int, uneven: bool) -> Tuple[int, int]:
-    """(64-key tiles per workgroup, workspace bytes) of a chunk's attention; (0, 0): a query tile's keys stay together."""
+def _prefill_split(batch: int, kv_heads: int, group: int, q_len: int, max_len: int, uneven: int) -> Tuple[int, int]:
+    """(64-key tiles per workgroup, workspace bytes) of a chunk's attention; (0, 0): a query tile's keys stay together.
+    ``uneven``: as ``trimkv_prefill_split_tiles`` takes it."""
     lib = _lib.load()
     tiles = lib.trimkv_prefill_split_tiles(batch, kv_heads, group, q_len, max_len, uneven)
     return tiles, lib.trimkv_prefill_split_workspace(batch, kv_heads, group, q_len, max_len, tiles)
@@ -222,8 +223,9 @@ def _prefill_split(batch: int, kv_heads: int, group: int, q_len: int, max_len: i
 
 def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.Tensor, batch: int, kv_heads: int, group: int,
                       seg_len: Optional[torch.Tensor], seg_start: Optional[torch.Tensor], cap: int, max_len: int,
-                      scale: float) -> torch.Tensor:
-    """``query`` [B, Hq, Q, D] (any strides with D contiguous) -> [B, Q, Hq, D], bottom-right causal."""
+                      scale: float, uneven: int = 0) -> torch.Tensor:
+    """``query`` [B, Hq, Q, D] (any strides with D contiguous) -> [B, Q, Hq, D], bottom-right causal.  ``uneven``: where the segments'
+    lengths are known to differ, their mean in percent of ``max_len`` (which launches are taken, not what they compute)."""
     if not query.is_cuda:
         raise _lib.TrimKVLibraryError("prefill attention runs on the GPU through libtrimkv_hip.so only (no CPU path)")
     lib = _lib.load()
@@ -234,7 +236,7 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
         out = torch.empty(B, Q, kv_heads, group, D, dtype=query.dtype, device=query.device)
         for a in range(0, group, g1):
             part = prefill_attention(q5[:, :, a:a + g1].reshape(B, kv_heads * g1, Q, D), k_rows, v_rows, batch, kv_heads, g1, seg_len,
-                                     seg_start, cap, max_len, scale)
+                                     seg_start, cap, max_len, scale, uneven)
             out[:, :, :, a:a + g1] = part.view(B, Q, kv_heads, g1, D)
         return out.view(B, Q, Hq, D)
     sb, sh, st, sd = query.stride()
@@ -246,7 +248,7 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
             k_rows.data_ptr(), v_rows.data_ptr(), _lib.ptr(seg_len), _lib.ptr(seg_start),
             batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len)
     stream = _lib.current_stream(query.device)
-    tiles, need = _prefill_split(batch, kv_heads, group, Q, max_len, seg_start is not None)
+    tiles, need = _prefill_split(batch, kv_heads, group, Q, max_len, uneven)
     if tiles:   # few query tiles: their keys divided among several workgroups
         try:
             work = torch.empty(need, dtype=torch.uint8, device=query.device)
@@ -513,7 +515,9 @@ def _ragged_common(query, key, value, flash_attn_kwargs, batch_size, num_kv_head
         out = decode_attention(q2, key, value, nseg, G, head_lens, seg_start, cap, max(1, max_len), D ** -0.5,
                                chunk=kw.get("chunk", 0), seg_order=kw.get("seg_order"), pieces=pieces)
         return out.view(B, 1, Hq, D), None, None
-    out = prefill_attention(query, key, value, batch_size, num_kv_heads, G, head_lens, seg_start, cap, max(1, max_len), D ** -0.5)
+    rows = kw.get("rows")    # held in all, where the caller's cache knows it
+    uneven = max(1, 100 * rows // (nseg * max_len)) if rows is not None and rows < nseg * max_len else 0
+    out = prefill_attention(query, key, value, batch_size, num_kv_heads, G, head_lens, seg_start, cap, max(1, max_len), D ** -0.5, uneven)
     return out, None, None
 
 

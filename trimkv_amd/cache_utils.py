@@ -1030,7 +1030,7 @@ class _RaggedCache(_SlabBacked):
         src = seg * slab.cap + (r - slab.cu[seg])
         flat = (slab.k.view(-1, slab.D).index_select(0, src), slab.v.view(-1, slab.D).index_select(0, src),
                 slab.lb.view(-1).index_select(0, src).unsqueeze(-1), slab.pos.view(-1).index_select(0, src).unsqueeze(-1))
-        kw = {"head_lens": slab.seg_len, "cu_seqlens_k": slab.cu, "max_len": slab.max_len}
+        kw = {"head_lens": slab.seg_len, "cu_seqlens_k": slab.cu, "max_len": slab.max_len, "rows": slab.total}
         return flat, kw
 
     def _update(self, key_states, value_states, retention_weights, cache_positions, layer_idx: int, packed: bool = False):
@@ -1065,7 +1065,7 @@ class _RaggedCache(_SlabBacked):
         # grid-split fallback (callers that ignore "pieces"): rows per piece for about attention_pieces pieces
         chunk = max(512, ((slab.total // self.attention_pieces + 63) // 64) * 64)
         kw = {"head_lens": slab.seg_len, "cu_seqlens_k": slab.cu,
-              "seg_start": self._seg_start(slab), "seg_cap": slab.cap, "max_len": slab.max_len, "chunk": chunk,
+              "seg_start": self._seg_start(slab), "seg_cap": slab.cap, "max_len": slab.max_len, "rows": slab.total, "chunk": chunk,
               "seg_order": slab.order, "pieces": self._piece_list(slab)}
         if slab.pending is not None:
             # head_lens / cu_seqlens_k still hold the values before this token: the attention call that receives this

@@ -877,9 +877,12 @@ extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_
 // for the merge's launch, 0.8 us per share that a row's merge walks, 0.045 us per workgroup for its 130 KB written and read.
 // Measured (us, D 128, whole -> split): 8 tiles of 2048 keys 44 -> 21, of 8192 keys 150 -> 31; 32 of 4096 79 -> 35; 56 of 2954
 // 64 -> 37; 96 of 4096 80 -> 57; 128 of 8192 155 -> 107; left whole: 96 of 2048 44 -> 40, of 1024 27 -> 30, 40 of 1024 27 -> 25.
-// Between 128 and 256 tiles of like length the chip's rate gains nothing from more workgroups (168 tiles of 2954 keys: 68 -> 77);
-// of unlike segments the longest one holds up the rest, and three shares let the others' CUs help: 168 .. 224 tiles, lengths
-// uniform up to 4096 keys 80 -> 74 .. 85 -> 83, to 10000 keys 188 -> 166 .. 197 -> 170; up to 3000 keys 63 -> 70, hence the line.
+// Between 128 and 256 tiles of like length the chip's rate gains nothing from more workgroups (192 tiles of 4096 keys 103 -> 119, of
+// 8192 175 -> 205); of unlike segments the longest one holds up the rest, and three shares let the others' CUs help.  By mean
+// length / longest (24 or 32 segments): 160 and 168 tiles, two rounds of the chip, 0.69 of 4100 keys 85 -> 84, 0.60 83 -> 79, 0.75
+// of 8192 152 -> 142, 0.68 151 -> 136, 0.55 of 10000 184 -> 157, but 0.77 of 4096 82 -> 84; more tiles up to 0.55: 192, 0.53 of
+// 8192 153 -> 131; 216, 0.53 157 -> 143; 224, 0.52 of 6000 117 -> 113, of 10000 194 -> 166, but 0.57 of 8192 166 -> 177; beyond 10000
+// keys or 224 tiles not at all (240, 0.52 of 12000 245 -> 260).  Up to 3000 keys 63 -> 70.
 extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
     if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0) return 0;
     int64_t tiles, rows;
@@ -900,7 +903,10 @@ extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, in
         return (int)take;
     }
     if (items >= 256) return 0;
-    if (items > 128) return uneven && key_tiles >= 64 ? (int)((key_tiles + 2) / 3) : 0;
+    if (items > 128) {
+        const bool pays = uneven > 0 && key_tiles >= 64 && (items <= 170 ? uneven <= 75 : uneven <= 55 && items <= 224 && key_tiles <= 160);
+        return pays ? (int)((key_tiles + 2) / 3) : 0;
+    }
     float best = 1.15f * (float)key_tiles - 8.0f;   // below that the second launch costs a caller whose queue runs dry as much
     int64_t take = 0;
     for (int64_t s = 2; s <= 32 && items * s <= 256; ++s) {
