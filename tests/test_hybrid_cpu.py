@@ -147,3 +147,11 @@ def test_oracle_router_by_hand():
 def test_oracle_norm_has_eps_inside_the_root():
     x = torch.tensor([3.0, 4.0], dtype=torch.float64)
     assert torch.allclose(ref.rms(x, 12.5), x / 5.0)
+
+
+def test_windows_of_many_pairs_are_not_split_for_their_length():
+    """A share has 1024 rows at most while the (sequence, KV head) pairs do not fill the chip by themselves; from 2048 pairs on a
+    window is one share, and no second launch."""
+    rule = _lib.load_hybrid().trimkv_window_decode_splits
+    assert [rule(b, 8, 4096) for b in (16, 64, 128, 255, 256, 257, 1024)] == [16, 4, 4, 4, 1, 1, 1]
+    assert [rule(64, 8, n) for n in (128, 1024, 6144, 16384)] == [1, 4, 6, 16] and rule(256, 8, 32768) == rule(2048, 1, 2048) == 1

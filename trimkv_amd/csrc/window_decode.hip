@@ -217,10 +217,14 @@ extern "C" int trimkv_window_decode_splits(int batch, int kv_heads, int capacity
     // the launch ends with the workgroup that has the most rows.  64 sequences of 256 .. 4096 rows x 8 heads of 128, a step of the
     // two-layer decoder: 370 us with the splits on the fast axis of the grid, 347 with the heads there, 341 with 512 rows at most,
     // which costs 64 full windows of 4096 rows 2 - 4 % (207 us).
+    // With enough pairs to fill the chip as they are (2048) others run while the longest ones finish, and splitting costs full
+    // windows more than it gives unequal ones.  With the bound of 1024 rows -> without, us, full windows | lengths from 256 rows
+    // up (log-uniform): 2048 pairs of 4096 rows 705 -> 650 | 263 -> 288, 4096 of 4096 1434 -> 1281 | 520 -> 500, of 2048 720 -> 644 |
+    // 335 -> 315; kept below: 512 of 16384 696 -> 659 | 216 -> 263, of 8192 351 -> 340 | 143 -> 154, 1024 of 4096 353 -> 342 | 155 -> 163.
     const int64_t pairs = (int64_t)batch * kv_heads;
     int64_t s = (2048 + pairs - 1) / pairs;
     const int most = (capacity + 127) / 128, least = (capacity + SHARE_ROWS - 1) / SHARE_ROWS;
-    s = s < least ? least : s;
+    if (pairs < 2048 && s < least) s = least;
     s = s < 1 ? 1 : s > most ? most : s;
     return (int)(s > 256 ? 256 : s);
 }
