@@ -229,6 +229,18 @@ def test_mlstm_segments_side_by_side(dtype):
     run_mlstm(s, dtype, [1100], [[512, 580, 8]], f_shift=6.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("name", ["square", "odd"])
+def test_mlstm_sequences_without_tokens_keep_their_state(name, dtype, monkeypatch):
+    """A packed step may hold sequences that bring nothing: first, last, or not begun yet; the state they left goes on behind it,
+    through chunks and token by token.  (The cache's own ``batch`` does not make such steps; the C entry point takes them.)"""
+    def batch(self, lengths, slots):
+        cu = torch.tensor([0] + list(lengths)).cumsum(0).int().to(DEV)
+        return ops.PackedBatch(tuple(lengths), tuple(slots), cu, torch.tensor(slots, dtype=torch.int32, device=DEV), self.seen, self.num_slots)
+    monkeypatch.setattr(HybridCache, "batch", batch)
+    run_mlstm(MSPECS[name], dtype, [21, 31, 12, 40], [[9, 0, 1, 11], [0, 20, 0, 11], [12, 0, 0, 0], [30, 0, 0, 10]])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("gate_scale,f_shift", [(30.0, 0.0), (1.0, 12.0), (1.0, -12.0)])
 def test_mlstm_extreme_gates(dtype, gate_scale, f_shift):

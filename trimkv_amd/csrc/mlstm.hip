@@ -30,6 +30,14 @@ struct MlstmArgs {
 __device__ __forceinline__ float log_input_gate(float z, float cap) { return cap * tanhf(z / cap); }
 __device__ __forceinline__ float log_forget_gate(float z, float cap) { return log_sigmoid_exact(cap * tanhf(z / cap)); }
 
+// A sequence without tokens in this step: S stays, n and m go to the copy that the next step reads (called by 256 threads).
+__device__ __forceinline__ void carry_norm(const MlstmArgs& a, int h, int slot) {
+    if (a.seen[2 * slot] == 0) return;            // nothing is read of a slot that has seen no token
+    const int parity = a.seen[2 * slot + 1] & 1;
+    const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
+    for (int d = threadIdx.x; d <= a.D; d += 256) a.nm[(1 - parity) * copy + at + d] = a.nm[parity * copy + at + d];
+}
+
 // A workgroup owns 64 value columns of one head: lane = column, wavefront w = rows w KW .. of S.
 template <typename T, int KMAX>
 __global__ __launch_bounds__(256) void mlstm_recurrent_kernel(MlstmArgs a) {
@@ -40,6 +48,10 @@ __global__ __launch_bounds__(256) void mlstm_recurrent_kernel(MlstmArgs a) {
     const bool cin = col < a.Dv;
     const int t0 = a.cu[b], len = a.cu[b + 1] - t0;
     const int slot = a.slots[b];
+    if (len <= 0) {                               // workgroup-uniform: there is no token to request
+        if (blockIdx.x == 0) carry_norm(a, h, slot);
+        return;
+    }
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int KW = (a.D + 3) / 4, d0 = w * KW, nd = max(0, min(KW, a.D - d0));
@@ -521,6 +533,10 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int h = blockIdx.y, b = blockIdx.z, col0 = blockIdx.x * 64, col = col0 + w * 16 + c;
     const int t0 = a.cu[b], len = a.cu[b + 1] - t0, slot = a.slots[b];
+    if (len <= 0) {                                   // workgroup-uniform: there is no token to request
+        if (blockIdx.x == 0) carry_norm(a, h, slot);
+        return;
+    }
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
