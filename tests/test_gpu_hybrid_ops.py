@@ -229,8 +229,8 @@ def test_mlstm_segments_side_by_side(dtype):
     run_mlstm(s, dtype, [1100], [[512, 580, 8]], f_shift=6.0)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
-@pytest.mark.parametrize("name", ["square", "odd"])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["square", "odd", "mid"])
 def test_mlstm_sequences_without_tokens_keep_their_state(name, dtype, monkeypatch):
     """A packed step may hold sequences that bring nothing: first, last, or not begun yet; the state they left goes on behind it,
     through chunks and token by token.  (The cache's own ``batch`` does not make such steps; the C entry point takes them.)"""

@@ -195,8 +195,11 @@ __global__ __launch_bounds__(256, DKT <= 4 ? 2 : 1) void mlstm_chunk_kernel(Chun
     const int t0 = a.cu[b], len_all = a.cu[b + 1] - t0;
     const int first = MODE == CHUNK_WHOLE ? 0 : seg * ca.seg_len;
     const int len = MODE == CHUNK_WHOLE ? len_all : min(len_all - first, ca.seg_len);
-    if (len <= 0) return;                             // workgroup-uniform, before any barrier
     const int slot = a.slots[b];
+    if (len <= 0) {                                   // workgroup-uniform, before any barrier (segments: mlstm_join_kernel carries n and m)
+        if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
+        return;
+    }
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int64_t sat = ((int64_t)b * a.H + h) * ca.nseg + seg;
