@@ -285,3 +285,41 @@ def test_tensors_that_update_returns_are_the_callers_own(cls, inference):
             cache.batch_select_indices(torch.tensor([1, 0]))
             check(cache[0])
     check(add(1, at + 900)[:4])
+
+
+@pytest.mark.parametrize("how,short", [("plain", True), ("scaling", True), ("sliding_window", False), ("wide_window", False), ("attention_mask", False), ("softcap", False),
+                                       ("dropout", False), ("copied_keys", False), ("group_list", False), ("chunk_knob", False)])
+def test_what_the_short_way_of_a_decode_step_takes_and_leaves(how, short, monkeypatch):
+    """A deferred append and its attention take the short way only when nothing but q, K and V has a say; every other call goes
+    the general way, and the result is that of separate launches either way."""
+    from trimkv_amd import get_attention_interface
+    from trimkv_amd.attn import hip_attn
+    attn, gen = get_attention_interface("trimkv_hip"), torch.Generator().manual_seed(3)
+    B, H, G, n = 2, 2, 3, 1500
+    plain, fused = _dense_pair()
+    taken, cuts = [], []
+    way, launch = hip_attn._decode_step, hip_attn.append_attend
+    monkeypatch.setattr(hip_attn, "_decode_step", lambda *a: taken.append(way(*a)) or taken[-1])
+    monkeypatch.setattr(hip_attn, "append_attend", lambda *a, **kw: cuts.append(kw.get("uniform_pps", 0)) or launch(*a, **kw))
+    for S, at in ((n, 0), (1, n)):
+        k, v = draw_kv(gen, B, H, S)
+        lb, pos = draw_log_beta(gen, B, H, S).to(DEV), torch.arange(at, at + S).to(DEV)
+        p, f = plain.update(k.to(DEV), v.to(DEV), lb, pos, 0), fused.update(k.to(DEV), v.to(DEV), lb, pos, 0)
+    q = torch.randn(B, H * G, 1, 128, generator=gen).to(torch.bfloat16).to(DEV)
+    kw = {"plain": {}, "scaling": {"scaling": 0.05}, "sliding_window": {"sliding_window": 700}, "wide_window": {"sliding_window": 4000},
+          "attention_mask": {"attention_mask": torch.ones(B, n + 1, dtype=torch.int64, device=DEV)}, "softcap": {"softcap": 20.0}, "dropout": {"dropout": 1e-9}}.get(how, {})
+    if how == "group_list":
+        monkeypatch.setattr(hip_attn, "_DENSE_PIECES_GROUPS", (1, 2))
+    if how == "chunk_knob":
+        monkeypatch.setattr(hip_attn, "dense_chunk", 512)
+    keys = f[0].clone() if how == "copied_keys" else f[0]
+    if how == "copied_keys":
+        keys[:, :, -1] = p[0][:, :, -1]                # the caller's copy is whole
+    mask = kw.pop("attention_mask", None)
+    want = attn(_Mod(), q, p[0], p[1], mask, flash_attn_kwargs=p[4], **kw)[0]
+    got = attn(_Mod(), q, keys, f[1], mask, flash_attn_kwargs=f[4], **kw)[0]
+    assert torch.equal(got, want)
+    assert any(t is not None for t in taken) == short
+    if how == "group_list":
+        assert cuts == [0]
+    _same_dense(plain, fused, [0])

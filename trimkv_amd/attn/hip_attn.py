@@ -349,10 +349,13 @@ def _decode_step(query: torch.Tensor, key: torch.Tensor, slab, scaling: Optional
     if (Q != 1 or G > _MAX_GROUP or Hq != G * H or B != slab.B or D != slab.D or slab.pending is None or slab.cu is not None or not query.is_cuda
             or query.dtype != slab.k.dtype or key.data_ptr() != slab.ptrs[0] or key.shape[2] != slab.max_len):
         return None
+    pps = _uniform_cut(B * H, slab.max_len)
+    if pps > 1 and (G not in _DENSE_PIECES_GROUPS or G not in _FUSED_PIECES_GROUPS):
+        return None
     q2 = query.reshape(B * Hq, D)
     if not q2.is_contiguous():
         q2 = q2.contiguous()
-    return append_attend(slab, q2, G, D ** -0.5 if scaling is None else scaling, uniform_pps=_uniform_cut(B * H, slab.max_len)).view(B, 1, Hq, D)
+    return append_attend(slab, q2, G, D ** -0.5 if scaling is None else scaling, uniform_pps=pps).view(B, 1, Hq, D)
 
 
 def dense_attention_forward(module: nn.Module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
