@@ -216,3 +216,11 @@ def test_pairs_with_chunks_of_their_own(on_host):
                                                 lists.data_ptr(), 4, lists.data_ptr() + 16, total, 7, ws.data_ptr(), need, _lib.current_stream(ws.device)), "rooms")
         assert (ws[need:] == 9).all()
         _check(cache, held, keep, str(first))
+
+
+@pytest.mark.parametrize("longest,segments,kept,spill,D,split", [
+    (8320, 64, 8192, 128, 128, True), (8320, 128, 8192, 128, 128, False), (12288, 32, 8192, 512, 64, True), (12288, 64, 8192, 512, 96, False),
+    (4096, 8, 2048, 512, 128, True), (4096, 8, 2047, 512, 128, False), (4096, 8, 2048, 512, 96, True), (4096, 8, 2048, 512, 64, False),
+    (2688, 8, 2559, 128, 64, False), (2688, 8, 2560, 128, 64, True), (32769, 8, 32000, 512, 128, False), (8320, 8, 8192, 128, 256, False)])
+def test_where_rows_are_moved_by_several_workgroups(longest, segments, kept, spill, D, split):
+    assert cache_utils.split_evict(longest, segments * longest, kept, spill, D) is split

@@ -93,23 +93,27 @@ _SPLIT_ROWS = 512           # kept rows per chunk (SPLIT_ROWS of csrc/evict.hip)
 
 
 def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -> bool:
-    """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split``): ``rows`` due rows
-    in all, the longest segment of ``longest``, at most ``kept`` of a segment's left, none losing more than ``spill``.  One workgroup per segment takes about
-    15 us + 18 ns a row of the longest one; three launches and the detour of the rows that cross a chunk's end take about 30 us
-    + 0.25 ns a row (0.4 ns when most rows cross).  Measured, whole -> split, segments of 128 features that lose 128 rows:
-    8 x 8320 167 -> 60 us, 32 x 8320 196 -> 107, 64 x 4224 117 -> 98, 64 x 2176 63 -> 66, 128 x 8320 253 -> 270; losing 4096:
-    8 x 12288 181 -> 89, 32 x 12288 207 -> 156, 64 x 12288 240 -> 257; of few kept rows one workgroup is done as soon: 16 segments of
-    4100 cut to 1100 58 -> 67, of 6945 cut to 4043 102 -> 74.  Not while a graph is captured: the launches' table may be uploaded
-    for the first time."""
-    return (2048 <= kept and longest <= 32768 and head_dim in (64, 96, 128) and rows * (5 if spill < 512 else 8) < 360 * longest - 300000
-            and not torch.cuda.is_current_stream_capturing())
+    """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split_rooms``): ``rows`` due
+    rows in all, the longest segment of ``longest``, at most ``kept`` of a segment's left, none losing more than ``spill``.  One
+    workgroup per segment takes about 15 us + 18 ns a row of the longest one; three launches and the detour of the rows that cross a
+    chunk's end take about 30 us + 0.25 ns a row (0.4 ns when most rows cross); both less with fewer features.  Measured, whole ->
+    split, us, segments x rows, of 128 / 96 / 64 features.  Split: losing 128 rows 8 x 8320 166 -> 56 / 145 -> 50 / 97 -> 46, 32 x 8320
+    185 -> 104 / 153 -> 87 / 106 -> 67, 64 x 8320 212 -> 159 / 174 -> 130 / 117 -> 95; losing 4096 8 x 12288 178 -> 85 / 162 -> 74 /
+    112 -> 64, 32 x 12288 199 -> 150 / 172 -> 129 / 117 -> 98.  Whole, where the line is on the safe side: 64 x 4224 112 -> 95 / 94 -> 81 /
+    64 -> 62; and where split is slower: 64 x 2176 61 -> 63 / 52 -> 55 / 37 -> 43, 128 x 8320 252 -> 269 / 209 -> 213 / 142 -> 153, losing
+    4096 64 x 12288 227 -> 254 / 193 -> 212 / 133 -> 150.  Of few kept rows one workgroup is done as soon: 16 segments of 4100 cut to
+    1100 58 -> 67, 8 of 4096 cut to 2048 72 -> 67 / 67 -> 60 / 53 -> 55; of 64 features 16 of 2860 cut to 2560 41 -> 37.
+    Not while a graph is captured: the launches' table may be uploaded for the first time."""
+    return ((2560 if head_dim == 64 else 2048) <= kept and longest <= 32768 and head_dim in (64, 96, 128)
+            and rows * (5 if spill < 512 else 8) < 360 * longest - 300000 and not torch.cuda.is_current_stream_capturing())
 
 
 def wide_group(segs: int, longest: int) -> bool:
     """Whether a budget that one layer's ``segs`` segments share is selected by a workgroup per segment (seven launches) instead of
     one in all, which reads them one after the other, five times over.  Measured, one -> wide, layers x groups of 8 segments: 5 x 2
-    of 2400 rows 99 -> 36 us, of 600 64 -> 27, 36 x 8 of 2400 234 -> 101, 36 x 1 of 300 73 -> 27; below the line the launches cost a
-    caller that is not ahead of the device what they save."""
+    of 2400 rows 99 -> 36 us, of 1100 85 -> 30, 36 x 8 of 2400 234 -> 101, 36 x 1 of 1100 85 -> 31.  The launches take 18 us of the host
+    instead of 4, whatever the size.  Below the line that is kept for the host: 5 x 2 of 600 rows 66 -> 27 us of the device, 36 x 1
+    of 300 73 -> 27, which a caller that is behind the device gains and one that the host holds up does not."""
     return segs * longest >= 8192
 
 
