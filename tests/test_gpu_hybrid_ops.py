@@ -296,6 +296,28 @@ def test_experts_with_row_counts_at_the_edges_of_tiles():
     close(y, want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each: 2^-8 of the largest each, and slack for their spread
 
 
+@pytest.mark.parametrize("ff,width", [(352, 640), (704, 352)])
+def test_experts_whose_steps_go_round_the_buffers(ff, width):
+    """Prompt-sized products of 12, 20 and 22 steps of 32 k: the five operand buffers are filled anew two to four times while
+    wavefronts with none to four blocks of 32 rows read them, in full tiles and in tiles of every number of blocks."""
+    counts = [0, 1, 33, 65, 97, 129, 161, 193, 225, 256, 257, 545]
+    E, T, wp, fp = len(counts), sum(counts), ops.padded(width), ops.padded(ff)
+    assert T >= 96 * E and {wp // 32, fp // 32} in ({20, 12}, {12, 22})
+    x, up, down = torch.zeros(T, wp), torch.zeros(E, fp, wp), torch.zeros(E, wp, fp)
+    x[:, :width] = rnd(T, width, seed=1)
+    up[:, :ff, :width] = rnd(E, ff, width, seed=2) * width ** -0.5
+    down[:, :width, :ff] = rnd(E, width, ff, seed=3) * ff ** -0.5
+    x, up, down = (t.to(torch.bfloat16) for t in (x, up, down))
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=torch.Generator().manual_seed(4))]
+    want = torch.empty(T, width, dtype=torch.float64)
+    for e in range(E):
+        want[ids == e] = ref.expert(x[ids == e].double()[:, :width], up[e].double()[:ff, :width], down[e].double()[:width, :ff])
+    args = (x.to(DEV), ids[:, None].int().to(DEV), ops.pack_matrix(up).contiguous().to(DEV), ops.pack_matrix(down).contiguous().to(DEV), width)
+    first = ops.experts(*args)
+    close(first[:, :width], want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each: 2^-8 of the largest each, and slack for their spread
+    assert all(torch.equal(ops.experts(*args), first) for _ in range(3))     # a buffer read too early or too late does not repeat itself
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("at", [3, 37, 64, 129])
 def test_values_that_are_not_finite_stay_out_of_rows_that_do_not_see_them(bad, at):
