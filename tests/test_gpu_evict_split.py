@@ -224,3 +224,23 @@ def test_pairs_with_chunks_of_their_own(on_host):
     (2688, 8, 2559, 128, 64, False), (2688, 8, 2560, 128, 64, True), (32769, 8, 32000, 512, 128, False), (8320, 8, 8192, 128, 256, False)])
 def test_where_rows_are_moved_by_several_workgroups(longest, segments, kept, spill, D, split):
     assert cache_utils.split_evict(longest, segments * longest, kept, spill, D) is split
+
+
+@pytest.mark.parametrize("entry", ["split", "split_listed", "host_layers"])
+@pytest.mark.parametrize("spill", [200, 512])
+def test_entry_points_that_give_every_pair_room_for_the_longest_segment(entry, spill):
+    lib, n, M = _lib.load(), 3300, 3100
+    keep = np.sort(np.random.default_rng(7).choice(n, size=M, replace=False))
+    cache, held = _filled(TrimKVCache, 2, 1, 2, n, 96, torch.float16, torch.float32, keep)
+    need = lib.trimkv_evict_split_workspace(4, n, 96, spill)
+    ws = torch.full((need + 4096,), 9, dtype=torch.uint8, device=DEV)
+    work = torch.tensor([2, 0, 3, 1], dtype=torch.int32, device=DEV)
+    shape = (2, 2, 96, _lib.F16, _lib.F32, M, None, 0, 0, n + 1, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST, 0, n, spill)
+    room = (ws.data_ptr(), need, _lib.current_stream(ws.device))
+    if entry == "host_layers":
+        _lib.check(lib.trimkv_evict_host_layers(cache._host_table([0, 1]).ctypes.data, *shape, *room), entry)
+    else:
+        listed = (work.data_ptr(), 4) if entry == "split_listed" else (None, 0)
+        _lib.check(lib.trimkv_evict_split(cache._device_tables([0, 1])["slabs"].data_ptr(), *shape, *listed, *room), entry)
+    assert (ws[need:] == 9).all()
+    _check(cache, held, keep, entry)

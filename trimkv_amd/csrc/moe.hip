@@ -220,7 +220,7 @@ __global__ __launch_bounds__(KS * 64) void grouped_skinny_kernel(GroupedArgs a) 
 // tiles of 32x32x16 MFMAs.  Steps of 32 k rotate through five LDS buffers filled by LDS-direct loads, four steps ahead: the
 // weights lane-linear as they lie in memory, token rows gathered, the 16-byte piece c of row r at c ^ ((r / 4) % 4), so that
 // the rows of a fragment read fall on different banks.
-// What bounds it is the way of the operands into LDS, not the matrix cores (busy 66 % of a compute unit's time): with the loads
+// What bounds it is the way of the operands into LDS, not the matrix cores (busy 61 % of a compute unit's time): with the loads
 // taken out the two products of 8192 tokens x 4 of 32 experts (4096 x 4608) take 1.93 ms, with loads that always hit 2.28 ms, as
 // it is 2.64 ms.  Reads and requests one by one between the products, four steps ahead, rows that are not there not multiplied
 // and equal shares for the XCDs: 2.76 -> 2.64 ms.  Two buffers of 64 k were slower (2.88 ms), four wavefronts of 128 x 128 outputs
