@@ -675,6 +675,20 @@ int trimkv_qk_norm_rope(const void* q, int64_t q_tok_stride, const void* k, int6
 int trimkv_silu_mul(const void* gate, int64_t gate_stride, const void* up, int64_t up_stride, void* out,
                     int ntok, int inter, int dtype, void* stream);
 
+/*
+ * trimkv_linear_rows -- out[m][n] = round(sum_k x[m][k] w[n][k] + bias[n]): a linear layer (w [n][k] as nn.Linear keeps it, bias
+ * [n] optional) over 1 .. 64 rows, the tokens of a decode step.  Sums are fp32 in an order that depends on the sizes only.
+ * trimkv_linear_rows_silu -- w [2 inter][k], bias [2 inter] optional: the first inter rows are the gate, the others the up
+ * matrix of a gated feed-forward; out[m][i] = silu(gate) * up [rows][inter].  round_all: the two products and silu(gate) are
+ * rounded to `dtype` first, as modules round them (Qwen3MLP :121); else only the result is.
+ * dtype bf16 or fp16; k a multiple of 64, strides (in elements, at most 2^24) of x and w multiples of 8, x and w 16-byte
+ * aligned.  libtrimkv_hybrid.so holds both as well.
+ */
+int trimkv_linear_rows(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, void* out, int64_t out_stride,
+                       int rows, int n, int k, int dtype, void* stream);
+int trimkv_linear_rows_silu(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, void* out, int64_t out_stride,
+                            int rows, int inter, int k, int round_all, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

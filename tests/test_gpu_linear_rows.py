@@ -1,0 +1,135 @@
+"""trimkv_linear_rows and trimkv_linear_rows_silu (a linear layer over the rows of a decode step) against 64-bit products.
+
+Bounds: fp32 sums of k products err by at most about k 2^-24 sum |x w| (any order), the result is rounded once (half a unit in the
+last place, 2^-9 of the value in bf16 and 2^-12 in fp16; twice that here, for values that straddle)."""
+import ctypes
+
+import pytest
+import torch
+from torch import nn
+
+from trimkv_amd import _lib, linear
+
+DEV = "cuda:0"
+EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _operands(rows, n, k, dtype, seed=0):
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    made = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).to(dtype)
+    return made(rows, k), made(n, k) * 0.1, made(n)
+
+
+def _check(got, x, w, bias, dtype):
+    exact, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if bias is not None:
+        exact = exact + bias.double()
+    bound = EPS[dtype] * exact.abs() + x.shape[1] * 2.0 ** -23 * size + 2.0 ** -24
+    err = (got.double() - exact).abs()
+    assert (err <= bound).all(), (float((err - bound).max()), (err > bound).nonzero()[:4].tolist())
+
+
+# rows: every number of row groups and their edges; n: ends of 16-row blocks and, from 4608 on, every number of blocks per tile and more
+# tiles than workgroups; k: fewer steps than wavefronts, numbers that do not divide among them
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 64), (1, 15, 128), (7, 16, 192), (8, 17, 320), (9, 40, 64), (16, 100, 1024), (17, 33, 448), (31, 2048, 512), (32, 18, 64), (33, 1000, 704),
+                                      (63, 47, 576), (64, 4096, 256), (1, 4608, 128), (16, 4612, 192), (32, 12288, 64), (5, 12291, 64), (64, 12280, 128), (64, 24576, 64),
+                                      (50, 24600, 128), (8, 70001, 64), (16, 50000, 64), (64, 50002, 64)])
+def test_linear_rows_matches_the_product(rows, n, k, dtype):
+    x, w, bias = _operands(rows, n, k, dtype, rows + n + k)
+    got = linear.linear(x, w)
+    _check(got, x, w, None, dtype)
+    assert torch.equal(got, linear.linear(x, w))                   # the order of the sums is fixed
+    _check(linear.linear(x, w, bias), x, w, bias, dtype)
+    assert torch.equal(got, linear.linear(x, w, library="hybrid"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("round_all", [True, False])
+@pytest.mark.parametrize("rows,inter,k", [(1, 1, 64), (3, 17, 128), (8, 100, 192), (16, 2049, 64), (16, 6144, 128), (32, 12288, 64), (40, 40, 576), (64, 1000, 64), (64, 6144, 128), (61, 12288, 64), (64, 20000, 64)])
+def test_linear_rows_silu_matches_the_two_products(rows, inter, k, round_all, dtype):
+    x, w, bias = _operands(rows, 2 * inter, k, dtype, rows + inter)
+    for b in (None, bias):
+        got = linear.silu_product(x, w, b, round_all)
+        exact = x.double() @ w.double().T + (0 if b is None else b.double())
+        size = (x.double().abs() @ w.double().abs().T) * (k * 2.0 ** -23)
+        (g, u), (dg, du) = exact.chunk(2, -1), size.chunk(2, -1)
+        act = torch.nn.functional.silu(g)
+        # silu's slope is at most 1.1; g, u, silu(g) and the result are rounded (round_all) or the result alone
+        dg, du = dg + EPS[dtype] * g.abs() * round_all, du + EPS[dtype] * u.abs() * round_all
+        bound = 1.1 * dg * (u.abs() + du) + act.abs() * du + EPS[dtype] * (1 + round_all) * (act * u).abs() + 1e-5 * (act * u).abs() + 2.0 ** -24
+        err = (got.double() - act * u).abs()
+        assert (err <= bound).all(), float((err - bound).max())
+
+
+@pytest.mark.gpu
+def test_rows_that_are_slices_and_what_goes_to_the_general_product():
+    x, w, bias = _operands(20, 300, 256, torch.bfloat16, 5)
+    wide = torch.zeros(20, 1, 320, dtype=torch.bfloat16, device=DEV)
+    wide[..., 64:] = x[:, None]
+    big = torch.zeros(340, 264, dtype=torch.bfloat16, device=DEV)
+    big[40:, 8:] = w
+    want = linear.linear(x, w, bias)
+    assert torch.equal(linear.linear(wide[..., 64:], big[40:, 8:], bias)[:, 0], want)
+    takes = lambda *a: linear._rows(*a) is not None
+    assert takes(x, w, bias) and takes(wide[..., 64:], big[40:, 8:], bias)
+    assert not takes(wide[..., 60:], big[40:, 4:], None)                    # 260 features, and not 16-byte aligned
+    assert not takes(wide[:, 0, 4:260], w, None)                            # 8 bytes off
+    assert not takes(torch.cat([x] * 4), w, None)                           # 80 rows
+    assert not takes(x[:0], w, None) and not takes(x.float(), w.float(), None) and not takes(x, w.half(), None)
+    assert not takes(x, w.t().contiguous().t(), None)                       # columns are contiguous
+    for args in ((wide[:, 0, 4:260], w), (torch.cat([x] * 4), w), (x[:0], w), (x, w.t().contiguous().t()), (x.float(), w.float())):
+        assert linear.linear(*args).shape == (args[0].shape[0], 300)
+    with torch.enable_grad():
+        p = nn.Parameter(w.clone())
+        assert not takes(x, p, None)
+        linear.linear(x, p).float().sum().backward()
+        assert p.grad is not None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert linear.linear(x, w).dtype == torch.float16
+
+
+@pytest.mark.gpu
+def test_linear_rows_on_a_stream_and_replayed_from_a_graph():
+    x, w, _ = _operands(16, 4608, 256, torch.bfloat16, 9)
+    want = linear.linear(x, w)
+    gate = linear.silu_product(x, w)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out, act = linear.linear(x, w), linear.silu_product(x, w)
+    for i in range(3):
+        out.zero_(), act.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(act, gate), i
+
+
+def test_bad_arguments_are_refused_without_a_launch():
+    lib, one = _lib.load(), ctypes.c_void_p(16)
+    call = lambda rows=4, n=16, k=64, xs=64, ws=64, os=16, x=one, w=one, dt=_lib.BF16: lib.trimkv_linear_rows(x, xs, w, ws, None, one, os, rows, n, k, dt, None)
+    assert call(rows=65) == -2 and call(rows=0) == -2 and call(n=0) == -2 and call(k=96) == -2 and call(k=0) == -2
+    assert call(xs=60) == -2 and call(ws=68) == -2 and call(os=8) == -2 and call(xs=1 << 25) == -2 and call(w=ctypes.c_void_p(24)) == -2
+    assert call(x=None) == -1 and call(dt=_lib.F32) == -3
+    assert lib.trimkv_linear_rows_silu(one, 64, one, 64, None, one, 8, 4, 16, 64, 1, _lib.BF16, None) == -2
+
+
+def test_modules_that_somebody_hooked_wrapped_or_replaced_are_called():
+    lin, x = nn.Linear(8, 4), torch.randn(2, 8)
+    assert torch.equal(linear.run(lin, x), lin(x))
+    seen = []
+    hook = lin.register_forward_hook(lambda m, a, out: seen.append(out.shape) or out + 1)
+    assert torch.equal(linear.run(lin, x), nn.functional.linear(x, lin.weight, lin.bias) + 1) and len(seen) == 1
+    hook.remove()
+    lin.forward = lambda y: y.sum()
+    assert linear.run(lin, x) == x.sum()
+
+    class Doubled(nn.Linear):
+        def forward(self, y):
+            return 2 * super().forward(y)
+    twice = Doubled(8, 4)
+    assert torch.equal(linear.run(twice, x), 2 * nn.functional.linear(x, twice.weight, twice.bias))

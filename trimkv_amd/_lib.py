@@ -37,6 +37,8 @@ SIGNATURES = {
     "trimkv_qk_norm_rope": (_i, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _i,
                                  _i, _i, _i, _i, _i, _i, _f, _i, _p]),
     "trimkv_silu_mul": (_i, [_p, _i64, _p, _i64, _p, _i, _i, _i, _p]),
+    "trimkv_linear_rows": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p]),
+    "trimkv_linear_rows_silu": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
     "trimkv_gate_hidden_packed": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
     "trimkv_gate_hidden_swiglu_packed": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
     "trimkv_append_gated": (_i, [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _i64, _i64,
@@ -126,6 +128,9 @@ HYBRID_SIGNATURES = {
     },
 }
 
+# entry points of trimkv_hip.h that another library holds as well
+SHARED = {"hybrid": ("trimkv_linear_rows", "trimkv_linear_rows_silu")}
+
 _lib = None
 _hybrid = {}
 
@@ -158,7 +163,7 @@ def load_hybrid(name: str = "hybrid"):
             f"{path} is missing: build it with `python -m trimkv_amd.build {name}` (hipcc, gfx950). "
             "There is no CPU fallback.")
     lib = C.CDLL(path)
-    for fn_name, (res, args) in HYBRID_SIGNATURES[name].items():
+    for fn_name, (res, args) in {**HYBRID_SIGNATURES[name], **{n: SIGNATURES[n] for n in SHARED.get(name, ())}}.items():
         fn = getattr(lib, fn_name)
         fn.restype = res
         fn.argtypes = args

@@ -1,0 +1,272 @@
+// Products of a few rows with a large matrix (the tokens of a decode step and a linear layer) -- gfx950.
+//
+//   trimkv_linear_rows        out[m][n] = sum_k x[m][k] w[n][k] (+ bias[n]), up to 64 rows x, w as nn.Linear keeps it
+//   trimkv_linear_rows_silu   out[m][n] = silu(gate) * up with gate = x . w[n] and up = x . w[inter + n]: a gated feed-forward's
+//                             first two matrices and the product of their outputs
+//
+// 16-bit operands, fp32 sums in a fixed order.
+//
+// What bounds it: the stream of weights, each byte of which is used for at most 64 rows, and on its way the rate at which one
+// compute unit takes operands in (57-60 GB/s measured, whatever the mix of w and x and however much is in flight), because every
+// workgroup also reads all of x.  Hence
+//  * operands travel through LDS.  In operand layout neighbouring lanes hold neighbouring rows, and a load of 64 lanes in 64 (or
+//    8 x 8) different lines is served one lane at a time: 16 B/clk per compute unit.  LDS-direct loads whose lanes run along
+//    the rows (8 rows x 128 bytes each) take in 28 B/clk; ds_read_b128 does the regrouping.  12288 x 2048 with 16 rows: 19 us
+//    with operand-layout loads, 11.4 here; 4096 x 4096 with 64 rows: 23.4 and 13.7;
+//  * a workgroup takes 16 NT rows of w, with NT chosen so that the busiest compute unit takes in least (rows_plan below);
+//  * the wavefronts of a workgroup take turns on k, 64 elements at a time, each with a ring of its own, so that the main loop
+//    has no barrier; their sums meet in LDS at the end of a tile while the next tile's loads are already under way.
+//
+// Measured in a graph of launches over matrices that no cache holds, us here | the vendor library's product:
+//            n x k      1 row        16 rows      32 rows      64 rows
+//      2048 x 2048    5.0 | 10.9    5.5 | 11.1    6.2 | 11.2    8.2 | 11.8
+//     12288 x 2048   11.7 | 16.6   11.4 | 16.7   12.2 | 16.9   14.8 | 18.2
+//      2048 x 6144    8.7 | 11.1   10.3 | 11.3   13.4 | 16.6   18.3 | 19.5
+//      4096 x 4096    8.3 | 15.7    9.3 | 15.5   10.4 | 13.4   13.7 | 15.2
+//     10240 x 4096   16.3 | 26.6   16.6 | 27.8   18.3 | 23.6   22.5 | 29.6
+//     24576 x 4096   34.4 | 45.2   35.5 | 45.5   36.8 | 50.2   42.1 | 50.1
+//      4096 x 12288  18.9 | 23.1   21.1 | 23.5   26.8 | 29.1   36.1 | 39.1
+#include "common.hip.h"
+
+namespace trimkv {
+
+typedef __bf16 lr_bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 lr_f16x8 __attribute__((ext_vector_type(8)));
+typedef float lr_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t lr_u32x4 __attribute__((ext_vector_type(4)));
+#define LR_LDS __attribute__((address_space(3)))
+
+struct LinearRowsArgs {
+    const uint16_t* x; int64_t x_stride;
+    const uint16_t* w; int64_t w_stride;
+    const uint16_t* bias;
+    uint16_t* out; int64_t out_stride;
+    int m, n, k;        // n: columns of out
+    int vec;            // four columns of out can be stored at once
+    int round_all;      // silu: the two products and silu(gate) are rounded before they are used, as modules do
+};
+
+template <bool F16>
+__device__ __forceinline__ lr_f32x4 lr_mfma(lr_u32x4 a, lr_u32x4 b, lr_f32x4 c) {
+    if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lr_f16x8, a), __builtin_bit_cast(lr_f16x8, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lr_bf16x8, a), __builtin_bit_cast(lr_bf16x8, b), c, 0, 0, 0);
+}
+template <bool F16> __device__ __forceinline__ float lr_load(uint16_t b) { return F16 ? f16_bits_to_f32(b) : bf16_bits_to_f32(b); }
+template <bool F16> __device__ __forceinline__ uint16_t lr_bits(float f) { return F16 ? f32_to_f16_bits(f) : f32_to_bf16_bits(f); }
+
+// 64 lanes x 16 bytes from base + off to LDS at lds + 16 * lane (base and lds wavefront-uniform).  The compiler neither counts
+// nor waits for these loads: whoever reads the LDS waits with an explicit s_waitcnt first.  ONCE: nobody reads the line again.
+template <bool ONCE>
+__device__ __forceinline__ void lr_load_to_lds(const uint16_t* base, uint32_t off, uint32_t lds) {
+    uint32_t saved;
+    if constexpr (ONCE)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved) : "v"(off), "s"(base), "s"(lds) : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                     : "=&s"(saved) : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+
+// XG groups of 8 rows of x, NT blocks of 16 rows of w (SILU: NT / 2 of gate, NT / 2 of up), W wavefronts, D steps of 64 elements
+// of k in flight per wavefront.  A step in LDS: row r holds its eight 16-byte pieces rotated by r / 2, which spreads the 16 rows of
+// an operand read over all banks (the rotation is in the lanes' source addresses).
+template <bool F16, bool SILU, int XG, int NT, int W, int D>
+__global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
+    constexpr int MT = (XG + 1) / 2, L = 2 * NT + XG, STEP = L * 1024, U = NT * MT, NB = SILU ? NT / 2 : NT;
+    static_assert((D - 1) * L < 64, "the wait counts at most 63 loads");
+    __shared__ __attribute__((aligned(1024))) char ring[W * D * STEP];
+    __shared__ lr_f32x4 part[U * (W - 1)][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+    const uint32_t ring_at = (uint32_t)(uintptr_t)(LR_LDS char*)ring + wave * D * STEP;
+    const char* mine = ring + wave * D * STEP;
+    // a load brings rows 8 j + lane / 8 of a block, position lane % 8; rows that are not there repeat the last one
+    uint32_t w_off[2], x_off[XG];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = 8 * j + (lane >> 3);
+        w_off[j] = (uint32_t)(min(row, a.n - 1) * a.w_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < XG; ++j) {
+        const int row = 8 * j + (lane >> 3);
+        x_off[j] = (uint32_t)(min(row, a.m - 1) * a.x_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
+    }
+    const int steps = a.k >> 6, first = min(wave, steps - 1), per_tile = (steps - wave + W - 1) / W, tiles = (a.n + 16 * NB - 1) / (16 * NB);
+    // the first column of block b of a tile: the last block of out is moved back so that all its rows exist
+    auto block_at = [&](int tile, int b) __attribute__((always_inline)) { return min((tile * NB + b % NB) * 16, max(a.n - 16, 0)); };
+    int ask_tile = blockIdx.x, ask_step = first, ask_slot = 0;
+    auto request = [&]() __attribute__((always_inline)) {
+        const uint32_t to = ring_at + ask_slot * STEP;
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+            const uint16_t* from = a.w + (int64_t)(block_at(ask_tile, b) + (SILU && b >= NB ? a.n : 0)) * a.w_stride + ask_step * 64;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) lr_load_to_lds<true>(from, w_off[j], to + (2 * b + j) * 1024);
+        }
+#pragma unroll
+        for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (2 * NT + j) * 1024);
+        ask_step += W;
+        if (ask_step >= steps) {        // behind the last tile: its steps again, never read
+            ask_step = first;
+            ask_tile = min(ask_tile + (int)gridDim.x, tiles - 1);
+        }
+        ask_slot = ask_slot + 1 == D ? 0 : ask_slot + 1;
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) request();
+    lr_f32x4 acc[U];
+    int slot = 0;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[u] = lr_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < per_tile; ++s) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * L) : "memory");
+            const char* p = mine + slot * STEP;
+            lr_u32x4 wf[2][NT], xf[2][MT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int b = 0; b < NT; ++b) wf[h][b] = *(const lr_u32x4*)(p + (b * 16 + r) * 128 + ((h * 4 + g + (r >> 1)) & 7) * 16);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const int row = XG == 1 ? r & 7 : t * 16 + r;       // 8 rows: columns 8 .. 15 repeat them
+                    xf[h][t] = *(const lr_u32x4*)(p + (NT * 16 + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // the step has been read: its room is free
+            __builtin_amdgcn_sched_barrier(0);
+            request();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int b = 0; b < NT; ++b)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) acc[b * MT + t] = lr_mfma<F16>(wf[h][b], xf[h][t], acc[b * MT + t]);
+            slot = slot + 1 == D ? 0 : slot + 1;
+        }
+        // the sums of 16 columns x 16 rows go to the wavefront they belong to (gate and up of a column to the same one)
+        auto owner = [](int u) { return (u / MT % NB * MT + u % MT) % W; };
+        if (tile != (int)blockIdx.x) asm volatile("s_barrier" ::: "memory");        // the sums of the tile before have been read
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (owner(u) != wave) part[u * (W - 1) + (wave - owner(u) + W) % W - 1][lane] = acc[u];
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        auto total = [&](int u) __attribute__((always_inline)) {
+            lr_f32x4 f = acc[u];
+#pragma unroll
+            for (int o = 0; o < W - 1; ++o) f += part[u * (W - 1) + o][lane];
+            return f;
+        };
+#pragma unroll
+        for (int u = 0; u < NB * MT; ++u) {
+            if (owner(u) != wave) continue;
+            const int m = u % MT * 16 + r, n = block_at(tile, u / MT) + 4 * g;      // this lane: columns n .. n + 3 of row m
+            if (m >= a.m) continue;
+            lr_f32x4 f = total(u);
+            uint16_t v[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (a.bias && n + c < a.n) f[c] += lr_load<F16>(a.bias[n + c]);
+            if constexpr (SILU) {
+                lr_f32x4 e = total(U / 2 + u);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (a.bias && n + c < a.n) e[c] += lr_load<F16>(a.bias[a.n + n + c]);
+                    if (a.round_all) {
+                        const float x = lr_load<F16>(lr_bits<F16>(f[c]));
+                        v[c] = lr_bits<F16>(lr_load<F16>(lr_bits<F16>(x / (1.0f + expf(-x)))) * lr_load<F16>(lr_bits<F16>(e[c])));
+                    } else v[c] = lr_bits<F16>(f[c] / (1.0f + expf(-f[c])) * e[c]);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[c] = lr_bits<F16>(f[c]);
+            }
+            uint16_t* o = a.out + (int64_t)m * a.out_stride + n;
+            if (a.vec) *(uint2*)o = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
+            else
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (n + c < a.n) o[c] = v[c];
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // loads into LDS that nobody reads have landed
+}
+
+constexpr int LR_CUS = 256;
+
+// Blocks of 16 rows of w per tile.  A compute unit that runs `rounds` tiles takes in rounds * (rows of w + rows of x) * k elements;
+// the least of that is the fastest (n x k = 12288 x 2048, 16 rows: one block 3 x 32, three blocks 1 x 64: 13.6 and 11.4 us;
+// 4608 x 2048, 64 rows: 2 x 80, 96, 112: 13.1, 10.6, 12.5).  Among equals the smaller one.
+static int rows_plan(int n, int x_rows, bool silu) {
+    static const int plain[] = {1, 2, 3, 6}, paired[] = {2, 4, 6};
+    const int* sizes = silu ? paired : plain;
+    int best = sizes[0];
+    int64_t least = INT64_MAX;
+    for (int i = 0; i < (silu ? 3 : 4); ++i) {
+        const int nt = sizes[i];
+        if (nt == 6 && x_rows < 64) continue;       // fewer rows of x: not faster than two or three blocks at any size measured
+        const int64_t cols = 16 * (silu ? nt / 2 : nt), tiles = (n + cols - 1) / cols, cost = (tiles + LR_CUS - 1) / LR_CUS * (16 * nt + x_rows);
+        if (cost < least) { least = cost; best = nt; }
+    }
+    return best;
+}
+
+template <bool F16, bool SILU, int XG, int NT, int W, int D>
+static void rows_launch(const LinearRowsArgs& a, hipStream_t s) {
+    constexpr int NB = SILU ? NT / 2 : NT, LDS = W * D * (2 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024;
+    static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
+    const int tiles = (a.n + 16 * NB - 1) / (16 * NB), most = LR_CUS * (160 * 1024 / LDS);
+    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, XG, NT, W, D>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
+}
+// wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 6 over the shapes above
+template <bool F16, int XG>
+static void rows_by_blocks(const LinearRowsArgs& a, bool silu, hipStream_t s) {
+    const int nt = rows_plan(a.n, 8 * XG, silu);
+    if constexpr (XG == 8) {
+        if (silu && nt == 6) return rows_launch<F16, true, 8, 6, 4, 1>(a, s);
+        if (silu && nt == 4) return rows_launch<F16, true, 8, 4, 2, 2>(a, s);
+        if (!silu && nt == 6) return rows_launch<F16, false, 8, 6, 4, 1>(a, s);
+    } else if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, 2>(a, s);
+    if (silu) rows_launch<F16, true, XG, 2, 4, 2>(a, s);
+    else if (nt == 1) rows_launch<F16, false, XG, 1, 4, XG < 4 ? 3 : 2>(a, s);
+    else if (nt == 2) rows_launch<F16, false, XG, 2, 4, 2>(a, s);
+    else rows_launch<F16, false, XG, 3, 4, 2>(a, s);
+}
+template <bool F16>
+static void rows_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
+    if (a.m <= 8) rows_by_blocks<F16, 1>(a, silu, s);
+    else if (a.m <= 16) rows_by_blocks<F16, 2>(a, silu, s);
+    else if (a.m <= 32) rows_by_blocks<F16, 4>(a, silu, s);
+    else rows_by_blocks<F16, 8>(a, silu, s);
+}
+
+}  // namespace trimkv
+
+using namespace trimkv;
+
+static int rows_check_and_launch(const char* fn, LinearRowsArgs a, bool silu, int dtype, void* stream) {
+    if (!a.x || !a.w || !a.out) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (dtype != TRIMKV_BF16 && dtype != TRIMKV_F16) return fail(TRIMKV_ERR_DTYPE, "%s: bf16 or fp16 only (dtype=%d)", fn, dtype);
+    if (a.m <= 0 || a.m > 64 || a.n <= 0 || a.n > (1 << 29) || a.k <= 0 || a.k % 64)
+        return fail(TRIMKV_ERR_SHAPE, "%s: bad sizes rows=%d (1 .. 64) n=%d k=%d (a multiple of 64)", fn, a.m, a.n, a.k);
+    if (a.x_stride < a.k || a.w_stride < a.k || a.out_stride < a.n || a.x_stride % 8 || a.w_stride % 8 || a.x_stride > (1 << 24) || a.w_stride > (1 << 24))
+        return fail(TRIMKV_ERR_SHAPE, "%s: strides %lld %lld (>= k, multiples of 8, at most 2^24) %lld (>= n)", fn, (long long)a.x_stride, (long long)a.w_stride, (long long)a.out_stride);
+    if (((uintptr_t)a.x | (uintptr_t)a.w) & 15) return fail(TRIMKV_ERR_SHAPE, "%s: x and w must be 16-byte aligned", fn);
+    a.vec = a.n % 4 == 0 && a.out_stride % 4 == 0 && !((uintptr_t)a.out & 7);
+    if (dtype == TRIMKV_F16) rows_by_rows<true>(a, silu, (hipStream_t)stream);
+    else rows_by_rows<false>(a, silu, (hipStream_t)stream);
+    return launch_status(fn);
+}
+
+extern "C" int trimkv_linear_rows(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, void* out, int64_t out_stride,
+                                  int rows, int n, int k, int dtype, void* stream) {
+    return rows_check_and_launch("trimkv_linear_rows",
+                                 LinearRowsArgs{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, n, k, 0, 0}, false, dtype, stream);
+}
+
+extern "C" int trimkv_linear_rows_silu(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, void* out, int64_t out_stride,
+                                       int rows, int inter, int k, int round_all, int dtype, void* stream) {
+    return rows_check_and_launch("trimkv_linear_rows_silu",
+                                 LinearRowsArgs{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, inter, k, 0, round_all}, true, dtype, stream);
+}

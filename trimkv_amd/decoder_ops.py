@@ -11,7 +11,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import _lib
+from . import _lib, linear
 
 enabled = True
 # Bumped whenever the decoders move parameters into another buffer (FusedRows in qwen3.py).  A captured graph holds the
@@ -34,6 +34,11 @@ def usable(*tensors: Optional[torch.Tensor]) -> bool:
         if t.dtype != first.dtype or t.device != first.device or (grad and t.requires_grad):
             return False
     return True
+
+
+def run_linear(module: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``module(x)``, the products of a decode step on trimkv_linear_rows."""
+    return linear.run(module, x) if enabled else module(x)
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None):

@@ -18,9 +18,9 @@ from typing import Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 import torch
 from torch import nn
-import torch.nn.functional as F
 
 from . import _lib, hybrid_ops as ops
+from .linear import linear
 from .generation import GreedyGeneration
 from .hybrid_cache import HybridCache
 
@@ -126,7 +126,7 @@ class PackedLinear(nn.Module):
         return [self.offsets[n][0] for n in names]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight)
+        return linear(x, self.weight, library="hybrid")
 
 
 class WindowAttention(nn.Module):
@@ -451,6 +451,6 @@ class HybridForCausalLM(GreedyGeneration, nn.Module):
         else:
             shape = (-1,) if rows is not None or min(batch.lengths) != batch.max_len else (B, batch.max_len)
         h = ops.rms_rows(x, rows, self.model.norm, self.config.norm_eps, self.model.dtype)
-        logits = F.linear(h, self.model.embed if self.head is None else self.head)
+        logits = linear(h, self.model.embed if self.head is None else self.head, library="hybrid")
         logits = logits.float() if self.config.logit_softcap is None else ops.soft_cap(logits, self.config.logit_softcap)
         return SimpleNamespace(logits=logits.view(*shape, logits.shape[-1]), past_key_values=cache)

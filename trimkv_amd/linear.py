@@ -1,0 +1,86 @@
+"""Linear layers over the rows of a decode step on trimkv_linear_rows; everything else goes to ``F.linear``.
+
+Both give fp32 sums rounded once; the order of the sums differs.
+"""
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+from torch import nn
+import torch.nn.functional as F
+from torch.nn.modules import module as _module
+
+from . import _lib
+
+MAX_ROWS = 64      # rows that trimkv_linear_rows takes
+
+
+def _plain(*tensors: Optional[torch.Tensor]) -> bool:
+    """Ordinary tensors of one 16-bit dtype on the current GPU that nobody differentiates or casts."""
+    first = tensors[0]
+    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda"):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is None:
+            continue
+        if type(t) not in (torch.Tensor, nn.Parameter) or t.dtype != first.dtype or t.device != first.device or (grad and t.requires_grad):
+            return False
+    return first.device.index == torch.cuda.current_device()
+
+
+def _rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """x as [rows, k] the way trimkv_linear_rows reads it, or None where it does not take this product."""
+    k = x.shape[-1] if x.dim() else 0
+    if k == 0 or k % 64 or not 0 < x.numel() <= MAX_ROWS * k or not _plain(x, weight, bias):
+        return None
+    if weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0 or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 8 or weight.data_ptr() % 16:
+        return None
+    if bias is not None and (bias.shape != weight.shape[:1] or not bias.is_contiguous()):
+        return None
+    x2 = x if x.dim() == 2 else x.reshape(-1, k)
+    if x2.stride(1) != 1 or x2.data_ptr() % 16 or (x2.shape[0] > 1 and (x2.stride(0) < k or x2.stride(0) % 8)):
+        return None
+    return None if max(x2.stride(0), weight.stride(0)) > 1 << 24 else x2
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, library: Optional[str] = None) -> torch.Tensor:
+    """``F.linear(x, weight, bias)``.  ``library``: which one holds the kernel (a name of ``_lib.SHARED``; None: libtrimkv_hip.so)."""
+    x2 = _rows(x, weight, bias)
+    if x2 is None:
+        return F.linear(x, weight, bias)
+    rows, k = x2.shape
+    n = weight.shape[0]
+    out = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
+    lib = _lib.load() if library is None else _lib.load_hybrid(library)
+    rc = lib.trimkv_linear_rows(x2.data_ptr(), x2.stride(0) if rows > 1 else k, weight.data_ptr(), weight.stride(0), _lib.ptr(bias), out.data_ptr(), n, rows, n, k,
+                                _lib.dtype_code(x.dtype), _lib.current_stream(x.device))
+    if rc:
+        _lib.check(rc, "trimkv_linear_rows") if library is None else _lib.check_hybrid(rc, "trimkv_linear_rows", library)
+    return out
+
+
+def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, round_all: bool = True, library: Optional[str] = None) -> Optional[torch.Tensor]:
+    """``silu(x @ gate.T) * (x @ up.T)`` with ``weight`` = gate over up, in one launch; None where trimkv_linear_rows_silu does not take it."""
+    x2 = _rows(x, weight, bias)
+    if x2 is None or weight.shape[0] % 2:
+        return None
+    rows, k = x2.shape
+    inter = weight.shape[0] // 2
+    out = torch.empty(*x.shape[:-1], inter, dtype=x.dtype, device=x.device)
+    lib = _lib.load() if library is None else _lib.load_hybrid(library)
+    rc = lib.trimkv_linear_rows_silu(x2.data_ptr(), x2.stride(0) if rows > 1 else k, weight.data_ptr(), weight.stride(0), _lib.ptr(bias), out.data_ptr(), inter, rows, inter, k,
+                                     int(round_all), _lib.dtype_code(x.dtype), _lib.current_stream(x.device))
+    if rc:
+        _lib.check(rc, "trimkv_linear_rows_silu") if library is None else _lib.check_hybrid(rc, "trimkv_linear_rows_silu", library)
+    return out
+
+
+def run(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``module(x)``; an ``nn.Linear`` that nobody has hooked, wrapped or replaced goes to ``linear`` with its parameters."""
+    if (type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+            or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks
+            or "forward" in module.__dict__):
+        return module(x)
+    return linear(x, module.weight, module.bias)

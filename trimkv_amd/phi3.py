@@ -44,10 +44,10 @@ class Phi3MLP(nn.Module):
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gate, up = self.gate_up_proj(x).chunk(2, dim=-1)
+        gate, up = decoder_ops.run_linear(self.gate_up_proj, x).chunk(2, dim=-1)
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
-            return self.down_proj(decoder_ops.silu_mul(gate, up))
-        return self.down_proj(up * F.silu(gate))
+            return decoder_ops.run_linear(self.down_proj, decoder_ops.silu_mul(gate, up))
+        return decoder_ops.run_linear(self.down_proj, up * F.silu(gate))
 
 
 class TrimKVPhi3Attention(TrimKVQwen3Attention):
@@ -63,7 +63,7 @@ class TrimKVPhi3Attention(TrimKVQwen3Attention):
     def _projections(self, hidden_states: torch.Tensor):
         B, S, _ = hidden_states.shape
         d = self.head_dim
-        q, k, v = self.qkv_proj(hidden_states).split([self.num_heads * d, self.num_key_value_heads * d, self.num_key_value_heads * d], dim=-1)
+        q, k, v = decoder_ops.run_linear(self.qkv_proj, hidden_states).split([self.num_heads * d, self.num_key_value_heads * d, self.num_key_value_heads * d], dim=-1)
         shape = (B, S, -1, d)
         return q.view(shape), k.view(shape), v.view(shape)
 

@@ -22,7 +22,7 @@ import torch
 from torch import nn
 import torch.nn.functional as F
 
-from . import decoder_ops
+from . import decoder_ops, linear
 from .attn import get_attention_interface
 from .cache_utils import LazyLogBeta, TrimKVCache
 from .gate import RetentionGate, RetentionGate2, RetentionGate3
@@ -162,7 +162,7 @@ class FusedRows:
             bias = None
         elif bias is not None:
             bias = bias[:rows]
-        return F.linear(x, self.weight[:rows], bias).split(sizes, dim=-1)
+        return linear.linear(x, self.weight[:rows], bias).split(sizes, dim=-1)
 
 
 class MLP(nn.Module):
@@ -180,8 +180,8 @@ class MLP(nn.Module):
         both = fused(x)
         gate, up = both if both is not None else (self.gate_proj(x), self.up_proj(x))
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
-            return self.down_proj(decoder_ops.silu_mul(gate, up))
-        return self.down_proj(F.silu(gate) * up)
+            return decoder_ops.run_linear(self.down_proj, decoder_ops.silu_mul(gate, up))
+        return decoder_ops.run_linear(self.down_proj, F.silu(gate) * up)
 
 
 def rotary_tables(position_ids: torch.Tensor, head_dim: int, theta: float, dtype: torch.dtype,
@@ -387,7 +387,7 @@ class TrimKVQwen3Attention(nn.Module):
         out, _, _ = attend(self, q, k, v, attention_mask=attention_mask, retention_weights=retention, kv_positions=kv_positions,
                            offset=offset, dropout=0.0, scaling=self.scaling, sliding_window=None, is_causal=True,
                            flash_attn_kwargs=fa_kwargs)
-        return self.o_proj(out.reshape(B, S, -1).contiguous())
+        return decoder_ops.run_linear(self.o_proj, out.reshape(B, S, -1).contiguous())
 
 
 class TrimKVQwen3DecoderLayer(nn.Module):
@@ -516,4 +516,4 @@ class TrimKVQwen3ForCausalLM(GreedyGeneration, nn.Module):
         h = out.last_hidden_state
         if logits_to_keep:
             h = h[:, -logits_to_keep:]
-        return SimpleNamespace(logits=self.lm_head(h), past_key_values=out.past_key_values)
+        return SimpleNamespace(logits=decoder_ops.run_linear(self.lm_head, h), past_key_values=out.past_key_values)
