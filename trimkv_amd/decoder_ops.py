@@ -153,3 +153,11 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     _lib.check(rc, "trimkv_silu_mul")
     counts["silu_mul"] += 1
     return out
+
+
+def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``silu_mul`` of the two halves of ``x @ weight.T`` in the product's own launch (a decode step's rows), or None."""
+    out = linear.silu_product(x, weight, bias) if enabled else None
+    if out is not None:
+        counts["silu_mul"] += 1
+    return out

@@ -20,7 +20,7 @@ import torch
 from torch import nn
 
 from . import _lib, hybrid_ops as ops
-from .linear import linear
+from .linear import linear, silu_product
 from .generation import GreedyGeneration
 from .hybrid_cache import HybridCache
 
@@ -265,7 +265,9 @@ class DenseMLP(nn.Module):
         return {"gate": self.gate_up.section("gate"), "up": self.gate_up.section("up"), "down": self.down.weight}
 
     def forward(self, x, xh):
-        return self.down(ops.silu_gate(self.gate_up(xh[:, :self.width]), self.ff)), None
+        xh = xh[:, :self.width]
+        act = silu_product(xh, self.gate_up.weight, round_all=False, library="hybrid")
+        return self.down(ops.silu_gate(self.gate_up(xh), self.ff) if act is None else act), None
 
 
 MIXERS = {"attention": WindowAttention, "mlstm": MLSTM}

@@ -77,10 +77,13 @@ def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return out
 
 
+def untouched(module: nn.Module) -> bool:
+    """An ``nn.Linear`` that nobody has hooked, wrapped or replaced: its parameters say all that calling it does."""
+    return not (type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks
+                or "forward" in module.__dict__)
+
+
 def run(module: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """``module(x)``; an ``nn.Linear`` that nobody has hooked, wrapped or replaced goes to ``linear`` with its parameters."""
-    if (type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-            or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks
-            or "forward" in module.__dict__):
-        return module(x)
-    return linear(x, module.weight, module.bias)
+    """``module(x)``; an untouched ``nn.Linear`` goes to ``linear`` with its parameters."""
+    return linear(x, module.weight, module.bias) if untouched(module) else module(x)

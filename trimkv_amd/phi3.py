@@ -14,7 +14,7 @@ import torch
 from torch import nn
 import torch.nn.functional as F
 
-from . import decoder_ops
+from . import decoder_ops, linear
 from .qwen3 import (TrimKVQwen3Attention, TrimKVQwen3Config, TrimKVQwen3DecoderLayer, TrimKVQwen3ForCausalLM, TrimKVQwen3Model)
 
 
@@ -44,6 +44,10 @@ class Phi3MLP(nn.Module):
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if linear.untouched(self.gate_up_proj):
+            act = decoder_ops.silu_product(x, self.gate_up_proj.weight)
+            if act is not None:
+                return decoder_ops.run_linear(self.down_proj, act)
         gate, up = decoder_ops.run_linear(self.gate_up_proj, x).chunk(2, dim=-1)
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
             return decoder_ops.run_linear(self.down_proj, decoder_ops.silu_mul(gate, up))

@@ -146,15 +146,22 @@ class FusedRows:
                 lin.bias.data = self.bias[off:off + n]
             off += n
 
-    def __call__(self, x: torch.Tensor, first: Optional[int] = None):
-        """The outputs of the modules for ``x`` as slices of one product, or None when that cannot be done here (training,
-        CPU, fp32, differing input widths).  ``first``: only the leading ``first`` modules (a prefix of the buffer)."""
+    def _usable(self, x: torch.Tensor) -> bool:
+        """Whether these modules can be one product here (not in training, on the CPU, in fp32, with differing input widths);
+        if so, their parameters lie in the buffer."""
         if not decoder_ops.usable(x, *(lin.weight for lin in self.linears)):
-            return None
+            return False
         if any(lin.in_features != self.linears[0].in_features or (lin.bias is not None and lin.bias.dtype != x.dtype) for lin in self.linears):
-            return None
+            return False
         if not self._in_place():
             self._fuse()
+        return True
+
+    def __call__(self, x: torch.Tensor, first: Optional[int] = None):
+        """The outputs of the modules for ``x`` as slices of one product, or None when that cannot be done here.  ``first``: only
+        the leading ``first`` modules (a prefix of the buffer)."""
+        if not self._usable(x):
+            return None
         sizes = [lin.out_features for lin in self.linears[:first]]
         rows = sum(sizes)
         bias = self.bias
@@ -163,6 +170,13 @@ class FusedRows:
         elif bias is not None:
             bias = bias[:rows]
         return linear.linear(x, self.weight[:rows], bias).split(sizes, dim=-1)
+
+    def silu_product(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """``silu(gate(x)) * up(x)`` of two modules (gate, up) of one size in one launch, or None when that cannot be done here."""
+        gate, up = self.linears
+        if gate.out_features != up.out_features or not self._usable(x):
+            return None
+        return decoder_ops.silu_product(x, self.weight, self.bias)
 
 
 class MLP(nn.Module):
@@ -177,6 +191,9 @@ class MLP(nn.Module):
         fused = self.__dict__.get("_gate_up")
         if fused is None:
             fused = self.__dict__["_gate_up"] = FusedRows(self.gate_proj, self.up_proj)
+        act = fused.silu_product(x)
+        if act is not None:
+            return decoder_ops.run_linear(self.down_proj, act)
         both = fused(x)
         gate, up = both if both is not None else (self.gate_proj(x), self.up_proj(x))
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
