@@ -628,7 +628,7 @@ int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, i
  * `workspace`: at least trimkv_prefill_split_workspace(...) bytes, 16-byte aligned, contents of no meaning before and after.
  * trimkv_prefill_split_tiles: the split_tiles at which this is expected to be faster than one workgroup per query tile, or 0
  * where it is not.  uneven: 0 if the segments are about as long as the longest, whose length is max_len; else their mean length
- * in percent of it, or 1 if all that is known is that they differ much.
+ * in percent of it, or 1 if all that is known is that they differ much (of no consequence for these two kernels).
  * Returns TRIMKV_OK or a negative trimkv_status (as trimkv_prefill_attn; split_tiles <= 0 or a workspace that is too small).
  */
 int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven);
@@ -637,6 +637,20 @@ int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int64_t q_strid
                               const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
                               int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
                               int max_len, int split_tiles, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
+ * trimkv_prefill_attn_shares -- trimkv_prefill_attn for chunks of 64 queries and more with the key tiles of all query tiles cut
+ * into equal runs, one per compute unit, by lengths that are read on the device; what a run leaves unfinished (at most two query
+ * tiles, fp32) is merged by a second launch.  Same operands and results (up to the rounding of the merge).
+ * `workspace`: at least trimkv_prefill_shares_workspace(...) bytes, 16-byte aligned, contents of no meaning before and after.
+ * trimkv_prefill_equal_shares: 1 where this is expected to be the fastest of the three; arguments as trimkv_prefill_split_tiles.
+ */
+int trimkv_prefill_equal_shares(int batch, int kv_heads, int group, int q_len, int max_len, int uneven);
+int64_t trimkv_prefill_shares_workspace(int batch, int kv_heads, int group, int q_len);
+int trimkv_prefill_attn_shares(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+                               const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
+                               int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
+                               int max_len, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * trimkv_rmsnorm / trimkv_qk_norm_rope / trimkv_silu_mul -- the element-wise work of a decoder layer around the cache

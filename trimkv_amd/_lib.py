@@ -91,6 +91,9 @@ SIGNATURES = {
     "trimkv_prefill_split_tiles": (_i, [_i, _i, _i, _i, _i, _i]),
     "trimkv_prefill_split_workspace": (_i64, [_i, _i, _i, _i, _i, _i]),
     "trimkv_prefill_attn_split": (_i, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p, _i64, _p]),
+    "trimkv_prefill_equal_shares": (_i, [_i, _i, _i, _i, _i, _i]),
+    "trimkv_prefill_shares_workspace": (_i64, [_i, _i, _i, _i]),
+    "trimkv_prefill_attn_shares": (_i, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _f, _i, _p, _i64, _p]),
     "trimkv_stream_probe_granule": (_i64, [_i]),
     "trimkv_stream_probe": (_i, [_p, _p, _i64, _i, _p, _p]),
 }

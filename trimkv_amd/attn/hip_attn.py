@@ -221,6 +221,13 @@ def _prefill_split(batch: int, kv_heads: int, group: int, q_len: int, max_len: i
     return tiles, lib.trimkv_prefill_split_workspace(batch, kv_heads, group, q_len, max_len, tiles)
 
 
+@functools.lru_cache(maxsize=1024)
+def _prefill_shares(batch: int, kv_heads: int, group: int, q_len: int, max_len: int, uneven: int) -> int:
+    """Workspace bytes of a chunk's attention whose keys are cut into equal shares over all query tiles; 0: they are not."""
+    lib = _lib.load()
+    return lib.trimkv_prefill_shares_workspace(batch, kv_heads, group, q_len) if lib.trimkv_prefill_equal_shares(batch, kv_heads, group, q_len, max_len, uneven) else 0
+
+
 def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.Tensor, batch: int, kv_heads: int, group: int,
                       seg_len: Optional[torch.Tensor], seg_start: Optional[torch.Tensor], cap: int, max_len: int,
                       scale: float, uneven: int = 0) -> torch.Tensor:
@@ -249,13 +256,17 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
             batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len)
     stream = _lib.current_stream(query.device)
     tiles, need = _prefill_split(batch, kv_heads, group, Q, max_len, uneven)
-    if tiles:   # few query tiles: their keys divided among several workgroups
+    shares = 0 if tiles else _prefill_shares(batch, kv_heads, group, Q, max_len, uneven)
+    if tiles or shares:   # few query tiles: their keys divided among several workgroups; more: all keys in equal shares where that pays
         try:
-            work = torch.empty(need, dtype=torch.uint8, device=query.device)
+            work = torch.empty(need or shares, dtype=torch.uint8, device=query.device)
         except torch.OutOfMemoryError:
             work = None
-        if work is not None:
+        if work is not None and tiles:
             _lib.check(lib.trimkv_prefill_attn_split(*args, tiles, work.data_ptr(), need, stream), "trimkv_prefill_attn_split")
+            return out
+        if work is not None:
+            _lib.check(lib.trimkv_prefill_attn_shares(*args, work.data_ptr(), shares, stream), "trimkv_prefill_attn_shares")
             return out
     _lib.check(lib.trimkv_prefill_attn(*args, stream), "trimkv_prefill_attn")
     return out

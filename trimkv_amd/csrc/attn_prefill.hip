@@ -24,6 +24,7 @@
 // (ds_read_b64_tr_b16); the small kernel gathers 8 dwords (d, d+1) per lane and splits them into an
 // even-d and an odd-d operand.
 #include "common.hip.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace trimkv {
@@ -33,6 +34,7 @@ typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
 typedef float pf_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 pf_bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t pf_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t pf_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int PF_D = 128;                  // head_dim the tiles are built for; 64 and 96 run zero-padded to it (q = 0 there)
 constexpr int PF_BN = 32;                  // keys per tile
@@ -48,6 +50,7 @@ struct PrefillArgs {
     int hd;                                         // real head_dim: rows of K, V, q and out hold hd elements
     float scale_log2;
     int split_tiles; float* part; float* part_ml;   // keys split over workgroups: tiles of keys apiece, unfinished outputs, their references and sums
+    int* plan; int query_tiles, items;              // equal shares: [0] units of a share, [1 + i] first unit of query tile i; query tiles of a segment, in all
 };
 
 template <int G>
@@ -360,29 +363,34 @@ __device__ __forceinline__ void pf2_load_to_lds(const char* sbase, uint32_t voff
                  : "=&s"(saved) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 
-// SPLIT: blockIdx.z takes split_tiles tiles of the keys.  Where a query tile has more than that, its workgroups leave unnormalised
-// outputs with their exponent references and row sums (fp32) for prefill_merge_kernel; else the one workgroup writes the result.
-template <bool F16, bool SPLIT>
-__global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a) {
+// tiles of keys that the last query of a query tile sees
+__device__ __forceinline__ int tiles_seen(const PrefillArgs& a, int seg, int tile) {
+    int n = a.seg_len ? a.seg_len[seg] : a.max_len;
+    n = max(0, min(n, a.max_len));
+    const int BT = (PF2_WAVES * 32) / a.group, t_last = min(a.q_len - 1, tile * BT + BT - 1);
+    return (max(0, min(n, n - a.q_len + t_last + 1)) + PF2_BN - 1) / PF2_BN;
+}
+// units of query tile i of the launch where shares are equal: its key tiles, one if it sees nothing (its output is written all the same)
+__device__ __forceinline__ int units_of(const PrefillArgs& a, int i) {
+    const int seg = i / a.query_tiles;
+    return max(1, tiles_seen(a, seg, i - seg * a.query_tiles));
+}
+constexpr int PF2_GROUPS = 256;                     // one workgroup per CU
+constexpr int PF2_LEAST = 4;                        // units of a share at least
+
+// One query tile against `count` tiles of keys from tile t_first on (PART; else against all of them).  Where that is not all that the
+// query tile sees, unnormalised outputs with their exponent references and row sums (fp32) are left in `slot` for a merge kernel.
+template <bool F16, bool PART, bool LOOP>
+__device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot) {
     extern __shared__ __attribute__((aligned(16))) char pf2_lds[];
     PF_LDS3 char* const lds3 = (PF_LDS3 char*)pf2_lds;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds3;
-
-    // Workgroups are handed to the 8 XCDs round robin in dispatch order (x fastest), and each XCD has its own L2.  All
-    // query tiles of a segment read the same K/V, so they are mapped to one XCD (segment s on XCD s % 8, its tiles in
-    // consecutive turns of that XCD, later times first: they see more keys): the K/V tiles that several of them walk at
-    // about the same time are then fetched into one L2 instead of eight.
-    int seg = blockIdx.y, tile = (int)gridDim.x - 1 - (int)blockIdx.x;
-    if ((gridDim.y & 7) == 0) {
-        const int lin = (int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x;
-        const int turn = lin >> 3;
-        seg = (lin & 7) + 8 * (turn / (int)gridDim.x);
-        tile = (int)gridDim.x - 1 - turn % (int)gridDim.x;
-    }
     const int b = seg / a.kv_heads, h = seg - b * a.kv_heads;
     int n = a.seg_len ? a.seg_len[seg] : a.max_len;
     n = max(0, min(n, a.max_len));
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x;
+    if (LOOP) asm volatile("" : "+v"(tid));                   // nothing of a query tile is worth a register during the one before it
+    const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform by construction; saying so keeps what derives from it in scalar registers
     const int j = lane & 31, hl = lane >> 5;    // MFMA column (query) and lane half
     const int G = a.group, Q = a.q_len;
@@ -391,30 +399,15 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     const int r = w * 32 + j;
     const int g = r % G;
     const int t_q = t_wg0 + r / G;              // this lane's query time
-    const bool q_ok = r < BT * G && t_q < Q;
     const int t_w_first = t_wg0 + (w * 32) / G;
     const int64_t row0 = a.seg_start ? (int64_t)a.seg_start[seg] : (int64_t)seg * a.cap;
 
-    // Q fragments (B operand of S^T): 8 d of step ks at d = ks * 16 + hl * 8, multiplied by scale * log2(e) and rounded back
-    // to 16 bits once, here: the score MFMAs then deliver exponents of two directly and the loop never multiplies a score.
-    pf_bf16x8 qf[8];
+    // The rows of Q are asked for in front of the first keys and turned into fragments behind them: one memory round trip for both.
+    pf_u32x4 qraw[8];
     {
         const uint16_t* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(h * G + g) * a.q_sh + (int64_t)min(t_q, Q - 1) * a.q_st;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int e0 = ks * 16 + hl * 8;
-            const pf_u32x4 raw = *(const pf_u32x4*)(qrow + min(e0, a.hd - 8));
-            pf_u32x4 sc;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                float lo, hi;
-                if (F16) { lo = f16_bits_to_f32((uint16_t)(raw[x] & 0xffffu)); hi = f16_bits_to_f32((uint16_t)(raw[x] >> 16)); }
-                else { lo = __uint_as_float(raw[x] << 16); hi = __uint_as_float(raw[x] & 0xffff0000u); }
-                sc[x] = pack_kv<F16>(lo * a.scale_log2, hi * a.scale_log2);
-            }
-            if (e0 >= a.hd) sc = pf_u32x4{0u, 0u, 0u, 0u};   // padded features: whatever K holds there counts for nothing
-            qf[ks] = __builtin_bit_cast(pf_bf16x8, sc);
-        }
+        for (int ks = 0; ks < 8; ++ks) qraw[ks] = *(const pf_u32x4*)(qrow + min(ks * 16 + hl * 8, a.hd - 8));
     }
 
     pf_f32x16 o[4];   // O^T: o[db][v] = d (db * 32 + 8 * (v / 4) + 4 * hl + v % 4) of query j
@@ -434,8 +427,6 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     const int t_last = min(Q - 1, t_wg0 + BT - 1);
     const int k_end = max(0, min(n, n - Q + t_last + 1));     // keys the query tile sees
     const int all_tiles = (k_end + PF2_BN - 1) / PF2_BN;
-    const int t_first = SPLIT ? (int)blockIdx.z * a.split_tiles : 0;   // the workgroup's first tile of keys
-    if (SPLIT && t_first > 0 && t_first >= all_tiles) return;
     const int vis_j = n - Q + t_q;                            // last key this lane's query sees
     const int vis_lo = n - Q + t_w_first;                     // ... the wavefront's first query
     const int last_row = max(n - 1, 0);
@@ -471,6 +462,28 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
             pf2_load_to_lds(vseg, r1 + st_vcol, dv + PF2_TILE / 2);
         }
     };
+
+    const int ntiles = PART ? min(all_tiles - t_first, count) : all_tiles;
+    if (ntiles > 0) {
+        request_tile(0, 0);
+        request_tile(1, 1);
+    }
+    // Q fragments (B operand of S^T): 8 d of step ks at d = ks * 16 + hl * 8, multiplied by scale * log2(e) and rounded back
+    // to 16 bits once, here: the score MFMAs then deliver exponents of two directly and the loop never multiplies a score.
+    pf_bf16x8 qf[8];
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+        pf_u32x4 sc;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            float lo, hi;
+            if (F16) { lo = f16_bits_to_f32((uint16_t)(qraw[ks][x] & 0xffffu)); hi = f16_bits_to_f32((uint16_t)(qraw[ks][x] >> 16)); }
+            else { lo = __uint_as_float(qraw[ks][x] << 16); hi = __uint_as_float(qraw[ks][x] & 0xffff0000u); }
+            sc[x] = pack_kv<F16>(lo * a.scale_log2, hi * a.scale_log2);
+        }
+        if (ks * 16 + hl * 8 >= a.hd) sc = pf_u32x4{0u, 0u, 0u, 0u};   // padded features: whatever K holds there counts for nothing
+        qf[ks] = __builtin_bit_cast(pf_bf16x8, sc);
+    }
 
     // per-lane LDS read offsets; the buffer, the 32-key block and the step are immediates on top of them
     PF_LDS3 char* k_ptr[8];
@@ -625,12 +638,9 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     // of block b + 1 and then P.V of block b.  Every wavefront walks all blocks of the workgroup's tiles: the blocks that
     // lie wholly above a wavefront's diagonal (at most two of up to several hundred, the workgroup spans BT query times)
     // are masked like the diagonal ones and contribute zeros, which keeps the loop free of per-wavefront branches.
-    const int ntiles = SPLIT ? min(all_tiles - t_first, a.split_tiles) : all_tiles;
     if (ntiles > 0) {
         pf_f32x16 s_a, s_b;   // scores of the current and of the next block, roles swapping every step
         pf_bf16x8 pre[PF2_PD];
-        request_tile(0, 0);
-        request_tile(1, 1);
         asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         __syncthreads();
         {
@@ -675,10 +685,9 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
 
     // the two halves of a query hold disjoint keys: add their sums, then normalise and store
     l_run += __shfl_xor(l_run, 32, 64);
-    if (SPLIT && all_tiles > a.split_tiles) {
-        const int64_t wg = ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile;
-        if (hl == 0) *(float2*)(a.part_ml + (wg * (PF2_WAVES * 32) + r) * 2) = make_float2(m_ref, l_run);
-        float4* po = (float4*)a.part + (wg * PF2_WAVES + w) * (16 * 64) + lane;   // in register order: 1 KB per store
+    if (PART && all_tiles > ntiles) {
+        if (hl == 0) *(float2*)(a.part_ml + (slot * (PF2_WAVES * 32) + r) * 2) = make_float2(m_ref, l_run);
+        float4* po = (float4*)a.part + (slot * PF2_WAVES + w) * (16 * 64) + lane;   // in register order: 1 KB per store
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -686,24 +695,101 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
                 po[(db * 4 + c) * 64] = make_float4(o[db][4 * c], o[db][4 * c + 1], o[db][4 * c + 2], o[db][4 * c + 3]);
         return;
     }
-    if (q_ok) {
-        const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-        char* orow = (char*)(a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + (h * G + g)) * a.hd);
+    // A lane holds four features of a row at a time: stored from there, a row of 256 bytes would leave in 16 pieces.  The wavefront's
+    // 32 rows take the way through LDS instead (8 KB of its own; the 16-byte piece c of row j at c ^ (j % 16)) and leave whole.
+    const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+    PF_LDS3 char* const mine = lds3 + w * 8192;
+    __syncthreads();                             // every wavefront has left the tiles
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
+    for (int db = 0; db < 4; ++db)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint2 pk = make_uint2(pack_kv<F16>(o[db][4 * c] * inv, o[db][4 * c + 1] * inv),
-                                            pack_kv<F16>(o[db][4 * c + 2] * inv, o[db][4 * c + 3] * inv));
-                if (db * 32 + 8 * c + 4 * hl < a.hd) *(uint2*)(orow + (db * 32 + 8 * c + 4 * hl) * 2) = pk;
-            }
-        }
+        for (int c = 0; c < 4; ++c)
+            *(PF_LDS3 pf_u32x2*)(mine + j * 256 + (((db * 4 + c) ^ (j & 15)) << 4) + hl * 8) =
+                pf_u32x2{pack_kv<F16>(o[db][4 * c] * inv, o[db][4 * c + 1] * inv), pack_kv<F16>(o[db][4 * c + 2] * inv, o[db][4 * c + 3] * inv)};
+    const int piece = lane & 15;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+        const int row = 4 * x + (lane >> 4), rr = w * 32 + row, t = t_wg0 + rr / G;
+        const pf_u32x4 v = *(const PF_LDS3 pf_u32x4*)(mine + row * 256 + ((piece ^ (row & 15)) << 4));
+        if (rr < BT * G && t < Q && piece * 8 < a.hd)
+            *(pf_u32x4*)(a.out + (((int64_t)b * Q + t) * (a.kv_heads * G) + (h * G + rr % G)) * a.hd + piece * 8) = v;
+    }
+}
+
+// A workgroup per query tile; SPLIT: blockIdx.z takes split_tiles tiles of the keys, and the merge kernel puts shares together.
+template <bool F16, bool SPLIT>
+__global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a) {
+    // Workgroups are handed to the 8 XCDs round robin in dispatch order (x fastest), and each XCD has its own L2.  All
+    // query tiles of a segment read the same K/V, so they are mapped to one XCD (segment s on XCD s % 8, its tiles in
+    // consecutive turns of that XCD, later times first: they see more keys): the K/V tiles that several of them walk at
+    // about the same time are then fetched into one L2 instead of eight.
+    int seg = blockIdx.y, tile = (int)gridDim.x - 1 - (int)blockIdx.x;
+    if ((gridDim.y & 7) == 0) {
+        const int lin = (int)blockIdx.y * (int)gridDim.x + (int)blockIdx.x;
+        const int turn = lin >> 3;
+        seg = (lin & 7) + 8 * (turn / (int)gridDim.x);
+        tile = (int)gridDim.x - 1 - turn % (int)gridDim.x;
+    }
+    const int t_first = SPLIT ? (int)blockIdx.z * a.split_tiles : 0;
+    if (SPLIT && t_first > 0 && t_first >= tiles_seen(a, seg, tile)) return;
+    attend_query_tile<F16, SPLIT, false>(a, seg, tile, t_first, a.split_tiles, ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile);
+}
+
+// Equal shares (gridDim.x workgroups, one per CU): the key tiles of all query tiles, one query tile after the other, are cut into
+// runs of equal length whatever the segments' lengths are.  A run ends one query tile, takes some whole ones and begins another, so
+// a workgroup leaves at most two unfinished outputs: slot 2 wg of the query tile it found begun, 2 wg + 1 of the one it leaves.
+// Runs that follow each other lie on one XCD: they read the same segment.
+// What it costs beyond the keys' 1.6 us per 64 of them: about 11 us per query tile begun (Q, the first keys, the pipeline's fill, the
+// rows on their way out) and the unfinished outputs.  Eight layers of 24 segments of 0.69 x 4100 keys, 777 queries of 2 heads each,
+// with appends and eviction 1451 -> 1317 us; sizes on either side of the rule at trimkv_prefill_equal_shares.
+template <bool F16>
+__global__ __launch_bounds__(PF2_THREADS) void prefill_shares_kernel(PrefillArgs a) {
+    __shared__ int sums[PF2_WAVES], found[2];
+    const int tid = threadIdx.x, lane = tid & 63, groups = (int)gridDim.x;
+    const int wg = (groups & 7) ? (int)blockIdx.x : ((int)blockIdx.x & 7) * (groups >> 3) + ((int)blockIdx.x >> 3);
+    // first units of all query tiles: a thread sums the ones it has, a scan over the threads says where they begin
+    const int each = (a.items + PF2_THREADS - 1) / PF2_THREADS, i0 = min(tid * each, a.items), i1 = min(i0 + each, a.items);
+    const int first = i0 < i1 ? units_of(a, i0) : 0;         // all there is up to 512 query tiles
+    int own = first;
+    for (int i = i0 + 1; i < i1; ++i) own += units_of(a, i);
+    int incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += o;
+    }
+    if (lane == 63) sums[tid >> 6] = incl;
+    __syncthreads();
+    int before = incl - own, total = 0;
+#pragma unroll
+    for (int x = 0; x < PF2_WAVES; ++x) {
+        if (x < (tid >> 6)) before += sums[x];
+        total += sums[x];
+    }
+    const int per = max((total + groups - 1) / groups, PF2_LEAST);
+    const int u0 = wg * per, u1 = min(u0 + per, total);
+    for (int i = i0, at = before; i < i1; ++i) {
+        const int c = i == i0 ? first : units_of(a, i);
+        if (wg == 0) a.plan[1 + i] = at;
+        if (u0 >= at && u0 < at + c) { found[0] = i; found[1] = u0 - at; }
+        at += c;
+    }
+    if (wg == 0 && tid == 0) a.plan[0] = per;
+    if (u0 >= u1) return;                        // the whole workgroup: nothing was left for it
+    __syncthreads();
+    int i = __builtin_amdgcn_readfirstlane(found[0]), t_first = __builtin_amdgcn_readfirstlane(found[1]);
+    for (int u = u0; u < u1; ++i, t_first = 0) {
+        const int seg = i / a.query_tiles, count = min(units_of(a, i) - t_first, u1 - u);
+        attend_query_tile<F16, true, true>(a, seg, i - seg * a.query_tiles, t_first, count, 2 * wg + (t_first == 0));
+        u += count;
+        __syncthreads();                         // every wavefront has left the LDS tiles
     }
 }
 
 // The shares of the keys put together: one wavefront per (query tile, 32 of its rows, 32 features), lanes as they wrote.
 // A share that a row saw nothing of has sum 0 and a reference of no meaning: it is left out.
-template <bool F16>
+// EQUAL: shares as prefill_shares_kernel cut them, of which the first is in its workgroup's second slot.
+template <bool F16, bool EQUAL>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int seg = blockIdx.y, tile = (int)blockIdx.x >> 3, w = (int)blockIdx.x & 7, tiles = (int)gridDim.x >> 3;
     const int b = seg / a.kv_heads, h = seg - b * a.kv_heads;
@@ -713,16 +799,22 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int G = a.group, Q = a.q_len, BT = (PF2_WAVES * 32) / G;
     const int t_last = min(Q - 1, tile * BT + BT - 1);
     const int all_tiles = (max(0, min(n, n - Q + t_last + 1)) + PF2_BN - 1) / PF2_BN;
-    if (all_tiles <= a.split_tiles) return;   // one share: its workgroup wrote the result
-    const int shares = (all_tiles + a.split_tiles - 1) / a.split_tiles;
+    int shares, first = 0;
+    if constexpr (EQUAL) {
+        const int per = a.plan[0], at = a.plan[1 + seg * tiles + tile];
+        first = at / per;
+        shares = (at + max(all_tiles, 1) - 1) / per - first + 1;
+    } else shares = (all_tiles + a.split_tiles - 1) / a.split_tiles;
+    if (shares <= 1) return;                  // its workgroup wrote the result
     const int r = w * 32 + j, g = r % G, t_q = tile * BT + r / G;
     if (r >= BT * G || t_q >= Q) return;
     const int64_t wg = (int64_t)seg * tiles + tile, per_share = (int64_t)gridDim.y * tiles;
-    const float2* ml = (const float2*)a.part_ml + wg * (PF2_WAVES * 32) + r;
-    const float4* po = (const float4*)a.part + (wg * PF2_WAVES + w) * (16 * 64) + db * (4 * 64) + lane;
+    auto slot = [&](int z) -> int64_t { return EQUAL ? 2 * (first + z) + (z == 0) : wg + z * per_share; };
+    const float2* ml = (const float2*)a.part_ml + r;
+    const float4* po = (const float4*)a.part + w * (16 * 64) + db * (4 * 64) + lane;
     float m = -3.0e38f;
     for (int z = 0; z < shares; ++z) {
-        const float2 x = ml[z * per_share * (PF2_WAVES * 32)];
+        const float2 x = ml[slot(z) * (PF2_WAVES * 32)];
         if ((__float_as_uint(x.y) << 1) != 0) m = __builtin_fmaxf(m, x.x);
     }
     float l = 0.0f;
@@ -731,10 +823,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     for (int c = 0; c < 4; ++c) o[c] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 2
     for (int z = 0; z < shares; ++z) {
-        const float2 x = ml[z * per_share * (PF2_WAVES * 32)];
+        const float2 x = ml[slot(z) * (PF2_WAVES * 32)];
         float4 v[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) v[c] = po[z * per_share * (PF2_WAVES * 16 * 64) + c * 64];
+        for (int c = 0; c < 4; ++c) v[c] = po[slot(z) * (PF2_WAVES * 16 * 64) + c * 64];
         const float f = (__float_as_uint(x.y) << 1) != 0 ? __builtin_amdgcn_exp2f(x.x - m) : 0.0f;
         l += x.y * f;
 #pragma unroll
@@ -752,13 +844,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 constexpr int PF_PART_ROW = (PF_D + 2) * 4;   // bytes that a row of a workgroup leaves for the merge
 
 // > 64 KB of dynamic LDS needs the attribute once per device (the flag is only ever set, so a race repeats the call at worst)
-template <bool F16, bool SPLIT>
+template <auto KERNEL>
 static int opt_in_lds() {
     static bool done[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
     if (dev < 0 || !done[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)prefill_attn_kernel<F16, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, PF2_LDS);
+        hipError_t e = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, PF2_LDS);
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) done[dev] = true;
     }
@@ -794,11 +886,19 @@ static int launch_prefill_split(const PrefillArgs& a, int nseg, hipStream_t st) 
         }
         return 0;
     }
-    if (int rc = opt_in_lds<F16, true>()) return rc;
+    if (int rc = opt_in_lds<prefill_attn_kernel<F16, true>>()) return rc;
     const int bt = (PF2_WAVES * 32) / a.group, tiles = (a.q_len + bt - 1) / bt;
     const int key_tiles = (a.max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + a.split_tiles - 1) / a.split_tiles;
     hipLaunchKernelGGL((prefill_attn_kernel<F16, true>), dim3(tiles, nseg, shares), dim3(PF2_THREADS), PF2_LDS, st, a);
-    hipLaunchKernelGGL(prefill_merge_kernel<F16>, dim3(tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((prefill_merge_kernel<F16, false>), dim3(tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
+    return 0;
+}
+
+template <bool F16>
+static int launch_prefill_shares(const PrefillArgs& a, int nseg, hipStream_t st) {
+    if (int rc = opt_in_lds<prefill_shares_kernel<F16>>()) return rc;
+    hipLaunchKernelGGL(prefill_shares_kernel<F16>, dim3(PF2_GROUPS), dim3(PF2_THREADS), PF2_LDS, st, a);
+    hipLaunchKernelGGL((prefill_merge_kernel<F16, true>), dim3(a.query_tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
     return 0;
 }
 
@@ -811,7 +911,7 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
         hipLaunchKernelGGL((prefill_small_kernel<G, F16, false>), dim3(tiles, nseg), dim3(C::THREADS), 0, st, a);
         return 0;
     }
-    if (int rc = opt_in_lds<F16, false>()) return rc;
+    if (int rc = opt_in_lds<prefill_attn_kernel<F16, false>>()) return rc;
     const int bt = (PF2_WAVES * 32) / G;
     hipLaunchKernelGGL((prefill_attn_kernel<F16, false>), dim3((a.q_len + bt - 1) / bt, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
     return 0;
@@ -840,7 +940,7 @@ static int prefill_args(const char* fn, PrefillArgs& a, const void* q, int64_t q
     a.q = (const uint16_t*)q; a.q_sb = q_stride_b; a.q_sh = q_stride_h; a.q_st = q_stride_t; a.out = (uint16_t*)out;
     a.k = (const char*)k_slab; a.v = (const char*)v_slab; a.seg_len = seg_len; a.seg_start = seg_start;
     a.kv_heads = kv_heads; a.group = group; a.q_len = q_len; a.cap = cap; a.max_len = max_len; a.hd = head_dim; a.scale_log2 = scale * 1.4426950408889634f;
-    a.split_tiles = 0; a.part = nullptr; a.part_ml = nullptr;
+    a.split_tiles = 0; a.part = nullptr; a.part_ml = nullptr; a.plan = nullptr; a.query_tiles = 0; a.items = 0;
     return 0;
 }
 
@@ -877,13 +977,8 @@ extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_
 // for the merge's launch, 0.8 us per share that a row's merge walks, 0.045 us per workgroup for its 130 KB written and read.
 // Measured (us, D 128, whole -> split): 8 tiles of 2048 keys 44 -> 21, of 8192 keys 150 -> 31; 32 of 4096 79 -> 35; 56 of 2954
 // 64 -> 37; 96 of 4096 80 -> 57; 128 of 8192 155 -> 107; left whole: 96 of 2048 44 -> 40, of 1024 27 -> 30, 40 of 1024 27 -> 25.
-// Between 128 and 256 tiles of like length the chip's rate gains nothing from more workgroups (192 tiles of 4096 keys 103 -> 119, of
-// 8192 175 -> 205); of unlike segments the longest one holds up the rest, and three shares let the others' CUs help.  By mean
-// length / longest (24 or 32 segments): 160 and 168 tiles, two rounds of the chip, 0.69 of 4100 keys 85 -> 84, 0.60 83 -> 79, 0.75
-// of 8192 152 -> 142, 0.68 151 -> 136, 0.55 of 10000 184 -> 157, but 0.77 of 4096 82 -> 84; more tiles up to 0.55: 192, 0.53 of
-// 8192 153 -> 131; 216, 0.53 157 -> 143; 224, 0.52 of 6000 117 -> 113, of 10000 194 -> 166, but 0.57 of 8192 166 -> 177; beyond 10000
-// keys or 224 tiles not at all (240, 0.52 of 12000 245 -> 260).  Up to 3000 keys 63 -> 70.
-extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
+// More query tiles: equal shares (below) or whole.
+extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int /*uneven*/) {
     if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0) return 0;
     int64_t tiles, rows;
     query_tiles(group, q_len, &tiles, &rows);
@@ -902,11 +997,7 @@ extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, in
         }
         return (int)take;
     }
-    if (items >= 256) return 0;
-    if (items > 128) {
-        const bool pays = uneven > 0 && key_tiles >= 64 && (items <= 170 ? uneven <= 75 : uneven <= 55 && items <= 224 && key_tiles <= 160);
-        return pays ? (int)((key_tiles + 2) / 3) : 0;
-    }
+    if (items > 128) return 0;
     float best = 1.15f * (float)key_tiles - 8.0f;   // below that the second launch costs a caller whose queue runs dry as much
     int64_t take = 0;
     for (int64_t s = 2; s <= 32 && items * s <= 256; ++s) {
@@ -944,6 +1035,67 @@ extern "C" int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int6
     a.part_ml = (float*)workspace + need / PF_PART_ROW * PF_D;
     hipStream_t st = (hipStream_t)stream;
     const int rc = dtype == TRIMKV_F16 ? launch_prefill_split<true>(a, batch * kv_heads, st) : launch_prefill_split<false>(a, batch * kv_heads, st);
+    if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
+    return launch_status(fn);
+}
+
+// ---- equal shares of all keys of a launch ----
+// More than 128 query tiles.  Whole, the chip is done when its longest query tile is, or a last round that fills part of it: 1.2 us per
+// 64 keys where a CU has little company, 1.6 where all are busy.  Equal shares take the mean of all CUs and pay for it with up to
+// 67 MB of unfinished outputs written and read, about 26 us.  Estimates fitted to 80 launches (136 .. 1104 query tiles of 2500,
+// 5000 and 9000 keys, mean length 52 .. 100 % of the longest); where they differ by 3 % and more the choice was the faster one
+// but for two of them (up to 7 %).  Whole -> shares, us: 168 tiles, 0.78 of 4100 keys 88 -> 83, 0.65 of 9000 170 -> 122; 264 tiles of
+// 9000 377 -> 269, of 5000 167 -> 149; 288, 0.52 of 9000 289 -> 185; 352 of 5000 220 -> 204; left whole: 216 of 2500 59 -> 67, 512
+// of 5000 174 -> 204, 704 of 9000 478 -> 495.
+extern "C" int trimkv_prefill_equal_shares(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
+    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len < 64 || max_len <= 0) return 0;
+    int64_t tiles, rows;
+    query_tiles(group, q_len, &tiles, &rows);
+    const int64_t items = tiles * batch * kv_heads;
+    if (items <= 128 || items > 32768 || (uneven && max_len < 3072)) return 0;
+    // in tiles of 64 keys: the longest segment, the mean query tile, the first one of a mean segment
+    const float even = uneven <= 0 ? 1.0f : uneven == 1 ? 0.6f : 0.01f * (float)uneven, all = (float)items / 256.0f;
+    const float longest = (float)max_len / 64.0f, keys = (float)max_len * even, bt = 256.0f / (float)group;
+    const float mean = std::max(1.0f, (keys - 0.5f * (float)q_len) / 64.0f + 0.5f + bt / 128.0f), least = std::max(1.0f, (keys - (float)q_len) / 64.0f);
+    const float shares = 26.0f + 25.0f * (1.0f - even) + 0.03f * (float)items + 1.6f * mean * all;
+    float whole;
+    if (items <= 256) whole = std::max(1.6f * mean * all + 20.0f, 1.2f * longest + 12.0f);
+    else {
+        const float rounds = (float)(items / 256), rest = (float)(items % 256), last = least + (mean - least) * rest / (float)items;
+        whole = rounds * (1.6f * mean + 8.0f) + (rest > 0.0f ? (0.96f + 0.34f * rest / 256.0f) * last + 8.0f : 0.0f) + 0.9f * (1.0f - even) * longest;
+    }
+    return whole > 1.03f * shares;
+}
+
+extern "C" int64_t trimkv_prefill_shares_workspace(int batch, int kv_heads, int group, int q_len) {
+    if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len < 64) return 0;
+    int64_t tiles, rows;
+    query_tiles(group, q_len, &tiles, &rows);
+    return (int64_t)2 * PF2_GROUPS * rows * PF_PART_ROW + (tiles * batch * kv_heads + 1) * 4;
+}
+
+extern "C" int trimkv_prefill_attn_shares(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t, void* out,
+                                          const void* k_slab, const void* v_slab, const int32_t* seg_len, const int32_t* seg_start,
+                                          int batch, int kv_heads, int group, int q_len, int cap, int head_dim, int dtype, float scale,
+                                          int max_len, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "trimkv_prefill_attn_shares";
+    PrefillArgs a;
+    if (int bad = prefill_args(fn, a, q, q_stride_b, q_stride_h, q_stride_t, out, k_slab, v_slab, seg_len, seg_start, batch, kv_heads,
+                               group, q_len, cap, head_dim, dtype, scale, max_len)) return bad;
+    if (q_len < 64) return fail(TRIMKV_ERR_SHAPE, "%s: chunks of 64 queries and more (got %d)", fn, q_len);
+    int64_t tiles, rows;
+    query_tiles(group, q_len, &tiles, &rows);
+    const int64_t items = tiles * batch * kv_heads, key_tiles = ((int64_t)max_len + PF2_BN - 1) / PF2_BN;
+    if (items > (1 << 24) || items * key_tiles > (1 << 30)) return fail(TRIMKV_ERR_SHAPE, "%s: %lld query tiles of %d keys are too many", fn, (long long)items, max_len);
+    const int64_t need = trimkv_prefill_shares_workspace(batch, kv_heads, group, q_len);
+    if (!workspace || workspace_bytes < need || (uintptr_t)workspace & 15)
+        return fail(TRIMKV_ERR_CAPACITY, "%s: needs a 16-byte aligned workspace of %lld bytes (got %lld)", fn, (long long)need, (long long)workspace_bytes);
+    a.part = (float*)workspace;
+    a.part_ml = a.part + (int64_t)2 * PF2_GROUPS * rows * PF_D;
+    a.plan = (int*)(a.part_ml + (int64_t)2 * PF2_GROUPS * rows * 2);
+    a.query_tiles = (int)tiles; a.items = (int)items;
+    hipStream_t st = (hipStream_t)stream;
+    const int rc = dtype == TRIMKV_F16 ? launch_prefill_shares<true>(a, batch * kv_heads, st) : launch_prefill_shares<false>(a, batch * kv_heads, st);
     if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
     return launch_status(fn);
 }
