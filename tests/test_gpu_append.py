@@ -1,0 +1,34 @@
+"""GPU tests of trimkv_append where a segment's new rows are spread over several workgroups, against plain indexing."""
+import pytest
+import torch
+
+from tests.gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("S,D,cap", [(127, 128, 400), (128, 128, 400), (129, 96, 400), (257, 64, 400), (300, 256, 1000), (147, 8, 1 << 20), (130945, 8, 131072)])
+def test_rows_lengths_and_prefix_sums(S, D, cap):
+    """Around the 128 rows of a workgroup; rows of more pieces than it has in flight; a slab of 2^20 rows and a chunk of 1024 workgroups, whose lengths a launch of its own
+    advances; segments that are empty, end flush with the slab, or would not fit (untouched)."""
+    from trimkv_amd import _lib
+    lib, B, H = _lib.load(), 2, 2
+    gen = torch.Generator().manual_seed(S)
+    nseg = B * H
+    lens = torch.tensor([0, cap - S, 7, cap - S + 1], dtype=torch.int32)
+    k, v = (torch.randn(B, H, S, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    lb, pos = torch.randn(B, H, S, generator=gen), torch.arange(5, 5 + S)
+    slabs = [torch.zeros(nseg, cap, D, dtype=torch.bfloat16, device=DEV) for _ in range(2)] + [torch.zeros(nseg, cap, device=DEV), torch.zeros(nseg, cap, dtype=torch.int64, device=DEV)]
+    want = [t.cpu() for t in slabs]
+    for s in range(nseg - 1):
+        n = int(lens[s])
+        for t, new in zip(want, (k.view(nseg, S, D), v.view(nseg, S, D), lb.view(nseg, S), pos.expand(nseg, S))):
+            t[s, n:n + S] = new[s]
+    seg_len, cu = lens.to(DEV), torch.zeros(nseg + 1, dtype=torch.int32, device=DEV)
+    kd, vd, lbd, pd = (t.to(DEV) for t in (k, v, lb, pos))
+    _lib.check(lib.trimkv_append(*(t.data_ptr() for t in slabs), seg_len.data_ptr(), cu.data_ptr(), nseg, H, cap, D, _lib.BF16, _lib.F32,
+                                 kd.data_ptr(), vd.data_ptr(), *kd.stride()[:3], lbd.data_ptr(), *lbd.stride(), pd.data_ptr(), 0, 0, 1,
+                                 S, cap, _lib.current_stream(kd.device)), "trimkv_append")
+    assert seg_len.tolist() == [S, cap, 7 + S, cap - S + 1]
+    assert cu.tolist() == [0, S, 2 * S, 3 * S, 0]
+    assert all(torch.equal(got.cpu(), w) for got, w in zip(slabs, want))
