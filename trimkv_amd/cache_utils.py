@@ -137,7 +137,7 @@ class _Slab:
         self.max_len = 0
         self.total = 0  # sum of lens (kept by the ragged caches, which size their split-K chunk from it)
         self.order = None  # ragged caches: segments by decreasing length/budget (dispatch order of the attention launch)
-        self.order_host = None  # the pinned copy it was uploaded from (kept until the next one replaces it)
+        self.order_host = None  # what it follows from (lengths or budgets), then the pinned copy it was uploaded from (kept until the next one replaces it)
         self.pending = None  # a one-token append that the next attention call will carry out (see _SlabBacked._defer)
         self.pieces = None   # ragged caches: (device piece list, number of pieces) of the decode-attention launch
         self.pieces_total, self.pieces_age = 0, 0
@@ -1069,8 +1069,10 @@ class _RaggedCache(_SlabBacked):
         # grid-split fallback (callers that ignore "pieces"): rows per piece for about attention_pieces pieces
         chunk = max(512, ((slab.total // self.attention_pieces + 63) // 64) * 64)
         kw = {"head_lens": slab.seg_len, "cu_seqlens_k": slab.cu,
-              "seg_start": self._seg_start(slab), "seg_cap": slab.cap, "max_len": slab.max_len, "rows": slab.total, "chunk": chunk,
-              "seg_order": slab.order, "pieces": self._piece_list(slab)}
+              "seg_start": self._seg_start(slab), "seg_cap": slab.cap, "max_len": slab.max_len, "rows": slab.total, "chunk": chunk}
+        # what only launches of one query row per sequence look at is not uploaded for a chunk
+        if key_states is None or S == 1:
+            kw["seg_order"], kw["pieces"] = self._dispatch_order(slab), self._piece_list(slab)
         if slab.pending is not None:
             # head_lens / cu_seqlens_k still hold the values before this token: the attention call that receives this
             # dictionary appends the row and advances them in the same launch
@@ -1097,8 +1099,9 @@ class _RaggedCache(_SlabBacked):
         room = 2 * nseg + 2 * self.attention_compute_units
         buf = slab.pieces_buf
         if buf is None or buf[0].shape[0] < room:
-            dev = torch.empty(room, 4, dtype=torch.int32, device=slab.k.device)
-            host = [torch.empty(room, 4, dtype=torch.int32, pin_memory=True) for _ in range(2)]
+            with torch.inference_mode(False):      # written again by steps that may be outside of the mode
+                dev = torch.empty(room, 4, dtype=torch.int32, device=slab.k.device)
+                host = [torch.empty(room, 4, dtype=torch.int32, pin_memory=True) for _ in range(2)]
             buf = slab.pieces_buf = [dev, host, [None, None], 0]
         dev, host, events, which = buf
         if events[which] is not None:
@@ -1348,12 +1351,18 @@ class _RaggedCache(_SlabBacked):
     def _set_dispatch_order(slab: _Slab, key) -> None:
         """Very uneven segments: hand the attention launch the segments longest first (``key`` = lengths or budgets),
         so that the long ones are not dispatched last.  Near-equal lengths need no order."""
-        key = np.asarray(key, dtype=np.int64)
-        if key.size < 16 or int(key.max()) * key.size <= 1.5 * max(1, int(key.sum())):
-            slab.order = None
-        else:   # through pinned memory, in stream order: a copy from pageable memory would wait for the whole stream
-            host = torch.from_numpy(np.argsort(-key, kind="stable").astype(np.int32)).pin_memory()
-            slab.order, slab.order_host = host.to(slab.k.device, non_blocking=True), host
+        key = np.array(key, dtype=np.int64)
+        slab.order, slab.order_host = None, None if key.size < 16 or int(key.max()) * key.size <= 1.5 * max(1, int(key.sum())) else key
+
+    @staticmethod
+    def _dispatch_order(slab: _Slab) -> Optional[torch.Tensor]:
+        """The order set last, on the device from its first use on."""
+        if slab.order is None and slab.order_host is not None:
+            # through pinned memory, in stream order: a copy from pageable memory would wait for the whole stream
+            if not torch.is_tensor(slab.order_host):
+                slab.order_host = torch.from_numpy(np.argsort(-slab.order_host, kind="stable").astype(np.int32)).pin_memory()
+            slab.order = slab.order_host.to(slab.k.device, non_blocking=True)
+        return slab.order
 
     def set_budgets(self, budgets) -> None:
         """Give every segment its own token budget: ``budgets`` is ``[nseg]`` (all layers alike) or
