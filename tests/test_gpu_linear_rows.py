@@ -133,3 +133,123 @@ def test_modules_that_somebody_hooked_wrapped_or_replaced_are_called():
             return 2 * super().forward(y)
     twice = Doubled(8, 4)
     assert torch.equal(linear.run(twice, x), 2 * nn.functional.linear(x, twice.weight, twice.bias))
+
+
+def _normed(x, norm):
+    """What the modules make of x, in 64 bits between their two roundings."""
+    h = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + norm.variance_epsilon)
+    return (h.to(torch.bfloat16).double() * norm.weight.double()).to(torch.bfloat16)
+
+
+# rows: every number of row groups and their edges; n: every number of blocks per tile, a last tile that is moved back, more tiles than
+# workgroups; k: fewer steps than wavefronts, numbers that do not divide among them
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k", [(1, 64, 64), (3, 320, 8192), (8, 4608, 192), (9, 112, 576), (16, 4624, 1024), (17, 64, 2048), (32, 2048, 704), (29, 8192, 128), (32, 8208, 64), (5, 50000, 64)])
+def test_linear_rows_with_a_residual(rows, n, k):
+    x, w, bias = _operands(rows, n, k, torch.bfloat16, rows + n + k)
+    wide = torch.zeros(rows, 1, n + 4, dtype=torch.bfloat16, device=DEV)
+    wide[..., 4:] = torch.randn(rows, 1, n, generator=torch.Generator(device=DEV).manual_seed(k), device=DEV) * 3
+    res = wide[..., 4:]
+    for b in (None, bias):
+        out, squares = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV), torch.full((rows, n // 16), float("nan"), device=DEV)
+        _lib.check(_lib.load().trimkv_linear_rows_add(x.data_ptr(), k, w.data_ptr(), k, _lib.ptr(b), res.data_ptr(), n + 4, out.data_ptr(), n, squares.data_ptr(),
+                                                      rows, n, k, _lib.BF16, _lib.current_stream(x.device)), "trimkv_linear_rows_add")
+        assert torch.equal(out, linear.linear(x, w, b) + res[:, 0])
+        want = out.double().square().view(rows, n // 16, 16).sum(-1)
+        assert ((squares.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("silu", [False, True])
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 64), (3, 40, 8192), (8, 4608, 192), (9, 100, 576), (16, 4616, 1024), (16, 12288, 64), (17, 33, 2048), (32, 2048, 704), (29, 9000, 128), (32, 12300, 64),
+                                      (5, 70001, 64), (16, 50000, 128)])
+def test_linear_rows_behind_a_norm(rows, n, k, silu):
+    """Against the norm in 64 bits with the modules' roundings: where the two disagree on a rounding, an element of the operand differs by
+    2^-7 of itself; each product is allowed that."""
+    from trimkv_amd.qwen3 import RMSNorm
+    x, w, bias = _operands(rows, (2 if silu else 1) * n, k, torch.bfloat16, rows + n + k)
+    x = (x.float() * 30).to(torch.bfloat16)
+    norm = RMSNorm(k, 1e-6).to(torch.bfloat16).to(DEV)
+    norm.weight.data.normal_(1.0, 0.3, generator=torch.Generator(device=DEV).manual_seed(k))
+    h = _normed(x, norm)
+    squares = x.float().square().view(rows, k // 16, 16).sum(-1)
+    for b in (None, bias):
+        with torch.no_grad():
+            d = linear.DeferredNorm(x, squares, norm)
+            got = linear.norm_product(d, w, b, silu)
+            plain = linear.silu_product(h, w, b) if silu else linear.linear(h, w, b)
+            assert (got != plain).float().mean() < 0.2                       # nearly always the very same operand
+            d.tensor()
+            assert linear.norm_product(d, w, b, silu) is None               # taken already
+        exact = h.double() @ w.double().T + (0 if b is None else b.double())
+        size = (h.double().abs() @ w.double().abs().T) * (2.0 ** -7 * min(1.0, 64 / k) + k * 2.0 ** -23)
+        if not silu:
+            bound = EPS[torch.bfloat16] * exact.abs() + size + 2.0 ** -24
+        else:
+            (g, u), (dg, du) = exact.chunk(2, -1), size.chunk(2, -1)
+            exact, act = torch.nn.functional.silu(g) * u, torch.nn.functional.silu(g)
+            dg, du = dg + EPS[torch.bfloat16] * g.abs(), du + EPS[torch.bfloat16] * u.abs()
+            bound = 1.1 * dg * (u.abs() + du) + act.abs() * du + 2 * EPS[torch.bfloat16] * exact.abs() + 1e-5 * exact.abs() + 2.0 ** -24
+        err = (got.double() - exact).abs()
+        assert (err <= bound).all(), float((err - bound).max())
+
+
+@pytest.mark.gpu
+def test_what_is_not_left_to_a_product():
+    x, w, bias = _operands(16, 320, 256, torch.bfloat16, 5)
+    lin = nn.Linear(256, 320, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        takes = linear.can_defer_product
+        assert takes(lin, x) and takes(lin, x[:, None]) and not takes(lin, torch.cat([x] * 3)) and not takes(nn.Linear(256, 300, device=DEV, dtype=torch.bfloat16), x)
+        assert not takes(lin.half(), x.half())
+        lin = lin.to(torch.bfloat16)
+        hook = lin.register_forward_hook(lambda m, a, out: out)
+        assert not takes(lin, x)
+        hook.remove()
+        weight, res = torch.ones(256, dtype=torch.bfloat16, device=DEV), torch.zeros(16, 512, dtype=torch.bfloat16, device=DEV)
+        assert linear.can_defer_norm(weight, x) and not linear.can_defer_norm(weight, res[:, :256]) and not linear.can_defer_norm(weight.half(), x) and not linear.can_defer_norm(weight[:8], x)
+    assert not takes(lin, x)                                                # somebody differentiates
+
+
+def test_bad_arguments_around_a_norm_are_refused_without_a_launch():
+    lib, one = _lib.load(), ctypes.c_void_p(16)
+    norm = lambda rows=4, k=64, sq=one, nw=one, dt=_lib.BF16: lib.trimkv_linear_rows_norm(one, k, sq, nw, 1e-6, one, k, None, one, 16, rows, 16, k, 0, 1, dt, None)
+    assert norm(rows=33) == -2 and norm(k=8256) == -2 and norm(nw=ctypes.c_void_p(24)) == -2 and norm(sq=None) == -1 and norm(nw=None) == -1 and norm(dt=_lib.F16) == -3
+    add = lambda rows=4, n=16, rs=16, os=16, res=one, sq=one, dt=_lib.BF16: lib.trimkv_linear_rows_add(one, 64, one, 64, None, res, rs, one, os, sq, rows, n, 64, dt, None)
+    assert add(rows=33) == -2 and add(n=24, rs=24, os=24) == -2 and add(rs=12) == -2 and add(rs=18) == -2 and add(os=18) == -2 and add(res=ctypes.c_void_p(20)) == -2
+    assert add(res=None) == -1 and add(sq=None) == -1 and add(dt=_lib.F32) == -3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("family,gate", [("qwen3", "rg"), ("qwen3", "rg2"), ("llama", "rg"), ("phi3", "rg")])
+def test_decode_steps_leave_adds_and_norms_to_the_products(family, gate, monkeypatch):
+    """Logits of decode steps with and without launches of their own for adds and norms, to rounding; hooks see what they saw."""
+    from trimkv_amd import qwen3
+    from tests.test_gpu_qwen3_shell import _family, _tiny_config
+    cfg = _tiny_config(family, retention_gate=gate)
+    torch.manual_seed(0)
+    model = _family(family)[1](cfg).to(torch.bfloat16).to(DEV).eval()
+    ids = torch.randint(0, cfg.vocab_size, (2, 40), generator=torch.Generator().manual_seed(4)).to(DEV)
+    taken, plain = [], linear.norm_product
+
+    def steps():
+        with torch.no_grad():
+            out, logits = model(ids[:, :30]), []
+            for i in range(30, 34):
+                out = model(ids[:, i:i + 1], past_key_values=out.past_key_values)
+                logits.append(out.logits[:, -1].float())
+        return torch.stack(logits)
+    monkeypatch.setattr(linear, "norm_product", lambda *a: (lambda out: taken.append(out is not None) or out)(plain(*a)))
+    got = steps()
+    assert sum(taken) == len(taken) == 4 * (cfg.num_hidden_layers if family == "phi3" else 2 * cfg.num_hidden_layers - 1)
+    monkeypatch.setattr(linear, "can_defer_product", lambda *a: False)
+    want = steps()
+    assert (got - want).abs().max() <= 2e-2 + 2e-2 * want.abs().max()
+    monkeypatch.undo()
+    seen = []
+    handles = [model.model.layers[1].register_forward_hook(lambda m, a, out: seen.append(type(out[1]))), model.model.layers[0].mlp.register_forward_hook(lambda m, a, out: seen.append(type(out))),
+               model.model.layers[1].self_attn.register_forward_hook(lambda m, a, out: seen.append(type(out))), model.model.layers[0].self_attn.o_proj.register_forward_hook(lambda m, a, out: seen.append(type(out)))]
+    hooked = steps()
+    assert seen == [torch.Tensor] * 20 and (hooked - want).abs().max() <= 2e-2 + 2e-2 * want.abs().max()
+    for handle in handles:
+        handle.remove()

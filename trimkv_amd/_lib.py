@@ -39,6 +39,8 @@ SIGNATURES = {
     "trimkv_silu_mul": (_i, [_p, _i64, _p, _i64, _p, _i, _i, _i, _p]),
     "trimkv_linear_rows": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p]),
     "trimkv_linear_rows_silu": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
+    "trimkv_linear_rows_add": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _p, _i64, _p, _i, _i, _i, _i, _p]),
+    "trimkv_linear_rows_norm": (_i, [_p, _i64, _p, _p, _f, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
     "trimkv_gate_hidden_packed": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
     "trimkv_gate_hidden_swiglu_packed": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
     "trimkv_append_gated": (_i, [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _p, _i64, _i64, _i64,

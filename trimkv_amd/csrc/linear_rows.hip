@@ -1,6 +1,8 @@
 // Products of a few rows with a large matrix (the tokens of a decode step and a linear layer) -- gfx950.
 //
 //   trimkv_linear_rows        out[m][n] = sum_k x[m][k] w[n][k] (+ bias[n]), up to 64 rows x, w as nn.Linear keeps it
+//   trimkv_linear_rows_add    the same plus a residual, with sums of the squares of the result for the norm behind it
+//   trimkv_linear_rows_norm   either of the others of the RMS norm of x
 //   trimkv_linear_rows_silu   out[m][n] = silu(gate) * up with gate = x . w[n] and up = x . w[inter + n]: a gated feed-forward's
 //                             first two matrices and the product of their outputs
 //
@@ -44,12 +46,25 @@ struct LinearRowsArgs {
     int m, n, k;        // n: columns of out
     int vec;            // four columns of out can be stored at once
     int round_all;      // silu: the two products and silu(gate) are rounded before they are used, as modules do
+    // a residual added to the product: the sums of the squares of what is stored, 16 columns at a time, go to squares [m][n / 16]
+    const uint16_t* res; int64_t res_stride;
+    // an RMS norm of x in front of the product: its weight; squares [m][k / 16] as above
+    const uint16_t* norm_w; float eps;
+    float* squares;
 };
 
 template <bool F16>
 __device__ __forceinline__ lr_f32x4 lr_mfma(lr_u32x4 a, lr_u32x4 b, lr_f32x4 c) {
     if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(lr_f16x8, a), __builtin_bit_cast(lr_f16x8, b), c, 0, 0, 0);
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lr_bf16x8, a), __builtin_bit_cast(lr_bf16x8, b), c, 0, 0, 0);
+}
+constexpr int LR_NORM_K = 8192, LR_NORM_ROWS = 32;        // longest and most rows with a norm in front of the product
+__device__ __forceinline__ float lr_lo(uint32_t p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float lr_hi(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
+__device__ __forceinline__ uint32_t lr_pack(float lo, float hi) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 template <bool F16> __device__ __forceinline__ float lr_load(uint16_t b) { return F16 ? f16_bits_to_f32(b) : bf16_bits_to_f32(b); }
 template <bool F16> __device__ __forceinline__ uint16_t lr_bits(float f) { return F16 ? f32_to_f16_bits(f) : f32_to_bf16_bits(f); }
@@ -70,12 +85,22 @@ __device__ __forceinline__ void lr_load_to_lds(const uint16_t* base, uint32_t of
 // XG groups of 8 rows of x, NT blocks of 16 rows of w (SILU: NT / 2 of gate, NT / 2 of up), W wavefronts, D steps of 64 elements
 // of k in flight per wavefront.  A step in LDS: row r holds its eight 16-byte pieces rotated by r / 2, which spreads the 16 rows of
 // an operand read over all banks (the rotation is in the lanes' source addresses).
-template <bool F16, bool SILU, int XG, int NT, int W, int D>
+// A decoder's residual add and RMS norm have no launch of their own (4.6 us, most of it latency): the product in front of them (ADD)
+// adds the residual where it rounds and leaves sums of squares, a few KB that the product behind them (NORM) adds up while its first
+// operands are on their way; x becomes round(round(x / rms) * weight), as modules round, on its way from LDS to the matrix cores.
+// A layer's four products with adds and norms, 16 rows: 43.6 -> 40.2 us at 2048 features and 6144, 92.0 -> 83.5 at 4096 and 12288; 1 row
+// 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102.  With more rows the arithmetic on the way no longer hides.
+enum { LR_PLAIN = 0, LR_ADD = 1, LR_NORM = 2 };
+template <bool F16, bool SILU, int MODE, int XG, int NT, int W, int D>
 __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
+    constexpr bool NORM = MODE == LR_NORM, ADD = MODE == LR_ADD;
+    static_assert(MODE == LR_PLAIN || !F16, "bf16 only");
     constexpr int MT = (XG + 1) / 2, L = 2 * NT + XG, STEP = L * 1024, U = NT * MT, NB = SILU ? NT / 2 : NT;
     static_assert((D - 1) * L < 64, "the wait counts at most 63 loads");
     __shared__ __attribute__((aligned(1024))) char ring[W * D * STEP];
     __shared__ lr_f32x4 part[U * (W - 1)][64];
+    __shared__ __attribute__((aligned(16))) uint16_t norm_w[NORM ? LR_NORM_K : 8];
+    __shared__ float scale[NORM ? LR_NORM_ROWS : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
     const uint32_t ring_at = (uint32_t)(uintptr_t)(LR_LDS char*)ring + wave * D * STEP;
     const char* mine = ring + wave * D * STEP;
@@ -112,8 +137,27 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         }
         ask_slot = ask_slot + 1 == D ? 0 : ask_slot + 1;
     };
+    float inv[MT], sum = 0.f;
+    constexpr int ROW_THREADS = 64 * W / (8 * XG);        // that add up the squares of one row
+    if constexpr (NORM) {       // the weight of the norm: 512 elements a load, of a last one with fewer the last 8 again
+        const uint32_t at = (uint32_t)(uintptr_t)(LR_LDS uint16_t*)norm_w;
+        for (int p = wave; p * 512 < a.k; p += W) lr_load_to_lds<false>(a.norm_w, (uint32_t)min(p * 512 + lane * 8, a.k - 8) * 2, at + p * 1024);
+        const float* from = a.squares + (int64_t)min((int)threadIdx.x / ROW_THREADS, a.m - 1) * (a.k >> 4);
+        for (int c = (threadIdx.x % ROW_THREADS) * 4; c < a.k >> 4; c += ROW_THREADS * 4) {
+            const lr_f32x4 f = *(const lr_f32x4*)(from + c);
+            sum += (f[0] + f[1]) + (f[2] + f[3]);
+        }
+    }
 #pragma unroll
     for (int d = 0; d < D; ++d) request();
+    if constexpr (NORM) {
+#pragma unroll
+        for (int d = 1; d < ROW_THREADS; d <<= 1) sum += __shfl_xor(sum, d, 64);
+        if (threadIdx.x % ROW_THREADS == 0) scale[threadIdx.x / ROW_THREADS] = rsqrtf(sum / (float)a.k + a.eps);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(D * L) : "memory");       // weight and scales are there for all wavefronts
+#pragma unroll
+        for (int t = 0; t < MT; ++t) inv[t] = scale[XG == 1 ? r & 7 : t * 16 + r];
+    }
     lr_f32x4 acc[U];
     int slot = 0;
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
@@ -122,7 +166,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         for (int s = 0; s < per_tile; ++s) {
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * L) : "memory");
             const char* p = mine + slot * STEP;
-            lr_u32x4 wf[2][NT], xf[2][MT];
+            lr_u32x4 wf[2][NT], xf[2][MT], nf[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -132,11 +176,23 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
                     const int row = XG == 1 ? r & 7 : t * 16 + r;       // 8 rows: columns 8 .. 15 repeat them
                     xf[h][t] = *(const lr_u32x4*)(p + (NT * 16 + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
                 }
+                if constexpr (NORM) nf[h] = *(const lr_u32x4*)(norm_w + (wave + s * W) * 64 + (h * 4 + g) * 8);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // the step has been read: its room is free
             __builtin_amdgcn_sched_barrier(0);
             request();
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (NORM) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint32_t y = lr_pack(lr_lo(xf[h][t][i]) * inv[t], lr_hi(xf[h][t][i]) * inv[t]);
+                            xf[h][t][i] = lr_pack(lr_lo(y) * lr_lo(nf[h][i]), lr_hi(y) * lr_hi(nf[h][i]));
+                        }
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -162,7 +218,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         for (int u = 0; u < NB * MT; ++u) {
             if (owner(u) != wave) continue;
             const int m = u % MT * 16 + r, n = block_at(tile, u / MT) + 4 * g;      // this lane: columns n .. n + 3 of row m
-            if (m >= a.m) continue;
+            if (m >= a.m && !ADD) continue;
             lr_f32x4 f = total(u);
             uint16_t v[4];
 #pragma unroll
@@ -181,6 +237,21 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
             } else {
 #pragma unroll
                 for (int c = 0; c < 4; ++c) v[c] = lr_bits<F16>(f[c]);
+            }
+            if constexpr (ADD) {            // n is a multiple of 16: four columns are there or none
+                const uint2 y = *(const uint2*)(a.res + (int64_t)min(m, a.m - 1) * a.res_stride + n);
+                const float old[4] = {lr_lo(y.x), lr_hi(y.x), lr_lo(y.y), lr_hi(y.y)};
+                float sq = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    v[c] = lr_bits<F16>(lr_load<F16>(v[c]) + old[c]);
+                    const float x = lr_load<F16>(v[c]);
+                    sq = fmaf(x, x, sq);
+                }
+                sq += __shfl_xor(sq, 16, 64);
+                sq += __shfl_xor(sq, 32, 64);
+                if (m >= a.m) continue;
+                if (g == 0) a.squares[(int64_t)m * (a.n >> 4) + (n >> 4)] = sq;
             }
             uint16_t* o = a.out + (int64_t)m * a.out_stride + n;
             if (a.vec) *(uint2*)o = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
@@ -212,26 +283,32 @@ static int rows_plan(int n, int x_rows, bool silu) {
     return best;
 }
 
-template <bool F16, bool SILU, int XG, int NT, int W, int D>
+template <bool F16, bool SILU, int XG, int NT, int W, int D, int MODE = LR_PLAIN>
 static void rows_launch(const LinearRowsArgs& a, hipStream_t s) {
-    constexpr int NB = SILU ? NT / 2 : NT, LDS = W * D * (2 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024;
+    constexpr int NB = SILU ? NT / 2 : NT, LDS = W * D * (2 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024 + (MODE == LR_NORM ? LR_NORM_K * 2 + LR_NORM_ROWS * 4 : 16);
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
     const int tiles = (a.n + 16 * NB - 1) / (16 * NB), most = LR_CUS * (160 * 1024 / LDS);
-    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, XG, NT, W, D>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
+    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NT, W, D>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
 }
 // wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 6 over the shapes above
-template <bool F16, int XG>
+template <bool F16, int XG, int MODE = LR_PLAIN>
 static void rows_by_blocks(const LinearRowsArgs& a, bool silu, hipStream_t s) {
     const int nt = rows_plan(a.n, 8 * XG, silu);
-    if constexpr (XG == 8) {
+    if constexpr (MODE == LR_NORM) {
+        if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, XG < 4 ? 3 : 2, MODE>(a, s);
+        if (silu) return rows_launch<F16, true, XG, 2, 4, 3, MODE>(a, s);
+        if (nt == 2) return rows_launch<F16, false, XG, 2, 4, 3, MODE>(a, s);
+    } else if constexpr (MODE == LR_ADD) {
+    } else if constexpr (XG == 8) {
         if (silu && nt == 6) return rows_launch<F16, true, 8, 6, 4, 1>(a, s);
         if (silu && nt == 4) return rows_launch<F16, true, 8, 4, 2, 2>(a, s);
         if (!silu && nt == 6) return rows_launch<F16, false, 8, 6, 4, 1>(a, s);
     } else if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, 2>(a, s);
-    if (silu) rows_launch<F16, true, XG, 2, 4, 2>(a, s);
-    else if (nt == 1) rows_launch<F16, false, XG, 1, 4, XG < 4 ? 3 : 2>(a, s);
-    else if (nt == 2) rows_launch<F16, false, XG, 2, 4, 2>(a, s);
-    else rows_launch<F16, false, XG, 3, 4, 2>(a, s);
+    if constexpr (MODE == LR_PLAIN)
+        if (silu) return rows_launch<F16, true, XG, 2, 4, 2>(a, s);
+    if (nt == 1) rows_launch<F16, false, XG, 1, 4, XG < 4 ? 3 : 2, MODE>(a, s);
+    else if (nt == 2) rows_launch<F16, false, XG, 2, 4, 2, MODE>(a, s);
+    else rows_launch<F16, false, XG, 3, 4, 2, MODE>(a, s);
 }
 template <bool F16>
 static void rows_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
@@ -239,6 +316,13 @@ static void rows_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
     else if (a.m <= 16) rows_by_blocks<F16, 2>(a, silu, s);
     else if (a.m <= 32) rows_by_blocks<F16, 4>(a, silu, s);
     else rows_by_blocks<F16, 8>(a, silu, s);
+}
+
+template <int MODE>
+static void norm_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
+    if (a.m <= 8) rows_by_blocks<false, 1, MODE>(a, silu, s);
+    else if (a.m <= 16) rows_by_blocks<false, 2, MODE>(a, silu, s);
+    else rows_by_blocks<false, 4, MODE>(a, silu, s);
 }
 
 }  // namespace trimkv
@@ -254,7 +338,9 @@ static int rows_check_and_launch(const char* fn, LinearRowsArgs a, bool silu, in
         return fail(TRIMKV_ERR_SHAPE, "%s: strides %lld %lld (>= k, multiples of 8, at most 2^24) %lld (>= n)", fn, (long long)a.x_stride, (long long)a.w_stride, (long long)a.out_stride);
     if (((uintptr_t)a.x | (uintptr_t)a.w) & 15) return fail(TRIMKV_ERR_SHAPE, "%s: x and w must be 16-byte aligned", fn);
     a.vec = a.n % 4 == 0 && a.out_stride % 4 == 0 && !((uintptr_t)a.out & 7);
-    if (dtype == TRIMKV_F16) rows_by_rows<true>(a, silu, (hipStream_t)stream);
+    if (a.norm_w) norm_by_rows<LR_NORM>(a, silu, (hipStream_t)stream);
+    else if (a.res) norm_by_rows<LR_ADD>(a, silu, (hipStream_t)stream);
+    else if (dtype == TRIMKV_F16) rows_by_rows<true>(a, silu, (hipStream_t)stream);
     else rows_by_rows<false>(a, silu, (hipStream_t)stream);
     return launch_status(fn);
 }
@@ -269,4 +355,29 @@ extern "C" int trimkv_linear_rows_silu(const void* x, int64_t x_stride, const vo
                                        int rows, int inter, int k, int round_all, int dtype, void* stream) {
     return rows_check_and_launch("trimkv_linear_rows_silu",
                                  LinearRowsArgs{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, inter, k, 0, round_all}, true, dtype, stream);
+}
+
+extern "C" int trimkv_linear_rows_add(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, const void* residual, int64_t residual_stride,
+                                      void* out, int64_t out_stride, float* squares, int rows, int n, int k, int dtype, void* stream) {
+    const char* fn = "trimkv_linear_rows_add";
+    if (!residual || !squares) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (dtype != TRIMKV_BF16) return fail(TRIMKV_ERR_DTYPE, "%s: bf16 only (dtype=%d)", fn, dtype);
+    if (rows > LR_NORM_ROWS || n % 16) return fail(TRIMKV_ERR_SHAPE, "%s: at most %d rows, n a multiple of 16 (got %d, %d)", fn, LR_NORM_ROWS, rows, n);
+    if (residual_stride < n || residual_stride % 4 || out_stride % 4 || ((uintptr_t)residual | (uintptr_t)out) & 7)
+        return fail(TRIMKV_ERR_SHAPE, "%s: residual and out must be 8-byte aligned, their strides multiples of 4 and at least n (%lld)", fn, (long long)residual_stride);
+    LinearRowsArgs a{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, n, k, 0, 0};
+    a.res = (const uint16_t*)residual; a.res_stride = residual_stride; a.squares = squares;
+    return rows_check_and_launch(fn, a, false, dtype, stream);
+}
+
+extern "C" int trimkv_linear_rows_norm(const void* x, int64_t x_stride, const float* squares, const void* norm_weight, float eps, const void* w, int64_t w_stride,
+                                       const void* bias, void* out, int64_t out_stride, int rows, int n, int k, int silu, int round_all, int dtype, void* stream) {
+    const char* fn = "trimkv_linear_rows_norm";
+    if (!squares || !norm_weight) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (dtype != TRIMKV_BF16) return fail(TRIMKV_ERR_DTYPE, "%s: bf16 only (dtype=%d)", fn, dtype);
+    if (rows > LR_NORM_ROWS || k > LR_NORM_K) return fail(TRIMKV_ERR_SHAPE, "%s: at most %d rows of %d (got %d of %d)", fn, LR_NORM_ROWS, LR_NORM_K, rows, k);
+    if ((uintptr_t)norm_weight & 15) return fail(TRIMKV_ERR_SHAPE, "%s: norm_weight must be 16-byte aligned", fn);
+    LinearRowsArgs a{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, n, k, 0, round_all};
+    a.norm_w = (const uint16_t*)norm_weight; a.eps = eps; a.squares = const_cast<float*>(squares);
+    return rows_check_and_launch(fn, a, silu != 0, dtype, stream);
 }

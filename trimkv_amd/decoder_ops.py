@@ -41,6 +41,11 @@ def run_linear(module: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     return linear.run(module, x) if enabled else module(x)
 
 
+def leave_or_run(module: torch.nn.Module, x: torch.Tensor, leave: bool):
+    """``run_linear``, or with ``leave`` a ``linear.DeferredProduct`` where the launch that adds the residual can take it."""
+    return linear.DeferredProduct(x, module) if leave and enabled and linear.can_defer_product(module, x) else run_linear(module, x)
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None):
     """``weight * norm(x)`` over the last axis; with ``residual`` returns ``(weight * norm(x + residual), x + residual)``."""
     hidden = x.shape[-1]
@@ -155,9 +160,26 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``silu_mul`` of the two halves of ``x @ weight.T`` in the product's own launch (a decode step's rows), or None."""
-    out = linear.silu_product(x, weight, bias) if enabled else None
+def _with_norm(x, weight: torch.Tensor, bias: Optional[torch.Tensor], silu: bool) -> Optional[torch.Tensor]:
+    out = linear.norm_product(x, weight, bias, silu) if type(x) is linear.DeferredNorm else None
+    if out is not None:
+        counts["rmsnorm"] += 1
+    return out
+
+
+def product(x, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """``x @ weight.T + bias``; ``x``: a tensor or a ``linear.DeferredNorm``, which is taken in the same launch where that can be."""
+    out = _with_norm(x, weight, bias, False)
+    return linear.linear(linear.tensor_of(x), weight, bias) if out is None else out
+
+
+def silu_product(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``silu_mul`` of the two halves of ``product(x, weight, bias)`` in the product's own launch (a decode step's rows), or None."""
+    if not enabled:
+        return None
+    out = _with_norm(x, weight, bias, True)
+    if out is None:
+        out = linear.silu_product(linear.tensor_of(x), weight, bias)
     if out is not None:
         counts["silu_mul"] += 1
     return out

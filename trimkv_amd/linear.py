@@ -77,11 +77,93 @@ def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return out
 
 
-def untouched(module: nn.Module) -> bool:
-    """An ``nn.Linear`` that nobody has hooked, wrapped or replaced: its parameters say all that calling it does."""
-    return not (type(module) is not nn.Linear or module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+def unhooked(module: nn.Module) -> bool:
+    """Nobody has hooked the module or replaced its ``forward``: calling it does what its class says."""
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
                 or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks
                 or "forward" in module.__dict__)
+
+
+def untouched(module: nn.Module) -> bool:
+    """An ``nn.Linear`` that nobody has hooked, wrapped or replaced: its parameters say all that calling it does."""
+    return type(module) is nn.Linear and unhooked(module)
+
+
+NORM_ROWS, NORM_K = 32, 8192      # what trimkv_linear_rows_add and trimkv_linear_rows_norm take
+
+
+class DeferredProduct:
+    """``module(x)`` of an untouched ``nn.Linear``, not taken yet: whoever adds a residual to it does so in its launch (``add_product``);
+    anybody else calls ``tensor``."""
+
+    __slots__ = ("x", "module")
+
+    def __init__(self, x: torch.Tensor, module: nn.Linear):
+        self.x, self.module = x, module
+
+    def tensor(self) -> torch.Tensor:
+        return run(self.module, self.x)
+
+
+class DeferredNorm:
+    """``norm(x)`` not taken yet, with the sums of squares of ``add_product``: a product takes it in its own launch (``norm_product``);
+    anybody else calls ``tensor``."""
+
+    __slots__ = ("x", "squares", "norm", "normed")
+
+    def __init__(self, x: torch.Tensor, squares: torch.Tensor, norm):
+        self.x, self.squares, self.norm, self.normed = x, squares, norm, None
+
+    shape = property(lambda self: self.x.shape)
+
+    def tensor(self) -> torch.Tensor:
+        if self.normed is None:
+            self.normed = self.norm(self.x)
+        return self.normed
+
+
+def tensor_of(x) -> torch.Tensor:
+    return x.tensor() if type(x) in (DeferredNorm, DeferredProduct) else x
+
+
+def can_defer_product(module: nn.Module, x: torch.Tensor) -> bool:
+    """Whether ``module(x)`` may wait for the residual that is added to it."""
+    w = module.weight
+    return (untouched(module) and x.dtype == torch.bfloat16 and 0 < x.numel() <= NORM_ROWS * x.shape[-1] and w.shape[0] % 64 == 0 and w.shape[0] <= NORM_K
+            and _rows(x, w, module.bias) is not None)
+
+
+def can_defer_norm(weight: torch.Tensor, residual: torch.Tensor) -> bool:
+    """Whether the product behind the norm of a sum with ``residual`` may take it along."""
+    k = residual.shape[-1]
+    return weight.shape == (k,) and weight.is_contiguous() and residual.is_contiguous() and not (weight.data_ptr() | residual.data_ptr()) % 16 and _plain(residual, weight)
+
+
+def add_product(p: DeferredProduct, residual: torch.Tensor):
+    """``(residual + module(x), squares)`` in one launch; both have passed ``can_defer_product`` and ``can_defer_norm``."""
+    w, bias = p.module.weight, p.module.bias
+    x2, n = _rows(p.x, w, bias), w.shape[0]
+    rows, k = x2.shape
+    out = torch.empty(residual.shape, dtype=residual.dtype, device=residual.device)
+    squares = torch.empty(rows, n // 16, dtype=torch.float32, device=residual.device)
+    _lib.check(_lib.load().trimkv_linear_rows_add(x2.data_ptr(), x2.stride(0) if rows > 1 else k, w.data_ptr(), w.stride(0), _lib.ptr(bias), residual.data_ptr(), n,
+                                                  out.data_ptr(), n, squares.data_ptr(), rows, n, k, _lib.BF16, _lib.current_stream(residual.device)), "trimkv_linear_rows_add")
+    return out, squares
+
+
+def norm_product(d: DeferredNorm, weight: torch.Tensor, bias: Optional[torch.Tensor], silu: bool = False) -> Optional[torch.Tensor]:
+    """``linear(d, weight, bias)`` or, ``silu``, ``silu_product`` of it with the norm in the same launch; None where that is not to be done
+    (the norm has been taken already, or the kernel does not take this product)."""
+    x2 = _rows(d.x, weight, bias) if d.normed is None else None
+    if x2 is None or (silu and weight.shape[0] % 2):
+        return None
+    rows, k = x2.shape
+    n = weight.shape[0] // 2 if silu else weight.shape[0]
+    out = torch.empty(*d.x.shape[:-1], n, dtype=d.x.dtype, device=d.x.device)
+    _lib.check(_lib.load().trimkv_linear_rows_norm(x2.data_ptr(), x2.stride(0) if rows > 1 else k, d.squares.data_ptr(), d.norm.weight.data_ptr(), float(d.norm.variance_epsilon),
+                                                   weight.data_ptr(), weight.stride(0), _lib.ptr(bias), out.data_ptr(), n, rows, n, k, int(silu), 1, _lib.BF16,
+                                                   _lib.current_stream(d.x.device)), "trimkv_linear_rows_norm")
+    return out
 
 
 def run(module: nn.Module, x: torch.Tensor) -> torch.Tensor:

@@ -43,11 +43,15 @@ class Phi3MLP(nn.Module):
         self.gate_up_proj = nn.Linear(config.hidden_size, 2 * config.intermediate_size, bias=False)
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def takes_deferred(self, x: torch.Tensor) -> bool:
+        return type(self).forward is Phi3MLP.forward
+
+    def forward(self, x: torch.Tensor, leave_product: bool = False) -> torch.Tensor:
         if linear.untouched(self.gate_up_proj):
             act = decoder_ops.silu_product(x, self.gate_up_proj.weight)
             if act is not None:
-                return decoder_ops.run_linear(self.down_proj, act)
+                return decoder_ops.leave_or_run(self.down_proj, act, leave_product)
+        x = linear.tensor_of(x)
         gate, up = decoder_ops.run_linear(self.gate_up_proj, x).chunk(2, dim=-1)
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
             return decoder_ops.run_linear(self.down_proj, decoder_ops.silu_mul(gate, up))
@@ -63,6 +67,9 @@ class TrimKVPhi3Attention(TrimKVQwen3Attention):
         self.num_heads, self.num_key_value_heads = config.num_attention_heads, config.num_key_value_heads
         self.qkv_proj = nn.Linear(config.hidden_size, (self.num_heads + 2 * self.num_key_value_heads) * d, bias=False)
         self.o_proj = nn.Linear(self.num_heads * d, config.hidden_size, bias=False)
+
+    def takes_deferred(self, x: torch.Tensor) -> bool:
+        return False      # the gate reads the normed hidden state as well
 
     def _projections(self, hidden_states: torch.Tensor):
         B, S, _ = hidden_states.shape

@@ -149,6 +149,8 @@ class FusedRows:
     def _usable(self, x: torch.Tensor) -> bool:
         """Whether these modules can be one product here (not in training, on the CPU, in fp32, with differing input widths);
         if so, their parameters lie in the buffer."""
+        if type(x) is linear.DeferredNorm:
+            x = x.x
         if not decoder_ops.usable(x, *(lin.weight for lin in self.linears)):
             return False
         if any(lin.in_features != self.linears[0].in_features or (lin.bias is not None and lin.bias.dtype != x.dtype) for lin in self.linears):
@@ -169,7 +171,7 @@ class FusedRows:
             bias = None
         elif bias is not None:
             bias = bias[:rows]
-        return linear.linear(x, self.weight[:rows], bias).split(sizes, dim=-1)
+        return decoder_ops.product(x, self.weight[:rows], bias).split(sizes, dim=-1)
 
     def silu_product(self, x: torch.Tensor) -> Optional[torch.Tensor]:
         """``silu(gate(x)) * up(x)`` of two modules (gate, up) of one size in one launch, or None when that cannot be done here."""
@@ -187,13 +189,18 @@ class MLP(nn.Module):
         self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=bias)
         self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=bias)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def takes_deferred(self, x: torch.Tensor) -> bool:
+        return type(self).forward is MLP.forward
+
+    def forward(self, x: torch.Tensor, leave_product: bool = False) -> torch.Tensor:
+        """``x``: also a ``linear.DeferredNorm``; ``leave_product``: the last product may come back as a ``linear.DeferredProduct``."""
         fused = self.__dict__.get("_gate_up")
         if fused is None:
             fused = self.__dict__["_gate_up"] = FusedRows(self.gate_proj, self.up_proj)
         act = fused.silu_product(x)
         if act is not None:
-            return decoder_ops.run_linear(self.down_proj, act)
+            return decoder_ops.leave_or_run(self.down_proj, act, leave_product)
+        x = linear.tensor_of(x)
         both = fused(x)
         gate, up = both if both is not None else (self.gate_proj(x), self.up_proj(x))
         if decoder_ops.usable(gate, up) and decoder_ops.silu_mul_ok(gate, up):
@@ -296,6 +303,7 @@ class TrimKVQwen3Attention(nn.Module):
         n = 4 if with_gate and len(linears) == 4 else 3
         qkv = fused(hidden_states, n)     # one product; q, k, v (and the gate's hidden layer) are slices of its output
         if qkv is None:
+            hidden_states = linear.tensor_of(hidden_states)
             qkv = (self.q_proj(hidden_states), self.k_proj(hidden_states), self.v_proj(hidden_states))
         out = (qkv[0].view(shape), qkv[1].view(shape), qkv[2].view(shape))
         return out + ((qkv[3] if len(qkv) == 4 else None),) if with_gate else out
@@ -372,20 +380,30 @@ class TrimKVQwen3Attention(nn.Module):
         self._gate_keep = (hidden_states, retention)
         return retention, done
 
-    def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position):
+    def takes_deferred(self, x: torch.Tensor) -> bool:
+        """Whether the projections are all that reads the normed hidden state (``x``: what it will be like)."""
+        cls = TrimKVQwen3Attention
+        if type(self).forward is not cls.forward or type(self)._qkv_rope is not cls._qkv_rope or type(self)._projections is not cls._projections:
+            return False
+        return self.config.retention_gate != "rg" or (self.fold_gate and not self.gate_on_side_stream and getattr(self.retention_gate, "_use_hip", lambda x: False)(x))
+
+    def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, leave_product: bool = False):
+        """``hidden_states``: also a ``linear.DeferredNorm`` (see ``takes_deferred``); ``leave_product``: the last product may come back
+        as a ``linear.DeferredProduct``."""
         B, S, _ = hidden_states.shape
+        deferred = type(hidden_states) is linear.DeferredNorm
         # `rg` sees the normed hidden state, before RoPE (qwen3:332-333); on the GPU this is a LazyLogBeta
         retention, gate_done = None, None
         cos, sin = position_embeddings
         if self.config.retention_gate == "rg":
-            if self.gate_on_side_stream and hidden_states.is_cuda and not self.training:
+            if not deferred and self.gate_on_side_stream and hidden_states.is_cuda and not self.training:
                 retention, gate_done = self._gate_beside_projections(hidden_states)
                 q, k, v = self._qkv_rope(hidden_states, cos, sin)
-            elif self.fold_gate and getattr(self.retention_gate, "_use_hip", lambda x: False)(hidden_states):
+            elif deferred or (self.fold_gate and getattr(self.retention_gate, "_use_hip", lambda x: False)(hidden_states)):
                 # the gate's first linear in the product of q, k, v, its second half in the norm + RoPE launch: no launch of its own
                 q, k, v, retention = self._qkv_rope(hidden_states, cos, sin, True)
                 if retention is None:
-                    retention = self.retention_gate(hidden_states)
+                    retention = self.retention_gate(linear.tensor_of(hidden_states))
             else:
                 retention = self.retention_gate(hidden_states)
                 q, k, v = self._qkv_rope(hidden_states, cos, sin)
@@ -396,7 +414,7 @@ class TrimKVQwen3Attention(nn.Module):
             retention = self.retention_gate(torch.cat([k, v], dim=-1)).transpose(1, 2)
         offset = past_key_values.get_seq_length(self.layer_idx)
         if gate_done is not None:
-            torch.cuda.current_stream(hidden_states.device).wait_event(gate_done)
+            torch.cuda.current_stream(k.device).wait_event(gate_done)
         k, v, retention, kv_positions, fa_kwargs = past_key_values.update(
             k, v, retention, cache_position, self.layer_idx,
             {"sin": sin, "cos": cos, "cache_position": cache_position, "attention_mask": attention_mask})
@@ -404,7 +422,7 @@ class TrimKVQwen3Attention(nn.Module):
         out, _, _ = attend(self, q, k, v, attention_mask=attention_mask, retention_weights=retention, kv_positions=kv_positions,
                            offset=offset, dropout=0.0, scaling=self.scaling, sliding_window=None, is_causal=True,
                            flash_attn_kwargs=fa_kwargs)
-        return decoder_ops.run_linear(self.o_proj, out.reshape(B, S, -1).contiguous())
+        return decoder_ops.leave_or_run(self.o_proj, out.reshape(B, S, -1).contiguous(), leave_product)
 
 
 class TrimKVQwen3DecoderLayer(nn.Module):
@@ -417,16 +435,31 @@ class TrimKVQwen3DecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(config.hidden_size, config.rms_norm_eps)
         self.post_attention_layernorm = RMSNorm(config.hidden_size, config.rms_norm_eps)
 
-    def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending=None):
+    def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending=None, leave_product: bool = False):
         """``pending``: the MLP output of the layer below, not yet added to ``hidden_states`` -- the add (qwen3:437) then rides
-        in this layer's first norm.  Returns ``(hidden_states, mlp_out)`` with the same add left to whoever comes next."""
+        in this layer's first norm.  Returns ``(hidden_states, mlp_out)`` with the same add left to whoever comes next;
+        ``leave_product``: ``mlp_out`` may be a ``linear.DeferredProduct``, into which the add goes (as ``pending`` may be one)."""
+        attn, mlp = self.self_attn, self.mlp
         if pending is None:
             normed = self.input_layernorm(hidden_states)
         else:
-            normed, hidden_states = self.input_layernorm.add_norm(pending, hidden_states)
-        attn_out = self.self_attn(normed, position_embeddings, attention_mask, past_key_values, cache_position)
-        normed, hidden_states = self.post_attention_layernorm.add_norm(attn_out, hidden_states)   # qwen3:431-435
-        return hidden_states, self.mlp(normed)
+            normed, hidden_states = self._add_norm(self.input_layernorm, pending, hidden_states, attn)
+        leaves = lambda module: {"leave_product": True} if hasattr(module, "takes_deferred") and linear.unhooked(module) else {}
+        attn_out = attn(normed, position_embeddings, attention_mask, past_key_values, cache_position, **leaves(attn))
+        normed, hidden_states = self._add_norm(self.post_attention_layernorm, attn_out, hidden_states, mlp)   # qwen3:431-435
+        return hidden_states, mlp(normed, **(leaves(mlp) if leave_product else {}))
+
+    @staticmethod
+    def _add_norm(norm, x, residual, reader):
+        """``norm.add_norm(x, residual)`` for ``reader``.  At a decode step the add goes into the product that ``x`` is the result of and
+        the norm into the one that ``reader`` begins with: neither has a launch of its own."""
+        if type(x) is linear.DeferredProduct:
+            if (type(norm) is RMSNorm and linear.unhooked(norm) and linear.unhooked(reader) and linear.can_defer_norm(norm.weight, residual)
+                    and getattr(reader, "takes_deferred", lambda x: False)(residual)):
+                total, squares = linear.add_product(x, residual)
+                return linear.DeferredNorm(total, squares, norm), total
+            x = x.tensor()
+        return norm.add_norm(x, residual)
 
 
 class TrimKVQwen3Model(nn.Module):
@@ -461,8 +494,9 @@ class TrimKVQwen3Model(nn.Module):
         hidden_states = inputs_embeds
         pending = None    # the last MLP output; its residual add rides in the next norm
         for layer in self.layers:
-            hidden_states, pending = layer(hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending)
-        hidden_states = self.norm(hidden_states) if pending is None else self.norm.add_norm(pending, hidden_states)[0]
+            leave = {"leave_product": True} if type(layer).forward is TrimKVQwen3DecoderLayer.forward and linear.unhooked(layer) else {}
+            hidden_states, pending = layer(hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending if leave else linear.tensor_of(pending), **leave)
+        hidden_states = self.norm(hidden_states) if pending is None else self.norm.add_norm(linear.tensor_of(pending), hidden_states)[0]
         c = self.config
         if c.compress_memory:   # qwen3:751-760: after every forward, prompt or decode step
             past_key_values.compress(strategy=c.compress_strategy, memory_size=c.memory_size, buffer_size=c.buffer_size,
