@@ -690,6 +690,12 @@ int trimkv_silu_mul(const void* gate, int64_t gate_stride, const void* up, int64
                     int ntok, int inter, int dtype, void* stream);
 
 /*
+ * trimkv_rope_tables -- cos, sin [ntok][2 half] (bf16 or fp16) of positions[t] * inv_freq[j] in fp32, the frequencies twice in a row
+ * (rotary embeddings whose features rotate in halves; apply_rotary_pos_emb, qwen3:125-151).
+ */
+int trimkv_rope_tables(const int64_t* positions, const float* inv_freq, void* cos, void* sin, int ntok, int half, int dtype, void* stream);
+
+/*
  * trimkv_linear_rows -- out[m][n] = round(sum_k x[m][k] w[n][k] + bias[n]): a linear layer (w [n][k] as nn.Linear keeps it, bias
  * [n] optional) over 1 .. 64 rows, the tokens of a decode step.  Sums are fp32 in an order that depends on the sizes only.
  * trimkv_linear_rows_silu -- w [2 inter][k], bias [2 inter] optional: the first inter rows are the gate, the others the up

@@ -326,3 +326,25 @@ def test_prompt_sized_launches():
     for got, want in ((gq, wq), (gk, wk)):
         tol = 2 * _ulp(want.float(), dtype) + 2 * _ulp(torch.full_like(want.float(), 4.0), dtype)
         assert ((got.float() - want.float()).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("pos,rd,theta,scaling", [
+    (torch.tensor([[0]]), 128, 1e6, None),
+    (torch.tensor([[7], [20479], [131071]]), 96, 1e4, None),
+    (torch.arange(3 * 257).view(3, 257).t(), 64, 5e5, {"rope_type": "llama3", "factor": 8.0, "low_freq_factor": 1.0, "high_freq_factor": 4.0, "original_max_position_embeddings": 8192}),
+])
+def test_rope_tables_are_what_torch_computes(pos, rd, theta, scaling, dtype):
+    """The same fp32 angles; cosine and sine of the two libraries may differ by a unit of fp32, which can turn a rounding."""
+    from trimkv_amd import decoder_ops
+    from trimkv_amd.qwen3 import rotary_tables
+    pos = pos.to(DEV)
+    got = [rotary_tables(pos, 128, theta, dtype, rd, scaling) for _ in range(2)]
+    decoder_ops.enabled = False
+    try:
+        want = rotary_tables(pos, 128, theta, dtype, rd, scaling)
+    finally:
+        decoder_ops.enabled = True
+    for g, again, w in zip(*got, want):
+        assert g.shape == w.shape == (*pos.shape, rd) and torch.equal(g, again)
+        assert ((g.double() - w.double()).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * w.double().abs() + 2.0 ** -24).all() and (g != w).float().mean() < 1e-3

@@ -37,6 +37,7 @@ SIGNATURES = {
     "trimkv_qk_norm_rope": (_i, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _i,
                                  _i, _i, _i, _i, _i, _i, _f, _i, _p]),
     "trimkv_silu_mul": (_i, [_p, _i64, _p, _i64, _p, _i, _i, _i, _p]),
+    "trimkv_rope_tables": (_i, [_p, _p, _p, _p, _i, _i, _i, _p]),
     "trimkv_linear_rows": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p]),
     "trimkv_linear_rows_silu": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
     "trimkv_linear_rows_add": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _p, _i64, _p, _i, _i, _i, _i, _p]),

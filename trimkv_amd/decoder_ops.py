@@ -70,6 +70,21 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optiona
     return out.view(x.shape), total.view(x.shape)
 
 
+def rope_tables_ok(positions: torch.Tensor, dtype: torch.dtype, rotary_dim: int) -> bool:
+    return (dtype in (torch.bfloat16, torch.float16) and positions.dtype == torch.int64 and positions.dim() == 2 and positions.numel() > 0 and rotary_dim > 0 and rotary_dim % 2 == 0
+            and type(positions) is torch.Tensor and positions.device.index == torch.cuda.current_device())
+
+
+def rope_tables(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype):
+    """cos, sin [B, S, 2 half] of ``positions`` [B, S] times ``inv_freq`` [half] (fp32), in one launch."""
+    positions, half = positions.contiguous(), inv_freq.shape[0]
+    cos, sin = (torch.empty(*positions.shape, 2 * half, dtype=dtype, device=positions.device) for _ in range(2))
+    rc = _lib.load().trimkv_rope_tables(positions.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), positions.numel(), half, _lib.dtype_code(dtype),
+                                        _lib.current_stream(positions.device))
+    _lib.check(rc, "trimkv_rope_tables")
+    return cos, sin
+
+
 def qk_norm_rope_ok(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
     """q, k [B, S, H, D] views of projection outputs (D contiguous, heads D apart, batch = S tokens apart), cos/sin
     [1 or B, S, R] contiguous with R even."""

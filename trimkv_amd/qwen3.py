@@ -214,7 +214,15 @@ def rotary_tables(position_ids: torch.Tensor, head_dim: int, theta: float, dtype
     None/"default", or the published "llama3" rule (wavelengths above ``original/low_freq_factor`` are slowed by
     ``factor``, those below ``original/high_freq_factor`` kept, a linear blend in between)."""
     rd = head_dim if rotary_dim is None else rotary_dim
-    inv_freq = 1.0 / (theta ** (torch.arange(0, rd, 2, device=position_ids.device, dtype=torch.float32) / rd))
+    if position_ids.is_cuda and decoder_ops.enabled and decoder_ops.rope_tables_ok(position_ids, dtype, rd):
+        return decoder_ops.rope_tables(position_ids, _kept_frequencies(position_ids.device, rd, theta, rope_scaling), dtype)
+    ang = position_ids[..., None].float() * _frequencies(position_ids.device, rd, theta, rope_scaling)
+    emb = torch.cat([ang, ang], dim=-1)
+    return emb.cos().to(dtype), emb.sin().to(dtype)
+
+
+def _frequencies(device, rd: int, theta: float, rope_scaling: Optional[dict]) -> torch.Tensor:
+    inv_freq = 1.0 / (theta ** (torch.arange(0, rd, 2, device=device, dtype=torch.float32) / rd))
     kind = (rope_scaling or {}).get("rope_type", (rope_scaling or {}).get("type", "default"))
     if kind == "llama3":
         factor, lo, hi = rope_scaling["factor"], rope_scaling["low_freq_factor"], rope_scaling["high_freq_factor"]
@@ -224,9 +232,25 @@ def rotary_tables(position_ids: torch.Tensor, head_dim: int, theta: float, dtype
         inv_freq = (1 - blend) * inv_freq / factor + blend * inv_freq
     elif kind != "default":
         raise NotImplementedError(f"rope scaling {kind!r}")
-    ang = position_ids[..., None].float() * inv_freq
-    emb = torch.cat([ang, ang], dim=-1)
-    return emb.cos().to(dtype), emb.sin().to(dtype)
+    return inv_freq
+
+
+_FREQUENCIES: dict = {}      # (device, sizes and scaling) -> what _frequencies gives there: constants
+
+
+def _kept_frequencies(device, rd: int, theta: float, rope_scaling: Optional[dict]) -> torch.Tensor:
+    key = (device, rd, theta, None if not rope_scaling else tuple(sorted((k, str(v)) for k, v in rope_scaling.items())))
+    freq = _FREQUENCIES.get(key)
+    if freq is None:
+        with torch.inference_mode(False), torch.no_grad():
+            freq = _frequencies(device, rd, theta, rope_scaling)
+        if torch.cuda.is_current_stream_capturing():      # memory of the graph's
+            return freq
+        torch.cuda.current_stream(device).synchronize()   # there for every stream from here on
+        if len(_FREQUENCIES) >= 64:
+            _FREQUENCIES.clear()
+        _FREQUENCIES[key] = freq
+    return freq
 
 
 def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
