@@ -72,15 +72,15 @@ def _workspace_zeroed(device, nbytes: int, stream: int) -> torch.Tensor:
     return ws
 
 
-def _uniform_cut(nseg: int, max_len: int) -> int:
+def _uniform_cut(nseg: int, max_len: int, least: int = 0) -> int:
     """Pieces per segment for segments of equal length -- the dense cache.  With fewer than 256 segments each is cut so
     that about 256 workgroups exist (a compute unit pulls about 50 GB/s whatever it runs, so all 256 are needed), but not
-    below 512 rows apiece; the pieces are merged inside the launch (``trimkv_decode_attn_uniform``), which saves the second
+    below ``least`` rows apiece (0: ``dense_min_rows``); the pieces are merged inside the launch (``trimkv_decode_attn_uniform``), which saves the second
     launch of the grid-split path.  1 when the segments are attended whole (256 segments or more, or short ones)."""
     if nseg >= 256 or nseg > 8192:
         return 1
     want = (dense_workgroups + nseg - 1) // nseg
-    chunk = max(dense_min_rows, (((max_len + want - 1) // want + 63) // 64) * 64)
+    chunk = max(least or dense_min_rows, (((max_len + want - 1) // want + 63) // 64) * 64)
     return max(1, (max_len + chunk - 1) // chunk)
 
 

@@ -602,7 +602,8 @@ class TrimKVCache(_SlabBacked):
         # Decode steps whose launches depend on no host-side length (begin_device_steps): what a HIP graph can replay.
         self.lengths_on_device = False
         self._seen_dev: Optional[torch.Tensor] = None   # device int64 [1]: tokens seen + 1, the query index of an eviction
-        self._device_pieces = None                      # (device piece list, entries) of the attention launch in that mode
+        self._device_pieces = None                      # (device piece list, entries) of the attention launch in that mode, if segments are cut
+        self._device_wholes = None                      # ... if they are not and there are few of them
 
     # ---- decode steps that a HIP graph can replay ------------------------------------------------
     def begin_device_steps(self, memory_size: int, buffer_size: int) -> None:
@@ -639,13 +640,19 @@ class TrimKVCache(_SlabBacked):
         # not happen while a graph is being captured)
         from .attn import hip_attn
         s0 = slabs[0]
-        pps = hip_attn._uniform_cut(s0.nseg, hint)
-        self._device_pieces = None
-        if pps > 1 and s0.nseg <= 8192:
+        # A workgroup takes 128 rows in about 2.5 us, which joining pieces costs as well: only where a launch is not much more than that
+        # does a finer cut than 512 rows show.  Replayed steps of 8 Qwen3-1.7B layers, at least 512 -> 128 rows: 8 segments of 300 rows
+        # 425 -> 409 us, of 1000 435 -> 414, 32 of 600 463 -> 442; 8 of 4000 440 -> 438, 128 of 2048 628 -> 627.
+        pps = hip_attn._uniform_cut(s0.nseg, hint, 128 if hint <= 1024 else 0)
+        self._device_pieces = self._device_wholes = None
+        if s0.nseg < 256:
             seg = np.arange(s0.nseg, dtype=np.int32)
             rows = [np.stack([seg, np.full_like(seg, p), np.full_like(seg, pps), seg * pps], axis=1) for p in range(pps)]
             plist = torch.from_numpy(np.concatenate(rows, axis=0)).to(dev)      # piece-major: the segment is the fast axis
-            self._device_pieces = (plist, s0.nseg * pps)
+            if pps > 1:
+                self._device_pieces = (plist, s0.nseg * pps)
+            else:      # segments attended whole, as a list too: the launch without one splits its grid and joins the parts in a second one
+                self._device_wholes = (plist, s0.nseg)
         self.lengths_on_device = True
 
     def end_device_steps(self) -> None:
@@ -773,7 +780,7 @@ class TrimKVCache(_SlabBacked):
         extra = {"seg_len": slab.seg_len, "max_len": slab.max_len, "seg_cap": slab.cap}
         if self.lengths_on_device:
             extra["lengths_on_device"] = True
-            extra["device_pieces"] = self._device_pieces
+            extra["device_pieces"] = self._device_pieces or self._device_wholes
         if slab.pending is not None:
             # the last of the max_len rows is not in the slab yet: the attention call that receives this dictionary writes it
             extra["pending_append"] = (self, slab)
