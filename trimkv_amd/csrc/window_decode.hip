@@ -46,7 +46,10 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
     const int per = a.H / a.G, passes = (per + GQ - 1) / GQ;
     // heads on the fast axis: workgroups go to the eight XCDs in turn, and with the splits there the XCDs of the later ones, which
     // short sequences do not have, would idle
-    const int split = blockIdx.z, g = blockIdx.x / passes, h0 = (blockIdx.x % passes) * GQ, b = blockIdx.y;
+    // The sequences begin five further on with every split: with them in one order the shares of a sequence, a multiple of `batch`
+    // workgroups apart, meet on the same compute units (8 sequences of 256 .. 4096 rows 27.5 -> 20.8 us in one order, 25.5 -> 21.0 in
+    // another, 16 of them 32.8 -> 30.0 and 30.1 -> 31.1).
+    const int split = blockIdx.z, g = blockIdx.x / passes, h0 = (blockIdx.x % passes) * GQ, b = (int)((blockIdx.y + 5 * blockIdx.z) % gridDim.y);
     const int nh = min(GQ, per - h0);
     const int slot = a.slots[b], cap = a.keep + a.size;
     const int n = min(a.seen[2 * slot] + 1, cap);
@@ -209,14 +212,14 @@ static void launch_window_decode(const WindowArgs& a, int batch, hipStream_t s) 
 
 using namespace trimkv;
 
-constexpr int SHARE_ROWS = 1024;
+constexpr int SHARE_ROWS = 820;
 
 extern "C" int trimkv_window_decode_splits(int batch, int kv_heads, int capacity) {
     if (batch <= 0 || kv_heads <= 0 || capacity <= 0) return 1;
-    // Enough workgroups to fill the chip, at least 128 rows for each and no more than 1024: a batch's sequences differ in length, and
-    // the launch ends with the workgroup that has the most rows.  64 sequences of 256 .. 4096 rows x 8 heads of 128, a step of the
-    // two-layer decoder: 370 us with the splits on the fast axis of the grid, 347 with the heads there, 341 with 512 rows at most,
-    // which costs 64 full windows of 4096 rows 2 - 4 % (207 us).
+    // Enough workgroups to fill the chip, at least 128 rows for each and no more than 820: a batch's sequences differ in length, and
+    // the launch ends with the workgroup that has the most rows.  At most 1024, 820, 512 rows, us: 64 sequences of 256 .. 4096 rows x 8
+    // heads of 128 84, 75, 77 (in another order 83, 80, 79), of 64 .. 1024 rows 35, 31, 28, of full windows of 4096 180, 180, 187;
+    // 128 sequences of 256 .. 4096 141, 137, 139, of full windows 358, 365, 372.
     // With enough pairs to fill the chip as they are (2048) others run while the longest ones finish, and splitting costs full
     // windows more than it gives unequal ones.  With the bound of 1024 rows -> without, us, full windows | lengths from 256 rows
     // up (log-uniform): 2048 pairs of 4096 rows 705 -> 650 | 263 -> 288, 4096 of 4096 1434 -> 1281 | 520 -> 500, of 2048 720 -> 644 |
