@@ -358,3 +358,28 @@ def test_decode_of_sequences_with_fewer_rows_than_the_batch_is_split_for(dtype):
     row, some, and all of them, decoded side by side."""
     spec = ops.WindowSpec(2, 1, 64, 64, 1500, 20, 0.15)
     run_window(spec, dtype, [4, 128, 129, 400, 1600], [[1] * 4, [125, 1, 1, 1], [126, 1, 1, 1], [397, 1, 1, 1], [1597, 1, 1, 1]])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (3, 7, 4128), (64, 32, 4096), (64, 33, 2080), (512, 16, 64), (513, 16, 2048), (128, 16, 260), (129, 16, 4)])
+def test_linear_f32_on_either_side_of_its_rules(dtype, rows, n, k):
+    """Rows of a decode step and more: fp32 sums of k exact products (bf16 weights) or fp32 ones, in any order."""
+    gen = torch.Generator(device=DEV).manual_seed(rows + n + k)
+    ks = (k + 7) // 8 * 8
+    x, w = torch.randn(rows, k + 4, generator=gen, device=DEV), torch.randn(n, ks, generator=gen, device=DEV).to(dtype)[:, :k]
+    out = ops.linear_f32(x[:, :k], w)
+    exact, size = x[:, :k].double() @ w.double().T, x[:, :k].double().abs() @ w.double().abs().T
+    assert ((out.double() - exact).abs() <= (k + 2) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4, 30, 1028, 2048, 2052, 4096, 4100])
+def test_rms_rows_of_every_width(dtype, width):
+    gen = torch.Generator(device=DEV).manual_seed(width)
+    x, w = torch.randn(9, (width + 67) // 4 * 4, generator=gen, device=DEV) * 3, torch.randn(width, generator=gen, device=DEV)
+    rows = torch.tensor([8, 0, 3], device=DEV)
+    for r in (None, rows):
+        out = ops.rms_rows(x[:, :width] if r is None else x[:, :width], r, w, 1e-6, dtype)
+        src = x[:, :width].double() if r is None else x[rows, :width].double()
+        want = src * torch.rsqrt(src.square().mean(-1, keepdim=True) + 1e-6) * w.double()
+        assert ((out.double() - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20) * want.abs() + 1e-30).all()
