@@ -102,7 +102,8 @@ class GraphedDecoder:
         if not cache.lengths_on_device:
             raise RuntimeError("GraphedDecoder: the cache has left the device-side step mode (end_device_steps)")
         self.static_in.copy_(x)
-        self.position.fill_(cache.get_seq_length())
+        if not self.hybrid:        # a HybridCache counts on the device
+            self.position.fill_(cache.get_seq_length())
         self.calls += 1
         if self.graph is not None and self._epoch != decoder_ops.layout_epoch:
             # some decoder's parameters were moved into another buffer since the capture (a module replaced, a model moved):
