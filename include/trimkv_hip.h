@@ -358,6 +358,18 @@ int trimkv_compact_threshold_layers(const trimkv_layer_slabs* layers, int nlayer
                                     void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * trimkv_compact_threshold_halves -- the same with the keys and the values of a segment moved by a workgroup each and the rest put in
+ * place by a second launch: for few, long segments.  TRIMKV_SCORE_ALPHA only, max_len up to 32768; `workspace`: at least
+ * trimkv_compact_halves_workspace(...) bytes, 8-byte aligned, contents of no meaning before and after.
+ */
+int trimkv_compact_threshold_halves(const trimkv_layer_slabs* layers, int nlayers, int nseg, int segs_per_group, int head_dim,
+                                    int kv_dtype, int lb_dtype,
+                                    const uint32_t* thr_key, const int32_t* tie_take, int thr_layer_stride,
+                                    const int32_t* tie_base, int64_t q_idx, int strategy, int rounding, int max_len,
+                                    void* workspace, size_t workspace_bytes, void* stream);
+size_t trimkv_compact_halves_workspace(int nlayers, int nseg, int max_len);
+
+/*
  * trimkv_build_cu_seqlens -- cu[0] = 0, cu[i+1] = cu[i] + seg_len[i] (int32), the offsets the
  * reference rebuilds with torch.cumsum after every eviction (cache_utils.py:412-416, 830-834).
  */

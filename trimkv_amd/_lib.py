@@ -68,6 +68,8 @@ SIGNATURES = {
     "trimkv_evict_host_layers": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _i, _i, _i, _i, _i, _p, _sz, _p]),
     "trimkv_evict_listed": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _i, _i, _i64, _p, _i, _i, _i, _i, _p, _i, _p, _sz, _p]),
     "trimkv_compact_threshold_layers": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _i, _p, _i64, _i, _i, _i, _p, _sz, _p]),
+    "trimkv_compact_threshold_halves": (_i, [_p, _i, _i, _i, _i, _i, _i, _p, _p, _i, _p, _i64, _i, _i, _i, _p, _sz, _p]),
+    "trimkv_compact_halves_workspace": (_sz, [_i, _i, _i]),
     "trimkv_build_cu_seqlens": (_i, [_p, _i, _p, _p]),
     "trimkv_build_cu_seqlens_layers": (_i, [_p, _p, _i, _i, _p]),
     "trimkv_decode_attn_workspace": (_sz, [_i, _i, _i, _i, _i]),

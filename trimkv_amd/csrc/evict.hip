@@ -326,6 +326,45 @@ __device__ __forceinline__ void move_segment(char* kseg, char* vseg, void* lbseg
     }
 }
 
+// The same for one of the two arrays of a segment, twice the rows at a time.
+__device__ __forceinline__ void move_rows(char* seg, const uint32_t* idx, int kept, int first_moved, int row_bytes, int lpr_shift) {
+    constexpr int P = 2 * EV_ROW_PASSES;
+    const int rpp = EV_THREADS >> lpr_shift, rl = threadIdx.x >> lpr_shift, piece = threadIdx.x & ((1 << lpr_shift) - 1), tile_rows = rpp * P;
+    const bool piece_ok = (piece << 4) < row_bytes;
+    const int piece_off = piece_ok ? (piece << 4) : 0;
+    auto issue = [&](int base, uint4 (&t)[P], bool (&mv)[P]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const int r = base + p * rpp + rl, src = (int)idx[min(r, kept - 1)];
+            mv[p] = r < kept && piece_ok && src != r;
+            t[p] = load_stream(seg + (int64_t)src * row_bytes + piece_off);
+        }
+    };
+    auto retire = [&](int base, uint4 (&t)[P], const bool (&mv)[P]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) land(t[p]);
+        __syncthreads();   // every thread holds its rows of this tile: the tile's destinations may be overwritten
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            if (mv[p]) store_stream(seg + (int64_t)(base + p * rpp + rl) * row_bytes + (piece << 4), t[p]);
+    };
+    uint4 ta[P], tb[P];
+    bool ma[P], mb[P];
+    int base = (first_moved / tile_rows) * tile_rows;
+    if (base < kept) issue(base, ta, ma);
+    while (base < kept) {
+        const bool more = base + tile_rows < kept;          // uniform across the workgroup
+        if (more) issue(base + tile_rows, tb, mb);
+        retire(base, ta, ma);
+        base += tile_rows;
+        if (!more) break;
+        const bool more2 = base + tile_rows < kept;
+        if (more2) issue(base + tile_rows, ta, ma);
+        retire(base, tb, mb);
+        base += tile_rows;
+    }
+}
+
 struct EvictArgs {
     char* k_slab; char* v_slab; char* lb_slab; int64_t* pos_slab; int32_t* seg_len;
     int nseg, cap, max_len, row_bytes, lpr_shift, kv_dtype, lb_dtype;
@@ -344,6 +383,9 @@ struct EvictArgs {
     // rows moved by launches of their own (trimkv_evict_split): per pair {rows kept, first row that moves, its first chunk, -}, and
     // per chunk of the scratch the list of its kept rows and room for split_spill rows.  A pair has split_chunks chunks, or those
     // from split_first[pair] to split_first[pair + 1] - 1 of split_total, split_chunks of them at most
+    // keys and values moved by a workgroup each (trimkv_compact_threshold_halves): per pair {rows kept or -1, first row that moves} and,
+    // max_len apiece, the positions and log beta of its kept rows, which the launch behind this one puts in place
+    int2* half_head; int64_t* half_pos; uint32_t* half_lb;
     int4* split_head; uint32_t* split_idx; char* split_stash; const int32_t* split_first; int split_total, split_chunks, split_spill;
 };
 
@@ -502,6 +544,9 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
     if (SELECT && a.split_head && threadIdx.x == 0) a.split_head[pair_of_block(a)] = make_int4(0, 0, 0, 0);   // nothing left to move, unless said otherwise below
     const int seg = N > 0 || a.layers ? select_pair(a, table, pair_of_block(a)) : blockIdx.x;
     if (seg < 0) return;
+    const bool halves = !SELECT && a.half_head, values = halves && blockIdx.z;
+    const int64_t pair = pair_of_block(a);
+    if (values && threadIdx.x == 0) a.half_head[pair] = make_int2(-1, 0);
     const int n = a.seg_len[seg];
     // nothing cached, a corrupt length, or more rows than the caller's bound (which sized the key array): touch nothing
     if (n <= 0 || n > a.cap || n > a.max_len) return;
@@ -547,6 +592,17 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
     }
     const int kept = compact_indices(keys, n, thr, take_eq, eq_base, scratch, &first_evicted);
     const int first_moved = first_evicted;
+    if (halves) {        // both workgroups have read lengths, positions and log beta as they were: nothing of these is written here
+        if (first_moved < kept) move_rows(values ? vseg : kseg, keys, kept, first_moved, a.row_bytes, a.lpr_shift);
+        if (!values) return;
+        for (int r = first_moved + threadIdx.x; r < kept; r += EV_THREADS) {
+            const int src = (int)keys[r];
+            a.half_pos[pair * a.max_len + r] = posseg[src];
+            a.half_lb[pair * a.max_len + r] = lb_bytes == 4 ? ((const uint32_t*)lbseg)[src] : (uint32_t)((const uint16_t*)lbseg)[src];
+        }
+        if (threadIdx.x == 0) a.half_head[pair] = make_int2(kept, first_moved);
+        return;
+    }
     if (a.kept_idx) {
         for (int r = threadIdx.x; r < kept && r < a.kept_stride; r += EV_THREADS)
             a.kept_idx[(int64_t)seg * a.kept_stride + r] = (int32_t)keys[r];
@@ -560,6 +616,25 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
     } else if (first_moved < kept)
         move_segment(kseg, vseg, lbseg, posseg, keys, kept, first_moved, a.row_bytes, a.lpr_shift, lb_bytes);
     if (threadIdx.x == 0) a.seg_len[seg] = kept;
+}
+
+// Positions, log beta and lengths of a compaction whose keys and values were moved by workgroups of their own.
+template <int N>
+__global__ __launch_bounds__(256) void half_finish_kernel(EvictArgs a, const SlabTable<N> table) {
+    const int64_t pair = pair_of_block(a);
+    const int2 head = a.half_head[pair];
+    if (head.x < 0) return;
+    const int seg = select_pair(a, table, (int)pair);
+    if (seg < 0) return;
+    const int lb_bytes = a.lb_dtype == TRIMKV_F32 ? 4 : 2;
+    char* lbseg = a.lb_slab + (int64_t)seg * a.cap * lb_bytes;
+    for (int r = head.y + threadIdx.x; r < head.x; r += 256) {
+        a.pos_slab[(int64_t)seg * a.cap + r] = a.half_pos[pair * a.max_len + r];
+        const uint32_t lb = a.half_lb[pair * a.max_len + r];
+        if (lb_bytes == 4) ((uint32_t*)lbseg)[r] = lb;
+        else ((uint16_t*)lbseg)[r] = (uint16_t)lb;
+    }
+    if (threadIdx.x == 0) a.seg_len[seg] = head.x;
 }
 
 // ---- shared-budget selection over groups of segments ----------------------------------------
@@ -893,7 +968,7 @@ static int launch_evict(const char* fn, EvictArgs& a, int max_len, void* workspa
     const size_t key_bytes = (size_t)max_len * 4;
     a.max_len = max_len;
     a.nlayers = nlayers;
-    const dim3 grid = a.work ? dim3(nwork, 1) : dim3(a.nseg, nlayers);
+    const dim3 grid = a.work ? dim3(nwork, 1) : dim3(a.nseg, nlayers, a.half_head ? 2 : 1);
     if (key_bytes <= (size_t)EV_LDS_KEY_BYTES) {
         // allow more than the default 64 KB of dynamic LDS (gfx950 has 160 KB per workgroup): once per device and
         // instantiation; the flag is only ever set, so a race repeats the call at worst
@@ -1154,12 +1229,12 @@ extern "C" int trimkv_evict_host_layers(const trimkv_layer_slabs* host_layers, i
                                strategy, rounding, sliding_window, max_len, nullptr, 0, workspace, workspace_bytes, stream, table);
 }
 
-extern "C" int trimkv_compact_threshold_layers(const trimkv_layer_slabs* layers, int nlayers, int nseg, int segs_per_group, int head_dim,
-                                               int kv_dtype, int lb_dtype,
-                                               const uint32_t* thr_key, const int32_t* tie_take, int thr_layer_stride,
-                                               const int32_t* tie_base, int64_t q_idx, int strategy, int rounding, int max_len,
-                                               void* workspace, size_t workspace_bytes, void* stream) {
-    const char* fn = "trimkv_compact_threshold_layers";
+static size_t halves_bytes(int64_t pairs, int max_len) { return (size_t)pairs * (8 + 12 * (size_t)max_len); }
+
+static int compact_layers_common(const char* fn, bool halves, const trimkv_layer_slabs* layers, int nlayers, int nseg, int segs_per_group, int head_dim,
+                                 int kv_dtype, int lb_dtype, const uint32_t* thr_key, const int32_t* tie_take, int thr_layer_stride,
+                                 const int32_t* tie_base, int64_t q_idx, int strategy, int rounding, int max_len,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
     int lpr_shift;
     int rc = check_layer_args(fn, layers, nlayers, nseg, head_dim, kv_dtype, lb_dtype, max_len, &lpr_shift);
     if (rc) return rc;
@@ -1173,7 +1248,33 @@ extern "C" int trimkv_compact_threshold_layers(const trimkv_layer_slabs* layers,
     a.nseg = nseg; a.row_bytes = head_dim * 2; a.lpr_shift = lpr_shift; a.kv_dtype = kv_dtype; a.lb_dtype = lb_dtype;
     a.strategy = strategy; a.rounding = rounding; a.sliding_window = 0;
     a.thr_key = thr_key; a.tie_take = tie_take; a.tie_base = tie_base; a.segs_per_group = segs_per_group;
-    return launch_evict<false>(fn, a, max_len, workspace, workspace_bytes, (hipStream_t)stream, nlayers);
+    hipStream_t st = (hipStream_t)stream;
+    if (!halves) return launch_evict<false>(fn, a, max_len, workspace, workspace_bytes, st, nlayers);
+    if (strategy != TRIMKV_SCORE_ALPHA) return fail(TRIMKV_ERR_UNSUPPORTED, "%s: scores that read the keys while they move", fn);
+    const int64_t pairs = (int64_t)nlayers * nseg;
+    if ((size_t)max_len * 4 > (size_t)EV_LDS_KEY_BYTES) return fail(TRIMKV_ERR_SHAPE, "%s: max_len=%d exceeds %d", fn, max_len, EV_LDS_KEY_BYTES / 4);
+    if (!workspace || workspace_bytes < halves_bytes(pairs, max_len) || (uintptr_t)workspace & 7)
+        return fail(TRIMKV_ERR_WORKSPACE, "%s: an 8-byte aligned workspace of %zu bytes needed, got %zu", fn, halves_bytes(pairs, max_len), workspace_bytes);
+    a.half_head = (int2*)workspace;
+    a.half_pos = (int64_t*)(a.half_head + pairs);
+    a.half_lb = (uint32_t*)(a.half_pos + pairs * max_len);
+    if (int bad = launch_evict<false>(fn, a, max_len, nullptr, 0, st, nlayers)) return bad;
+    hipLaunchKernelGGL(half_finish_kernel<0>, dim3(nseg, nlayers), dim3(256), 0, st, a, SlabTable<0>{});
+    return launch_status(fn);
+}
+
+#define TRIMKV_COMPACT_PARAMS                                                                                                                   \
+    const trimkv_layer_slabs *layers, int nlayers, int nseg, int segs_per_group, int head_dim, int kv_dtype, int lb_dtype,                      \
+        const uint32_t *thr_key, const int32_t *tie_take, int thr_layer_stride, const int32_t *tie_base, int64_t q_idx, int strategy,           \
+        int rounding, int max_len, void *workspace, size_t workspace_bytes, void *stream
+#define TRIMKV_COMPACT_ARGS                                                                                                                     \
+    layers, nlayers, nseg, segs_per_group, head_dim, kv_dtype, lb_dtype, thr_key, tie_take, thr_layer_stride, tie_base, q_idx, strategy,        \
+        rounding, max_len, workspace, workspace_bytes, stream
+
+extern "C" int trimkv_compact_threshold_layers(TRIMKV_COMPACT_PARAMS) { return compact_layers_common("trimkv_compact_threshold_layers", false, TRIMKV_COMPACT_ARGS); }
+extern "C" int trimkv_compact_threshold_halves(TRIMKV_COMPACT_PARAMS) { return compact_layers_common("trimkv_compact_threshold_halves", true, TRIMKV_COMPACT_ARGS); }
+extern "C" size_t trimkv_compact_halves_workspace(int nlayers, int nseg, int max_len) {
+    return nlayers <= 0 || nseg <= 0 || max_len <= 0 ? 0 : halves_bytes((int64_t)nlayers * nseg, max_len);
 }
 
 static int group_threshold_common(const char* fn, int per_layer, const void* const* lb_slabs, const int64_t* const* pos_slabs,
