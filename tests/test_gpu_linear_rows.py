@@ -135,6 +135,37 @@ def test_modules_that_somebody_hooked_wrapped_or_replaced_are_called():
     assert torch.equal(linear.run(twice, x), 2 * nn.functional.linear(x, twice.weight, twice.bias))
 
 
+def test_modules_with_a_forward_of_their_own_are_not_asked_to_leave_a_product():
+    """Subclasses written before there was such an argument: the decoder calls them as it always did."""
+    from trimkv_amd import qwen3
+    from tests.test_gpu_qwen3_shell import _family, _tiny_config
+    cfg = _tiny_config("qwen3")
+    torch.manual_seed(0)
+    model = _family("qwen3")[1](cfg).eval()
+    layer, above = model.model.layers[:2]
+    assert all(linear.may_leave(m) for m in (layer, layer.mlp, layer.self_attn))
+
+    class OwnMLP(qwen3.MLP):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    class OwnAttention(type(layer.self_attn)):
+        def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position):
+            return torch.zeros_like(hidden_states)
+
+    class OwnLayer(type(layer)):
+        def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending=None):
+            return hidden_states + pending, torch.ones_like(hidden_states)
+    above.__class__, layer.mlp.__class__, layer.self_attn.__class__ = OwnLayer, OwnMLP, OwnAttention
+    assert not any(linear.may_leave(m) for m in (above, layer.mlp, layer.self_attn))
+    with torch.no_grad():
+        h, mlp = torch.randn(1, 6, cfg.hidden_size), layer.mlp
+        total, out = layer(h, (None, None), None, None, None, leave_product=True)
+        x = layer.post_attention_layernorm(h)
+        assert torch.equal(total, h) and torch.allclose(out, 2 * mlp.down_proj(nn.functional.silu(mlp.gate_proj(x)) * mlp.up_proj(x)))
+        assert torch.equal(above(total, None, None, None, None, out)[0], h + out)
+
+
 def _normed(x, norm):
     """What the modules make of x, in 64 bits between their two roundings."""
     h = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + norm.variance_epsilon)

@@ -89,6 +89,17 @@ def untouched(module: nn.Module) -> bool:
     return type(module) is nn.Linear and unhooked(module)
 
 
+def leaving(forward):
+    """Marks a module's ``forward`` that takes ``leave_product``; what a subclass puts in its place need not."""
+    forward.leaves_product = True
+    return forward
+
+
+def may_leave(module: nn.Module) -> dict:
+    """The keyword argument with which ``module`` may leave its last product to the caller, if it knows it and nobody looks at its output."""
+    return {"leave_product": True} if getattr(type(module).forward, "leaves_product", False) and unhooked(module) else {}
+
+
 NORM_ROWS, NORM_K = 32, 8192      # what trimkv_linear_rows_add and trimkv_linear_rows_norm take
 
 

@@ -46,6 +46,7 @@ class Phi3MLP(nn.Module):
     def takes_deferred(self, x: torch.Tensor) -> bool:
         return type(self).forward is Phi3MLP.forward
 
+    @linear.leaving
     def forward(self, x: torch.Tensor, leave_product: bool = False) -> torch.Tensor:
         if linear.untouched(self.gate_up_proj):
             act = decoder_ops.silu_product(x, self.gate_up_proj.weight)

@@ -192,6 +192,7 @@ class MLP(nn.Module):
     def takes_deferred(self, x: torch.Tensor) -> bool:
         return type(self).forward is MLP.forward
 
+    @linear.leaving
     def forward(self, x: torch.Tensor, leave_product: bool = False) -> torch.Tensor:
         """``x``: also a ``linear.DeferredNorm``; ``leave_product``: the last product may come back as a ``linear.DeferredProduct``."""
         fused = self.__dict__.get("_gate_up")
@@ -411,6 +412,7 @@ class TrimKVQwen3Attention(nn.Module):
             return False
         return self.config.retention_gate != "rg" or (self.fold_gate and not self.gate_on_side_stream and getattr(self.retention_gate, "_use_hip", lambda x: False)(x))
 
+    @linear.leaving
     def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, leave_product: bool = False):
         """``hidden_states``: also a ``linear.DeferredNorm`` (see ``takes_deferred``); ``leave_product``: the last product may come back
         as a ``linear.DeferredProduct``."""
@@ -459,6 +461,7 @@ class TrimKVQwen3DecoderLayer(nn.Module):
         self.input_layernorm = RMSNorm(config.hidden_size, config.rms_norm_eps)
         self.post_attention_layernorm = RMSNorm(config.hidden_size, config.rms_norm_eps)
 
+    @linear.leaving
     def forward(self, hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending=None, leave_product: bool = False):
         """``pending``: the MLP output of the layer below, not yet added to ``hidden_states`` -- the add (qwen3:437) then rides
         in this layer's first norm.  Returns ``(hidden_states, mlp_out)`` with the same add left to whoever comes next;
@@ -468,10 +471,9 @@ class TrimKVQwen3DecoderLayer(nn.Module):
             normed = self.input_layernorm(hidden_states)
         else:
             normed, hidden_states = self._add_norm(self.input_layernorm, pending, hidden_states, attn)
-        leaves = lambda module: {"leave_product": True} if hasattr(module, "takes_deferred") and linear.unhooked(module) else {}
-        attn_out = attn(normed, position_embeddings, attention_mask, past_key_values, cache_position, **leaves(attn))
+        attn_out = attn(normed, position_embeddings, attention_mask, past_key_values, cache_position, **linear.may_leave(attn))
         normed, hidden_states = self._add_norm(self.post_attention_layernorm, attn_out, hidden_states, mlp)   # qwen3:431-435
-        return hidden_states, mlp(normed, **(leaves(mlp) if leave_product else {}))
+        return hidden_states, mlp(normed, **(linear.may_leave(mlp) if leave_product else {}))
 
     @staticmethod
     def _add_norm(norm, x, residual, reader):
@@ -518,7 +520,7 @@ class TrimKVQwen3Model(nn.Module):
         hidden_states = inputs_embeds
         pending = None    # the last MLP output; its residual add rides in the next norm
         for layer in self.layers:
-            leave = {"leave_product": True} if type(layer).forward is TrimKVQwen3DecoderLayer.forward and linear.unhooked(layer) else {}
+            leave = linear.may_leave(layer)
             hidden_states, pending = layer(hidden_states, position_embeddings, attention_mask, past_key_values, cache_position, pending if leave else linear.tensor_of(pending), **leave)
         hidden_states = self.norm(hidden_states) if pending is None else self.norm.add_norm(linear.tensor_of(pending), hidden_states)[0]
         c = self.config
