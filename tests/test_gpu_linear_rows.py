@@ -166,6 +166,25 @@ def test_modules_with_a_forward_of_their_own_are_not_asked_to_leave_a_product():
         assert torch.equal(above(total, None, None, None, None, out)[0], h + out)
 
 
+@pytest.mark.gpu
+def test_who_follows_operations_gets_the_general_product():
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w, bias = _operands(8, 64, 128, torch.bfloat16, 9)
+    with torch.no_grad():
+        want = nn.functional.linear(x, w, bias)
+        assert torch.equal(torch.func.vmap(lambda row: linear.linear(row, w, bias))(x), torch.func.vmap(lambda row: nn.functional.linear(row, w, bias))(x))
+        assert linear._rows(x, w, bias) is not None
+        with forward_ad.dual_level():
+            tangent = forward_ad.unpack_dual(linear.linear(forward_ad.make_dual(x, torch.ones_like(x)), w)).tangent
+        assert torch.equal(tangent, nn.functional.linear(torch.ones_like(x), w))
+        with FlopCounterMode(display=False) as counted:
+            assert torch.equal(linear.linear(x, w, bias), want)
+        assert counted.get_total_flops() == 2 * x.shape[0] * w.numel()
+        traced = torch.jit.trace(lambda t: linear.linear(t, w, bias), x, check_trace=False)
+        assert torch.equal(traced(x + 1), nn.functional.linear(x + 1, w, bias))
+
+
 def _normed(x, norm):
     """What the modules make of x, in 64 bits between their two roundings."""
     h = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + norm.variance_epsilon)

@@ -9,6 +9,7 @@ from typing import Optional
 import torch
 from torch import nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
 from . import _lib
@@ -16,10 +17,17 @@ from . import _lib
 MAX_ROWS = 64      # rows that trimkv_linear_rows takes
 
 
+def _watched() -> bool:
+    """Somebody follows the operations themselves (vmap and torch.func, forward-mode derivatives, tracing, compiling, dispatch modes): a
+    launch of ours would be lost on them, and inside of vmap a tensor has no address."""
+    return (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0)
+
+
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary tensors of one 16-bit dtype on the current GPU that nobody differentiates or casts."""
+    """Ordinary tensors of one 16-bit dtype on the current GPU that nobody differentiates, casts or follows."""
     first = tensors[0]
-    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda"):
+    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or _watched():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
