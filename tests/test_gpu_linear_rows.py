@@ -29,13 +29,14 @@ def _check(got, x, w, bias, dtype):
     assert (err <= bound).all(), (float((err - bound).max()), (err > bound).nonzero()[:4].tolist())
 
 
-# rows: every number of row groups and their edges; n: ends of 16-row blocks and, from 4608 on, every number of blocks per tile and more
+# rows: every number of row groups and their edges; n: ends of 8-row (up to 2048) and 16-row blocks and, from 4608 on, every number of blocks per tile and more
 # tiles than workgroups; k: fewer steps than wavefronts, numbers that do not divide among them
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 64), (1, 15, 128), (7, 16, 192), (8, 17, 320), (9, 40, 64), (16, 100, 1024), (17, 33, 448), (31, 2048, 512), (32, 18, 64), (33, 1000, 704),
                                       (63, 47, 576), (64, 4096, 256), (1, 4608, 128), (16, 4612, 192), (32, 12288, 64), (5, 12291, 64), (64, 12280, 128), (64, 24576, 64),
-                                      (50, 24600, 128), (8, 70001, 64), (16, 50000, 64), (64, 50002, 64)])
+                                      (50, 24600, 128), (8, 70001, 64), (16, 50000, 64), (64, 50002, 64),
+                                      (1, 7, 64), (8, 8, 128), (33, 9, 64), (16, 2041, 192), (64, 2048, 704), (8, 2049, 64), (24, 2056, 64)])
 def test_linear_rows_matches_the_product(rows, n, k, dtype):
     x, w, bias = _operands(rows, n, k, dtype, rows + n + k)
     got = linear.linear(x, w)
@@ -194,19 +195,19 @@ def _normed(x, norm):
 # rows: every number of row groups and their edges; n: every number of blocks per tile, a last tile that is moved back, more tiles than
 # workgroups; k: fewer steps than wavefronts, numbers that do not divide among them
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,n,k", [(1, 64, 64), (3, 320, 8192), (8, 4608, 192), (9, 112, 576), (16, 4624, 1024), (17, 64, 2048), (32, 2048, 704), (29, 8192, 128), (32, 8208, 64), (5, 50000, 64)])
+@pytest.mark.parametrize("rows,n,k", [(1, 64, 64), (3, 320, 8192), (8, 4608, 192), (9, 112, 576), (16, 4624, 1024), (17, 64, 2048), (32, 2048, 704), (29, 8192, 128), (32, 8208, 64), (5, 50000, 64), (16, 2048, 128), (8, 2064, 64), (1, 16, 64)])
 def test_linear_rows_with_a_residual(rows, n, k):
     x, w, bias = _operands(rows, n, k, torch.bfloat16, rows + n + k)
     wide = torch.zeros(rows, 1, n + 4, dtype=torch.bfloat16, device=DEV)
     wide[..., 4:] = torch.randn(rows, 1, n, generator=torch.Generator(device=DEV).manual_seed(k), device=DEV) * 3
     res = wide[..., 4:]
     for b in (None, bias):
-        out, squares = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV), torch.full((rows, n // 16), float("nan"), device=DEV)
+        out, squares = torch.empty(rows, n, dtype=torch.bfloat16, device=DEV), torch.full((rows, n // 8), float("nan"), device=DEV)
         _lib.check(_lib.load().trimkv_linear_rows_add(x.data_ptr(), k, w.data_ptr(), k, _lib.ptr(b), res.data_ptr(), n + 4, out.data_ptr(), n, squares.data_ptr(),
                                                       rows, n, k, _lib.BF16, _lib.current_stream(x.device)), "trimkv_linear_rows_add")
         assert torch.equal(out, linear.linear(x, w, b) + res[:, 0])
-        want = out.double().square().view(rows, n // 16, 16).sum(-1)
-        assert ((squares.double() - want).abs() <= 16 * 2.0 ** -24 * want).all()
+        want = out.double().square().view(rows, n // 8, 8).sum(-1)
+        assert ((squares.double() - want).abs() <= 8 * 2.0 ** -24 * want).all()
 
 
 @pytest.mark.gpu
@@ -222,7 +223,7 @@ def test_linear_rows_behind_a_norm(rows, n, k, silu):
     norm = RMSNorm(k, 1e-6).to(torch.bfloat16).to(DEV)
     norm.weight.data.normal_(1.0, 0.3, generator=torch.Generator(device=DEV).manual_seed(k))
     h = _normed(x, norm)
-    squares = x.float().square().view(rows, k // 16, 16).sum(-1)
+    squares = x.float().square().view(rows, k // 8, 8).sum(-1)
     for b in (None, bias):
         with torch.no_grad():
             d = linear.DeferredNorm(x, squares, norm)

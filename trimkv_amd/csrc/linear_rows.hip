@@ -15,15 +15,15 @@
 //    8 x 8) different lines is served one lane at a time: 16 B/clk per compute unit.  LDS-direct loads whose lanes run along
 //    the rows (8 rows x 128 bytes each) take in 28 B/clk; ds_read_b128 does the regrouping.  12288 x 2048 with 16 rows: 19 us
 //    with operand-layout loads, 11.4 here; 4096 x 4096 with 64 rows: 23.4 and 13.7;
-//  * a workgroup takes 16 NT rows of w, with NT chosen so that the busiest compute unit takes in least (rows_plan below);
+//  * a workgroup takes 16 NT rows of w, or 8, chosen so that the busiest compute unit takes in least (rows_plan below);
 //  * the wavefronts of a workgroup take turns on k, 64 elements at a time, each with a ring of its own, so that the main loop
 //    has no barrier; their sums meet in LDS at the end of a tile while the next tile's loads are already under way.
 //
 // Measured in a graph of launches over matrices that no cache holds, us here | the vendor library's product:
 //            n x k      1 row        16 rows      32 rows      64 rows
-//      2048 x 2048    5.0 | 10.9    5.5 | 11.1    6.2 | 11.2    8.2 | 11.8
+//      2048 x 2048    4.3 | 10.9    5.0 | 11.1    6.1 | 11.2    7.9 | 11.8
 //     12288 x 2048   11.7 | 16.6   11.4 | 16.7   12.2 | 16.9   14.8 | 18.2
-//      2048 x 6144    8.7 | 11.1   10.3 | 11.3   13.4 | 16.6   18.3 | 19.5
+//      2048 x 6144    7.3 | 11.1    8.6 | 11.3   11.5 | 16.6   17.2 | 19.5
 //      4096 x 4096    8.3 | 15.7    9.3 | 15.5   10.4 | 13.4   13.7 | 15.2
 //     10240 x 4096   16.3 | 26.6   16.6 | 27.8   18.3 | 23.6   22.5 | 29.6
 //     24576 x 4096   34.4 | 45.2   35.5 | 45.5   36.8 | 50.2   42.1 | 50.1
@@ -46,9 +46,9 @@ struct LinearRowsArgs {
     int m, n, k;        // n: columns of out
     int vec;            // four columns of out can be stored at once
     int round_all;      // silu: the two products and silu(gate) are rounded before they are used, as modules do
-    // a residual added to the product: the sums of the squares of what is stored, 16 columns at a time, go to squares [m][n / 16]
+    // a residual added to the product: the sums of the squares of what is stored, 8 columns at a time, go to squares [m][n / 8]
     const uint16_t* res; int64_t res_stride;
-    // an RMS norm of x in front of the product: its weight; squares [m][k / 16] as above
+    // an RMS norm of x in front of the product: its weight; squares [m][k / 8] as above
     const uint16_t* norm_w; float eps;
     float* squares;
 };
@@ -82,20 +82,22 @@ __device__ __forceinline__ void lr_load_to_lds(const uint16_t* base, uint32_t of
                      : "=&s"(saved) : "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
-// XG groups of 8 rows of x, NT blocks of 16 rows of w (SILU: NT / 2 of gate, NT / 2 of up), W wavefronts, D steps of 64 elements
+// XG groups of 8 rows of x, NT blocks of 16 rows of w (SILU: NT / 2 of gate, NT / 2 of up; HALF: one of 8), W wavefronts, D steps of 64 elements
 // of k in flight per wavefront.  A step in LDS: row r holds its eight 16-byte pieces rotated by r / 2, which spreads the 16 rows of
 // an operand read over all banks (the rotation is in the lanes' source addresses).
 // A decoder's residual add and RMS norm have no launch of their own (4.6 us, most of it latency): the product in front of them (ADD)
 // adds the residual where it rounds and leaves sums of squares, a few KB that the product behind them (NORM) adds up while its first
 // operands are on their way; x becomes round(round(x / rms) * weight), as modules round, on its way from LDS to the matrix cores.
 // A layer's four products with adds and norms, 16 rows: 43.6 -> 40.2 us at 2048 features and 6144, 92.0 -> 83.5 at 4096 and 12288; 1 row
-// 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102.  With more rows the arithmetic on the way no longer hides.
+// 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102 (all in blocks of 16).  With more rows the arithmetic on the way no longer hides.
 enum { LR_PLAIN = 0, LR_ADD = 1, LR_NORM = 2 };
-template <bool F16, bool SILU, int MODE, int XG, int NT, int W, int D>
+template <bool F16, bool SILU, int MODE, int XG, int NT, int W, int D, bool HALF>
 __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     constexpr bool NORM = MODE == LR_NORM, ADD = MODE == LR_ADD;
     static_assert(MODE == LR_PLAIN || !F16, "bf16 only");
-    constexpr int MT = (XG + 1) / 2, L = 2 * NT + XG, STEP = L * 1024, U = NT * MT, NB = SILU ? NT / 2 : NT;
+    constexpr int COLS = HALF ? 8 : 16, WG = COLS / 8;       // rows of w in a block, and loads of a step for them
+    constexpr int MT = (XG + 1) / 2, L = WG * NT + XG, STEP = L * 1024, U = NT * MT, NB = SILU ? NT / 2 : NT;
+    static_assert(!HALF || (NT == 1 && !SILU), "one half block");
     static_assert((D - 1) * L < 64, "the wait counts at most 63 loads");
     __shared__ __attribute__((aligned(1024))) char ring[W * D * STEP];
     __shared__ lr_f32x4 part[U * (W - 1)][64];
@@ -105,9 +107,9 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     const uint32_t ring_at = (uint32_t)(uintptr_t)(LR_LDS char*)ring + wave * D * STEP;
     const char* mine = ring + wave * D * STEP;
     // a load brings rows 8 j + lane / 8 of a block, position lane % 8; rows that are not there repeat the last one
-    uint32_t w_off[2], x_off[XG];
+    uint32_t w_off[WG], x_off[XG];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < WG; ++j) {
         const int row = 8 * j + (lane >> 3);
         w_off[j] = (uint32_t)(min(row, a.n - 1) * a.w_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
     }
@@ -116,9 +118,9 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         const int row = 8 * j + (lane >> 3);
         x_off[j] = (uint32_t)(min(row, a.m - 1) * a.x_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
     }
-    const int steps = a.k >> 6, first = min(wave, steps - 1), per_tile = (steps - wave + W - 1) / W, tiles = (a.n + 16 * NB - 1) / (16 * NB);
+    const int steps = a.k >> 6, first = min(wave, steps - 1), per_tile = (steps - wave + W - 1) / W, tiles = (a.n + COLS * NB - 1) / (COLS * NB);
     // the first column of block b of a tile: the last block of out is moved back so that all its rows exist
-    auto block_at = [&](int tile, int b) __attribute__((always_inline)) { return min((tile * NB + b % NB) * 16, max(a.n - 16, 0)); };
+    auto block_at = [&](int tile, int b) __attribute__((always_inline)) { return min((tile * NB + b % NB) * COLS, max(a.n - COLS, 0)); };
     int ask_tile = blockIdx.x, ask_step = first, ask_slot = 0;
     auto request = [&]() __attribute__((always_inline)) {
         const uint32_t to = ring_at + ask_slot * STEP;
@@ -126,10 +128,10 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         for (int b = 0; b < NT; ++b) {
             const uint16_t* from = a.w + (int64_t)(block_at(ask_tile, b) + (SILU && b >= NB ? a.n : 0)) * a.w_stride + ask_step * 64;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) lr_load_to_lds<true>(from, w_off[j], to + (2 * b + j) * 1024);
+            for (int j = 0; j < WG; ++j) lr_load_to_lds<true>(from, w_off[j], to + (WG * b + j) * 1024);
         }
 #pragma unroll
-        for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (2 * NT + j) * 1024);
+        for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (WG * NT + j) * 1024);
         ask_step += W;
         if (ask_step >= steps) {        // behind the last tile: its steps again, never read
             ask_step = first;
@@ -142,8 +144,8 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     if constexpr (NORM) {       // the weight of the norm: 512 elements a load, of a last one with fewer the last 8 again
         const uint32_t at = (uint32_t)(uintptr_t)(LR_LDS uint16_t*)norm_w;
         for (int p = wave; p * 512 < a.k; p += W) lr_load_to_lds<false>(a.norm_w, (uint32_t)min(p * 512 + lane * 8, a.k - 8) * 2, at + p * 1024);
-        const float* from = a.squares + (int64_t)min((int)threadIdx.x / ROW_THREADS, a.m - 1) * (a.k >> 4);
-        for (int c = (threadIdx.x % ROW_THREADS) * 4; c < a.k >> 4; c += ROW_THREADS * 4) {
+        const float* from = a.squares + (int64_t)min((int)threadIdx.x / ROW_THREADS, a.m - 1) * (a.k >> 3);
+        for (int c = (threadIdx.x % ROW_THREADS) * 4; c < a.k >> 3; c += ROW_THREADS * 4) {
             const lr_f32x4 f = *(const lr_f32x4*)(from + c);
             sum += (f[0] + f[1]) + (f[2] + f[3]);
         }
@@ -170,11 +172,14 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
-                for (int b = 0; b < NT; ++b) wf[h][b] = *(const lr_u32x4*)(p + (b * 16 + r) * 128 + ((h * 4 + g + (r >> 1)) & 7) * 16);
+                for (int b = 0; b < NT; ++b) {
+                    const int row = HALF ? r & 7 : b * 16 + r;          // a half block: rows 8 .. 15 repeat it
+                    wf[h][b] = *(const lr_u32x4*)(p + row * 128 + ((h * 4 + g + ((HALF ? row : r) >> 1)) & 7) * 16);
+                }
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
                     const int row = XG == 1 ? r & 7 : t * 16 + r;       // 8 rows: columns 8 .. 15 repeat them
-                    xf[h][t] = *(const lr_u32x4*)(p + (NT * 16 + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
+                    xf[h][t] = *(const lr_u32x4*)(p + (NT * COLS + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
                 }
                 if constexpr (NORM) nf[h] = *(const lr_u32x4*)(norm_w + (wave + s * W) * 64 + (h * 4 + g) * 8);
             }
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         };
 #pragma unroll
         for (int u = 0; u < NB * MT; ++u) {
-            if (owner(u) != wave) continue;
+            if (owner(u) != wave || (HALF && g >= 2)) continue;
             const int m = u % MT * 16 + r, n = block_at(tile, u / MT) + 4 * g;      // this lane: columns n .. n + 3 of row m
             if (m >= a.m && !ADD) continue;
             lr_f32x4 f = total(u);
@@ -249,9 +254,8 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
                     sq = fmaf(x, x, sq);
                 }
                 sq += __shfl_xor(sq, 16, 64);
-                sq += __shfl_xor(sq, 32, 64);
                 if (m >= a.m) continue;
-                if (g == 0) a.squares[(int64_t)m * (a.n >> 4) + (n >> 4)] = sq;
+                if ((g & 1) == 0) a.squares[(int64_t)m * (a.n >> 3) + (n >> 3)] = sq;
             }
             uint16_t* o = a.out + (int64_t)m * a.out_stride + n;
             if (a.vec) *(uint2*)o = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
@@ -269,7 +273,12 @@ constexpr int LR_CUS = 256;
 // Blocks of 16 rows of w per tile.  A compute unit that runs `rounds` tiles takes in rounds * (rows of w + rows of x) * k elements;
 // the least of that is the fastest (n x k = 12288 x 2048, 16 rows: one block 3 x 32, three blocks 1 x 64: 13.6 and 11.4 us;
 // 4608 x 2048, 64 rows: 2 x 80, 96, 112: 13.1, 10.6, 12.5).  Among equals the smaller one.
-static int rows_plan(int n, int x_rows, bool silu) {
+// 0: half a block, 8 rows, for n up to 2048, where 16 apiece leave half of the compute units idle and take in more for each.  16 -> 8
+// rows, us: 2048 x 6144 with 1, 16, 32, 64 rows of x 8.6 -> 7.3, 10.3 -> 8.6, 13.3 -> 11.5, 18.5 -> 17.2; 2048 x 2048 4.8 -> 4.3, 5.5 -> 5.0,
+// 6.3 -> 6.1, 8.3 -> 7.9; 1024 x 4096 6.3 -> 5.6, 7.2 -> 6.3, 9.0 -> 7.9, 12.4 -> 11.4; 512 x 2048 4.4 -> 4.1, 5.2 -> 4.9, 6.0 -> 5.7, 7.8 -> 7.5.  Half
+// of the matrix cores' rows are repeats then, which nothing waits for.  From 2049 on 8 rows apiece would be two rounds.
+static int rows_plan(int n, int x_rows, bool silu, bool half) {
+    if (half && !silu && n <= 8 * LR_CUS) return 0;
     static const int plain[] = {1, 2, 3, 6}, paired[] = {2, 4, 6};
     const int* sizes = silu ? paired : plain;
     int best = sizes[0];
@@ -283,17 +292,19 @@ static int rows_plan(int n, int x_rows, bool silu) {
     return best;
 }
 
-template <bool F16, bool SILU, int XG, int NT, int W, int D, int MODE = LR_PLAIN>
+template <bool F16, bool SILU, int XG, int NT, int W, int D, int MODE = LR_PLAIN, bool HALF = false>
 static void rows_launch(const LinearRowsArgs& a, hipStream_t s) {
-    constexpr int NB = SILU ? NT / 2 : NT, LDS = W * D * (2 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024 + (MODE == LR_NORM ? LR_NORM_K * 2 + LR_NORM_ROWS * 4 : 16);
+    constexpr int COLS = HALF ? 8 : 16, NB = SILU ? NT / 2 : NT, LDS = W * D * (COLS / 8 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024 + (MODE == LR_NORM ? LR_NORM_K * 2 + LR_NORM_ROWS * 4 : 16);
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
-    const int tiles = (a.n + 16 * NB - 1) / (16 * NB), most = LR_CUS * (160 * 1024 / LDS);
-    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NT, W, D>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
+    const int tiles = (a.n + COLS * NB - 1) / (COLS * NB), most = LR_CUS * (160 * 1024 / LDS);
+    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NT, W, D, HALF>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
 }
 // wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 6 over the shapes above
 template <bool F16, int XG, int MODE = LR_PLAIN>
 static void rows_by_blocks(const LinearRowsArgs& a, bool silu, hipStream_t s) {
-    const int nt = rows_plan(a.n, 8 * XG, silu);
+    const int nt = rows_plan(a.n, 8 * XG, silu, MODE != LR_NORM);
+    if constexpr (MODE != LR_NORM)
+        if (nt == 0) return rows_launch<F16, false, XG, 1, 4, XG < 4 ? 4 : XG < 8 ? 3 : 2, MODE, true>(a, s);
     if constexpr (MODE == LR_NORM) {
         if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, XG < 4 ? 3 : 2, MODE>(a, s);
         if (silu) return rows_launch<F16, true, XG, 2, 4, 3, MODE>(a, s);

@@ -164,7 +164,7 @@ def add_product(p: DeferredProduct, residual: torch.Tensor):
     x2, n = _rows(p.x, w, bias), w.shape[0]
     rows, k = x2.shape
     out = torch.empty(residual.shape, dtype=residual.dtype, device=residual.device)
-    squares = torch.empty(rows, n // 16, dtype=torch.float32, device=residual.device)
+    squares = torch.empty(rows, n // 8, dtype=torch.float32, device=residual.device)
     _lib.check(_lib.load().trimkv_linear_rows_add(x2.data_ptr(), x2.stride(0) if rows > 1 else k, w.data_ptr(), w.stride(0), _lib.ptr(bias), residual.data_ptr(), n,
                                                   out.data_ptr(), n, squares.data_ptr(), rows, n, k, _lib.BF16, _lib.current_stream(residual.device)), "trimkv_linear_rows_add")
     return out, squares
