@@ -640,7 +640,7 @@ int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_stride_h, i
  * `workspace`: at least trimkv_prefill_split_workspace(...) bytes, 16-byte aligned, contents of no meaning before and after.
  * trimkv_prefill_split_tiles: the split_tiles at which this is expected to be faster than one workgroup per query tile, or 0
  * where it is not.  uneven: 0 if the segments are about as long as the longest, whose length is max_len; else their mean length
- * in percent of it, or 1 if all that is known is that they differ much (of no consequence for these two kernels).
+ * in percent of it, or 1 if all that is known is that they differ much.
  * Returns TRIMKV_OK or a negative trimkv_status (as trimkv_prefill_attn; split_tiles <= 0 or a workspace that is too small).
  */
 int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven);

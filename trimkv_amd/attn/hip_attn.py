@@ -255,8 +255,8 @@ def prefill_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.T
             k_rows.data_ptr(), v_rows.data_ptr(), _lib.ptr(seg_len), _lib.ptr(seg_start),
             batch, kv_heads, group, Q, cap, D, _lib.dtype_code(query.dtype), float(scale), max_len)
     stream = _lib.current_stream(query.device)
-    tiles, need = _prefill_split(batch, kv_heads, group, Q, max_len, uneven)
-    shares = 0 if tiles else _prefill_shares(batch, kv_heads, group, Q, max_len, uneven)
+    shares = _prefill_shares(batch, kv_heads, group, Q, max_len, uneven)
+    tiles, need = (0, 0) if shares else _prefill_split(batch, kv_heads, group, Q, max_len, uneven)
     if tiles or shares:   # few query tiles: their keys divided among several workgroups; more: all keys in equal shares where that pays
         try:
             work = torch.empty(need or shares, dtype=torch.uint8, device=query.device)

@@ -977,8 +977,10 @@ extern "C" int trimkv_prefill_attn(const void* q, int64_t q_stride_b, int64_t q_
 // for the merge's launch, 0.8 us per share that a row's merge walks, 0.045 us per workgroup for its 130 KB written and read.
 // Measured (us, D 128, whole -> split): 8 tiles of 2048 keys 44 -> 21, of 8192 keys 150 -> 31; 32 of 4096 79 -> 35; 56 of 2954
 // 64 -> 37; 96 of 4096 80 -> 57; 128 of 8192 155 -> 107; left whole: 96 of 2048 44 -> 40, of 1024 27 -> 30, 40 of 1024 27 -> 25.
-// More query tiles: equal shares (below) or whole.
-extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int /*uneven*/) {
+// Between 128 and 256 tiles: for callers that do not take equal shares (below), which are faster there.  Of unlike segments the longest
+// one holds up the rest, and three shares let the others' CUs help: 160 and 168 tiles, mean length / longest 0.60 of 4100 keys 83 -> 79,
+// 0.68 of 8192 151 -> 136; 192 tiles, 0.53 of 8192 153 -> 131; 224, 0.52 of 10000 194 -> 166, but 0.57 of 8192 166 -> 177.
+extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
     if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len <= 0 || max_len <= 0) return 0;
     int64_t tiles, rows;
     query_tiles(group, q_len, &tiles, &rows);
@@ -997,7 +999,11 @@ extern "C" int trimkv_prefill_split_tiles(int batch, int kv_heads, int group, in
         }
         return (int)take;
     }
-    if (items > 128) return 0;
+    if (items >= 256) return 0;
+    if (items > 128) {
+        const bool pays = uneven > 0 && key_tiles >= 64 && (items <= 170 ? uneven <= 75 : uneven <= 55 && items <= 224 && key_tiles <= 160);
+        return pays ? (int)((key_tiles + 2) / 3) : 0;
+    }
     float best = 1.15f * (float)key_tiles - 8.0f;   // below that the second launch costs a caller whose queue runs dry as much
     int64_t take = 0;
     for (int64_t s = 2; s <= 32 && items * s <= 256; ++s) {
