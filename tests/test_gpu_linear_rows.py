@@ -110,6 +110,39 @@ def test_linear_rows_on_a_stream_and_replayed_from_a_graph():
         assert torch.equal(out, want) and torch.equal(act, gate), i
 
 
+# fewer outputs than a block has rows, in fours: the lanes of the columns that are not there store nothing
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 3, 16, 33, 64])
+@pytest.mark.parametrize("form,n", [("plain", 4), ("plain", 8), ("plain", 12), ("silu", 4), ("silu", 8), ("silu", 12), ("norm", 4), ("norm", 8), ("norm", 12), ("norm silu", 4), ("norm silu", 12)])
+def test_outputs_narrower_than_a_block_stay_inside_of_their_rows(form, n, rows, dtype):
+    k, lib, silu = 128, _lib.load(), "silu" in form
+    if "norm" in form and (rows > linear.NORM_ROWS or dtype != torch.bfloat16):
+        pytest.skip("what the norm form takes")
+    x, w, bias = _operands(rows, n * (1 + silu), k, dtype, rows + n)
+    out = torch.full((rows * n + 64,), 7.0, dtype=dtype, device=DEV)
+    tail, at = (_lib.dtype_code(dtype), _lib.current_stream(x.device)), (w.data_ptr(), k, bias.data_ptr(), out.data_ptr(), n, rows, n, k)
+    if "norm" in form:
+        norm = torch.ones(k, dtype=dtype, device=DEV)
+        squares = x.float().pow(2).view(rows, k // 8, 8).sum(-1)
+        _lib.check(lib.trimkv_linear_rows_norm(x.data_ptr(), k, squares.data_ptr(), norm.data_ptr(), 1e-6, *at, int(silu), 1, *tail), form)
+        x = (x.double() * torch.rsqrt(squares.double().sum(-1, keepdim=True) / k + 1e-6)).to(dtype)
+    elif silu:
+        _lib.check(lib.trimkv_linear_rows_silu(x.data_ptr(), k, *at, 1, *tail), form)
+    else:
+        _lib.check(lib.trimkv_linear_rows(x.data_ptr(), k, *at, *tail), form)
+    assert (out[rows * n:] == 7.0).all()
+    eps = EPS[dtype]
+    exact, size = x.double() @ w.double().T + bias.double(), x.double().abs() @ w.double().abs().T
+    slack = size * (k * 2.0 ** -23 + 2 * eps * ("norm" in form)) + 2.0 ** -24      # order of the sums; a normed row's last bit or two
+    if silu:        # as in the test of the silu form, every step rounded
+        (g, u), (dg, du) = exact.chunk(2, -1), (slack + eps * exact.abs()).chunk(2, -1)
+        act = torch.nn.functional.silu(g)
+        exact, slack = act * u, 1.1 * dg * (u.abs() + du) + act.abs() * du + (eps + 1e-5) * (act * u).abs()
+    err = (out[:rows * n].view(rows, n).double() - exact).abs()
+    assert (err <= slack + eps * exact.abs()).all(), float(err.max())
+
+
 def test_bad_arguments_are_refused_without_a_launch():
     lib, one = _lib.load(), ctypes.c_void_p(16)
     call = lambda rows=4, n=16, k=64, xs=64, ws=64, os=16, x=one, w=one, dt=_lib.BF16: lib.trimkv_linear_rows(x, xs, w, ws, None, one, os, rows, n, k, dt, None)

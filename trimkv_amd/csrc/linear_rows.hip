@@ -223,7 +223,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         for (int u = 0; u < NB * MT; ++u) {
             if (owner(u) != wave || (HALF && g >= 2)) continue;
             const int m = u % MT * 16 + r, n = block_at(tile, u / MT) + 4 * g;      // this lane: columns n .. n + 3 of row m
-            if (m >= a.m && !ADD) continue;
+            if ((m >= a.m && !ADD) || n >= a.n) continue;       // a matrix of fewer rows than a block: no such columns
             lr_f32x4 f = total(u);
             uint16_t v[4];
 #pragma unroll
