@@ -200,6 +200,30 @@ def test_modules_with_a_forward_of_their_own_are_not_asked_to_leave_a_product():
         assert torch.equal(above(total, None, None, None, None, out)[0], h + out)
 
 
+@pytest.mark.parametrize("outputs", [128, 1024])
+def test_a_product_of_another_width_than_the_residual_is_refused(outputs, monkeypatch):
+    """A last product replaced by a wider or narrower one: the sum raises, as modules do; no launch adds past a row's end."""
+    from trimkv_amd import qwen3
+    from tests.test_gpu_qwen3_shell import _family, _tiny_config
+    cfg = _tiny_config("qwen3")
+    layer = _family("qwen3")[1](cfg).eval().model.layers[0]
+    launched = []
+    monkeypatch.setattr(linear, "can_defer_norm", lambda weight, residual: True)          # as if all of this were on a GPU
+    monkeypatch.setattr(linear, "add_product", lambda p, residual: launched.append(p) or (residual, residual))
+    monkeypatch.setattr(qwen3.MLP, "takes_deferred", lambda self, x: True)
+    norm, hidden = layer.post_attention_layernorm, cfg.hidden_size
+    x, residual = torch.randn(1, 2, 48), torch.randn(1, 2, hidden)
+    with pytest.raises(RuntimeError, match="must match"):
+        layer._add_norm(norm, linear.DeferredProduct(x, nn.Linear(48, outputs)), residual, layer.mlp)
+    with pytest.raises(RuntimeError, match="must match"):        # ... or more rows
+        layer._add_norm(norm, linear.DeferredProduct(torch.randn(1, 3, 48), nn.Linear(48, hidden)), residual, layer.mlp)
+    # ... and a product of another type than the residual is added as tensors of two types are
+    assert layer._add_norm(norm, linear.DeferredProduct(x, nn.Linear(48, hidden)), residual.double(), layer.mlp)[1].dtype == torch.float64
+    assert not launched
+    layer._add_norm(norm, linear.DeferredProduct(x, nn.Linear(48, hidden)), residual, layer.mlp)
+    assert len(launched) == 1
+
+
 @pytest.mark.gpu
 def test_who_follows_operations_gets_the_general_product():
     from torch.autograd import forward_ad

@@ -120,6 +120,8 @@ class DeferredProduct:
     def __init__(self, x: torch.Tensor, module: nn.Linear):
         self.x, self.module = x, module
 
+    shape = property(lambda self: (*self.x.shape[:-1], self.module.weight.shape[0]))
+
     def tensor(self) -> torch.Tensor:
         return run(self.module, self.x)
 
@@ -159,7 +161,7 @@ def can_defer_norm(weight: torch.Tensor, residual: torch.Tensor) -> bool:
 
 
 def add_product(p: DeferredProduct, residual: torch.Tensor):
-    """``(residual + module(x), squares)`` in one launch; both have passed ``can_defer_product`` and ``can_defer_norm``."""
+    """``(residual + module(x), squares)`` in one launch; both have passed ``can_defer_product`` and ``can_defer_norm`` and are of one shape."""
     w, bias = p.module.weight, p.module.bias
     x2, n = _rows(p.x, w, bias), w.shape[0]
     rows, k = x2.shape

@@ -480,7 +480,7 @@ class TrimKVQwen3DecoderLayer(nn.Module):
         """``norm.add_norm(x, residual)`` for ``reader``.  At a decode step the add goes into the product that ``x`` is the result of and
         the norm into the one that ``reader`` begins with: neither has a launch of its own."""
         if type(x) is linear.DeferredProduct:
-            if (type(norm) is RMSNorm and linear.unhooked(norm) and linear.unhooked(reader) and linear.can_defer_norm(norm.weight, residual)
+            if (x.shape == residual.shape and x.x.dtype == residual.dtype and type(norm) is RMSNorm and linear.unhooked(norm) and linear.unhooked(reader) and linear.can_defer_norm(norm.weight, residual)
                     and getattr(reader, "takes_deferred", lambda x: False)(residual)):
                 total, squares = linear.add_product(x, residual)
                 return linear.DeferredNorm(total, squares, norm), total
