@@ -282,3 +282,27 @@ def test_checkpoint_to_tokens_with_and_without_a_graph(tmp_path):
     assert torch.equal(graphed, torch.cat(toks, dim=1))
     after = model.state_dict()
     assert set(after) == set(full) and all(torch.equal(after[k].cpu(), full[k]) for k in full)
+
+
+def test_replayed_steps_keep_their_rotary_frequencies():
+    """A captured step reads the frequencies by address: other models and settings that come and go leave them alone."""
+    from trimkv_amd.graphed import GraphedDecoder
+    from trimkv_amd.qwen3 import rotary_tables
+    cfg, model = _model("qwen3", "rg")
+    ids = torch.randint(0, cfg.vocab_size, (2, 30), generator=torch.Generator().manual_seed(3)).to(DEV)
+    with torch.no_grad():
+        cache_g, cache_e = (model(ids[:, :20], logits_to_keep=1).past_key_values for _ in range(2))
+        dec = GraphedDecoder(model, cache_g, logits_to_keep=1)
+        cache_e.begin_device_steps(cfg.memory_size, cfg.buffer_size)
+        others = []
+        for i in range(10):
+            tok = ids[:, 20 + i:21 + i]
+            got = dec(input_ids=tok).logits
+            want = model(tok, past_key_values=cache_e, cache_position=torch.tensor([20 + i], device=DEV), logits_to_keep=1).logits
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), i
+            if i == 4:
+                for j in range(80):
+                    rotary_tables(torch.arange(4, device=DEV)[None], cfg.head_dim, 1000.0 + j, torch.bfloat16)
+                others = [torch.full((cfg.head_dim // 2,), 1e3, device=DEV) for _ in range(500)]      # whatever was given back is in other hands now
+    assert len(others) == 500

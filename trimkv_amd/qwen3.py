@@ -210,13 +210,16 @@ class MLP(nn.Module):
 
 
 def rotary_tables(position_ids: torch.Tensor, head_dim: int, theta: float, dtype: torch.dtype,
-                  rotary_dim: Optional[int] = None, rope_scaling: Optional[dict] = None):
+                  rotary_dim: Optional[int] = None, rope_scaling: Optional[dict] = None, kept: Optional[dict] = None):
     """cos, sin [B, S, rotary_dim] of RoPE (frequencies theta^(-2i/rotary_dim), halves concatenated).  ``rope_scaling``:
     None/"default", or the published "llama3" rule (wavelengths above ``original/low_freq_factor`` are slowed by
-    ``factor``, those below ``original/high_freq_factor`` kept, a linear blend in between)."""
+    ``factor``, those below ``original/high_freq_factor`` kept, a linear blend in between).  ``kept``: where the caller keeps the
+    frequencies from one call to the next, one entry per device and setting."""
     rd = head_dim if rotary_dim is None else rotary_dim
     if position_ids.is_cuda and decoder_ops.enabled and decoder_ops.rope_tables_ok(position_ids, dtype, rd):
-        return decoder_ops.rope_tables(position_ids, _kept_frequencies(position_ids.device, rd, theta, rope_scaling), dtype)
+        device = position_ids.device
+        freq = _frequencies(device, rd, theta, rope_scaling) if kept is None else _kept_frequencies(kept, device, rd, theta, rope_scaling)
+        return decoder_ops.rope_tables(position_ids, freq, dtype)
     ang = position_ids[..., None].float() * _frequencies(position_ids.device, rd, theta, rope_scaling)
     emb = torch.cat([ang, ang], dim=-1)
     return emb.cos().to(dtype), emb.sin().to(dtype)
@@ -236,21 +239,16 @@ def _frequencies(device, rd: int, theta: float, rope_scaling: Optional[dict]) ->
     return inv_freq
 
 
-_FREQUENCIES: dict = {}      # (device, sizes and scaling) -> what _frequencies gives there: constants
-
-
-def _kept_frequencies(device, rd: int, theta: float, rope_scaling: Optional[dict]) -> torch.Tensor:
+def _kept_frequencies(kept: dict, device, rd: int, theta: float, rope_scaling: Optional[dict]) -> torch.Tensor:
+    """What ``_frequencies`` gives, from ``kept`` if it is there.  Nothing leaves ``kept``: captured graphs of its owner hold the addresses."""
     key = (device, rd, theta, None if not rope_scaling else tuple(sorted((k, str(v)) for k, v in rope_scaling.items())))
-    freq = _FREQUENCIES.get(key)
-    if freq is None:
+    freq = kept.get(key)
+    if freq is None or freq.device != device:
         with torch.inference_mode(False), torch.no_grad():
             freq = _frequencies(device, rd, theta, rope_scaling)
-        if torch.cuda.is_current_stream_capturing():      # memory of the graph's
-            return freq
-        torch.cuda.current_stream(device).synchronize()   # there for every stream from here on
-        if len(_FREQUENCIES) >= 64:
-            _FREQUENCIES.clear()
-        _FREQUENCIES[key] = freq
+        if not torch.cuda.is_current_stream_capturing() and len(kept) < 64:      # memory of a graph's pool is not kept
+            torch.cuda.current_stream(device).synchronize()   # there for every stream from here on
+            kept[key] = freq
     return freq
 
 
@@ -516,7 +514,8 @@ class TrimKVQwen3Model(nn.Module):
             position_ids = cache_position.unsqueeze(0)
         c = self.config
         position_embeddings = rotary_tables(position_ids, c.head_dim, c.rope_theta, inputs_embeds.dtype,
-                                            int(c.head_dim * getattr(c, "partial_rotary_factor", 1.0)), getattr(c, "rope_scaling", None))
+                                            int(c.head_dim * getattr(c, "partial_rotary_factor", 1.0)), getattr(c, "rope_scaling", None),
+                                            self.__dict__.setdefault("_rotary_frequencies", {}))
         hidden_states = inputs_embeds
         pending = None    # the last MLP output; its residual add rides in the next norm
         for layer in self.layers:
