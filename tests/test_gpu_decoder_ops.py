@@ -348,3 +348,21 @@ def test_rope_tables_are_what_torch_computes(pos, rd, theta, scaling, dtype):
     for g, again, w in zip(*got, want):
         assert g.shape == w.shape == (*pos.shape, rd) and torch.equal(g, again)
         assert ((g.double() - w.double()).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * w.double().abs() + 2.0 ** -24).all() and (g != w).float().mean() < 1e-3
+
+
+def test_rope_tables_under_vmap_and_in_a_trace_are_the_torch_expressions():
+    """Somebody follows the operations: a launch of ours would have no address to read, or leave the first positions in the trace."""
+    from trimkv_amd import decoder_ops
+    from trimkv_amd.qwen3 import rotary_tables
+    pos = torch.arange(12, device=DEV).view(3, 1, 4)
+    tables = lambda p: rotary_tables(p, 128, 1e4, torch.bfloat16)
+    assert decoder_ops.rope_tables_ok(pos[0], torch.bfloat16, 128)
+    decoder_ops.enabled = False
+    try:
+        want, later = [tables(p) for p in pos], tables(pos[0] + 100)
+    finally:
+        decoder_ops.enabled = True
+    for got, each in zip(torch.func.vmap(tables)(pos), zip(*want)):
+        assert torch.equal(got, torch.stack(each))
+    traced = torch.jit.trace(tables, (pos[0],), check_trace=False)
+    assert all(torch.equal(g, w) for g, w in zip(traced(pos[0] + 100), later))

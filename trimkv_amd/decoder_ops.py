@@ -72,7 +72,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optiona
 
 def rope_tables_ok(positions: torch.Tensor, dtype: torch.dtype, rotary_dim: int) -> bool:
     return (dtype in (torch.bfloat16, torch.float16) and positions.dtype == torch.int64 and positions.dim() == 2 and positions.numel() > 0 and rotary_dim > 0 and rotary_dim % 2 == 0
-            and type(positions) is torch.Tensor and positions.device.index == torch.cuda.current_device())
+            and type(positions) is torch.Tensor and positions.is_cuda and positions.device.index == torch.cuda.current_device() and not linear.watched())
 
 
 def rope_tables(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype):

@@ -17,7 +17,7 @@ from . import _lib
 MAX_ROWS = 64      # rows that trimkv_linear_rows takes
 
 
-def _watched() -> bool:
+def watched() -> bool:
     """Somebody follows the operations themselves (vmap and torch.func, forward-mode derivatives, tracing, compiling, dispatch modes): a
     launch of ours would be lost on them, and inside of vmap a tensor has no address."""
     return (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
@@ -27,7 +27,7 @@ def _watched() -> bool:
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
     """Ordinary tensors of one 16-bit dtype on the current GPU that nobody differentiates, casts or follows."""
     first = tensors[0]
-    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or _watched():
+    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or watched():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:

@@ -216,7 +216,7 @@ def rotary_tables(position_ids: torch.Tensor, head_dim: int, theta: float, dtype
     ``factor``, those below ``original/high_freq_factor`` kept, a linear blend in between).  ``kept``: where the caller keeps the
     frequencies from one call to the next, one entry per device and setting."""
     rd = head_dim if rotary_dim is None else rotary_dim
-    if position_ids.is_cuda and decoder_ops.enabled and decoder_ops.rope_tables_ok(position_ids, dtype, rd):
+    if decoder_ops.enabled and decoder_ops.rope_tables_ok(position_ids, dtype, rd):
         device = position_ids.device
         freq = _frequencies(device, rd, theta, rope_scaling) if kept is None else _kept_frequencies(kept, device, rd, theta, rope_scaling)
         return decoder_ops.rope_tables(position_ids, freq, dtype)
