@@ -243,6 +243,20 @@ def test_who_follows_operations_gets_the_general_product():
         assert torch.equal(traced(x + 1), nn.functional.linear(x + 1, w, bias))
 
 
+def test_function_modes_follow_operations_and_a_default_device_does_not():
+    from torch.overrides import TorchFunctionMode
+
+    class Counting(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    assert not linear.watched()
+    with torch.device("cpu"):
+        assert not linear.watched()
+        with Counting():
+            assert linear.watched()
+    assert not linear.watched()
+
+
 def _normed(x, norm):
     """What the modules make of x, in 64 bits between their two roundings."""
     h = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + norm.variance_epsilon)

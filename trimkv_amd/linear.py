@@ -11,6 +11,8 @@ from torch import nn
 import torch.nn.functional as F
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -18,10 +20,11 @@ MAX_ROWS = 64      # rows that trimkv_linear_rows takes
 
 
 def watched() -> bool:
-    """Somebody follows the operations themselves (vmap and torch.func, forward-mode derivatives, tracing, compiling, dispatch modes): a
-    launch of ours would be lost on them, and inside of vmap a tensor has no address."""
+    """Somebody follows the operations themselves (vmap and torch.func, forward-mode derivatives, tracing, compiling, dispatch modes, function
+    modes other than that of a default device): a launch of ours would be lost on them, and inside of vmap a tensor has no address."""
     return (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
-            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0)
+            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or (torch._C._len_torch_function_stack() > 0 and any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())))
 
 
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
