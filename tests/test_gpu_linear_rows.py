@@ -169,6 +169,28 @@ def test_modules_that_somebody_hooked_wrapped_or_replaced_are_called():
     assert torch.equal(linear.run(twice, x), 2 * nn.functional.linear(x, twice.weight, twice.bias))
 
 
+def test_a_packed_product_that_somebody_hooked_wrapped_or_replaced_is_called(monkeypatch):
+    from trimkv_amd import hybrid
+    mlp, xh, asked = hybrid.DenseMLP({"ff": 8}, 64, torch.float32), torch.randn(3, 64), []
+    nn.init.normal_(mlp.gate_up.weight), nn.init.normal_(mlp.down.weight)
+    monkeypatch.setattr(hybrid, "silu_product", lambda x, w, **kw: asked.append(w) or torch.zeros(len(x), 8))          # as if it took every product
+    monkeypatch.setattr(hybrid.ops, "silu_gate", lambda both, ff: nn.functional.silu(both[:, :ff]) * both[:, ff:])
+    want = lambda scale: mlp.down(hybrid.ops.silu_gate(scale * nn.functional.linear(xh, mlp.gate_up.weight), 8))
+    assert torch.equal(mlp(None, xh)[0], torch.zeros(3, 64)) and len(asked) == 1
+    hook = mlp.gate_up.register_forward_hook(lambda m, a, out: 2 * out)
+    assert torch.equal(mlp(None, xh)[0], want(2))
+    hook.remove()
+    mlp.gate_up.forward = lambda x: 3 * nn.functional.linear(x, mlp.gate_up.weight)
+    assert torch.equal(mlp(None, xh)[0], want(3))
+    del mlp.gate_up.forward
+
+    class Quadrupled(hybrid.PackedLinear):
+        def forward(self, x):
+            return 4 * super().forward(x)
+    mlp.gate_up.__class__ = Quadrupled
+    assert torch.equal(mlp(None, xh)[0], want(4)) and len(asked) == 1
+
+
 def test_modules_with_a_forward_of_their_own_are_not_asked_to_leave_a_product():
     """Subclasses written before there was such an argument: the decoder calls them as it always did."""
     from trimkv_amd import qwen3

@@ -20,7 +20,7 @@ import torch
 from torch import nn
 
 from . import _lib, hybrid_ops as ops
-from .linear import linear, silu_product
+from .linear import linear, silu_product, unhooked
 from .generation import GreedyGeneration
 from .hybrid_cache import HybridCache
 
@@ -266,7 +266,9 @@ class DenseMLP(nn.Module):
 
     def forward(self, x, xh):
         xh = xh[:, :self.width]
-        act = silu_product(xh, self.gate_up.weight, round_all=False, library="hybrid")
+        # a packed product that somebody hooked, wrapped or replaced is called
+        plain = type(self.gate_up) is PackedLinear and unhooked(self.gate_up)
+        act = silu_product(xh, self.gate_up.weight, round_all=False, library="hybrid") if plain else None
         return self.down(ops.silu_gate(self.gate_up(xh), self.ff) if act is None else act), None
 
 
