@@ -167,6 +167,9 @@ def test_modules_that_somebody_hooked_wrapped_or_replaced_are_called():
             return 2 * super().forward(y)
     twice = Doubled(8, 4)
     assert torch.equal(linear.run(twice, x), 2 * nn.functional.linear(x, twice.weight, twice.bias))
+    from trimkv_amd import decoder_ops
+    for other in (twice, nn.Sequential(nn.Linear(8, 4), nn.ReLU()), nn.Identity()):        # with a weight of its own or without
+        assert torch.equal(decoder_ops.leave_or_run(other, x, True), other(x))
 
 
 def test_a_packed_product_that_somebody_hooked_wrapped_or_replaced_is_called(monkeypatch):

@@ -152,8 +152,10 @@ def tensor_of(x) -> torch.Tensor:
 
 def can_defer_product(module: nn.Module, x: torch.Tensor) -> bool:
     """Whether ``module(x)`` may wait for the residual that is added to it."""
+    if not untouched(module):
+        return False
     w = module.weight
-    return (untouched(module) and x.dtype == torch.bfloat16 and 0 < x.numel() <= NORM_ROWS * x.shape[-1] and w.shape[0] % 64 == 0 and w.shape[0] <= NORM_K
+    return (x.dtype == torch.bfloat16 and 0 < x.numel() <= NORM_ROWS * x.shape[-1] and w.shape[0] % 64 == 0 and w.shape[0] <= NORM_K
             and _rows(x, w, module.bias) is not None)
 
 
