@@ -726,7 +726,7 @@ int trimkv_linear_rows_silu(const void* x, int64_t x_stride, const void* w, int6
  * aligned, their strides multiples of 4.
  * trimkv_linear_rows_norm -- trimkv_linear_rows or, with silu, trimkv_linear_rows_silu (n then counts the gate's rows) over
  * round(round(x / sqrt(mean(x^2) + eps)) * norm_weight), where the sums in squares [rows][k / 8] say what mean(x^2) is.  bf16, up to
- * 32 rows of up to 8192; norm_weight [k] 16-byte aligned.
+ * 32 rows of up to 8192; squares and norm_weight [k] 16-byte aligned.
  */
 int trimkv_linear_rows_add(const void* x, int64_t x_stride, const void* w, int64_t w_stride, const void* bias, const void* residual, int64_t residual_stride,
                            void* out, int64_t out_stride, float* squares, int rows, int n, int k, int dtype, void* stream);

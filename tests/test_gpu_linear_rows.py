@@ -361,7 +361,7 @@ def test_what_is_not_left_to_a_product():
 def test_bad_arguments_around_a_norm_are_refused_without_a_launch():
     lib, one = _lib.load(), ctypes.c_void_p(16)
     norm = lambda rows=4, k=64, sq=one, nw=one, dt=_lib.BF16: lib.trimkv_linear_rows_norm(one, k, sq, nw, 1e-6, one, k, None, one, 16, rows, 16, k, 0, 1, dt, None)
-    assert norm(rows=33) == -2 and norm(k=8256) == -2 and norm(nw=ctypes.c_void_p(24)) == -2 and norm(sq=None) == -1 and norm(nw=None) == -1 and norm(dt=_lib.F16) == -3
+    assert norm(rows=33) == -2 and norm(k=8256) == -2 and norm(nw=ctypes.c_void_p(24)) == -2 and norm(sq=ctypes.c_void_p(20)) == -2 and norm(sq=None) == -1 and norm(nw=None) == -1 and norm(dt=_lib.F16) == -3
     add = lambda rows=4, n=16, rs=16, os=16, res=one, sq=one, dt=_lib.BF16: lib.trimkv_linear_rows_add(one, 64, one, 64, None, res, rs, one, os, sq, rows, n, 64, dt, None)
     assert add(rows=33) == -2 and add(n=24, rs=24, os=24) == -2 and add(rs=12) == -2 and add(rs=18) == -2 and add(os=18) == -2 and add(res=ctypes.c_void_p(20)) == -2
     assert add(res=None) == -1 and add(sq=None) == -1 and add(dt=_lib.F32) == -3

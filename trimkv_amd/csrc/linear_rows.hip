@@ -387,7 +387,7 @@ extern "C" int trimkv_linear_rows_norm(const void* x, int64_t x_stride, const fl
     if (!squares || !norm_weight) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (dtype != TRIMKV_BF16) return fail(TRIMKV_ERR_DTYPE, "%s: bf16 only (dtype=%d)", fn, dtype);
     if (rows > LR_NORM_ROWS || k > LR_NORM_K) return fail(TRIMKV_ERR_SHAPE, "%s: at most %d rows of %d (got %d of %d)", fn, LR_NORM_ROWS, LR_NORM_K, rows, k);
-    if ((uintptr_t)norm_weight & 15) return fail(TRIMKV_ERR_SHAPE, "%s: norm_weight must be 16-byte aligned", fn);
+    if (((uintptr_t)norm_weight | (uintptr_t)squares) & 15) return fail(TRIMKV_ERR_SHAPE, "%s: squares and norm_weight must be 16-byte aligned", fn);
     LinearRowsArgs a{(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (const uint16_t*)bias, (uint16_t*)out, out_stride, rows, n, k, 0, round_all};
     a.norm_w = (const uint16_t*)norm_weight; a.eps = eps; a.squares = const_cast<float*>(squares);
     return rows_check_and_launch(fn, a, silu != 0, dtype, stream);
