@@ -164,3 +164,45 @@ def test_decode_step_including_eviction_replays_from_a_hip_graph(G):
             pos = graphed["layers"][1]["POS"][:, :M]
             assert (pos[:, 1:] > pos[:, :-1]).all()                    # kept rows stay in temporal order
     assert evictions == 3
+
+
+@pytest.mark.parametrize("uneven", [False, True])
+@pytest.mark.parametrize("fused", [False, True])
+def test_a_ragged_step_is_captured_right_behind_its_prompt(uneven, fused):
+    """No token step has run: the launch's list of pieces is not on the device and nothing may be uploaded.  What is replayed is the eager
+    step with its keys divided otherwise: u max|v| for probabilities rounded against other references, the row sums and the output, twice (bf16)."""
+    from types import SimpleNamespace
+    from trimkv_amd import BatchedDynamicBudgetTrimKVCache, get_attention_interface
+    B, H, G, D, P = 4, 8, 2, 128, 600
+    attend, module = get_attention_interface("db_attn_flash_batched"), SimpleNamespace(training=False, num_key_value_groups=G, is_causal=True)
+
+    def prompt():
+        gen = torch.Generator(device=DEV).manual_seed(1)
+        made = lambda *shape: torch.randn(*shape, generator=gen, device=DEV).to(torch.bfloat16)
+        cache = BatchedDynamicBudgetTrimKVCache()
+        cache.fuse_decode_append = fused
+        if uneven:
+            cache.set_budgets(torch.linspace(64, 590, B * H).long())
+        k, v = made(B, H, P, D), made(B, H, P, D)
+        cache.update(k, v, torch.randn(B, H, P, generator=gen, device=DEV), torch.arange(P, device=DEV), 0)
+        if uneven:
+            cache.evict_to_budgets(buffer_size=0)
+        return cache, made(B, H, 1, D), made(B, H, 1, D), made(B, H * G, 1, D), v
+
+    pos, lb = torch.full((1,), P, device=DEV), torch.zeros(B, H, 1, device=DEV)
+
+    def step(cache, k, v, q, _):
+        keys, values, _, _, kw = cache.update(k, v, lb, pos, 0)
+        return attend(module, q, keys, values, None, flash_attn_kwargs=kw)[0]
+
+    with torch.no_grad():
+        eager, graphed = prompt(), prompt()
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+            out = step(*graphed)
+        want = step(*eager)
+        graph.replay()
+        torch.cuda.synchronize()
+    assert float((out.float() - want.float()).abs().max()) <= 6 * 2.0 ** -9 * float(eager[4].abs().max())
+    assert torch.equal(graphed[0]._slabs[0].seg_len, eager[0]._slabs[0].seg_len)

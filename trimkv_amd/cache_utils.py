@@ -1105,6 +1105,8 @@ class _RaggedCache(_SlabBacked):
         if (slab.pieces is not None and slab.pieces_age < self.attention_replan_steps
                 and abs(slab.total - slab.pieces_total) * 25 <= slab.pieces_total):
             return slab.pieces
+        if torch.cuda.is_current_stream_capturing():
+            return slab.pieces        # nothing is uploaded into a graph: the list there is, or none (the launch cuts its grid by rows then)
         nseg = slab.lens.size
         if nseg > 8192:
             slab.pieces = None
@@ -1380,7 +1382,7 @@ class _RaggedCache(_SlabBacked):
     @staticmethod
     def _dispatch_order(slab: _Slab) -> Optional[torch.Tensor]:
         """The order set last, on the device from its first use on."""
-        if slab.order is None and slab.order_host is not None:
+        if slab.order is None and slab.order_host is not None and not torch.cuda.is_current_stream_capturing():
             # through pinned memory, in stream order: a copy from pageable memory would wait for the whole stream
             if not torch.is_tensor(slab.order_host):
                 slab.order_host = torch.from_numpy(np.argsort(-slab.order_host, kind="stable").astype(np.int32)).pin_memory()
