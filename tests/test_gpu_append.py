@@ -32,3 +32,17 @@ def test_rows_lengths_and_prefix_sums(S, D, cap):
     assert seg_len.tolist() == [S, cap, 7 + S, cap - S + 1]
     assert cu.tolist() == [0, S, 2 * S, 3 * S, 0]
     assert all(torch.equal(got.cpu(), w) for got, w in zip(slabs, want))
+
+
+@pytest.mark.parametrize("S,length", [(100, (1 << 20) + 5), (100, 2 ** 31 - 100), (300, (3 << 20) + 5), (300, 2 ** 31 - 1), (300, -5)])
+def test_lengths_that_cannot_be_are_left_alone(S, length):
+    """One workgroup to a segment takes a length as it is; three leave a count of up to two in its upper bits."""
+    from trimkv_amd import _lib
+    lib, cap, D = _lib.load(), 400, 64
+    k = torch.ones(1, 2, S, D, dtype=torch.bfloat16, device=DEV)
+    slabs = [torch.zeros(2, cap, D, dtype=torch.bfloat16, device=DEV) for _ in range(2)] + [torch.zeros(2, cap, device=DEV), torch.zeros(2, cap, dtype=torch.int64, device=DEV)]
+    seg_len, lb, pos = torch.tensor([length, 3], dtype=torch.int32, device=DEV), torch.ones(1, 2, S, device=DEV), torch.ones(S, dtype=torch.int64, device=DEV)
+    _lib.check(lib.trimkv_append(*(t.data_ptr() for t in slabs), seg_len.data_ptr(), None, 2, 2, cap, D, _lib.BF16, _lib.F32, k.data_ptr(), k.data_ptr(), *k.stride()[:3],
+                                 lb.data_ptr(), *lb.stride(), pos.data_ptr(), 0, 0, 1, S, cap, _lib.current_stream(k.device)), "trimkv_append")
+    assert seg_len.tolist() == [length, 3 + S]
+    assert all(not t[0].any() and t[1].float().sum() == t[1, 3:3 + S].numel() for t in slabs)

@@ -52,14 +52,15 @@ __global__ __launch_bounds__(AP_THREADS) void append_kernel(AppendArgs a) {
     };
     const int raw = a.seg_len[seg];
     fetch(threadIdx.x);
-    int n0 = a.counted && raw >= 0 ? raw & AP_LEN_MASK : raw;
+    const bool shared = a.counted && gridDim.y > 1;          // the upper bits hold the workgroups that have counted themselves, which is not all of them
+    int n0 = shared && raw >= 0 && (raw >> AP_LEN_BITS) < (int)gridDim.y ? raw & AP_LEN_MASK : raw;
     asm volatile("" : "+v"(n0));            // it has landed when the barrier is reached
     // Never write past the slab: the host checks its bound, this guards a stale bound.
-    const bool fits = (n0 >= 0) && (n0 + a.s_new <= a.cap);
+    const bool fits = n0 >= 0 && n0 <= a.cap - a.s_new;
     __syncthreads();                        // every thread has read the length before it may be rewritten
     const bool counts = a.counted && fits && threadIdx.x == 0;
     int before = 0;
-    if (counts) before = atomicAdd(&a.seg_len[seg], 1 << AP_LEN_BITS) >> AP_LEN_BITS;
+    if (counts && shared) before = atomicAdd(&a.seg_len[seg], 1 << AP_LEN_BITS) >> AP_LEN_BITS;
     if (fits) {
         const int64_t dst_row0 = (int64_t)seg * a.cap + n0, d = (dst_row0 + s_begin) * a.row_bytes;      // rows lie one behind the other
         for (int at = threadIdx.x;;) {
