@@ -54,9 +54,9 @@ def test_equal_shares_match_the_whole_and_the_oracle(G, D, dtype, Q, lens):
         assert ok, err
 
 
-@pytest.mark.parametrize("B,H,G,Q,n,pays", [(3, 8, 2, 777, 9000, True), (1, 8, 4, 2100, 4200, True), (1, 8, 4, 2040, 2100, False)])
+@pytest.mark.parametrize("B,H,G,Q,n,pays", [(3, 8, 2, 777, 9000, True), (1, 8, 4, 2100, 4200, True), (1, 8, 4, 2040, 2100, False), (4, 8, 5, 2048, 7000, False)])
 def test_the_public_call_follows_the_rule(B, H, G, Q, n, pays, monkeypatch):
-    """168 and 264 query tiles of long caches in equal shares, 256 of short ones whole: both as the whole kernel has it."""
+    """168 and 264 query tiles of long caches in equal shares, 256 of short ones and 1312 of many segments whole: all as the whole kernel has it."""
     from trimkv_amd import _lib
     from trimkv_amd.attn import hip_attn
     lib = _lib.load()

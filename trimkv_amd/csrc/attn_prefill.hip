@@ -1049,16 +1049,20 @@ extern "C" int trimkv_prefill_attn_split(const void* q, int64_t q_stride_b, int6
 // More than 128 query tiles.  Whole, the chip is done when its longest query tile is, or a last round that fills part of it: 1.2 us per
 // 64 keys where a CU has little company, 1.6 where all are busy.  Equal shares take the mean of all CUs and pay for it with up to
 // 67 MB of unfinished outputs written and read, about 26 us.  Estimates fitted to 80 launches (136 .. 1104 query tiles of 2500,
-// 5000 and 9000 keys, mean length 52 .. 100 % of the longest); where they differ by 3 % and more the choice was the faster one
-// but for two of them (up to 7 %).  Whole -> shares, us: 168 tiles, 0.78 of 4100 keys 88 -> 83, 0.65 of 9000 170 -> 122; 264 tiles of
-// 9000 377 -> 269, of 5000 167 -> 149; 288, 0.52 of 9000 289 -> 185; 352 of 5000 220 -> 204; left whole: 216 of 2500 59 -> 67, 512
-// of 5000 174 -> 204, 704 of 9000 478 -> 495.
+// 5000 and 9000 keys, mean length 52 .. 100 % of the longest) and compared with 340 more (168 .. 8192 query tiles of 8 .. 128 segments, 3100 .. 40000 keys,
+// mean length 55 .. 100 %, chunks of 300 .. 8192): where they differ by 3 % the choice is the faster one, but from 512 query tiles of 32 segments on, where
+// lengths average out and the workgroups of an XCD no longer walk the same keys at about the same time, shares lost by up to 15 % (1312
+// tiles, 32 segments of 40000 keys 5761 -> 6228 us, 1056 tiles, 96 of 7000 814 -> 854).  11 % and more with the rows held there leave nothing that is
+// slower by 3 %, and give up 2 .. 12 % at 13 of the 340 (most: 512 tiles, 64 segments of 0.55 x 11000 keys, 427 -> 382).  Beyond 8192 tiles or 40960 keys nothing
+// was measured.  Whole -> shares, us: 168 tiles, 0.78 of 4100 keys 88 -> 83, 0.65 of 9000 170 -> 122; 264 tiles of 9000 377 -> 269, of 5000 167 -> 149;
+// 288, 0.52 of 9000 289 -> 185; 352 of 5000 220 -> 204; 1296 of 12000 1407 -> 1369, of 32000 4263 -> 4051; 2576, 0.7 of 16000 2722 -> 2221; left
+// whole: 216 of 2500 59 -> 67, 512 of 5000 174 -> 204, 704 of 9000 478 -> 495, 2048 of 8704 1381 -> 1485, 8192 of 16000 11355 -> 13595.
 extern "C" int trimkv_prefill_equal_shares(int batch, int kv_heads, int group, int q_len, int max_len, int uneven) {
     if (batch <= 0 || kv_heads <= 0 || group < 1 || group > 8 || q_len < 64 || max_len <= 0) return 0;
     int64_t tiles, rows;
     query_tiles(group, q_len, &tiles, &rows);
     const int64_t items = tiles * batch * kv_heads;
-    if (items <= 128 || items > 32768 || (uneven && max_len < 3072)) return 0;
+    if (items <= 128 || items > 8192 || max_len > 40960 || (uneven && max_len < 3072)) return 0;
     // in tiles of 64 keys: the longest segment, the mean query tile, the first one of a mean segment
     const float even = uneven <= 0 ? 1.0f : uneven == 1 ? 0.6f : 0.01f * (float)uneven, all = (float)items / 256.0f;
     const float longest = (float)max_len / 64.0f, keys = (float)max_len * even, bt = 256.0f / (float)group;
@@ -1070,7 +1074,9 @@ extern "C" int trimkv_prefill_equal_shares(int batch, int kv_heads, int group, i
         const float rounds = (float)(items / 256), rest = (float)(items % 256), last = least + (mean - least) * rest / (float)items;
         whole = rounds * (1.6f * mean + 8.0f) + (rest > 0.0f ? (0.96f + 0.34f * rest / 256.0f) * last + 8.0f : 0.0f) + 0.9f * (1.0f - even) * longest;
     }
-    return whole > 1.03f * shares;
+    const int64_t segs = (int64_t)batch * kv_heads;
+    const float margin = segs >= 32 && items >= 512 ? 1.11f + 0.02f * (float)(segs * max_len) / 524288.0f : 1.03f;
+    return keys >= (float)q_len && whole > margin * shares;      // a segment holds at least the chunk
 }
 
 extern "C" int64_t trimkv_prefill_shares_workspace(int batch, int kv_heads, int group, int q_len) {
