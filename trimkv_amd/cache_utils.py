@@ -108,12 +108,16 @@ def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -
             and rows * (5 if spill < 512 else 8) < 360 * longest - 300000 and not torch.cuda.is_current_stream_capturing())
 
 
-def compact_halves(segs: int, longest: int) -> bool:
+def compact_halves(segs: int, longest: int, rows: int) -> bool:
     """Whether a compaction moves keys and values by workgroups of their own: its launch lasts as long as its longest segment, and two
-    workgroups take that one in less time.  A chunk with its eviction, whole -> halves, us: 16 segments of up to 8000 rows 309 -> 273, 64
-    of 4000 636 -> 602, 192 1041 -> 1000, 512 1995 -> 1936; 128 of up to 1500 466 -> 463.  The scratch for what is put in place
-    afterwards is 12 bytes a row, 48 MB at most."""
-    return segs <= 512 and 1024 <= longest <= 32768 and segs * longest <= 1 << 22
+    workgroups take that one in less time.  ``rows``: of all segments.  Up to 128 segments all of these workgroups have a compute unit of their own;
+    beyond that it pays where few segments are long.  The compaction alone, whole -> halves, us, segments x longest (mean / longest): 64 x 1100 (0.55)
+    24.4 -> 22.1, 128 x 2048 (0.5) 41 -> 35, x 8000 (0.3) 148 -> 103; 160 x 6000 (0.5) 1.07 times as fast, 256 x 6000 (0.4) 1.13, 192 x 3000 (0.28) 1.2; left
+    whole: 192 x 2048 (0.8) 54 -> 60, 160 x 8000 (0.8) 173 -> 199, 256 x 1500 (0.4) 0.93 times as fast, 512 x 3000 (0.15) 0.9, x 1500 0.8.
+    The scratch for what is put in place afterwards is 12 bytes a row, 48 MB at most."""
+    if segs > 512 or longest > 32768 or segs * longest > 1 << 22:
+        return False
+    return longest >= (1024 if segs <= 128 else 3000 if segs <= 256 else 6000) and (segs <= 128 or 2 * rows <= segs * longest)
 
 
 def wide_group(segs: int, longest: int) -> bool:
@@ -1261,7 +1265,7 @@ class _RaggedCache(_SlabBacked):
         table = self._device_tables(layers)["slabs"]
         lib = _lib.load()
         code = self._strategy_code(strategy)
-        halves = code == _lib.SCORE_ALPHA and compact_halves(len(layers) * s0.nseg, max_len)
+        halves = code == _lib.SCORE_ALPHA and compact_halves(len(layers) * s0.nseg, max_len, sum(self._slabs[l].total for l in layers))
         ws = None
         if halves:
             try:
