@@ -46,6 +46,18 @@ def test_linear_rows_matches_the_product(rows, n, k, dtype):
     assert torch.equal(got, linear.linear(x, w, library="hybrid"))
 
 
+# what linear.linear leaves to the general product is still the entry point's to take
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n,k", [(33, 12289, 64), (64, 16384, 128), (64, 24576, 64), (50, 24600, 128), (64, 50002, 64)])
+def test_many_rows_of_wide_matrices(rows, n, k, dtype):
+    x, w, bias = _operands(rows, n, k, dtype, rows + n + k)
+    assert torch.equal(linear.linear(x, w, bias), nn.functional.linear(x, w, bias)) and n > linear.WIDE and rows > linear.WIDE_ROWS
+    out = torch.empty(rows, n, dtype=dtype, device=DEV)
+    _lib.check(_lib.load().trimkv_linear_rows(x.data_ptr(), k, w.data_ptr(), k, bias.data_ptr(), out.data_ptr(), n, rows, n, k, _lib.dtype_code(dtype), _lib.current_stream(x.device)), "wide")
+    _check(out, x, w, bias, dtype)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("round_all", [True, False])

@@ -17,6 +17,12 @@ from torch.utils._device import DeviceContext
 from . import _lib
 
 MAX_ROWS = 64      # rows that trimkv_linear_rows takes
+# More rows than WIDE_ROWS times more outputs than WIDE, heads of language models above all, are left to the general product: workgroups there take 96 rows of w
+# and have one step in flight.  us here | general, 48 rows and 64: 16384 x 3072 26.8 | 23.1, 27.9 | 23.4; 32064 x 3072 51.0 | 47.2, 53.8 | 38.6; 128256 x 4096
+# 230 | 214, 243 | 216; 151936 x 4096 265 | 261, 278 | 270; given up: 24576 x 4096 41.6 | 44.7, 41.9 | 45.5, 49152 x 2048 47.9 | 51.9, 50.4 | 54.5.  Up to
+# 32 rows all are taken: 32064 x 3072 with 1, 16, 32 rows 31.5 | 41.0, 33.2 | 42.0, 39.4 | 37.1; 151936 x 2048 101 | 207, 109 | 208, 128 | 153; 151936 x
+# 5120 238 | 307, 263 | 330, 319 | 364.  12288 x 4096 with 48 and 64: 22.8 | 24.5, 24.3 | 25.1.
+WIDE_ROWS, WIDE = 32, 12288
 
 
 def watched() -> bool:
@@ -59,7 +65,7 @@ def _rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, library: Optional[str] = None) -> torch.Tensor:
     """``F.linear(x, weight, bias)``.  ``library``: which one holds the kernel (a name of ``_lib.SHARED``; None: libtrimkv_hip.so)."""
     x2 = _rows(x, weight, bias)
-    if x2 is None:
+    if x2 is None or (x2.shape[0] > WIDE_ROWS and weight.shape[0] > WIDE):
         return F.linear(x, weight, bias)
     rows, k = x2.shape
     n = weight.shape[0]
