@@ -142,3 +142,15 @@ def test_arguments_are_checked():
     assert _plan(lens, ncu=0)[0] < 0
     assert _plan(np.array([5, -1], dtype=np.int32))[0] < 0
     assert _plan(lens, min_rows=0)[0] < 0
+
+
+def test_rules_choose_divided_launches_where_they_were_measured_faster():
+    """Equal shares of a chunk's keys, and keys and values of a compaction by a workgroup each: both sides of each line."""
+    from trimkv_amd.cache_utils import compact_halves
+    shares = _lib.load().trimkv_prefill_equal_shares
+    assert shares(3, 8, 2, 777, 9000, 65) and shares(2, 8, 5, 4096, 12288, 0) and shares(2, 8, 5, 4096, 32000, 70)
+    assert not shares(4, 8, 5, 2048, 40000, 0) and not shares(12, 8, 4, 700, 7000, 0) and not shares(4, 8, 4, 2048, 32000, 70)      # many segments
+    assert not shares(2, 8, 5, 4096, 40961, 0) and not shares(1, 8, 5, 8192, 8704, 70)                                             # not measured; shorter than the chunk
+    assert compact_halves(128, 1024, 128 * 1000) and compact_halves(160, 6000, 160 * 3000) and compact_halves(512, 8000, 512 * 1200)
+    assert not compact_halves(128, 1023, 9000) and not compact_halves(160, 8000, 160 * 6400) and not compact_halves(192, 2048, 192 * 700) and not compact_halves(512, 3000, 512 * 500)
+    assert not compact_halves(513, 8000, 8000) and not compact_halves(8, 32769, 8000) and not compact_halves(512, 8193, 8193)
