@@ -112,12 +112,14 @@ def compact_halves(segs: int, longest: int, rows: int) -> bool:
     """Whether a compaction moves keys and values by workgroups of their own: its launch lasts as long as its longest segment, and two
     workgroups take that one in less time.  ``rows``: of all segments.  Up to 128 segments all of these workgroups have a compute unit of their own;
     beyond that it pays where few segments are long.  The compaction alone, whole -> halves, us, segments x longest (mean / longest): 64 x 1100 (0.55)
-    24.4 -> 22.1, 128 x 2048 (0.5) 41 -> 35, x 8000 (0.3) 148 -> 103; 160 x 6000 (0.5) 1.07 times as fast, 256 x 6000 (0.4) 1.13, 192 x 3000 (0.28) 1.2; left
-    whole: 192 x 2048 (0.8) 54 -> 60, 160 x 8000 (0.8) 173 -> 199, 256 x 1500 (0.4) 0.93 times as fast, 512 x 3000 (0.15) 0.9, x 1500 0.8.
+    24.4 -> 22.1, 128 x 2048 (0.5) 41 -> 35, x 8000 (0.3) 148 -> 103; times as fast with lognormal lengths: 192 x 3000 (0.67, 0.45, 0.28) 1.0, 1.09, 1.2, 160 x
+    6000 (0.71, 0.51, 0.34) 0.95, 1.07, 1.17, 256 x 6000 (0.64, 0.42) 1.05, 1.13, 512 x 6000 1.03, 1.07; three prompts of 777 tokens with their
+    evictions, 192 x 5097 (0.55) 898 -> 878 us, x 4076 (0.69) 1207 -> 1199.  Left whole: 192 x 2048 (0.8) 54 -> 60, 160 x 8000 (0.8) 173 -> 199, 256 x
+    1500 (0.4) 0.93 times as fast, 512 x 3000 (0.15) 0.9, x 1500 0.8.
     The scratch for what is put in place afterwards is 12 bytes a row, 48 MB at most."""
     if segs > 512 or longest > 32768 or segs * longest > 1 << 22:
         return False
-    return longest >= (1024 if segs <= 128 else 3000 if segs <= 256 else 6000) and (segs <= 128 or 2 * rows <= segs * longest)
+    return longest >= (1024 if segs <= 128 else 3000 if segs <= 256 else 4000) and (segs <= 128 or 10 * rows <= 7 * segs * longest)
 
 
 def wide_group(segs: int, longest: int) -> bool:
