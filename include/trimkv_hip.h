@@ -723,7 +723,7 @@ int trimkv_linear_rows_silu(const void* x, int64_t x_stride, const void* w, int6
 /*
  * trimkv_linear_rows_add -- trimkv_linear_rows, its result rounded, plus a residual, rounded again; squares [rows][n / 8] receives
  * sums of the squares of the result over 8 columns at a time.  bf16, up to 32 rows; n a multiple of 16, residual and out 8-byte
- * aligned, their strides multiples of 4.
+ * aligned, their strides multiples of 4; out must not overlap the residual (columns may be taken twice).
  * trimkv_linear_rows_norm -- trimkv_linear_rows or, with silu, trimkv_linear_rows_silu (n then counts the gate's rows) over
  * round(round(x / sqrt(mean(x^2) + eps)) * norm_weight), where the sums in squares [rows][k / 8] say what mean(x^2) is.  bf16, up to
  * 32 rows of up to 8192; squares and norm_weight [k] 16-byte aligned.
