@@ -62,3 +62,18 @@ def test_bad_arguments_are_refused():
     call = lambda strategy=_lib.SCORE_ALPHA, max_len=64, ws=p, size=4096: lib.trimkv_compact_threshold_halves(p, 1, 2, 2, 8, _lib.BF16, _lib.F32, p, p, 0, p, 10, strategy, _lib.ROUND_NATIVE, max_len,
                                                                                                               ws, size, None)
     assert call(strategy=_lib.SCORE_KNORM_ALPHA) < 0 and call(max_len=32769, size=1 << 30) < 0 and call(ws=None) < 0 and call(size=100) < 0 and call(ws=p + 4) < 0
+
+
+def test_a_cache_keeps_no_scratch_of_halves():
+    from trimkv_amd import BatchedDynamicBudgetTrimKVCache
+    from trimkv_amd.cache_utils import compact_halves
+    L, B, H, S, D, keep = 2, 2, 4, 1500, 64, 500
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    cache = BatchedDynamicBudgetTrimKVCache()
+    for l in range(L):
+        k, v = (torch.randn(B, H, S, D, generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2))
+        cache.update(k, v, -torch.rand(B, H, S, generator=gen, device=DEV), torch.arange(S, device=DEV), l)
+    assert compact_halves(L * B * H, S, L * B * H * S)
+    cache.compress(strategy="alpha", memory_size=keep, buffer_size=0)
+    assert cache.get_total_cached_tokens() == L * B * H * keep
+    assert sum(t.numel() for t in cache._ws.values()) < 12 * L * B * H * S

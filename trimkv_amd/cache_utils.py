@@ -1271,7 +1271,8 @@ class _RaggedCache(_SlabBacked):
         ws = None
         if halves:
             try:
-                ws = self._workspace(lib.trimkv_compact_halves_workspace(len(layers), s0.nseg, max_len), dev)
+                # goes back to the allocator behind the launches
+                ws = torch.empty(lib.trimkv_compact_halves_workspace(len(layers), s0.nseg, max_len), dtype=torch.uint8, device=dev)
             except torch.OutOfMemoryError:
                 halves = False
         if not halves:
