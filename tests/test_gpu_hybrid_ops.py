@@ -296,6 +296,26 @@ def test_experts_with_row_counts_at_the_edges_of_tiles():
     close(y, want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each: 2^-8 of the largest each, and slack for their spread
 
 
+@pytest.mark.parametrize("ff,width", [(64, 64), (128, 192), (192, 320), (576, 256), (264, 520)])
+def test_experts_of_either_tile_height(ff, width):
+    """Products of one, two, three and more steps of 64 k, outputs that end in the first or the second half of a tile, and tiles of
+    256 and of 128 rows on either side of the line between them."""
+    counts = [300, 1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 384, 385, 640, 0, 17]
+    E, T, wp, fp = len(counts), sum(counts), ops.padded(width), ops.padded(ff)
+    assert T >= 12 * E and T >= 1200
+    x, up, down = torch.zeros(T, wp), torch.zeros(E, fp, wp), torch.zeros(E, wp, fp)
+    x[:, :width] = rnd(T, width, seed=1)
+    up[:, :ff, :width] = rnd(E, ff, width, seed=2) * width ** -0.5
+    down[:, :width, :ff] = rnd(E, width, ff, seed=3) * ff ** -0.5
+    x, up, down = (t.to(torch.bfloat16) for t in (x, up, down))
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=torch.Generator().manual_seed(4))]
+    y = ops.experts(x.to(DEV), ids[:, None].int().to(DEV), ops.pack_matrix(up).contiguous().to(DEV), ops.pack_matrix(down).contiguous().to(DEV), width)
+    want = torch.empty(T, width, dtype=torch.float64)
+    for e in range(E):
+        want[ids == e] = ref.expert(x[ids == e].double()[:, :width], up[e].double()[:ff, :width], down[e].double()[:width, :ff])
+    close(y[:, :width], want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each, as above
+
+
 @pytest.mark.parametrize("ff,width", [(352, 640), (704, 352)])
 def test_experts_whose_steps_go_round_the_buffers(ff, width):
     """Prompt-sized products of 12, 20 and 22 steps of 32 k: the five operand buffers are filled anew two to four times while

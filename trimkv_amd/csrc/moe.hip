@@ -10,7 +10,7 @@
 // k 0..7 of the 32 outputs, then k 8..15 (lane l of a wavefront: output l % 32, k 8 (l / 32) .. + 7), so that a load
 // instruction reads 1 KiB in one piece: [E][n padded / 32][k padded / 16][2][32][8].  n and k are padded with zeros to
 // multiples of 64, activations are rows of k padded elements: no kernel has a tail along k.
-#include "hybrid.hip.h"
+#include "tiles.hip.h"
 #include <type_traits>
 
 namespace trimkv {
@@ -216,141 +216,96 @@ __global__ __launch_bounds__(KS * 64) void grouped_skinny_kernel(GroupedArgs a) 
     }
 }
 
-// bf16, many rows per expert (prompts): WM YT x 32 rows by WN XT x 32 outputs per workgroup of WM WN wavefronts, each XT x YT
-// tiles of 32x32x16 MFMAs.  Steps of 32 k rotate through five LDS buffers filled by LDS-direct loads, four steps ahead: the
-// weights lane-linear as they lie in memory, token rows gathered, the 16-byte piece c of row r at c ^ ((r / 4) % 4), so that
-// the rows of a fragment read fall on different banks.
-// What bounds it is the way of the operands into LDS, not the matrix cores (busy 61 % of a compute unit's time): with the loads
-// taken out the two products of 8192 tokens x 4 of 32 experts (4096 x 4608) take 1.93 ms, with loads that always hit 2.28 ms, as
-// it is 2.64 ms.  Reads and requests one by one between the products, four steps ahead, rows that are not there not multiplied
-// and equal shares for the XCDs: 2.76 -> 2.64 ms.  Two buffers of 64 k were slower (2.88 ms), four wavefronts of 128 x 128 outputs
-// the same.
-template <bool UP, int XT, int YT, int WN, int WM>
-__global__ __launch_bounds__(WN * WM * 64) void grouped_big_kernel(GroupedArgs a, int n_tiles) {
-    constexpr int THREADS = WN * WM * 64, TM = WM * YT * 32, TN = WN * XT * 32, RL = THREADS / 4, XB = TM * 64, BUF = (TM + TN) * 64;
-    constexpr int XL = TM / RL, WL = TN / 16 / (WN * WM), AHEAD = 4;
-    static_assert(TM % RL == 0 && TN / 16 % (WN * WM) == 0, "whole loads");
+// bf16, more than a few rows per expert (prompts): 256 rows x 256 outputs per workgroup (tiles.hip.h), or 128 rows of the last tile
+// of an expert that holds no more.  With 8192 tokens x 4 of 32 experts (4096 x 4608) it is bound by the clock that the matrix cores leave
+// the chip (1.7 GHz, pipes busy 73 % of a compute unit's time) and by what the L2s fetch: 1.46 PFLOP/s where four rows in a row are one token's
+// and all weights fit the last level of cache, 1.2 PFLOP/s with the rows of a random choice, 1.03 with experts of unequal size, whose last
+// tiles are part empty.  Both products take 2.2 ms; a kernel that fed 32x32x16 products from five buffers of 32 k, all wavefronts in step,
+// took 2.6 ms.
+template <bool UP>
+__global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_tiles, int experts) {
     extern __shared__ __attribute__((aligned(16))) char gb_lds[];
     HY_LDS char* const lds3 = (HY_LDS char*)gb_lds;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)lds3;
-    // The tiles in blocks of 4 row tiles x all outputs, row tiles fastest, cut into eight equal runs, one for each XCD: the rows
-    // and the weights that neighbouring workgroups read stay in its L2.
-    const int total = a.tiles[0], share = (total * n_tiles + 7) / 8, turn = blockIdx.x >> 3, at = (blockIdx.x & 7) * share + turn;
-    if (turn >= share || at >= total * n_tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, hl = lane >> 4, wm = w >> 2, wn = w & 3;
+    // Row tiles that are full come first in the plan.  They and the others are taken apart, in blocks of 4 row tiles x all outputs, row tiles fastest, cut
+    // into eight equal runs, one for each XCD: the rows and the weights that neighbouring workgroups read stay in its L2, every XCD
+    // has as much to do, and the launch ends on short tiles.
+    int full = 0;
+    for (int e = lane; e < experts; e += 64) full += (a.offsets[e + 1] - a.offsets[e]) >> 8;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) full += __shfl_xor(full, d, 64);
+    full = __builtin_amdgcn_readfirstlane(full);
+    const int xcd = blockIdx.x & 7, parts = a.tiles[0] - full;
+    auto from = [&](int tiles, int i) { return (int)((int64_t)tiles * n_tiles * i / 8); };
+    int at = from(full, xcd) + (blockIdx.x >> 3), total = full, base = 0;
+    if (at >= from(full, xcd + 1)) {
+        at = from(parts, xcd) + at - from(full, xcd + 1);
+        if (at >= from(parts, xcd + 1)) return;
+        total = parts;
+        base = full;
+    }
     const int blk = at / (4 * n_tiles), in = at - blk * 4 * n_tiles, high = min(4, total - 4 * blk);
-    const int nt = in / high, rt = 4 * blk + in % high;
-    const int e = a.tiles[1 + 2 * rt], m0 = a.tiles[2 + 2 * rt], mend = a.offsets[e + 1], n0 = nt * TN;
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 31, hl = lane >> 5;
-    // Wavefronts of one wn share a SIMD and take turns on the tile's blocks of 32 rows, of which only those with rows are
-    // multiplied: the last tile of an expert costs what it holds.
-    const int wn = w % WN, wm = w / WN, kb16 = a.kp >> 4;
-    const int blocks = __builtin_amdgcn_readfirstlane((min(mend - m0, TM) + 31) / 32), mine = (blocks - wm + WM - 1) / WM;
-    const uint16_t* xp[XL]; const char* wp[WL];
-    const int lrow = tid >> 2, piece = ((tid & 3) ^ ((lrow >> 2) & 3)) * 8;       // RL is a multiple of 16: one swizzle for all loads
+    const int nt = in / high, rt = base + 4 * blk + in % high;
+    const int e = a.tiles[1 + 2 * rt], m0 = a.tiles[2 + 2 * rt], rows = __builtin_amdgcn_readfirstlane(a.offsets[e + 1] - m0), n0 = nt * 256, kb16 = a.kp >> 4;
+    HY_LDS int32_t* const to = (HY_LDS int32_t*)(lds3 + tile_lds(1, 2));      // rows of y; the barriers of the walk lie between here and the stores
+    if (!UP && tid < 256) to[tid] = a.order[m0 + min(tid, rows - 1)];
+    const uint32_t source = tile_packed_source(lane) * 16;
+    const int nb0 = n0 >> 5, nbs = a.np >> 5;
+    const char* const wb = (const char*)a.w + (int64_t)e * nbs * kb16 * 1024;
+    auto go = [&](auto halves) __attribute__((always_inline)) {
+        constexpr int XH = decltype(halves)::value;
+        const uint16_t* xp[XH][2];
 #pragma unroll
-    for (int x = 0; x < XL; ++x) {
-        const int i = min(m0 + x * RL + lrow, mend - 1);
-        xp[x] = (const uint16_t*)a.x + (UP ? (int64_t)(a.order[i] / a.top) : (int64_t)i) * a.xs + piece;
-    }
+        for (int h = 0; h < XH; ++h)
 #pragma unroll
-    for (int x = 0; x < WL; ++x) {                                                // block w WL + x of the step: outputs / 2, k half % 2
-        const int b = w * WL + x, nb = min((n0 >> 5) + (b >> 1), (a.np >> 5) - 1);
-        wp[x] = (const char*)a.w + (((int64_t)e * (a.np >> 5) + nb) * kb16 + (b & 1)) * 1024;
-    }
-    const uint32_t woff = lane * 16;
-    const int steps = a.kp / 32;
-    // load i of step s, of the wavefront's XL + WL of them
-    auto request = [&](int s, int buf, int i) __attribute__((always_inline)) {
-        const int sc = min(s, steps - 1);                                         // past the end: re-read, never used
-        const uint32_t dst = lds0 + buf * BUF;
-        if (i < XL) load_to_lds16(xp[i] + sc * 32, dst + i * RL * 64 + w * 1024);
-        else load_to_lds16_at(wp[i - XL] + (int64_t)sc * 2048, woff, dst + XB + (w * WL + i - XL) * 1024);
-    };
-    hy_f32x16 acc[XT][YT];
-#pragma unroll
-    for (int x = 0; x < XT; ++x)
-#pragma unroll
-        for (int y = 0; y < YT; ++y)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.0f;
-    const int sw = (j >> 2) & 3;
-    HY_LDS char* const xr = lds3 + (wm * 32 + j) * 64;            // of block wm + WM y: + y WM 2048
-    HY_LDS char* const wr = lds3 + XB + wn * XT * 2048 + lane * 16;
-    constexpr int N = XL + WL;
-    // The first half of a step is in registers when the step begins; its products run behind the reads of the second half and
-    // the requests of step s + AHEAD, the second half's products behind the reads of the next step's first half.  The wavefronts
-    // meet where step s + 1 has landed everywhere and nobody reads step s - 1, whose buffer is requested anew, any more.
-    auto walk = [&](auto count) __attribute__((always_inline)) {
-        constexpr int YC = decltype(count)::value;    // blocks of rows of this wavefront
-        hy_bf16x8 xf[2][YC + 1], wf[2][XT];
-        auto fetch = [&](int ks, int buf, int i) __attribute__((always_inline)) { // operand i of half a step (16 of its 32 k)
-            const int off = buf * BUF;
-            if (i < YC) xf[ks][i] = *(const HY_LDS hy_bf16x8*)(xr + off + i * WM * 2048 + (((2 * ks + hl) ^ sw) << 4));
-            else if (YC && i < YC + XT) wf[ks][i - YC] = *(const HY_LDS hy_bf16x8*)(wr + off + (i - YC) * 2048 + ks * 1024);
-        };
-        auto multiply = [&](int ks, int i) __attribute__((always_inline)) {
-            if (i < XT * YC) acc[i / max(YC, 1)][i % max(YC, 1)] = mfma32(wf[ks][i / max(YC, 1)], xf[ks][i % max(YC, 1)], acc[i / max(YC, 1)][i % max(YC, 1)]);
-        };
-        constexpr int SLOTS = XT * YC > XT + YC ? XT * YC : XT + YC;
-#pragma unroll
-        for (int i = 0; i < XT + YC; ++i) fetch(0, 0, i);
-        int buf = 0, next = 1, last = AHEAD;          // of step s, s + 1 and s + AHEAD
-        for (int s = 0; s < steps; ++s) {
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((AHEAD - 2) * N) : "memory");
-#pragma unroll
-            for (int i = 0; i < 2 * SLOTS; ++i) {
-                multiply(i / SLOTS, i % SLOTS);
-                if (i < SLOTS) fetch(1, buf, i); else fetch(0, next, i - SLOTS);
-                // the requests are spread over the step: in one burst they queue up in front of the L1 and the products wait
-#pragma unroll
-                for (int x = i * N / (2 * SLOTS); x < (i + 1) * N / (2 * SLOTS); ++x) request(s + AHEAD, last, x);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 2; ++i) {
+                const int r = h * 128 + (2 * w + i) * 8 + (lane >> 3), x = m0 + min(r, rows - 1);
+                xp[h][i] = (const uint16_t*)a.x + (UP ? (int64_t)(a.order[x] / a.top) : (int64_t)x) * a.xs + (((lane & 7) ^ tile_swizzle_x(r)) << 3);
             }
-            buf = next;
-            next = next == AHEAD ? 0 : next + 1;
-            last = last == AHEAD ? 0 : last + 1;
-        }
+        hy_f32x4 acc[XH][2][4][2];
+        walk_tile<XH, 2, true>(lds3, a.kp >> 6, [&](int h, int i, int step, uint32_t dst) __attribute__((always_inline)) { load_to_lds16(xp[h][i] + step * 64, dst); },
+            [&](int h, int i, int step, uint32_t dst) __attribute__((always_inline)) {
+                const int b = 2 * w + i, nb = min(nb0 + h * 4 + (b >> 2), nbs - 1);
+                load_to_lds16_at(wb + ((int64_t)nb * kb16 + step * 4 + (b & 3)) * 1024, source, dst);
+            }, acc);
+#pragma unroll
+        for (int xh = 0; xh < XH; ++xh)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = xh * 128 + wm * 64 + r * 16 + j;
+                if (i >= rows) continue;
+                uint16_t* const y = (uint16_t*)a.y + (UP ? (int64_t)(m0 + i) : (int64_t)to[i]) * a.ys;
+#pragma unroll
+                for (int wh = 0; wh < 2; ++wh) {
+                    const int n = n0 + wh * 128 + wn * 32 + hl * 8;
+                    float f[8];
+#pragma unroll
+                    for (int v = 0; v < 8; ++v) f[v] = expert_act<UP>(acc[xh][wh][r][v >> 2][v & 3]);
+                    if (n + 7 < a.n && a.ys % 8 == 0) { *(uint4*)(y + n) = make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7])); continue; }
+#pragma unroll
+                    for (int v = 0; v < 8; ++v)
+                        if (n + v < a.n) y[n + v] = f32_to_bf16_bits(f[v]);
+                }
+            }
     };
-#pragma unroll
-    for (int p = 0; p < AHEAD; ++p)
-#pragma unroll
-        for (int i = 0; i < N; ++i) request(p, p, i);
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"((AHEAD - 1) * N) : "memory");
-    __syncthreads();
-    static_assert(YT == 4, "one walk for every number of blocks");
-    if (mine == 4) walk(std::integral_constant<int, 4>{});
-    else if (mine == 3) walk(std::integral_constant<int, 3>{});
-    else if (mine == 2) walk(std::integral_constant<int, 2>{});
-    else if (mine == 1) walk(std::integral_constant<int, 1>{});
-    else walk(std::integral_constant<int, 0>{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS after the workgroup has gone
-    // acc[x][y]: outputs n0 + (wn XT + x) 32 + 8 (v / 4) + 4 hl + v % 4 of row m0 + (wm + WM y) 32 + j
-#pragma unroll
-    for (int y = 0; y < YT; ++y) {
-        const int i = m0 + (wm + WM * y) * 32 + j;
-        if (i >= mend) continue;
-        uint16_t* yr = (uint16_t*)a.y + (UP ? (int64_t)i : (int64_t)a.order[i]) * a.ys;
-#pragma unroll
-        for (int x = 0; x < XT; ++x)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                store_outputs<UP>(a, yr, n0 + (wn * XT + x) * 32 + 8 * c + 4 * hl, acc[x][y][4 * c], acc[x][y][4 * c + 1], acc[x][y][4 * c + 2], acc[x][y][4 * c + 3]);
-    }
+    if (rows > 128) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 1>{});
 }
 
-template <bool UP, int XT, int YT, int WN, int WM>
-static int launch_big(const GroupedArgs& a, int most, hipStream_t s) {
-    constexpr int LDS = 5 * (WM * YT + WN * XT) * 32 * 64;
+template <bool UP>
+static int launch_big(const GroupedArgs& a, int most, int experts, hipStream_t s) {
+    constexpr int LDS = tile_lds(1, 2) + 1024;
+    static_assert(tile_lds(2, 2) <= tile_lds(1, 2) && LDS <= 163840, "both forms fit");
     static bool opted_in[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
     if (dev < 0 || !opted_in[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)grouped_big_kernel<UP, XT, YT, WN, WM>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        hipError_t e = hipFuncSetAttribute((const void*)grouped_big_kernel<UP>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) opted_in[dev] = true;
     }
-    const int n_tiles = (a.np + WN * XT * 32 - 1) / (WN * XT * 32), blocks = 8 * ((most * n_tiles + 7) / 8);
-    hipLaunchKernelGGL((grouped_big_kernel<UP, XT, YT, WN, WM>), dim3(blocks), dim3(WN * WM * 64), LDS, s, a, n_tiles);
+    const int n_tiles = (a.np + 255) / 256, blocks = 8 * (most * n_tiles / 8 + 2);
+    hipLaunchKernelGGL((grouped_big_kernel<UP>), dim3(blocks), dim3(512), LDS, s, a, n_tiles, experts);
     return 0;
 }
 
@@ -400,7 +355,7 @@ extern "C" int trimkv_moe_gemm(const void* x, int64_t x_stride, const void* w, v
     const int most = rows < experts ? rows : (rows - experts) / tile + experts;     // no more row tiles than this
     const dim3 grid(most, n_padded / 64);
     if (tile == 256) {
-        const int rc = up ? launch_big<true, 2, 4, 4, 2>(a, most, s) : launch_big<false, 2, 4, 4, 2>(a, most, s);
+        const int rc = up ? launch_big<true>(a, most, experts, s) : launch_big<false>(a, most, experts, s);
         if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
     } else if (dtype == TRIMKV_BF16) {
         const dim3 g(most, n_padded / 32);

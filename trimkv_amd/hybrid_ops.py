@@ -288,8 +288,11 @@ def experts(x: torch.Tensor, ids: torch.Tensor, up: torch.Tensor, down: torch.Te
     E, ffp, wp = up.shape[0], up.shape[1] * 32, up.shape[2] * 16
     T, top = ids.shape
     M, dev, lib, st, code = T * top, x.device, _lib.load_hybrid("moe"), _lib.current_stream(x.device), _lib.dtype_code(up.dtype)
-    # rows per expert: many -> tiles of the matrix-bound kernel, a few -> the weights stream past them
-    tile = 16 if up.dtype == torch.float32 else 256 if M >= 96 * E else 32
+    # A few rows per expert: the weights stream past them, once per 32.  From a dozen on the tiles of the matrix-bound kernel read them once, given enough
+    # tiles to fill the chip.  us with 32 | 256, both products: 32 experts of 4096 x 4608 with 8, 16, 64, 96 rows each 415 | 439, 509 | 438, 1567 | 467,
+    # 2222 | 485; 32 of 2048 x 2304 with 8, 12, 16: 114 | 128, 126 | 131, 142 | 131; 8 of 2048 x 2304 with 12, 16: 56 | 54, 64 | 55; 4 of them with 24, 32,
+    # 48: 47 | 54, 56 | 54, 76 | 55; 8 of 1024 x 1024 with 32, 48: 29 | 33, 39 | 34.
+    tile = 16 if up.dtype == torch.float32 else 256 if M >= 12 * E and M * ((min(ffp, wp) + 255) // 256) >= 1200 else 32
     most = M if M < E else (M - E) // tile + E
     order = torch.empty(M, dtype=torch.int32, device=dev)
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
