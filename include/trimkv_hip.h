@@ -732,6 +732,20 @@ int trimkv_linear_rows_add(const void* x, int64_t x_stride, const void* w, int64
                            void* out, int64_t out_stride, float* squares, int rows, int n, int k, int dtype, void* stream);
 int trimkv_linear_rows_norm(const void* x, int64_t x_stride, const float* squares, const void* norm_weight, float eps, const void* w, int64_t w_stride,
                             const void* bias, void* out, int64_t out_stride, int rows, int n, int k, int silu, int round_all, int dtype, void* stream);
+/*
+ * trimkv_linear_tiles -- out[m][n] = round(sum_k x[m][k] w[n][k]): a linear layer over many rows, the tokens of a prompt.
+ * trimkv_linear_tiles_silu -- w [2 inter][k]: silu(gate) * up as trimkv_linear_rows_silu.
+ * bf16; k a multiple of 64, up to 2^24 rows and outputs, strides (in elements) of x and w multiples of 8 up to 2^20, x and w 16-byte
+ * aligned.  form: how the work is cut, 0: by sizes; 1, 2, 3: tiles of 256, 192 or 128 rows x 256 outputs (silu: x 128), without silu also + 8, + 16: rows, columns
+ * that fill no whole tile go in tiles of 128 x 128, and 4: all do.
+ * trimkv_linear_tiles_form -- the form by sizes, or 0 where a general product is faster (few rows).
+ * libtrimkv_hybrid.so holds them as well.
+ */
+int trimkv_linear_tiles(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int64_t out_stride, int rows, int n, int k, int form,
+                        int dtype, void* stream);
+int trimkv_linear_tiles_silu(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out, int64_t out_stride, int rows, int inter, int k,
+                             int round_all, int form, int dtype, void* stream);
+int trimkv_linear_tiles_form(int rows, int n, int k, int silu);
 
 #ifdef __cplusplus
 }

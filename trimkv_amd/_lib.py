@@ -40,6 +40,9 @@ SIGNATURES = {
     "trimkv_rope_tables": (_i, [_p, _p, _p, _p, _i, _i, _i, _p]),
     "trimkv_linear_rows": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p]),
     "trimkv_linear_rows_silu": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
+    "trimkv_linear_tiles": (_i, [_p, _i64, _p, _i64, _p, _i64, _i, _i, _i, _i, _i, _p]),
+    "trimkv_linear_tiles_silu": (_i, [_p, _i64, _p, _i64, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
+    "trimkv_linear_tiles_form": (_i, [_i, _i, _i, _i]),
     "trimkv_linear_rows_add": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _p, _i64, _p, _i, _i, _i, _i, _p]),
     "trimkv_linear_rows_norm": (_i, [_p, _i64, _p, _p, _f, _p, _i64, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
     "trimkv_gate_hidden_packed": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p]),
@@ -137,7 +140,7 @@ HYBRID_SIGNATURES = {
 }
 
 # entry points of trimkv_hip.h that another library holds as well
-SHARED = {"hybrid": ("trimkv_linear_rows", "trimkv_linear_rows_silu")}
+SHARED = {"hybrid": ("trimkv_linear_rows", "trimkv_linear_rows_silu", "trimkv_linear_tiles", "trimkv_linear_tiles_silu", "trimkv_linear_tiles_form")}
 
 _lib = None
 _hybrid = {}

@@ -16,8 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB_PATH = os.path.join(HERE, "libtrimkv_hip.so")
-SOURCES = ["api.hip", "append.hip", "evict.hip", "attn_decode.hip", "attn_decode_append.hip", "attn_decode_pieces.hip", "attn_decode_append_pieces.hip", "attn_decode_append_gated.hip", "attn_decode_append_pieces_gated.hip", "pieces_plan.hip", "attn_prefill.hip", "gate.hip", "stream_probe.hip", "decoder_ops.hip", "linear_rows.hip"]
-HYBRID_SOURCES = ["hybrid_ops.hip", "window_attn.hip", "window_decode.hip", "linear_rows.hip"]
+SOURCES = ["api.hip", "append.hip", "evict.hip", "attn_decode.hip", "attn_decode_append.hip", "attn_decode_pieces.hip", "attn_decode_append_pieces.hip", "attn_decode_append_gated.hip", "attn_decode_append_pieces_gated.hip", "pieces_plan.hip", "attn_prefill.hip", "gate.hip", "stream_probe.hip", "decoder_ops.hip", "linear_rows.hip", "linear_tiles.hip"]
+HYBRID_SOURCES = ["hybrid_ops.hip", "window_attn.hip", "window_decode.hip", "linear_rows.hip", "linear_tiles.hip"]
 LIBRARIES = {"hip": (LIB_PATH, SOURCES), "hybrid": (os.path.join(HERE, "libtrimkv_hybrid.so"), HYBRID_SOURCES),
              "mlstm": (os.path.join(HERE, "libtrimkv_mlstm.so"), ["mlstm.hip"]), "moe": (os.path.join(HERE, "libtrimkv_moe.so"), ["moe.hip"])}
 
@@ -63,7 +63,7 @@ def build(verbose: bool = True, only_changed: bool = False, libraries=tuple(LIBR
     def compile_one(src):
         return _run([hipcc] + HIPCC_FLAGS + EXTRA_FLAGS.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj_of(src)])
 
-    srcs = list(dict.fromkeys(srcs))       # linear_rows.hip belongs to two libraries
+    srcs = list(dict.fromkeys(srcs))       # linear_rows.hip and linear_tiles.hip belong to two libraries
     if srcs:
         with ThreadPoolExecutor(max_workers=min(os.cpu_count() or 4, 8, len(srcs))) as ex:
             for src, out in zip(srcs, ex.map(compile_one, srcs)):

@@ -216,8 +216,8 @@ __global__ __launch_bounds__(KS * 64) void grouped_skinny_kernel(GroupedArgs a) 
     }
 }
 
-// bf16, more than a few rows per expert (prompts): 256 rows x 256 outputs per workgroup (tiles.hip.h), or 128 rows of the last tile
-// of an expert that holds no more.  With 8192 tokens x 4 of 32 experts (4096 x 4608) it is bound by the clock that the matrix cores leave
+// bf16, more than a few rows per expert (prompts): 256 rows x 256 outputs per workgroup (tiles.hip.h), or 192 or 128 rows of the
+// last tile of an expert that holds no more.  With 8192 tokens x 4 of 32 experts (4096 x 4608) it is bound by the clock that the matrix cores leave
 // the chip (1.7 GHz, pipes busy 73 % of a compute unit's time) and by what the L2s fetch: 1.46 PFLOP/s where four rows in a row are one token's
 // and all weights fit the last level of cache, 1.2 PFLOP/s with the rows of a random choice, 1.03 with experts of unequal size, whose last
 // tiles are part empty.  Both products take 2.2 ms; a kernel that fed 32x32x16 products from five buffers of 32 k, all wavefronts in step,
@@ -252,18 +252,18 @@ __global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_t
     const uint32_t source = tile_packed_source(lane) * 16;
     const int nb0 = n0 >> 5, nbs = a.np >> 5;
     const char* const wb = (const char*)a.w + (int64_t)e * nbs * kb16 * 1024;
-    auto go = [&](auto halves) __attribute__((always_inline)) {
-        constexpr int XH = decltype(halves)::value;
+    auto go = [&](auto halves, auto blocks) __attribute__((always_inline)) {
+        constexpr int XH = decltype(halves)::value, R = decltype(blocks)::value;
         const uint16_t* xp[XH][2];
 #pragma unroll
         for (int h = 0; h < XH; ++h)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int r = h * 128 + (2 * w + i) * 8 + (lane >> 3), x = m0 + min(r, rows - 1);
+                const int r = h * 32 * R + tile_x_load<R>(w, i) * 8 + (lane >> 3), x = m0 + min(r, rows - 1);
                 xp[h][i] = (const uint16_t*)a.x + (UP ? (int64_t)(a.order[x] / a.top) : (int64_t)x) * a.xs + (((lane & 7) ^ tile_swizzle_x(r)) << 3);
             }
-        hy_f32x4 acc[XH][2][4][2];
-        walk_tile<XH, 2, true>(lds3, a.kp >> 6, [&](int h, int i, int step, uint32_t dst) __attribute__((always_inline)) { load_to_lds16(xp[h][i] + step * 64, dst); },
+        hy_f32x4 acc[XH][2][R][2];
+        walk_tile<XH, 2, R, true>(lds3, a.kp >> 6, [&](int h, int i, int step, uint32_t dst) __attribute__((always_inline)) { load_to_lds16(xp[h][i] + step * 64, dst); },
             [&](int h, int i, int step, uint32_t dst) __attribute__((always_inline)) {
                 const int b = 2 * w + i, nb = min(nb0 + h * 4 + (b >> 2), nbs - 1);
                 load_to_lds16_at(wb + ((int64_t)nb * kb16 + step * 4 + (b & 3)) * 1024, source, dst);
@@ -271,8 +271,8 @@ __global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_t
 #pragma unroll
         for (int xh = 0; xh < XH; ++xh)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = xh * 128 + wm * 64 + r * 16 + j;
+            for (int r = 0; r < R; ++r) {
+                const int i = xh * 32 * R + wm * 16 * R + r * 16 + j;
                 if (i >= rows) continue;
                 uint16_t* const y = (uint16_t*)a.y + (UP ? (int64_t)(m0 + i) : (int64_t)to[i]) * a.ys;
 #pragma unroll
@@ -288,8 +288,10 @@ __global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_t
                 }
             }
     };
-    if (rows > 128) go(std::integral_constant<int, 2>{});
-    else go(std::integral_constant<int, 1>{});
+    const std::integral_constant<int, 1> one; const std::integral_constant<int, 2> two; const std::integral_constant<int, 3> three; const std::integral_constant<int, 4> four;
+    if (rows > 192) go(two, four);
+    else if (rows > 128) go(two, three);
+    else go(one, four);
 }
 
 template <bool UP>

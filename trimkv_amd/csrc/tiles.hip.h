@@ -5,13 +5,13 @@
 
 namespace trimkv {
 
-// A workgroup of 8 wavefronts multiplies XH x 128 rows of x with WH x 128 rows of w ("outputs") in steps of 64 k, which rotate
-// through tile_buffers() LDS buffers filled by LDS-direct loads.  In a buffer, half h of x (128 rows of 64 k, 16 KiB) lies at
-// h 16 KiB, half h of w behind those of x.
+// A workgroup of 8 wavefronts multiplies XH halves of 32 R rows of x (R = 4 or 3) with WH halves of 128 rows of w ("outputs") in steps of 64 k,
+// which rotate through tile_buffers() LDS buffers filled by LDS-direct loads.  In a buffer, half h of x (4 R KiB) lies at h 4 R KiB,
+// half h of w (16 KiB) behind those of x.
 //
 // A step has XH WH phases, one for each pair of halves, and each phase two parts: reading the fragments that it needs (and
-// requesting 16 KiB of a later step), then 16 products of 16x16x32 per wavefront.  The wavefronts of rows 0 .. 63 of a half and
-// those of rows 64 .. 127, one of each on every SIMD, are half a phase apart: while one multiplies, the other reads.  The
+// requesting as much of a later step), then 4 R products of 16x16x32 per wavefront.  The wavefronts of the first 16 R rows of a half and
+// those of the others, one of each on every SIMD, are half a phase apart: while one multiplies, the other reads.  The
 // barrier between the parts keeps them so, and with it the matrix cores never wait for LDS (16 fragments of 1 KiB are 4 x 8 KiB
 // or 256 of a compute unit's cycles, as long as the products take); it also guards the buffers: what a part has read is requested anew
 // two parts later at the earliest, what it reads has landed in the whole workgroup two parts before.
@@ -20,7 +20,7 @@ namespace trimkv {
 // w read a phase ahead: 1.37 -> 1.44 at 32768 x 4608 x 4096 (12, 4, 8 and no fragments of a phase become 8, 4, 8 and 4).  A barrier before the last two or four products of a
 // phase instead of behind them: 1.33.
 constexpr int tile_buffers(int xh, int wh) { return xh + wh == 4 ? 2 : xh + wh == 3 ? 3 : 4; }
-constexpr int tile_lds(int xh, int wh) { return tile_buffers(xh, wh) * (xh + wh) * 16384; }
+constexpr int tile_lds(int xh, int wh, int r = 4) { return tile_buffers(xh, wh) * (xh * r * 4096 + wh * 16384); }
 
 // Where a fragment's outputs lie among the 32 of a wavefront: fragment c, MFMA row i <-> output 8 (i / 4) + 4 c + i % 4, so that a lane's
 // accumulators of both fragments are eight outputs in a row.
@@ -32,6 +32,9 @@ __device__ __forceinline__ int tile_swizzle_x(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int tile_swizzle_w(int r) { return ((r >> 1) & 1) | (((r >> 3) & 3) << 1); }
 // w in blocks of 32 outputs x 16 k (two halves of 8 k): place p of a block in LDS is taken from this place in memory
 __device__ __forceinline__ int tile_packed_source(int p) { return (p & 32) + tile_output((p >> 4) & 1, p & 15); }
+
+// KiB (8 rows) of a half of x that wavefront w requests as its load i; of 12 KiB the last wavefronts request one twice
+template <int R> __device__ __forceinline__ int tile_x_load(int w, int i) { return R == 4 ? 2 * w + i : i && w < 4 ? 8 + w : w; }
 
 __device__ __forceinline__ void tile_meet() {
     __builtin_amdgcn_sched_barrier(0);
@@ -45,17 +48,18 @@ template <int N> __device__ __forceinline__ void tile_meet_landed() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// acc[xh][wh][r][c][v]: row 128 xh + 64 (w / 4) + 16 r + lane % 16, output 128 wh + 32 (w % 4) + 8 (lane / 16) + 4 c + v for wavefront w.
-// request_x(h, i, step, lds_addr), request_w(...): the wavefront's LDS-direct load i (of 2) of half h of that step: 1 KiB each, KiB 2 w + i of the half;
-// x and row-major w: 8 rows of 128 bytes; packed w: block 2 w + i, of 32 outputs x 16 k (outputs 32 ((2 w + i) / 4), k 16 ((2 w + i) % 4)).
-template <int XH, int WH, bool PACKED, class RequestX, class RequestW>
-__device__ __forceinline__ void walk_tile(HY_LDS char* lds3, int steps, RequestX request_x, RequestW request_w, hy_f32x4 (&acc)[XH][WH][4][2]) {
-    constexpr int B = tile_buffers(XH, WH), BUF = (XH + WH) * 16384, XB = XH * 16384;
+// acc[xh][wh][r][c][v]: row 32 R xh + 16 R (w / 4) + 16 r + lane % 16, output 128 wh + 32 (w % 4) + 8 (lane / 16) + 4 c + v for wavefront w.
+// request_x(h, i, step, lds_addr), request_w(...): the wavefront's LDS-direct load i (of 2) of half h of that step: 1 KiB each, of x KiB tile_x_load<R>(w, i)
+// of the half, of w KiB 2 w + i; x and row-major w: 8 rows of 128 bytes; packed w: block 2 w + i, of 32 outputs x 16 k (outputs
+// 32 ((2 w + i) / 4), k 16 ((2 w + i) % 4)).
+template <int XH, int WH, int R, bool PACKED, class RequestX, class RequestW>
+__device__ __forceinline__ void walk_tile(HY_LDS char* lds3, int steps, RequestX request_x, RequestW request_w, hy_f32x4 (&acc)[XH][WH][R][2]) {
+    constexpr int B = tile_buffers(XH, WH), HALF = R * 4096, XB = XH * HALF, BUF = XB + WH * 16384;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds3;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, hl = lane >> 4, wm = w >> 2, wn = w & 3;
     auto x_of = [&](int step, int buf, int h) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) request_x(h, i, min(step, steps - 1), lds0 + buf * BUF + h * 16384 + (2 * w + i) * 1024);      // past the end: read again, never used
+        for (int i = 0; i < 2; ++i) request_x(h, i, min(step, steps - 1), lds0 + buf * BUF + h * HALF + tile_x_load<R>(w, i) * 1024);      // past the end: read again, never used
     };
     auto w_of = [&](int step, int buf, int h) __attribute__((always_inline)) {
 #pragma unroll
@@ -66,16 +70,16 @@ __device__ __forceinline__ void walk_tile(HY_LDS char* lds3, int steps, RequestX
 #pragma unroll
         for (int wh = 0; wh < WH; ++wh)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[xh][wh][i >> 1][i & 1] = hy_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    hy_bf16x8 xf[4][2], wf[3][2][2];
-    HY_LDS char* const xr = lds3 + (wm * 64 + j) * 128;
+            for (int i = 0; i < 2 * R; ++i) acc[xh][wh][i >> 1][i & 1] = hy_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    hy_bf16x8 xf[R][2], wf[3][2][2];
+    HY_LDS char* const xr = lds3 + (wm * 16 * R + j) * 128;
     HY_LDS char* const wr = lds3 + XB + (PACKED ? wn * 4096 + (hl >> 1) * 1024 + (hl & 1) * 512 + j * 16 : (wn * 32 + tile_output(0, j)) * 128);
     const int xsw = tile_swizzle_x(j), wsw = tile_swizzle_w(tile_output(0, j));
     auto read_x = [&](int buf, int h) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int q = 0; q < 2; ++q) xf[r][q] = *(const HY_LDS hy_bf16x8*)(xr + buf * BUF + h * 16384 + r * 2048 + (((4 * q + hl) ^ xsw) << 4));
+            for (int q = 0; q < 2; ++q) xf[r][q] = *(const HY_LDS hy_bf16x8*)(xr + buf * BUF + h * HALF + r * 2048 + (((4 * q + hl) ^ xsw) << 4));
     };
     auto read_w = [&](int buf, int h, int to) __attribute__((always_inline)) {
 #pragma unroll
@@ -89,7 +93,10 @@ __device__ __forceinline__ void walk_tile(HY_LDS char* lds3, int steps, RequestX
     auto multiply = [&](int xh, int wh, int from) __attribute__((always_inline)) {
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[xh][wh][(i >> 1) & 3][i & 1] = mfma16(wf[from][i & 1][i >> 3], xf[(i >> 1) & 3][i >> 3], acc[xh][wh][(i >> 1) & 3][i & 1]);
+        for (int i = 0; i < 4 * R; ++i) {
+            const int q = i / (2 * R), r = i / 2 % R, c = i & 1;
+            acc[xh][wh][r][c] = mfma16(wf[from][c][q], xf[r][q], acc[xh][wh][r][c]);
+        }
         __builtin_amdgcn_s_setprio(0);
         tile_meet();
     };

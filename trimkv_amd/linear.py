@@ -1,4 +1,5 @@
-"""Linear layers over the rows of a decode step on trimkv_linear_rows; everything else goes to ``F.linear``.
+"""Linear layers over the rows of a decode step on trimkv_linear_rows and over those of a prompt on trimkv_linear_tiles; everything else goes to
+``F.linear``.
 
 Both give fp32 sums rounded once; the order of the sums differs.
 """
@@ -62,10 +63,33 @@ def _rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -
     return None if max(x2.stride(0), weight.stride(0)) > 1 << 24 else x2
 
 
+def _tiles(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], silu: bool, library: Optional[str]):
+    """``(x as [rows, k], form)`` the way trimkv_linear_tiles takes this product, or None where it does not or is not faster."""
+    k = x.shape[-1] if x.dim() else 0
+    if bias is not None or k == 0 or k % 64 or x.numel() <= MAX_ROWS * k or x.dtype != torch.bfloat16 or not _plain(x, weight):
+        return None
+    if weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0 or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 8 or weight.data_ptr() % 16:
+        return None
+    if x.dim() != 2 and not x.is_contiguous():
+        return None
+    x2 = x if x.dim() == 2 else x.view(-1, k)
+    if x2.stride(1) != 1 or x2.data_ptr() % 16 or x2.stride(0) < k or x2.stride(0) % 8 or max(x2.stride(0), weight.stride(0)) > 1 << 20:
+        return None
+    n = weight.shape[0] // 2 if silu else weight.shape[0]
+    if max(x2.shape[0], n) > 1 << 24 or (silu and weight.shape[0] % 2):
+        return None
+    lib = _lib.load() if library is None else _lib.load_hybrid(library)
+    form = lib.trimkv_linear_tiles_form(x2.shape[0], n, k, int(silu))
+    return (x2, form) if form else None
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, library: Optional[str] = None) -> torch.Tensor:
     """``F.linear(x, weight, bias)``.  ``library``: which one holds the kernel (a name of ``_lib.SHARED``; None: libtrimkv_hip.so)."""
     x2 = _rows(x, weight, bias)
-    if x2 is None or (x2.shape[0] > WIDE_ROWS and weight.shape[0] > WIDE):
+    if x2 is None:
+        many = _tiles(x, weight, bias, False, library)
+        return F.linear(x, weight, bias) if many is None else _tile_product(x, *many, weight, library)
+    if x2.shape[0] > WIDE_ROWS and weight.shape[0] > WIDE:
         return F.linear(x, weight, bias)
     rows, k = x2.shape
     n = weight.shape[0]
@@ -78,10 +102,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     return out
 
 
+def _tile_product(x: torch.Tensor, x2: torch.Tensor, form: int, weight: torch.Tensor, library: Optional[str], silu: bool = False, round_all: bool = True) -> torch.Tensor:
+    rows, k = x2.shape
+    n = weight.shape[0] // 2 if silu else weight.shape[0]
+    out = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
+    lib = _lib.load() if library is None else _lib.load_hybrid(library)
+    at, tail = (x2.data_ptr(), x2.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), n, rows, n, k), (form, _lib.BF16, _lib.current_stream(x.device))
+    rc = lib.trimkv_linear_tiles_silu(*at, int(round_all), *tail) if silu else lib.trimkv_linear_tiles(*at, *tail)
+    if rc:
+        _lib.check(rc, "trimkv_linear_tiles") if library is None else _lib.check_hybrid(rc, "trimkv_linear_tiles", library)
+    return out
+
+
 def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, round_all: bool = True, library: Optional[str] = None) -> Optional[torch.Tensor]:
-    """``silu(x @ gate.T) * (x @ up.T)`` with ``weight`` = gate over up, in one launch; None where trimkv_linear_rows_silu does not take it."""
+    """``silu(x @ gate.T) * (x @ up.T)`` with ``weight`` = gate over up, in one launch; None where neither trimkv_linear_rows_silu nor
+    trimkv_linear_tiles_silu takes it."""
     x2 = _rows(x, weight, bias)
-    if x2 is None or weight.shape[0] % 2:
+    if x2 is None:
+        many = _tiles(x, weight, bias, True, library)
+        return None if many is None else _tile_product(x, *many, weight, library, True, round_all)
+    if weight.shape[0] % 2:
         return None
     rows, k = x2.shape
     inter = weight.shape[0] // 2
