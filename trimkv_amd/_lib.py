@@ -164,6 +164,21 @@ def load():
     return lib
 
 
+_step = None
+
+
+def step():
+    """The extension module of decode steps' host side (csrc/step.cpp); raises if it has not been built."""
+    global _step
+    if _step is None:
+        try:
+            from . import _step as module
+        except ImportError as e:
+            raise TrimKVLibraryError(f"trimkv_amd/_step.so is missing or does not load ({e}): build it with `python -m trimkv_amd.build step`. There is no fallback.") from e
+        _step = module
+    return _step
+
+
 def load_hybrid(name: str = "hybrid"):
     """The ctypes handle of one of the hybrid decoders' libraries (loaded once); raises if it has not been built."""
     if name in _hybrid:

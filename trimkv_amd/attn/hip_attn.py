@@ -18,6 +18,7 @@ ragged entry points ignore ``attention_mask`` and ``scaling`` (flash_attn.py:15,
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import os
 import warnings
@@ -77,10 +78,13 @@ def _uniform_cut(nseg: int, max_len: int, least: int = 0) -> int:
     that about 256 workgroups exist (a compute unit pulls about 50 GB/s whatever it runs, so all 256 are needed), but not
     below ``least`` rows apiece (0: ``dense_min_rows``); the pieces are merged inside the launch (``trimkv_decode_attn_uniform``), which saves the second
     launch of the grid-split path.  1 when the segments are attended whole (256 segments or more, or short ones)."""
-    if nseg >= 256 or nseg > 8192:
-        return 1
-    want = (dense_workgroups + nseg - 1) // nseg
-    chunk = max(least or dense_min_rows, (((max_len + want - 1) // want + 63) // 64) * 64)
+    return 1 if nseg >= 256 else _cut(nseg, max_len, least or dense_min_rows, dense_workgroups)
+
+
+@functools.lru_cache(maxsize=4096)
+def _cut(nseg: int, max_len: int, least: int, workgroups: int) -> int:
+    want = (workgroups + nseg - 1) // nseg
+    chunk = max(least, (((max_len + want - 1) // want + 63) // 64) * 64)
     return max(1, (max_len + chunk - 1) // chunk)
 
 
@@ -143,44 +147,60 @@ def decode_attention(query: torch.Tensor, k_rows: torch.Tensor, v_rows: torch.Te
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _pieces_workspace(pieces: int, group: int) -> int:
+    return _lib.load().trimkv_decode_attn_pieces_workspace(pieces, group)
+
+
+@functools.lru_cache(maxsize=1)
+def _entry() -> int:
+    """Address of ``trimkv_append_attend_step``."""
+    return ctypes.cast(_lib.load().trimkv_append_attend_step, ctypes.c_void_p).value
+
+
+def _empty_out(query: torch.Tensor) -> torch.Tensor:
+    if query.dim() != 4:
+        return torch.empty_like(query)
+    B, Hq, Q, D = query.shape
+    return torch.empty(B, Q, Hq, D, dtype=query.dtype, device=query.device)
+
+
 def append_attend(slab, query: torch.Tensor, group: int, scale: float, chunk: int = 0,
                   seg_order: Optional[torch.Tensor] = None, pieces=None, uniform_pps: int = 0, bound: int = 0) -> torch.Tensor:
     """The deferred one-token append of ``slab`` (a cache layer whose ``update`` ran with ``fuse_decode_append``) and the
-    attention over the layer including that token, in one launch: ``trimkv_append_attend``.  ``query`` [nseg*group, D]
-    contiguous -> [nseg*group, D].  Clears the pending append.  ``bound`` > 0: the launch is sized for segments of up to
+    attention over the layer including that token, in one launch: ``trimkv_append_attend``.  ``query`` contiguous, [nseg*group, D]
+    -> [nseg*group, D] or [B,Hq,1,D] -> [B,1,Hq,D].  Clears the pending append.  ``bound`` > 0: the launch is sized for segments of up to
     that many rows instead of the host's record of the longest one (a step that must not depend on host-side lengths)."""
     lib = _lib.load()
     nseg, d = slab.B * slab.H, slab.D
-    out = torch.empty_like(query)
     st = _lib.current_stream(query.device)
     # a log beta that the retention gate left unfinished (LazyLogBeta) is finished by the same launch: the gated entry points
-    gated = not torch.is_tensor(slab.pending[3])
-    if uniform_pps > 0:      # a dense cache: every segment holds max_len - 1 rows before this token; length and cut are launch arguments
-        ws = _workspace_zeroed(query.device, lib.trimkv_decode_attn_pieces_workspace(nseg * uniform_pps, group), st) if uniform_pps > 1 else None
+    gated = not isinstance(slab.pending[3], torch.Tensor)
+    if uniform_pps > 0 or pieces is not None:
+        # a dense cache: every segment holds max_len - 1 rows before this token; length and cut are launch arguments.  Ragged lengths: one launch over the
+        # (segment, piece) list.  Either is merged inside the launch
+        count = uniform_pps if uniform_pps > 0 else pieces[1]
+        rows = slab.max_len - 1 if uniform_pps > 0 else bound if bound > 0 else slab.max_len
+        plist = 0 if uniform_pps > 0 else pieces[0].data_ptr()
+        ws = _workspace_zeroed(query.device, _pieces_workspace(nseg * uniform_pps if uniform_pps > 0 else count, group), st) if uniform_pps != 1 else None
         wp, wn = (0, 0) if ws is None else (ws.data_ptr(), ws.numel())
-        if gated:
+        if not gated:      # the call is made for every layer of every step
+            out = _lib.step().attend(slab, query, group, scale, rows, count, plist, wp, wn, st, _entry())
+            if type(out) is int:
+                _lib.check(out, "trimkv_append_attend_uniform" if uniform_pps > 0 else "trimkv_append_attend_pieces")
+            return out
+        out = _empty_out(query)
+        if uniform_pps > 0:
             rc = lib.trimkv_append_attend_uniform_gated(query.data_ptr(), out.data_ptr(), *slab.ptrs, nseg, slab.H, slab.cap, d, group, *slab.codes, *slab.pending[0], scale,
-                                                        slab.max_len - 1, uniform_pps, wp, wn, st)
-        else:      # one block of arguments instead of 34: the call is made for every layer of every step
-            rc = lib.trimkv_append_attend_step(slab.step_args(query.data_ptr(), out.data_ptr(), slab.pending[0], group, scale, slab.max_len - 1, uniform_pps, 0, wp, wn), st)
-        if rc:
-            _lib.check(rc, "trimkv_append_attend_uniform_gated" if gated else "trimkv_append_attend_uniform")
-        slab.pending = None
-        return out
-    if pieces is not None:   # ragged lengths: one launch over the (segment, piece) list, merged inside it
-        plist, npieces = pieces
-        ws = _workspace_zeroed(query.device, lib.trimkv_decode_attn_pieces_workspace(npieces, group), st)
-        most = bound if bound > 0 else slab.max_len
-        if gated:
-            rc = lib.trimkv_append_attend_pieces_gated(query.data_ptr(), out.data_ptr(), *slab.ptrs, plist.data_ptr(), npieces, nseg, slab.H, slab.cap, d, group, *slab.codes,
-                                                       *slab.pending[0], scale, most, ws.data_ptr(), ws.numel(), st)
+                                                        rows, count, wp, wn, st)
         else:
-            rc = lib.trimkv_append_attend_step(slab.step_args(query.data_ptr(), out.data_ptr(), slab.pending[0], group, scale, most, npieces, plist.data_ptr(),
-                                                              ws.data_ptr(), ws.numel()), st)
+            rc = lib.trimkv_append_attend_pieces_gated(query.data_ptr(), out.data_ptr(), *slab.ptrs, plist, count, nseg, slab.H, slab.cap, d, group, *slab.codes,
+                                                       *slab.pending[0], scale, rows, wp, wn, st)
         if rc:
-            _lib.check(rc, "trimkv_append_attend_pieces_gated" if gated else "trimkv_append_attend_pieces")
+            _lib.check(rc, "trimkv_append_attend_uniform_gated" if uniform_pps > 0 else "trimkv_append_attend_pieces_gated")
         slab.pending = None
         return out
+    out = _empty_out(query)
     max_len = bound if bound > 0 else slab.max_len
     ws_bytes = lib.trimkv_decode_attn_workspace(nseg, group, d, max_len, chunk)
     ws = _workspace(query.device, ws_bytes, st) if ws_bytes else None
@@ -354,19 +374,13 @@ def _dense_torch_attention(query, key, value, attention_mask, scale: float, caus
 def _decode_step(query: torch.Tensor, key: torch.Tensor, slab, scaling: Optional[float]) -> Optional[torch.Tensor]:
     """The usual decode step of a dense cache (one query row per sequence, the layer's append deferred to this call, nothing masked)
     without the general path's questions: the call costs the host about half.  None: not that case."""
-    B, Hq, Q, D = query.shape
-    H = slab.H
-    G = Hq // H
-    if (Q != 1 or G > _MAX_GROUP or Hq != G * H or B != slab.B or D != slab.D or slab.pending is None or slab.cu is not None or not query.is_cuda
-            or query.dtype != slab.k.dtype or key.data_ptr() != slab.ptrs[0] or key.shape[2] != slab.max_len):
+    G = _lib.step().fits(query, key, slab)
+    if not 0 < G <= _MAX_GROUP:
         return None
-    pps = _uniform_cut(B * H, slab.max_len)
+    pps = _uniform_cut(slab.nseg, slab.max_len)
     if pps > 1 and (G not in _DENSE_PIECES_GROUPS or G not in _FUSED_PIECES_GROUPS):
         return None
-    q2 = query.reshape(B * Hq, D)
-    if not q2.is_contiguous():
-        q2 = q2.contiguous()
-    return append_attend(slab, q2, G, D ** -0.5 if scaling is None else scaling, uniform_pps=pps).view(B, 1, Hq, D)
+    return append_attend(slab, query if query.is_contiguous() else query.contiguous(), G, slab.D ** -0.5 if scaling is None else scaling, uniform_pps=pps)
 
 
 def dense_attention_forward(module: nn.Module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -408,13 +422,10 @@ def dense_attention_forward(module: nn.Module, query: torch.Tensor, key: torch.T
     slab = _take_pending(flash_attn_kwargs, query, key, G, Q == 1 and attention_mask is None and window is None and plain,
                          True if pps > 1 or dev_pieces is not None else None)
     if slab is not None:
-        q2 = query.reshape(B * Hq, D)
-        if not q2.is_contiguous():
-            q2 = q2.contiguous()
         if slab.cu is not None:
             pps = 0
-        return append_attend(slab, q2, G, scale, chunk=dense_chunk, uniform_pps=pps, pieces=dev_pieces,
-                             bound=slab.cap if on_device else 0).view(B, 1, Hq, D), None, None
+        return append_attend(slab, query if query.is_contiguous() else query.contiguous(), G, scale, chunk=dense_chunk, uniform_pps=pps, pieces=dev_pieces,
+                             bound=slab.cap if on_device else 0), None, None
     kernel_ok = plain and query.dtype in (torch.bfloat16, torch.float16) and D in (64, 96, 128)
     seg_first = None
     if kernel_ok and Q == 1:
@@ -502,11 +513,8 @@ def _ragged_common(query, key, value, flash_attn_kwargs, batch_size, num_kv_head
     G = Hq // num_kv_heads
     slab = _take_pending(kw, query, key, G, Q == 1 and kw.get("seg_start") is not None and not dropout_p, kw.get("pieces"))
     if slab is not None:
-        q2 = query.reshape(B * Hq, D)
-        if not q2.is_contiguous():
-            q2 = q2.contiguous()
-        out = append_attend(slab, q2, G, D ** -0.5, chunk=kw.get("chunk", 0), seg_order=kw.get("seg_order"), pieces=kw.get("pieces"))
-        return out.view(B, 1, Hq, D), None, None
+        return append_attend(slab, query if query.is_contiguous() else query.contiguous(), G, D ** -0.5, chunk=kw.get("chunk", 0), seg_order=kw.get("seg_order"),
+                             pieces=kw.get("pieces")), None, None
     seg_start = kw.get("seg_start")
     if seg_start is None:  # packed rows, as the reference stores them
         seg_start = cu[:-1]

@@ -2,7 +2,9 @@
 libtrimkv_hybrid.so (what the hybrid decoders share, windowed attention), libtrimkv_mlstm.so and libtrimkv_moe.so (their
 recurrent layers and routed experts).
 
-Usage: ``python -m trimkv_amd.build [--changed] [hip|hybrid|mlstm|moe ...]`` (hipcc cross-compiles without a GPU; ``--changed``
+and the extension module _step.so, the host side of decode steps (C++ against Python's and torch's headers).
+
+Usage: ``python -m trimkv_amd.build [--changed] [hip|hybrid|mlstm|moe|step ...]`` (hipcc cross-compiles without a GPU; ``--changed``
 recompiles only the sources whose object file is older than its inputs; no name: all of them).
 """
 from __future__ import annotations
@@ -10,12 +12,14 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB_PATH = os.path.join(HERE, "libtrimkv_hip.so")
+STEP_PATH = os.path.join(HERE, "_step.so")
 SOURCES = ["api.hip", "append.hip", "evict.hip", "attn_decode.hip", "attn_decode_append.hip", "attn_decode_pieces.hip", "attn_decode_append_pieces.hip", "attn_decode_append_gated.hip", "attn_decode_append_pieces_gated.hip", "pieces_plan.hip", "attn_prefill.hip", "gate.hip", "stream_probe.hip", "decoder_ops.hip", "linear_rows.hip", "linear_tiles.hip"]
 HYBRID_SOURCES = ["hybrid_ops.hip", "window_attn.hip", "window_decode.hip", "linear_rows.hip", "linear_tiles.hip"]
 LIBRARIES = {"hip": (LIB_PATH, SOURCES), "hybrid": (os.path.join(HERE, "libtrimkv_hybrid.so"), HYBRID_SOURCES),
@@ -49,9 +53,30 @@ def _stale(src: str, obj: str) -> bool:
     return any(os.path.getmtime(d) > os.path.getmtime(obj) for d in deps)
 
 
-def build(verbose: bool = True, only_changed: bool = False, libraries=tuple(LIBRARIES)) -> str:
+def _build_step(verbose: bool, only_changed: bool) -> None:
+    src = os.path.join(CSRC, "step.cpp")
+    if only_changed and not _stale("step.cpp", STEP_PATH):
+        return
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    part = "%s.%d" % (STEP_PATH, os.getpid())
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + INCLUDE, "-I" + inc,
+          "-I" + os.path.join(inc, "torch", "csrc", "api", "include"), "-I" + sysconfig.get_paths()["include"], "-o", part, src,
+          "-L" + lib, "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath," + lib])
+    os.replace(part, STEP_PATH)
+    if verbose:
+        print("built", STEP_PATH)
+
+
+def build(verbose: bool = True, only_changed: bool = False, libraries=(*LIBRARIES, "step")) -> str:
     """Compile every source of the named libraries (or, with ``only_changed``, the ones whose object is older than its
     inputs) and link them."""
+    if "step" in libraries:
+        _build_step(verbose, only_changed)
+        libraries = tuple(n for n in libraries if n != "step")
+        if not libraries:
+            return STEP_PATH
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
@@ -81,12 +106,12 @@ def build(verbose: bool = True, only_changed: bool = False, libraries=tuple(LIBR
 
 def ensure(libraries) -> None:
     """Build those of the named libraries that are not there (a fresh checkout)."""
-    missing = tuple(n for n in libraries if not os.path.exists(LIBRARIES[n][0]))
+    missing = tuple(n for n in libraries if not os.path.exists(STEP_PATH if n == "step" else LIBRARIES[n][0]))
     if missing:
         build(verbose=False, only_changed=True, libraries=missing)
 
 
 if __name__ == "__main__":
     names = [a for a in sys.argv[1:] if not a.startswith("--")]
-    build(only_changed="--changed" in sys.argv[1:], libraries=tuple(names) or tuple(LIBRARIES))
+    build(only_changed="--changed" in sys.argv[1:], libraries=tuple(names) or (*LIBRARIES, "step"))
     sys.exit(0)

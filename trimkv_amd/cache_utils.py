@@ -17,7 +17,6 @@ There is no CPU path: tensors must live on the GPU and the library must be built
 """
 from __future__ import annotations
 
-import ctypes
 import math
 import struct
 from typing import Any, Dict, Iterable, List, Optional, Tuple
@@ -135,7 +134,7 @@ class _Slab:
     """Device storage of one layer."""
 
     __slots__ = ("k", "v", "lb", "pos", "seg_len", "cu", "B", "H", "D", "cap", "lens", "max_len", "k4", "v4", "lb3", "pos3", "ptrs", "order",
-                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host", "row_shape", "strides", "step",
+                 "pending", "codes", "total", "pieces", "pieces_total", "pieces_age", "pieces_buf", "order_host", "row_shape", "step",
                  "seg_start")
 
     def __init__(self, B, H, D, cap, kv_dtype, lb_dtype, device, ragged: bool):
@@ -167,33 +166,20 @@ class _Slab:
                      None if self.cu is None else self.cu.data_ptr())
         self.codes = (_lib.dtype_code(self.k.dtype), _lib.dtype_code(self.lb.dtype))
         self.row_shape = (B, H, 1, D)
-        self.strides = (self.k4.stride(), self.lb3.stride())
         self.seg_start = None
-        self.step = None
+        k, v, lb, pos, seg_len, cu = self.ptrs
+        self.step = bytearray(self._STEP_FIXED.pack(k, v, lb, pos, seg_len, cu or 0, B * H, H, cap, D, *self.codes)) + bytearray(self._STEP.size)
 
-    # struct trimkv_append_step: what stays while the storage does not move, then what a step brings
+    # struct trimkv_append_step: what stays while the storage does not move, then what a step brings (filled in by native code)
     _STEP_FIXED, _STEP = struct.Struct("12q"), struct.Struct("13qd5q")
 
-    def step_args(self, q: int, out: int, new: tuple, group: int, scale: float, rows: int, count: int, pieces: int, ws: int, ws_bytes: int) -> int:
-        """Address of a filled-in ``trimkv_append_step`` of this layer (valid until the next call)."""
-        buf = self.step
-        if buf is None:
-            buf = self.step = ctypes.create_string_buffer(self._STEP_FIXED.size + self._STEP.size)
-            k, v, lb, pos, seg_len, cu = self.ptrs
-            self._STEP_FIXED.pack_into(buf, 0, k, v, lb, pos, seg_len, cu or 0, self.nseg, self.H, self.cap, self.D, *self.codes)
-        self._STEP.pack_into(buf, self._STEP_FIXED.size, q, out, *new, group, scale, rows, count, pieces, ws, ws_bytes)
-        return ctypes.addressof(buf)
-
     def rows(self, n: int):
-        """The first ``n`` rows of K, V, log beta and positions as [B,Hkv,n,...] views, new objects for every caller (as_strided:
-        a decode step makes four per layer, 0.67 us each against 1.03 by narrow)."""
-        B, H, (s4, s3) = self.B, self.H, self.strides
-        four, three = (B, H, n, self.D), (B, H, n)
-        return self.k.as_strided(four, s4), self.v.as_strided(four, s4), self.lb.as_strided(three, s3), self.pos.as_strided(three, s3)
+        """The first ``n`` rows of K, V, log beta and positions as [B,Hkv,n,...] views, new objects for every caller."""
+        return _lib.step().views(self, n)
 
     def flat(self):
         """K, V, log beta and positions with the segments one behind the other, [nseg * cap, ...]."""
-        return self.k.view(-1, self.D), self.v.view(-1, self.D), self.lb.view(-1, 1), self.pos.view(-1, 1)
+        return _lib.step().views(self, -1)
 
     @property
     def nseg(self) -> int:
@@ -273,6 +259,9 @@ class _SlabBacked(_CacheBase):
         (``_flush``).  Returns False when this update cannot be deferred (the ordinary append runs then)."""
         if slab.pending is not None:
             self._flush(slab)
+        if _lib.step().defer(slab, k, v, lb, pos):
+            return True
+        # what native code leaves: an unfinished log beta, a slab that has to grow, and all that cannot be deferred
         lazy = isinstance(lb, LazyLogBeta)
         if not k.is_cuda or not (lazy or lb.is_cuda):
             return False
