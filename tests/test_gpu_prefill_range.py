@@ -1,0 +1,81 @@
+"""GPU tests of the chunk-prefill attention where scores outgrow the exponent reference that a row began with: within what bf16's exponents take, beyond
+it (the workgroup's second, careful way), gradually (the reference moves by the row sums) and in fp16, against the fp32 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.attn_ref import ragged_attention
+from tests.gpu_util import DEV, attn_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _heights(how, n):
+    """Height of every key along the direction that all queries share; 1 is about 65 powers of two of a score."""
+    at = torch.arange(n, dtype=torch.float32)
+    return {"jump": (at >= 700).float() * 6, "small jump": (at >= 700).float() * 0.8, "climb": at * (6 / n), "steep": ((at - 300) / 400).clamp(0, 1) * 6, "fall": 6 - at * (6 / n),
+            "peak": (at == 1000).float() * 6, "last": (at == n - 140).float() * 6, "steps": (at / 300).floor()}[how]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("G,D,Q", [(1, 128, 300), (5, 64, 130)])
+@pytest.mark.parametrize("how", ["jump", "small jump", "climb", "steep", "fall", "peak", "last", "steps"])
+def test_scores_that_outgrow_their_reference(how, G, D, Q, dtype):
+    from trimkv_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(G + D)
+    B, H, lens = 1, 2, [1500, 1100]
+    N, longest = sum(lens), max(lens)
+    base = torch.randn(D, generator=gen)
+    base = base * (D ** 0.5 / base.norm())
+    k = (torch.cat([_heights(how, n) for n in lens])[:, None] * base + 0.3 * torch.randn(N, D, generator=gen)).to(dtype)
+    v = torch.randn(N, D, generator=gen).to(dtype)
+    q = (45.0 / D ** 0.5 * base + 0.3 * torch.randn(B, H * G, Q, D, generator=gen)).to(dtype)      # 45 nats, 65 powers of two
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32)
+    # Q * scale is rounded once: the oracle takes it as the kernel does, so that large scores agree
+    c = D ** -0.5 * 1.4426950408889634
+    rounded = (q.float() * c).to(dtype).double() / c
+    s = torch.einsum("bhgqd,bhnd->bhgqn", rounded.view(B, H, G, Q, D), torch.stack([torch.cat([x.double(), torch.zeros(longest - x.shape[0], D, dtype=torch.float64)]) for x in k.split(lens)])[None]) * D ** -0.5
+    ln = torch.tensor(lens)
+    seen = torch.arange(longest)[None, None, :] <= (ln[:, None, None] - Q + torch.arange(Q)[None, :, None])
+    p = torch.softmax(s.masked_fill(~seen[None, :, None], -float("inf")), -1)
+    want = torch.einsum("bhgqn,bhnd->bqhgd", p, torch.stack([torch.cat([x.double(), torch.zeros(longest - x.shape[0], D, dtype=torch.float64)]) for x in v.split(lens)])[None]).reshape(B, Q, H * G, D)
+    qd, kd, vd, start, lend = q.to(DEV), k.to(DEV), v.to(DEV), cu[:-1].contiguous().to(DEV), ln.int().to(DEV)
+    stream = _lib.current_stream(qd.device)
+    # P and the row sums rounded to 16 bits, one rounding of the output, as in the divided launches' bound: 6 u max|v|
+    bound = 6 * float(v.abs().max()) * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+
+    def call(name, *more):
+        out = torch.full((B, Q, H * G, D), float("nan"), dtype=dtype, device=DEV)
+        _lib.check(getattr(lib, name)(qd.data_ptr(), *qd.stride()[:3], out.data_ptr(), kd.data_ptr(), vd.data_ptr(), lend.data_ptr(), start.data_ptr(),
+                                      B, H, G, Q, longest, D, _lib.dtype_code(dtype), D ** -0.5, longest, *more, stream), name)
+        return out.cpu()
+
+    outs = {"whole": call("trimkv_prefill_attn")}
+    for tiles in (1, 5):
+        need = lib.trimkv_prefill_split_workspace(B, H, G, Q, longest, tiles)
+        work = torch.full((need // 4,), float("nan"), device=DEV)
+        outs[f"split {tiles}"] = call("trimkv_prefill_attn_split", tiles, work.data_ptr(), need)
+    need = lib.trimkv_prefill_shares_workspace(B, H, G, Q)
+    work = torch.full((need // 4,), float("nan"), device=DEV)
+    outs["shares"] = call("trimkv_prefill_attn_shares", work.data_ptr(), need)
+    for name, out in outs.items():
+        assert out.isfinite().all(), name
+        assert float((out.double() - want).abs().max()) <= bound, (name, float((out.double() - want).abs().max()), bound)
+
+
+@pytest.mark.parametrize("what,value", [("k", float("nan")), ("v", float("inf")), ("q", float("inf"))])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(what, value):
+    from trimkv_amd.attn.hip_attn import prefill_attention
+    gen = torch.Generator().manual_seed(1)
+    H, G, Q, n = 2, 2, 200, 900
+    q, k, v = (torch.randn(1, H * G, Q, 128, generator=gen).to(torch.bfloat16), *(torch.randn(H * n, 128, generator=gen).to(torch.bfloat16) for _ in range(2)))
+    clean = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), 1, H, G, None, None, n, n, 128 ** -0.5).cpu()
+    {"k": k, "v": v}.get(what, q.view(-1, 128))[5, 7] = value      # row 5 of the first segment, seen by all queries of its heads; or the sixth query of the first head
+    out = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), 1, H, G, None, None, n, n, 128 ** -0.5).cpu()
+    assert torch.equal(out[:, :, G:], clean[:, :, G:])             # the second segment
+    hit = out[0, 5, 0] if what == "q" else out[0, :, :G, 7] if what == "v" else out[0, :, :G]
+    assert not hit.isfinite().any()
+    if what == "v":
+        rest = [d for d in range(128) if d != 7]
+        assert out[0, :, :G][..., rest].isfinite().all()

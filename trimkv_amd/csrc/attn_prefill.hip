@@ -7,16 +7,16 @@
 // plus the chunk's own tokens <= t, i.e. keys j <= n - Q_LEN + t.
 //
 // Two kernels share the formulation below.  prefill_attn_kernel (chunks of 64 queries and more) gives
-// a wavefront 32 queries and uses v_mfma_f32_32x32x16_bf16 on 64-key tiles that LDS-direct loads
+// a wavefront 32 queries, two groups of MFMA columns, on 64-key tiles that LDS-direct loads
 // rotate through four LDS buffers; prefill_small_kernel (short chunks) gives a wavefront
-// 16 queries and uses v_mfma_f32_16x16x32_bf16 on 32-key tiles.
+// 16 queries on 32-key tiles.  Both use v_mfma_f32_16x16x32_bf16.
 //
 // A workgroup owns BT consecutive query times of one segment for all G query heads of its KV head,
 // one wavefront per (head, 16 or 32 times), so a K/V tile staged in LDS is shared by the whole group.
 // Per tile a wavefront computes
 //     S^T[key][query] = K . Q^T           (A = K rows from LDS, B = Q rows held in registers)
 //     O^T[d][query]  += V^T . P^T         (A = V columns gathered from LDS, B = P^T)
-// Both products put the query on the MFMA column index, which is the lane index modulo 16 (32): every
+// Both products put the query on the MFMA column index, which is the lane index modulo 16: every
 // per-query quantity (running max, sum, rescale factor) lives in the lane that needs it, and the
 // probabilities a lane holds after the first product are exactly the keys its B operand of the
 // second product wants -- P never crosses lanes.  V is row-major in memory, so its A operand
@@ -70,12 +70,6 @@ template <bool F16>
 __device__ __forceinline__ pf_f32x4 mfma_16x16x32(pf_bf16x8 a, pf_bf16x8 b, pf_f32x4 c) {
     if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pf_f16x8, a), __builtin_bit_cast(pf_f16x8, b), c, 0, 0, 0);
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-typedef float pf_f32x16_fwd __attribute__((ext_vector_type(16)));
-template <bool F16>
-__device__ __forceinline__ pf_f32x16_fwd mfma_32x32x16(pf_bf16x8 a, pf_bf16x8 b, pf_f32x16_fwd c) {
-    if constexpr (F16) return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pf_f16x8, a), __builtin_bit_cast(pf_f16x8, b), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
     pf_f32x2 f = {lo, hi};
@@ -313,14 +307,24 @@ __global__ __launch_bounds__(256) void prefill_small_merge_kernel(PrefillArgs a)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Large-chunk kernel: 32 queries per wavefront, 64-key tiles, v_mfma_f32_32x32x16_bf16.
+// Large-chunk kernel: 32 queries per wavefront, 64-key tiles, v_mfma_f32_16x16x32_bf16.
 //
-// MFMA 32x32x16 register layout (lane l, half hl = l / 32):
-//   A (32 x 16): row l % 32, k = 8 * hl + 0..7          B (16 x 32): column l % 32, k = 8 * hl + 0..7
-//   C (32 x 32): column l % 32, register v holds row 8 * (v / 4) + 4 * hl + v % 4
-// S^T = K . Q^T per 32-key block: after it a lane holds, for its query, keys 8c + 4hl + i (c, i in 0..3).
-// The second product consumes 16 keys per MFMA; step st takes from lane half hl the keys of c = 2st and
-// 2st + 1, i.e. registers v = 8st .. 8st + 7 in order: keys 16 st + 4 hl + 0..3 and 16 st + 8 + 4 hl + 0..3.
+// MFMA 16x16x32 register layout (lane l, row group ig = l / 16):
+//   A (16 x 32): row l % 16, k = 8 * ig + 0..7          B (32 x 16): column l % 16, k = 8 * ig + 0..7
+//   C (16 x 16): column l % 16, register v holds row 4 * ig + v
+// S^T = K . Q^T per 32-key block, two groups of 16 keys by two of 16 queries: after it a lane holds, for its query of either group,
+// keys 4 ig + 0..3 and 16 + 4 ig + 0..3.  The second product consumes 32 keys per MFMA; its k index 8 ig + e stands for key 4 ig + e (e < 4) or
+// 16 + 4 ig + e - 4, so that a lane's probabilities are its B operand.
+//
+// What bounds it is the clock that the chip holds under matrix load, and beside it the issue of vector instructions: matrix cores and vector ALU of a SIMD
+// take turns when two wavefronts want both.  16x16x32 products cost less of the clock than 32x32x16 (registers only, random operands: 2.06 against 1.80 PFLOP/s at
+// 2.02 and 1.76 GHz), but leave less room beside them (with two and four vector instructions per 32 cycles of product 1.85 | 1.66 and 1.64 | 1.55).  Hence
+// the parts of a block in which one wavefront of a SIMD only multiplies while the other does the rest (`block` below), and in bf16 no row
+// maxima (ATTEND_SUMS): 16 exponentials, 8 packs and 8 row sums per 32 products are left.
+// 16 segments of 12288 keys, 4096 queries of 5 heads: 1.17 PFLOP/s with 32x32x16, exponentials between the products and matrix pipes busy
+// 73 % at 1.58 GHz; the same with 16x16x32 1.16, 59 % at 1.88; in two parts 1.22; without maxima 1.28 PFLOP/s, 69 % at 1.77.  Row sums on the matrix cores as well
+// (32 more cycles of them, 8 vector instructions less): +1 %, and -1 % where shares are equal; packs and row sums in the part that multiplies:
+// 0.97; V read in the part that does not: 1.19.
 //
 // K and V tiles are staged by LDS-direct loads (global_load_lds_dwordx4): a tile never passes through registers and
 // no VALU instruction takes part in staging.
@@ -329,7 +333,7 @@ __global__ __launch_bounds__(256) void prefill_small_merge_kernel(PrefillArgs a)
 // lane fetches is free, and that is where the bank swizzle comes from:
 //   K: piece c of row r sits at position c ^ (r & 15): the 16 rows a b128 fragment read touches (one piece index,
 //      consecutive rows) fall on all 64 banks.
-//   V: the 32-byte pair p of row r sits at pair position p ^ (2 (r & 3)).  The A operand of O^T += V^T.P^T (8 keys at
+//   V: the 32-byte pair p of row r sits at pair position p ^ pf2_v_swizzle(r).  The A operand of O^T += V^T.P^T (8 keys at
 //      one d per lane) is read with two ds_read_b64_tr_b16: within 16 lanes, lane i supplies 8 bytes (4 d of one key,
 //      key = base + i / 4, d = d0 + 4 (i % 4) ..) and receives the four keys base .. base + 3 at d = d0 + i.
 // The compiler does not see the LDS-direct loads (inline assembly: the builtin would make it wait for all of them before
@@ -345,13 +349,14 @@ constexpr int PF2_NBUF = 4;                         // tiles in rotation: two be
 constexpr int PF2_TILE = PF2_BN * PF_D * 2;         // bytes of one K (or V) tile: rows of 256 bytes
 constexpr int PF2_VBASE = PF2_NBUF * PF2_TILE;      // 65536: K tiles below, V tiles above
 constexpr int PF2_LDS = 2 * PF2_NBUF * PF2_TILE;    // 131072
-constexpr int PF2_PD = 3;                           // LDS operand reads in flight ahead of the MFMA that consumes them
 constexpr float PF2_LAZY = 6.0f;                    // O is rescaled only when a row maximum grows by more than 2^6
 
 // A workgroup is always 8 wavefronts (two per SIMD, 256 registers each) and owns 256 / G consecutive query times
 // for all G heads: MFMA column c of wavefront w is row r = 32w + c of the workgroup, time r / G, head r % G.
 // Every per-query quantity is per lane, so a wavefront may mix heads freely; time-major rows keep the
 // spread of a wavefront's causal limits small.
+constexpr float PF2_MOST = 1.0e12f;                 // without maxima: 2^40, the row sum from which on O is rescaled
+
 constexpr int PF2_WAVES = 8;
 constexpr int PF2_THREADS = PF2_WAVES * 64;
 static_assert(PF2_THREADS * 2 * 16 == PF2_TILE, "a thread stages two 16-byte pieces of K and two of V per tile");
@@ -362,6 +367,9 @@ __device__ __forceinline__ void pf2_load_to_lds(const char* sbase, uint32_t voff
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
                  : "=&s"(saved) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
+
+// V: where the 32-byte pairs of row r lie (pair p at p ^ this): the rows that 32 lanes of a transposing read touch fall on different banks
+__device__ __forceinline__ int pf2_v_swizzle(int r) { return 2 * (r & 3) + ((r >> 2) & 1); }
 
 // tiles of keys that the last query of a query tile sees
 __device__ __forceinline__ int tiles_seen(const PrefillArgs& a, int seg, int tile) {
@@ -380,8 +388,15 @@ constexpr int PF2_LEAST = 4;                        // units of a share at least
 
 // One query tile against `count` tiles of keys from tile t_first on (PART; else against all of them).  Where that is not all that the
 // query tile sees, unnormalised outputs with their exponent references and row sums (fp32) are left in `slot` for a merge kernel.
-template <bool F16, bool PART, bool LOOP>
-__device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot) {
+//
+// HOW: what keeps the exponentials in range.  ATTEND_MAXIMA (fp16): the exponent reference of a row stays within 2^PF2_LAZY of its largest score.  ATTEND_SUMS (bf16,
+// whose P has fp32's exponents): once set it moves only where the row's sum has grown beyond PF2_MOST, which takes no maxima; a score that exceeds the
+// reference by 2^7 within a block overflows then, and whatever is not finite at the end (an input that is not among it) sets *again (0 before), for
+// the caller to have it done again with ATTEND_CAREFULLY over what it has written: maxima as in fp16, one block after the other.
+enum { ATTEND_MAXIMA, ATTEND_SUMS, ATTEND_CAREFULLY };
+template <bool F16, bool PART, bool LOOP, int HOW>
+__device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot, PF_LDS3 int* again) {
+    constexpr bool MAXIMA = HOW != ATTEND_SUMS;
     extern __shared__ __attribute__((aligned(16))) char pf2_lds[];
     PF_LDS3 char* const lds3 = (PF_LDS3 char*)pf2_lds;
     const uint32_t lds0 = (uint32_t)(uintptr_t)lds3;
@@ -389,46 +404,47 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
     int n = a.seg_len ? a.seg_len[seg] : a.max_len;
     n = max(0, min(n, a.max_len));
     int tid = threadIdx.x;
-    if (LOOP) asm volatile("" : "+v"(tid));                   // nothing of a query tile is worth a register during the one before it
+    asm volatile("" : "+v"(tid));                             // nothing of a query tile is worth a register during the one before it
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform by construction; saying so keeps what derives from it in scalar registers
-    const int j = lane & 31, hl = lane >> 5;    // MFMA column (query) and lane half
+    const int j = lane & 15, ig = lane >> 4;    // MFMA column (query, of either group of 16) and row group
     const int G = a.group, Q = a.q_len;
     const int BT = (PF2_WAVES * 32) / G;        // query times per workgroup; rows BT * G .. 255 are padding
     const int t_wg0 = tile * BT;
-    const int r = w * 32 + j;
-    const int g = r % G;
-    const int t_q = t_wg0 + r / G;              // this lane's query time
     const int t_w_first = t_wg0 + (w * 32) / G;
     const int64_t row0 = a.seg_start ? (int64_t)a.seg_start[seg] : (int64_t)seg * a.cap;
 
     // The rows of Q are asked for in front of the first keys and turned into fragments behind them: one memory round trip for both.
-    pf_u32x4 qraw[8];
-    {
-        const uint16_t* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(h * G + g) * a.q_sh + (int64_t)min(t_q, Q - 1) * a.q_st;
+    pf_u32x4 qraw[2][4];
+    int vis_j[2];                               // last key that this lane's query of either group sees
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qraw[ks] = *(const pf_u32x4*)(qrow + min(ks * 16 + hl * 8, a.hd - 8));
+    for (int qg = 0; qg < 2; ++qg) {
+        const int r = w * 32 + qg * 16 + j, t_q = t_wg0 + r / G;
+        vis_j[qg] = n - Q + t_q;
+        const uint16_t* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(h * G + r % G) * a.q_sh + (int64_t)min(t_q, Q - 1) * a.q_st;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) qraw[qg][ks] = *(const pf_u32x4*)(qrow + min(ks * 32 + ig * 8, a.hd - 8));
     }
 
-    pf_f32x16 o[4];   // O^T: o[db][v] = d (db * 32 + 8 * (v / 4) + 4 * hl + v % 4) of query j
+    // O^T: o[dg / 2][8 (dg % 2) + 4 qg + v] = d (16 dg + 4 ig + v) of query 16 qg + j.  Blocks of 16 and not of 4: the compiler gives a block of 4 other
+    // registers with every MFMA and copies all of them back where the rescaling branch joins, a part of a larger block stays where it is.
+    pf_f32x16 o[4];
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[db][v] = 0.0f;
-    // Exponent reference (log2 units) and this lane's share of the row sum.  The score MFMAs start from -m_ref in their
-    // accumulator (negm, all 16 registers alike: a lane is one query), so what they deliver is already s - m_ref.  The
+    auto o_of = [&](int dg, int qg, int v) __attribute__((always_inline)) { return o[dg >> 1][8 * (dg & 1) + 4 * qg + v]; };
+    // Exponent references (log2 units) and this lane's shares of the row sums.  The score MFMAs start from -m_ref in their
+    // accumulator (negm, all 4 registers alike: a lane is one query), so what they deliver is already s - m_ref.  The
     // reference starts at 0 and is moved onto the row maximum by the first block.  A query that sees no key at all
     // (segment shorter than the chunk) keeps reference 0: its masked scores give exp2(-huge) = 0, never exp2(0).
-    float m_ref = 0.0f, l_run = 0.0f;
-    pf_f32x16 negm;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) negm[v] = 0.0f;
+    float m_ref[2] = {0.0f, 0.0f}, l_run[2] = {0.0f, 0.0f};
+    pf_f32x4 negm[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
 
     const int t_last = min(Q - 1, t_wg0 + BT - 1);
     const int k_end = max(0, min(n, n - Q + t_last + 1));     // keys the query tile sees
     const int all_tiles = (k_end + PF2_BN - 1) / PF2_BN;
-    const int vis_j = n - Q + t_q;                            // last key this lane's query sees
-    const int vis_lo = n - Q + t_w_first;                     // ... the wavefront's first query
+    const int vis_lo = n - Q + t_w_first;                     // last key that the wavefront's first query sees
     const int last_row = max(n - 1, 0);
 
     // ---- staging: global -> LDS ----
@@ -440,7 +456,7 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
     const char* vseg = a.v + row0 * (int64_t)row_bytes;
     const int st_row = tid >> 4, st_pos = tid & 15;
     const uint32_t st_kcol = min((uint32_t)(st_pos ^ (st_row & 15)) * 16u, row_bytes - 16u);
-    const uint32_t st_vcol = min((uint32_t)((((st_pos >> 1) ^ (2 * (st_row & 3))) << 1) | (st_pos & 1)) * 16u, row_bytes - 16u);
+    const uint32_t st_vcol = min((uint32_t)((((st_pos >> 1) ^ pf2_v_swizzle(st_row)) << 1) | (st_pos & 1)) * 16u, row_bytes - 16u);
     const uint32_t st_koff = (uint32_t)st_row * row_bytes + st_kcol;     // offsets inside a tile whose 64 rows all exist
     const uint32_t st_voff = (uint32_t)st_row * row_bytes + st_vcol;
     auto request_tile = [&](int tt, int buf) __attribute__((always_inline)) {
@@ -464,248 +480,292 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
     };
 
     const int ntiles = PART ? min(all_tiles - t_first, count) : all_tiles;
-    if (ntiles > 0) {
+    if (ntiles > 0 && HOW != ATTEND_CAREFULLY) {
         request_tile(0, 0);
         request_tile(1, 1);
     }
-    // Q fragments (B operand of S^T): 8 d of step ks at d = ks * 16 + hl * 8, multiplied by scale * log2(e) and rounded back
+    // Q fragments (B operand of S^T): 8 d of step ks at d = ks * 32 + ig * 8, multiplied by scale * log2(e) and rounded back
     // to 16 bits once, here: the score MFMAs then deliver exponents of two directly and the loop never multiplies a score.
-    pf_bf16x8 qf[8];
+    pf_bf16x8 qf[2][4];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-        pf_u32x4 sc;
+    for (int qg = 0; qg < 2; ++qg)
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            float lo, hi;
-            if (F16) { lo = f16_bits_to_f32((uint16_t)(qraw[ks][x] & 0xffffu)); hi = f16_bits_to_f32((uint16_t)(qraw[ks][x] >> 16)); }
-            else { lo = __uint_as_float(qraw[ks][x] << 16); hi = __uint_as_float(qraw[ks][x] & 0xffff0000u); }
-            sc[x] = pack_kv<F16>(lo * a.scale_log2, hi * a.scale_log2);
+        for (int ks = 0; ks < 4; ++ks) {
+            pf_u32x4 sc;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const uint32_t raw = qraw[qg][ks][x];
+                float lo, hi;
+                if (F16) { lo = f16_bits_to_f32((uint16_t)(raw & 0xffffu)); hi = f16_bits_to_f32((uint16_t)(raw >> 16)); }
+                else { lo = __uint_as_float(raw << 16); hi = __uint_as_float(raw & 0xffff0000u); }
+                sc[x] = pack_kv<F16>(lo * a.scale_log2, hi * a.scale_log2);
+            }
+            if (ks * 32 + ig * 8 >= a.hd) sc = pf_u32x4{0u, 0u, 0u, 0u};   // padded features: whatever K holds there counts for nothing
+            qf[qg][ks] = __builtin_bit_cast(pf_bf16x8, sc);
         }
-        if (ks * 16 + hl * 8 >= a.hd) sc = pf_u32x4{0u, 0u, 0u, 0u};   // padded features: whatever K holds there counts for nothing
-        qf[ks] = __builtin_bit_cast(pf_bf16x8, sc);
-    }
 
-    // per-lane LDS read offsets; the buffer, the 32-key block and the step are immediates on top of them
-    PF_LDS3 char* k_ptr[8];
-    PF_LDS3 char* v_ptr[4];
+    // per-lane LDS read offsets; the buffer, the 32-key block, the key group and the step are immediates on top of them
+    PF_LDS3 char* k_ptr[4];
+    PF_LDS3 char* v_ptr[8];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-        k_ptr[ks] = lds3 + (j * 256 + (((2 * ks + hl) ^ (j & 15)) << 4));
+    for (int ks = 0; ks < 4; ++ks) {
+        k_ptr[ks] = lds3 + (j * 256 + (((4 * ks + ig) ^ j) << 4));
         asm volatile("" : "+v"(k_ptr[ks]));          // a value in a register from here on, not an expression to recompute in the loop
     }
     {
-        const int i = lane & 15, jhalf = (lane >> 4) & 1;
-        const int kx = 4 * hl + (i >> 2);            // key (within its group of 8) this lane supplies to the transposing read
+        const int kx = 4 * ig + (j >> 2);            // key (within its group of 16) this lane supplies to the transposing read
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
-            v_ptr[db] = lds3 + (PF2_VBASE + kx * 256 + (((2 * db + jhalf) ^ (2 * (kx & 3))) << 5) + (i & 3) * 8);
-            asm volatile("" : "+v"(v_ptr[db]));
+        for (int dg = 0; dg < 8; ++dg) {
+            v_ptr[dg] = lds3 + (PF2_VBASE + kx * 256 + ((dg ^ pf2_v_swizzle(kx)) << 5) + (j & 3) * 8);
+            asm volatile("" : "+v"(v_ptr[dg]));
         }
     }
-    auto k_frag = [&](int imm, int ks) __attribute__((always_inline)) {
-        return *(const PF_LDS3 pf_bf16x8*)(k_ptr[ks] + imm);
+    // fragment m of a block's keys: step m / 2, keys 16 (m % 2) ..
+    auto k_frag = [&](int imm, int m) __attribute__((always_inline)) {
+        return *(const PF_LDS3 pf_bf16x8*)(k_ptr[m >> 1] + imm + (m & 1) * 16 * 256);
     };
-    auto v_frag = [&](int imm, int st, int db) __attribute__((always_inline)) {
-        PF_LDS3 char* p = v_ptr[db] + imm + st * 16 * 256;
-        const pf_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PF_LDS3 pf_s16x4*)p);                // keys 16 st + 4 hl + 0..3
-        const pf_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PF_LDS3 pf_s16x4*)(p + 8 * 256));    // ... + 8
+    auto v_frag = [&](int imm, int dg) __attribute__((always_inline)) {
+        PF_LDS3 char* p = v_ptr[dg] + imm;
+        const pf_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PF_LDS3 pf_s16x4*)p);                 // keys 4 ig + 0..3
+        const pf_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((PF_LDS3 pf_s16x4*)(p + 16 * 256));    // ... + 16
         return __builtin_bit_cast(pf_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
+    struct Scores { pf_f32x4 g[2][2]; };             // g[kg][qg][v]: key 16 kg + 4 ig + v of the block, query 16 qg + j
+    struct Pair { float x[2]; };                     // of the lane's two queries
 
     // Mask (diagonal blocks only), row maximum, and the lazy move of the exponent reference: O and l are
     // rescaled only when some row of the wavefront outgrows its reference by 2^PF2_LAZY.  FIRST: the wavefront's first
     // block puts the reference on the row maximum wherever it lies (O and l are still zero: nothing to rescale).
     // tmax: the maximum of s before masking, as the step computed it under its P.V MFMAs (ignored by FIRST).
-    auto max16 = [&](const pf_f32x16& s) __attribute__((always_inline)) {
-        float t = s[0];
+    auto max8 = [&](const Scores& s, int qg) __attribute__((always_inline)) {
+        float t = s.g[0][qg][0];
 #pragma unroll
-        for (int v = 1; v < 16; ++v) t = __builtin_fmaxf(t, s[v]);
+        for (int v = 1; v < 8; ++v) t = __builtin_fmaxf(t, s.g[v >> 2][qg][v & 3]);
         return t;
     };
-    auto prepare = [&](pf_f32x16& s, int blk, float tmax, auto first_c) __attribute__((always_inline)) {
-        constexpr bool FIRST = decltype(first_c)::value;
-        if (FIRST) tmax = max16(s);
+    auto prepare = [&](Scores& s, int blk, Pair tmax, auto first_c, auto look_c) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first_c)::value, LOOK = FIRST || MAXIMA || decltype(look_c)::value;     // sums are looked at now and then
         const int key0 = (blk + 2 * t_first) * 32;
         if (key0 + 31 > vis_lo) {   // wave-uniform: some query of the wavefront does not see the whole block
             // (the empty volatile statement keeps this a branch: as 48 speculated selects it would run for every block)
             asm volatile("" ::: );
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int key = key0 + 8 * (v >> 2) + 4 * hl + (v & 3);
-                s[v] = key <= vis_j ? s[v] : PF_NEG;
+                const int key = key0 + 16 * (v >> 3) + 4 * ig + (v & 3), qg = (v >> 2) & 1;
+                s.g[v >> 3][qg][v & 3] = key <= vis_j[qg] ? s.g[v >> 3][qg][v & 3] : PF_NEG;
             }
-            tmax = max16(s);
+            if (MAXIMA && !FIRST) tmax = Pair{{max8(s, 0), max8(s, 1)}};
         }
-        if (FIRST || __builtin_amdgcn_ballot_w64(tmax > PF2_LAZY) != 0) {
-            const float t2 = __builtin_fmaxf(tmax, __shfl_xor(tmax, 32, 64));   // both halves of a query agree on the reference
-            // how far the reference moves: onto the maximum (first block; not at all for a row that sees nothing), else up only
-            const float d = FIRST ? (t2 > 0.5f * PF_NEG ? t2 : 0.0f) : __builtin_fmaxf(t2, 0.0f);
-            m_ref += d;
+        if (FIRST) tmax = Pair{{max8(s, 0), max8(s, 1)}};
+        if (!FIRST && !MAXIMA) tmax = Pair{{l_run[0], l_run[1]}};
+        if (FIRST || (LOOK && __builtin_amdgcn_ballot_w64(__builtin_fmaxf(tmax.x[0], tmax.x[1]) > (MAXIMA ? PF2_LAZY : PF2_MOST)) != 0)) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) { s[v] -= d; negm[v] = -m_ref; }
-            if (!FIRST) {
-                const float alpha = __builtin_amdgcn_exp2f(-d);
-                l_run *= alpha;
+            for (int qg = 0; qg < 2; ++qg) {
+                float t2 = __builtin_fmaxf(tmax.x[qg], __shfl_xor(tmax.x[qg], 16, 64));   // the four row groups of a query agree on the reference
+                t2 = __builtin_fmaxf(t2, __shfl_xor(t2, 32, 64));
+                // how far the reference moves: onto the maximum (first block; not at all for a row that sees nothing), else up only; without maxima by the
+                // exponent of the largest sum (0 of what is not finite)
+                const float d = FIRST ? (t2 > 0.5f * PF_NEG ? t2 : 0.0f) : MAXIMA ? __builtin_fmaxf(t2, 0.0f) : __builtin_fmaxf((float)__builtin_amdgcn_frexp_expf(t2), 0.0f);
+                m_ref[qg] += d;
 #pragma unroll
-                for (int db = 0; db < 4; ++db)
+                for (int v = 0; v < 4; ++v) { s.g[0][qg][v] -= d; s.g[1][qg][v] -= d; negm[qg][v] = -m_ref[qg]; }
+                if (!FIRST) {
+                    const float alpha = __builtin_amdgcn_exp2f(-d);
+                    l_run[qg] *= alpha;
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) o[db][v] *= alpha;
+                    for (int dg = 0; dg < 8; ++dg)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) o[dg >> 1][8 * (dg & 1) + 4 * qg + v] *= alpha;
+                }
             }
         }
     };
-    // P = exp2(s - ref) as bf16 (two scores -> one dword) and the row sum of the rounded P
-    auto p_pair = [&](const pf_f32x16& s, int x) __attribute__((always_inline)) {
-        const float p0 = __builtin_amdgcn_exp2f(s[2 * x]);
-        const float p1 = __builtin_amdgcn_exp2f(s[2 * x + 1]);
+    // P = exp2(s - ref) as bf16 (two scores -> one dword) and the row sum of the rounded P; pair x = 4 qg + 2 kg + half: in the order in
+    // which the P operand takes them
+    auto p_pair = [&](const Scores& s, int x) __attribute__((always_inline)) {
+        const int qg = x >> 2, kg = (x >> 1) & 1, v = 2 * (x & 1);
+        const float p0 = __builtin_amdgcn_exp2f(s.g[kg][qg][v]);
+        const float p1 = __builtin_amdgcn_exp2f(s.g[kg][qg][v + 1]);
         const uint32_t pw = pack_kv<F16>(p0, p1);
-        l_run = add_pair<F16>(pw, l_run);
+        l_run[qg] = add_pair<F16>(pw, l_run[qg]);
         return pw;
     };
-    // One pipeline step, in issue order (the fences keep the compiler from regrouping it): the 8 MFMAs of the next
-    // block's scores, each followed by one eighth of this block's exponentials; then the 8 MFMAs of P.V, with the maximum
-    // of the next block's scores computed in their shadow.  s_cur and s_nxt are two register blocks that swap roles from
-    // step to step (no copy).  The 16 MFMA operands of a step (8 K fragments, then 8 V fragments) belong to one stream of
-    // LDS reads that runs across steps: each is requested PD MFMAs before the one that consumes it, so the first PD K
-    // fragments of a step were requested by the step before it (pre[], in and out).
-    //   kimm, vimm: byte offsets of this step's K block and V block; nkimm: of the next step's K block
-    //   HAS_NEXT = false: last block of the wavefront, no scores to compute.  FEEDS_NEXT = false: no step follows that wants K.
-    //   SYNC: the iteration's barrier, between the two groups of MFMAs (the score MFMAs drain while the wavefront waits).
-    // Returns the row maximum of s_nxt (this lane's 16 scores).
-    auto step = [&](const pf_f32x16& s_cur, pf_f32x16& s_nxt, pf_bf16x8 (&pre)[PF2_PD], auto kimm_c, auto vimm_c, auto nkimm_c, auto has_next,
-                    auto feeds_next, auto sync_c) __attribute__((always_inline)) -> float {
-        constexpr bool HAS_NEXT = decltype(has_next)::value, FEEDS_NEXT = decltype(feeds_next)::value, SYNC = decltype(sync_c)::value;
-        const int KIMM = kimm_c, VIMM = vimm_c, NKIMM = nkimm_c;   // integral constants in the main loop (instruction immediates), plain ints in the tail
-        constexpr int PD = PF2_PD;
-        pf_bf16x8 frag[16 + PD];
-        uint32_t pw[8];
-        auto request = [&](int m) __attribute__((always_inline)) {
-            if (m < 8) {
-                if (HAS_NEXT) frag[m] = k_frag(KIMM, m);
-            } else if (m < 16) {
-                frag[m] = v_frag(VIMM, (m - 8) >> 2, (m - 8) & 3);
-            } else if (FEEDS_NEXT) {
-                frag[m] = k_frag(NKIMM, m - 16);
-            }
-        };
+    auto meet = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // A block of 32 keys has two parts: the exponentials of its scores while the LDS operands of what follows are read, then 32 MFMAs, P.V of the
+    // block and the scores of the next one.  The wavefronts 4 .. 7 are one part behind the others, so that on every SIMD one
+    // wavefront multiplies while the other one does everything else; the barrier between the parts keeps them so.
+    //   vimm, kimm: byte offsets of this block's V and of the next block's K; LAND: the tile after this one has landed behind this part
+    auto max3 = [](float x, float y, float z) __attribute__((always_inline)) { return __builtin_fmaxf(__builtin_fmaxf(x, y), z); };
+    auto block = [&](Scores& s, auto vimm, auto kimm, auto land) __attribute__((always_inline)) -> Pair {
+        pf_bf16x8 kf[8], vf[8];
 #pragma unroll
-        for (int m = 0; m < PD; ++m) frag[m] = pre[m];
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            request(ks + PD);
-            pw[ks] = p_pair(s_cur, ks);
-            if (HAS_NEXT) s_nxt = mfma_32x32x16<F16>(frag[ks], qf[ks], ks == 0 ? negm : s_nxt);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (SYNC) {   // behind the barrier the next tile is visible: every thread has waited for its own four loads of it
-            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");   // (the four of the tile after it may still be in flight)
-            __syncthreads();
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int m = 0; m < 8; ++m) kf[m] = k_frag(kimm, m);
         pf_bf16x8 pfrag[2];
+        uint32_t pw[8];
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            const pf_u32x4 pq = {pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]};
-            pfrag[st] = __builtin_bit_cast(pf_bf16x8, pq);
+        for (int x = 0; x < 8; ++x) pw[x] = p_pair(s, x);
+#pragma unroll
+        for (int qg = 0; qg < 2; ++qg) {
+            const pf_u32x4 pq = {pw[4 * qg], pw[4 * qg + 1], pw[4 * qg + 2], pw[4 * qg + 3]};
+            pfrag[qg] = __builtin_bit_cast(pf_bf16x8, pq);
         }
-        // the maximum of the next block's scores as a tree of three-input maxima, one or two per P.V MFMA from the third
-        // on (the last score MFMA has landed by then); the empty volatile statements fix where each is computed: between
-        // these two MFMAs, not after the last one
-        float mt[7];
-        auto max3 = [](float x, float y, float z) __attribute__((always_inline)) { return __builtin_fmaxf(__builtin_fmaxf(x, y), z); };
+        asm volatile("" : "+v"(pfrag[0]), "+v"(pfrag[1]), "+v"(l_run[0]), "+v"(l_run[1]));
+        __builtin_amdgcn_sched_barrier(0);
+        if (decltype(land)::value) asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");      // (the four loads of the tile after it may still be in flight)
+        else asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            request(8 + i + PD);
-            o[i & 3] = mfma_32x32x16<F16>(frag[8 + i], pfrag[i >> 2], o[i & 3]);
-            if (HAS_NEXT) {
-                if (i >= 2 && i <= 6) { mt[i - 2] = max3(s_nxt[3 * (i - 2)], s_nxt[3 * (i - 2) + 1], s_nxt[3 * (i - 2) + 2]); asm volatile("" : "+v"(mt[i - 2])); }
-                if (i == 6) { mt[5] = max3(mt[0], mt[1], s_nxt[15]); asm volatile("" : "+v"(mt[5])); }
-                if (i == 7) { mt[6] = max3(mt[2], mt[3], mt[4]); asm volatile("" : "+v"(mt[6])); }
+        for (int m = 0; m < 8; ++m) {
+            vf[m] = v_frag(vimm, m);
+#pragma unroll
+            for (int qg = 0; qg < 2; ++qg) s.g[m & 1][qg] = mfma_16x16x32<F16>(kf[m], qf[qg][m >> 1], m < 2 ? negm[qg] : s.g[m & 1][qg]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float mt[2][3];
+        Pair mx = {{0.0f, 0.0f}};
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+#pragma unroll
+            for (int qg = 0; qg < 2; ++qg) {
+                pf_f32x16& all = o[m >> 1];
+                const int at = 8 * (m & 1) + 4 * qg;
+                const pf_f32x4 r = mfma_16x16x32<F16>(vf[m], pfrag[qg], pf_f32x4{all[at], all[at + 1], all[at + 2], all[at + 3]});
+#pragma unroll
+                for (int v = 0; v < 4; ++v) all[at + v] = r[v];
+            }
+            if (MAXIMA && m >= 2) {          // trees of three-input maxima (the last score MFMA has landed by then)
+                const int qg = m & 1;
+                const pf_f32x4 lo = s.g[0][qg], hi = s.g[1][qg];
+                if (m < 4) { mt[qg][0] = max3(lo[0], lo[1], lo[2]); asm volatile("" : "+v"(mt[qg][0])); }
+                else if (m < 6) { mt[qg][1] = max3(hi[0], hi[1], hi[2]); asm volatile("" : "+v"(mt[qg][1])); }
+                else {
+                    mt[qg][2] = max3(lo[3], hi[3], mt[qg][0]);
+                    mx.x[qg] = __builtin_fmaxf(mt[qg][1], mt[qg][2]);
+                    asm volatile("" : "+v"(mx.x[qg]));
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (FEEDS_NEXT) {
-#pragma unroll
-            for (int m = 0; m < PD; ++m) pre[m] = frag[16 + m];
-        }
-        float mx = HAS_NEXT ? __builtin_fmaxf(mt[5], mt[6]) : 0.0f;
-        // both values are wanted here, at the end of the step: without this the compiler moves the maxima and the row-sum
-        // additions behind the branch that follows, out of the shadow of the MFMAs
-        asm volatile("" : "+v"(mx), "+v"(l_run));
+        __builtin_amdgcn_s_setprio(0);
+        meet();
         return mx;
     };
 
-    // Pipeline over 32-key blocks: while the exponentials of block b run on the VALU, the MFMA unit computes the scores
-    // of block b + 1 and then P.V of block b.  Every wavefront walks all blocks of the workgroup's tiles: the blocks that
+    // Every wavefront walks all blocks of the workgroup's tiles: the blocks that
     // lie wholly above a wavefront's diagonal (at most two of up to several hundred, the workgroup spans BT query times)
     // are masked like the diagonal ones and contribute zeros, which keeps the loop free of per-wavefront branches.
-    if (ntiles > 0) {
-        pf_f32x16 s_a, s_b;   // scores of the current and of the next block, roles swapping every step
-        pf_bf16x8 pre[PF2_PD];
+    if constexpr (HOW == ATTEND_CAREFULLY) {
+#pragma clang loop unroll(disable)
+        for (int blk = 0; blk < 2 * ntiles; ++blk) {
+            const int off = (blk & 1) * (PF2_TILE / 2);
+            if (!(blk & 1)) {
+                __syncthreads();                 // every wavefront has left the tile before
+                request_tile(blk >> 1, 0);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+            }
+            Scores s;
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+#pragma unroll
+                for (int qg = 0; qg < 2; ++qg) s.g[m & 1][qg] = mfma_16x16x32<F16>(k_frag(off, m), qf[qg][m >> 1], m < 2 ? negm[qg] : s.g[m & 1][qg]);
+            if (blk == 0) prepare(s, 0, Pair{{0.0f, 0.0f}}, std::true_type{}, std::true_type{});
+            else prepare(s, blk, Pair{{max8(s, 0), max8(s, 1)}}, std::false_type{}, std::true_type{});
+            uint32_t pw[8];
+#pragma unroll
+            for (int x = 0; x < 8; ++x) pw[x] = p_pair(s, x);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                const pf_bf16x8 v = v_frag(off, m);
+#pragma unroll
+                for (int qg = 0; qg < 2; ++qg) {
+                    const pf_u32x4 pq = {pw[4 * qg], pw[4 * qg + 1], pw[4 * qg + 2], pw[4 * qg + 3]};
+                    pf_f32x16& all = o[m >> 1];
+                    const int at = 8 * (m & 1) + 4 * qg;
+                    const pf_f32x4 r = mfma_16x16x32<F16>(v, __builtin_bit_cast(pf_bf16x8, pq), pf_f32x4{all[at], all[at + 1], all[at + 2], all[at + 3]});
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) all[at + x] = r[x];
+                }
+            }
+        }
+    } else if (ntiles > 0) {
+        Scores s;
         asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         __syncthreads();
-        {
-            s_a = negm;
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) s_a = mfma_32x32x16<F16>(k_frag(0, ks), qf[ks], s_a);
+        for (int m = 0; m < 8; ++m)
 #pragma unroll
-            for (int m = 0; m < PF2_PD; ++m) pre[m] = k_frag(PF2_TILE / 2, m);
-        }
-        prepare(s_a, 0, 0.0f, std::true_type{});
+            for (int qg = 0; qg < 2; ++qg) s.g[m & 1][qg] = mfma_16x16x32<F16>(k_frag(0, m), qf[qg][m >> 1], m < 2 ? negm[qg] : s.g[m & 1][qg]);
+        prepare(s, 0, Pair{{0.0f, 0.0f}}, std::true_type{}, std::true_type{});
+        if (w >= PF2_WAVES / 2) meet();
         // Iteration t (tile t in the buffer at off0, tile t + 1 at off1): blocks 2t and 2t + 1, and the scores of block 2t + 2.
-        // Tile t + 2 is requested first, into the buffer tile t - 2 used (every wavefront left it before the barrier of
-        // iteration t - 1).  The one barrier of an iteration sits inside its first step, between the score MFMAs and the
-        // P.V MFMAs: behind it tile t + 1 is visible, in time for the K fragments that the end of that step requests.
-        auto iteration = [&](int t, int b2, auto off0, auto off1) __attribute__((always_inline)) {
+        // Tile t + 2 is requested first, into the buffer tile t - 2 used (every wavefront has left it).  Behind the first part of block 2t tile t + 1 has landed
+        // everywhere, in time for the K that the second block's first part reads.
+        auto iteration = [&](int t, int b2, auto off0, auto off1, auto look) __attribute__((always_inline)) {
             constexpr std::integral_constant<int, PF2_TILE / 2> half{};
             request_tile(t + 2, b2);          // unconditional (rows clamped): the count of loads in flight stays fixed
-            const float ma = step(s_a, s_b, pre, off0 + half, off0, off1, std::true_type{}, std::true_type{}, std::true_type{});
-            prepare(s_b, 2 * t + 1, ma, std::false_type{});
-            const float mb = step(s_b, s_a, pre, off1, off0 + half, off1 + half, std::true_type{}, std::true_type{}, std::false_type{});
-            prepare(s_a, 2 * t + 2, mb, std::false_type{});
+            const Pair ma = block(s, off0, off0 + half, std::true_type{});
+            prepare(s, 2 * t + 1, ma, std::false_type{}, std::false_type{});
+            const Pair mb = block(s, off0 + half, off1, std::false_type{});
+            prepare(s, 2 * t + 2, mb, std::false_type{}, look);
         };
         using I0 = std::integral_constant<int, 0>; using I1 = std::integral_constant<int, PF2_TILE>;
         using I2 = std::integral_constant<int, 2 * PF2_TILE>; using I3 = std::integral_constant<int, 3 * PF2_TILE>;
         int t = 0;
         for (; t + 4 < ntiles; t += 4) {      // four tiles per turn: buffer offsets are immediates of the LDS reads
-            iteration(t, 2, I0{}, I1{});
-            iteration(t + 1, 3, I1{}, I2{});
-            iteration(t + 2, 0, I2{}, I3{});
-            iteration(t + 3, 1, I3{}, I0{});
+            iteration(t, 2, I0{}, I1{}, std::false_type{});
+            iteration(t + 1, 3, I1{}, I2{}, std::false_type{});
+            iteration(t + 2, 0, I2{}, I3{}, std::false_type{});
+            iteration(t + 3, 1, I3{}, I0{}, std::true_type{});
         }
-        for (; t + 1 < ntiles; ++t)           // up to three more, offsets computed
-            iteration(t, (t + 2) & 3, (t & 3) * PF2_TILE, ((t + 1) & 3) * PF2_TILE);
-        {   // the last tile: its second block has no successor
-            const int off = (t & 3) * PF2_TILE;
-            const float ma = step(s_a, s_b, pre, off + PF2_TILE / 2, off, 0, std::true_type{}, std::false_type{}, std::false_type{});
-            prepare(s_b, 2 * t + 1, ma, std::false_type{});
-            step(s_b, s_a, pre, 0, off + PF2_TILE / 2, 0, std::false_type{}, std::false_type{}, std::false_type{});
-        }
+        // up to four more, offsets computed; the scores that the last block leaves are of keys that are not there, and nobody reads them
+        for (; t < ntiles; ++t) iteration(t, (t + 2) & 3, (t & 3) * PF2_TILE, ((t + 1) & 3) * PF2_TILE, std::true_type{});
+        if (w < PF2_WAVES / 2) meet();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the look-ahead tiles were requested too: nothing may land after the wavefront has gone
     }
 
-    // the two halves of a query hold disjoint keys: add their sums, then normalise and store
-    l_run += __shfl_xor(l_run, 32, 64);
-    if (PART && all_tiles > ntiles) {
-        if (hl == 0) *(float2*)(a.part_ml + (slot * (PF2_WAVES * 32) + r) * 2) = make_float2(m_ref, l_run);
-        float4* po = (float4*)a.part + (slot * PF2_WAVES + w) * (16 * 64) + lane;   // in register order: 1 KB per store
+    if (HOW == ATTEND_SUMS) {
+        float sign = l_run[0] * 0.0f + l_run[1] * 0.0f;       // 0, or not a number
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                po[(db * 4 + c) * 64] = make_float4(o[db][4 * c], o[db][4 * c + 1], o[db][4 * c + 2], o[db][4 * c + 3]);
+            for (int v = 0; v < 16; ++v) sign = fmaf(o[db][v], 0.0f, sign);
+        if (!(sign == 0.0f)) *again = 1;
+    }
+    // the four row groups of a query hold disjoint keys: add their sums, then normalise and store
+#pragma unroll
+    for (int qg = 0; qg < 2; ++qg) {
+        l_run[qg] += __shfl_xor(l_run[qg], 16, 64);
+        l_run[qg] += __shfl_xor(l_run[qg], 32, 64);
+    }
+    if (PART && all_tiles > ntiles) {
+#pragma unroll
+        for (int qg = 0; qg < 2; ++qg)
+            if (ig == 0) *(float2*)(a.part_ml + (slot * (PF2_WAVES * 32) + w * 32 + qg * 16 + j) * 2) = make_float2(m_ref[qg], l_run[qg]);
+        float4* po = (float4*)a.part + (slot * PF2_WAVES + w) * (16 * 64) + lane;   // in register order: 1 KB per store
+#pragma unroll
+        for (int dg = 0; dg < 8; ++dg)
+#pragma unroll
+            for (int qg = 0; qg < 2; ++qg) po[(qg * 8 + dg) * 64] = make_float4(o_of(dg, qg, 0), o_of(dg, qg, 1), o_of(dg, qg, 2), o_of(dg, qg, 3));
         return;
     }
     // A lane holds four features of a row at a time: stored from there, a row of 256 bytes would leave in 16 pieces.  The wavefront's
     // 32 rows take the way through LDS instead (8 KB of its own; the 16-byte piece c of row j at c ^ (j % 16)) and leave whole.
-    const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     PF_LDS3 char* const mine = lds3 + w * 8192;
     __syncthreads();                             // every wavefront has left the tiles
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int qg = 0; qg < 2; ++qg) {
+        const float inv = l_run[qg] > 0.0f ? 1.0f / l_run[qg] : 0.0f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            *(PF_LDS3 pf_u32x2*)(mine + j * 256 + (((db * 4 + c) ^ (j & 15)) << 4) + hl * 8) =
-                pf_u32x2{pack_kv<F16>(o[db][4 * c] * inv, o[db][4 * c + 1] * inv), pack_kv<F16>(o[db][4 * c + 2] * inv, o[db][4 * c + 3] * inv)};
+        for (int dg = 0; dg < 8; ++dg)
+            *(PF_LDS3 pf_u32x2*)(mine + (qg * 16 + j) * 256 + (((dg * 2 + (ig >> 1)) ^ j) << 4) + (ig & 1) * 8) =
+                pf_u32x2{pack_kv<F16>(o_of(dg, qg, 0) * inv, o_of(dg, qg, 1) * inv), pack_kv<F16>(o_of(dg, qg, 2) * inv, o_of(dg, qg, 3) * inv)};
+    }
     const int piece = lane & 15;
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
@@ -713,6 +773,20 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
         const pf_u32x4 v = *(const PF_LDS3 pf_u32x4*)(mine + row * 256 + ((piece ^ (row & 15)) << 4));
         if (rr < BT * G && t < Q && piece * 8 < a.hd)
             *(pf_u32x4*)(a.out + (((int64_t)b * Q + t) * (a.kv_heads * G) + (h * G + rr % G)) * a.hd + piece * 8) = v;
+    }
+}
+
+// ends with every wavefront having left the LDS tiles; `again` is 0 then, as it is in front
+template <bool F16, bool PART, bool LOOP>
+__device__ __forceinline__ void attend_query_tile_once(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot, PF_LDS3 int* again) {
+    attend_query_tile<F16, PART, LOOP, F16 ? ATTEND_MAXIMA : ATTEND_SUMS>(a, seg, tile, t_first, count, slot, again);
+    if (F16 && !LOOP) return;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");       // for LDS: nobody waits for the stores
+    if (!F16 && __builtin_amdgcn_readfirstlane(*again)) {
+        __syncthreads();                         // everyone has read it
+        if (threadIdx.x == 0) *again = 0;
+        attend_query_tile<F16, PART, LOOP, ATTEND_CAREFULLY>(a, seg, tile, t_first, count, slot, again);
+        __syncthreads();
     }
 }
 
@@ -732,7 +806,9 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     }
     const int t_first = SPLIT ? (int)blockIdx.z * a.split_tiles : 0;
     if (SPLIT && t_first > 0 && t_first >= tiles_seen(a, seg, tile)) return;
-    attend_query_tile<F16, SPLIT, false>(a, seg, tile, t_first, a.split_tiles, ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile);
+    __shared__ int again;
+    if (threadIdx.x == 0) again = 0;             // a barrier lies between this and whoever looks at it
+    attend_query_tile_once<F16, SPLIT, false>(a, seg, tile, t_first, a.split_tiles, ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile, (PF_LDS3 int*)&again);
 }
 
 // Equal shares (gridDim.x workgroups, one per CU): the key tiles of all query tiles, one query tile after the other, are cut into
@@ -744,7 +820,7 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
 // with appends and eviction 1451 -> 1317 us; sizes on either side of the rule at trimkv_prefill_equal_shares.
 template <bool F16>
 __global__ __launch_bounds__(PF2_THREADS) void prefill_shares_kernel(PrefillArgs a) {
-    __shared__ int sums[PF2_WAVES], found[2];
+    __shared__ int sums[PF2_WAVES], found[2], again;
     const int tid = threadIdx.x, lane = tid & 63, groups = (int)gridDim.x;
     const int wg = (groups & 7) ? (int)blockIdx.x : ((int)blockIdx.x & 7) * (groups >> 3) + ((int)blockIdx.x >> 3);
     // first units of all query tiles: a thread sums the ones it has, a scan over the threads says where they begin
@@ -774,19 +850,19 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_shares_kernel(PrefillArgs
         if (u0 >= at && u0 < at + c) { found[0] = i; found[1] = u0 - at; }
         at += c;
     }
+    if (tid == 0) again = 0;
     if (wg == 0 && tid == 0) a.plan[0] = per;
     if (u0 >= u1) return;                        // the whole workgroup: nothing was left for it
     __syncthreads();
     int i = __builtin_amdgcn_readfirstlane(found[0]), t_first = __builtin_amdgcn_readfirstlane(found[1]);
     for (int u = u0; u < u1; ++i, t_first = 0) {
         const int seg = i / a.query_tiles, count = min(units_of(a, i) - t_first, u1 - u);
-        attend_query_tile<F16, true, true>(a, seg, i - seg * a.query_tiles, t_first, count, 2 * wg + (t_first == 0));
+        attend_query_tile_once<F16, true, true>(a, seg, i - seg * a.query_tiles, t_first, count, 2 * wg + (t_first == 0), (PF_LDS3 int*)&again);
         u += count;
-        __syncthreads();                         // every wavefront has left the LDS tiles
     }
 }
 
-// The shares of the keys put together: one wavefront per (query tile, 32 of its rows, 32 features), lanes as they wrote.
+// The shares of the keys put together: one wavefront per (query tile, 16 of its rows, 64 features), lanes as they wrote.
 // A share that a row saw nothing of has sum 0 and a reference of no meaning: it is left out.
 // EQUAL: shares as prefill_shares_kernel cut them, of which the first is in its workgroup's second slot.
 template <bool F16, bool EQUAL>
@@ -795,7 +871,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int b = seg / a.kv_heads, h = seg - b * a.kv_heads;
     int n = a.seg_len ? a.seg_len[seg] : a.max_len;
     n = max(0, min(n, a.max_len));
-    const int db = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, hl = lane >> 5;
+    const int half = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, ig = lane >> 4;       // half / 2: of the features, half % 2: of the rows
     const int G = a.group, Q = a.q_len, BT = (PF2_WAVES * 32) / G;
     const int t_last = min(Q - 1, tile * BT + BT - 1);
     const int all_tiles = (max(0, min(n, n - Q + t_last + 1)) + PF2_BN - 1) / PF2_BN;
@@ -806,12 +882,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
         shares = (at + max(all_tiles, 1) - 1) / per - first + 1;
     } else shares = (all_tiles + a.split_tiles - 1) / a.split_tiles;
     if (shares <= 1) return;                  // its workgroup wrote the result
-    const int r = w * 32 + j, g = r % G, t_q = tile * BT + r / G;
+    const int r = w * 32 + (half & 1) * 16 + j, g = r % G, t_q = tile * BT + r / G;
     if (r >= BT * G || t_q >= Q) return;
     const int64_t wg = (int64_t)seg * tiles + tile, per_share = (int64_t)gridDim.y * tiles;
     auto slot = [&](int z) -> int64_t { return EQUAL ? 2 * (first + z) + (z == 0) : wg + z * per_share; };
     const float2* ml = (const float2*)a.part_ml + r;
-    const float4* po = (const float4*)a.part + w * (16 * 64) + db * (4 * 64) + lane;
+    const float4* po = (const float4*)a.part + w * (16 * 64) + ((half & 1) * 8 + (half >> 1) * 4) * 64 + lane;
     float m = -3.0e38f;
     for (int z = 0; z < shares; ++z) {
         const float2 x = ml[slot(z) * (PF2_WAVES * 32)];
@@ -836,7 +912,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     char* orow = (char*)(a.out + (((int64_t)b * Q + t_q) * (a.kv_heads * G) + (h * G + g)) * a.hd);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        const int d = db * 32 + 8 * c + 4 * hl;
+        const int d = (half >> 1) * 64 + 16 * c + 4 * ig;
         if (d < a.hd) *(uint2*)(orow + d * 2) = make_uint2(pack_kv<F16>(o[c].x * inv, o[c].y * inv), pack_kv<F16>(o[c].z * inv, o[c].w * inv));
     }
 }
