@@ -316,6 +316,26 @@ def test_experts_of_either_tile_height(ff, width):
     close(y[:, :width], want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each, as above
 
 
+@pytest.mark.parametrize("E,ff,width", [(1, 2560, 64), (64, 64, 576), (65, 320, 64), (150, 64, 320)])
+def test_experts_cut_into_runs(E, ff, width):
+    """As many experts as a wavefront has lanes, more of them and a single one, most of them with a few rows or none beside some with
+    several tiles: runs of tiles that begin within an expert and between two, and more workgroups than tiles."""
+    counts = [0 if e % 7 == 3 else 1 + (e * 37) % 40 if e % 11 else 1300 + 90 * (e % 5) for e in range(E)]
+    T = sum(counts)
+    assert T >= 12 * E and T >= 1200
+    x = rnd(T, ops.padded(width), seed=1, dtype=torch.bfloat16)
+    up, down = torch.zeros(E, ops.padded(ff), ops.padded(width)), torch.zeros(E, ops.padded(width), ops.padded(ff))
+    up[:, :ff, :width] = rnd(E, ff, width, seed=2) * width ** -0.5
+    down[:, :width, :ff] = rnd(E, width, ff, seed=3) * ff ** -0.5
+    up, down = up.to(torch.bfloat16), down.to(torch.bfloat16)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])[torch.randperm(T, generator=torch.Generator().manual_seed(4))]
+    y = ops.experts(x.to(DEV), ids[:, None].int().to(DEV), ops.pack_matrix(up).contiguous().to(DEV), ops.pack_matrix(down).contiguous().to(DEV), width)
+    want = torch.empty(T, width, dtype=torch.float64)
+    for e in range(E):
+        want[ids == e] = ref.expert(x[ids == e].double(), up[e].double(), down[e].double())[:, :width]
+    close(y, want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each, as above
+
+
 @pytest.mark.parametrize("ff,width", [(352, 640), (704, 352)])
 def test_experts_whose_steps_go_round_the_buffers(ff, width):
     """Prompt-sized products of 12, 20 and 22 steps of 32 k: the five operand buffers are filled anew two to four times while

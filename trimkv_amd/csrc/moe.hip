@@ -76,37 +76,35 @@ __global__ __launch_bounds__(256) void route_kernel(const float* z, const float*
 
 // One workgroup orders all rows (a step's few thousand, or a prompt's tens of thousands): counts, offsets and scatter in LDS.
 __global__ __launch_bounds__(1024) void plan_kernel(const int32_t* ids, int rows, int E, int tile, int32_t* order, int32_t* offsets, int32_t* tiles) {
-    extern __shared__ int32_t pl[];               // cursor [E], tile cursor [E], cursor of the last tile if it is not full [E]
-    int32_t* cursor = pl; int32_t* tcur = pl + E; int32_t* tlast = tcur + E;
-    const bool apart = tile >= 256;               // tiles of the matrix-bound kernel: those that are not full come last, so that the launch ends on short ones
+    extern __shared__ int32_t pl[];               // cursor [E], tile cursor [E]
+    int32_t* cursor = pl; int32_t* tcur = pl + E;
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += 1024) cursor[e] = 0;
     __syncthreads();
     for (int i = tid; i < rows; i += 1024) atomicAdd(&cursor[ids[i]], 1);
     __syncthreads();
     if (tid < 64) {                               // exclusive sums over experts, 64 at a time
-        int base = 0, tbase = 0, lbase = 0;
+        int base = 0, tbase = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + tid, c = e < E ? cursor[e] : 0, nt = apart ? c / tile : (c + tile - 1) / tile, nl = apart && c % tile ? 1 : 0;
-            int s = c, ts = nt, ls = nl;
+            const int e = e0 + tid, c = e < E ? cursor[e] : 0, nt = (c + tile - 1) / tile;
+            int s = c, ts = nt;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(s, d, 64), to = __shfl_up(ts, d, 64), lo = __shfl_up(ls, d, 64);
-                if (tid >= d) { s += o; ts += to; ls += lo; }
+                const int o = __shfl_up(s, d, 64), to = __shfl_up(ts, d, 64);
+                if (tid >= d) { s += o; ts += to; }
             }
-            if (e < E) { offsets[e] = base + s - c; cursor[e] = base + s - c; tcur[e] = tbase + ts - nt; tlast[e] = lbase + ls - nl; }
+            if (e < E) { offsets[e] = base + s - c; cursor[e] = base + s - c; tcur[e] = tbase + ts - nt; }
             base += __shfl(s, 63, 64);
             tbase += __shfl(ts, 63, 64);
-            lbase += __shfl(ls, 63, 64);
         }
-        if (tid == 0) { offsets[E] = base; tiles[0] = tbase + lbase; pl[3 * E] = tbase; }
+        if (tid == 0) { offsets[E] = base; tiles[0] = tbase; }
     }
     __syncthreads();
     // tiles[1 + 2 i] = expert, tiles[2 + 2 i] = first row of tile i
     for (int e = tid; e < E; e += 1024) {
         const int first = cursor[e], c = (e + 1 < E ? cursor[e + 1] : rows) - first;
         for (int x = 0; x * tile < c; ++x) {
-            const int i = apart && (x + 1) * tile > c ? pl[3 * E] + tlast[e] : tcur[e] + x;
+            const int i = tcur[e] + x;
             tiles[1 + 2 * i] = e;
             tiles[2 + 2 * i] = first + x * tile;
         }
@@ -217,36 +215,71 @@ __global__ __launch_bounds__(KS * 64) void grouped_skinny_kernel(GroupedArgs a) 
 }
 
 // bf16, more than a few rows per expert (prompts): 256 rows x 256 outputs per workgroup (tiles.hip.h), or 192 or 128 rows of the
-// last tile of an expert that holds no more.  With 8192 tokens x 4 of 32 experts (4096 x 4608) it is bound by the clock that the matrix cores leave
-// the chip (1.7 GHz, pipes busy 73 % of a compute unit's time) and by what the L2s fetch: 1.46 PFLOP/s where four rows in a row are one token's
-// and all weights fit the last level of cache, 1.2 PFLOP/s with the rows of a random choice, 1.03 with experts of unequal size, whose last
-// tiles are part empty.  Both products take 2.2 ms; a kernel that fed 32x32x16 products from five buffers of 32 k, all wavefronts in step,
-// took 2.6 ms.
+// last tile of an expert that holds no more.  It is bound by the matrix cores at the clock that they leave the chip (1.7 GHz): 8192 tokens x 4 of 32
+// experts of 4096 x 4608 take 875 us where every expert has 1024 rows (1.42 PFLOP/s; rows in any order, the gather costs nothing) and 1020 where
+// counts differ by a factor of 4 (143 row tiles, 32 of them part empty: 870 us of work for 256 compute units; the rest are units that wait
+// for the next workgroup of their shader engine, 5 %, and the last tiles, 6 %).
+// With the tiles that are not full last, as the shorter work to end on, the same took 1158: each of them reads its expert's weights
+// alone then, 2 MB of w for 128 rows, and 128 rows last 87 us instead of 61.  A kernel that fed 32x32x16 products from five
+// buffers of 32 k, all wavefronts in step, took 1300.
 template <bool UP>
 __global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_tiles, int experts) {
     extern __shared__ __attribute__((aligned(16))) char gb_lds[];
     HY_LDS char* const lds3 = (HY_LDS char*)gb_lds;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, hl = lane >> 4, wm = w >> 2, wn = w & 3;
-    // Row tiles that are full come first in the plan.  They and the others are taken apart, in blocks of 4 row tiles x all outputs, row tiles fastest, cut
-    // into eight equal runs, one for each XCD: the rows and the weights that neighbouring workgroups read stay in its L2, every XCD
-    // has as much to do, and the launch ends on short tiles.
-    int full = 0;
-    for (int e = lane; e < experts; e += 64) full += (a.offsets[e + 1] - a.offsets[e]) >> 8;
+    // The tiles of an expert stay together, for the weights that they share in an XCD's L2: in blocks of up to 4 of them x all columns of outputs,
+    // row tiles fastest.  The whole is cut at columns of blocks into eight runs, one for each XCD, that cost the same: 6, 5 and 4
+    // for a tile of 256, 192 and 128 rows (90, 74 and 61 us at 4096 k).  Equal numbers of tiles instead: 1107 us for 1020.
+    int e = 0, m0 = 0, nt = 0;
+    {
+        auto cost_of = [](int c) __attribute__((always_inline)) { const int p = c & 255; return 6 * (c >> 8) + (p > 192 ? 6 : p > 128 ? 5 : p ? 4 : 0); };
+        const int c0 = lane < experts ? a.offsets[lane + 1] - a.offsets[lane] : 0;
+        auto rows_of = [&](int e0) __attribute__((always_inline)) { return e0 == 0 ? c0 : e0 + lane < experts ? a.offsets[e0 + lane + 1] - a.offsets[e0 + lane] : 0; };
+        auto scan = [&](int v) __attribute__((always_inline)) {
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) full += __shfl_xor(full, d, 64);
-    full = __builtin_amdgcn_readfirstlane(full);
-    const int xcd = blockIdx.x & 7, parts = a.tiles[0] - full;
-    auto from = [&](int tiles, int i) { return (int)((int64_t)tiles * n_tiles * i / 8); };
-    int at = from(full, xcd) + (blockIdx.x >> 3), total = full, base = 0;
-    if (at >= from(full, xcd + 1)) {
-        at = from(parts, xcd) + at - from(full, xcd + 1);
-        if (at >= from(parts, xcd + 1)) return;
-        total = parts;
-        base = full;
+            for (int d = 1; d < 64; d <<= 1) { const int o = __shfl_up(v, d, 64); if (lane >= d) v += o; }
+            return v;
+        };
+        int total = 0;
+        for (int e0 = 0; e0 < experts; e0 += 64) total += __builtin_amdgcn_readlane(scan(cost_of(rows_of(e0))), 63);
+        const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+        int from = 0, until = 0, found = 0;
+        for (int end = 0; end < 2; ++end) {
+            const int t = (int)((int64_t)total * n_tiles * (xcd + end) / 8);
+            int cost = 0, tiles = 0, at = -1;
+            for (int e0 = 0; e0 < experts && at < 0; e0 += 64) {
+                const int c = rows_of(e0), mine = cost_of(c), n = (c + 255) >> 8, cs = cost + scan(mine), ts = tiles + scan(n);
+                const unsigned long long in = __ballot(cs * n_tiles > t);
+                if (in) {
+                    const int l = __builtin_ctzll(in), of = __builtin_amdgcn_readlane(n, l), whole = __builtin_amdgcn_readlane(mine, l);
+                    int rest = t - (__builtin_amdgcn_readlane(cs, l) - whole) * n_tiles;
+                    const int b = rest / (24 * n_tiles), high = min(4, of - 4 * b);
+                    rest -= b * 24 * n_tiles;
+                    at = (__builtin_amdgcn_readlane(ts, l) - of + 4 * b) * n_tiles + rest / min(24, whole - 24 * b) * high;
+                }
+                cost = __builtin_amdgcn_readlane(cs, 63);
+                tiles = __builtin_amdgcn_readlane(ts, 63);
+            }
+            (end ? until : from) = at < 0 ? tiles * n_tiles : at;
+        }
+        const int at = from + k;
+        if (at >= until) return;
+        int tiles = 0;
+        for (int e0 = 0; e0 < experts && !found; e0 += 64) {
+            const int n = (rows_of(e0) + 255) >> 8, ts = tiles + scan(n);
+            const unsigned long long in = __ballot(ts * n_tiles > at);
+            if (in) {
+                const int l = __builtin_ctzll(in), of = __builtin_amdgcn_readlane(n, l), i = at - (__builtin_amdgcn_readlane(ts, l) - of) * n_tiles;
+                const int b = i / (4 * n_tiles), j = i - b * 4 * n_tiles, high = min(4, of - 4 * b);
+                nt = j / high;
+                e = e0 + l;
+                m0 = a.offsets[e] + (4 * b + j % high) * 256;
+                found = 1;
+            }
+            tiles = __builtin_amdgcn_readlane(ts, 63);
+        }
     }
-    const int blk = at / (4 * n_tiles), in = at - blk * 4 * n_tiles, high = min(4, total - 4 * blk);
-    const int nt = in / high, rt = base + 4 * blk + in % high;
-    const int e = a.tiles[1 + 2 * rt], m0 = a.tiles[2 + 2 * rt], rows = __builtin_amdgcn_readfirstlane(a.offsets[e + 1] - m0), n0 = nt * 256, kb16 = a.kp >> 4;
+    const int rows = __builtin_amdgcn_readfirstlane(a.offsets[e + 1] - m0), n0 = nt * 256, kb16 = a.kp >> 4;
     HY_LDS int32_t* const to = (HY_LDS int32_t*)(lds3 + tile_lds(1, 2));      // rows of y; the barriers of the walk lie between here and the stores
     if (!UP && tid < 256) to[tid] = a.order[m0 + min(tid, rows - 1)];
     const uint32_t source = tile_packed_source(lane) * 16;
@@ -295,7 +328,7 @@ __global__ __launch_bounds__(512) void grouped_big_kernel(GroupedArgs a, int n_t
 }
 
 template <bool UP>
-static int launch_big(const GroupedArgs& a, int most, int experts, hipStream_t s) {
+static int launch_big(const GroupedArgs& a, int rows, int experts, hipStream_t s) {
     constexpr int LDS = tile_lds(1, 2) + 1024;
     static_assert(tile_lds(2, 2) <= tile_lds(1, 2) && LDS <= 163840, "both forms fit");
     static bool opted_in[64] = {};
@@ -306,7 +339,8 @@ static int launch_big(const GroupedArgs& a, int most, int experts, hipStream_t s
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) opted_in[dev] = true;
     }
-    const int n_tiles = (a.np + 255) / 256, blocks = 8 * (most * n_tiles / 8 + 2);
+    // A run has no more workgroups than its cost / 4 and the tiles of a column; the cost of all is at most 6 per 256 rows and 4 per expert.
+    const int n_tiles = (a.np + 255) / 256, blocks = 8 * ((int)((int64_t)(6 * (rows / 256) + 4 * (experts < rows ? experts : rows) + 6) * n_tiles / 32) + 8);
     hipLaunchKernelGGL((grouped_big_kernel<UP>), dim3(blocks), dim3(512), LDS, s, a, n_tiles, experts);
     return 0;
 }
@@ -339,7 +373,7 @@ extern "C" int trimkv_moe_plan(const int32_t* ids, int rows, int experts, int ti
     const char* fn = "trimkv_moe_plan";
     if (!ids || !order || !offsets || !tiles) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (rows <= 0 || experts <= 0 || experts > ROUTE_MAX_E || tile <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: bad sizes rows=%d experts=%d tile=%d", fn, rows, experts, tile);
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), (3 * experts + 1) * sizeof(int32_t), (hipStream_t)stream, ids, rows, experts, tile, order, offsets, tiles);
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 2 * experts * sizeof(int32_t), (hipStream_t)stream, ids, rows, experts, tile, order, offsets, tiles);
     return launch_status(fn);
 }
 
@@ -357,7 +391,7 @@ extern "C" int trimkv_moe_gemm(const void* x, int64_t x_stride, const void* w, v
     const int most = rows < experts ? rows : (rows - experts) / tile + experts;     // no more row tiles than this
     const dim3 grid(most, n_padded / 64);
     if (tile == 256) {
-        const int rc = up ? launch_big<true>(a, most, experts, s) : launch_big<false>(a, most, experts, s);
+        const int rc = up ? launch_big<true>(a, rows, experts, s) : launch_big<false>(a, rows, experts, s);
         if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
     } else if (dtype == TRIMKV_BF16) {
         const dim3 g(most, n_padded / 32);
