@@ -316,6 +316,24 @@ def test_experts_of_either_tile_height(ff, width):
     close(y[:, :width], want, 1.2e-2)      # hidden values and outputs rounded to bf16 once each, as above
 
 
+@pytest.mark.parametrize("rows,E,tile", [(2048, 5, 32), (2049, 5, 32), (10007, 300, 256), (32767, 64, 256), (33001, 1, 256), (70001, 1024, 16)])
+def test_plan_by_several_workgroups(rows, E, tile):
+    """Rows just within and beyond a workgroup's, in chunks that end within a round of loads, and more chunks than workgroups."""
+    from trimkv_amd import _lib
+    ids = torch.randint(0, E, (rows,), generator=torch.Generator().manual_seed(rows)).int()
+    ids[ids == E // 2] = 0                                  # an expert without rows, unless it is the only one
+    most, dev_ids = (rows - E) // tile + E, ids.to(DEV)
+    order, offsets, tiles = (torch.full((n,), -1, dtype=torch.int32, device=DEV) for n in (rows, E + 1, 1 + 2 * most))
+    assert _lib.load_hybrid("moe").trimkv_moe_plan(dev_ids.data_ptr(), rows, E, tile, order.data_ptr(), offsets.data_ptr(), tiles.data_ptr(),
+                                                   _lib.current_stream(dev_ids.device)) == 0
+    counts = torch.bincount(ids.long(), minlength=E)
+    order, offsets, tiles = order.cpu().long(), offsets.cpu().long(), tiles.cpu().tolist()
+    assert torch.equal(order.sort().values, torch.arange(rows)) and torch.equal(offsets.diff(), counts) and offsets[0] == 0
+    assert torch.equal(ids[order].long(), torch.repeat_interleave(torch.arange(E), counts))
+    want = [v for e in range(E) for r in range(0, int(counts[e]), tile) for v in (e, int(offsets[e]) + r)]
+    assert tiles[0] == len(want) // 2 and tiles[1:1 + len(want)] == want
+
+
 @pytest.mark.parametrize("E,ff,width", [(1, 2560, 64), (64, 64, 576), (65, 320, 64), (150, 64, 320)])
 def test_experts_cut_into_runs(E, ff, width):
     """As many experts as a wavefront has lanes, more of them and a single one, most of them with a few rows or none beside some with
