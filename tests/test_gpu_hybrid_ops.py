@@ -1,4 +1,6 @@
 """The mechanisms of the hybrid decoders one by one against the plain oracle (oracle/hybrid_ref.py), on the GPU."""
+import math
+
 import pytest
 import torch
 
@@ -227,6 +229,38 @@ def test_mlstm_segments_side_by_side(dtype):
     run_mlstm(s, dtype, [1100, 70, 513], [[1100], [70], [513]], f_shift=5.0)
     run_mlstm(s, dtype, [1400], [[30, 1300] + [1] * 70], f_shift=6.0)
     run_mlstm(s, dtype, [1100], [[512, 580, 8]], f_shift=6.0)
+
+
+@pytest.mark.parametrize("H,D,Dv,lens", [(2, 128, 64, [128, 7]), (2, 128, 64, [193, 449, 64]), (3, 20, 68, [700, 320]), (1, 256, 136, [129]), (8, 128, 256, [511, 300])])
+def test_mlstm_fp32_segments_against_one_chain(H, D, Dv, lens):
+    """fp32 portions of two chunks and from three on, segments of one chunk and of several, the last of them short or missing: the same as the
+    one chain that runs without a workspace, also from a state that is there already and with a value that is not finite."""
+    from trimkv_amd import _lib
+    lib, B, T, width = _lib.load_hybrid("mlstm"), len(lens), sum(lens), 2 * H * D + H * Dv
+    need = lib.trimkv_mlstm_workspace(B, max(lens), H, D, Dv, _lib.F32)
+    assert (need > 0) == (max(lens) > 2 * (64 if D <= 128 else 32))
+    proj, gates, ib, fb = rnd(T, width, seed=1).to(DEV), rnd(T, 2 * H, seed=2).to(DEV), rnd(H, seed=3).to(DEV), (4 + rnd(H, seed=4)).to(DEV)
+    bad = lens[0] - 40                                          # of head 0 and sequence 0, in its last segment
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(DEV)
+    slots = torch.arange(B, 0, -1, dtype=torch.int32, device=DEV)
+    seen = torch.tensor([0, 0] + [9, 1] * B, dtype=torch.int32, device=DEV)
+    seen[2 * B] = 0                                             # sequence 0 is fresh
+    for value in (None, math.inf, math.nan):
+        if value is not None:
+            proj[bad, 2 * H * D + 3] = value
+        got = []
+        for floats in (0, need):
+            S, nm, o = rnd(B + 1, H, D, Dv, seed=5).to(DEV), rnd(2, B + 1, H, D + 1, seed=6).to(DEV), torch.zeros(T, H, Dv, device=DEV)
+            ws = torch.full((floats,), math.nan, device=DEV) if floats else None
+            assert lib.trimkv_mlstm(proj.data_ptr(), width, 0, H * D, 2 * H * D, gates.data_ptr(), ib.data_ptr(), fb.data_ptr(), 9.0, S.data_ptr(), nm.data_ptr(),
+                                    cu.data_ptr(), slots.data_ptr(), seen.data_ptr(), o.data_ptr(), B, max(lens), H, D, Dv, B + 1, D ** -0.5, _lib.ptr(ws), _lib.F32,
+                                    _lib.current_stream(proj.device)) == 0
+            got.append((o, S[1:], nm[:, 1:]))
+        for one, cut in zip(*got):
+            assert torch.equal(one.isfinite(), cut.isfinite())
+            one, cut = one.nan_to_num(0, 0, 0).double(), cut.nan_to_num(0, 0, 0).double()
+            assert (one - cut).norm() <= 4e-6 * one.norm()      # sums of 2^-24 terms whose order differs, over chunks of 64
+        assert value is None or (not got[1][0][bad, 0, 3].isfinite() and got[1][0][:bad].isfinite().all())
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

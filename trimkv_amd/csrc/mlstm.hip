@@ -12,6 +12,7 @@
 //   mlstm_chunk_kernel      prompts in bf16 on the matrix cores, 64 tokens at a time
 //   mlstm_chunk_f32_kernel  the same in fp32
 #include "hybrid.hip.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace trimkv {
@@ -508,8 +509,10 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
 // 16 x + 4 g + r, in which the accumulators of S are an operand as they are and an A operand is four consecutive floats in LDS.
 // LDS rows are a multiple of 16 plus 4 floats apart, so that reads along rows and down columns fall on different banks.
 //
-// Bound by the serial chain of chunks (16 us each at 128 features, 6 us of which are products).  300 + 511 tokens of 8 heads of
-// 128 x 256: 129 us; token by token 1314 us (2.6 us a token).
+// Bound by the serial chain of chunks (16 us each at 128 features, 6 us of which are products) on too few workgroups.  Where that
+// leaves enough chunks side by side they are cut into segments as in bf16, as many as there are compute units for (two workgroups do
+// not fit one): every segment's own state, the join, the outputs.  us in one chain | in segments, 8 heads of 128 x 256: 300 + 511 tokens 127 | 68 (four segments), 511 126 | 46 (eight), 256
+// 65 | 41, three sequences of 600 (two segments) 160 | 129; 4 heads of 64 x 128 and 1000 tokens 161 | 33.  Token by token 1314 us.
 // A value that is not finite must not reach earlier tokens of its chunk through 0 x inf: such chunks take the products of the
 // diagonal blocks one token at a time.
 template <int DT, int TC>
@@ -524,8 +527,13 @@ __device__ __forceinline__ double shfl_up_d(double v, int d) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-template <int DT, int TC>
-__global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
+// A number in double among floats
+__device__ __forceinline__ double load_double(const float* p) { double x; __builtin_memcpy(&x, p, 8); return x; }
+__device__ __forceinline__ void store_double(float* p, double x) { __builtin_memcpy(p, &x, 8); }
+
+template <int DT, int TC, int MODE>
+__global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(ChunkArgs ca) {
+    const MlstmArgs& a = ca.a;
     using C = F32Cfg<DT, TC>;
     constexpr int DB = DT / 16, TB = TC / 16, LD = C::LD, LV = C::LV, LW = C::LW, QL = TC * DT / 1024, VL = TC * 64 / 1024;
     extern __shared__ __attribute__((aligned(16))) float cf_lds[];
@@ -534,17 +542,20 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
     int* const odd = (int*)(den + TC);                // chunk + 1 whose values were not all finite
     double* const gD = (double*)(cf_lds + C::G0); double* const gM = gD + TC; double* const gm = gM + TC;           // d_s, M_t; m_0 and F_C
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, b = blockIdx.z, col0 = blockIdx.x * 64, col = col0 + w * 16 + c;
-    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, slot = a.slots[b];
-    if (len <= 0) {                                   // workgroup-uniform: there is no token to request
-        if (blockIdx.x == 0) carry_norm(a, h, slot);
+    const int vt = (a.Dv + 63) / 64, seg = MODE == CHUNK_WHOLE ? 0 : blockIdx.x / vt, first = MODE == CHUNK_WHOLE ? 0 : seg * ca.seg_len;
+    const int h = blockIdx.y, b = blockIdx.z, col0 = ((int)blockIdx.x - seg * vt) * 64, col = col0 + w * 16 + c;
+    const int t0 = a.cu[b] + first, rest = a.cu[b + 1] - t0, len = MODE == CHUNK_WHOLE ? rest : min(rest, ca.seg_len), slot = a.slots[b];
+    if (len <= 0) {                                   // workgroup-uniform: there is no token to request (segments: the join carries n and m)
+        if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
         return;
     }
+    const int64_t sat = ((int64_t)b * a.H + h) * ca.nseg + seg;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
-    const float* nm_in = a.nm + parity * copy + at;
-    float* Sp = a.S + ((int64_t)slot * a.H + h) * a.D * a.Dv;
+    const bool zero = MODE == CHUNK_LOCAL || (MODE == CHUNK_WHOLE && fresh);
+    const float* n_in = MODE == CHUNK_OUTPUT ? ca.seg_n + sat * a.D : a.nm + parity * copy + at;
+    float* Sp = MODE == CHUNK_WHOLE ? a.S + ((int64_t)slot * a.H + h) * a.D * a.Dv : ca.seg_S + sat * a.D * a.Dv;
     hy_u32x4 qn[QL], kn[QL], vn[VL];
     float zi, zf;                                     // raw gates, lane = token
     auto fetch = [&](int ch) __attribute__((always_inline)) {
@@ -556,7 +567,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
             const int p = x * 256 + tid, r = p / (DT / 4), e = (p % (DT / 4)) * 4;
             const float* row = (const float*)a.p + (int64_t)(t0 + min(ch * TC + r, len - 1)) * a.p_stride + h * a.D;
             // loads are unconditional (a load under a branch is waited for on the spot); what is not there becomes zero
-            qn[x] = *(const hy_u32x4*)(row + a.q_off + min(e, a.D - 4));
+            if (MODE != CHUNK_LOCAL) qn[x] = *(const hy_u32x4*)(row + a.q_off + min(e, a.D - 4));
             kn[x] = *(const hy_u32x4*)(row + a.k_off + min(e, a.D - 4));
         }
 #pragma unroll
@@ -572,13 +583,14 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int d = 16 * x + 4 * g + r;
-            const float old = Sp[(int64_t)min(d, a.D - 1) * a.Dv + min(col, a.Dv - 1)];
-            S[x][r] = fresh || d >= a.D || col >= a.Dv ? 0.0f : old;
+            const float old = MODE == CHUNK_LOCAL ? 0.0f : Sp[(int64_t)min(d, a.D - 1) * a.Dv + min(col, a.Dv - 1)];
+            S[x][r] = zero || d >= a.D || col >= a.Dv ? 0.0f : old;
         }
-    for (int d = tid; d < DT; d += 256) n[d] = fresh || d >= a.D ? 0.0f : nm_in[d];
-    if (tid == 0) { *odd = 0; gm[0] = fresh ? 0.0 : (double)nm_in[a.D]; }
+    for (int d = tid; d < DT; d += 256) n[d] = zero || d >= a.D ? 0.0f : n_in[d];
+    if (tid == 0) { *odd = 0; gm[0] = MODE == CHUNK_LOCAL ? -1.0e30 : MODE == CHUNK_OUTPUT ? load_double(ca.seg_m + 2 * sat) : fresh ? 0.0 : (double)n_in[a.D]; }
     const float ib = a.ib[h], fb = a.fb[h];
     const int nchunks = (len + TC - 1) / TC;
+    double gates = 0.0;                               // sum of the segment's f (thread 0)
     for (int ch = 0; ch < nchunks; ++ch) {
         const int base = ch * TC, rows = min(TC, len - base);
         __syncthreads();                              // the last chunk is done with
@@ -586,8 +598,10 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
 #pragma unroll
         for (int x = 0; x < QL; ++x) {
             const int p = x * 256 + tid, r = p / (DT / 4), e = (p % (DT / 4)) * 4;
-            const float4 qq = __builtin_bit_cast(float4, kept4(qn[x], e < a.D));
-            *(float4*)(q + r * LD + e) = make_float4(qq.x * a.qscale, qq.y * a.qscale, qq.z * a.qscale, qq.w * a.qscale);
+            if (MODE != CHUNK_LOCAL) {
+                const float4 qq = __builtin_bit_cast(float4, kept4(qn[x], e < a.D));
+                *(float4*)(q + r * LD + e) = make_float4(qq.x * a.qscale, qq.y * a.qscale, qq.z * a.qscale, qq.w * a.qscale);
+            }
             *(hy_u32x4*)(k + r * LD + e) = kept4(kn[x], e < a.D && r < rows);
         }
 #pragma unroll
@@ -621,7 +635,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
         if (ch + 1 < nchunks) fetch(ch + 1);
         const double MC = gM[TC - 1];
         // weighted scores of the blocks s <= t, transposed: column t, rows s
-        for (int x = w; x < TB * (TB + 1) / 2; x += 4) {
+        for (int x = w; MODE != CHUNK_LOCAL && x < TB * (TB + 1) / 2; x += 4) {
             int tb = 0, sb = x;
             while (sb > tb) { ++tb; sb -= tb; }
             hy_f32x4 p = {0.f, 0.f, 0.f, 0.f};
@@ -642,7 +656,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
         }
         if (tid >= 256 - TC) end[tid - (256 - TC)] = expf((float)(gD[tid - (256 - TC)] - MC));
         __syncthreads();
-        {                                             // n.q of every token: 256 / TC threads share one
+        if (MODE != CHUNK_LOCAL) {                    // n.q of every token: 256 / TC threads share one
             constexpr int SH = 256 / TC;
             const int t = tid / SH, x = tid % SH;
             float old = 0.0f, own = 0.0f;
@@ -657,7 +671,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
         }
         hy_f32x4 o[TB];
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb) {             // S_0^T q
+        for (int tb = 0; MODE != CHUNK_LOCAL && tb < TB; ++tb) {      // S_0^T q
             o[tb] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
             const float* qr = q + (tb * 16 + c) * LD + 4 * g;
 #pragma unroll
@@ -671,6 +685,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
             const float4 f = *(const float4*)(carry + tb * 16 + 4 * g);
             o[tb][0] *= f.x; o[tb][1] *= f.y; o[tb][2] *= f.z; o[tb][3] *= f.w;
         }
+        const bool on = MODE != CHUNK_OUTPUT || ch + 1 < nchunks;     // the state behind the segment's last chunk is the join's
         const float keep = expf((float)(gm[0] - MC));
 #pragma unroll
         for (int x = 0; x < DB; ++x) S[x] *= keep;
@@ -683,7 +698,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) vv[r] = v[(sb * 16 + 4 * g + r) * LV + w * 16 + c];
 #pragma unroll
-            for (int tb = sb; tb < TB; ++tb) {
+            for (int tb = sb; MODE != CHUNK_LOCAL && tb < TB; ++tb) {
                 if (tb > sb || plain) {
                     const float4 f = *(const float4*)(wt + (tb * 16 + c) * LW + sb * 16 + 4 * g);
                     o[tb] = mfma16_f32(f.x, vv[0], o[tb]);
@@ -698,7 +713,7 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; on && r < 4; ++r) {
                 const float f = vv[r] * ee[r];
                 const float* kr = k + (sb * 16 + 4 * g + r) * LD + c;
 #pragma unroll
@@ -706,12 +721,12 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
             }
         }
         __syncthreads();                              // denominators are there, n.q has been taken
-        for (int d = tid; d < DT; d += 256) {
+        for (int d = tid; on && d < DT; d += 256) {
             float x = n[d] * keep;
             for (int s = 0; s < rows; ++s) x += end[s] * k[s * LD + d];
             n[d] = x;
         }
-        if (col < a.Dv) {
+        if (MODE != CHUNK_LOCAL && col < a.Dv) {
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb)
 #pragma unroll
@@ -720,8 +735,9 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
                     if (t < rows) ((float*)a.o)[((int64_t)(t0 + base + t) * a.H + h) * a.Dv + col] = o[tb][r] * den[t];
                 }
         }
-        if (tid == 0) gm[0] = gm[1] + MC;             // read again behind the next barrier
+        if (tid == 0) { gates += gm[1]; gm[0] = gm[1] + MC; }         // read again behind the next barrier
     }
+    if (MODE == CHUNK_OUTPUT) return;
     __syncthreads();
     if (col < a.Dv) {
 #pragma unroll
@@ -732,26 +748,85 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(MlstmArgs a) {
                 if (d < a.D) Sp[(int64_t)d * a.Dv + col] = S[x][r];
             }
     }
-    if (blockIdx.x == 0) {
-        float* nm_out = a.nm + (1 - parity) * copy + at;
-        for (int d = tid; d < a.D; d += 256) nm_out[d] = n[d];
-        if (tid == 0) nm_out[a.D] = (float)gm[0];
+    if (col0 == 0) {
+        float* n_out = MODE == CHUNK_LOCAL ? ca.seg_n + sat * a.D : a.nm + (1 - parity) * copy + at;
+        for (int d = tid; d < a.D; d += 256) n_out[d] = n[d];
+        if (tid == 0) {
+            if (MODE == CHUNK_LOCAL) { store_double(ca.seg_g + 4 * sat, gates); store_double(ca.seg_g + 4 * sat + 2, gm[0]); }
+            else n_out[a.D] = (float)gm[0];
+        }
     }
 }
 
-template <int DT, int TC>
-static int launch_chunk_f32(const MlstmArgs& a, int batch, hipStream_t s) {
+// mlstm_join_kernel for these segments: sums of f and stabilisers in double (seg_g: 2, seg_m: 1), natural logarithms.  It is bound by memory
+// (5 us for 8 heads of 128 x 256 and two sequences of four segments), so that sums in double cost nothing.
+__global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca) {
+    const MlstmArgs& a = ca.a;
+    const int h = blockIdx.y, b = blockIdx.z, len = a.cu[b + 1] - a.cu[b], slot = a.slots[b];
+    const int e = (blockIdx.x * 256 + threadIdx.x) * 4, nS = a.D * a.Dv;        // D and Dv are multiples of 4
+    if (e >= nS + a.D) return;
+    const bool fresh = a.seen[2 * slot] == 0;
+    const int parity = a.seen[2 * slot + 1] & 1;
+    const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
+    const float* in = a.nm + parity * copy + at;
+    float* S = a.S + ((int64_t)slot * a.H + h) * nS;
+    double m = fresh ? 0.0 : (double)in[a.D];
+    double cur[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) cur[x] = fresh ? 0.0 : (double)(e < nS ? S[e + x] : in[e - nS + x]);
+    const int64_t s0 = ((int64_t)b * a.H + h) * ca.nseg;
+    for (int s = 0; s < ca.nseg && s * ca.seg_len < len; ++s) {
+        float* p = e < nS ? ca.seg_S + (s0 + s) * nS + e : ca.seg_n + (s0 + s) * a.D + (e - nS);
+        const double f = load_double(ca.seg_g + 4 * (s0 + s)), ms = load_double(ca.seg_g + 4 * (s0 + s) + 2), mn = fmax(f + m, ms);
+        const double old = exp(f + m - mn), now = exp(ms - mn);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const float own = p[x];
+            p[x] = (float)cur[x];
+            cur[x] = old * cur[x] + now * own;
+        }
+        if (e == 0) store_double(ca.seg_m + 2 * (s0 + s), m);
+        m = mn;
+    }
+    float* out = a.nm + (1 - parity) * copy + at;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+        if (e < nS) S[e + x] = (float)cur[x]; else out[e - nS + x] = (float)cur[x];
+    if (e == 0) out[a.D] = (float)m;
+}
+
+template <int DT, int TC, int MODE>
+static int launch_chunk_f32(const ChunkArgs& c, dim3 grid, hipStream_t s) {
     constexpr int LDS = F32Cfg<DT, TC>::LDS;
     static bool opted_in[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
     if (dev < 0 || !opted_in[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)mlstm_chunk_f32_kernel<DT, TC>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        hipError_t e = hipFuncSetAttribute((const void*)mlstm_chunk_f32_kernel<DT, TC, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) opted_in[dev] = true;
     }
-    hipLaunchKernelGGL((mlstm_chunk_f32_kernel<DT, TC>), dim3((a.Dv + 63) / 64, a.H, batch), dim3(256), LDS, s, a);
+    hipLaunchKernelGGL((mlstm_chunk_f32_kernel<DT, TC, MODE>), grid, dim3(256), LDS, s, c);
     return 0;
+}
+template <int DT, int TC>
+static int launch_chunked_f32(const ChunkArgs& c, int batch, hipStream_t s) {
+    const MlstmArgs& a = c.a;
+    const int vt = (a.Dv + 63) / 64;
+    if (c.nseg == 1) return launch_chunk_f32<DT, TC, CHUNK_WHOLE>(c, dim3(vt, a.H, batch), s);
+    if (int rc = launch_chunk_f32<DT, TC, CHUNK_LOCAL>(c, dim3(vt * c.nseg, a.H, batch), s)) return rc;
+    hipLaunchKernelGGL(mlstm_join_f32_kernel, dim3((a.D * a.Dv + a.D + 1023) / 1024, a.H, batch), dim3(256), 0, s, c);
+    return launch_chunk_f32<DT, TC, CHUNK_OUTPUT>(c, dim3(vt * c.nseg, a.H, batch), s);
+}
+static int chunk_f32_tokens(int dim) { return dim <= 128 ? 64 : 32; }
+// A segment of c chunks costs 24 us per chunk in its two passes and 20 for the join and the launches, a chain 16 per chunk.  Measured, chain | segments: 4
+// chunks in segments of one 65 | 41, of two 71 | 74; 10 in segments of five 160 | 129.
+static int chunk_f32_segments(int batch, int max_len, int heads, int dim, int vdim) {
+    const int64_t wgs = (int64_t)batch * heads * ((vdim + 63) / 64);
+    const int chunks = (max_len + chunk_f32_tokens(dim) - 1) / chunk_f32_tokens(dim), n = (int)std::min<int64_t>(256 / wgs, chunks);
+    if (n < 2) return 1;
+    const int of = (chunks + n - 1) / n;
+    return 6 * of + 5 < 4 * chunks ? (chunks + of - 1) / of : 1;
 }
 // Portions of a few tokens stay with the token-by-token kernel: a chunk costs 16 us however few tokens it holds, a token 2.6 us.
 constexpr int F32_CHUNK_FROM = 8;
@@ -801,7 +876,12 @@ using namespace trimkv;
 extern "C" const char* trimkv_mlstm_last_error(void) { return err_buf(); }
 
 extern "C" int64_t trimkv_mlstm_workspace(int batch, int max_len, int heads, int dim, int vdim, int dtype) {
-    if (batch <= 0 || max_len <= 1 || heads <= 0 || dim <= 0 || vdim <= 0 || dtype != TRIMKV_BF16) return 0;
+    if (batch <= 0 || max_len <= 1 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
+    if (dtype == TRIMKV_F32) {
+        const int n = chunk_f32_segments(batch, max_len, heads, dim, vdim);
+        return n == 1 || dim > 256 || dim % 4 || vdim % 4 ? 0 : (int64_t)batch * heads * n * ((int64_t)dim * vdim + dim + 6);
+    }
+    if (dtype != TRIMKV_BF16) return 0;
     const int n = chunk_segments(batch, max_len, heads, vdim);
     return n == 1 ? 0 : (int64_t)batch * heads * n * ((int64_t)dim * vdim + dim + 3);
 }
@@ -837,7 +917,15 @@ extern "C" int trimkv_mlstm(const void* proj, int64_t proj_stride, int q_off, in
         return launch_status(fn);
     }
     if (chunk_f32_fits(a, dtype, max_len)) {
-        const int rc = dim <= 64 ? launch_chunk_f32<64, 64>(a, batch, s) : dim <= 128 ? launch_chunk_f32<128, 64>(a, batch, s) : launch_chunk_f32<256, 32>(a, batch, s);
+        ChunkArgs c{a};
+        c.nseg = workspace ? chunk_f32_segments(batch, max_len, heads, dim, vdim) : 1;
+        if (c.nseg > 1) {
+            const int tc = chunk_f32_tokens(dim);
+            c.seg_len = ((max_len + tc - 1) / tc + c.nseg - 1) / c.nseg * tc;
+            const int64_t n = (int64_t)batch * heads * c.nseg;
+            c.seg_S = workspace; c.seg_n = c.seg_S + n * dim * vdim; c.seg_g = c.seg_n + n * dim; c.seg_m = c.seg_g + 4 * n;
+        }
+        const int rc = dim <= 64 ? launch_chunked_f32<64, 64>(c, batch, s) : dim <= 128 ? launch_chunked_f32<128, 64>(c, batch, s) : launch_chunked_f32<256, 32>(c, batch, s);
         if (rc) return fail(rc, "%s: hipFuncSetAttribute failed (%d)", fn, rc);
         return launch_status(fn);
     }
