@@ -152,6 +152,35 @@ def test_window_edges_stand_out(name, dtype, how):
         run_window(s, dtype, [n], [cuts], stand_out=[(0, qi, kj)])
 
 
+@pytest.mark.parametrize("spec,seqs,cuts", [
+    ((48, 1, 32, 40, 40, 3, 0.2), [150, 33], [[90, 60], [33]]),                  # more heads to a KV head than 32 rows hold
+    ((32, 1, 64, 64, 70, 0, 0.1), [131, 64], [[65, 66], [64]]),                  # one time to 32 rows
+    ((5, 1, 128, 100, 64, 10, 0.1), [200, 1, 63], [[7, 193], [1], [31, 32]]),    # rows of a workgroup that are nobody's, part of a ring's only tile
+    ((2, 2, 36, 128, 200, 64, 0.15), [700], [[300, 200, 200]]),                  # a ring that has gone round
+    ((8, 8, 12, 8, 90, 5, 0.3), [577] + [200 - 9 * i for i in range(8)], [[300, 277]] + [[100, 100 - 9 * i] for i in range(8)]),    # 64 rows: many tiles
+])
+def test_window_fp32_rows_of_a_workgroup(spec, seqs, cuts):
+    """32 rows to a workgroup with the keys in two halves, and 64 rows, over rings and portions that end within a tile."""
+    run_window(ops.WindowSpec(*spec), torch.float32, seqs, cuts)
+
+
+@pytest.mark.parametrize("H,G,T", [(4, 2, 200), (48, 1, 130)])
+def test_window_fp32_values_that_are_not_finite(H, G, T):
+    """An infinite value reaches the rows that see its key and no other, in either half of a tile."""
+    s, D = ops.WindowSpec(H, G, 64, 64, 50, 3, 0.1), 64
+    offs = [0, H * D, (H + G) * D, (H + 2 * G) * D]
+    for at in (70, 110, T - 1):
+        proj = rnd(T, offs[3] + H * D, seed=7)
+        proj[at, offs[2]] = float("inf")
+        cache = HybridCache([s], torch.float32, DEV, num_slots=1)
+        batch = cache.batch([T], cache.allocate(1))
+        w = torch.ones(H * D, device=DEV)
+        out = ops.window_attention(proj.to(DEV), offs, w, w[:G * D], 1e-5, s, cache.layers_state[0], batch).cpu()
+        seen = torch.zeros(T, H * D, dtype=torch.bool)
+        seen[at:at + 50, [h * D for h in range(H // G)]] = True
+        assert torch.equal(~out.isfinite(), seen)
+
+
 def test_window_sensitivity_of_the_edge_test():
     """The inputs of the edge test tell windows apart: with the key just inside, a window one token shorter moves the output."""
     s = SPECS["tiny"]

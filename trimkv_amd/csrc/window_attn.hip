@@ -68,32 +68,34 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowArgs a) {
 
 // ---- fp32 prompts on the matrix cores --------------------------------------------------------------
 // A workgroup owns 64 rows (consecutive query times x the query heads of one KV head), 16 per wavefront, and walks tiles of 64
-// keys.  Both products run on 16x16x4 fp32 MFMAs, transposed: S^T = K . Q^T, O^T += V^T . P^T, so a row is a column of the
-// accumulators (lane % 16) and the probabilities a lane holds behind the first product are its operand of the second.  With
-// g = lane / 16, A and B hold k = g of row / column lane % 16 and register r of C row 4 g + r; the sums take features in the order
-// 16 x + 4 g + r and keys likewise, so that a lane reads four consecutive floats of K.  LDS rows are DT + 4 floats apart: reads of
-// either product fall on different banks.  The next tile waits in registers.
+// keys; or 32 rows, with half of every tile for two wavefronts each, whose sums are put together at the end.  Both products run on 16x16x4 fp32 MFMAs,
+// transposed: S^T = K . Q^T, O^T += V^T . P^T, so a row is a column of the accumulators (lane % 16) and the probabilities a lane
+// holds behind the first product are its operand of the second.  With g = lane / 16, A and B hold k = g of row / column lane % 16
+// and register r of C row 4 g + r; the sums take features in the order 16 x + 4 g + r and keys likewise, so that a lane reads
+// four consecutive floats of K.  LDS rows are DT + 4 floats apart: reads of either product fall on different banks.  The next
+// tile waits in registers; a tile is all of the ring or all of the portion, so that its rows are one base and a stride.
 //
-// Bound by the matrix cores' fp32 rate (a sixteenth of bf16) and, for short prompts, by the few workgroups there are.  300 + 511
-// tokens, 16 heads of 128 (8 KV heads): 70 us; a wavefront per query row, which this replaces for head sizes up to 128, took
-// 1060 us there, bound by its row-wise loads.
+// Bound by the matrix cores' fp32 rate (a sixteenth of bf16), 1.75 us a tile of 32 rows, and as much again of other vector instructions.  The longest
+// rows of all heads go first: with a head's workgroups one behind the other the launch ended on long ones, 16 heads of 128 (8 KV heads): three
+// prompts of 1000 tokens 300 us for 165, one of 4000 730 for 585.  300 + 511 tokens: 72 us with 64 rows in that order, 51 with 32; a
+// wavefront per query row, which this replaces for head sizes up to 128, took 1060 us there, bound by its row-wise loads.
 // NaNs and infinities of keys that a row does not see must not reach it through 0 x inf: tiles with such values in V take their
 // second product one key at a time.
-template <int DT>
-__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
-    constexpr int LD = DT + 4, DB = DT / 16, PIECES = DT / 4, LOADS = 64 * PIECES / 256;
+template <int DT, int ROWS>
+__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a, int heads) {      // heads: KV heads of all sequences
+    constexpr int LD = DT + 4, DB = DT / 16, PIECES = DT / 4, LOADS = 64 * PIECES / 256, RW = ROWS / 16, KS = 4 / RW, KB = 4 / KS;
     extern __shared__ __attribute__((aligned(16))) char wf_lds[];
     float* const kt = (float*)wf_lds; float* const vt = kt + 64 * LD;
     int* const where = (int*)(vt + 64 * LD);          // position of every key of the tile; past the end: beyond all queries
     int* const odd = where + 64;                      // number of tiles + 1 whose V held something that is not finite
-    const int b = blockIdx.y / a.G, g = blockIdx.y % a.G, slot = a.slots[b];
-    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, per = a.H / a.G, bt = 64 / per;
-    // later times first: they walk the most tiles
-    const int first = ((int)gridDim.x - 1 - (int)blockIdx.x) * bt;
+    const int bg = blockIdx.x % heads, b = bg / a.G, g = bg % a.G, slot = a.slots[b];
+    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, per = a.H / a.G, bt = ROWS / per;
+    // later times of all heads first: they walk the most tiles
+    const int first = (int)((gridDim.x - 1 - blockIdx.x) / heads) * bt;
     if (first >= len) return;                         // workgroup-uniform, before any barrier
     const int past = a.seen[2 * slot], cap = a.keep + a.size, nring = min(past, cap), last = min(first + bt, len) - 1;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, gr = lane >> 4;
-    const int row = w * 16 + c, t = min(first + row / per, last), h = g * per + row % per, i = past + t;
+    const int kb0 = w / RW * KB, row = w % RW * 16 + c, t = min(first + row / per, last), h = g * per + row % per, i = past + t;
     const bool live = row < bt * per && first + row / per < len;
     const float* rk = (const float*)a.rk + ((int64_t)slot * a.G + g) * cap * a.Dp;
     const float* rv = (const float*)a.rv + ((int64_t)slot * a.G + g) * cap * a.Dvp;
@@ -107,30 +109,30 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
 #pragma unroll
         for (int x = 0; x < DB; ++x) q[x] = __builtin_bit_cast(float4, kept4(__builtin_bit_cast(hy_u32x4, q[x]), 16 * x + 4 * gr < a.Dp));
     }
-    // keys in the order ring, portion; a portion's tile that no row sees is skipped
-    const int nkeys = nring + last + 1, ntiles = (nkeys + 63) / 64;
+    // tiles of the ring, then tiles of the portion; one of the portion that no row sees is skipped
+    const int rtiles = (nring + 63) / 64, ntiles = rtiles + (last + 64) / 64;
     auto next_tile = [&](int x) {
         for (; x < ntiles; ++x) {
-            const int lo = past + x * 64 - nring, hi = lo + 63;      // positions, if the tile is all portion
-            if (x * 64 < nring || hi > past + first - a.size || lo < a.keep) break;
+            const int lo = past + (x - rtiles) * 64, hi = lo + 63;   // positions, if the tile is of the portion
+            if (x < rtiles || hi > past + first - a.size || lo < a.keep) break;
         }
         return x;
     };
+    auto keys_of = [&](int x) { return min(64, x < rtiles ? nring - x * 64 : last + 1 - (x - rtiles) * 64); };
     hy_u32x4 kn[LOADS], vn[LOADS];
     int where_n = 0;
+    const int piece = tid % PIECES * 4, ek = min(piece, a.Dp - 4), ev = min(piece, a.Dvp - 4), r0 = tid / PIECES;
     auto fetch = [&](int x) __attribute__((always_inline)) {
+        const bool ring = x < rtiles;
+        const int from = ring ? x * 64 : (x - rtiles) * 64, step = ring ? 1 : a.G, end = keys_of(x) - 1;
+        const float* kb = (ring ? rk : pk) + (int64_t)from * step * a.Dp; const float* vb = (ring ? rv : pv) + (int64_t)from * step * a.Dvp;
 #pragma unroll
         for (int y = 0; y < LOADS; ++y) {
-            const int p = y * 256 + tid, r = p / PIECES, e = (p % PIECES) * 4, key = x * 64 + r;
-            // loads are unconditional (a load under a branch is waited for on the spot); what is not there becomes zero
-            const int kc = min(key, nkeys - 1), ek = min(e, a.Dp - 4), ev = min(e, a.Dvp - 4);
-            const bool ring = kc < nring;
-            const int64_t at = ring ? kc : (int64_t)(kc - nring) * a.G;
-            kn[y] = *(const hy_u32x4*)((ring ? rk : pk) + at * a.Dp + ek);
-            vn[y] = *(const hy_u32x4*)((ring ? rv : pv) + at * a.Dvp + ev);
+            const int r = min(y * (256 / PIECES) + r0, end);        // loads are unconditional (a load under a branch is waited for on the spot)
+            kn[y] = *(const hy_u32x4*)(kb + (uint32_t)(r * (step * a.Dp) + ek));
+            vn[y] = *(const hy_u32x4*)(vb + (uint32_t)(r * (step * a.Dvp) + ev));
         }
-        const int key = x * 64 + (tid & 63);
-        where_n = key >= nkeys ? 0x7fffffff : key < nring ? ring_position(key, past, a.keep, a.size) : past + key - nring;
+        where_n = lane > end ? 0x7fffffff : ring ? ring_position(from + lane, past, a.keep, a.size) : past + from + lane;
     };
     hy_f32x4 o[DB];
 #pragma unroll
@@ -142,13 +144,13 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
     while (tile < ntiles) {
         __syncthreads();                              // the last tile is done with
         bool fine = true;
+        const int here = keys_of(tile);
 #pragma unroll
-        for (int y = 0; y < LOADS; ++y) {
-            const int p = y * 256 + tid, r = p / PIECES, e = (p % PIECES) * 4;
-            const bool in = tile * 64 + r < nkeys;
-            const hy_u32x4 vv = kept4(vn[y], in && e < a.Dvp);
-            *(hy_u32x4*)(kt + r * LD + e) = kept4(kn[y], in && e < a.Dp);
-            *(hy_u32x4*)(vt + r * LD + e) = vv;
+        for (int y = 0; y < LOADS; ++y) {             // what is not there becomes zero
+            const int r = y * (256 / PIECES) + r0;
+            const hy_u32x4 vv = kept4(vn[y], r < here && piece < a.Dvp);
+            *(hy_u32x4*)(kt + r * LD + piece) = kept4(kn[y], r < here && piece < a.Dp);
+            *(hy_u32x4*)(vt + r * LD + piece) = vv;
             fine = fine && finite_bits(vv);
         }
         if (tid < 64) where[tid] = where_n;
@@ -157,21 +159,35 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
         const int now = tile;
         tile = next_tile(tile + 1);
         if (tile < ntiles) fetch(tile);
-        hy_f32x4 s[4];
+        hy_f32x4 s[KB];
         float top = WA_NEG;
+        {                                             // fragments of K are read one step of 16 features ahead
+            const float* kr = kt + (kb0 * 16 + c) * LD + 4 * gr;
+            float4 f[2][KB];
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            s[kb] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
-            const float* kr = kt + (kb * 16 + c) * LD + 4 * gr;
+            for (int kb = 0; kb < KB; ++kb) {
+                s[kb] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
+                f[0][kb] = *(const float4*)(kr + kb * 16 * LD);
+            }
 #pragma unroll
             for (int x = 0; x < DB; ++x) {
-                const float4 f = *(const float4*)(kr + 16 * x);
-                s[kb] = mfma16_f32(f.x, q[x].x, s[kb]);
-                s[kb] = mfma16_f32(f.y, q[x].y, s[kb]);
-                s[kb] = mfma16_f32(f.z, q[x].z, s[kb]);
-                s[kb] = mfma16_f32(f.w, q[x].w, s[kb]);
+                if (x + 1 < DB) {
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb) f[~x & 1][kb] = *(const float4*)(kr + kb * 16 * LD + 16 * (x + 1));
+                }
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb) {
+                        const float4 g4 = f[x & 1][kb];
+                        s[kb] = mfma16_f32(y == 0 ? g4.x : y == 1 ? g4.y : y == 2 ? g4.z : g4.w, y == 0 ? q[x].x : y == 1 ? q[x].y : y == 2 ? q[x].z : q[x].w, s[kb]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            const int4 at = *(const int4*)(where + kb * 16 + 4 * gr);
+        }
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            const int4 at = *(const int4*)(where + (kb0 + kb) * 16 + 4 * gr);
             const int pos[4] = {at.x, at.y, at.z, at.w};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -185,34 +201,40 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
         m = mn;
         l *= alpha;
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) { s[kb][r] = exp2f(s[kb][r] - mn); l += s[kb][r]; }
 #pragma unroll
         for (int x = 0; x < DB; ++x) o[x] *= alpha;
         if (*odd != now + 1) {
+            const float* vr = vt + (kb0 * 16 + 4 * gr) * LD + c;       // one key ahead, as above
+            float f[2][DB];
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
+            for (int x = 0; x < DB; ++x) f[0][x] = vr[16 * x];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float* vr = vt + (kb * 16 + 4 * gr + r) * LD + c;
+            for (int y = 0; y < 4 * KB; ++y) {
+                if (y + 1 < 4 * KB) {
 #pragma unroll
-                    for (int x = 0; x < DB; ++x) o[x] = mfma16_f32(vr[16 * x], s[kb][r], o[x]);
+                    for (int x = 0; x < DB; ++x) f[~y & 1][x] = vr[((y + 1) / 4 * 16 + (y + 1) % 4) * LD + 16 * x];
                 }
+#pragma unroll
+                for (int x = 0; x < DB; ++x) o[x] = mfma16_f32(f[y & 1][x], s[y / 4][y % 4], o[x]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         } else {                                      // workgroup-uniform: the keys' place takes the probabilities
             __syncthreads();
-            float* const ps = kt + w * 1024;          // [key][row]
+            float* const ps = kt + w * (KB * 256);    // [key][row]
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
+            for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) ps[(kb * 16 + 4 * gr + r) * 16 + c] = s[kb][r];
             __syncthreads();
 #pragma unroll 1
-            for (int key = 0; key < 64; ++key) {
+            for (int key = 0; key < KB * 16; ++key) {
                 const float p = ps[key * 16 + c];
 #pragma unroll
                 for (int x = 0; x < DB; ++x) {
-                    const float4 f = *(const float4*)(vt + key * LD + 16 * x + 4 * gr);
+                    const float4 f = *(const float4*)(vt + (kb0 * 16 + key) * LD + 16 * x + 4 * gr);
                     o[x][0] += p == 0.0f ? 0.0f : p * f.x;
                     o[x][1] += p == 0.0f ? 0.0f : p * f.y;
                     o[x][2] += p == 0.0f ? 0.0f : p * f.z;
@@ -223,6 +245,28 @@ __global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a) {
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if constexpr (KS == 2) {                          // the wavefronts of the first keys take the others' sums
+        hy_f32x4* const po = (hy_f32x4*)kt + w % RW * (DB * 64) + lane;
+        float2* const pm = (float2*)vt + w % RW * 64 + lane;
+        __syncthreads();
+        if (w >= RW) {
+#pragma unroll
+            for (int x = 0; x < DB; ++x) po[x * 64] = o[x];
+            *pm = make_float2(m, l);
+        }
+        __syncthreads();
+        if (w >= RW) return;
+        const float2 other = *pm;
+        const float mn = fmaxf(m, other.x), ours = exp2f(m - mn), theirs = exp2f(other.x - mn);
+        m = mn;
+        l = (ours == 0.0f ? 0.0f : l * ours) + (theirs == 0.0f ? 0.0f : other.y * theirs);
+#pragma unroll
+        for (int x = 0; x < DB; ++x) {
+            const hy_f32x4 f = po[x * 64];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[x][r] = (ours == 0.0f ? 0.0f : o[x][r] * ours) + (theirs == 0.0f ? 0.0f : f[r] * theirs);
+        }
+    }
     if (!live) return;
     const float inv = 1.0f / (l + window_sink(a, m));
     float* out = (float*)a.out + ((int64_t)(t0 + t) * a.H + h) * a.Dv;
@@ -513,20 +557,31 @@ static int launch_window_prefill(const WindowArgs& a, int batch, int max_len, hi
     return 0;
 }
 
-template <int DT>
-static int launch_window_prefill_f32(const WindowArgs& a, int batch, int max_len, hipStream_t s) {
+template <int DT, int ROWS>
+static int launch_window_rows_f32(const WindowArgs& a, int batch, int max_len, hipStream_t s) {
     constexpr int LDS = (2 * 64 * (DT + 4) + 64 + 4) * 4;
     static bool opted_in[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
     if (dev < 0 || !opted_in[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void*)window_prefill_f32_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        hipError_t e = hipFuncSetAttribute((const void*)window_prefill_f32_kernel<DT, ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) return (int)e;
         if (dev >= 0) opted_in[dev] = true;
     }
-    const int bt = 64 / (a.H / a.G);
-    hipLaunchKernelGGL((window_prefill_f32_kernel<DT>), dim3((max_len + bt - 1) / bt, batch * a.G), dim3(256), LDS, s, a);
+    const int bt = ROWS / (a.H / a.G);
+    hipLaunchKernelGGL((window_prefill_f32_kernel<DT, ROWS>), dim3((max_len + bt - 1) / bt * batch * a.G), dim3(256), LDS, s, a, batch * a.G);
     return 0;
+}
+
+// 32 rows to a workgroup while 64 would leave compute units without a second one.  us with 32 | 64 rows, 8 KV heads of 128 with two
+// query heads each: 600 tokens (152 workgroups of 64 rows) 55 | 73, 300 + 511 (256) 51 | 64, three times 600 (456) 85 | 94, three times 1000 (768) 187 | 165,
+// three times 2000 627 | 552.
+constexpr int F32_HALF_ROWS = 512;
+template <int DT>
+static int launch_window_prefill_f32(const WindowArgs& a, int batch, int max_len, hipStream_t s) {
+    const int per = a.H / a.G;
+    const int64_t wgs = (int64_t)((max_len + 64 / per - 1) / (64 / per)) * batch * a.G;
+    return per <= 32 && wgs <= F32_HALF_ROWS ? launch_window_rows_f32<DT, 32>(a, batch, max_len, s) : launch_window_rows_f32<DT, 64>(a, batch, max_len, s);
 }
 
 }  // namespace trimkv
