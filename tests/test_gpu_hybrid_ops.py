@@ -260,6 +260,15 @@ def test_mlstm_segments_side_by_side(dtype):
     run_mlstm(s, dtype, [1100], [[512, 580, 8]], f_shift=6.0)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_mlstm_segments_of_unequal_sequences(dtype):
+    """More sequences than a wavefront has lanes, long ones at either end and among the others, and segments that are shorter than the longest
+    sequence by itself would have them."""
+    seqs = [900] + [1 + i % 5 for i in range(66)] + [1301, 64, 65, 130]
+    run_mlstm(ops.MlstmSpec(1, 32, 24, 8.0), dtype, seqs, [[n] for n in seqs], f_shift=5.0)
+    run_mlstm(ops.MlstmSpec(2, 32, 24, 8.0), dtype, [64, 2000, 3, 700], [[60, 4], [1, 1999], [3], [699, 1]], f_shift=5.0)
+
+
 @pytest.mark.parametrize("H,D,Dv,lens", [(2, 128, 64, [128, 7]), (2, 128, 64, [193, 449, 64]), (3, 20, 68, [700, 320]), (1, 256, 136, [129]), (8, 128, 256, [511, 300])])
 def test_mlstm_fp32_segments_against_one_chain(H, D, Dv, lens):
     """fp32 portions of two chunks and from three on, segments of one chunk and of several, the last of them short or missing: the same as the

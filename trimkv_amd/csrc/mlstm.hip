@@ -145,10 +145,49 @@ __global__ __launch_bounds__(256) void mlstm_recurrent_kernel(MlstmArgs a) {
 // mlstm_join_kernel chains them into the state each segment starts from, pass 2 computes the outputs.
 struct ChunkArgs {
     MlstmArgs a;
-    float* seg_S; float* seg_n; float* seg_g; float* seg_m;     // [batch][H][nseg] x (D Dv, D, 2: sum of f and stabiliser, 1)
-    int seg_len, nseg;
+    float* seg_S; float* seg_n; float* seg_g; float* seg_m;     // [batch * nseg][H] x (D Dv, D, 2: sum of f and stabiliser, 1)
+    int seg_len, nseg, batch;                                   // no longer than seg_len, no more than batch * nseg in all
 };
 enum { CHUNK_WHOLE = 0, CHUNK_LOCAL = 1, CHUNK_OUTPUT = 2 };
+
+// The segments of all sequences, one sequence after the other.  They are as short as the number of tokens that are there lets them be (a
+// multiple of `unit`; sum of ceil(len / s) <= T / s + batch), not as the longest sequence times the batch would, and workgroups without a
+// segment come last instead of in between, where they spoil the spread of the others over the compute units: prompts of 701, 3999, 1536
+// and 2050 tokens (8 heads of 128 x 256) 137 -> 111 us, of 16, 3000, 40, 100 and 512 107 -> 67; four of 4000 161 on either side.
+__device__ __forceinline__ int segment_length(const ChunkArgs& ca, int unit) {
+    const int room = ca.batch * (ca.nseg - 1), total = ca.a.cu[ca.batch] - ca.a.cu[0];
+    return min(ca.seg_len, max(unit, ((total + room - 1) / room + unit - 1) / unit * unit));
+}
+__device__ __forceinline__ int segments_of(const ChunkArgs& ca, int b, int seg_len) {
+    return b < ca.batch ? (max(ca.a.cu[b + 1] - ca.a.cu[b], 0) + seg_len - 1) / seg_len : 0;
+}
+// Sequence of segment `at`, and how many segments there are in front of the sequence's own; b = -1: there are not as many segments
+struct SegmentOf { int b, before; };
+__device__ __forceinline__ SegmentOf segment_at(const ChunkArgs& ca, int at, int seg_len) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int b0 = 0; b0 < ca.batch; b0 += 64) {
+        const int own = segments_of(ca, b0 + lane, seg_len);
+        int upto = own;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) { const int o = __shfl_up(upto, d, 64); if (lane >= d) upto += o; }
+        const unsigned long long behind = __ballot(base + upto > at);
+        if (behind) {
+            const int l = __builtin_ctzll(behind);
+            return {b0 + l, base + __builtin_amdgcn_readlane(upto - own, l)};
+        }
+        base += __builtin_amdgcn_readlane(upto, 63);
+    }
+    return {-1, 0};
+}
+__device__ __forceinline__ int segments_before(const ChunkArgs& ca, int b, int seg_len) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+    for (int x = lane; x < b; x += 64) n += segments_of(ca, x, seg_len);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d, 64);
+    return __builtin_amdgcn_readfirstlane(n);
+}
 
 template <int DKT>
 struct ChunkCfg {
@@ -192,10 +231,16 @@ __global__ __launch_bounds__(256, DKT <= 4 ? 2 : 1) void mlstm_chunk_kernel(Chun
     float* const n = gM + 128; float* const qn = n + DK; float* const dsum = qn + 64;
     float* const wgt = dsum + 96;                     // [4][64]: every wavefront's own copy of exp(d_s - M_C)
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 31, hl = lane >> 5;
-    const int vt = (a.Dv + 127) / 128, seg = blockIdx.x / vt, dv0 = (blockIdx.x % vt) * 128, h = blockIdx.y, b = blockIdx.z;
-    const int t0 = a.cu[b], len_all = a.cu[b + 1] - t0;
-    const int first = MODE == CHUNK_WHOLE ? 0 : seg * ca.seg_len;
-    const int len = MODE == CHUNK_WHOLE ? len_all : min(len_all - first, ca.seg_len);
+    const int vt = (a.Dv + 127) / 128, nth = blockIdx.x / vt, dv0 = (blockIdx.x % vt) * 128, h = blockIdx.y;
+    int b = blockIdx.z, first = 0, seg_len = 0x7fffffff;
+    if (MODE != CHUNK_WHOLE) {
+        seg_len = segment_length(ca, 64);
+        const SegmentOf found = segment_at(ca, nth, seg_len);
+        if (found.b < 0) return;                      // workgroup-uniform, before any barrier
+        b = found.b;
+        first = (nth - found.before) * seg_len;
+    }
+    const int t0 = a.cu[b], len_all = a.cu[b + 1] - t0, len = min(len_all - first, seg_len);
     const int slot = a.slots[b];
     if (len <= 0) {                                   // workgroup-uniform, before any barrier (segments: mlstm_join_kernel carries n and m)
         if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
@@ -203,7 +248,7 @@ __global__ __launch_bounds__(256, DKT <= 4 ? 2 : 1) void mlstm_chunk_kernel(Chun
     }
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
-    const int64_t sat = ((int64_t)b * a.H + h) * ca.nseg + seg;
+    const int64_t sat = (int64_t)nth * a.H + h;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
     const int col = dv0 + w * 32 + j;
     const bool live = dv0 + w * 32 < a.Dv;            // wavefront-uniform
@@ -479,6 +524,7 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
     const MlstmArgs& a = ca.a;
     const int h = blockIdx.y, b = blockIdx.z, len = a.cu[b + 1] - a.cu[b], slot = a.slots[b];
     const int e = blockIdx.x * 256 + threadIdx.x, nS = a.D * a.Dv;
+    const int seg_len = segment_length(ca, 64), s0 = segments_before(ca, b, seg_len);
     if (e >= nS + a.D) return;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
@@ -486,12 +532,12 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
     const float* in = a.nm + parity * copy + at;
     float* S = a.S + ((int64_t)slot * a.H + h) * nS;
     float m = fresh ? 0.0f : in[a.D] * LOG2E, cur = fresh ? 0.0f : e < nS ? S[e] : in[e - nS];
-    const int64_t s0 = ((int64_t)b * a.H + h) * ca.nseg;
-    for (int s = 0; s < ca.nseg && s * ca.seg_len < len; ++s) {
-        float* p = e < nS ? ca.seg_S + (s0 + s) * nS + e : ca.seg_n + (s0 + s) * a.D + (e - nS);
-        const float own = *p, f = ca.seg_g[2 * (s0 + s)], ms = ca.seg_g[2 * (s0 + s) + 1];
+    for (int x = 0; x * seg_len < len; ++x) {
+        const int64_t s = (int64_t)(s0 + x) * a.H + h;
+        float* p = e < nS ? ca.seg_S + s * nS + e : ca.seg_n + s * a.D + (e - nS);
+        const float own = *p, f = ca.seg_g[2 * s], ms = ca.seg_g[2 * s + 1];
         *p = cur;
-        if (e == 0) ca.seg_m[s0 + s] = m;
+        if (e == 0) ca.seg_m[s] = m;
         const float mn = fmaxf(f + m, ms);
         cur = exp_fast(f + m - mn) * cur + exp_fast(ms - mn) * own;
         m = mn;
@@ -542,14 +588,21 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(ChunkArgs ca) {
     int* const odd = (int*)(den + TC);                // chunk + 1 whose values were not all finite
     double* const gD = (double*)(cf_lds + C::G0); double* const gM = gD + TC; double* const gm = gM + TC;           // d_s, M_t; m_0 and F_C
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    const int vt = (a.Dv + 63) / 64, seg = MODE == CHUNK_WHOLE ? 0 : blockIdx.x / vt, first = MODE == CHUNK_WHOLE ? 0 : seg * ca.seg_len;
-    const int h = blockIdx.y, b = blockIdx.z, col0 = ((int)blockIdx.x - seg * vt) * 64, col = col0 + w * 16 + c;
-    const int t0 = a.cu[b] + first, rest = a.cu[b + 1] - t0, len = MODE == CHUNK_WHOLE ? rest : min(rest, ca.seg_len), slot = a.slots[b];
+    const int vt = (a.Dv + 63) / 64, nth = blockIdx.x / vt, h = blockIdx.y, col0 = (blockIdx.x % vt) * 64, col = col0 + w * 16 + c;
+    int b = blockIdx.z, first = 0, seg_len = 0x7fffffff;
+    if (MODE != CHUNK_WHOLE) {
+        seg_len = segment_length(ca, TC);
+        const SegmentOf found = segment_at(ca, nth, seg_len);
+        if (found.b < 0) return;                      // workgroup-uniform, before any barrier
+        b = found.b;
+        first = (nth - found.before) * seg_len;
+    }
+    const int t0 = a.cu[b] + first, len = min(a.cu[b + 1] - t0, seg_len), slot = a.slots[b];
     if (len <= 0) {                                   // workgroup-uniform: there is no token to request (segments: the join carries n and m)
         if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
         return;
     }
-    const int64_t sat = ((int64_t)b * a.H + h) * ca.nseg + seg;
+    const int64_t sat = (int64_t)nth * a.H + h;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
@@ -760,10 +813,11 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(ChunkArgs ca) {
 
 // mlstm_join_kernel for these segments: sums of f and stabilisers in double (seg_g: 2, seg_m: 1), natural logarithms.  It is bound by memory
 // (5 us for 8 heads of 128 x 256 and two sequences of four segments), so that sums in double cost nothing.
-__global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca) {
+__global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca, int unit) {
     const MlstmArgs& a = ca.a;
     const int h = blockIdx.y, b = blockIdx.z, len = a.cu[b + 1] - a.cu[b], slot = a.slots[b];
     const int e = (blockIdx.x * 256 + threadIdx.x) * 4, nS = a.D * a.Dv;        // D and Dv are multiples of 4
+    const int seg_len = segment_length(ca, unit), s0 = segments_before(ca, b, seg_len);
     if (e >= nS + a.D) return;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
@@ -774,10 +828,10 @@ __global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca) {
     double cur[4];
 #pragma unroll
     for (int x = 0; x < 4; ++x) cur[x] = fresh ? 0.0 : (double)(e < nS ? S[e + x] : in[e - nS + x]);
-    const int64_t s0 = ((int64_t)b * a.H + h) * ca.nseg;
-    for (int s = 0; s < ca.nseg && s * ca.seg_len < len; ++s) {
-        float* p = e < nS ? ca.seg_S + (s0 + s) * nS + e : ca.seg_n + (s0 + s) * a.D + (e - nS);
-        const double f = load_double(ca.seg_g + 4 * (s0 + s)), ms = load_double(ca.seg_g + 4 * (s0 + s) + 2), mn = fmax(f + m, ms);
+    for (int y = 0; y * seg_len < len; ++y) {
+        const int64_t s = (int64_t)(s0 + y) * a.H + h;
+        float* p = e < nS ? ca.seg_S + s * nS + e : ca.seg_n + s * a.D + (e - nS);
+        const double f = load_double(ca.seg_g + 4 * s), ms = load_double(ca.seg_g + 4 * s + 2), mn = fmax(f + m, ms);
         const double old = exp(f + m - mn), now = exp(ms - mn);
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
@@ -785,7 +839,7 @@ __global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca) {
             p[x] = (float)cur[x];
             cur[x] = old * cur[x] + now * own;
         }
-        if (e == 0) store_double(ca.seg_m + 2 * (s0 + s), m);
+        if (e == 0) store_double(ca.seg_m + 2 * s, m);
         m = mn;
     }
     float* out = a.nm + (1 - parity) * copy + at;
@@ -814,9 +868,9 @@ static int launch_chunked_f32(const ChunkArgs& c, int batch, hipStream_t s) {
     const MlstmArgs& a = c.a;
     const int vt = (a.Dv + 63) / 64;
     if (c.nseg == 1) return launch_chunk_f32<DT, TC, CHUNK_WHOLE>(c, dim3(vt, a.H, batch), s);
-    if (int rc = launch_chunk_f32<DT, TC, CHUNK_LOCAL>(c, dim3(vt * c.nseg, a.H, batch), s)) return rc;
-    hipLaunchKernelGGL(mlstm_join_f32_kernel, dim3((a.D * a.Dv + a.D + 1023) / 1024, a.H, batch), dim3(256), 0, s, c);
-    return launch_chunk_f32<DT, TC, CHUNK_OUTPUT>(c, dim3(vt * c.nseg, a.H, batch), s);
+    if (int rc = launch_chunk_f32<DT, TC, CHUNK_LOCAL>(c, dim3(vt * c.nseg * batch, a.H), s)) return rc;
+    hipLaunchKernelGGL(mlstm_join_f32_kernel, dim3((a.D * a.Dv + a.D + 1023) / 1024, a.H, batch), dim3(256), 0, s, c, TC);
+    return launch_chunk_f32<DT, TC, CHUNK_OUTPUT>(c, dim3(vt * c.nseg * batch, a.H), s);
 }
 static int chunk_f32_tokens(int dim) { return dim <= 128 ? 64 : 32; }
 // A segment of c chunks costs 24 us per chunk in its two passes and 20 for the join and the launches, a chain 16 per chunk.  Measured, chain | segments: 4
@@ -853,20 +907,24 @@ static int launch_chunked(const ChunkArgs& c, int batch, hipStream_t s) {
     const MlstmArgs& a = c.a;
     const int vt = (a.Dv + 127) / 128;
     if (c.nseg == 1) return launch_chunk<DKT, CHUNK_WHOLE, FULL>(c, dim3(vt, a.H, batch), s);
-    if (int rc = launch_chunk<DKT, CHUNK_LOCAL, FULL>(c, dim3(vt * c.nseg, a.H, batch), s)) return rc;
+    if (int rc = launch_chunk<DKT, CHUNK_LOCAL, FULL>(c, dim3(vt * c.nseg * batch, a.H), s)) return rc;
     hipLaunchKernelGGL(mlstm_join_kernel, dim3((a.D * a.Dv + a.D + 255) / 256, a.H, batch), dim3(256), 0, s, c);
-    return launch_chunk<DKT, CHUNK_OUTPUT, FULL>(c, dim3(vt * c.nseg, a.H, batch), s);
+    return launch_chunk<DKT, CHUNK_OUTPUT, FULL>(c, dim3(vt * c.nseg * batch, a.H), s);
 }
 // the chunk kernel reads 16-byte pieces of rows and holds one head's query/key features in registers
 static bool chunk_fits(int64_t proj_stride, int q_off, int k_off, int v_off, int dim, int vdim, int dtype, int max_len, const void* proj) {
     return dtype == TRIMKV_BF16 && max_len > 1 && dim <= 256 && dim % 8 == 0 && vdim % 8 == 0 && proj_stride % 8 == 0 && (q_off | k_off | v_off) % 8 == 0 && !((uintptr_t)proj & 15);
 }
+// Two workgroups fit a compute unit and hide each other's loads: 512 of them, of at least four chunks each.  Shorter segments while every one has a
+// compute unit of its own, where they are worth the passes: about 12 us per chunk and 24 for the join and the launches against 8.5 per
+// chunk of one chain.  8 heads of 128 x 256, us with segments of four and more | of fewer: 2048 tokens 60 | 48, 600 64 | 47, twice 1024 61 | 50;
+// not taken: 300 tokens 41 | 44, three times 256 36 | 42, eight times 400 60 | 77.
 static int chunk_segments(int batch, int max_len, int heads, int vdim) {
-    const int64_t wgs = (int64_t)batch * heads * ((vdim + 127) / 128);
-    int64_t n = (512 + wgs - 1) / wgs;                // two rounds of the chip
-    const int most = max_len / 256;                   // at least four chunks each
-    n = n > most ? most : n;
-    return n < 1 ? 1 : (int)n;
+    const int64_t wgs = (int64_t)batch * heads * ((vdim + 127) / 128), chunks = (max_len + 63) / 64;
+    const int64_t both = std::max<int64_t>(1, std::min<int64_t>((512 + wgs - 1) / wgs, max_len / 256)), single = std::min<int64_t>(256 / wgs, max_len / 128);
+    if (single <= both) return (int)both;
+    const int64_t of = (chunks + single - 1) / single;
+    return (int)(24 * of + 48 < 17 * chunks ? single : both);
 }
 
 }  // namespace trimkv
@@ -900,6 +958,7 @@ extern "C" int trimkv_mlstm(const void* proj, int64_t proj_stride, int q_off, in
     hipStream_t s = (hipStream_t)stream;
     if (chunk_fits(proj_stride, q_off, k_off, v_off, dim, vdim, dtype, max_len, proj)) {
         ChunkArgs c{a};
+        c.batch = batch;
         c.nseg = chunk_segments(batch, max_len, heads, vdim);
         if (c.nseg > 1) {
             if (!workspace) return fail(TRIMKV_ERR_WORKSPACE, "%s: a prompt of %d tokens needs a workspace (trimkv_mlstm_workspace)", fn, max_len);
@@ -918,6 +977,7 @@ extern "C" int trimkv_mlstm(const void* proj, int64_t proj_stride, int q_off, in
     }
     if (chunk_f32_fits(a, dtype, max_len)) {
         ChunkArgs c{a};
+        c.batch = batch;
         c.nseg = workspace ? chunk_f32_segments(batch, max_len, heads, dim, vdim) : 1;
         if (c.nseg > 1) {
             const int tc = chunk_f32_tokens(dim);
