@@ -502,6 +502,12 @@ def test_linear_f32_on_either_side_of_its_rules(dtype, rows, n, k):
     assert ((out.double() - exact).abs() <= (k + 2) * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("rows,n,k", [(2047, 33, 64), (2048, 33, 96), (2049, 16, 288), (3071, 17, 96), (3072, 17, 128), (5000, 16, 32), (4097, 64, 160)])
+def test_linear_f32_of_prompts(rows, n, k):
+    """Either side of the rules between the two divisions of a prompt's rows."""
+    test_linear_f32_on_either_side_of_its_rules(torch.bfloat16, rows, n, k)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("width", [4, 30, 1028, 2048, 2052, 4096, 4100])
 def test_rms_rows_of_every_width(dtype, width):
