@@ -17,6 +17,17 @@ def _heights(how, n):
             "peak": (at == 1000).float() * 6, "last": (at == n - 140).float() * 6, "steps": (at / 300).floor()}[how]
 
 
+def _whole(q, k, v, lens, B, H, G, n, at_most):
+    """Undivided query tiles; lengths and starts are there, so that a bound of the lengths beyond them only chooses the kernel."""
+    from trimkv_amd import _lib
+    D, Q = q.shape[-1], q.shape[2]
+    start = torch.arange(B * H, dtype=torch.int32, device=DEV) * n
+    out = torch.empty(B, Q, H * G, D, dtype=q.dtype, device=DEV)
+    _lib.check(_lib.load().trimkv_prefill_attn(q.data_ptr(), *q.stride()[:3], out.data_ptr(), k.data_ptr(), v.data_ptr(), lens.data_ptr(), start.data_ptr(),
+                                               B, H, G, Q, n, D, _lib.dtype_code(q.dtype), D ** -0.5, at_most, _lib.current_stream(q.device)), "trimkv_prefill_attn")
+    return out
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("G,D,Q", [(1, 128, 300), (5, 64, 130)])
 @pytest.mark.parametrize("how", ["jump", "small jump", "climb", "steep", "fall", "peak", "last", "steps"])
@@ -45,13 +56,14 @@ def test_scores_that_outgrow_their_reference(how, G, D, Q, dtype):
     # P and the row sums rounded to 16 bits, one rounding of the output, as in the divided launches' bound: 6 u max|v|
     bound = 6 * float(v.abs().max()) * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
 
-    def call(name, *more):
+    def call(name, *more, at_most=longest):
         out = torch.full((B, Q, H * G, D), float("nan"), dtype=dtype, device=DEV)
         _lib.check(getattr(lib, name)(qd.data_ptr(), *qd.stride()[:3], out.data_ptr(), kd.data_ptr(), vd.data_ptr(), lend.data_ptr(), start.data_ptr(),
-                                      B, H, G, Q, longest, D, _lib.dtype_code(dtype), D ** -0.5, longest, *more, stream), name)
+                                      B, H, G, Q, longest, D, _lib.dtype_code(dtype), D ** -0.5, at_most, *more, stream), name)
         return out.cpu()
 
-    outs = {"whole": call("trimkv_prefill_attn")}
+    # a bound of the lengths that says much work: the kernel of launches that fill the chip
+    outs = {"whole": call("trimkv_prefill_attn"), "whole, in two parts": call("trimkv_prefill_attn", at_most=1 << 20)}
     for tiles in (1, 5):
         need = lib.trimkv_prefill_split_workspace(B, H, G, Q, longest, tiles)
         work = torch.full((need // 4,), float("nan"), device=DEV)
@@ -64,18 +76,31 @@ def test_scores_that_outgrow_their_reference(how, G, D, Q, dtype):
         assert float((out.double() - want).abs().max()) <= bound, (name, float((out.double() - want).abs().max()), bound)
 
 
+@pytest.mark.parametrize("at_most", [900, 1 << 20])
 @pytest.mark.parametrize("what,value", [("k", float("nan")), ("v", float("inf")), ("q", float("inf"))])
-def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(what, value):
-    from trimkv_amd.attn.hip_attn import prefill_attention
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(what, value, at_most):
     gen = torch.Generator().manual_seed(1)
     H, G, Q, n = 2, 2, 200, 900
     q, k, v = (torch.randn(1, H * G, Q, 128, generator=gen).to(torch.bfloat16), *(torch.randn(H * n, 128, generator=gen).to(torch.bfloat16) for _ in range(2)))
-    clean = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), 1, H, G, None, None, n, n, 128 ** -0.5).cpu()
+    lens = torch.full((H,), n, dtype=torch.int32, device=DEV)
+    clean = _whole(q.to(DEV), k.to(DEV), v.to(DEV), lens, 1, H, G, n, at_most).cpu()
     {"k": k, "v": v}.get(what, q.view(-1, 128))[5, 7] = value      # row 5 of the first segment, seen by all queries of its heads; or the sixth query of the first head
-    out = prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), 1, H, G, None, None, n, n, 128 ** -0.5).cpu()
+    out = _whole(q.to(DEV), k.to(DEV), v.to(DEV), lens, 1, H, G, n, at_most).cpu()
     assert torch.equal(out[:, :, G:], clean[:, :, G:])             # the second segment
     hit = out[0, 5, 0] if what == "q" else out[0, :, :G, 7] if what == "v" else out[0, :, :G]
     assert not hit.isfinite().any()
     if what == "v":
         rest = [d for d in range(128) if d != 7]
         assert out[0, :, :G][..., rest].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,G,D,Q,n", [(1, 1, 8, 128, 64, 64), (2, 3, 3, 96, 97, 200), (1, 8, 1, 64, 257, 321), (3, 8, 5, 128, 130, 1025), (1, 2, 4, 128, 400, 300)])
+def test_both_kernels_of_whole_query_tiles(B, H, G, D, Q, n, dtype):
+    """Little work and much of it, as the bound of the lengths says: the same up to the roundings of P and of the sums."""
+    gen = torch.Generator().manual_seed(n)
+    q = torch.randn(B, H * G, Q, D, generator=gen).to(dtype).to(DEV)
+    k, v = (torch.randn(B * H * n, D, generator=gen).to(dtype).to(DEV) for _ in range(2))
+    lens = torch.tensor([max(1, n - 17 * i) for i in range(B * H)], dtype=torch.int32, device=DEV)
+    few, two = (_whole(q, k, v, lens, B, H, G, n, at_most).double() for at_most in (n, 1 << 20))
+    assert float((few - two).abs().max()) <= 6 * float(v.abs().max()) * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)

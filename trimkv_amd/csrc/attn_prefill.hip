@@ -316,6 +316,7 @@ __global__ __launch_bounds__(256) void prefill_small_merge_kernel(PrefillArgs a)
 // keys 4 ig + 0..3 and 16 + 4 ig + 0..3.  The second product consumes 32 keys per MFMA; its k index 8 ig + e stands for key 4 ig + e (e < 4) or
 // 16 + 4 ig + e - 4, so that a lane's probabilities are its B operand.
 //
+// For launches that fill the chip; the others, and keys in shares by sizes, are attn_prefill_few.hip.h's.
 // What bounds it is the clock that the chip holds under matrix load, and beside it the issue of vector instructions: matrix cores and vector ALU of a SIMD
 // take turns when two wavefronts want both.  16x16x32 products cost less of the clock than 32x32x16 (registers only, random operands: 2.06 against 1.80 PFLOP/s at
 // 2.02 and 1.76 GHz), but leave less room beside them (with two and four vector instructions per 32 cycles of product 1.85 | 1.66 and 1.64 | 1.55).  Hence
@@ -385,6 +386,10 @@ __device__ __forceinline__ int units_of(const PrefillArgs& a, int i) {
 }
 constexpr int PF2_GROUPS = 256;                     // one workgroup per CU
 constexpr int PF2_LEAST = 4;                        // units of a share at least
+
+}  // namespace trimkv
+#include "attn_prefill_few.hip.h"
+namespace trimkv {
 
 // One query tile against `count` tiles of keys from tile t_first on (PART; else against all of them).  Where that is not all that the
 // query tile sees, unnormalised outputs with their exponent references and row sums (fp32) are left in `slot` for a merge kernel.
@@ -790,8 +795,8 @@ __device__ __forceinline__ void attend_query_tile_once(const PrefillArgs& a, int
     }
 }
 
-// A workgroup per query tile; SPLIT: blockIdx.z takes split_tiles tiles of the keys, and the merge kernel puts shares together.
-template <bool F16, bool SPLIT>
+// A workgroup per query tile.
+template <bool F16>
 __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a) {
     // Workgroups are handed to the 8 XCDs round robin in dispatch order (x fastest), and each XCD has its own L2.  All
     // query tiles of a segment read the same K/V, so they are mapped to one XCD (segment s on XCD s % 8, its tiles in
@@ -804,11 +809,9 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
         seg = (lin & 7) + 8 * (turn / (int)gridDim.x);
         tile = (int)gridDim.x - 1 - turn % (int)gridDim.x;
     }
-    const int t_first = SPLIT ? (int)blockIdx.z * a.split_tiles : 0;
-    if (SPLIT && t_first > 0 && t_first >= tiles_seen(a, seg, tile)) return;
     __shared__ int again;
     if (threadIdx.x == 0) again = 0;             // a barrier lies between this and whoever looks at it
-    attend_query_tile_once<F16, SPLIT, false>(a, seg, tile, t_first, a.split_tiles, ((int64_t)blockIdx.z * gridDim.y + seg) * gridDim.x + tile, (PF_LDS3 int*)&again);
+    attend_query_tile_once<F16, false, false>(a, seg, tile, 0, 0, 0, (PF_LDS3 int*)&again);
 }
 
 // Equal shares (gridDim.x workgroups, one per CU): the key tiles of all query tiles, one query tile after the other, are cut into
@@ -864,8 +867,8 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_shares_kernel(PrefillArgs
 
 // The shares of the keys put together: one wavefront per (query tile, 16 of its rows, 64 features), lanes as they wrote.
 // A share that a row saw nothing of has sum 0 and a reference of no meaning: it is left out.
-// EQUAL: shares as prefill_shares_kernel cut them, of which the first is in its workgroup's second slot.
-template <bool F16, bool EQUAL>
+// Shares as prefill_shares_kernel cut them, of which the first is in its workgroup's second slot.
+template <bool F16>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int seg = blockIdx.y, tile = (int)blockIdx.x >> 3, w = (int)blockIdx.x & 7, tiles = (int)gridDim.x >> 3;
     const int b = seg / a.kv_heads, h = seg - b * a.kv_heads;
@@ -875,17 +878,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     const int G = a.group, Q = a.q_len, BT = (PF2_WAVES * 32) / G;
     const int t_last = min(Q - 1, tile * BT + BT - 1);
     const int all_tiles = (max(0, min(n, n - Q + t_last + 1)) + PF2_BN - 1) / PF2_BN;
-    int shares, first = 0;
-    if constexpr (EQUAL) {
-        const int per = a.plan[0], at = a.plan[1 + seg * tiles + tile];
-        first = at / per;
-        shares = (at + max(all_tiles, 1) - 1) / per - first + 1;
-    } else shares = (all_tiles + a.split_tiles - 1) / a.split_tiles;
+    const int per = a.plan[0], at = a.plan[1 + seg * tiles + tile], first = at / per, shares = (at + max(all_tiles, 1) - 1) / per - first + 1;
     if (shares <= 1) return;                  // its workgroup wrote the result
     const int r = w * 32 + (half & 1) * 16 + j, g = r % G, t_q = tile * BT + r / G;
     if (r >= BT * G || t_q >= Q) return;
-    const int64_t wg = (int64_t)seg * tiles + tile, per_share = (int64_t)gridDim.y * tiles;
-    auto slot = [&](int z) -> int64_t { return EQUAL ? 2 * (first + z) + (z == 0) : wg + z * per_share; };
+    auto slot = [&](int z) -> int64_t { return 2 * (first + z) + (z == 0); };
     const float2* ml = (const float2*)a.part_ml + r;
     const float4* po = (const float4*)a.part + w * (16 * 64) + ((half & 1) * 8 + (half >> 1) * 4) * 64 + lane;
     float m = -3.0e38f;
@@ -962,11 +959,11 @@ static int launch_prefill_split(const PrefillArgs& a, int nseg, hipStream_t st) 
         }
         return 0;
     }
-    if (int rc = opt_in_lds<prefill_attn_kernel<F16, true>>()) return rc;
+    if (int rc = opt_in_lds<few::prefill_few_kernel<F16, true>>()) return rc;
     const int bt = (PF2_WAVES * 32) / a.group, tiles = (a.q_len + bt - 1) / bt;
     const int key_tiles = (a.max_len + PF2_BN - 1) / PF2_BN, shares = (key_tiles + a.split_tiles - 1) / a.split_tiles;
-    hipLaunchKernelGGL((prefill_attn_kernel<F16, true>), dim3(tiles, nseg, shares), dim3(PF2_THREADS), PF2_LDS, st, a);
-    hipLaunchKernelGGL((prefill_merge_kernel<F16, false>), dim3(tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((few::prefill_few_kernel<F16, true>), dim3(tiles, nseg, shares), dim3(PF2_THREADS), PF2_LDS, st, a);
+    hipLaunchKernelGGL((few::prefill_few_merge_kernel<F16>), dim3(tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
     return 0;
 }
 
@@ -974,7 +971,7 @@ template <bool F16>
 static int launch_prefill_shares(const PrefillArgs& a, int nseg, hipStream_t st) {
     if (int rc = opt_in_lds<prefill_shares_kernel<F16>>()) return rc;
     hipLaunchKernelGGL(prefill_shares_kernel<F16>, dim3(PF2_GROUPS), dim3(PF2_THREADS), PF2_LDS, st, a);
-    hipLaunchKernelGGL((prefill_merge_kernel<F16, true>), dim3(a.query_tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((prefill_merge_kernel<F16>), dim3(a.query_tiles * PF2_WAVES, nseg), dim3(256), 0, st, a);
     return 0;
 }
 
@@ -987,9 +984,17 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
         hipLaunchKernelGGL((prefill_small_kernel<G, F16, false>), dim3(tiles, nseg), dim3(C::THREADS), 0, st, a);
         return 0;
     }
-    if (int rc = opt_in_lds<prefill_attn_kernel<F16, false>>()) return rc;
-    const int bt = (PF2_WAVES * 32) / G;
-    hipLaunchKernelGGL((prefill_attn_kernel<F16, false>), dim3((a.q_len + bt - 1) / bt, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
+    const int bt = (PF2_WAVES * 32) / G, tiles = (a.q_len + bt - 1) / bt;
+    // Less work than takes the clock down, in query tiles x keys: all wavefronts in step.  us in step | in two parts, tiles x keys: bf16 64 x 2048 46 | 48, 128 x
+    // 4096 83.7 | 85.8, 320 x 600 44 | 46, 192 x 4000 90 | 86, 512 x 4096 178 | 163, 1024 x 1500 144 | 139; fp16 128 x 4096 83 | 94, 256 x 2100 52 | 56, 192 x 4000
+    // 94 | 96, 256 x 8192 226 | 218, 1024 x 1500 151 | 151.
+    if ((int64_t)tiles * nseg * a.max_len < (F16 ? 1200000 : 600000)) {
+        if (int rc = opt_in_lds<few::prefill_few_kernel<F16, false>>()) return rc;
+        hipLaunchKernelGGL((few::prefill_few_kernel<F16, false>), dim3(tiles, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
+        return 0;
+    }
+    if (int rc = opt_in_lds<prefill_attn_kernel<F16>>()) return rc;
+    hipLaunchKernelGGL((prefill_attn_kernel<F16>), dim3(tiles, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
     return 0;
 }
 

@@ -7,6 +7,7 @@
 //
 // In the prefill kernel the probabilities enter the second product as two bf16 terms each (17 bits).
 #include "window.hip.h"
+#include <algorithm>
 
 namespace trimkv {
 
@@ -82,17 +83,17 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowArgs a) {
 // NaNs and infinities of keys that a row does not see must not reach it through 0 x inf: tiles with such values in V take their
 // second product one key at a time.
 template <int DT, int ROWS>
-__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a, int heads) {      // heads: KV heads of all sequences
+__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a, int tiles) {      // grid: KV heads of all sequences x tiles of rows (in z what y does not hold)
     constexpr int LD = DT + 4, DB = DT / 16, PIECES = DT / 4, LOADS = 64 * PIECES / 256, RW = ROWS / 16, KS = 4 / RW, KB = 4 / KS;
     extern __shared__ __attribute__((aligned(16))) char wf_lds[];
     float* const kt = (float*)wf_lds; float* const vt = kt + 64 * LD;
     int* const where = (int*)(vt + 64 * LD);          // position of every key of the tile; past the end: beyond all queries
     int* const odd = where + 64;                      // number of tiles + 1 whose V held something that is not finite
-    const int bg = blockIdx.x % heads, b = bg / a.G, g = bg % a.G, slot = a.slots[b];
+    const int bg = blockIdx.x, b = bg / a.G, g = bg % a.G, slot = a.slots[b];
     const int t0 = a.cu[b], len = a.cu[b + 1] - t0, per = a.H / a.G, bt = ROWS / per;
     // later times of all heads first: they walk the most tiles
-    const int first = (int)((gridDim.x - 1 - blockIdx.x) / heads) * bt;
-    if (first >= len) return;                         // workgroup-uniform, before any barrier
+    const int nth = (int)(blockIdx.z * gridDim.y + blockIdx.y), first = (tiles - 1 - nth) * bt;
+    if (nth >= tiles || first >= len) return;                         // workgroup-uniform, before any barrier
     const int past = a.seen[2 * slot], cap = a.keep + a.size, nring = min(past, cap), last = min(first + bt, len) - 1;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, gr = lane >> 4;
     const int kb0 = w / RW * KB, row = w % RW * 16 + c, t = min(first + row / per, last), h = g * per + row % per, i = past + t;
@@ -569,7 +570,8 @@ static int launch_window_rows_f32(const WindowArgs& a, int batch, int max_len, h
         if (dev >= 0) opted_in[dev] = true;
     }
     const int bt = ROWS / (a.H / a.G);
-    hipLaunchKernelGGL((window_prefill_f32_kernel<DT, ROWS>), dim3((max_len + bt - 1) / bt * batch * a.G), dim3(256), LDS, s, a, batch * a.G);
+    const int tiles = (max_len + bt - 1) / bt, y = std::min(tiles, 65535);
+    hipLaunchKernelGGL((window_prefill_f32_kernel<DT, ROWS>), dim3(batch * a.G, y, (tiles + y - 1) / y), dim3(256), LDS, s, a, tiles);
     return 0;
 }
 
