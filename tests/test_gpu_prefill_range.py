@@ -76,6 +76,40 @@ def test_scores_that_outgrow_their_reference(how, G, D, Q, dtype):
         assert float((out.double() - want).abs().max()) <= bound, (name, float((out.double() - want).abs().max()), bound)
 
 
+@pytest.mark.parametrize("keys", [1, 4])
+@pytest.mark.parametrize("at", ["first turn", "middle", "end"])
+def test_row_sums_up_to_the_last_powers_of_two(at, keys):
+    """One row of a query tile outgrows its reference by 118 to 134 powers of two, segment by segment half a power more: sums that the reference is moved by,
+    those whose inverse is no normal number any more, and those that overflow.  Values are small, so that it is the sums that do."""
+    from trimkv_amd import _lib
+    lib = _lib.load()
+    H, Q, n, D = 33, 300, 1100, 128
+    gen = torch.Generator().manual_seed(keys)
+    q, k, v = 0.3 * torch.randn(1, H, Q, D, generator=gen), 0.3 * torch.randn(H, n, D, generator=gen), (torch.rand(H, n, D, generator=gen) - 0.5)
+    first = {"first turn": 100, "middle": 600, "end": n - Q + 5 - keys + 1}[at]
+    q[..., 0] = k[..., 0] = 0.0
+    for t in (5, 256 + 7):                                         # a row of either query tile; the first one sees nothing behind the keys of "end"
+        q[0, :, t, 0] = 4.0 * D ** 0.5 / 1.4426950408889634        # 4 powers of two per unit of a key, up to one rounding
+    k[:, first:first + keys, 0] = (118 + 0.5 * torch.arange(H))[:, None] / 4
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    c = D ** -0.5 * 1.4426950408889634
+    s = torch.einsum("hqd,hnd->hqn", (q[0].float() * c).to(torch.bfloat16).double(), k.double())       # powers of two, as the kernel rounds Q
+    p = torch.exp2(s.masked_fill(torch.arange(n)[None, :] > n - Q + torch.arange(Q)[:, None], -float("inf")) - s.amax(-1, keepdim=True))
+    want = ((p @ v.double()) / p.sum(-1, keepdim=True)).transpose(0, 1)[None]                          # [1, Q, H, D]
+    qd, kd, vd, lens = q.to(DEV), k.to(DEV), v.to(DEV), torch.full((H,), n, dtype=torch.int32, device=DEV)
+    bound = 6 * float(v.abs().max()) * 2.0 ** -9                    # as above
+    outs = {"in two parts": _whole(qd, kd, vd, lens, 1, H, 1, n, 1 << 20), "in step": _whole(qd, kd, vd, lens, 1, H, 1, n, n)}
+    shares = torch.full((1, Q, H, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    need = lib.trimkv_prefill_shares_workspace(1, H, 1, Q)
+    work = torch.full((need // 4,), float("nan"), device=DEV)
+    _lib.check(lib.trimkv_prefill_attn_shares(qd.data_ptr(), *qd.stride()[:3], shares.data_ptr(), kd.data_ptr(), vd.data_ptr(), lens.data_ptr(), None, 1, H, 1, Q, n, D,
+                                              _lib.BF16, D ** -0.5, n, work.data_ptr(), need, _lib.current_stream(qd.device)), "trimkv_prefill_attn_shares")
+    outs["shares"] = shares
+    for name, out in outs.items():
+        far = (out.cpu().double() - want).abs().amax((0, 1, 3))     # of every segment
+        assert far.max() <= bound, (name, [118 + 0.5 * i for i in range(H) if not far[i] <= bound], bound)
+
+
 @pytest.mark.parametrize("at_most", [900, 1 << 20])
 @pytest.mark.parametrize("what,value", [("k", float("nan")), ("v", float("inf")), ("q", float("inf"))])
 def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(what, value, at_most):

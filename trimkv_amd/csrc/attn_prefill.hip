@@ -575,12 +575,15 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
 #pragma unroll
                 for (int v = 0; v < 4; ++v) { s.g[0][qg][v] -= d; s.g[1][qg][v] -= d; negm[qg][v] = -m_ref[qg]; }
                 if (!FIRST) {
-                    const float alpha = __builtin_amdgcn_exp2f(-d);
-                    l_run[qg] *= alpha;
+                    // Sums of 2^126 and more move the reference by 127 or 128, and v_exp_f32 gives 0 there instead of the denormal number: they are scaled by their
+                    // exponent.  What a maximum that far away does not leave is nothing to the new one.
+                    const float alpha = MAXIMA ? __builtin_amdgcn_exp2f(-d) : 0.0f;
+                    auto moved = [&](float x) __attribute__((always_inline)) { return MAXIMA ? x * alpha : __builtin_ldexpf(x, -(int)d); };
+                    l_run[qg] = moved(l_run[qg]);
 #pragma unroll
                     for (int dg = 0; dg < 8; ++dg)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) o[dg >> 1][8 * (dg & 1) + 4 * qg + v] *= alpha;
+                        for (int v = 0; v < 4; ++v) o[dg >> 1][8 * (dg & 1) + 4 * qg + v] = moved(o[dg >> 1][8 * (dg & 1) + 4 * qg + v]);
                 }
             }
         }
