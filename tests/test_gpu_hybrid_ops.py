@@ -302,6 +302,32 @@ def test_mlstm_fp32_segments_against_one_chain(H, D, Dv, lens):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("lens", [[700, 1500], [3000], [40, 513, 9, 1200]])
+def test_mlstm_sequences_longer_than_they_were_said_to_be(lens, dtype):
+    """A max_len below the longest sequence costs time only: segments stay within the workspace that it asks for, and no token is left out."""
+    from trimkv_amd import _lib
+    lib, B, T, H, D, Dv, said = _lib.load_hybrid("mlstm"), len(lens), sum(lens), 2, 64, 128, 512
+    width, code = 2 * H * D + H * Dv, _lib.dtype_code(dtype)
+    proj, gates, ib, fb = rnd(T, width, seed=1).to(dtype).to(DEV), rnd(T, 2 * H, seed=2).to(DEV), rnd(H, seed=3).to(DEV), (4 + rnd(H, seed=4)).to(DEV)
+    cu = torch.tensor([0] + lens).cumsum(0).int().to(DEV)
+    slots = torch.arange(B, dtype=torch.int32, device=DEV)
+    seen = torch.tensor([9, 1] * B, dtype=torch.int32, device=DEV)
+    got = []
+    for max_len in (max(lens), said):
+        need = lib.trimkv_mlstm_workspace(B, max_len, H, D, Dv, code)
+        assert need > 0
+        ws = torch.full((4 * need + (1 << 20),), 7.0, device=DEV)
+        S, nm, o = rnd(B, H, D, Dv, seed=5).to(DEV), rnd(2, B, H, D + 1, seed=6).to(DEV), torch.zeros(T, H, Dv, dtype=dtype, device=DEV)
+        assert lib.trimkv_mlstm(proj.data_ptr(), width, 0, H * D, 2 * H * D, gates.data_ptr(), ib.data_ptr(), fb.data_ptr(), 9.0, S.data_ptr(), nm.data_ptr(),
+                                cu.data_ptr(), slots.data_ptr(), seen.data_ptr(), o.data_ptr(), B, max_len, H, D, Dv, B, D ** -0.5, ws.data_ptr(), code,
+                                _lib.current_stream(proj.device)) == 0
+        assert (ws[need:] == 7.0).all()
+        got.append((o, S, nm))
+    for right, short in zip(*got):
+        assert (right.double() - short.double()).norm() <= (4e-6 if dtype == torch.float32 else 1e-2) * right.double().norm()      # as for segments against one chain; bf16 as above
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["square", "odd", "mid"])
 def test_mlstm_sequences_without_tokens_keep_their_state(name, dtype, monkeypatch):
     """A packed step may hold sequences that bring nothing: first, last, or not begun yet; the state they left goes on behind it,

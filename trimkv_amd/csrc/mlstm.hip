@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void mlstm_recurrent_kernel(MlstmArgs a) {
 struct ChunkArgs {
     MlstmArgs a;
     float* seg_S; float* seg_n; float* seg_g; float* seg_m;     // [batch * nseg][H] x (D Dv, D, 2: sum of f and stabiliser, 1)
-    int seg_len, nseg, batch;                                   // no longer than seg_len, no more than batch * nseg in all
+    int seg_len, nseg, batch;                                   // no longer than seg_len for sequences up to max_len, no more than batch * nseg in all
 };
 enum { CHUNK_WHOLE = 0, CHUNK_LOCAL = 1, CHUNK_OUTPUT = 2 };
 
@@ -154,9 +154,13 @@ enum { CHUNK_WHOLE = 0, CHUNK_LOCAL = 1, CHUNK_OUTPUT = 2 };
 // multiple of `unit`; sum of ceil(len / s) <= T / s + batch), not as the longest sequence times the batch would, and workgroups without a
 // segment come last instead of in between, where they spoil the spread of the others over the compute units: prompts of 701, 3999, 1536
 // and 2050 tokens (8 heads of 128 x 256) 137 -> 111 us, of 16, 3000, 40, 100 and 512 107 -> 67; four of 4000 161 on either side.
+// seg_len alone bounds their number only while no sequence is longer than the caller's max_len.
 __device__ __forceinline__ int segment_length(const ChunkArgs& ca, int unit) {
-    const int room = ca.batch * (ca.nseg - 1), total = ca.a.cu[ca.batch] - ca.a.cu[0];
-    return min(ca.seg_len, max(unit, ((total + room - 1) / room + unit - 1) / unit * unit));
+    const int room = ca.batch * (ca.nseg - 1), total = ca.a.cu[ca.batch] - ca.a.cu[0], most = ca.nseg * ca.seg_len;
+    bool longer = false;
+    for (int x = threadIdx.x & 63; x < ca.batch; x += 64) longer = longer || ca.a.cu[x + 1] - ca.a.cu[x] > most;
+    const int len = max(unit, ((total + room - 1) / room + unit - 1) / unit * unit);
+    return __ballot(longer) ? len : min(ca.seg_len, len);
 }
 __device__ __forceinline__ int segments_of(const ChunkArgs& ca, int b, int seg_len) {
     return b < ca.batch ? (max(ca.a.cu[b + 1] - ca.a.cu[b], 0) + seg_len - 1) / seg_len : 0;
