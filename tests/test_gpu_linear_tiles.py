@@ -3,6 +3,7 @@
 Bounds: fp32 sums of k products err by at most about k 2^-24 sum |x w| (any order), the result is rounded once (half a unit in the
 last place, 2^-9 of the value in bf16; twice that here, for values that straddle)."""
 import ctypes
+import random
 
 import pytest
 import torch
@@ -142,3 +143,24 @@ def test_bad_arguments_are_refused_without_a_launch():
     silu = lambda form: lib.trimkv_linear_tiles_silu(one, 64, one, 64, one, 16, 400, 16, 64, 1, form, _lib.BF16, None)
     assert silu(4) == -2 and silu(9) == -2
     assert lib.trimkv_linear_tiles_form(0, 64, 64, 0) == 0 and lib.trimkv_linear_tiles_form(64, 64, 32, 0) == 0
+
+
+def test_sizes_are_asked_first(monkeypatch):
+    """The host bounds prompts of a few hundred tokens: a product of too few outputs for tiles goes to the general one by its sizes alone."""
+    asked = []
+    monkeypatch.setattr(linear, "_plain", lambda *a: asked.append(a))
+    for rows, n in ((65, 4096), (142, 6144), (300, 6300)):
+        x, w = torch.randn(rows, 64).to(torch.bfloat16), torch.randn(n, 64).to(torch.bfloat16)
+        assert torch.equal(linear.linear(x, w), torch.nn.functional.linear(x, w)) and linear.silu_product(x, w) is None and not asked
+    assert torch.equal(linear.linear(x[:64], w), torch.nn.functional.linear(x[:64], w)) and asked      # a decode step's rows are
+
+
+def test_few_outputs_are_never_done_on_tiles():
+    """The line that is drawn by rows x outputs alone leaves nothing to the general product that the estimate of tiles would take."""
+    rng = random.Random(5)
+    for _ in range(60000):
+        silu = rng.random() < 0.5
+        k, n = 64 * round(2 ** rng.uniform(0, 11)), round(2 ** rng.uniform(0, 17))
+        rows = (linear.LEAST_SILU_OUTPUTS if silu else linear.LEAST_OUTPUTS) * rng.uniform(0.5, 1) // n
+        if rows >= 1:
+            assert _lib.load().trimkv_linear_tiles_form(int(rows), n, k, int(silu)) == 0, (rows, n, k, silu)

@@ -5,6 +5,7 @@ Both give fp32 sums rounded once; the order of the sums differs.
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
@@ -24,6 +25,13 @@ MAX_ROWS = 64      # rows that trimkv_linear_rows takes
 # 32 rows all are taken: 32064 x 3072 with 1, 16, 32 rows 31.5 | 41.0, 33.2 | 42.0, 39.4 | 37.1; 151936 x 2048 101 | 207, 109 | 208, 128 | 153; 151936 x
 # 5120 238 | 307, 263 | 330, 319 | 364.  12288 x 4096 with 48 and 64: 22.8 | 24.5, 24.3 | 25.1.
 WIDE_ROWS, WIDE = 32, 12288
+
+
+# Fewer rows x outputs than this are never done on tiles, whatever k is: they would fill less than half of the chip.  (trimkv_linear_tiles_form wants the
+# operations at its rate for no less than a round of tiles takes by its estimate, 0.77 (1 + 0.49 k / 64) us, with silu 0.77 (1 + 0.83 k / 64).)  Sizes are asked before
+# all else, because the host bounds prompts of a few hundred tokens: with the other checks in front 142 tokens through three layers of 2048 took 750 us
+# for 615, through two layers with recurrence 337 for 298.
+LEAST_OUTPUTS, LEAST_SILU_OUTPUTS = 1_900_000, 1_370_000
 
 
 def watched() -> bool:
@@ -51,7 +59,12 @@ def _plain(*tensors: Optional[torch.Tensor]) -> bool:
 def _rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """x as [rows, k] the way trimkv_linear_rows reads it, or None where it does not take this product."""
     k = x.shape[-1] if x.dim() else 0
-    if k == 0 or k % 64 or not 0 < x.numel() <= MAX_ROWS * k or not _plain(x, weight, bias):
+    return _step_rows(x, weight, bias, k) if 0 < x.numel() <= MAX_ROWS * k else None
+
+
+def _step_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], k: int) -> Optional[torch.Tensor]:
+    """``_rows`` of no more of them than trimkv_linear_rows takes, and of one at least."""
+    if k % 64 or not _plain(x, weight, bias):
         return None
     if weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0 or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 8 or weight.data_ptr() % 16:
         return None
@@ -63,32 +76,47 @@ def _rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -
     return None if max(x2.stride(0), weight.stride(0)) > 1 << 24 else x2
 
 
+@functools.lru_cache(maxsize=4096)
+def _form(rows: int, n: int, k: int, silu: bool, library: Optional[str]) -> int:
+    return (_lib.load() if library is None else _lib.load_hybrid(library)).trimkv_linear_tiles_form(rows, n, k, int(silu))
+
+
 def _tiles(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], silu: bool, library: Optional[str]):
     """``(x as [rows, k], form)`` the way trimkv_linear_tiles takes this product, or None where it does not or is not faster."""
     k = x.shape[-1] if x.dim() else 0
-    if bias is not None or k == 0 or k % 64 or x.numel() <= MAX_ROWS * k or x.dtype != torch.bfloat16 or not _plain(x, weight):
+    return _prompt_rows(x, weight, bias, k, x.numel(), silu, library) if x.numel() > MAX_ROWS * k else None
+
+
+def _prompt_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], k: int, size: int, silu: bool, library: Optional[str]):
+    """``_tiles`` of more rows than trimkv_linear_rows takes; ``size``: the numbers of x."""
+    if bias is not None or k == 0 or k % 64 or x.dtype != torch.bfloat16 or not x.is_cuda or weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0:
         return None
-    if weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0 or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 8 or weight.data_ptr() % 16:
+    rows, n = size // k, weight.shape[0] // 2 if silu else weight.shape[0]
+    # sizes in front of what takes longer to find out; sizes that are no numbers belong to somebody who follows the operations
+    if torch.compiler.is_compiling() or type(rows) is not int or type(n) is not int or max(rows, n) > 1 << 24 or (silu and weight.shape[0] % 2):
+        return None
+    form = _form(rows, n, k, silu, library)
+    if not form or not _plain(x, weight) or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 8 or weight.data_ptr() % 16:
         return None
     if x.dim() != 2 and not x.is_contiguous():
         return None
     x2 = x if x.dim() == 2 else x.view(-1, k)
     if x2.stride(1) != 1 or x2.data_ptr() % 16 or x2.stride(0) < k or x2.stride(0) % 8 or max(x2.stride(0), weight.stride(0)) > 1 << 20:
         return None
-    n = weight.shape[0] // 2 if silu else weight.shape[0]
-    if max(x2.shape[0], n) > 1 << 24 or (silu and weight.shape[0] % 2):
-        return None
-    lib = _lib.load() if library is None else _lib.load_hybrid(library)
-    form = lib.trimkv_linear_tiles_form(x2.shape[0], n, k, int(silu))
-    return (x2, form) if form else None
+    return x2, form
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, library: Optional[str] = None) -> torch.Tensor:
     """``F.linear(x, weight, bias)``.  ``library``: which one holds the kernel (a name of ``_lib.SHARED``; None: libtrimkv_hip.so)."""
-    x2 = _rows(x, weight, bias)
-    if x2 is None:
-        many = _tiles(x, weight, bias, False, library)
+    k, size = x.shape[-1] if x.dim() else 0, x.numel()
+    if size > MAX_ROWS * k:
+        if size * weight.numel() < LEAST_OUTPUTS * k * k:
+            return F.linear(x, weight, bias)
+        many = _prompt_rows(x, weight, bias, k, size, False, library)
         return F.linear(x, weight, bias) if many is None else _tile_product(x, *many, weight, library)
+    x2 = _step_rows(x, weight, bias, k) if size else None
+    if x2 is None:
+        return F.linear(x, weight, bias)
     if x2.shape[0] > WIDE_ROWS and weight.shape[0] > WIDE:
         return F.linear(x, weight, bias)
     rows, k = x2.shape
@@ -117,10 +145,15 @@ def _tile_product(x: torch.Tensor, x2: torch.Tensor, form: int, weight: torch.Te
 def silu_product(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, round_all: bool = True, library: Optional[str] = None) -> Optional[torch.Tensor]:
     """``silu(x @ gate.T) * (x @ up.T)`` with ``weight`` = gate over up, in one launch; None where neither trimkv_linear_rows_silu nor
     trimkv_linear_tiles_silu takes it."""
-    x2 = _rows(x, weight, bias)
-    if x2 is None:
-        many = _tiles(x, weight, bias, True, library)
+    k, size = x.shape[-1] if x.dim() else 0, x.numel()
+    if size > MAX_ROWS * k:
+        if size * weight.numel() < 2 * LEAST_SILU_OUTPUTS * k * k:
+            return None
+        many = _prompt_rows(x, weight, bias, k, size, True, library)
         return None if many is None else _tile_product(x, *many, weight, library, True, round_all)
+    x2 = _step_rows(x, weight, bias, k) if size else None
+    if x2 is None:
+        return None
     if weight.shape[0] % 2:
         return None
     rows, k = x2.shape
