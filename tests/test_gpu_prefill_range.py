@@ -138,3 +138,20 @@ def test_both_kernels_of_whole_query_tiles(B, H, G, D, Q, n, dtype):
     lens = torch.tensor([max(1, n - 17 * i) for i in range(B * H)], dtype=torch.int32, device=DEV)
     few, two = (_whole(q, k, v, lens, B, H, G, n, at_most).double() for at_most in (n, 1 << 20))
     assert float((few - two).abs().max()) <= 6 * float(v.abs().max()) * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+
+
+@pytest.mark.parametrize("dtype,n", [(torch.bfloat16, 4000), (torch.float16, 8000)])
+def test_query_tiles_for_two_thirds_of_the_chip_are_attended_in_step(dtype, n):
+    """160 query tiles of long keys go to the kernel that divided launches have, which is the faster one there: bit for bit what a single share gives."""
+    from trimkv_amd import _lib
+    H, G, Q, D = 8, 8, 640, 64
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    q = torch.randn(1, H * G, Q, D, generator=gen, device=DEV).to(dtype)
+    k, v = (torch.randn(H * n, D, generator=gen, device=DEV).to(dtype) for _ in range(2))
+    lens = torch.full((H,), n, dtype=torch.int32, device=DEV)
+    one, lib, share = torch.empty(1, Q, H * G, D, dtype=dtype, device=DEV), _lib.load(), (n + 63) // 64
+    need = lib.trimkv_prefill_split_workspace(1, H, G, Q, n, share)
+    work = torch.empty(need, dtype=torch.uint8, device=DEV)
+    _lib.check(lib.trimkv_prefill_attn_split(q.data_ptr(), *q.stride()[:3], one.data_ptr(), k.data_ptr(), v.data_ptr(), lens.data_ptr(), None, 1, H, G, Q, n, D,
+                                             _lib.dtype_code(dtype), D ** -0.5, n, share, work.data_ptr(), need, _lib.current_stream(q.device)), "trimkv_prefill_attn_split")
+    assert torch.equal(_whole(q, k, v, lens, 1, H, G, n, n), one)

@@ -990,8 +990,11 @@ static int launch_prefill(const PrefillArgs& a, int nseg, hipStream_t st) {
     const int bt = (PF2_WAVES * 32) / G, tiles = (a.q_len + bt - 1) / bt;
     // Less work than takes the clock down, in query tiles x keys: all wavefronts in step.  us in step | in two parts, tiles x keys: bf16 64 x 2048 46 | 48, 128 x
     // 4096 83.7 | 85.8, 320 x 600 44 | 46, 192 x 4000 90 | 86, 512 x 4096 178 | 163, 1024 x 1500 144 | 139; fp16 128 x 4096 83 | 94, 256 x 2100 52 | 56, 192 x 4000
-    // 94 | 96, 256 x 8192 226 | 218, 1024 x 1500 151 | 151.
-    if ((int64_t)tiles * nseg * a.max_len < (F16 ? 1200000 : 600000)) {
+    // 94 | 96, 256 x 8192 226 | 218, 1024 x 1500 151 | 151.  Nor do long keys take it down where a third of the compute units has no tile: bf16 128 x 9000 167 |
+    // 177, 136 x 5395 107 | 111, 160 x 8000 155 | 159, 168 x 5395 111 | 111, 192 x 6000 128 | 123; fp16 160 x 8000 167 | 180, 168 x 8000 168 | 176, 192 x
+    // 8000 180 | 179 (beyond 16000 keys not measured).
+    const int64_t items = (int64_t)tiles * nseg;
+    if (items * a.max_len < (F16 ? 1200000 : 600000) || (items <= 168 && a.max_len <= 65536)) {
         if (int rc = opt_in_lds<few::prefill_few_kernel<F16, false>>()) return rc;
         hipLaunchKernelGGL((few::prefill_few_kernel<F16, false>), dim3(tiles, nseg), dim3(PF2_THREADS), PF2_LDS, st, a);
         return 0;
