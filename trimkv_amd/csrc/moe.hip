@@ -85,15 +85,20 @@ __global__ __launch_bounds__(1024) void plan_kernel(const int32_t* ids, int rows
     const int tid = threadIdx.x, per = (rows + gridDim.x - 1) / gridDim.x, mine = blockIdx.x * per, end = min(rows, mine + per);
     for (int e = tid; e < 2 * E; e += 1024) pl[e] = 0;
     __syncthreads();
-    auto each = [&](int from, int to, auto&& f) __attribute__((always_inline)) {      // eight experts requested together
-        for (int i0 = from + tid; i0 < to; i0 += 8192) {
-            int id[8];
+    auto each = [&](int from, int to, auto&& f) __attribute__((always_inline)) {
+        auto some = [&](auto count) __attribute__((always_inline)) {      // so many experts requested together
+            constexpr int U = decltype(count)::value;
+            for (int i0 = from + tid; i0 < to; i0 += U * 1024) {
+                int id[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) id[u] = ids[min(i0 + u * 1024, to - 1)];
+                for (int u = 0; u < U; ++u) id[u] = ids[min(i0 + u * 1024, to - 1)];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (i0 + u * 1024 < to) f(i0 + u * 1024, id[u]);
-        }
+                for (int u = 0; u < U; ++u)
+                    if (i0 + u * 1024 < to) f(i0 + u * 1024, id[u]);
+            }
+        };
+        if (to - from <= 2048) some(std::integral_constant<int, 2>{});      // 2048 rows: eight each, of which six are none, take 4.2 us for 3.7
+        else some(std::integral_constant<int, 8>{});
     };
     each(0, rows, [&](int i, int e) __attribute__((always_inline)) { atomicAdd(&pl[i < mine ? e : E + e], 1); });
     __syncthreads();
