@@ -397,9 +397,12 @@ namespace trimkv {
 // HOW: what keeps the exponentials in range.  ATTEND_MAXIMA (fp16): the exponent reference of a row stays within 2^PF2_LAZY of its largest score.  ATTEND_SUMS (bf16,
 // whose P has fp32's exponents): once set it moves only where the row's sum has grown beyond PF2_MOST, which takes no maxima; a score that exceeds the
 // reference by 2^7 within a block overflows then, and whatever is not finite at the end (an input that is not among it) sets *again (0 before), for
-// the caller to have it done again with ATTEND_CAREFULLY over what it has written: maxima as in fp16, one block after the other.
-enum { ATTEND_MAXIMA, ATTEND_SUMS, ATTEND_CAREFULLY };
-template <bool F16, bool PART, bool LOOP, int HOW>
+// the caller to have it done again with ATTEND_MAXIMA over what it has written.
+// What that costs falls on query tiles with a row that holds a score more than 88 nats above the first block's largest, or a value that is not finite.  16 segments of
+// 6000 keys, 2048 queries of 4 heads: 246 us without (272 for the loop of few::, which has maxima always), 387 where one query tile of 32 of each segment has such
+// a row, 444 where each one has, 497 where all rows are such.
+enum { ATTEND_MAXIMA, ATTEND_SUMS };
+template <bool F16, bool PART, int HOW>
 __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot, PF_LDS3 int* again) {
     constexpr bool MAXIMA = HOW != ATTEND_SUMS;
     extern __shared__ __attribute__((aligned(16))) char pf2_lds[];
@@ -485,7 +488,7 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
     };
 
     const int ntiles = PART ? min(all_tiles - t_first, count) : all_tiles;
-    if (ntiles > 0 && HOW != ATTEND_CAREFULLY) {
+    if (ntiles > 0) {
         request_tile(0, 0);
         request_tile(1, 1);
     }
@@ -667,41 +670,7 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
     // Every wavefront walks all blocks of the workgroup's tiles: the blocks that
     // lie wholly above a wavefront's diagonal (at most two of up to several hundred, the workgroup spans BT query times)
     // are masked like the diagonal ones and contribute zeros, which keeps the loop free of per-wavefront branches.
-    if constexpr (HOW == ATTEND_CAREFULLY) {
-#pragma clang loop unroll(disable)
-        for (int blk = 0; blk < 2 * ntiles; ++blk) {
-            const int off = (blk & 1) * (PF2_TILE / 2);
-            if (!(blk & 1)) {
-                __syncthreads();                 // every wavefront has left the tile before
-                request_tile(blk >> 1, 0);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __syncthreads();
-            }
-            Scores s;
-#pragma unroll
-            for (int m = 0; m < 8; ++m)
-#pragma unroll
-                for (int qg = 0; qg < 2; ++qg) s.g[m & 1][qg] = mfma_16x16x32<F16>(k_frag(off, m), qf[qg][m >> 1], m < 2 ? negm[qg] : s.g[m & 1][qg]);
-            if (blk == 0) prepare(s, 0, Pair{{0.0f, 0.0f}}, std::true_type{}, std::true_type{});
-            else prepare(s, blk, Pair{{max8(s, 0), max8(s, 1)}}, std::false_type{}, std::true_type{});
-            uint32_t pw[8];
-#pragma unroll
-            for (int x = 0; x < 8; ++x) pw[x] = p_pair(s, x);
-#pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const pf_bf16x8 v = v_frag(off, m);
-#pragma unroll
-                for (int qg = 0; qg < 2; ++qg) {
-                    const pf_u32x4 pq = {pw[4 * qg], pw[4 * qg + 1], pw[4 * qg + 2], pw[4 * qg + 3]};
-                    pf_f32x16& all = o[m >> 1];
-                    const int at = 8 * (m & 1) + 4 * qg;
-                    const pf_f32x4 r = mfma_16x16x32<F16>(v, __builtin_bit_cast(pf_bf16x8, pq), pf_f32x4{all[at], all[at + 1], all[at + 2], all[at + 3]});
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) all[at + x] = r[x];
-                }
-            }
-        }
-    } else if (ntiles > 0) {
+    if (ntiles > 0) {
         Scores s;
         asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
         __syncthreads();
@@ -785,15 +754,15 @@ __device__ __forceinline__ void attend_query_tile(const PrefillArgs& a, int seg,
 }
 
 // ends with every wavefront having left the LDS tiles; `again` is 0 then, as it is in front
-template <bool F16, bool PART, bool LOOP>
+template <bool F16, bool PART>
 __device__ __forceinline__ void attend_query_tile_once(const PrefillArgs& a, int seg, int tile, int t_first, int count, int64_t slot, PF_LDS3 int* again) {
-    attend_query_tile<F16, PART, LOOP, F16 ? ATTEND_MAXIMA : ATTEND_SUMS>(a, seg, tile, t_first, count, slot, again);
-    if (F16 && !LOOP) return;
+    attend_query_tile<F16, PART, F16 ? ATTEND_MAXIMA : ATTEND_SUMS>(a, seg, tile, t_first, count, slot, again);
+    if (F16 && !PART) return;              // a workgroup of PART has another query tile behind this one
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");       // for LDS: nobody waits for the stores
     if (!F16 && __builtin_amdgcn_readfirstlane(*again)) {
         __syncthreads();                         // everyone has read it
         if (threadIdx.x == 0) *again = 0;
-        attend_query_tile<F16, PART, LOOP, ATTEND_CAREFULLY>(a, seg, tile, t_first, count, slot, again);
+        attend_query_tile<F16, PART, ATTEND_MAXIMA>(a, seg, tile, t_first, count, slot, again);
         __syncthreads();
     }
 }
@@ -814,7 +783,7 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_attn_kernel(PrefillArgs a
     }
     __shared__ int again;
     if (threadIdx.x == 0) again = 0;             // a barrier lies between this and whoever looks at it
-    attend_query_tile_once<F16, false, false>(a, seg, tile, 0, 0, 0, (PF_LDS3 int*)&again);
+    attend_query_tile_once<F16, false>(a, seg, tile, 0, 0, 0, (PF_LDS3 int*)&again);
 }
 
 // Equal shares (gridDim.x workgroups, one per CU): the key tiles of all query tiles, one query tile after the other, are cut into
@@ -863,7 +832,7 @@ __global__ __launch_bounds__(PF2_THREADS) void prefill_shares_kernel(PrefillArgs
     int i = __builtin_amdgcn_readfirstlane(found[0]), t_first = __builtin_amdgcn_readfirstlane(found[1]);
     for (int u = u0; u < u1; ++i, t_first = 0) {
         const int seg = i / a.query_tiles, count = min(units_of(a, i) - t_first, u1 - u);
-        attend_query_tile_once<F16, true, true>(a, seg, i - seg * a.query_tiles, t_first, count, 2 * wg + (t_first == 0), (PF_LDS3 int*)&again);
+        attend_query_tile_once<F16, true>(a, seg, i - seg * a.query_tiles, t_first, count, 2 * wg + (t_first == 0), (PF_LDS3 int*)&again);
         u += count;
     }
 }
