@@ -164,3 +164,10 @@ def test_few_outputs_are_never_done_on_tiles():
         rows = (linear.LEAST_SILU_OUTPUTS if silu else linear.LEAST_OUTPUTS) * rng.uniform(0.5, 1) // n
         if rows >= 1:
             assert _lib.load().trimkv_linear_tiles_form(int(rows), n, k, int(silu)) == 0, (rows, n, k, silu)
+
+
+@pytest.mark.parametrize("rows,n,k,silu,taken", [(680, 6144, 4096, 0, False), (1599, 3072, 8192, 0, False), (206, 8192, 3072, 1, False), (1409, 3072, 3072, 0, False), (4096, 1536, 1024, 0, True),
+                                                 (613, 4112, 2048, 0, True), (1656, 4096, 4096, 0, True), (412, 12288, 2048, 1, True), (8192, 12288, 4096, 1, True)])
+def test_products_of_long_k_need_more_of_the_chip(rows, n, k, silu, taken):
+    """Sizes that were measured on either side of the rule's two lines: the general product divides k, and is faster where tiles leave compute units idle."""
+    assert bool(_lib.load().trimkv_linear_tiles_form(rows, n, k, silu)) == taken

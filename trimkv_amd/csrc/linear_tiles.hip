@@ -190,16 +190,17 @@ extern "C" int trimkv_linear_tiles_silu(const void* x, int64_t x_stride, const v
     return tiles_check_and_launch("trimkv_linear_tiles_silu", {(const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, (uint16_t*)out, out_stride, rows, inter, k, round_all}, form, true, dtype, stream);
 }
 
-// Products that the tiles take at less than RATE (by the estimate) have too few of them to fill the chip, and those of the vendor's library that divide k are
-// faster: 64 .. 600 rows above all.  us here | general: 82 x 2048 x 2048 (rows x n x k) 16 | 8, 467 x 2048 x 6144 42 | 26, 856 x 1024 x 4096 30 | 19, 1301 x 3072 x 3072
-// 37 | 32; 613 x 4112 x 2048 20 | 21, 1656 x 4096 x 4096 52 | 56, 2252 x 4112 x 2048 35 | 43, 8286 x 6144 x 2048 164 | 230, 8286 x 2048 x 2048 64 | 69,
-// 8192 x 6176 x 4096 293 | 380, 8192 x 4096 x 4096 180 | 178, 9688 x 6176 x 4096 349 | 494, 8192 x 4096 x 12288 521 | 521.  Of 103 products above the line
-// the geometric mean is 1.07, the worst 0.87; of 30 below it three are lost.  With silu, a launch less (us here | general and silu): 177 rows of 12288 x 2048 27 | 27,
-// 412 29 | 34, 8192 of 24576 x 4096 1058 | 1140.
+// Products that the tiles take at less than RATE (by the estimate) have too few of them to fill the chip.  The vendor's library divides long k where outputs are
+// few, so that the line is higher there.  Of 930 products of 70 .. 10000 rows, 512 .. 151936 outputs and k up to 17408: above the line 480, 1.14 times as fast on
+// average, 29 of them slower by 3 % and more (15 by 8 %); with silu, a launch less, 415, 1.15, 14 (3).  Between RATE for short k and for long, where
+// k is longer than 2048: 164, 0.98, 90; with silu 38, 0.93, 29.  us here | general (rows x n x k): 82 x 2048 x 2048 16 | 8, 613 x 4112 x 2048 20 | 21, 2252 x
+// 4112 x 2048 35 | 43, 8286 x 6144 x 2048 164 | 230, 8286 x 2048 x 2048 64 | 69, 680 x 6144 x 4096 50 | 46, 1599 x 3072 x 8192 94 | 77, 1656 x
+// 4096 x 4096 52 | 56, 8192 x 6176 x 4096 293 | 380, 8192 x 4096 x 4096 180 | 178, 8192 x 4096 x 12288 521 | 521; with silu 177 rows of 12288 x
+// 2048 27 | 27, 412 29 | 34, 206 of 8192 x 3072 43 | 36, 8192 of 12288 x 4096 1058 | 1140.
 extern "C" int trimkv_linear_tiles_form(int rows, int n, int k, int silu) {
-    constexpr float RATE = 0.65e9f, RATE_SILU = 0.55e9f;      // operations per us
+    const float rate = k <= 2048 ? (silu ? 0.55e9f : 0.65e9f) : silu ? 0.8e9f : 1.0e9f;      // RATE: operations per us
     if (rows <= 0 || n <= 0 || k < 64) return 0;
     float cost;
     const int form = tiles_form(rows, n, k, silu != 0, &cost);
-    return 2.0f * rows * n * k * (silu ? 2 : 1) >= (silu ? RATE_SILU : RATE) * cost ? form : 0;
+    return 2.0f * rows * n * k * (silu ? 2 : 1) >= rate * cost ? form : 0;
 }
