@@ -508,6 +508,18 @@ def test_values_that_are_not_finite_stay_out_of_rows_that_do_not_see_them(bad, a
     assert not rb[at:, 0].isfinite().any()
 
 
+@pytest.mark.parametrize("heads,kv_heads,seqs", [
+    (4, 2, [1, 130, 2, 16, 15, 17, 129, 3]),                                          # 32 rows to a workgroup, one tile and several
+    (4, 1, [700, 5, 1, 699, 8, 9]),                                                   # more tiles than a wavefront has lanes
+    (4, 2, [300] + [1 + i % 5 for i in range(62)] + [299, 64, 65, 1, 40, 33] * 2),    # more sequences than lanes; 64 rows
+    (2, 2, [1] * 64), (2, 2, [33] * 65),
+])
+def test_window_fp32_prompts_of_unequal_lengths(heads, kv_heads, seqs):
+    """Workgroups find their tile among those that are there, the last ones of all sequences first: every tile of every sequence is done, once."""
+    run_window(ops.WindowSpec(heads, kv_heads, 24, 40, 50, 3, 0.3), torch.float32, seqs, [[n] for n in seqs])
+    run_window(ops.WindowSpec(heads, kv_heads, 24, 40, 50, 3, 0.3), torch.float32, seqs, [[n // 3] * 2 + [n - 2 * (n // 3)] if n > 8 else [n] for n in seqs])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_decode_of_sequences_with_fewer_rows_than_the_batch_is_split_for(dtype):
     """A window of 1520 rows is split over twelve workgroups (127 rows each): sequences that fill one row, one share, one share and a

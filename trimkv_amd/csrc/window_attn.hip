@@ -79,21 +79,70 @@ __global__ __launch_bounds__(256) void window_rows_kernel(WindowArgs a) {
 // Bound by the matrix cores' fp32 rate (a sixteenth of bf16), 1.75 us a tile of 32 rows, and as much again of other vector instructions.  The longest
 // rows of all heads go first: with a head's workgroups one behind the other the launch ended on long ones, 16 heads of 128 (8 KV heads): three
 // prompts of 1000 tokens 300 us for 165, one of 4000 730 for 585.  300 + 511 tokens: 72 us with 64 rows in that order, 51 with 32; a
-// wavefront per query row, which this replaces for head sizes up to 128, took 1060 us there, bound by its row-wise loads.
+// wavefront per query row, which this replaces for head sizes up to 128, took 1060 us there, bound by its row-wise loads.  Rows that are not there come last
+// (row_tile_at): in between, where every eighth workgroup has work, those all go to a few compute units.  Prompts of 2238, 25, 3, 14, 35, 2, 40 and 40 tokens, 8 heads
+// of 96 (2 KV heads) 107 us for 499, of 2128 and 296, 16 of 128 295 for 428; finding the place takes 0.7 us.
 // NaNs and infinities of keys that a row does not see must not reach it through 0 x inf: tiles with such values in V take their
 // second product one key at a time.
+
+// Place `at` among the tiles of bt rows of all sequences (up to `tiles` of each), the last ones first: those of tile t stand behind those of all later
+// ones.  64 candidates for t at once: how many stand in front of the end of t is a sum over the sequences.
+struct RowTile { int b, tile, t0, len, slot; };      // b = -1: there are not as many
+__device__ __forceinline__ RowTile row_tile_at(const WindowArgs& a, int batch, int tiles, int bt, int at) {
+    const int lane = threadIdx.x & 63;
+    int start = 0, len = 0, slot = 0, own = 0;
+    auto take = [&](int b0) __attribute__((always_inline)) {      // sequences b0 .. b0 + 63, one to a lane
+        const int b = min(b0 + lane, batch - 1);
+        start = a.cu[b]; len = a.cu[b + 1] - start; slot = a.slots[b];
+        own = b0 + lane < batch ? min((max(len, 0) + bt - 1) / bt, tiles) : 0;
+    };
+    take(0);
+    if (batch == 1) {                                             // every lane has the sequence, the first one its number of tiles
+        own = __builtin_amdgcn_readfirstlane(own);
+        return {at < own ? 0 : -1, own - 1 - at, start, len, slot};
+    }
+    int lo = 0, span = tiles, upto;                               // t is in lo .. lo + span - 1; places up to the end of lo
+    do {
+        const int step = (span + 63) / 64, t = lo + lane * step;
+        int n = 0;
+        for (int b0 = 0; b0 < batch; b0 += 64) {
+            if (batch > 64) take(b0);
+            for (int j = 0; j < min(64, batch - b0); ++j) n += max(__builtin_amdgcn_readlane(own, j) - t, 0);
+        }
+        const unsigned long long behind = __ballot(n > at && lane * step < span);
+        if (!behind) return {-1, 0, 0, 0, 0};                     // in the first round only
+        const int l = 63 - __builtin_clzll(behind);
+        lo += l * step;
+        span = min(step, span - l * step);
+        upto = __builtin_amdgcn_readlane(n, l);
+    } while (span > 1);
+    int k = upto - at;                                            // from the last sequence that has the tile
+    for (int b0 = (batch - 1) / 64 * 64; b0 >= 0; b0 -= 64) {
+        if (batch > 64) take(b0);
+        const unsigned long long has = __ballot(own > lo);
+        const int n = __popcll(has);
+        if (k <= n) {
+            const int l = __builtin_ctzll(__ballot(own > lo && __popcll(has >> lane) == k));
+            return {b0 + l, lo, __builtin_amdgcn_readlane(start, l), __builtin_amdgcn_readlane(len, l), __builtin_amdgcn_readlane(slot, l)};
+        }
+        k -= n;
+    }
+    return {-1, 0, 0, 0, 0};
+}
+
 template <int DT, int ROWS>
-__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a, int tiles) {      // grid: KV heads of all sequences x tiles of rows (in z what y does not hold)
+__global__ __launch_bounds__(256) void window_prefill_f32_kernel(WindowArgs a, int batch, int tiles) {      // grid: KV heads x tiles of rows of all sequences (in z what y does not hold)
     constexpr int LD = DT + 4, DB = DT / 16, PIECES = DT / 4, LOADS = 64 * PIECES / 256, RW = ROWS / 16, KS = 4 / RW, KB = 4 / KS;
     extern __shared__ __attribute__((aligned(16))) char wf_lds[];
     float* const kt = (float*)wf_lds; float* const vt = kt + 64 * LD;
     int* const where = (int*)(vt + 64 * LD);          // position of every key of the tile; past the end: beyond all queries
     int* const odd = where + 64;                      // number of tiles + 1 whose V held something that is not finite
-    const int bg = blockIdx.x, b = bg / a.G, g = bg % a.G, slot = a.slots[b];
-    const int t0 = a.cu[b], len = a.cu[b + 1] - t0, per = a.H / a.G, bt = ROWS / per;
     // later times of all heads first: they walk the most tiles
-    const int nth = (int)(blockIdx.z * gridDim.y + blockIdx.y), first = (tiles - 1 - nth) * bt;
-    if (nth >= tiles || first >= len) return;                         // workgroup-uniform, before any barrier
+    const int per = a.H / a.G, bt = ROWS / per, g = blockIdx.x;
+    const RowTile mine = row_tile_at(a, batch, tiles, bt, (int)min(blockIdx.z * gridDim.y + blockIdx.y, 0x7fffffffu));
+    if (mine.b < 0) return;                           // workgroup-uniform, before any barrier
+    const int t0 = __builtin_amdgcn_readfirstlane(mine.t0), len = __builtin_amdgcn_readfirstlane(mine.len), slot = __builtin_amdgcn_readfirstlane(mine.slot);
+    const int first = __builtin_amdgcn_readfirstlane(mine.tile) * bt;
     const int past = a.seen[2 * slot], cap = a.keep + a.size, nring = min(past, cap), last = min(first + bt, len) - 1;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, gr = lane >> 4;
     const int kb0 = w / RW * KB, row = w % RW * 16 + c, t = min(first + row / per, last), h = g * per + row % per, i = past + t;
@@ -570,8 +619,9 @@ static int launch_window_rows_f32(const WindowArgs& a, int batch, int max_len, h
         if (dev >= 0) opted_in[dev] = true;
     }
     const int bt = ROWS / (a.H / a.G);
-    const int tiles = (max_len + bt - 1) / bt, y = std::min(tiles, 65535);
-    hipLaunchKernelGGL((window_prefill_f32_kernel<DT, ROWS>), dim3(batch * a.G, y, (tiles + y - 1) / y), dim3(256), LDS, s, a, tiles);
+    const int tiles = (max_len + bt - 1) / bt;
+    const int64_t all = (int64_t)tiles * batch, y = std::min<int64_t>(all, 65535);
+    hipLaunchKernelGGL((window_prefill_f32_kernel<DT, ROWS>), dim3(a.G, (unsigned)y, (unsigned)((all + y - 1) / y)), dim3(256), LDS, s, a, batch, tiles);
     return 0;
 }
 
