@@ -546,6 +546,12 @@ def test_linear_f32_of_prompts(rows, n, k):
     test_linear_f32_on_either_side_of_its_rules(torch.bfloat16, rows, n, k)
 
 
+@pytest.mark.parametrize("rows,n,k", [(4096, 16, 96), (4097, 16, 96), (4100, 5, 32), (2048, 32, 64), (2049, 32, 160), (2050, 17, 32)])
+def test_linear_f32_of_more_workgroups_than_compute_units(rows, n, k):
+    """Sixteen wavefronts to a workgroup up to 256 of them, four beyond."""
+    test_linear_f32_on_either_side_of_its_rules(torch.bfloat16, rows, n, k)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("width", [4, 30, 1028, 2048, 2052, 4096, 4100])
 def test_rms_rows_of_every_width(dtype, width):

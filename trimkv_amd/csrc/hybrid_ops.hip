@@ -718,10 +718,14 @@ extern "C" int trimkv_linear_f32(const float* x, int64_t x_stride, const void* w
     }
     if (dtype == TRIMKV_BF16 && k % 32 == 0) {
         const bf16_t* wb = (const bf16_t*)w;
-        // us of 64 outputs by four wavefronts | 16 by sixteen, 32 outputs of 4096 features: 2048 rows 18.4 | 12.6, 4096 19.9 | 28.2, 8192 37.5 | 50.4; 64 of
-        // them, 8192 rows: 45 | 91.  16 by four, 16 outputs of 2048 features: 4000 rows 9.3 | 7.3, 8286 18.0 | 18.4.
-        if (n > 32 ? rows >= 2048 : n > 16 && rows >= 3072)
+        // 16 outputs by sixteen wavefronts while every such workgroup has a compute unit, else 16 or 64 by four.  us by four | by sixteen: 16 outputs of 2048 features 4000
+        // rows 9.4 | 7.6, 4500 12.6 | 12.8, 9000 18.1 | 18.8, of 4096 features 4000 rows 17.9 | 17.7, 5500 23.5 | 27.2, 16000 45 | 52 (given up: 7500 31.6 |
+        // 29.3); 32 outputs of 4096 features (64 by four) 2048 rows 18.5 | 12.6, 2049 18.6 | 25.8, 8192 37.5 | 50.4; 64 of them, 8192 rows: 45 | 91.
+        const int64_t groups = (int64_t)((rows + 15) / 16) * ((n + 15) / 16);
+        if (n > 32 ? rows >= 2048 : n > 16 && groups > 256)
             hipLaunchKernelGGL((linear_f32_mfma_kernel<4, 4>), dim3((rows + 15) / 16, (n + 63) / 64), dim3(256), 0, st_, x, x_stride, wb, w_stride, out, rows, n, k);
+        else if (n <= 16 && groups > 256)
+            hipLaunchKernelGGL((linear_f32_mfma_kernel<1, 4>), dim3((rows + 15) / 16, 1), dim3(256), 0, st_, x, x_stride, wb, w_stride, out, rows, n, k);
         else
             hipLaunchKernelGGL((linear_f32_mfma_kernel<1, 16>), dim3((rows + 15) / 16, (n + 15) / 16), dim3(1024), 0, st_, x, x_stride, wb, w_stride, out, rows, n, k);
         return launch_status(fn);
