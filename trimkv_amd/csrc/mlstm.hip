@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256) void mlstm_recurrent_kernel(MlstmArgs a) {
 // mlstm_join_kernel chains them into the state each segment starts from, pass 2 computes the outputs.
 struct ChunkArgs {
     MlstmArgs a;
-    float* seg_S; float* seg_n; float* seg_g; float* seg_m;     // [batch * nseg][H] x (D Dv, D, 2: sum of f and stabiliser, 1)
+    float* seg_S; float* seg_n; float* seg_g; float* seg_m;     // [H][batch * nseg] x (D Dv, D, 2: sum of f and stabiliser, 1)
     int seg_len, nseg, batch;                                   // no longer than seg_len for sequences up to max_len, no more than batch * nseg in all
 };
 enum { CHUNK_WHOLE = 0, CHUNK_LOCAL = 1, CHUNK_OUTPUT = 2 };
@@ -153,41 +153,63 @@ enum { CHUNK_WHOLE = 0, CHUNK_LOCAL = 1, CHUNK_OUTPUT = 2 };
 // The segments of all sequences, one sequence after the other.  They are as short as the number of tokens that are there lets them be (a
 // multiple of `unit`; sum of ceil(len / s) <= T / s + batch), not as the longest sequence times the batch would, and workgroups without a
 // segment come last instead of in between, where they spoil the spread of the others over the compute units: prompts of 701, 3999, 1536
-// and 2050 tokens (8 heads of 128 x 256) 137 -> 111 us, of 16, 3000, 40, 100 and 512 107 -> 67; four of 4000 161 on either side.
+// and 2050 tokens (8 heads of 128 x 256) 128 -> 101 us, of 16, 3000, 40, 100 and 512 107 -> 63; four of 4000 144 on either side.  A head's segments follow each
+// other in memory: with the heads of a segment side by side (2 MB from one segment of 16 heads of 128 x 256 to the next) a launch of 93 us took 96.
 // seg_len alone bounds their number only while no sequence is longer than the caller's max_len.
-__device__ __forceinline__ int segment_length(const ChunkArgs& ca, int unit) {
-    const int room = ca.batch * (ca.nseg - 1), total = ca.a.cu[ca.batch] - ca.a.cu[0], most = ca.nseg * ca.seg_len;
-    bool longer = false;
-    for (int x = threadIdx.x & 63; x < ca.batch; x += 64) longer = longer || ca.a.cu[x + 1] - ca.a.cu[x] > most;
+// Looking a segment up stands in front of everything else: all that the first 64 sequences (nearly always all) say is requested at once, one to a lane.
+struct Sequences { int start, len, slot, seg_len; };
+__device__ __forceinline__ Sequences sequences(const ChunkArgs& ca, int unit) {
+    const int lane = threadIdx.x & 63, x = min(lane, ca.batch - 1), room = ca.batch * (ca.nseg - 1), most = ca.nseg * ca.seg_len;
+    const int start = ca.a.cu[x], end = ca.a.cu[x + 1], slot = ca.a.slots[x];
+    int total = __builtin_amdgcn_readlane(end, min(ca.batch, 64) - 1) - __builtin_amdgcn_readlane(start, 0);
+    bool longer = end - start > most;
+    if (ca.batch > 64) {
+        total = ca.a.cu[ca.batch] - ca.a.cu[0];
+        for (int y = lane; y < ca.batch; y += 64) longer = longer || ca.a.cu[y + 1] - ca.a.cu[y] > most;
+    }
     const int len = max(unit, ((total + room - 1) / room + unit - 1) / unit * unit);
-    return __ballot(longer) ? len : min(ca.seg_len, len);
+    return {start, lane < ca.batch ? max(end - start, 0) : 0, slot, __ballot(longer) ? len : min(ca.seg_len, len)};
 }
 __device__ __forceinline__ int segments_of(const ChunkArgs& ca, int b, int seg_len) {
     return b < ca.batch ? (max(ca.a.cu[b + 1] - ca.a.cu[b], 0) + seg_len - 1) / seg_len : 0;
 }
-// Sequence of segment `at`, and how many segments there are in front of the sequence's own; b = -1: there are not as many segments
-struct SegmentOf { int b, before; };
-__device__ __forceinline__ SegmentOf segment_at(const ChunkArgs& ca, int at, int seg_len) {
+// Sequence of segment `at` and how many segments there are in front of the sequence's own; b = -1: there are not as many segments
+struct SegmentOf { int b, before, start, len, slot; };
+__device__ __forceinline__ SegmentOf segment_at(const ChunkArgs& ca, const Sequences& q, int at) {
     const int lane = threadIdx.x & 63;
+    auto of_lane = [&](int l, int before) __attribute__((always_inline)) {
+        return SegmentOf{l, before, __builtin_amdgcn_readlane(q.start, l), __builtin_amdgcn_readlane(q.len, l), __builtin_amdgcn_readlane(q.slot, l)};
+    };
     int base = 0;
+    if (ca.batch <= 8) {
+        const int own = (q.len + q.seg_len - 1) / q.seg_len;
+        for (int l = 0; l < ca.batch; ++l) {
+            const int n = __builtin_amdgcn_readlane(own, l);
+            if (at < base + n) return of_lane(l, base);
+            base += n;
+        }
+        return {-1, 0, 0, 0, 0};
+    }
     for (int b0 = 0; b0 < ca.batch; b0 += 64) {
-        const int own = segments_of(ca, b0 + lane, seg_len);
+        const int own = b0 ? segments_of(ca, b0 + lane, q.seg_len) : (q.len + q.seg_len - 1) / q.seg_len;
         int upto = own;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) { const int o = __shfl_up(upto, d, 64); if (lane >= d) upto += o; }
         const unsigned long long behind = __ballot(base + upto > at);
         if (behind) {
-            const int l = __builtin_ctzll(behind);
-            return {b0 + l, base + __builtin_amdgcn_readlane(upto - own, l)};
+            const int l = __builtin_ctzll(behind), before = base + __builtin_amdgcn_readlane(upto - own, l), b = b0 + l;
+            if (!b0) return of_lane(l, before);
+            return {b, before, ca.a.cu[b], ca.a.cu[b + 1] - ca.a.cu[b], ca.a.slots[b]};
         }
         base += __builtin_amdgcn_readlane(upto, 63);
     }
-    return {-1, 0};
+    return {-1, 0, 0, 0, 0};
 }
-__device__ __forceinline__ int segments_before(const ChunkArgs& ca, int b, int seg_len) {
+__device__ __forceinline__ int segments_before(const ChunkArgs& ca, const Sequences& q, int b) {
+    if (b == 0) return 0;
     const int lane = threadIdx.x & 63;
-    int n = 0;
-    for (int x = lane; x < b; x += 64) n += segments_of(ca, x, seg_len);
+    int n = lane < b ? (q.len + q.seg_len - 1) / q.seg_len : 0;
+    for (int x = lane + 64; x < b; x += 64) n += segments_of(ca, x, q.seg_len);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d, 64);
     return __builtin_amdgcn_readfirstlane(n);
@@ -236,23 +258,24 @@ __global__ __launch_bounds__(256, DKT <= 4 ? 2 : 1) void mlstm_chunk_kernel(Chun
     float* const wgt = dsum + 96;                     // [4][64]: every wavefront's own copy of exp(d_s - M_C)
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 31, hl = lane >> 5;
     const int vt = (a.Dv + 127) / 128, nth = blockIdx.x / vt, dv0 = (blockIdx.x % vt) * 128, h = blockIdx.y;
-    int b = blockIdx.z, first = 0, seg_len = 0x7fffffff;
-    if (MODE != CHUNK_WHOLE) {
-        seg_len = segment_length(ca, 64);
-        const SegmentOf found = segment_at(ca, nth, seg_len);
+    int t0, len, slot, first = 0;                     // the sequence's first token, the segment's (of the sequence) and how many it holds
+    if (MODE == CHUNK_WHOLE) {
+        const int b = blockIdx.z;
+        t0 = a.cu[b]; len = a.cu[b + 1] - t0; slot = a.slots[b];
+    } else {
+        const Sequences all = sequences(ca, 64);
+        const SegmentOf found = segment_at(ca, all, nth);
         if (found.b < 0) return;                      // workgroup-uniform, before any barrier
-        b = found.b;
-        first = (nth - found.before) * seg_len;
+        first = (nth - found.before) * all.seg_len;
+        t0 = found.start; len = min(found.len - first, all.seg_len); slot = found.slot;
     }
-    const int t0 = a.cu[b], len_all = a.cu[b + 1] - t0, len = min(len_all - first, seg_len);
-    const int slot = a.slots[b];
     if (len <= 0) {                                   // workgroup-uniform, before any barrier (segments: mlstm_join_kernel carries n and m)
         if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
         return;
     }
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
-    const int64_t sat = (int64_t)nth * a.H + h;
+    const int64_t sat = (int64_t)h * (ca.batch * ca.nseg) + nth;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
     const int col = dv0 + w * 32 + j;
     const bool live = dv0 + w * 32 < a.Dv;            // wavefront-uniform
@@ -528,7 +551,8 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
     const MlstmArgs& a = ca.a;
     const int h = blockIdx.y, b = blockIdx.z, len = a.cu[b + 1] - a.cu[b], slot = a.slots[b];
     const int e = blockIdx.x * 256 + threadIdx.x, nS = a.D * a.Dv;
-    const int seg_len = segment_length(ca, 64), s0 = segments_before(ca, b, seg_len);
+    const Sequences all = sequences(ca, 64);
+    const int seg_len = all.seg_len, s0 = segments_before(ca, all, b);
     if (e >= nS + a.D) return;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
@@ -537,7 +561,7 @@ __global__ __launch_bounds__(256) void mlstm_join_kernel(ChunkArgs ca) {
     float* S = a.S + ((int64_t)slot * a.H + h) * nS;
     float m = fresh ? 0.0f : in[a.D] * LOG2E, cur = fresh ? 0.0f : e < nS ? S[e] : in[e - nS];
     for (int x = 0; x * seg_len < len; ++x) {
-        const int64_t s = (int64_t)(s0 + x) * a.H + h;
+        const int64_t s = (int64_t)h * (ca.batch * ca.nseg) + s0 + x;
         float* p = e < nS ? ca.seg_S + s * nS + e : ca.seg_n + s * a.D + (e - nS);
         const float own = *p, f = ca.seg_g[2 * s], ms = ca.seg_g[2 * s + 1];
         *p = cur;
@@ -593,20 +617,22 @@ __global__ __launch_bounds__(256) void mlstm_chunk_f32_kernel(ChunkArgs ca) {
     double* const gD = (double*)(cf_lds + C::G0); double* const gM = gD + TC; double* const gm = gM + TC;           // d_s, M_t; m_0 and F_C
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int vt = (a.Dv + 63) / 64, nth = blockIdx.x / vt, h = blockIdx.y, col0 = (blockIdx.x % vt) * 64, col = col0 + w * 16 + c;
-    int b = blockIdx.z, first = 0, seg_len = 0x7fffffff;
-    if (MODE != CHUNK_WHOLE) {
-        seg_len = segment_length(ca, TC);
-        const SegmentOf found = segment_at(ca, nth, seg_len);
+    int t0, len, slot;
+    if (MODE == CHUNK_WHOLE) {
+        const int b = blockIdx.z;
+        t0 = a.cu[b]; len = a.cu[b + 1] - t0; slot = a.slots[b];
+    } else {
+        const Sequences all = sequences(ca, TC);
+        const SegmentOf found = segment_at(ca, all, nth);
         if (found.b < 0) return;                      // workgroup-uniform, before any barrier
-        b = found.b;
-        first = (nth - found.before) * seg_len;
+        const int first = (nth - found.before) * all.seg_len;
+        t0 = found.start + first; len = min(found.len - first, all.seg_len); slot = found.slot;
     }
-    const int t0 = a.cu[b] + first, len = min(a.cu[b + 1] - t0, seg_len), slot = a.slots[b];
     if (len <= 0) {                                   // workgroup-uniform: there is no token to request (segments: the join carries n and m)
         if (MODE == CHUNK_WHOLE && blockIdx.x == 0) carry_norm(a, h, slot);
         return;
     }
-    const int64_t sat = (int64_t)nth * a.H + h;
+    const int64_t sat = (int64_t)h * (ca.batch * ca.nseg) + nth;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
     const int64_t copy = (int64_t)a.nslots * a.H * (a.D + 1), at = ((int64_t)slot * a.H + h) * (a.D + 1);
@@ -821,7 +847,8 @@ __global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca, int u
     const MlstmArgs& a = ca.a;
     const int h = blockIdx.y, b = blockIdx.z, len = a.cu[b + 1] - a.cu[b], slot = a.slots[b];
     const int e = (blockIdx.x * 256 + threadIdx.x) * 4, nS = a.D * a.Dv;        // D and Dv are multiples of 4
-    const int seg_len = segment_length(ca, unit), s0 = segments_before(ca, b, seg_len);
+    const Sequences all = sequences(ca, unit);
+    const int seg_len = all.seg_len, s0 = segments_before(ca, all, b);
     if (e >= nS + a.D) return;
     const bool fresh = a.seen[2 * slot] == 0;
     const int parity = a.seen[2 * slot + 1] & 1;
@@ -833,7 +860,7 @@ __global__ __launch_bounds__(256) void mlstm_join_f32_kernel(ChunkArgs ca, int u
 #pragma unroll
     for (int x = 0; x < 4; ++x) cur[x] = fresh ? 0.0 : (double)(e < nS ? S[e + x] : in[e - nS + x]);
     for (int y = 0; y * seg_len < len; ++y) {
-        const int64_t s = (int64_t)(s0 + y) * a.H + h;
+        const int64_t s = (int64_t)h * (ca.batch * ca.nseg) + s0 + y;
         float* p = e < nS ? ca.seg_S + s * nS + e : ca.seg_n + s * a.D + (e - nS);
         const double f = load_double(ca.seg_g + 4 * s), ms = load_double(ca.seg_g + 4 * s + 2), mn = fmax(f + m, ms);
         const double old = exp(f + m - mn), now = exp(ms - mn);
