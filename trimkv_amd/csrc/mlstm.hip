@@ -905,13 +905,14 @@ static int launch_chunked_f32(const ChunkArgs& c, int batch, hipStream_t s) {
 }
 static int chunk_f32_tokens(int dim) { return dim <= 128 ? 64 : 32; }
 // A segment of c chunks costs 24 us per chunk in its two passes and 20 for the join and the launches, a chain 16 per chunk.  Measured, chain | segments: 4
-// chunks in segments of one 65 | 41, of two 71 | 74; 10 in segments of five 160 | 129.
+// chunks in segments of one 65 | 41, of two 71 | 74; 10 in segments of five 160 | 129.  Chunks of 32 tokens (more than 128 features) 14 in a chain, and 34 for
+// the join of larger states: 4 in segments of one 56 | 58, 5 69 | 51.
 static int chunk_f32_segments(int batch, int max_len, int heads, int dim, int vdim) {
     const int64_t wgs = (int64_t)batch * heads * ((vdim + 63) / 64);
     const int chunks = (max_len + chunk_f32_tokens(dim) - 1) / chunk_f32_tokens(dim), n = (int)std::min<int64_t>(256 / wgs, chunks);
     if (n < 2) return 1;
     const int of = (chunks + n - 1) / n;
-    return 6 * of + 5 < 4 * chunks ? (chunks + of - 1) / of : 1;
+    return (dim > 128 ? 12 * of + 17 < 7 * chunks : 6 * of + 5 < 4 * chunks) ? (chunks + of - 1) / of : 1;
 }
 // Portions of a few tokens stay with the token-by-token kernel: a chunk costs 16 us however few tokens it holds, a token 2.6 us.
 constexpr int F32_CHUNK_FROM = 8;
