@@ -96,7 +96,8 @@ int trimkv_window_decode(const void* q, const void* ring_k, const void* ring_v, 
 /* mLSTM over portions (equations in csrc/mlstm.hip). gates [tokens][2 heads]: W_i h, W_f h without biases.  state
  * [slot][heads][dim][vdim]; norm_state [2][num_slots][heads][dim + 1] (n and m, by parity of the slot's steps).
  * out [tokens][heads][vdim] in dtype, before the head norm.  dim up to 512.  workspace: trimkv_mlstm_workspace(...) floats (0: NULL will do), for the states
- * between the segments of long prompts (fp32 without one: a single chain).  A sequence may bring no token (cu[b + 1] == cu[b], in a batch of others): its state
+ * between the segments of long prompts (fp32 without one: a single chain).  max_len: the longest sequence's tokens; less costs time, no token is left
+ * out and the workspace is not exceeded.  A sequence may bring no token (cu[b + 1] == cu[b], in a batch of others): its state
  * stays. */
 int64_t trimkv_mlstm_workspace(int batch, int max_len, int heads, int dim, int vdim, int dtype);
 int trimkv_mlstm(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* gates, const float* i_bias,

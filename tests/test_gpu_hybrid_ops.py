@@ -454,11 +454,11 @@ def test_experts_cut_into_runs(E, ff, width):
 
 @pytest.mark.parametrize("ff,width", [(352, 640), (704, 352)])
 def test_experts_whose_steps_go_round_the_buffers(ff, width):
-    """Prompt-sized products of 12, 20 and 22 steps of 32 k: the five operand buffers are filled anew two to four times while
-    wavefronts with none to four blocks of 32 rows read them, in full tiles and in tiles of every number of blocks."""
+    """Prompt-sized products of 6, 10 and 11 steps of 64 k: the operand buffers, two of them for tiles of 256 and 192 rows and three for tiles of 128, are
+    filled anew two to five times, with an even and an odd number of steps, in full tiles and in ones that hold any part of their rows."""
     counts = [0, 1, 33, 65, 97, 129, 161, 193, 225, 256, 257, 545]
     E, T, wp, fp = len(counts), sum(counts), ops.padded(width), ops.padded(ff)
-    assert T >= 96 * E and {wp // 32, fp // 32} in ({20, 12}, {12, 22})
+    assert T >= 96 * E and {wp // 64, fp // 64} in ({10, 6}, {6, 11})
     x, up, down = torch.zeros(T, wp), torch.zeros(E, fp, wp), torch.zeros(E, wp, fp)
     x[:, :width] = rnd(T, width, seed=1)
     up[:, :ff, :width] = rnd(E, ff, width, seed=2) * width ** -0.5

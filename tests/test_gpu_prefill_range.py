@@ -1,5 +1,6 @@
-"""GPU tests of the chunk-prefill attention where scores outgrow the exponent reference that a row began with: within what bf16's exponents take, beyond
-it (the workgroup's second, careful way), gradually (the reference moves by the row sums) and in fp16, against the fp32 oracle."""
+"""GPU tests of the chunk-prefill attention where scores outgrow the exponent reference that a row began with: within what bf16's exponents take, up to the last
+powers of two of a row sum, beyond them (the query tile is done again, with row maxima), gradually (the reference moves by the row sums) and in fp16, against
+64-bit sums."""
 import numpy as np
 import pytest
 import torch

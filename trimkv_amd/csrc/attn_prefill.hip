@@ -6,17 +6,21 @@
 // prefill (src/trimkv/attn/__init__.py:15-26): query t of the chunk sees every older cached token
 // plus the chunk's own tokens <= t, i.e. keys j <= n - Q_LEN + t.
 //
-// Two kernels share the formulation below.  prefill_attn_kernel (chunks of 64 queries and more) gives
-// a wavefront 32 queries, two groups of MFMA columns, on 64-key tiles that LDS-direct loads
-// rotate through four LDS buffers; prefill_small_kernel (short chunks) gives a wavefront
-// 16 queries on 32-key tiles.  Both use v_mfma_f32_16x16x32_bf16.
+// The kernels share the formulation below.
+//   prefill_small_kernel    chunks of fewer than 64 queries: 16 queries to a wavefront, 32-key tiles, 16x16x32 MFMAs, running row maxima
+//   prefill_attn_kernel     longer ones whose query tiles fill the chip: 32 queries to a wavefront, two groups of MFMA columns, on 64-key tiles that LDS-direct
+//                           loads rotate through four LDS buffers, 16x16x32 MFMAs, wavefronts half a block apart; fp16 keeps row maxima, bf16 none (ATTEND_SUMS)
+//   prefill_shares_kernel   the same loop over equal shares of all keys, whose outputs prefill_merge_kernel puts together (trimkv_prefill_attn_shares)
+//   few::prefill_few_kernel little work, or keys divided by sizes (trimkv_prefill_attn_split): 32 queries to a wavefront, 32x32x16 MFMAs, all
+//                           wavefronts in step, row maxima (attn_prefill_few.hip.h)
+// Which of them takes a call: launch_prefill, trimkv_prefill_split_tiles and trimkv_prefill_equal_shares.
 //
 // A workgroup owns BT consecutive query times of one segment for all G query heads of its KV head,
 // one wavefront per (head, 16 or 32 times), so a K/V tile staged in LDS is shared by the whole group.
 // Per tile a wavefront computes
 //     S^T[key][query] = K . Q^T           (A = K rows from LDS, B = Q rows held in registers)
 //     O^T[d][query]  += V^T . P^T         (A = V columns gathered from LDS, B = P^T)
-// Both products put the query on the MFMA column index, which is the lane index modulo 16: every
+// Both products put the query on the MFMA column index, which is the lane index modulo 16 (32 for 32x32x16): every
 // per-query quantity (running max, sum, rescale factor) lives in the lane that needs it, and the
 // probabilities a lane holds after the first product are exactly the keys its B operand of the
 // second product wants -- P never crosses lanes.  V is row-major in memory, so its A operand
