@@ -104,6 +104,13 @@ def build(verbose: bool = True, only_changed: bool = False, libraries=(*LIBRARIE
     return LIBRARIES[libraries[-1]][0]
 
 
+def ensure(libraries) -> None:
+    """Build those of the named libraries that are not there (``bin/trace_run`` in a fresh checkout: what its model needs)."""
+    missing = tuple(n for n in libraries if not os.path.exists(STEP_PATH if n == "step" else LIBRARIES[n][0]))
+    if missing:
+        build(verbose=False, only_changed=True, libraries=missing)
+
+
 if __name__ == "__main__":
     names = [a for a in sys.argv[1:] if not a.startswith("--")]
     build(only_changed="--changed" in sys.argv[1:], libraries=tuple(names) or (*LIBRARIES, "step"))
