@@ -36,6 +36,12 @@ int trimkv_embed_scaled(const int64_t* ids, const void* table, float scale, floa
  * three bf16 terms).  k and x_stride multiples of 4, w_stride a multiple of 8; 16-byte aligned. */
 int trimkv_linear_f32(const float* x, int64_t x_stride, const void* w, int64_t w_stride, float* out, int rows, int n, int k, int dtype, void* stream);
 
+/* out[m][n] = sum_k x[m][k] w[n][k] in fp32: a linear layer over many rows, the tokens of a prompt (each number split exactly into three bf16 terms, six of the
+ * nine products taken, fp32 sums; blocks whose results are not finite once more by fp32 products).  k a multiple of 32, strides of x and w multiples of 4 up to 2^20, x and w
+ * 16-byte aligned; rows, n <= 2^22.  form: how the launch is cut, 0: by sizes.  _form: what that is. */
+int trimkv_linear_f32_tiles(const float* x, int64_t x_stride, const float* w, int64_t w_stride, float* out, int64_t out_stride, int rows, int n, int k, int form, void* stream);
+int trimkv_linear_f32_tiles_form(int rows, int n, int k);
+
 /* x[t] += mult * w * y' / sqrt(mean(y'^2) + eps), y' = y[t] or, with y_weight [tokens][top], sum_j y_weight[t][j] * y[t * top + j].
  * xh (optional): the new x in dtype, same stride, or with next_w (needs xh) its RMS norm times that weight. width <= 16384. */
 int trimkv_residual_norm(const void* y, int64_t y_stride, const float* y_weight, int top, float* x, const float* w, float mult, void* xh,

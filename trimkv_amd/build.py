@@ -21,7 +21,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB_PATH = os.path.join(HERE, "libtrimkv_hip.so")
 STEP_PATH = os.path.join(HERE, "_step.so")
 SOURCES = ["api.hip", "append.hip", "evict.hip", "attn_decode.hip", "attn_decode_append.hip", "attn_decode_pieces.hip", "attn_decode_append_pieces.hip", "attn_decode_append_gated.hip", "attn_decode_append_pieces_gated.hip", "pieces_plan.hip", "attn_prefill.hip", "gate.hip", "stream_probe.hip", "decoder_ops.hip", "linear_rows.hip", "linear_tiles.hip"]
-HYBRID_SOURCES = ["hybrid_ops.hip", "window_attn.hip", "window_decode.hip", "linear_rows.hip", "linear_tiles.hip"]
+HYBRID_SOURCES = ["hybrid_ops.hip", "window_attn.hip", "window_decode.hip", "linear_rows.hip", "linear_tiles.hip", "linear_f32_tiles.hip"]
 LIBRARIES = {"hip": (LIB_PATH, SOURCES), "hybrid": (os.path.join(HERE, "libtrimkv_hybrid.so"), HYBRID_SOURCES),
              "mlstm": (os.path.join(HERE, "libtrimkv_mlstm.so"), ["mlstm.hip"]), "moe": (os.path.join(HERE, "libtrimkv_moe.so"), ["moe.hip"])}
 

@@ -1,7 +1,7 @@
-"""Linear layers over the rows of a decode step on trimkv_linear_rows and over those of a prompt on trimkv_linear_tiles; everything else goes to
-``F.linear``.
+"""Linear layers over the rows of a decode step on trimkv_linear_rows and over those of a prompt on trimkv_linear_tiles, those of the hybrid decoders in fp32 on
+trimkv_linear_f32_tiles; everything else goes to ``F.linear``.
 
-Both give fp32 sums rounded once; the order of the sums differs.
+All give fp32 sums rounded once; the order of the sums differs.
 """
 from __future__ import annotations
 
@@ -42,10 +42,10 @@ def watched() -> bool:
             or (torch._C._len_torch_function_stack() > 0 and any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())))
 
 
-def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary tensors of one 16-bit dtype on the current GPU that nobody differentiates, casts or follows."""
+def _plain(*tensors: Optional[torch.Tensor], dtypes=(torch.bfloat16, torch.float16)) -> bool:
+    """Ordinary tensors of one dtype (of 16 bits, if not told otherwise) on the current GPU that nobody differentiates, casts or follows."""
     first = tensors[0]
-    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or watched():
+    if not first.is_cuda or first.dtype not in dtypes or torch.is_autocast_enabled("cuda") or watched():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
@@ -106,8 +106,48 @@ def _prompt_rows(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     return x2, form
 
 
+@functools.lru_cache(maxsize=4096)
+def _f32_form(rows: int, n: int, k: int, library: str) -> int:
+    return _lib.load_hybrid(library).trimkv_linear_f32_tiles_form(rows, n, k)
+
+
+def _f32_rows(x: torch.Tensor, weight: torch.Tensor, library: str):
+    """``(x as [rows, k], form)`` the way trimkv_linear_f32_tiles takes this product, or None where it does not or is not faster."""
+    k = x.shape[-1] if x.dim() else 0
+    if torch.compiler.is_compiling() or k == 0 or weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0:
+        return None
+    rows, n = x.numel() // k, weight.shape[0]
+    if type(rows) is not int or type(n) is not int or not 0 < rows <= 1 << 22 or n > 1 << 22:
+        return None
+    form = _f32_form(rows, n, k, library)
+    if not form or not _plain(x, weight, dtypes=(torch.float32,)) or weight.stride(1) != 1 or weight.stride(0) < k or weight.stride(0) % 4 or weight.data_ptr() % 16:
+        return None
+    if x.dim() != 2 and not x.is_contiguous():
+        return None
+    x2 = x if x.dim() == 2 else x.view(-1, k)
+    if x2.stride(1) != 1 or x2.data_ptr() % 16 or x2.stride(0) < k or x2.stride(0) % 4 or max(x2.stride(0), weight.stride(0)) > 1 << 20:
+        return None
+    return x2, form
+
+
+def _f32_product(x: torch.Tensor, weight: torch.Tensor, library: str) -> torch.Tensor:
+    many = _f32_rows(x, weight, library)
+    if many is None:
+        return F.linear(x, weight)
+    x2, form = many
+    (rows, k), n = x2.shape, weight.shape[0]
+    out = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
+    rc = _lib.load_hybrid(library).trimkv_linear_f32_tiles(x2.data_ptr(), x2.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), n, rows, n, k, form,
+                                                           _lib.current_stream(x.device))
+    if rc:
+        _lib.check_hybrid(rc, "trimkv_linear_f32_tiles", library)
+    return out
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, library: Optional[str] = None) -> torch.Tensor:
     """``F.linear(x, weight, bias)``.  ``library``: which one holds the kernel (a name of ``_lib.SHARED``; None: libtrimkv_hip.so)."""
+    if library is not None and bias is None and x.dtype == torch.float32:
+        return _f32_product(x, weight, library)
     k, size = x.shape[-1] if x.dim() else 0, x.numel()
     if size > MAX_ROWS * k:
         if size * weight.numel() < LEAST_OUTPUTS * k * k:
