@@ -116,6 +116,10 @@ int trimkv_head_norm_gate(const void* o, const void* gate, int64_t gate_stride, 
 /* seen[slots[b]] += {cu[b+1] - cu[b], 1}. */
 int trimkv_advance(int32_t* seen, const int32_t* slots, const int32_t* cu, int batch, void* stream);
 
+/* out[i] = values[i] and seen[slots[i]] = {0, 0}: values and slots are HOST pointers, read before the call returns (they travel in launches' arguments). */
+int trimkv_put_words(int32_t* out, const int32_t* values, int count, void* stream);
+int trimkv_reset_slots(int32_t* seen, const int32_t* slots, int count, int num_slots, void* stream);
+
 /* Sigmoid routing: choice = sigmoid(logits) + correction; `keep_groups` of `groups` equal groups of neighbours with the
  * largest sums of their two largest choices are open; the `top` largest open choices win (lower index first among equals).
  * weights: the plain sigmoids of the chosen. experts <= 1024. */

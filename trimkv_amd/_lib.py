@@ -127,6 +127,8 @@ HYBRID_SIGNATURES = {
         "trimkv_window_decode": (_i, [_p, _p, _p, _p, _p, _p, _i64, _p, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _p, _i, _p]),
         "trimkv_head_norm_gate": (_i, [_p, _p, _i64, _p, _p, _i, _i, _i, _f, _i, _p]),
         "trimkv_advance": (_i, [_p, _p, _p, _i, _p]),
+        "trimkv_put_words": (_i, [_p, _p, _i, _p]),
+        "trimkv_reset_slots": (_i, [_p, _p, _i, _i, _p]),
     },
     "mlstm": {
         "trimkv_mlstm_last_error": (C.c_char_p, []),

@@ -14,6 +14,7 @@
 //   trimkv_ring_store      the rows of a prompt that outlive it, into the window ring
 //   trimkv_head_norm_gate  per-head RMS norm, weight and sigmoid gate behind a recurrence
 //   trimkv_advance         tokens and steps seen per sequence slot
+//   trimkv_put_words       a few words from host memory, trimkv_reset_slots: slots that have seen nothing
 #include "hybrid.hip.h"
 #include <type_traits>
 
@@ -676,6 +677,20 @@ __global__ void advance_kernel(int32_t* seen, const int32_t* slots, const int32_
     seen[2 * slot + 1] += 1;
 }
 
+// A few numbers of the host's travel in a launch's arguments: a copy from pageable memory would wait for all that the stream holds.
+constexpr int PUT_WORDS = 512;
+struct PutWords { int32_t v[PUT_WORDS]; };
+
+__global__ void put_words_kernel(int32_t* out, PutWords p, int count) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i < count) out[i] = p.v[i];
+}
+
+__global__ void reset_slots_kernel(int32_t* seen, PutWords p, int count) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i < count) seen[2 * (int64_t)p.v[i]] = seen[2 * (int64_t)p.v[i] + 1] = 0;
+}
+
 }  // namespace trimkv
 
 using namespace trimkv;
@@ -902,5 +917,33 @@ extern "C" int trimkv_advance(int32_t* seen, const int32_t* slots, const int32_t
     if (!seen || !slots || !cu) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
     if (batch <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: bad batch %d", fn, batch);
     hipLaunchKernelGGL(advance_kernel, dim3((batch + 63) / 64), dim3(64), 0, (hipStream_t)stream, seen, slots, cu, batch);
+    return launch_status(fn);
+}
+
+extern "C" int trimkv_put_words(int32_t* out, const int32_t* values, int count, void* stream) {
+    const char* fn = "trimkv_put_words";
+    if (!out || !values) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (count <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: bad count %d", fn, count);
+    for (int at = 0; at < count; at += PUT_WORDS) {
+        const int n = count - at < PUT_WORDS ? count - at : PUT_WORDS;
+        PutWords p;
+        for (int i = 0; i < n; ++i) p.v[i] = values[at + i];
+        hipLaunchKernelGGL(put_words_kernel, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream, out + at, p, n);
+    }
+    return launch_status(fn);
+}
+
+extern "C" int trimkv_reset_slots(int32_t* seen, const int32_t* slots, int count, int num_slots, void* stream) {
+    const char* fn = "trimkv_reset_slots";
+    if (!seen || !slots) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (count <= 0) return fail(TRIMKV_ERR_SHAPE, "%s: bad count %d", fn, count);
+    for (int i = 0; i < count; ++i)
+        if (slots[i] < 0 || slots[i] >= num_slots) return fail(TRIMKV_ERR_SHAPE, "%s: slot %d of %d", fn, slots[i], num_slots);
+    for (int at = 0; at < count; at += PUT_WORDS) {
+        const int n = count - at < PUT_WORDS ? count - at : PUT_WORDS;
+        PutWords p;
+        for (int i = 0; i < n; ++i) p.v[i] = slots[at + i];
+        hipLaunchKernelGGL(reset_slots_kernel, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream, seen, p, n);
+    }
     return launch_status(fn);
 }

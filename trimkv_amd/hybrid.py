@@ -450,7 +450,7 @@ class HybridForCausalLM(GreedyGeneration, nn.Module):
             for n in batch.lengths:
                 at += n
                 ends += range(at - keep, at)
-            rows = torch.tensor(ends, device=x.device)
+            rows = ops.put(ends, torch.int64, x.device)
             shape = (B, keep)
         else:
             shape = (-1,) if rows is not None or min(batch.lengths) != batch.max_len else (B, batch.max_len)

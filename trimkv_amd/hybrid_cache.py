@@ -13,7 +13,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from .hybrid_ops import PackedBatch, advance
+from .hybrid_ops import PackedBatch, advance, put, reset_slots
 
 try:
     from transformers.cache_utils import Cache as _CacheBase
@@ -63,8 +63,10 @@ class HybridCache(_CacheBase):
         """``n`` fresh sequences at the end of the batch; returns their slots."""
         if len(self._free) < n:
             self._grow(max(self.num_slots - len(self._free) + n, self.num_slots + self.num_slots // 2))
-        slots, self._free = self._free[:n], self._free[n:]
-        self.seen[torch.tensor(slots, device=self.device)] = 0
+        slots = self._free[:n]
+        if slots:
+            reset_slots(self.seen, slots)
+        self._free = self._free[n:]
         for s in slots:
             self.tokens_seen[s] = 0
         self.active += slots
@@ -93,7 +95,7 @@ class HybridCache(_CacheBase):
             cu = [0]
             for n in lengths:
                 cu.append(cu[-1] + n)
-            both = torch.tensor(cu + list(slots), dtype=torch.int32).to(self.device)
+            both = put(cu + list(slots), torch.int32, self.device)
             hit = self._batches[(lengths, slots)] = (both[:len(cu)], both[len(cu):])
         return PackedBatch(lengths, slots, hit[0], hit[1], self.seen, self.num_slots)
 
