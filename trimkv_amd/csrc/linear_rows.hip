@@ -118,11 +118,12 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         const int row = 8 * j + (lane >> 3);
         x_off[j] = (uint32_t)(min(row, a.m - 1) * a.x_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
     }
-    const int steps = a.k >> 6, first = min(wave, steps - 1), per_tile = (steps - wave + W - 1) / W, tiles = (a.n + COLS * NB - 1) / (COLS * NB);
+    const int steps = a.k >> 6, first = wave, per_tile = (steps - wave + W - 1) / W, tiles = (a.n + COLS * NB - 1) / (COLS * NB);
     // the first column of block b of a tile: the last block of out is moved back so that all its rows exist
     auto block_at = [&](int tile, int b) __attribute__((always_inline)) { return min((tile * NB + b % NB) * COLS, max(a.n - COLS, 0)); };
-    int ask_tile = blockIdx.x, ask_step = first, ask_slot = 0;
-    auto request = [&]() __attribute__((always_inline)) {
+    int ask_tile = blockIdx.x, ask_step = first, ask_slot = 0, left = per_tile * ((tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
+    auto request = [&]() __attribute__((always_inline)) {       // left: steps that have not been requested; below 0 fewer than D are on their way
+        if (--left < 0) return;
         const uint32_t to = ring_at + ask_slot * STEP;
 #pragma unroll
         for (int b = 0; b < NT; ++b) {
@@ -133,9 +134,9 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
         for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (WG * NT + j) * 1024);
         ask_step += W;
-        if (ask_step >= steps) {        // behind the last tile: its steps again, never read
+        if (ask_step >= steps) {
             ask_step = first;
-            ask_tile = min(ask_tile + (int)gridDim.x, tiles - 1);
+            ask_tile += (int)gridDim.x;
         }
         ask_slot = ask_slot + 1 == D ? 0 : ask_slot + 1;
     };
@@ -156,7 +157,9 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
         for (int d = 1; d < ROW_THREADS; d <<= 1) sum += __shfl_xor(sum, d, 64);
         if (threadIdx.x % ROW_THREADS == 0) scale[threadIdx.x / ROW_THREADS] = rsqrtf(sum / (float)a.k + a.eps);
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(D * L) : "memory");       // weight and scales are there for all wavefronts
+        // weight and scales are there for all wavefronts
+        if (left >= 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(D * L) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
         for (int t = 0; t < MT; ++t) inv[t] = scale[XG == 1 ? r & 7 : t * 16 + r];
     }
@@ -166,7 +169,8 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
         for (int u = 0; u < U; ++u) acc[u] = lr_f32x4{0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s < per_tile; ++s) {
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * L) : "memory");
+            if (left >= 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * L) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             const char* p = mine + slot * STEP;
             lr_u32x4 wf[2][NT], xf[2][MT], nf[2];
 #pragma unroll
@@ -265,7 +269,6 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
                     if (n + c < a.n) o[c] = v[c];
         }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // loads into LDS that nobody reads have landed
 }
 
 constexpr int LR_CUS = 256;
@@ -299,27 +302,34 @@ static void rows_launch(const LinearRowsArgs& a, hipStream_t s) {
     const int tiles = (a.n + COLS * NB - 1) / (COLS * NB), most = LR_CUS * (160 * 1024 / LDS);
     hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NT, W, D, HALF>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
 }
-// wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 6 over the shapes above
+// Wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 8 over the shapes above.  Eight wavefronts where their steps fit: each has half as many steps, one
+// behind the other, and up to 8 KB of a step of all are asked for before the first one is used.  Four wavefronts and requests behind the last step, which nobody
+// read -> eight and none, us: add 2048 x 2048 with 4, 16, 32 rows 4.8 -> 4.4, 5.5 -> 5.0, 6.9 -> 6.0, 2048 x 6144 7.7 -> 6.7, 9.2 -> 9.0, 12.2 -> 11.8, 4096 x 4096 8.4 -> 8.1,
+// 9.4 -> 9.0, 10.8 -> 10.5; norm 4608 x 2048 7.6 -> 6.9, 8.3 -> 7.7, 10.9 -> 9.0, 6656 x 4096 14.5 -> 13.7, 15.5 -> 14.0, 17.6 -> 15.9; norm and silu 2 x 6144 x 2048 13.7 -> 12.4,
+// 14.3 -> 12.5, 15.3 -> 14.4, 2 x 12288 x 4096 33.3 -> 32.4, 34.4 -> 32.7, 41.1 -> 39.3.  64 rows, four wavefronts: 4096 x 4096 13.9 -> 13.4, 12288 x 4096 23.8 -> 23.2, 1024 x 4096 11.5 -> 11.1.
 template <bool F16, int XG, int MODE = LR_PLAIN>
 static void rows_by_blocks(const LinearRowsArgs& a, bool silu, hipStream_t s) {
     const int nt = rows_plan(a.n, 8 * XG, silu, MODE != LR_NORM);
     if constexpr (MODE != LR_NORM)
-        if (nt == 0) return rows_launch<F16, false, XG, 1, 4, XG < 4 ? 4 : XG < 8 ? 3 : 2, MODE, true>(a, s);
-    if constexpr (MODE == LR_NORM) {
-        if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, XG < 4 ? 3 : 2, MODE>(a, s);
-        if (silu) return rows_launch<F16, true, XG, 2, 4, 3, MODE>(a, s);
-        if (nt == 2) return rows_launch<F16, false, XG, 2, 4, 3, MODE>(a, s);
-    } else if constexpr (MODE == LR_ADD) {
-    } else if constexpr (XG == 8) {
+        if (nt == 0) return rows_launch<F16, false, XG, 1, XG == 8 ? 4 : 8, XG == 1 ? 4 : 2, MODE, true>(a, s);
+    if constexpr (XG == 8) {
         if (silu && nt == 6) return rows_launch<F16, true, 8, 6, 4, 1>(a, s);
         if (silu && nt == 4) return rows_launch<F16, true, 8, 4, 2, 2>(a, s);
-        if (!silu && nt == 6) return rows_launch<F16, false, 8, 6, 4, 1>(a, s);
-    } else if (silu && nt == 4) return rows_launch<F16, true, XG, 4, 4, 2>(a, s);
-    if constexpr (MODE == LR_PLAIN)
-        if (silu) return rows_launch<F16, true, XG, 2, 4, 2>(a, s);
-    if (nt == 1) rows_launch<F16, false, XG, 1, 4, XG < 4 ? 3 : 2, MODE>(a, s);
-    else if (nt == 2) rows_launch<F16, false, XG, 2, 4, 2, MODE>(a, s);
-    else rows_launch<F16, false, XG, 3, 4, 2, MODE>(a, s);
+        if (silu) return rows_launch<F16, true, 8, 2, 4, 2>(a, s);
+        if (nt == 6) return rows_launch<F16, false, 8, 6, 4, 1>(a, s);
+        if (nt == 1) return rows_launch<F16, false, 8, 1, 4, 2>(a, s);
+        if (nt == 2) return rows_launch<F16, false, 8, 2, 4, 2>(a, s);
+        return rows_launch<F16, false, 8, 3, 4, 2>(a, s);
+    } else {
+        constexpr int D = XG == 4 ? 1 : 2;
+        if constexpr (MODE != LR_ADD) {
+            if (silu && nt == 4) return rows_launch<F16, true, XG, 4, XG == 4 ? 4 : 8, XG == 4 ? 2 : 1, MODE>(a, s);
+            if (silu) return rows_launch<F16, true, XG, 2, 8, D, MODE>(a, s);
+        }
+        if (nt == 1) return rows_launch<F16, false, XG, 1, 8, 2, MODE>(a, s);
+        if (nt == 2) return rows_launch<F16, false, XG, 2, 8, D, MODE>(a, s);
+        rows_launch<F16, false, XG, 3, MODE == LR_NORM ? 4 : 8, MODE == LR_NORM ? 2 : D, MODE>(a, s);      // (LDS: the norm's weight beside it)
+    }
 }
 template <bool F16>
 static void rows_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
