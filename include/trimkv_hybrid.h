@@ -47,6 +47,11 @@ int trimkv_linear_f32_tiles_form(int rows, int n, int k);
 int trimkv_residual_norm(const void* y, int64_t y_stride, const float* y_weight, int top, float* x, const float* w, float mult, void* xh,
                          const float* next_w, int tokens, int width, int x_stride, float eps, int dtype, void* stream);
 
+/* Behind the last layer of a step: out[t] [width] in dtype = the RMS norm times out_w of what trimkv_residual_norm would make of x[t] (x stays as it is), and what
+ * trimkv_advance does (batch <= tokens). */
+int trimkv_last_norm(const void* y, int64_t y_stride, const float* y_weight, int top, const float* x, int x_stride, const float* w, float mult, void* out,
+                     const float* out_w, int tokens, int width, float eps, int32_t* seen, const int32_t* slots, const int32_t* cu, int batch, int dtype, void* stream);
+
 /* out[i] = w * x[r] / sqrt(mean(x[r]^2) + eps) with r = rows[i] (NULL: r = i); out [count][width] in dtype. */
 int trimkv_rms_rows(const float* x, int x_stride, const int64_t* rows, const float* w, void* out, int count, int width, float eps, int dtype, void* stream);
 

@@ -115,6 +115,7 @@ HYBRID_SIGNATURES = {
         "trimkv_linear_f32_tiles": (_i, [_p, _i64, _p, _i64, _p, _i64, _i, _i, _i, _i, _p]),
         "trimkv_linear_f32_tiles_form": (_i, [_i, _i, _i]),
         "trimkv_residual_norm": (_i, [_p, _i64, _p, _i, _p, _p, _f, _p, _p, _i, _i, _i, _f, _i, _p]),
+        "trimkv_last_norm": (_i, [_p, _i64, _p, _i, _p, _i, _p, _f, _p, _p, _i, _i, _f, _p, _p, _p, _i, _i, _p]),
         "trimkv_rms_rows": (_i, [_p, _i, _p, _p, _p, _i, _i, _f, _i, _p]),
         "trimkv_qkv_norm": (_i, [_p, _i64, _i, _i, _i, _p, _p, _f, _i, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p]),
         "trimkv_rotary_table": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _p]),

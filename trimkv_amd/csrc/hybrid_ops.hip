@@ -205,9 +205,13 @@ struct ResidualNormArgs {
     const void* y; int64_t y_stride; const float* y_weight; int top;
     float* x; const float* w; void* xh; int width, xs; float eps;
     float mult; const float* next_w;                  // next_w: xh = next_w * rms(new x) instead of a copy
+    int64_t hs;                                       // rows of xh are that far apart
+    int32_t* seen; const int32_t* slots; const int32_t* cu; int batch;      // LAST: the step's tokens count from now on
 };
+// LAST: behind the last layer, whose x nobody reads any more: it stays as it is, and with it go the launches of the model's norm and of
+// trimkv_advance.  8286 rows of 2048 in one trace each: 34 + 17 + 5 us, now 29.
 // NV > 0: rows of up to 1024 NV elements, four at a time, held in registers; everything is requested before the reduction.
-template <typename T, int NV>
+template <typename T, int NV, bool LAST>
 __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) {
     extern __shared__ float row[];     // NV = 0: width floats, y of this token summed over its experts
     __shared__ float part[4], part2[4];
@@ -215,8 +219,13 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
     const int tid = threadIdx.x;
     const T* y = (const T*)a.y + t * a.top * a.y_stride;
     float* xr = a.x + t * a.xs;
-    T* hr = (T*)a.xh + t * a.xs;
+    T* hr = (T*)a.xh + t * a.hs;
     float ss = 0.0f;
+    if (LAST && t < a.batch && tid == 0) {
+        const int slot = a.slots[t];
+        a.seen[2 * slot] += a.cu[t + 1] - a.cu[t];
+        a.seen[2 * slot + 1] += 1;
+    }
     if constexpr (NV > 0) {
         float4 s[NV], f[NV], w[NV];
 #pragma unroll
@@ -250,14 +259,14 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
             const int i = (v * 256 + tid) * 4;
             if (i < a.width) {
                 f[v].x += s[v].x * inv * w[v].x; f[v].y += s[v].y * inv * w[v].y; f[v].z += s[v].z * inv * w[v].z; f[v].w += s[v].w * inv * w[v].w;
-                *(float4*)(xr + i) = f[v];
-                if (a.next_w) {
+                if (!LAST) *(float4*)(xr + i) = f[v];
+                if (LAST || a.next_w) {
                     s2 += f[v].x * f[v].x + f[v].y * f[v].y + f[v].z * f[v].z + f[v].w * f[v].w;
                     w[v] = *(const float4*)(a.next_w + i);
                 } else if (a.xh) st4(hr + i, f[v]);
             }
         }
-        if (!a.next_w) return;
+        if (!LAST && !a.next_w) return;
         const float inv2 = 1.0f / sqrtf(block_sum_f(s2, part2, 4) / (float)a.width + a.eps);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
@@ -276,7 +285,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
         float s2 = 0.0f;
         for (int i = tid; i < a.width; i += 256) {      // a thread re-reads what it wrote itself
             const float f = xr[i] + row[i] * inv * a.w[i];
-            xr[i] = f;
+            if (!LAST) xr[i] = f;
             row[i] = f;
             s2 += f * f;
             if (a.xh && !a.next_w) st(hr + i, f);
@@ -750,24 +759,36 @@ extern "C" int trimkv_linear_f32(const float* x, int64_t x_stride, const void* w
     return launch_status(fn);
 }
 
+template <bool LAST>
+static int residual_norm_launch(const char* fn, const ResidualNormArgs& a, int tokens, int dtype, void* stream) {
+    HY_CHECK_DTYPE(fn, dtype);
+    if (tokens <= 0 || a.width <= 0 || a.width > 16384 || a.top < 1 || a.xs < a.width || a.y_stride < a.width || a.hs < a.width)
+        return fail(TRIMKV_ERR_SHAPE, "%s: bad sizes tokens=%d width=%d top=%d", fn, tokens, a.width, a.top);
+    if (!a.y_weight && a.top != 1) return fail(TRIMKV_ERR_SHAPE, "%s: several rows per token need weights", fn);
+    const bool vec = a.width % 4 == 0 && a.xs % 4 == 0 && a.y_stride % 4 == 0 && a.hs % 4 == 0 && !(((uintptr_t)a.y | (uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.xh | (uintptr_t)a.next_w) & 15);
+    const size_t lds = (size_t)a.width * 4;
+    HY_BY_DTYPE(dtype, T,
+        if (vec && a.width <= 1024) hipLaunchKernelGGL((residual_norm_kernel<T, 1, LAST>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
+        else if (vec && a.width <= 2048) hipLaunchKernelGGL((residual_norm_kernel<T, 2, LAST>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
+        else if (vec && a.width <= 4096) hipLaunchKernelGGL((residual_norm_kernel<T, 4, LAST>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
+        else if (vec && a.width <= 8192) hipLaunchKernelGGL((residual_norm_kernel<T, 8, LAST>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL((residual_norm_kernel<T, 0, LAST>), dim3(tokens), dim3(256), lds, (hipStream_t)stream, a));
+    return launch_status(fn);
+}
+
 extern "C" int trimkv_residual_norm(const void* y, int64_t y_stride, const float* y_weight, int top, float* x, const float* w, float mult, void* xh,
                                     const float* next_w, int tokens, int width, int x_stride, float eps, int dtype, void* stream) {
     const char* fn = "trimkv_residual_norm";
     if (!y || !x || !w || (next_w && !xh)) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
-    HY_CHECK_DTYPE(fn, dtype);
-    if (tokens <= 0 || width <= 0 || width > 16384 || top < 1 || x_stride < width || y_stride < width)
-        return fail(TRIMKV_ERR_SHAPE, "%s: bad sizes tokens=%d width=%d top=%d", fn, tokens, width, top);
-    if (!y_weight && top != 1) return fail(TRIMKV_ERR_SHAPE, "%s: several rows per token need weights", fn);
-    ResidualNormArgs a{y, y_stride, y_weight, top, x, w, xh, width, x_stride, eps, mult, next_w};
-    const bool vec = width % 4 == 0 && x_stride % 4 == 0 && y_stride % 4 == 0 && !(((uintptr_t)y | (uintptr_t)x | (uintptr_t)w | (uintptr_t)xh | (uintptr_t)next_w) & 15);
-    const size_t lds = (size_t)width * 4;
-    HY_BY_DTYPE(dtype, T,
-        if (vec && width <= 1024) hipLaunchKernelGGL((residual_norm_kernel<T, 1>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
-        else if (vec && width <= 2048) hipLaunchKernelGGL((residual_norm_kernel<T, 2>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
-        else if (vec && width <= 4096) hipLaunchKernelGGL((residual_norm_kernel<T, 4>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
-        else if (vec && width <= 8192) hipLaunchKernelGGL((residual_norm_kernel<T, 8>), dim3(tokens), dim3(256), 0, (hipStream_t)stream, a);
-        else hipLaunchKernelGGL((residual_norm_kernel<T, 0>), dim3(tokens), dim3(256), lds, (hipStream_t)stream, a));
-    return launch_status(fn);
+    return residual_norm_launch<false>(fn, {y, y_stride, y_weight, top, x, w, xh, width, x_stride, eps, mult, next_w, x_stride}, tokens, dtype, stream);
+}
+
+extern "C" int trimkv_last_norm(const void* y, int64_t y_stride, const float* y_weight, int top, const float* x, int x_stride, const float* w, float mult, void* out,
+                                const float* out_w, int tokens, int width, float eps, int32_t* seen, const int32_t* slots, const int32_t* cu, int batch, int dtype, void* stream) {
+    const char* fn = "trimkv_last_norm";
+    if (!y || !x || !w || !out || !out_w || !seen || !slots || !cu) return fail(TRIMKV_ERR_NULL, "%s: null pointer argument", fn);
+    if (batch <= 0 || batch > tokens) return fail(TRIMKV_ERR_SHAPE, "%s: bad batch %d of %d tokens", fn, batch, tokens);
+    return residual_norm_launch<true>(fn, {y, y_stride, y_weight, top, const_cast<float*>(x), w, out, width, x_stride, eps, mult, out_w, width, seen, slots, cu, batch}, tokens, dtype, stream);
 }
 
 extern "C" int trimkv_rms_rows(const float* x, int x_stride, const int64_t* rows, const float* w, void* out, int count, int width, float eps, int dtype, void* stream) {

@@ -300,18 +300,23 @@ class HybridLayer(nn.Module):
             out.update({f"mlp.{k}": v for k, v in self.mlp.tensors().items()})
         return out
 
-    def forward(self, x, xh, state, batch, next_norm: Optional[torch.Tensor] = None):
+    def forward(self, x, xh, state, batch, next_norm: Optional[torch.Tensor] = None, out_norm: Optional[torch.Tensor] = None):
         """Advances the stream x (fp32) in place.  xh, in the matrices' dtype, is what the mixer reads and, afterwards, what the
         next layer's mixer reads: a copy of the stream (None in fp32, where the stream itself is read), or with norms on both
-        sides its norm, for the next layer with weight ``next_norm`` (None: nobody reads it)."""
+        sides its norm, for the next layer with weight ``next_norm`` (None: nobody reads it).  ``out_norm``: the last layer of a step leaves x
+        as it is and returns the stream's norm with that weight; the step's tokens count then."""
         src = x if xh is None else xh
         y = self.mix(x, src, state, batch)
         if self.mlp is None:
-            self._add(x, xh, y, self.norm1b if self.both else self.norm1, next_norm)
-            return
+            return self._end(x, xh, y, self.norm1b if self.both else self.norm1, next_norm, None, out_norm, batch)
         self._add(x, xh, y, self.norm1b if self.both else self.norm1, self.norm2 if self.both else None)
         y, weights = self.mlp(x, src)
-        self._add(x, xh, y, self.norm2b if self.both else self.norm2, next_norm, weights)
+        return self._end(x, xh, y, self.norm2b if self.both else self.norm2, next_norm, weights, out_norm, batch)
+
+    def _end(self, x, xh, y, norm, next_norm, weights, out_norm, batch):
+        if out_norm is not None:
+            return ops.last_norm(x, y, norm, self.eps, weights, self.mult, out_norm, batch)
+        self._add(x, xh, y, norm, next_norm, weights)
 
     def _add(self, x, xh, y, norm, next_norm, weights=None):
         ops.residual_norm(x, None if self.both and next_norm is None else xh, y, norm, self.eps, weights, self.mult, next_norm)
@@ -329,19 +334,28 @@ class HybridModel(nn.Module):
     def new_cache(self, num_slots: int = 0) -> HybridCache:
         return HybridCache([self.layers[run.index].mix.spec for run in self.runs], self.dtype, self.embed.device, num_slots)
 
-    def forward(self, ids: torch.Tensor, cache: HybridCache, batch: ops.PackedBatch, layers_out: Optional[List[torch.Tensor]] = None):
-        """The fp32 residual stream [T, width padded] behind the last layer; ``layers_out`` receives a copy behind every layer run."""
-        cfg, stream = self.config, None
+    def forward(self, ids: torch.Tensor, cache: HybridCache, batch: ops.PackedBatch, layers_out: Optional[List[torch.Tensor]] = None, normed: bool = False):
+        """The fp32 residual stream [T, width padded] behind the last layer; ``layers_out`` receives a copy behind every layer run.  ``normed``: the model's norm
+        of it [T, width] in the matrices' dtype."""
+        cfg, stream, out = self.config, None, None
+        last = self.layers[self.runs[-1].index]
+        # in the last layer's own launch where nobody looks at the stream behind it
+        fused = normed and layers_out is None and type(last) is HybridLayer and unhooked(last)
         for n, (run, state) in enumerate(zip(self.runs, cache.layers_state)):
             layer = self.layers[run.index]
             if n == 0 or run.again:
                 stream = ops.embed_scaled(ids, self.embed, cfg.embedding_scale, ops.padded(cfg.hidden_size), layer.entry_norm, cfg.norm_eps, add_to=stream)
             following = self.runs[n + 1] if n + 1 < len(self.runs) else None
+            if fused and following is None:
+                out = layer(*stream, state, batch, out_norm=self.norm)
+                break
             layer(*stream, state, batch, self.layers[following.index].entry_norm if following and not following.again else None)
             if layers_out is not None:
                 layers_out.append(stream[0][:, :cfg.hidden_size].clone())
-        cache.advance(batch)
-        return stream[0]
+        cache.advance(batch, counted=fused)
+        if normed and not fused:
+            out = ops.rms_rows(stream[0], None, self.norm, cfg.norm_eps, self.dtype)
+        return out if normed else stream[0]
 
 
 class HybridForCausalLM(GreedyGeneration, nn.Module):
@@ -441,8 +455,10 @@ class HybridForCausalLM(GreedyGeneration, nn.Module):
         if slots is None and not cache.active:
             cache.allocate(B)
         batch = cache.batch(lengths, slots)
-        x = self.model(packed.contiguous(), cache, batch, layers_out)
         keep = int(logits_to_keep)
+        # the logits of some rows only, or somebody looks at the stream
+        some = rows is not None or (keep and batch.max_len > 1) or type(self.model) is not HybridModel or not unhooked(self.model)
+        x = self.model(packed.contiguous(), cache, batch, layers_out) if some else self.model(packed.contiguous(), cache, batch, layers_out, normed=True)
         if rows is None and keep and batch.max_len > 1:
             if keep > min(batch.lengths):
                 raise ValueError(f"logits_to_keep {keep} exceeds the shortest sequence of the step")
@@ -454,7 +470,7 @@ class HybridForCausalLM(GreedyGeneration, nn.Module):
             shape = (B, keep)
         else:
             shape = (-1,) if rows is not None or min(batch.lengths) != batch.max_len else (B, batch.max_len)
-        h = ops.rms_rows(x, rows, self.model.norm, self.config.norm_eps, self.model.dtype)
+        h = ops.rms_rows(x, rows, self.model.norm, self.config.norm_eps, self.model.dtype) if some else x
         logits = linear(h, self.model.embed if self.head is None else self.head, library="hybrid")
         logits = logits.float() if self.config.logit_softcap is None else ops.soft_cap(logits, self.config.logit_softcap)
         return SimpleNamespace(logits=logits.view(*shape, logits.shape[-1]), past_key_values=cache)

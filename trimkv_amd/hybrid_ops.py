@@ -130,6 +130,17 @@ def residual_norm(x: torch.Tensor, xh: Optional[torch.Tensor], y: torch.Tensor, 
                                                    _lib.dtype_code(y.dtype), _lib.current_stream(x.device)), "trimkv_residual_norm")
 
 
+def last_norm(x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, eps: float, y_weight: Optional[torch.Tensor], mult: float, out_w: torch.Tensor, batch: PackedBatch) -> torch.Tensor:
+    """``out_w * rms(x + mult * w * rms(y))`` in y's dtype, and the step's tokens count from now on (``advance``); x stays as it is."""
+    _require(y.dtype, y)
+    _require(torch.float32, x, w, y_weight, out_w)
+    out = torch.empty(x.shape[0], w.shape[0], dtype=y.dtype, device=x.device)
+    _check(_lib.load_hybrid().trimkv_last_norm(y.data_ptr(), y.stride(0), _lib.ptr(y_weight), 1 if y_weight is None else y_weight.shape[1], x.data_ptr(), x.stride(0), w.data_ptr(),
+                                               mult, out.data_ptr(), out_w.data_ptr(), x.shape[0], w.shape[0], eps, batch.seen_dev.data_ptr(), batch.slots_dev.data_ptr(),
+                                               batch.cu_dev.data_ptr(), batch.batch, _lib.dtype_code(y.dtype), _lib.current_stream(x.device)), "trimkv_last_norm")
+    return out
+
+
 def rms_rows(x: torch.Tensor, rows: Optional[torch.Tensor], w: torch.Tensor, eps: float, dtype: torch.dtype) -> torch.Tensor:
     _require(torch.float32, x, w)
     count = x.shape[0] if rows is None else rows.numel()
