@@ -38,13 +38,9 @@ inline int dtype_bytes(int dt) {
 
 // ---- device: dtype conversions ---------------------------------------------------------------
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-// round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet), the rounding torch uses
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// round-to-nearest-even fp32 -> bf16 bit pattern (NaN kept quiet), the rounding torch uses: v_cvt_pk_bf16_f32.  Written out with integers, the same bits for all 2^32
+// numbers, it took seven instructions and a branch for the NaN, which in kernels of a few rows was most of what they did
+__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t b) {
     _Float16 h = __builtin_bit_cast(_Float16, b);
     return (float)h;

@@ -74,6 +74,17 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(NormArgs a) {
     }
 }
 
+// sum over 16 lanes in every one of them: lanes 1, 2, 4 and 8 apart in turn (a mirror brings what the lane 4 or 8 apart has: from the second step on
+// neighbours hold the same)
+template <int CTRL>
+__device__ __forceinline__ float dop_dpp(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true)); }
+__device__ __forceinline__ float dop_sum16(float v) {
+    v += dop_dpp<0xB1>(v);         // quad_perm 1,0,3,2
+    v += dop_dpp<0x4E>(v);         // quad_perm 2,3,0,1
+    v += dop_dpp<0x141>(v);        // row_half_mirror
+    return v + dop_dpp<0x140>(v);  // row_mirror
+}
+
 // ---- per-head norm + RoPE, one wavefront per (token, head) -----------------------------------
 struct RopeArgs {
     const uint16_t* q; const uint16_t* k; const uint16_t* v; const uint16_t* qw; const uint16_t* kw; const uint16_t* cos; const uint16_t* sin;
@@ -91,24 +102,21 @@ struct RopeArgs {
 // together (a wavefront that walked units and heads one after the other spent a memory round trip on each: 20 us).
 template <bool F16>
 __device__ __forceinline__ void gate_second_half(const RopeArgs& a, int64_t t, int chunk, int lane) {
-    const int u = chunk * 64 + lane;
+    const int u = chunk * 64 + lane, uc = min(u, a.gate_inter - 1);
     const bool in = u < a.gate_inter;
+    const uint16_t raw = a.gate_h[t * a.gate_tok_stride + uc];
     float act = 0.0f;
-    if (in) {
-        const float x = dop_load<F16>(a.gate_h[t * a.gate_tok_stride + u]);
-        act = dop_round<F16>(x / (1.0f + __expf(-x)));
-    }
     for (int h0 = 0; h0 < a.hkv; h0 += 8) {
-        float w[8];
+        uint16_t w[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) w[i] = in && h0 + i < a.hkv ? dop_load<F16>(a.gate_w2[(int64_t)(h0 + i) * a.gate_inter + u]) : 0.0f;
+        for (int i = 0; i < 8; ++i) w[i] = a.gate_w2[(int64_t)min(h0 + i, a.hkv - 1) * a.gate_inter + uc];
+        if (h0 == 0 && in) {
+            const float x = dop_load<F16>(raw);
+            act = dop_round<F16>(x / (1.0f + __expf(-x)));
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            float p = act * w[i];
-            p += __shfl_xor(p, 1, 64);
-            p += __shfl_xor(p, 2, 64);
-            p += __shfl_xor(p, 4, 64);
-            p += __shfl_xor(p, 8, 64);
+            const float p = dop_sum16(in ? act * dop_load<F16>(w[i]) : 0.0f);
             if (in && (lane & 15) == 0 && h0 + i < a.hkv) a.gate_part[((int64_t)(u >> 4) * a.ntok + t) * a.hkv + h0 + i] = p;
         }
     }
@@ -168,35 +176,45 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
 // of fewer than 128 features leave lanes idle).  Needs 16-byte aligned rows, head_dim % 8 == 0 and rotary_dim % 16 == 0, so
 // that a lane's eight features lie on one side of the rotation's halfway point and its partner features in ONE other lane.
 // At 8 x 4096 tokens of the Qwen3-8B shape: 351 us (2.3 TB/s) against 945 us with the 2-byte accesses of the kernel above.
-template <bool F16>
+// A decode step's few rows are latency alone: the norm's weight, cosines and sines are requested with the row, and quotients are taken in 32 bits while
+// they fit (16 tokens of 16 + 8 + 8 heads with a gate in a graph of launches 3.9 -> 2.7 us, the rounding in one instruction and the sums without LDS included).
+template <bool F16, typename I>        // I: holds the rows
 __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64_t total_rows, int64_t row_waves) {
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kv_units = a.hq + a.hkv + (a.v ? a.hkv : 0);
     if (wave >= row_waves) {        // behind the rows: the gate's wavefronts, 64 units of one token each
         if (!a.gate_h) return;
         const int chunks = (a.gate_inter + 63) >> 6;
         const int64_t g = wave - row_waves;
         if (g >= (int64_t)a.ntok * chunks) return;
-        gate_second_half<F16>(a, g / chunks, (int)(g % chunks), lane);
+        const int64_t tok = (int64_t)((I)g / (I)chunks);
+        gate_second_half<F16>(a, tok, (int)(g - tok * chunks), lane);
         return;
     }
     const int slot = lane >> 4, lr = lane & 15;
     const int64_t row = wave * 4 + slot;
     const bool live = row < total_rows && lr * 8 < a.d;
     const int64_t rr = min(row, total_rows - 1);
-    const int64_t t = rr / kv_units;
+    const int64_t t = (int64_t)((I)rr / (I)kv_units);
     const int h = (int)(rr - t * kv_units);
     const int kind = h < a.hq ? 0 : h < a.hq + a.hkv ? 1 : 2;
     const int head = kind == 0 ? h : kind == 1 ? h - a.hq : h - a.hq - a.hkv, nh = kind == 0 ? a.hq : a.hkv;
     const uint16_t* src = (kind == 0 ? a.q + t * a.q_tok_stride : kind == 1 ? a.k + t * a.k_tok_stride : a.v + t * a.v_tok_stride) + (int64_t)head * a.d;
     const uint16_t* w = kind == 0 ? a.qw : kind == 1 ? a.kw : nullptr;
     const int rd = kind == 2 ? 0 : a.rd;
-    const int64_t b = t / a.seq, s = t - b * a.seq;
+    const int64_t b = (int64_t)((I)t / (I)a.seq), s = t - b * a.seq;
     uint16_t* dst = (kind == 0 ? a.q_out : kind == 1 ? a.k_out : a.v_out) + ((b * nh + head) * a.seq + s) * a.d;
     const int e0 = lr * 8;
-    Vec8 xv; xv.v = make_uint4(0, 0, 0, 0);
+    const bool turned = live && e0 < rd;
+    Vec8 xv, wv, cv, sv;
+    xv.v = wv.v = cv.v = sv.v = make_uint4(0, 0, 0, 0);
     if (live) xv.v = *(const uint4*)(src + e0);
+    if (live && w) wv.v = *(const uint4*)(w + e0);
+    if (turned) {
+        cv.v = *(const uint4*)(a.cos + b * a.cs_batch_stride + s * a.rd + e0);
+        sv.v = *(const uint4*)(a.sin + b * a.cs_batch_stride + s * a.rd + e0);
+    }
     float y[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] = dop_load<F16>(xv.h[j]);
@@ -204,10 +222,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) ss += y[j] * y[j];
-        ss += __shfl_xor(ss, 1, 64); ss += __shfl_xor(ss, 2, 64); ss += __shfl_xor(ss, 4, 64); ss += __shfl_xor(ss, 8, 64);
+        ss = dop_sum16(ss);
         const float inv = rsqrtf(ss / (float)a.d + a.eps);
-        Vec8 wv; wv.v = make_uint4(0, 0, 0, 0);
-        if (live) wv.v = *(const uint4*)(w + e0);
 #pragma unroll
         for (int j = 0; j < 8; ++j) y[j] = dop_round<F16>(dop_load<F16>(wv.h[j]) * dop_round<F16>(y[j] * inv));
     }
@@ -219,10 +235,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64
 #pragma unroll
     for (int j = 0; j < 8; ++j) r[j] = __shfl(y[j], partner, 64);
     Vec8 ov;
-    if (live && e0 < rd) {
-        Vec8 cv, sv;
-        cv.v = *(const uint4*)(a.cos + b * a.cs_batch_stride + s * a.rd + e0);
-        sv.v = *(const uint4*)(a.sin + b * a.cs_batch_stride + s * a.rd + e0);
+    if (turned) {
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             ov.h[j] = dop_bits<F16>(dop_round<F16>(y[j] * dop_load<F16>(cv.h[j])) + dop_round<F16>((low ? -r[j] : r[j]) * dop_load<F16>(sv.h[j])));
@@ -335,8 +348,10 @@ extern "C" int trimkv_qk_norm_rope(const void* q, int64_t q_tok_stride, const vo
         const int64_t gate_waves = gate_hidden ? (int64_t)batch * seq * ((gate_inter + 63) / 64) : 0;
         const int64_t blocks = (row_waves + gate_waves + 3) / 4;
         if (blocks > 0x7fffffffLL) return fail(TRIMKV_ERR_SHAPE, "%s: too many (token, head) pairs", fn);
-        if (dtype == TRIMKV_F16) hipLaunchKernelGGL(qk_norm_rope_vec_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, st, a, total_rows, row_waves);
-        else hipLaunchKernelGGL(qk_norm_rope_vec_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, st, a, total_rows, row_waves);
+        const bool wide = blocks > 0x0fffffff;        // rows, 16 to a workgroup, that 32 bits do not hold
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, a, total_rows, row_waves); };
+        if (dtype == TRIMKV_F16) wide ? go(qk_norm_rope_vec_kernel<true, int64_t>) : go(qk_norm_rope_vec_kernel<true, uint32_t>);
+        else wide ? go(qk_norm_rope_vec_kernel<false, int64_t>) : go(qk_norm_rope_vec_kernel<false, uint32_t>);
         return launch_status(fn);
     }
     const int64_t blocks = (a.units + 3) / 4;
