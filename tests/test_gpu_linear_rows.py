@@ -46,6 +46,25 @@ def test_linear_rows_matches_the_product(rows, n, k, dtype):
     assert torch.equal(got, linear.linear(x, w, library="hybrid"))
 
 
+# odd numbers of groups of 8 rows of w (3: 24 columns apiece, 5: 40), with a last tile that lacks groups or part of one; k of more steps than wavefronts, of which
+# tiles begin anywhere
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [4, 16, 32, 64])
+@pytest.mark.parametrize("n,k", [(4608, 1216), (4601, 704), (6144, 576), (6139, 1088), (10240, 832), (10236, 640), (10203, 1344)])
+def test_odd_numbers_of_groups_and_tiles_that_begin_anywhere(n, k, rows, dtype):
+    x, w, bias = _operands(rows, n, k, dtype, rows + n + k)
+    got = linear.linear(x, w, bias)
+    _check(got, x, w, bias, dtype)
+    assert torch.equal(got, linear.linear(x, w, bias))
+    if n % 2 == 0:
+        a, b = (linear.linear(x, part, half) for part, half in zip(w.chunk(2), bias.chunk(2)))
+        want = torch.nn.functional.silu(a.double()) * b.double()
+        # silu's slope is at most 1.1; both products of either side are rounded (and their sums differ by less), then silu and the result
+        bound = EPS[dtype] * (2.2 * a.double().abs() * b.double().abs() + 3.2 * want.abs()) + 1e-2 * EPS[dtype]
+        assert ((linear.silu_product(x, w, bias, True).double() - want).abs() <= bound).all()
+
+
 # what linear.linear leaves to the general product is still the entry point's to take
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

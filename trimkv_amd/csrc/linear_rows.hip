@@ -15,18 +15,18 @@
 //    8 x 8) different lines is served one lane at a time: 16 B/clk per compute unit.  LDS-direct loads whose lanes run along
 //    the rows (8 rows x 128 bytes each) take in 28 B/clk; ds_read_b128 does the regrouping.  12288 x 2048 with 16 rows: 19 us
 //    with operand-layout loads, 11.4 here; 4096 x 4096 with 64 rows: 23.4 and 13.7;
-//  * a workgroup takes 16 NT rows of w, or 8, chosen so that the busiest compute unit takes in least (rows_plan below);
+//  * a workgroup takes 8 NG rows of w, NG chosen so that the busiest compute unit takes in least (rows_plan below);
 //  * the wavefronts of a workgroup take turns on k, 64 elements at a time, each with a ring of its own, so that the main loop
 //    has no barrier; their sums meet in LDS at the end of a tile while the next tile's loads are already under way.
 //
 // Measured in a graph of launches over matrices that no cache holds, us here | the vendor library's product:
 //            n x k      1 row        16 rows      32 rows      64 rows
-//      2048 x 2048    4.3 | 10.9    5.0 | 11.1    6.1 | 11.2    7.9 | 11.8
-//     12288 x 2048   11.7 | 16.6   11.4 | 16.7   12.2 | 16.9   14.8 | 18.2
-//      2048 x 6144    7.3 | 11.1    8.6 | 11.3   11.5 | 16.6   17.2 | 19.5
-//      4096 x 4096    8.3 | 15.7    9.3 | 15.5   10.4 | 13.4   13.7 | 15.2
-//     10240 x 4096   16.3 | 26.6   16.6 | 27.8   18.3 | 23.6   22.5 | 29.6
-//     24576 x 4096   34.4 | 45.2   35.5 | 45.5   36.8 | 50.2   42.1 | 50.1
+//      2048 x 2048    3.8 | 10.9    4.7 | 11.1    6.0 | 11.2    7.2 | 11.8
+//     12288 x 2048   10.1 | 16.6   10.5 | 16.7   11.1 | 16.9   13.9 | 18.2
+//      2048 x 6144    6.6 | 11.1    8.5 | 11.3   11.5 | 16.6   16.4 | 19.5
+//      4096 x 4096    7.5 | 15.7    8.6 | 15.5   11.1 | 13.4   13.1 | 15.2
+//     10240 x 4096   15.0 | 26.6   15.6 | 27.8   16.8 | 23.6   21.3 | 29.6
+//     24576 x 4096   32.7 | 45.2   32.7 | 45.5   35.1 | 50.2   40.8 | 50.1
 //      4096 x 12288  18.9 | 23.1   21.1 | 23.5   26.8 | 29.1   36.1 | 39.1
 #include "common.hip.h"
 
@@ -82,22 +82,21 @@ __device__ __forceinline__ void lr_load_to_lds(const uint16_t* base, uint32_t of
                      : "=&s"(saved) : "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
-// XG groups of 8 rows of x, NT blocks of 16 rows of w (SILU: NT / 2 of gate, NT / 2 of up; HALF: one of 8), W wavefronts, D steps of 64 elements
-// of k in flight per wavefront.  A step in LDS: row r holds its eight 16-byte pieces rotated by r / 2, which spreads the 16 rows of
-// an operand read over all banks (the rotation is in the lanes' source addresses).
+// XG groups of 8 rows of x, NG groups of 8 rows of w, two to a block of the matrix cores (SILU: 8 of gate and 8 of up; of an odd number the last block repeats
+// its half), W wavefronts, D steps of 64 elements of k in flight per wavefront.  A step in LDS: row r of a block holds its eight 16-byte pieces rotated by r / 2,
+// which spreads the 16 rows of an operand read over all banks (the rotation is in the lanes' source addresses).
 // A decoder's residual add and RMS norm have no launch of their own (4.6 us, most of it latency): the product in front of them (ADD)
 // adds the residual where it rounds and leaves sums of squares, a few KB that the product behind them (NORM) adds up while its first
 // operands are on their way; x becomes round(round(x / rms) * weight), as modules round, on its way from LDS to the matrix cores.
 // A layer's four products with adds and norms, 16 rows: 43.6 -> 40.2 us at 2048 features and 6144, 92.0 -> 83.5 at 4096 and 12288; 1 row
 // 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102 (all in blocks of 16).  With more rows the arithmetic on the way no longer hides.
 enum { LR_PLAIN = 0, LR_ADD = 1, LR_NORM = 2 };
-template <bool F16, bool SILU, int MODE, int XG, int NT, int W, int D, bool HALF>
+template <bool F16, bool SILU, int MODE, int XG, int NG, int W, int D>
 __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     constexpr bool NORM = MODE == LR_NORM, ADD = MODE == LR_ADD;
     static_assert(MODE == LR_PLAIN || !F16, "bf16 only");
-    constexpr int COLS = HALF ? 8 : 16, WG = COLS / 8;       // rows of w in a block, and loads of a step for them
-    constexpr int MT = (XG + 1) / 2, L = WG * NT + XG, STEP = L * 1024, U = NT * MT, NB = SILU ? NT / 2 : NT;
-    static_assert(!HALF || (NT == 1 && !SILU), "one half block");
+    static_assert(!SILU || NG % 2 == 0, "gate and up");
+    constexpr int NT = (NG + 1) / 2, MT = (XG + 1) / 2, L = NG + XG, STEP = L * 1024, U = NT * MT, CG = SILU ? NG / 2 : NG;     // CG: groups of 8 columns of a tile
     static_assert((D - 1) * L < 64, "the wait counts at most 63 loads");
     __shared__ __attribute__((aligned(1024))) char ring[W * D * STEP];
     __shared__ lr_f32x4 part[U * (W - 1)][64];
@@ -106,37 +105,37 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
     const uint32_t ring_at = (uint32_t)(uintptr_t)(LR_LDS char*)ring + wave * D * STEP;
     const char* mine = ring + wave * D * STEP;
-    // a load brings rows 8 j + lane / 8 of a block, position lane % 8; rows that are not there repeat the last one
-    uint32_t w_off[WG], x_off[XG];
+    // a load brings 8 rows, position lane % 8 of row lane / 8; rows that are not there repeat the last one
+    uint32_t w_off[2], x_off[XG];
 #pragma unroll
-    for (int j = 0; j < WG; ++j) {
-        const int row = 8 * j + (lane >> 3);
-        w_off[j] = (uint32_t)(min(row, a.n - 1) * a.w_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
-    }
+    for (int j = 0; j < 2; ++j) w_off[j] = (uint32_t)(min(lane >> 3, a.n - 1) * a.w_stride * 2) + (((lane & 7) - (8 * j + (lane >> 3)) / 2) & 7) * 16;
 #pragma unroll
     for (int j = 0; j < XG; ++j) {
         const int row = 8 * j + (lane >> 3);
         x_off[j] = (uint32_t)(min(row, a.m - 1) * a.x_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
     }
-    const int steps = a.k >> 6, first = wave, per_tile = (steps - wave + W - 1) / W, tiles = (a.n + COLS * NB - 1) / (COLS * NB);
-    // the first column of block b of a tile: the last block of out is moved back so that all its rows exist
-    auto block_at = [&](int tile, int b) __attribute__((always_inline)) { return min((tile * NB + b % NB) * COLS, max(a.n - COLS, 0)); };
-    int ask_tile = blockIdx.x, ask_step = first, ask_slot = 0, left = per_tile * ((tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
+    const int steps = a.k >> 6, first = wave, per_tile = (steps - wave + W - 1) / W, tiles = (a.n + 8 * CG - 1) / (8 * CG);
+    // the first column of group c of a tile: the last one of out is moved back so that all its rows exist
+    auto column_at = [&](int tile, int c) __attribute__((always_inline)) { return min((tile * CG + c) * 8, max(a.n - 8, 0)); };
+    // where a tile begins along k: eight neighbours, one on each XCD, at the same place, the next eight elsewhere (multiples of the golden section, spread evenly)
+    auto first_of = [&](int tile) __attribute__((always_inline)) { return first + (int)__umulhi(((uint32_t)tile >> 3) * 0x9e3779b9u, (uint32_t)per_tile) * W; };
+    int ask_tile = blockIdx.x, ask_step = first_of(blockIdx.x), ask_left = per_tile, ask_slot = 0;
+    int left = per_tile * ((tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x);
     auto request = [&]() __attribute__((always_inline)) {       // left: steps that have not been requested; below 0 fewer than D are on their way
         if (--left < 0) return;
         const uint32_t to = ring_at + ask_slot * STEP;
 #pragma unroll
-        for (int b = 0; b < NT; ++b) {
-            const uint16_t* from = a.w + (int64_t)(block_at(ask_tile, b) + (SILU && b >= NB ? a.n : 0)) * a.w_stride + ask_step * 64;
-#pragma unroll
-            for (int j = 0; j < WG; ++j) lr_load_to_lds<true>(from, w_off[j], to + (WG * b + j) * 1024);
+        for (int j = 0; j < NG; ++j) {
+            const int64_t row = SILU ? column_at(ask_tile, j / 2) + (j % 2 ? a.n : 0) : column_at(ask_tile, j);
+            lr_load_to_lds<true>(a.w + row * a.w_stride + ask_step * 64, w_off[j % 2], to + j * 1024);
         }
 #pragma unroll
-        for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (WG * NT + j) * 1024);
-        ask_step += W;
-        if (ask_step >= steps) {
-            ask_step = first;
+        for (int j = 0; j < XG; ++j) lr_load_to_lds<false>(a.x + ask_step * 64, x_off[j], to + (NG + j) * 1024);
+        ask_step = ask_step + W < steps ? ask_step + W : first;
+        if (--ask_left == 0) {
+            ask_left = per_tile;
             ask_tile += (int)gridDim.x;
+            ask_step = first_of(ask_tile);
         }
         ask_slot = ask_slot + 1 == D ? 0 : ask_slot + 1;
     };
@@ -168,6 +167,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
     for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
 #pragma unroll
         for (int u = 0; u < U; ++u) acc[u] = lr_f32x4{0.f, 0.f, 0.f, 0.f};
+        int step = first_of(tile);
         for (int s = 0; s < per_tile; ++s) {
             if (left >= 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * L) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -177,15 +177,15 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
             for (int h = 0; h < 2; ++h) {
 #pragma unroll
                 for (int b = 0; b < NT; ++b) {
-                    const int row = HALF ? r & 7 : b * 16 + r;          // a half block: rows 8 .. 15 repeat it
-                    wf[h][b] = *(const lr_u32x4*)(p + row * 128 + ((h * 4 + g + ((HALF ? row : r) >> 1)) & 7) * 16);
+                    const int row = 2 * b + 1 == NG ? r & 7 : r;        // half a block: rows 8 .. 15 repeat it
+                    wf[h][b] = *(const lr_u32x4*)(p + (b * 16 + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
                 }
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
                     const int row = XG == 1 ? r & 7 : t * 16 + r;       // 8 rows: columns 8 .. 15 repeat them
-                    xf[h][t] = *(const lr_u32x4*)(p + (NT * COLS + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
+                    xf[h][t] = *(const lr_u32x4*)(p + (NG * 8 + row) * 128 + ((h * 4 + g + (row >> 1)) & 7) * 16);
                 }
-                if constexpr (NORM) nf[h] = *(const lr_u32x4*)(norm_w + (wave + s * W) * 64 + (h * 4 + g) * 8);
+                if constexpr (NORM) nf[h] = *(const lr_u32x4*)(norm_w + step * 64 + (h * 4 + g) * 8);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // the step has been read: its room is free
             __builtin_amdgcn_sched_barrier(0);
@@ -209,35 +209,34 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
                     for (int t = 0; t < MT; ++t) acc[b * MT + t] = lr_mfma<F16>(wf[h][b], xf[h][t], acc[b * MT + t]);
             slot = slot + 1 == D ? 0 : slot + 1;
+            step = step + W < steps ? step + W : first;
         }
-        // the sums of 16 columns x 16 rows go to the wavefront they belong to (gate and up of a column to the same one)
-        auto owner = [](int u) { return (u / MT % NB * MT + u % MT) % W; };
+        // the sums of a block and 16 rows go to the wavefront they belong to
         if (tile != (int)blockIdx.x) asm volatile("s_barrier" ::: "memory");        // the sums of the tile before have been read
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (owner(u) != wave) part[u * (W - 1) + (wave - owner(u) + W) % W - 1][lane] = acc[u];
+            if (u % W != wave) part[u * (W - 1) + (wave - u % W + W) % W - 1][lane] = acc[u];
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        auto total = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u % W != wave || (u / MT * 2 + 1 == NG && g >= 2)) continue;
+            // this lane: columns n .. n + 3 of row m (SILU: lanes 32 .. 63 have up of what lanes 0 .. 31 have gate of)
+            const int c8 = SILU ? u / MT : u / MT * 2 + (g >> 1), m = u % MT * 16 + r, n = column_at(tile, c8) + 4 * (g & 1);
+            if ((tile * CG + c8) * 8 >= a.n || n >= a.n || (m >= a.m && !ADD)) continue;       // no such columns, or no such row
             lr_f32x4 f = acc[u];
 #pragma unroll
             for (int o = 0; o < W - 1; ++o) f += part[u * (W - 1) + o][lane];
-            return f;
-        };
-#pragma unroll
-        for (int u = 0; u < NB * MT; ++u) {
-            if (owner(u) != wave || (HALF && g >= 2)) continue;
-            const int m = u % MT * 16 + r, n = block_at(tile, u / MT) + 4 * g;      // this lane: columns n .. n + 3 of row m
-            if ((m >= a.m && !ADD) || n >= a.n) continue;       // a matrix of fewer rows than a block: no such columns
-            lr_f32x4 f = total(u);
             uint16_t v[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                if (a.bias && n + c < a.n) f[c] += lr_load<F16>(a.bias[n + c]);
+                if (a.bias && n + c < a.n) f[c] += lr_load<F16>(a.bias[(SILU && g >= 2 ? a.n : 0) + n + c]);
             if constexpr (SILU) {
-                lr_f32x4 e = total(U / 2 + u);
+                lr_f32x4 e;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) e[c] = __shfl_xor(f[c], 32, 64);
+                if (g >= 2) continue;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    if (a.bias && n + c < a.n) e[c] += lr_load<F16>(a.bias[a.n + n + c]);
                     if (a.round_all) {
                         const float x = lr_load<F16>(lr_bits<F16>(f[c]));
                         v[c] = lr_bits<F16>(lr_load<F16>(lr_bits<F16>(x / (1.0f + expf(-x)))) * lr_load<F16>(lr_bits<F16>(e[c])));
@@ -247,7 +246,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c) v[c] = lr_bits<F16>(f[c]);
             }
-            if constexpr (ADD) {            // n is a multiple of 16: four columns are there or none
+            if constexpr (ADD) {            // n is a multiple of 16: eight columns are there or none
                 const uint2 y = *(const uint2*)(a.res + (int64_t)min(m, a.m - 1) * a.res_stride + n);
                 const float old[4] = {lr_lo(y.x), lr_hi(y.x), lr_lo(y.y), lr_hi(y.y)};
                 float sq = 0.f;
@@ -273,77 +272,77 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
 
 constexpr int LR_CUS = 256;
 
-// Blocks of 16 rows of w per tile.  A compute unit that runs `rounds` tiles takes in rounds * (rows of w + rows of x) * k elements;
-// the least of that is the fastest (n x k = 12288 x 2048, 16 rows: one block 3 x 32, three blocks 1 x 64: 13.6 and 11.4 us;
-// 4608 x 2048, 64 rows: 2 x 80, 96, 112: 13.1, 10.6, 12.5).  Among equals the smaller one.
-// 0: half a block, 8 rows, for n up to 2048, where 16 apiece leave half of the compute units idle and take in more for each.  16 -> 8
-// rows, us: 2048 x 6144 with 1, 16, 32, 64 rows of x 8.6 -> 7.3, 10.3 -> 8.6, 13.3 -> 11.5, 18.5 -> 17.2; 2048 x 2048 4.8 -> 4.3, 5.5 -> 5.0,
-// 6.3 -> 6.1, 8.3 -> 7.9; 1024 x 4096 6.3 -> 5.6, 7.2 -> 6.3, 9.0 -> 7.9, 12.4 -> 11.4; 512 x 2048 4.4 -> 4.1, 5.2 -> 4.9, 6.0 -> 5.7, 7.8 -> 7.5.  Half
-// of the matrix cores' rows are repeats then, which nothing waits for.  From 2049 on 8 rows apiece would be two rounds.
-static int rows_plan(int n, int x_rows, bool silu, bool half) {
-    if (half && !silu && n <= 8 * LR_CUS) return 0;
-    static const int plain[] = {1, 2, 3, 6}, paired[] = {2, 4, 6};
+// Groups of 8 rows of w per tile.  A compute unit that runs `rounds` tiles takes in rounds * (rows of w + rows of x) * k elements;
+// the least of that is the fastest (12288 x 4096, 64 rows: 5, 6, 8 groups 2 x 104, 112, 128: 28.5, 22.4, 25.4 us; 4608 x 2048, 16 rows: 2, 3, 4, 5 groups 2 x 32,
+// 40, 48, 56: 7.6, 6.9, 7.2, 7.9).  Among equals the smaller one.  In blocks of 16 only, and gate and up in blocks of their own, a tile often had more than its
+// compute unit's share while others had none.  Blocks of 16, all beginning at the first k -> groups of 8, eight tiles at each beginning, us, 16 rows if not said: norm and silu
+// 2 x 6144 x 2048 12.6 -> 11.2 (4 rows 12.6 -> 11.4, 32 rows 14.7 -> 12.6), norm 4608 x 2048 7.6 -> 6.9 (9.0 -> 8.4), 6656 x 4096 14.5 -> 12.6, add 4096 x 4096 8.9 -> 8.2, 64 rows: 10240 x
+// 4096 22.0 -> 20.8, 6144 x 2048 10.3 -> 9.6, 12288 x 4096 23.3 -> 22.4, silu 2 x 12288 x 4096 44.3 -> 40.0.  The beginnings alone: 0 .. 7 % of these (2048 x 6144 8.6 -> 8.5, 64
+// rows of 2 x 12288 x 4096 46.0 -> 40.0): tiles that begin together otherwise ask the same few channels of memory for the same k.
+static int rows_plan(int n, int x_rows, bool silu) {
+    static const int plain[] = {1, 2, 3, 4, 5, 6, 8, 12}, paired[] = {2, 4, 6, 8, 12};
     const int* sizes = silu ? paired : plain;
+    const int most = x_rows < 64 ? (silu ? 4 : 6) : (silu ? 5 : 8);     // fewer rows of x: more than that was not faster at any size measured
     int best = sizes[0];
     int64_t least = INT64_MAX;
-    for (int i = 0; i < (silu ? 3 : 4); ++i) {
-        const int nt = sizes[i];
-        if (nt == 6 && x_rows < 64) continue;       // fewer rows of x: not faster than two or three blocks at any size measured
-        const int64_t cols = 16 * (silu ? nt / 2 : nt), tiles = (n + cols - 1) / cols, cost = (tiles + LR_CUS - 1) / LR_CUS * (16 * nt + x_rows);
-        if (cost < least) { least = cost; best = nt; }
+    for (int i = 0; i < most; ++i) {
+        const int ng = sizes[i];
+        const int64_t cols = 8 * (silu ? ng / 2 : ng), tiles = (n + cols - 1) / cols, cost = (tiles + LR_CUS - 1) / LR_CUS * (8 * ng + x_rows);
+        if (cost < least) { least = cost; best = ng; }
     }
     return best;
 }
 
-template <bool F16, bool SILU, int XG, int NT, int W, int D, int MODE = LR_PLAIN, bool HALF = false>
+template <bool F16, bool SILU, int XG, int NG, int W, int D, int MODE>
 static void rows_launch(const LinearRowsArgs& a, hipStream_t s) {
-    constexpr int COLS = HALF ? 8 : 16, NB = SILU ? NT / 2 : NT, LDS = W * D * (COLS / 8 * NT + XG) * 1024 + (W - 1) * NT * ((XG + 1) / 2) * 1024 + (MODE == LR_NORM ? LR_NORM_K * 2 + LR_NORM_ROWS * 4 : 16);
+    constexpr int CG = SILU ? NG / 2 : NG, SUMS = (W - 1) * ((NG + 1) / 2) * ((XG + 1) / 2) * 1024;
+    constexpr int LDS = W * D * (NG + XG) * 1024 + SUMS + (MODE == LR_NORM ? LR_NORM_K * 2 + LR_NORM_ROWS * 4 : 32);
     static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
-    const int tiles = (a.n + COLS * NB - 1) / (COLS * NB), most = LR_CUS * (160 * 1024 / LDS);
-    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NT, W, D, HALF>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
+    const int tiles = (a.n + 8 * CG - 1) / (8 * CG), most = LR_CUS * (160 * 1024 / LDS);
+    hipLaunchKernelGGL((linear_rows_kernel<F16, SILU, MODE, XG, NG, W, D>), dim3(tiles < most ? tiles : most), dim3(64 * W), 0, s, a);
 }
-// Wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 8 over the shapes above.  Eight wavefronts where their steps fit: each has half as many steps, one
-// behind the other, and up to 8 KB of a step of all are asked for before the first one is used.  Four wavefronts and requests behind the last step, which nobody
-// read -> eight and none, us: add 2048 x 2048 with 4, 16, 32 rows 4.8 -> 4.4, 5.5 -> 5.0, 6.9 -> 6.0, 2048 x 6144 7.7 -> 6.7, 9.2 -> 9.0, 12.2 -> 11.8, 4096 x 4096 8.4 -> 8.1,
-// 9.4 -> 9.0, 10.8 -> 10.5; norm 4608 x 2048 7.6 -> 6.9, 8.3 -> 7.7, 10.9 -> 9.0, 6656 x 4096 14.5 -> 13.7, 15.5 -> 14.0, 17.6 -> 15.9; norm and silu 2 x 6144 x 2048 13.7 -> 12.4,
-// 14.3 -> 12.5, 15.3 -> 14.4, 2 x 12288 x 4096 33.3 -> 32.4, 34.4 -> 32.7, 41.1 -> 39.3.  64 rows, four wavefronts: 4096 x 4096 13.9 -> 13.4, 12288 x 4096 23.8 -> 23.2, 1024 x 4096 11.5 -> 11.1.
+// Wavefronts and depth: the fastest of 2, 4, 8 and 1 .. 4 over the shapes above, as far as LDS reaches.  Eight wavefronts up to 32 rows: each has half as many steps
+// of four, one behind the other, and up to 8 KB of a step of all are asked for before the first one is used; with 64 rows their sums take the room of a second step.
 template <bool F16, int XG, int MODE = LR_PLAIN>
-static void rows_by_blocks(const LinearRowsArgs& a, bool silu, hipStream_t s) {
-    const int nt = rows_plan(a.n, 8 * XG, silu, MODE != LR_NORM);
-    if constexpr (MODE != LR_NORM)
-        if (nt == 0) return rows_launch<F16, false, XG, 1, XG == 8 ? 4 : 8, XG == 1 ? 4 : 2, MODE, true>(a, s);
-    if constexpr (XG == 8) {
-        if (silu && nt == 6) return rows_launch<F16, true, 8, 6, 4, 1>(a, s);
-        if (silu && nt == 4) return rows_launch<F16, true, 8, 4, 2, 2>(a, s);
-        if (silu) return rows_launch<F16, true, 8, 2, 4, 2>(a, s);
-        if (nt == 6) return rows_launch<F16, false, 8, 6, 4, 1>(a, s);
-        if (nt == 1) return rows_launch<F16, false, 8, 1, 4, 2>(a, s);
-        if (nt == 2) return rows_launch<F16, false, 8, 2, 4, 2>(a, s);
-        return rows_launch<F16, false, 8, 3, 4, 2>(a, s);
-    } else {
-        constexpr int D = XG == 4 ? 1 : 2;
-        if constexpr (MODE != LR_ADD) {
-            if (silu && nt == 4) return rows_launch<F16, true, XG, 4, XG == 4 ? 4 : 8, XG == 4 ? 2 : 1, MODE>(a, s);
-            if (silu) return rows_launch<F16, true, XG, 2, 8, D, MODE>(a, s);
+static void rows_by_groups(const LinearRowsArgs& a, bool silu, hipStream_t s) {
+    const int ng = rows_plan(a.n, 8 * XG, silu);
+    constexpr bool MANY = XG == 8, SOME = XG == 4;
+    if constexpr (MODE != LR_ADD)
+        if (silu) {
+            if constexpr (MANY)
+                if (ng == 12) return rows_launch<F16, true, XG, 12, 4, 1, MODE>(a, s);
+            if (ng == 8) return rows_launch<F16, true, XG, 8, MANY ? 2 : SOME ? 4 : 8, MANY || SOME ? 2 : 1, MODE>(a, s);
+            if (ng == 6) return rows_launch<F16, true, XG, 6, MANY ? 4 : 8, MANY ? 2 : 1, MODE>(a, s);
+            if (ng == 4) return rows_launch<F16, true, XG, 4, MANY ? 4 : 8, MANY || XG == 1 ? 2 : 1, MODE>(a, s);
+            return rows_launch<F16, true, XG, 2, MANY ? 4 : 8, MANY ? 2 : 1, MODE>(a, s);
         }
-        if (nt == 1) return rows_launch<F16, false, XG, 1, 8, 2, MODE>(a, s);
-        if (nt == 2) return rows_launch<F16, false, XG, 2, 8, D, MODE>(a, s);
-        rows_launch<F16, false, XG, 3, MODE == LR_NORM ? 4 : 8, MODE == LR_NORM ? 2 : D, MODE>(a, s);      // (LDS: the norm's weight beside it)
+    if constexpr (MANY) {
+        if (ng == 12) return rows_launch<F16, false, XG, 12, 4, 1, MODE>(a, s);
+        if (ng == 8) return rows_launch<F16, false, XG, 8, 4, 1, MODE>(a, s);
+    }
+    constexpr int W = MANY ? 4 : 8, D = SOME ? 1 : 2;
+    switch (ng) {
+        case 1: return rows_launch<F16, false, XG, 1, W, XG == 1 ? 4 : 2, MODE>(a, s);
+        case 2: return rows_launch<F16, false, XG, 2, W, 2, MODE>(a, s);
+        case 3: return rows_launch<F16, false, XG, 3, W, D, MODE>(a, s);
+        case 4: return rows_launch<F16, false, XG, 4, W, D, MODE>(a, s);
+        case 5: return rows_launch<F16, false, XG, 5, W, XG == 2 ? 1 : D, MODE>(a, s);
+        default: return rows_launch<F16, false, XG, 6, W, XG == 2 && MODE == LR_NORM ? 1 : D, MODE>(a, s);
     }
 }
 template <bool F16>
 static void rows_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
-    if (a.m <= 8) rows_by_blocks<F16, 1>(a, silu, s);
-    else if (a.m <= 16) rows_by_blocks<F16, 2>(a, silu, s);
-    else if (a.m <= 32) rows_by_blocks<F16, 4>(a, silu, s);
-    else rows_by_blocks<F16, 8>(a, silu, s);
+    if (a.m <= 8) rows_by_groups<F16, 1>(a, silu, s);
+    else if (a.m <= 16) rows_by_groups<F16, 2>(a, silu, s);
+    else if (a.m <= 32) rows_by_groups<F16, 4>(a, silu, s);
+    else rows_by_groups<F16, 8>(a, silu, s);
 }
 
 template <int MODE>
 static void norm_by_rows(const LinearRowsArgs& a, bool silu, hipStream_t s) {
-    if (a.m <= 8) rows_by_blocks<false, 1, MODE>(a, silu, s);
-    else if (a.m <= 16) rows_by_blocks<false, 2, MODE>(a, silu, s);
-    else rows_by_blocks<false, 4, MODE>(a, silu, s);
+    if (a.m <= 8) rows_by_groups<false, 1, MODE>(a, silu, s);
+    else if (a.m <= 16) rows_by_groups<false, 2, MODE>(a, silu, s);
+    else rows_by_groups<false, 4, MODE>(a, silu, s);
 }
 
 }  // namespace trimkv
