@@ -94,17 +94,17 @@ _SPLIT_ROWS = 512           # kept rows per chunk (SPLIT_ROWS of csrc/evict.hip)
 def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -> bool:
     """Whether the rows of an eviction's segments are moved by several workgroups each (``trimkv_evict_split_rooms``): ``rows`` due
     rows in all, the longest segment of ``longest``, at most ``kept`` of a segment's left, none losing more than ``spill``.  One
-    workgroup per segment takes about 15 us + 18 ns a row of the longest one; three launches and the detour of the rows that cross a
-    chunk's end take about 30 us + 0.25 ns a row (0.4 ns when most rows cross); both less with fewer features.  Measured, whole ->
-    split, us, segments x rows, of 128 / 96 / 64 features.  Split: losing 128 rows 8 x 8320 166 -> 56 / 145 -> 50 / 97 -> 46, 32 x 8320
-    185 -> 104 / 153 -> 87 / 106 -> 67, 64 x 8320 212 -> 159 / 174 -> 130 / 117 -> 95; losing 4096 8 x 12288 178 -> 85 / 162 -> 74 /
-    112 -> 64, 32 x 12288 199 -> 150 / 172 -> 129 / 117 -> 98.  Whole, where the line is on the safe side: 64 x 4224 112 -> 95 / 94 -> 81 /
-    64 -> 62; and where split is slower: 64 x 2176 61 -> 63 / 52 -> 55 / 37 -> 43, 128 x 8320 252 -> 269 / 209 -> 213 / 142 -> 153, losing
-    4096 64 x 12288 227 -> 254 / 193 -> 212 / 133 -> 150.  Of few kept rows one workgroup is done as soon: 16 segments of 4100 cut to
-    1100 58 -> 67, 8 of 4096 cut to 2048 72 -> 67 / 67 -> 60 / 53 -> 55; of 64 features 16 of 2860 cut to 2560 41 -> 37.
+    workgroup per segment takes about 15 us + 12 to 22 ns a row of the longest one; three launches and the detour of the rows that cross a
+    chunk's end take about 17 us + 0.23 ns a row (all losing many: 20 us and as much); both less with fewer features.  Measured, whole ->
+    split, us, segments x rows, of 128 / 96 / 64 features.  Split: losing 128 rows 8 x 2176 35 -> 24 / 35 -> 23, 32 x 3200 72 -> 40 / 60 -> 35 / 39 -> 29, 64 x
+    4224 110 -> 80 / 92 -> 66 / 62 -> 50, 64 x 8320 208 -> 141 / 173 -> 112 / 115 -> 83; losing 4096 32 x 12288 186 -> 112 / 163 -> 98 / 106 -> 73, 2048 32 x
+    4096 53 -> 45 / 47 -> 38.  Whole, where the line is on the safe side: 64 x 2176 59 -> 44 / 49 -> 38 / 33 -> 30, 128 x 4224 133 -> 136 / 110 -> 108 / 73 -> 81;
+    and where split is slower: 128 x 2176 69 -> 77 / 60 -> 63 / 38 -> 46, 256 x 4224 224 -> 253 / 179 -> 196 / 118 -> 141, losing half 64 x 4096 62 -> 63 /
+    53 -> 58 / 35 -> 43, 128 x 6144 102 -> 148 / 93 -> 122 / 60 -> 86.  Of few kept rows one workgroup is done as soon: 8 x 1152 cut to 1024 24 -> 22 / 23 -> 22 / 18 -> 21,
+    16 x 4100 to 1100 32 -> 31 / 30 -> 30 / 23 -> 27; of 64 features 8 x 2176 cut to 2048 24 -> 22, 8 x 4096 27 -> 25.
     Not while a graph is captured: the launches' table may be uploaded for the first time."""
     return ((2560 if head_dim == 64 else 2048) <= kept and longest <= 32768 and head_dim in (64, 96, 128)
-            and rows * (5 if spill < 512 else 8) < 360 * longest - 300000 and not torch.cuda.is_current_stream_capturing())
+            and (rows * 5 < 400 * longest - 150000 if spill < 512 else rows * 8 < 360 * longest - 300000) and not torch.cuda.is_current_stream_capturing())
 
 
 def compact_halves(segs: int, longest: int, rows: int) -> bool:
@@ -511,7 +511,7 @@ class _SlabBacked(_CacheBase):
             pairs, rows, kept = due
             if not split_evict(int(rows.max()), int(rows.sum()), int(kept.max()), spill, s0.D):
                 return None
-            chunks = np.where(kept >= 1024, -(-kept // _SPLIT_ROWS), 0)      # with fewer rows than that the kernel does not split
+            chunks = np.where(kept >= 640, -(-kept // _SPLIT_ROWS), 0)      # with fewer rows than that the kernel does not split
             first = np.concatenate([[0], np.cumsum(chunks)])
             most, total, count = int(chunks.max()), int(first[-1]), int(pairs.size)
             if total == 0:

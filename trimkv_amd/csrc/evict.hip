@@ -208,7 +208,9 @@ __device__ __forceinline__ int compact_indices(uint32_t* keys, int n, uint32_t t
                 eq_before += is_eq ? 1 : 0;
             }
         }
-        if (my_first_evicted < n) atomicMin(first_evicted_lds, my_first_evicted);
+        // lanes ascend: the first one of a wavefront that lost a row has the smallest (every thread at one address: 12 us of 14 where 4096 of 12288 rows go)
+        const unsigned long long lost = __ballot(my_first_evicted < n);
+        if (lost && (threadIdx.x & 63) == __builtin_ctzll(lost)) atomicMin(first_evicted_lds, my_first_evicted);
         gt_base += (int)(tot & 0xffffu);
         eq_base += (int)(tot >> 16);
     }
@@ -426,7 +428,12 @@ __device__ __forceinline__ int pair_of_block(const EvictArgs& a) { return a.work
 // inside its own rows nobody else touches; those behind them (the last ones of the chunk, no more than were evicted) are
 // copied aside by split_stash_kernel before split_move_kernel overwrites anything.  The order between the two is the order
 // of launches: nothing waits inside a launch.
-constexpr int SPLIT_ROWS = 512, SPLIT_FROM = 1024;      // rows per chunk; segments with fewer rows to move stay whole
+//
+// Segments of fewer than SPLIT_FROM rows to move stay whole: what one workgroup moves behind its selection (14 ns a row) is then done before the longest segments are
+// selected, and scratch follows the rows of long ones.  With 1024 a segment of 950 rows took 22.4 us in the first launch and the longest, of 8320, 15.5.  The chunks find
+// what lies behind them with one load and a count (a binary search is ten loads one behind the other).  Between token steps of 256 heads with lognormal budgets up
+// to 8192 rows 24.6 + 6.7 + 15.9 -> 18.5 + 5.3 + 9.6 us, 16 segments of 12288 rows losing 4096 28 + 46 + 56 -> 23 + 45 + 46.
+constexpr int SPLIT_ROWS = 512, SPLIT_FROM = 640;      // rows per chunk; fewest rows to move
 
 __device__ __forceinline__ int64_t split_stash_bytes(const EvictArgs& a) { return (int64_t)a.split_spill * (2 * a.row_bytes + 12); }
 // the pair's first chunk of the scratch and how many it has there (none if the list says what cannot be)
@@ -435,26 +442,27 @@ __device__ __forceinline__ int2 split_room(const EvictArgs& a, int pair) {
     const int at = a.split_first[pair], end = a.split_first[pair + 1];
     return at < 0 || end > a.split_total ? make_int2(0, 0) : make_int2(at, min(end - at, a.split_chunks));
 }
-// first row of lo .. hi - 1 whose source is `end` or behind it (sources ascend)
-__device__ __forceinline__ int first_spilled(const uint32_t* idx, int lo, int hi, int end) {
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if ((int)idx[mid] >= end) hi = mid; else lo = mid + 1;
-    }
-    return lo;
-}
-
 // blockIdx: chunk, pair, 0 = keys / 1 = values and metadata
 template <int PPR, int N>      // 16-byte pieces per row; layers in the arguments
 __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const SlabTable<N> table) {
-    const int chunk = blockIdx.x, pair = blockIdx.y;
+    __shared__ uint32_t sources[SPLIT_ROWS];
+    const int chunk = blockIdx.x, pair = blockIdx.y, end = (chunk + 1) * SPLIT_ROWS;
     const int4 head = a.split_head[pair];
-    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
-    if (lo >= hi) return;
     const int seg = select_pair(a, table, pair);
+    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min(end, head.x);
+    if (seg < 0 || lo >= hi) return;
     const uint32_t* idx = a.split_idx + (int64_t)head.z * SPLIT_ROWS;
-    const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS), m = hi - from;
-    if (seg < 0 || m <= 0) return;
+    // sources ascend: those behind the chunk's own rows are the last ones
+    int from = lo;
+#pragma unroll
+    for (int x = 0; x < SPLIT_ROWS / 256; ++x) {
+        const int r = lo + x * 256 + (int)threadIdx.x;
+        const uint32_t source = idx[min(r, hi - 1)];
+        sources[x * 256 + threadIdx.x] = source;
+        from += __syncthreads_count(r < hi && (int)source < end);
+    }
+    const int m = hi - from;
+    if (m <= 0) return;
     char* stash = a.split_stash + (int64_t)(head.z + chunk) * split_stash_bytes(a);
     const char* src = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
     char* dst = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
@@ -463,7 +471,7 @@ __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const Sla
 #pragma unroll
         for (int p = 0; p < 8; ++p) {
             const int q = min(base + p * 256 + (int)threadIdx.x, m * PPR - 1);
-            t[p] = load_stream(src + (int64_t)idx[from + q / PPR] * a.row_bytes + (q % PPR) * 16);
+            t[p] = load_stream(src + (int64_t)sources[from - lo + q / PPR] * a.row_bytes + (q % PPR) * 16);
         }
 #pragma unroll
         for (int p = 0; p < 8; ++p) {
@@ -478,7 +486,7 @@ __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const Sla
         const char* lbseg = a.lb_slab + (int64_t)seg * a.cap * lb_bytes;
         const int64_t* posseg = a.pos_slab + (int64_t)seg * a.cap;
         for (int r = threadIdx.x; r < m; r += 256) {
-            const int s = (int)idx[from + r];
+            const int s = (int)sources[from - lo + r];
             pos[r] = posseg[s];
             lb[r] = lb_bytes == 4 ? ((const uint32_t*)lbseg)[s] : (uint32_t)((const uint16_t*)lbseg)[s];
         }
@@ -487,31 +495,31 @@ __global__ __launch_bounds__(256) void split_stash_kernel(EvictArgs a, const Sla
 
 template <int PPR, int N>
 __global__ __launch_bounds__(SPLIT_ROWS) void split_move_kernel(EvictArgs a, const SlabTable<N> table) {
-    const int chunk = blockIdx.x, pair = blockIdx.y, tid = threadIdx.x;
+    __shared__ uint32_t sources[SPLIT_ROWS];
+    const int chunk = blockIdx.x, pair = blockIdx.y, tid = threadIdx.x, end = (chunk + 1) * SPLIT_ROWS;
     const int4 head = a.split_head[pair];
-    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min((chunk + 1) * SPLIT_ROWS, head.x);
-    if (lo >= hi) return;
     const int seg = select_pair(a, table, pair);
-    if (seg < 0) return;
-    const uint32_t* idx = a.split_idx + (int64_t)head.z * SPLIT_ROWS;
-    const int from = first_spilled(idx, lo, hi, (chunk + 1) * SPLIT_ROWS);
+    const int lo = max(chunk * SPLIT_ROWS, head.y), hi = min(end, head.x);
+    if (seg < 0 || lo >= hi) return;
+    const int r = min(lo + tid, hi - 1), s = (int)a.split_idx[(int64_t)head.z * SPLIT_ROWS + r];
+    sources[tid] = (uint32_t)s;
+    const int from = lo + __syncthreads_count(lo + tid < hi && s < end);
     const char* stash = a.split_stash + (int64_t)(head.z + chunk) * split_stash_bytes(a);
     const char* kept = stash + (blockIdx.z ? (int64_t)a.split_spill * a.row_bytes : 0);
     char* rows = (blockIdx.z ? a.v_slab : a.k_slab) + (int64_t)seg * a.cap * a.row_bytes;
     uint4 t[PPR];
 #pragma unroll
     for (int p = 0; p < PPR; ++p) {
-        const int q = p * SPLIT_ROWS + tid, r = min(lo + q / PPR, hi - 1), c = (q % PPR) * 16;
-        t[p] = load_stream(r < from ? rows + (int64_t)idx[r] * a.row_bytes + c : kept + (int64_t)(r - from) * a.row_bytes + c);
+        const int q = p * SPLIT_ROWS + tid, row = min(lo + q / PPR, hi - 1), c = (q % PPR) * 16;
+        t[p] = load_stream(row < from ? rows + (int64_t)sources[row - lo] * a.row_bytes + c : kept + (int64_t)(row - from) * a.row_bytes + c);
     }
-    const int lb_bytes = a.lb_dtype == TRIMKV_F32 ? 4 : 2, r = min(lo + tid, hi - 1);
+    const int lb_bytes = a.lb_dtype == TRIMKV_F32 ? 4 : 2;
     char* lbseg = a.lb_slab + (int64_t)seg * a.cap * lb_bytes;
     int64_t* posseg = a.pos_slab + (int64_t)seg * a.cap;
     int64_t pos = 0;
     uint32_t lb = 0;
     if (blockIdx.z) {
         const int64_t* kpos = (const int64_t*)(stash + (int64_t)a.split_spill * 2 * a.row_bytes);
-        const int s = (int)idx[r];
         pos = r < from ? posseg[s] : kpos[r - from];
         lb = r >= from ? ((const uint32_t*)(kpos + a.split_spill))[r - from] : lb_bytes == 4 ? ((const uint32_t*)lbseg)[s] : (uint32_t)((const uint16_t*)lbseg)[s];
     }
@@ -574,7 +582,9 @@ __global__ __launch_bounds__(EV_THREADS) void evict_kernel(EvictArgs a, const Sl
     if (SELECT) {
         ((uint2*)hist)[threadIdx.x] = make_uint2(0u, 0u);
         __syncthreads();
-        for_each_key<EV_THREADS, 4>(s, n, [&](int i, uint32_t key) { keys[i] = key; atomicAdd(&hist[first_digit(key)], 1u); });
+        auto take = [&](int i, uint32_t key) { keys[i] = key; atomicAdd(&hist[first_digit(key)], 1u); };
+        if (n <= 4 * EV_THREADS) for_each_key<EV_THREADS, 4>(s, n, take);
+        else for_each_key<EV_THREADS, 8>(s, n, take);
     } else {
         for_each_key<EV_THREADS, 4>(s, n, [&](int i, uint32_t key) { keys[i] = key; });
         __syncthreads();
