@@ -528,6 +528,14 @@ def test_decode_of_sequences_with_fewer_rows_than_the_batch_is_split_for(dtype):
     run_window(spec, dtype, [4, 128, 129, 400, 1600], [[1] * 4, [125, 1, 1, 1], [126, 1, 1, 1], [397, 1, 1, 1], [1597, 1, 1, 1]])
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(2, 1, 128, 128), (6, 2, 72, 100), (4, 1, 100, 128), (8, 2, 128, 72), (5, 1, 128, 128), (16, 2, 96, 96), (12, 1, 128, 120), (1, 1, 128, 128)])
+def test_decode_rows_of_sixteen_lanes_shared_by_heads(heads, kv_heads, dim, vdim):
+    """In bf16 a step's products of 2, 4 or 8 heads and 8, 4 or 2 rows for each four are summed together: fewer rows than a step has, one row more, several shares; heads
+    that are not there; head sizes that leave lanes without features."""
+    seqs = [3, 17, 34, 65, 131, 420]
+    run_window(ops.WindowSpec(heads, kv_heads, dim, vdim, 290, 11, 0.13), torch.bfloat16, seqs, [[n - 3] + [1] * 3 if n > 3 else [1] * 3 for n in seqs])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 32), (3, 7, 4128), (64, 32, 4096), (64, 33, 2080), (512, 16, 64), (513, 16, 2048), (128, 16, 260), (129, 16, 4)])
 def test_linear_f32_on_either_side_of_its_rules(dtype, rows, n, k):

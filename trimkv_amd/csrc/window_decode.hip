@@ -38,9 +38,51 @@ __device__ __forceinline__ void widen(Raw8f r, float (&f)[8]) {
     f[0] = r.lo.x; f[1] = r.lo.y; f[2] = r.lo.z; f[3] = r.lo.w; f[4] = r.hi.x; f[5] = r.hi.y; f[6] = r.hi.z; f[7] = r.hi.w;
 }
 
+// Rows of 16 lanes in bf16: a lane's sixteen products (16 / GQ rows and GQ heads) are added up over the lanes of a row so that lane c ends with the sum of
+// product summed_at(c).  Its bits 0, 1, 2 and 3 pick the half that it keeps at each step (of bits 3, 1, 2 and 0 of the product's place).
+__device__ __forceinline__ float sum_to_lanes(float (&v)[16], int c) {
+    auto fold = [&](int half, bool upper, auto ctrl) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (i >= half) continue;
+            const float stays = upper ? v[i + half] : v[i], goes = upper ? v[i] : v[i + half];
+            v[i] = stays + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(goes), decltype(ctrl)::value, 0xf, 0xf, true));
+        }
+    };
+    fold(8, c & 4, std::integral_constant<int, 0x141>{});       // row_half_mirror: lane c ^ 7
+    fold(4, c & 1, std::integral_constant<int, 0xB1>{});        // lane c ^ 1
+    fold(2, c & 2, std::integral_constant<int, 0x4E>{});        // lane c ^ 2
+    fold(1, c & 8, std::integral_constant<int, 0x128>{});       // row_ror:8: lane c ^ 8
+    return v[0];
+}
+// place of (row u, head x): rows on the low lane bits, so that lanes c ^ 1, c ^ 2 and c ^ 7 have other rows of one head
+template <int GQ> __device__ __forceinline__ constexpr int place_of(int u, int x) {
+    const int c = u + x * (16 / GQ);                 // the lane that ends with it
+    return (c & 4) << 1 | (c & 1) << 2 | (c & 2) | c >> 3;
+}
+template <int CTRL> __device__ __forceinline__ float dpp_max(float v) {
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ float dot8(hy_u32x4 a, hy_u32x4 b) {
+    float d = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t p = a[i], r = b[i];          // a bit cast of a vector's element itself takes the first one
+        d = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(hy_bf16x2, p), __builtin_bit_cast(hy_bf16x2, r), d, false);
+    }
+    return d;
+}
+
+// Rows of 16 lanes in bf16, shared by two heads or more: with every product summed over a row's lanes by itself (four additions in each of them) and every
+// exponential taken by all sixteen, vector instructions bounded it.  Here the sums of sixteen products take 15 additions together, a lane takes one exponential of a
+// step, and factors that are 1 are not multiplied with; the rest is the stream of rows and sequences of unlike length, whose workgroups do not end together.  us, with
+// the combination: 8 KV heads of 128, 64 sequences of 256 .. 4096 rows, 4 heads each 85 -> 73, of 4096 184 -> 175, of 64 .. 1024 35 -> 29, 128 of 256 .. 4096 151 -> 132; 8
+// heads each, 32 of 256 .. 4096 80 -> 57; 2 heads each, 64 of 128 .. 2048 41.5 -> 39.  Rows of all sequences cut into equal shares for as many workgroups as are
+// resident: 75 - 79, of 4096 165, of 4 .. 64 52 for 12: not taken.
 template <typename T, int L, int GQ>
 __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
-    constexpr int R = 64 / L, U = GQ >= 8 ? 2 : 4, WAVES = 4;
+    constexpr bool SHARED = std::is_same<T, bf16_t>::value && L == 16 && GQ >= 2;
+    constexpr int R = 64 / L, U = SHARED ? 16 / GQ : GQ >= 8 ? 2 : 4, WAVES = 4;
     extern __shared__ float lds[];                  // [WAVES][GQ][L * 8 + 2]
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int per = a.H / a.G, passes = (per + GQ - 1) / GQ;
@@ -58,14 +100,6 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
     const bool kin = e < a.Dp, vin = e < a.Dvp;     // padded dims are multiples of 8
     const T* rk = (const T*)a.rk + ((int64_t)slot * a.G + g) * cap * a.Dp + (kin ? e : 0);
     const T* rv = (const T*)a.rv + ((int64_t)slot * a.G + g) * cap * a.Dvp + (vin ? e : 0);
-    float q[GQ][8];
-#pragma unroll
-    for (int x = 0; x < GQ; ++x) {
-        widen(raw8((const T*)a.q + ((int64_t)b * a.H + g * per + h0 + min(x, nh - 1)) * a.Dp + (kin ? e : 0)), q[x]);
-#pragma unroll
-        for (int y = 0; y < 8; ++y) q[x][y] = kin ? q[x][y] * a.scale_log2 : 0.0f;
-    }
-    if (r0 >= n) return;                            // a short sequence has fewer shares; the combination knows (q is on its way by now)
     float m[GQ], l[GQ], acc[GQ][8];
 #pragma unroll
     for (int x = 0; x < GQ; ++x) {
@@ -73,50 +107,133 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowArgs a) {
 #pragma unroll
         for (int y = 0; y < 8; ++y) acc[x][y] = 0.0f;
     }
-    using Raw = decltype(raw8((const T*)nullptr));
-    for (int base = r0 + wv * R * U; base < r1; base += WAVES * R * U) {
-        Raw kr[U], vr[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) kr[u] = raw8(rk + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dp);
-#pragma unroll
-        for (int u = 0; u < U; ++u) vr[u] = raw8(rv + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dvp);
-        float s[U][GQ];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float kf[8];
-            widen(kr[u], kf);
-            const bool in = base + u * R + sub < r1;
-#pragma unroll
-            for (int x = 0; x < GQ; ++x) {
-                float d = 0.0f;
-#pragma unroll
-                for (int y = 0; y < 8; ++y) d = fmaf(q[x][y], kf[y], d);
-                d = group_sum<L>(d);
-                s[u][x] = in ? d : WA_NEG;
-            }
-        }
+    if constexpr (SHARED) {
+        hy_u32x4 q[GQ];
 #pragma unroll
         for (int x = 0; x < GQ; ++x) {
-            float mn = m[x];
-#pragma unroll
-            for (int u = 0; u < U; ++u) mn = fmaxf(mn, s[u][x]);
-            const float alpha = __builtin_amdgcn_exp2f(m[x] - mn);
-            m[x] = mn;
-            float ps = 0.0f;
-#pragma unroll
-            for (int u = 0; u < U; ++u) { s[u][x] = s[u][x] > 0.5f * WA_NEG ? __builtin_amdgcn_exp2f(s[u][x] - mn) : 0.0f; ps += s[u][x]; }
-            l[x] = l[x] * alpha + ps;
-#pragma unroll
-            for (int y = 0; y < 8; ++y) acc[x][y] *= alpha;
+            q[x] = raw8((const T*)a.q + ((int64_t)b * a.H + g * per + h0 + min(x, nh - 1)) * a.Dp + (kin ? e : 0));
+            q[x] = kin ? q[x] : hy_u32x4{0, 0, 0, 0};
         }
+        if (r0 >= n) return;                        // a short sequence has fewer shares; the combination knows (q is on its way by now)
+        const int c = lane & 15, mine = c % U;      // this lane's row of a step; its head is c / U
+        float* const sh = lds + wv * 128 + sub * 16;            // a step's probabilities of this row of lanes, [U][GQ], and 64 further on its heads' factors
+        float top = WA_NEG, sum = 0.0f;
+        hy_u32x4 kn[U], vn[U];
+        auto request = [&](int base) __attribute__((always_inline)) {       // rows that are not there are the last one again
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float vf[8];
-            widen(vr[u], vf);
+            for (int u = 0; u < U; ++u) kn[u] = raw8(rk + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dp);
 #pragma unroll
-            for (int x = 0; x < GQ; ++x)
+            for (int u = 0; u < U; ++u) vn[u] = raw8(rv + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dvp);
+        };
+        constexpr bool AHEAD = U <= 4;              // the next step's rows are requested before this one's are used, where registers allow it
+        if (AHEAD) request(r0 + wv * R * U);
+        for (int base = r0 + wv * R * U; base < r1; base += WAVES * R * U) {
+            if (!AHEAD) request(base);
+            hy_u32x4 kr[U], vr[U];
 #pragma unroll
-                for (int y = 0; y < 8; ++y) acc[x][y] = fmaf(s[u][x], vf[y], acc[x][y]);
+            for (int u = 0; u < U; ++u) { kr[u] = kn[u]; vr[u] = vn[u]; }
+            if (AHEAD) request(base + WAVES * R * U);
+            float d[16];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int x = 0; x < GQ; ++x) d[place_of<GQ>(u, x)] = dot8(q[x], kr[u]);
+            float s = sum_to_lanes(d, c) * a.scale_log2;
+            s = base + mine * R + sub < r1 ? s : WA_NEG;
+            float mn = dpp_max<0xB1>(s);
+            if constexpr (U >= 4) mn = dpp_max<0x4E>(mn);
+            if constexpr (U >= 8) mn = dpp_max<0x141>(mn);
+            mn = fmaxf(top, mn);
+            const float alpha = __builtin_amdgcn_exp2f(top - mn), p = s > 0.5f * WA_NEG ? __builtin_amdgcn_exp2f(s - mn) : 0.0f;
+            top = mn;
+            sum = sum * alpha + p;
+            sh[mine * GQ + c / U] = p;
+            const bool moved = __builtin_amdgcn_ballot_w64(!(alpha == 1.0f)) != 0;      // wavefront-uniform; seldom after the first rows
+            if (moved && mine == 0) sh[64 + c / U] = alpha;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // of this wavefront's own
+            if (moved) {
+#pragma unroll
+                for (int x = 0; x < GQ; ++x) {
+                    const float f = sh[64 + x];
+#pragma unroll
+                    for (int y = 0; y < 8; ++y) acc[x][y] *= f;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float vf[8], w[GQ];
+                widen(vr[u], vf);
+#pragma unroll
+                for (int x = 0; x < GQ; ++x) w[x] = sh[u * GQ + x];
+#pragma unroll
+                for (int x = 0; x < GQ; ++x)
+#pragma unroll
+                    for (int y = 0; y < 8; ++y) acc[x][y] = fmaf(w[x], vf[y], acc[x][y]);
+            }
+            asm volatile("" ::: "memory");          // the next step's are written behind these reads
+        }
+        sum = dpp_add<0xB1>(sum);
+        if constexpr (U >= 4) sum = dpp_add<0x4E>(sum);
+        if constexpr (U >= 8) sum = dpp_add<0x141>(sum);
+        if (mine == 0) { sh[c / U] = top; sh[64 + c / U] = sum; }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int x = 0; x < GQ; ++x) { m[x] = sh[x]; l[x] = sh[64 + x]; }
+        __syncthreads();                            // the sums below take this room
+    } else {
+        float q[GQ][8];
+#pragma unroll
+        for (int x = 0; x < GQ; ++x) {
+            widen(raw8((const T*)a.q + ((int64_t)b * a.H + g * per + h0 + min(x, nh - 1)) * a.Dp + (kin ? e : 0)), q[x]);
+#pragma unroll
+            for (int y = 0; y < 8; ++y) q[x][y] = kin ? q[x][y] * a.scale_log2 : 0.0f;
+        }
+        if (r0 >= n) return;
+        using Raw = decltype(raw8((const T*)nullptr));
+        for (int base = r0 + wv * R * U; base < r1; base += WAVES * R * U) {
+            Raw kr[U], vr[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) kr[u] = raw8(rk + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dp);
+#pragma unroll
+            for (int u = 0; u < U; ++u) vr[u] = raw8(rv + (int64_t)min(base + u * R + sub, r1 - 1) * a.Dvp);
+            float s[U][GQ];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float kf[8];
+                widen(kr[u], kf);
+                const bool in = base + u * R + sub < r1;
+#pragma unroll
+                for (int x = 0; x < GQ; ++x) {
+                    float d = 0.0f;
+#pragma unroll
+                    for (int y = 0; y < 8; ++y) d = fmaf(q[x][y], kf[y], d);
+                    d = group_sum<L>(d);
+                    s[u][x] = in ? d : WA_NEG;
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < GQ; ++x) {
+                float mn = m[x];
+#pragma unroll
+                for (int u = 0; u < U; ++u) mn = fmaxf(mn, s[u][x]);
+                const float alpha = __builtin_amdgcn_exp2f(m[x] - mn);
+                m[x] = mn;
+                float ps = 0.0f;
+#pragma unroll
+                for (int u = 0; u < U; ++u) { s[u][x] = s[u][x] > 0.5f * WA_NEG ? __builtin_amdgcn_exp2f(s[u][x] - mn) : 0.0f; ps += s[u][x]; }
+                l[x] = l[x] * alpha + ps;
+#pragma unroll
+                for (int y = 0; y < 8; ++y) acc[x][y] *= alpha;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float vf[8];
+                widen(vr[u], vf);
+#pragma unroll
+                for (int x = 0; x < GQ; ++x)
+#pragma unroll
+                    for (int y = 0; y < 8; ++y) acc[x][y] = fmaf(s[u][x], vf[y], acc[x][y]);
+            }
         }
     }
     // lanes that hold the same features of different rows meet, then the wavefronts
