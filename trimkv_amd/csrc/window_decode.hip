@@ -335,10 +335,10 @@ extern "C" int trimkv_window_decode_splits(int batch, int kv_heads, int capacity
     if (batch <= 0 || kv_heads <= 0 || capacity <= 0) return 1;
     // Enough workgroups to fill the chip, at least 128 rows for each and no more than 1024: a batch's sequences differ in length, and
     // the launch ends with the workgroup that has the most rows.  At most 1024, 820, 512 rows, us: 64 sequences of 256 .. 4096 rows x 8
-    // heads of 128 84, 75, 77 (in another order 83, 80, 79), of 64 .. 1024 rows 35, 31, 28, of full windows of 4096 180, 180, 187;
-    // 128 sequences of 256 .. 4096 141, 137, 139, of full windows 358, 365, 372: fewer rows than 1024 cost the fuller batches.
+    // heads of 128 71, 73, 71 (in another order 76, 76, 73), of 64 .. 1024 rows 29, 28, 29, of full windows of 4096 176, 173, 180;
+    // 128 sequences of 256 .. 4096 134, 133, 132, of full windows 346, 353, 361: fewer rows than 1024 cost the fuller batches.
     // With enough pairs to fill the chip as they are (2048) others run while the longest ones finish, and splitting costs full
-    // windows more than it gives unequal ones.  With the bound of 1024 rows -> without, us, full windows | lengths from 256 rows
+    // windows more than it gives unequal ones.  With the bound of 1024 rows -> without, us, before a row's lanes shared their sums, full windows | lengths from 256 rows
     // up (log-uniform): 2048 pairs of 4096 rows 705 -> 650 | 263 -> 288, 4096 of 4096 1434 -> 1281 | 520 -> 500, of 2048 720 -> 644 |
     // 335 -> 315; kept below: 512 of 16384 696 -> 659 | 216 -> 263, of 8192 351 -> 340 | 143 -> 154, 1024 of 4096 353 -> 342 | 155 -> 163.
     const int64_t pairs = (int64_t)batch * kv_heads;
