@@ -29,8 +29,8 @@ def _check(got, x, w, bias, dtype):
     assert (err <= bound).all(), (float((err - bound).max()), (err > bound).nonzero()[:4].tolist())
 
 
-# rows: every number of row groups and their edges; n: ends of 8-row (up to 2048) and 16-row blocks and, from 4608 on, every number of blocks per tile and more
-# tiles than workgroups; k: fewer steps than wavefronts, numbers that do not divide among them
+# rows: every number of row groups and their edges; n: ends of groups of 8 columns and of tiles, every number of groups per tile and more tiles than workgroups;
+# k: fewer steps than wavefronts, numbers that do not divide among them
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 64), (1, 15, 128), (7, 16, 192), (8, 17, 320), (9, 40, 64), (16, 100, 1024), (17, 33, 448), (31, 2048, 512), (32, 18, 64), (33, 1000, 704),
@@ -63,6 +63,34 @@ def test_odd_numbers_of_groups_and_tiles_that_begin_anywhere(n, k, rows, dtype):
         # silu's slope is at most 1.1; both products of either side are rounded (and their sums differ by less), then silu and the result
         bound = EPS[dtype] * (2.2 * a.double().abs() * b.double().abs() + 3.2 * want.abs()) + 1e-2 * EPS[dtype]
         assert ((linear.silu_product(x, w, bias, True).double() - want).abs() <= bound).all()
+
+
+# n that is no multiple of 8: the last group of 8 columns is moved back over the one before it.  1985, 1988, 1028, 68 and 32003: the last group alone in a tile that begins
+# elsewhere along k than the one before; 6139, 10236, 4601: in one tile with it
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [5, 16, 32, 64])
+@pytest.mark.parametrize("n,k", [(68, 4096), (1028, 4096), (1985, 2048), (1988, 2048), (4601, 1024), (6139, 1088), (10236, 640), (32003, 1024)])
+def test_every_column_has_one_writer(n, k, rows, dtype):
+    """The second half of k takes back what the first half added, so that results are what rounding left of their sums and no two orders give the same.  Rows of zeros up to
+    the next multiple of 8 change neither tiles nor beginnings, and no group is moved: the bits are the same."""
+    x, w, bias = _operands(rows, n, k // 2, dtype, rows + n + k)
+    x, w = torch.cat([x, x], 1) * 16, torch.cat([w, -w], 1) * 16
+    padded = torch.nn.functional.pad(w, (0, 0, 0, -n % 8))
+
+    def product(w):     # linear.linear sends the widest to the general product
+        out = torch.empty(rows, w.shape[0], dtype=dtype, device=DEV)
+        _lib.check(_lib.load().trimkv_linear_rows(x.data_ptr(), k, w.data_ptr(), k, None, out.data_ptr(), w.shape[0], rows, w.shape[0], k, _lib.dtype_code(dtype),
+                                                  _lib.current_stream(x.device)), "product")
+        return out
+    got, want = product(w), product(padded)[:, :n]
+    assert (want[:, -8:] != 0).any(1).all()
+    assert torch.equal(got, want)
+    if n <= 10236:
+        x, gate, up = x * 64, w, w.roll(1, 0)
+        got = linear.silu_product(x, torch.cat([gate, up]), None, False)
+        want = linear.silu_product(x, torch.cat([torch.nn.functional.pad(t, (0, 0, 0, -n % 8)) for t in (gate, up)]), None, False)[:, :n]
+        assert torch.equal(got, want)
 
 
 # what linear.linear leaves to the general product is still the entry point's to take

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
         x_off[j] = (uint32_t)(min(row, a.m - 1) * a.x_stride * 2) + (((lane & 7) - (row >> 1)) & 7) * 16;
     }
     const int steps = a.k >> 6, first = wave, per_tile = (steps - wave + W - 1) / W, tiles = (a.n + 8 * CG - 1) / (8 * CG);
-    // the first column of group c of a tile: the last one of out is moved back so that all its rows exist
+    // the first column of group c of a tile: the last one of out is moved back so that all its rows exist (it stores the columns that are its own)
     auto column_at = [&](int tile, int c) __attribute__((always_inline)) { return min((tile * CG + c) * 8, max(a.n - 8, 0)); };
     // where a tile begins along k: eight neighbours, one on each XCD, at the same place, the next eight elsewhere (multiples of the golden section, spread evenly)
     auto first_of = [&](int tile) __attribute__((always_inline)) { return first + (int)__umulhi(((uint32_t)tile >> 3) * 0x9e3779b9u, (uint32_t)per_tile) * W; };
@@ -222,7 +222,9 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
             if (u % W != wave || (u / MT * 2 + 1 == NG && g >= 2)) continue;
             // this lane: columns n .. n + 3 of row m (SILU: lanes 32 .. 63 have up of what lanes 0 .. 31 have gate of)
             const int c8 = SILU ? u / MT : u / MT * 2 + (g >> 1), m = u % MT * 16 + r, n = column_at(tile, c8) + 4 * (g & 1);
-            if ((tile * CG + c8) * 8 >= a.n || n >= a.n || (m >= a.m && !ADD)) continue;       // no such columns, or no such row
+            // Columns below `own` are the group's before, whose sums may have begun elsewhere along k: a column has one writer
+            const int own = (tile * CG + c8) * 8;
+            if (own >= a.n || n >= a.n || n + 4 <= own || (m >= a.m && !ADD)) continue;       // no such columns, another group's, or no such row
             lr_f32x4 f = acc[u];
 #pragma unroll
             for (int o = 0; o < W - 1; ++o) f += part[u * (W - 1) + o][lane];
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
             else
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    if (n + c < a.n) o[c] = v[c];
+                    if (n + c >= own && n + c < a.n) o[c] = v[c];
         }
     }
 }
