@@ -6,7 +6,7 @@
  * Conventions as in trimkv_hip.h: device pointers throughout, work enqueued on `stream`, no allocation and no host
  * synchronisation, 0 / negative trimkv_status / positive hipError_t, text of the last error of the calling thread from
  * trimkv_hybrid_last_error() (trimkv_mlstm_last_error(), trimkv_moe_last_error() of the other two).  `dtype` is the type of activations and matrices: TRIMKV_BF16 or TRIMKV_F32 (everything in
- * true fp32).  Norm weights, biases, gates, router logits, recurrent state and the residual stream are fp32 always.
+ * fp32; where bf16 terms stand for fp32 numbers they hold them whole).  Norm weights, biases, gates, router logits, recurrent state and the residual stream are fp32 always.
  *
  * Batches are packed: the tokens of all sequences of a step lie one after the other, sequence b owns tokens
  * cu[b] .. cu[b+1]-1 (cu [batch+1] int32).  What a sequence leaves behind lives in a slot, slots[b] (int32); seen [slots][2]
@@ -36,9 +36,10 @@ int trimkv_embed_scaled(const int64_t* ids, const void* table, float scale, floa
  * three bf16 terms).  k and x_stride multiples of 4, w_stride a multiple of 8; 16-byte aligned. */
 int trimkv_linear_f32(const float* x, int64_t x_stride, const void* w, int64_t w_stride, float* out, int rows, int n, int k, int dtype, void* stream);
 
-/* out[m][n] = sum_k x[m][k] w[n][k] in fp32: a linear layer over many rows, the tokens of a prompt (each number split exactly into three bf16 terms, six of the
- * nine products taken, fp32 sums; blocks whose results are not finite once more by fp32 products).  k a multiple of 32, strides of x and w multiples of 4 up to 2^20, x and w
- * 16-byte aligned; rows, n <= 2^22.  form: how the launch is cut, 0: by sizes.  _form: what that is. */
+/* out[m][n] = sum_k x[m][k] w[n][k] in fp32: a linear layer over many rows, the tokens of a prompt.  Each number is split into three bf16 terms, exactly, and six of the nine
+ * products are taken (the others are at most 3 * 2^-25 |x w|), with fp32 sums: 3.5e-7 (2-norm) from the exact result for k = 2048.  Blocks whose results are not finite, and blocks
+ * where numbers below 2^-103, which three terms do not hold, could be seen in the result, are done by fp32 products.  k a multiple of 32, strides of x and w multiples of 4 up
+ * to 2^20, x and w 16-byte aligned; rows, n <= 2^22.  form: how the launch is cut, 0: by sizes.  _form: what that is. */
 int trimkv_linear_f32_tiles(const float* x, int64_t x_stride, const float* w, int64_t w_stride, float* out, int64_t out_stride, int rows, int n, int k, int form, void* stream);
 int trimkv_linear_f32_tiles_form(int rows, int n, int k);
 

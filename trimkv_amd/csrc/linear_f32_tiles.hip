@@ -4,22 +4,25 @@
 //   trimkv_linear_f32_tiles_form   how it is cut by sizes
 //
 // What bounds it: the matrix cores.  Their fp32 instructions do 157 TFLOP/s at most (the vendor library's product 97 - 120 at the sizes below); three
-// bf16 terms hold all 24 bits of an fp32 number, and six of the nine products of two such sums (those above 2^-24 of the largest) on the bf16 instructions take
-// 2.7 times fewer cycles.  The operands come as fp32 and are split on their way, once for every tile that they are in: beside 6 MU NU matrix instructions for
-// MU x NU blocks of 16 x 16 x 32 stand 28 (MU + NU) vector instructions, seven for a pair of numbers: v_cvt_pk_bf16_f32 takes a term of both, v_dot2_f32_bf16
-// what is left of one, exactly (with masks, subtractions and packs eleven: 5 % slower).  Matrix and vector instructions of one wavefront follow one another (spread between one
-// another, v_dot2 waits for the matrix cores and the others gain nothing measurable), so that the tiles run at 185 - 197 TFLOP/s of fp32 product.  Hence
+// bf16 terms hold all 24 bits of an fp32 number from 2^-103 on, and six of the nine products of two such sums (those above 2^-24 of the largest; the others are 3 * 2^-25 of
+// |x w| at most) on the bf16 instructions take 2.7 times fewer cycles.  The operands come as fp32 and are split on their way, once for every tile that they are in: beside 6 MU NU
+// matrix instructions for MU x NU blocks of 16 x 16 x 32 stand 32 (MU + NU) vector instructions, eight for a pair of numbers: v_cvt_pk_bf16_f32 takes a term of both,
+// v_dot2_f32_bf16 what is left of one, exactly (with masks, subtractions and packs four more: 5 % slower), and v_max3_f32 follows the largest.  Matrix and vector instructions of one wavefront follow one another (spread between one
+// another, v_dot2 waits for the matrix cores and the others gain nothing measurable), so that the tiles run at 178 - 189 TFLOP/s of fp32 product.  Hence
 //  * all four wavefronts of a workgroup have the same tile and take turns on k, 32 at a time, each with LDS of its own: nothing is split twice and the main
 //    loop has no barrier; their sums meet in LDS at the end;
 //  * a tile may have any number of blocks of 16 either way, so that a launch can be cut into what fills the compute units (f32_tiles_form);
 //  * x is held, w streams past it: 16 rows of w are requested, one period of k later read, split, and multiplied, all while their neighbours are.
 // Error against 64 bits (2-norm, relative; numbers of a normal distribution): 3.5e-7 for k = 2048, 5.0e-7 for 4096, that of the sums (the vendor library's
 // product 8.1e-7, 1.1e-6; fp32 matrix instructions in this file's order 4.1e-7).
-// What bf16 terms do not hold, infinities, NaN and numbers that round to infinity, ends as a result that is not finite: blocks with such results are done
-// again by fp32 matrix instructions.
+// What bf16 terms do not hold is done by fp32 matrix instructions.  Infinities, NaN and numbers that round to infinity end as results that are not finite: blocks with such
+// results are done again.  Numbers below 2^-103 lose up to 2^-125 each.  That is nothing beside a result of 2^-97 k times the largest number and more; a tile with a smaller
+// result looks through its rows, and blocks with a row that has such a number are done again (rows 2^-118 times a normal distribution, against a matrix 2^100 times, without it:
+// error 8.8e-6, 2^-126 2.3e-3, 2^-134 0.6; now 4.1e-7).  Following the largest costs 3 - 5 % of a launch, a row of zeros in each tile 40 %: 811 x 6144 x 2048 117 -> 122 us, 160 with
+// such rows (the vendor library's 205), 900 if all of x is below 2^-103.  With the smallest number followed instead, single zeros sent tiles to look.
 //
-// Measured (rows x n x k, us here | the vendor library's product): 811 x 6144 x 2048 107 | 205, 811 x 2048 x 2048 42 | 58, 811 x 1024 x 2048 25 | 35, 300 x 6144 x
-// 2048 42 | 64, 300 x 2048 x 2048 21 | 28, 100 x 2048 x 2048 14 | 21, 30 x 6144 x 2048 14 | 21, 1700 x 6144 x 2048 222 | 373, 811 x 4096 x 4096 151 | 248.
+// Measured (rows x n x k, us here | the vendor library's product): 811 x 6144 x 2048 122 | 205, 811 x 2048 x 2048 45 | 58, 811 x 1024 x 2048 27 | 35, 300 x 6144 x
+// 2048 46 | 64, 300 x 2048 x 2048 23 | 28, 100 x 2048 x 2048 15 | 21, 30 x 6144 x 2048 17 | 21, 1700 x 6144 x 2048 242 | 373, 811 x 4096 x 4096 166 | 248.
 #include "hybrid.hip.h"
 
 namespace trimkv {
@@ -47,13 +50,21 @@ __device__ __forceinline__ float ft_rest(uint32_t p, uint32_t minus, float f) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(hy_bf16x2, p), __builtin_bit_cast(hy_bf16x2, minus), f, false);
 }
 
-__device__ __forceinline__ void split8(const hy_f32x4 (&v)[2], Terms& o) {
+// Three bf16 terms hold the 24 bits of numbers from 2^-103 on (and 0): below, what the last ones stand for is under 2^-126 and may be lost
+constexpr uint32_t FT_LEAST = (127u - 103u) << 23;       // bits of 2^-103
+__device__ __forceinline__ float ft_most(float most, float a, float b) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(a), "v"(b));
+    return most;
+}
+
+__device__ __forceinline__ void split8(const hy_f32x4 (&v)[2], Terms& o, float& most) {
     uint32_t low, high;
     asm("s_mov_b32 %0, 0xbf80" : "=s"(low));
     asm("s_mov_b32 %0, 0xbf800000" : "=s"(high));
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         float a = v[p >> 1][2 * (p & 1)], b = v[p >> 1][2 * (p & 1) + 1];
+        most = ft_most(most, a, b);
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const uint32_t u = pack2(a, b);
@@ -63,20 +74,21 @@ __device__ __forceinline__ void split8(const hy_f32x4 (&v)[2], Terms& o) {
     }
 }
 
-constexpr int ft_lds(int MU, int NU, int D) { return D * (MU + NU) * 8 > MU * NU * 3 ? D * (MU + NU) * 8192 : MU * NU * 3072; }
+// the wavefronts' rings, or their sums and eight words behind these
+constexpr int ft_lds(int MU, int NU, int D) { return D * (MU + NU) * 8 > MU * NU * 3 ? D * (MU + NU) * 8192 : MU * NU * 3072 + 32; }
 
-// 16 x 16 results by fp32 matrix instructions, for a whole wavefront
+// 16 x 16 results by fp32 matrix instructions, for a whole wavefront.  Four sums of k / 4 products: one of all errs by 8.1e-7 for k = 2048
 __device__ __forceinline__ hy_f32x4 f32_block(const F32TilesArgs& a, int m0, int n0) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const float* const x = a.x + (int64_t)min(m0 + r, a.m - 1) * a.xs + 4 * g;
     const float* const w = a.w + (int64_t)min(n0 + r, a.n - 1) * a.ws + 4 * g;
-    hy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    hy_f32x4 acc[4] = {};
     for (int k = 0; k < a.k; k += 16) {
         const hy_f32x4 xf = *(const hy_f32x4*)(x + k), wf = *(const hy_f32x4*)(w + k);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = mfma16_f32(wf[i], xf[i], acc);
+        for (int i = 0; i < 4; ++i) acc[i] = mfma16_f32(wf[i], xf[i], acc[i]);
     }
-    return acc;
+    return (acc[0] + acc[1]) + (acc[2] + acc[3]);
 }
 
 // MU x NU blocks of 16 x 16 to a tile, D periods of k in LDS.  Two workgroups to a compute unit where registers and LDS (80 KB) allow it.
@@ -110,6 +122,7 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
         ft_load_unit(from, from - 1024, off[j][0], off[j][1], ring_at + (slot * L + j) * 2048);
     };
     hy_f32x4 acc[U];
+    float most = 0.f;        // of the numbers this lane has split
 #pragma unroll
     for (int u = 0; u < U; ++u) acc[u] = hy_f32x4{0.f, 0.f, 0.f, 0.f};
     struct Raw { hy_f32x4 v[2]; };
@@ -140,10 +153,10 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
 #pragma unroll
         for (int i = 0; i < R1; ++i) request(tail(i), D, 0);
         int slot = 0, after = D > 1 ? 1 : 0;
-        split8(first.v, cur);
+        split8(first.v, cur, most);
         for (int p = 0; p < periods; ++p) {
 #pragma unroll
-            for (int i = 0; i < MU; ++i) split8(hraw[i].v, held[i]);
+            for (int i = 0; i < MU; ++i) split8(hraw[i].v, held[i], most);
 #pragma unroll
             for (int j = 0; j < NU; ++j) {
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -170,7 +183,7 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
                     coming = read(MU + 1, after);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                split8(now.v, nxt);
+                split8(now.v, nxt, most);
                 constexpr int X[6] = {0, 2, 1, 0, 1, 0}, W[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
                 for (int q = 0; q < 6; ++q)
@@ -188,6 +201,10 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
     // sums of the four wavefronts meet in LDS; unit u belongs to wavefront u % 4
     __syncthreads();
     hy_f32x4(*part)[64] = (hy_f32x4(*)[64])lds;
+    int* const words = (int*)(lds + U * 3072);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) most = fmaxf(most, __shfl_xor(most, d, 64));
+    if (lane == 0) words[wave] = __float_as_int(most);
 #pragma unroll
     for (int u = 0; u < U; ++u)
         if (u % 4 != wave) part[u * 3 + (wave - u % 4 + 4) % 4 - 1][lane] = acc[u];
@@ -202,15 +219,44 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
             for (int c = 0; c < 4; ++c)
                 if (n + c < a.n) y[c] = s[c];
     };
+    // 2^-125 of up to k numbers, times as many as large as any here, may be lost: less than 2^-27 of a result of `sure` or more
+    most = fmaxf(fmaxf(__int_as_float(words[0]), __int_as_float(words[1])), fmaxf(__int_as_float(words[2]), __int_as_float(words[3])));
+    const float sure = most * 0x1p-97f * (float)a.k;
     uint32_t again = 0;
+    bool unsure = false;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if (u % 4 != wave) continue;
         hy_f32x4 s = acc[u];
 #pragma unroll
         for (int o = 0; o < 3; ++o) s += part[u * 3 + o][lane];
+        unsure |= fminf(fminf(fabsf(s[0]), fabsf(s[1])), fminf(fabsf(s[2]), fabsf(s[3]))) < sure;
         if (__any(!finite_bits(__builtin_bit_cast(hy_u32x4, s)))) again |= 1u << (u / 4);
         else store(u, s);
+    }
+    // Smaller results, rows of zeros above all: blocks with a row of x or of w that has a number of less than 2^-103 are done again as well
+    unsure = __any(unsure);
+    if (lane == 0) words[4 + wave] = unsure;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (words[4] | words[5] | words[6] | words[7]) {
+        uint32_t rows = 0;        // bit j: unit j has such a row
+        for (int p = 0; p < periods; ++p)
+#pragma unroll
+            for (int j = 0; j < L; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const hy_u32x4 v = *(const hy_u32x4*)((j < MU ? xb : wb) + (int64_t)(wave + 4 * p) * 128 + off[j][h]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) rows |= (v[i] & 0x7fffffffu) - 1u < FT_LEAST - 1u ? 1u << j : 0u;
+                }
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) rows |= __shfl_xor(rows, d, 64);
+        if (lane == 0) words[wave] = (int)rows;
+        __syncthreads();
+        rows = (uint32_t)__builtin_amdgcn_readfirstlane(words[0] | words[1] | words[2] | words[3]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u % 4 == wave && (rows >> (u / NU) & 1 || rows >> (MU + u % NU) & 1)) again |= 1u << (u / 4);
     }
     for (int i = 0; again >> i; ++i)
         if (again >> i & 1) store(4 * i + wave, f32_block(a, m0 + (4 * i + wave) / NU * 16, n0 + (4 * i + wave) % NU * 16));
@@ -219,7 +265,7 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
 struct F32Form { int mu, nu, d; bool pairs; float begin, period; };      // pairs: two workgroups to a compute unit
 
 // A form takes begin + period * periods of 128 k (us) for a round of a tile per compute unit; with two workgroups to each, the beginnings of later
-// rounds pass unseen.  Measured with 128 .. 1024 tiles of k = 512, 2048 and 4096.
+// rounds pass unseen.  Measured with 128 .. 1024 tiles of k = 512, 2048 and 4096, without the largest number followed: as it is 3 - 5 % more, of all forms alike.
 constexpr F32Form F32_FORMS[] = {{1, 4, 2, true, 4.2f, 0.69f}, {2, 3, 2, true, 3.6f, 0.80f}, {2, 6, 1, true, 3.8f, 1.34f}, {3, 4, 1, true, 3.9f, 1.20f}, {4, 4, 1, true, 4.8f, 1.43f},
                                  {3, 6, 1, true, 4.6f, 1.68f}, {4, 5, 1, true, 5.2f, 1.72f}, {4, 6, 1, true, 5.2f, 2.05f}, {5, 6, 1, false, 6.8f, 2.34f}, {3, 9, 1, false, 7.0f, 2.37f},
                                  {4, 8, 1, false, 7.4f, 2.50f}, {4, 10, 1, false, 8.0f, 3.10f}, {6, 8, 1, false, 9.0f, 3.50f}};
