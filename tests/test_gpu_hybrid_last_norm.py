@@ -6,6 +6,7 @@ import torch
 
 from .hybrid_util import attention, build, config, mlstm, weights
 from trimkv_amd import hybrid_ops as ops
+from trimkv_amd.hybrid_cache import HybridCache
 
 DEV = "cuda:0"
 
@@ -49,3 +50,31 @@ def test_who_looks_at_the_stream_sees_it():
         handle.remove()
     for s in streams:
         assert torch.equal(s[:, :copies[-1].shape[1]], copies[-1])
+
+
+@pytest.mark.gpu
+def test_caches_that_count_tokens_by_a_way_of_their_own():
+    """A subclass or an instance with an ``advance`` of its own is asked once a step, and tokens count once."""
+    class Own(HybridCache):
+        def advance(self, batch):
+            asked.append(batch.lengths)
+            super().advance(batch)
+
+    cfg = config([attention(), mlstm()])
+    model = build(cfg, weights(cfg), torch.bfloat16).to(DEV).eval()
+    ids = torch.randint(0, 97, (9,), device=DEV)
+
+    def steps(cache):
+        out = model(ids, past_key_values=cache, lengths=[5, 4]).logits, model(ids[:2], past_key_values=cache, lengths=[1, 1]).logits
+        return *out, cache.seen.tolist(), list(cache.tokens_seen)
+    want, asked = steps(model.new_cache(2)), []
+    own, patched = model.new_cache(2), model.new_cache(2)
+    own.__class__ = Own
+    real = patched.advance
+    patched.advance = lambda batch: (asked.append(batch.lengths), real(batch))
+    for cache in (own, patched):
+        got = steps(cache)
+        assert asked == [(5, 4), (1, 1)] and got[2:] == want[2:]
+        for a, b in zip(got[:2], want[:2]):
+            assert torch.allclose(a, b, rtol=2 ** -6, atol=1e-2)
+        asked.clear()

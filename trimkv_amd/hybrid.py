@@ -339,8 +339,8 @@ class HybridModel(nn.Module):
         of it [T, width] in the matrices' dtype."""
         cfg, stream, out = self.config, None, None
         last = self.layers[self.runs[-1].index]
-        # in the last layer's own launch where nobody looks at the stream behind it
-        fused = normed and layers_out is None and type(last) is HybridLayer and unhooked(last)
+        # in the last layer's own launch, which counts the step's tokens too, where nobody looks at the stream behind it or counts by a way of their own
+        fused = normed and layers_out is None and type(last) is HybridLayer and unhooked(last) and getattr(cache.advance, "__func__", None) is HybridCache.advance
         for n, (run, state) in enumerate(zip(self.runs, cache.layers_state)):
             layer = self.layers[run.index]
             if n == 0 or run.again:
@@ -352,7 +352,10 @@ class HybridModel(nn.Module):
             layer(*stream, state, batch, self.layers[following.index].entry_norm if following and not following.again else None)
             if layers_out is not None:
                 layers_out.append(stream[0][:, :cfg.hidden_size].clone())
-        cache.advance(batch, counted=fused)
+        if fused:
+            cache._count(batch)
+        else:
+            cache.advance(batch)
         if normed and not fused:
             out = ops.rms_rows(stream[0], None, self.norm, cfg.norm_eps, self.dtype)
         return out if normed else stream[0]

@@ -99,10 +99,13 @@ class HybridCache(_CacheBase):
             hit = self._batches[(lengths, slots)] = (both[:len(cu)], both[len(cu):])
         return PackedBatch(lengths, slots, hit[0], hit[1], self.seen, self.num_slots)
 
-    def advance(self, batch: PackedBatch, counted: bool = False) -> None:
-        """The step is done: its tokens count from now on (``counted``: on the device they do already)."""
-        if not counted:
-            advance(batch)
+    def advance(self, batch: PackedBatch) -> None:
+        """The step is done: its tokens count from now on."""
+        advance(batch)
+        self._count(batch)
+
+    def _count(self, batch: PackedBatch) -> None:
+        """``advance`` of the host's numbers alone, behind a launch that has moved on the device's."""
         for s, n in zip(batch.slots, batch.lengths):
             self.tokens_seen[s] += n
 
