@@ -6,7 +6,7 @@ both.  There is no CPU path and no torch fallback.
 """
 from __future__ import annotations
 
-import ctypes
+from array import array
 from dataclasses import dataclass, field
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -65,28 +65,29 @@ class PackedBatch:
         return self.max_len == 1
 
 
-def _host_words(values: Sequence[int], what: str):
+def _host_words(values: Sequence[int], dtype: torch.dtype, what: str) -> array:
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError(f"{what} cannot be recorded into a graph: replays would repeat this step's numbers")
-    return (ctypes.c_int32 * len(values))(*values)
+    return array("q" if dtype == torch.int64 else "i", values)
 
 
 def put(values: Sequence[int], dtype: torch.dtype, device: torch.device) -> torch.Tensor:
-    """``torch.tensor(values, dtype=dtype, device=device)`` of int32 or int64, without a wait for what the stream holds."""
+    """``torch.tensor(values, dtype=dtype, device=device)`` of int32 or int64, without a wait for what the stream holds: 1, 256 and 16384 of int64 11, 10 and 301 us of the
+    host for 16, 29 and 770, on an idle stream."""
     out = torch.empty(len(values), dtype=dtype, device=device)
     if not values:
         return out
-    words = _host_words([w for v in values for w in (v & 0xffffffff, v >> 32 & 0xffffffff)] if dtype == torch.int64 else values, "put")
+    words = _host_words(values, dtype, "put")
     with torch.cuda.device(device):
-        _check(_lib.load_hybrid().trimkv_put_words(out.data_ptr(), ctypes.addressof(words), len(words), _lib.current_stream(out.device)), "trimkv_put_words")
+        _check(_lib.load_hybrid().trimkv_put_words(out.data_ptr(), words.buffer_info()[0], len(words) * words.itemsize // 4, _lib.current_stream(out.device)), "trimkv_put_words")
     return out
 
 
 def reset_slots(seen: torch.Tensor, slots: Sequence[int]) -> None:
     """``seen[slots] = 0`` without a wait for what the stream holds."""
-    words = _host_words(slots, "handing out slots")
+    words = _host_words(slots, torch.int32, "handing out slots")
     with torch.cuda.device(seen.device):
-        _check(_lib.load_hybrid().trimkv_reset_slots(seen.data_ptr(), ctypes.addressof(words), len(words), seen.shape[0], _lib.current_stream(seen.device)), "trimkv_reset_slots")
+        _check(_lib.load_hybrid().trimkv_reset_slots(seen.data_ptr(), words.buffer_info()[0], len(words), seen.shape[0], _lib.current_stream(seen.device)), "trimkv_reset_slots")
 
 
 def embed_scaled(ids: torch.Tensor, table: torch.Tensor, scale: float, stride: int, norm: Optional[torch.Tensor] = None, eps: float = 0.0,
