@@ -213,3 +213,11 @@ def test_keys_are_divided_for_many_query_tiles_only_where_lengths_differ_much():
         assert rule(232, n, 1) == rule(248, n, 40) == 0
         assert rule(64, n, 0) == rule(64, n, 30) > 0
     assert rule(168, 4032, 1) == rule(176, 10304, 1) == 0 and rule(168, 10304, 1) > 0
+
+
+def test_chunks_of_split_evictions_are_the_kernels():
+    """Rows per chunk and the fewest that go to chunks: the host sizes scratch and lists by them."""
+    from trimkv_amd import build, cache_utils
+    source = open(os.path.join(build.CSRC, "evict.hip")).read()
+    found = re.search(r"SPLIT_ROWS = (\d+), SPLIT_FROM = (\d+);", source)
+    assert tuple(map(int, found.groups())) == (cache_utils._SPLIT_ROWS, cache_utils._SPLIT_FROM)

@@ -104,14 +104,9 @@ def test_layers_in_the_arguments_and_in_a_device_table(layers, split, monkeypatc
         assert (("host", *every) in cache._table_cache) == (layers <= 48)
 
 
-@pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
-@pytest.mark.parametrize("budget", [0, 1, 700, 10 ** 6])
-def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(budget, lb_dtype, strategy):
-    """Ties by the hundred, empty segments, lengths around the 256 and 1024 rows a workgroup reads at a time."""
+def _selected_both_ways(lens, cap, budget, lb_dtype, strategy):
     lib, gen = _lib.load(), torch.Generator().manual_seed(budget % 97)
-    L, B, H, cap, D = 3, 2, 4, 1300, 64
-    nseg = B * H
-    lens = torch.tensor([[0, 1, 255, 256, 257, 1023, 1024, 1025], [1300, 1300, 64, 65, 0, 0, 0, 0], [5, 900, 1281, 1279, 3, 1, 2, 700]], dtype=torch.int32)
+    (L, nseg), B, H, D = lens.shape, 2, 4, 64
     lb = [(-torch.randint(1, 6, (nseg, cap), generator=gen) / 8.0).to(lb_dtype).to(DEV) for _ in range(L)]
     pos = [torch.arange(cap, device=DEV).div(3, rounding_mode="floor").repeat(nseg, 1).contiguous() for _ in range(L)]
     k = [torch.randn(nseg, cap, D, generator=gen).to(torch.bfloat16).to(DEV) for _ in range(L)]
@@ -133,6 +128,22 @@ def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(bud
         assert torch.equal(a, b)
     want = lens.view(L, B, H).sum(-1).clamp(max=budget)
     assert torch.equal(results[0][3].view(L, B, H).sum(-1).int(), want.int())
+
+
+@pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
+@pytest.mark.parametrize("budget", [0, 1, 700, 10 ** 6])
+def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(budget, lb_dtype, strategy):
+    """Ties by the hundred, empty segments, lengths around the rows of wavefronts (64) and of the 1024 threads that read at a time."""
+    lens = torch.tensor([[0, 1, 255, 256, 257, 1023, 1024, 1025], [1300, 1300, 64, 65, 0, 0, 0, 0], [5, 900, 1281, 1279, 3, 1, 2, 700]], dtype=torch.int32)
+    _selected_both_ways(lens, 1300, budget, lb_dtype, strategy)
+
+
+@pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
+@pytest.mark.parametrize("budget", [4096, 12000])
+def test_segments_of_more_rows_than_a_workgroup_has_in_flight(budget, lb_dtype, strategy):
+    """4096 rows are four for each thread: one less, as many, one more, twice as many and some."""
+    lens = torch.tensor([[4095, 4096, 4097, 8191, 8192, 8193, 8200, 0], [5119, 5120, 5121, 3, 8200, 8200, 4097, 4096]], dtype=torch.int32)
+    _selected_both_ways(lens, 8200, budget, lb_dtype, strategy)
 
 
 def _uneven(split, monkeypatch):
@@ -218,7 +229,29 @@ def test_pairs_with_chunks_of_their_own(on_host):
         _check(cache, held, keep, str(first))
 
 
+@pytest.mark.parametrize("moved", [639, 640, 641])
+@pytest.mark.parametrize("first", [0, 100, 512, 700])
+def test_fewest_rows_that_are_moved_by_several_workgroups(first, moved):
+    """A kept prefix stays where it is; behind it 640 rows go to chunks, 639 do not, listed and not."""
+    lib, M = _lib.load(), first + moved
+    n, spill, per = M + 150, 200, -(-M // 512)
+    keep = np.concatenate([np.arange(first), first + 1 + np.sort(np.random.default_rng(first + moved).choice(n - first - 1, size=moved, replace=False))])
+    need = lib.trimkv_evict_split_rooms_workspace(4, 4 * per, 128, spill)
+    lists = torch.tensor([3, 0, 2, 1] + [per * i for i in range(5)], dtype=torch.int32, device=DEV)
+    for listed in (False, True):
+        cache, held = _filled(TrimKVCache, 2, 1, 2, n, 128, torch.bfloat16, torch.float32, keep)
+        ws = torch.full((need + 4096,), 9, dtype=torch.uint8, device=DEV)
+        _lib.check(lib.trimkv_evict_split_rooms(cache._host_table([0, 1]).ctypes.data, 1, 2, 2, 128, _lib.BF16, _lib.F32, M, None, 0, 0, n + 1, _lib.SCORE_ALPHA, _lib.ROUND_UPCAST,
+                                                0, n, spill, lists.data_ptr() if listed else None, 4, lists.data_ptr() + 16 if listed else None, 4 * per, per, ws.data_ptr(), need,
+                                                _lib.current_stream(ws.device)), "rooms")
+        assert (ws[need:] == 9).all()
+        assert (int((ws[:need] != 9).sum()) > 4 * 16) == (moved >= cache_utils._SPLIT_FROM)       # more than a head for each pair: lists of rows
+        _check(cache, held, keep, f"{first} {moved} {listed}")
+
+
 @pytest.mark.parametrize("longest,segments,kept,spill,D,split", [
+    (2176, 64, 2048, 128, 128, True), (2176, 64, 2048, 128, 96, True), (2176, 64, 2048, 128, 64, False), (2176, 66, 2048, 128, 128, True), (2176, 67, 2048, 128, 128, False),
+    (4224, 64, 4096, 128, 64, True), (4224, 72, 4096, 511, 128, True), (4224, 73, 4096, 128, 128, False), (4224, 64, 4096, 512, 128, False),
     (8320, 64, 8192, 128, 128, True), (8320, 128, 8192, 128, 128, False), (12288, 32, 8192, 512, 64, True), (12288, 64, 8192, 512, 96, False),
     (4096, 8, 2048, 512, 128, True), (4096, 8, 2047, 512, 128, False), (4096, 8, 2048, 512, 96, True), (4096, 8, 2048, 512, 64, False),
     (2688, 8, 2559, 128, 64, False), (2688, 8, 2560, 128, 64, True), (32769, 8, 32000, 512, 128, False), (8320, 8, 8192, 128, 256, False)])

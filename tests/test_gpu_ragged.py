@@ -451,11 +451,38 @@ def test_decode_attention_dispatch_order_changes_nothing_but_scheduling():
     assert torch.equal(got.view(nseg, G, D)[untouched], base.view(nseg, G, D)[untouched])
 
 
+@pytest.mark.parametrize("nlayers,H", [(140, 8), (1, 1100), (3, 700)])
+def test_wide_selection_carries_ties_from_one_round_of_segments_to_the_next(nlayers, H):
+    """More than 1024 (layer, segment) pairs in a group, which the scan takes 1024 at a time, and one score for all rows: the earlier ones of the pairs in (layer, segment)
+    order are kept, wherever the budget ends."""
+    from trimkv_amd import _lib as L
+    lib, rng, cap, D = L.load(), np.random.default_rng(nlayers), 24, 64
+    lens = rng.integers(0, cap + 1, size=(nlayers, H)).astype(np.int32)
+    lens.reshape(-1)[[0, 1022, 1023, 1024, 1025]] = [0, 3, cap, 1, 2]
+    lb, pos = torch.full((nlayers, H, cap), -0.5, device=DEV), torch.full((nlayers, H, cap), 3, dtype=torch.int64, device=DEV)
+    ln = torch.from_numpy(lens).to(DEV)
+    tables = [torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64, device=DEV) for ts in (lb, pos, ln)]
+    before = np.concatenate([[0], np.cumsum(lens.reshape(-1))])
+    for budget in (int(before[1023]), int(before[1024]) - 1, int(before[1024]), int(before[1024]) + 1, int(before[1026]) - 1, int(before[-1]) - 5):
+        outs = []
+        for wide in (False, True):
+            out = [torch.full(s, -1, dtype=torch.int32, device=DEV) for s in ((1,), (1,), (nlayers, H), (nlayers, H), (nlayers, H))]
+            args = (tables[0].data_ptr(), tables[1].data_ptr(), None, tables[2].data_ptr(), nlayers, H, H, cap, D, L.BF16, L.F32, budget, 0, 0.0, 9, L.SCORE_ALPHA, L.ROUND_NATIVE,
+                    *(t.data_ptr() for t in out))
+            ws = torch.full((lib.trimkv_group_threshold_workspace(nlayers, H, H),), 255, dtype=torch.uint8, device=DEV)
+            st = L.current_stream(torch.device(DEV))
+            L.check(lib.trimkv_group_threshold_wide(*args, ws.data_ptr(), ws.numel(), st) if wide else lib.trimkv_group_threshold(*args, st), "wide" if wide else "single")
+            outs.append([t.cpu() for t in out])
+        for a, b in zip(*outs):
+            assert torch.equal(a, b)
+        assert (outs[1][3].numpy().reshape(-1) == np.clip(budget - before[:-1], 0, lens.reshape(-1))).all()
+
+
 @pytest.mark.parametrize("nlayers,B,H,budget,threshold", [(3, 2, 4, 500, None), (40, 1, 8, 3000, None), (40, 1, 8, 10 ** 9, None),
                                                           (5, 3, 2, 0, None), (6, 2, 4, 0, -0.7), (2, 1, 2, 77, None)])
 def test_wide_group_threshold_equals_the_single_workgroup_selection(nlayers, B, H, budget, threshold):
     """trimkv_group_threshold_wide must return exactly what trimkv_group_threshold returns: cut key, tie quota, per-segment
-    kept counts and tie bases -- with heavy ties (log beta on a coarse grid), ragged and empty segments, more than 256
+    kept counts and tie bases -- with heavy ties (log beta on a coarse grid), ragged and empty segments, hundreds of
     (layer, segment) pairs per group, budgets of zero and beyond the token count, and the threshold mode."""
     from trimkv_amd import _lib as L
     lib = L.load()

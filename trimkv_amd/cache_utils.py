@@ -88,7 +88,7 @@ class LazyLogBeta:
 
 
 SPLIT_SCRATCH = 256 << 20   # most bytes that a split eviction takes for the length of its launches
-_SPLIT_ROWS = 512           # kept rows per chunk (SPLIT_ROWS of csrc/evict.hip)
+_SPLIT_ROWS, _SPLIT_FROM = 512, 640     # kept rows per chunk; fewest rows to move that go to chunks (both as in csrc/evict.hip)
 
 
 def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -> bool:
@@ -97,8 +97,8 @@ def split_evict(longest: int, rows: int, kept: int, spill: int, head_dim: int) -
     workgroup per segment takes about 15 us + 12 to 22 ns a row of the longest one; three launches and the detour of the rows that cross a
     chunk's end take about 17 us + 0.23 ns a row (all losing many: 20 us and as much); both less with fewer features.  Measured, whole ->
     split, us, segments x rows, of 128 / 96 / 64 features.  Split: losing 128 rows 8 x 2176 35 -> 24 / 35 -> 23, 32 x 3200 72 -> 40 / 60 -> 35 / 39 -> 29, 64 x
-    4224 110 -> 80 / 92 -> 66 / 62 -> 50, 64 x 8320 208 -> 141 / 173 -> 112 / 115 -> 83; losing 4096 32 x 12288 186 -> 112 / 163 -> 98 / 106 -> 73, 2048 32 x
-    4096 53 -> 45 / 47 -> 38.  Whole, where the line is on the safe side: 64 x 2176 59 -> 44 / 49 -> 38 / 33 -> 30, 128 x 4224 133 -> 136 / 110 -> 108 / 73 -> 81;
+    2176 59 -> 44 / 49 -> 38, 64 x 4224 110 -> 80 / 92 -> 66 / 62 -> 50, 64 x 8320 208 -> 141 / 173 -> 112 / 115 -> 83; losing 4096 32 x 12288 186 -> 112 / 163 -> 98 / 106 -> 73, 2048 32 x
+    4096 53 -> 45 / 47 -> 38.  Whole, where the line is on the safe side: 64 x 2176 of 64 features 33 -> 30, 128 x 4224 133 -> 136 / 110 -> 108 / 73 -> 81;
     and where split is slower: 128 x 2176 69 -> 77 / 60 -> 63 / 38 -> 46, 256 x 4224 224 -> 253 / 179 -> 196 / 118 -> 141, losing half 64 x 4096 62 -> 63 /
     53 -> 58 / 35 -> 43, 128 x 6144 102 -> 148 / 93 -> 122 / 60 -> 86.  Of few kept rows one workgroup is done as soon: 8 x 1152 cut to 1024 24 -> 22 / 23 -> 22 / 18 -> 21,
     16 x 4100 to 1100 32 -> 31 / 30 -> 30 / 23 -> 27; of 64 features 8 x 2176 cut to 2048 24 -> 22, 8 x 4096 27 -> 25.
@@ -511,7 +511,7 @@ class _SlabBacked(_CacheBase):
             pairs, rows, kept = due
             if not split_evict(int(rows.max()), int(rows.sum()), int(kept.max()), spill, s0.D):
                 return None
-            chunks = np.where(kept >= 640, -(-kept // _SPLIT_ROWS), 0)      # with fewer rows than that the kernel does not split
+            chunks = np.where(kept >= _SPLIT_FROM, -(-kept // _SPLIT_ROWS), 0)      # with fewer rows than that the kernel does not split
             first = np.concatenate([[0], np.cumsum(chunks)])
             most, total, count = int(chunks.max()), int(first[-1]), int(pairs.size)
             if total == 0:
