@@ -19,11 +19,13 @@ from torch.utils._device import DeviceContext
 from . import _lib
 
 MAX_ROWS = 64      # rows that trimkv_linear_rows takes
-# More rows than WIDE_ROWS times more outputs than WIDE, heads of language models above all, are left to the general product: workgroups there take 96 rows of w
-# and have one step in flight.  us here | general, 48 rows and 64: 16384 x 3072 26.8 | 23.1, 27.9 | 23.4; 32064 x 3072 51.0 | 47.2, 53.8 | 38.6; 128256 x 4096
-# 230 | 214, 243 | 216; 151936 x 4096 265 | 261, 278 | 270; given up: 24576 x 4096 41.6 | 44.7, 41.9 | 45.5, 49152 x 2048 47.9 | 51.9, 50.4 | 54.5.  Up to
-# 32 rows all are taken: 32064 x 3072 with 1, 16, 32 rows 31.5 | 41.0, 33.2 | 42.0, 39.4 | 37.1; 151936 x 2048 101 | 207, 109 | 208, 128 | 153; 151936 x
-# 5120 238 | 307, 263 | 330, 319 | 364.  12288 x 4096 with 48 and 64: 22.8 | 24.5, 24.3 | 25.1.
+# More rows than WIDE_ROWS times more outputs than WIDE, heads of language models above all, are left to the general product.  us here | general, 33 rows, 48 and 64.  For it:
+# 151936 x 5120 303 | 291, 324 | 295, 337 | 298; 128256 x 4096 205 | 206, 218 | 207, 221 | 209; 13824 x 5120 31.8 | 29.4, 33.4 | 30.6, 35.4 | 31.7; 100352 x 5120 209 | 280,
+# 219 | 184, 233 | 215.  Alike or mixed: 34816 x 5120 78 | 80, 82 | 81, 86 | 86; 32064 x 3072 41.6 | 39.5, 42.4 | 52.3, 42.2 | 38.7; 151936 x 4096 241 | 254, 254 | 268, 260 | 259;
+# 16384 x 3072 22.7 | 23.3, 22.8 | 23.6, 23.2 | 23.8.  Given up, since tiles take any number of 8 rows of w: 16384 x 4096 27 | 31 all three, 24576 x 4096 39 | 46, 28672 x 4096 47 | 51,
+# 47 | 60, 49 | 52, 49152 x 2048 40 | 49, 41 | 48, 43 | 49, 151936 x 2048 130 | 153, 135 | 143, 141 | 152; a line in k as well as n would keep these.  Below it: 12288 x 4096 20 | 25,
+# 21 | 25, 22 | 26, 8192 x 8192 27 | 31, 29 | 32, 31.5 | 31.7 (one row 22.6 | 28.6).  Up to 32 rows all are taken, in blocks of 16 rows of w then: 32064 x 3072 with 1, 16, 32 rows
+# 31.5 | 41.0, 33.2 | 42.0, 39.4 | 37.1; 151936 x 2048 101 | 207, 109 | 208, 128 | 153; 151936 x 5120 238 | 307, 263 | 330, 319 | 364.
 WIDE_ROWS, WIDE = 32, 12288
 
 
