@@ -152,6 +152,16 @@ def test_linear_takes_it_where_it_is_faster():
         _lib._hybrid["hybrid"] = lib
 
 
+def test_other_devices_need_no_library(monkeypatch):
+    def missing(*_):
+        raise _lib.TrimKVLibraryError("missing")
+    monkeypatch.setattr(_lib, "load_hybrid", missing)
+    linear._f32_form.cache_clear()
+    x, w = torch.randn(300, 64), torch.randn(96, 64)
+    assert torch.equal(linear.linear(x, w, library="hybrid"), F.linear(x, w))
+    assert linear.linear(x.to("meta"), w.to("meta"), library="hybrid").shape == (300, 96)
+
+
 def test_bad_calls_are_refused():
     lib = ctypes.CDLL(_lib.HYBRID_LIB_PATHS["hybrid"])
     fn = lib.trimkv_linear_f32_tiles

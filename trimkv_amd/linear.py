@@ -116,7 +116,7 @@ def _f32_form(rows: int, n: int, k: int, library: str) -> int:
 def _f32_rows(x: torch.Tensor, weight: torch.Tensor, library: str):
     """``(x as [rows, k], form)`` the way trimkv_linear_f32_tiles takes this product, or None where it does not or is not faster."""
     k = x.shape[-1] if x.dim() else 0
-    if torch.compiler.is_compiling() or k == 0 or weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0:
+    if not x.is_cuda or torch.compiler.is_compiling() or k == 0 or weight.dim() != 2 or weight.shape[1] != k or weight.shape[0] == 0:
         return None
     rows, n = x.numel() // k, weight.shape[0]
     if type(rows) is not int or type(n) is not int or not 0 < rows <= 1 << 22 or n > 1 << 22:
