@@ -6,7 +6,7 @@
  * Conventions as in trimkv_hip.h: device pointers throughout, work enqueued on `stream`, no allocation and no host
  * synchronisation, 0 / negative trimkv_status / positive hipError_t, text of the last error of the calling thread from
  * trimkv_hybrid_last_error() (trimkv_mlstm_last_error(), trimkv_moe_last_error() of the other two).  `dtype` is the type of activations and matrices: TRIMKV_BF16 or TRIMKV_F32 (everything in
- * fp32; where bf16 terms stand for fp32 numbers they hold them whole).  Norm weights, biases, gates, router logits, recurrent state and the residual stream are fp32 always.
+ * fp32).  Norm weights, biases, gates, router logits, recurrent state and the residual stream are fp32 always.
  *
  * Batches are packed: the tokens of all sequences of a step lie one after the other, sequence b owns tokens
  * cu[b] .. cu[b+1]-1 (cu [batch+1] int32).  What a sequence leaves behind lives in a slot, slots[b] (int32); seen [slots][2]

@@ -133,7 +133,7 @@ def _selected_both_ways(lens, cap, budget, lb_dtype, strategy):
 @pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
 @pytest.mark.parametrize("budget", [0, 1, 700, 10 ** 6])
 def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(budget, lb_dtype, strategy):
-    """Ties by the hundred, empty segments, lengths around the rows of wavefronts (64) and of the 1024 threads that read at a time."""
+    """Ties by the hundred, empty segments, lengths around the rows of wavefronts (64) and of the 256 or 1024 threads that read at a time."""
     lens = torch.tensor([[0, 1, 255, 256, 257, 1023, 1024, 1025], [1300, 1300, 64, 65, 0, 0, 0, 0], [5, 900, 1281, 1279, 3, 1, 2, 700]], dtype=torch.int32)
     _selected_both_ways(lens, 1300, budget, lb_dtype, strategy)
 
@@ -141,9 +141,18 @@ def test_budgets_of_a_layer_selected_by_one_workgroup_and_by_one_per_segment(bud
 @pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "alpha"), (torch.float32, "knorm")])
 @pytest.mark.parametrize("budget", [4096, 12000])
 def test_segments_of_more_rows_than_a_workgroup_has_in_flight(budget, lb_dtype, strategy):
-    """4096 rows are four for each thread: one less, as many, one more, twice as many and some."""
+    """4096 rows are four for each of 1024 threads: one less, as many, one more, twice as many and some."""
     lens = torch.tensor([[4095, 4096, 4097, 8191, 8192, 8193, 8200, 0], [5119, 5120, 5121, 3, 8200, 8200, 4097, 4096]], dtype=torch.int32)
     _selected_both_ways(lens, 8200, budget, lb_dtype, strategy)
+
+
+@pytest.mark.parametrize("lb_dtype,strategy", [(torch.float32, "alpha"), (torch.bfloat16, "knorm")])
+@pytest.mark.parametrize("layers,cap", [(32, 1024), (32, 1025), (33, 1025), (3, 1024)])
+def test_either_side_of_where_workgroups_are_large(layers, cap, lb_dtype, strategy):
+    """256 segments and 264; room for 1024 rows and for one more."""
+    lens = torch.from_numpy(np.random.default_rng(layers + cap).integers(0, cap + 1, size=(layers, 8)).astype(np.int32))
+    lens[0, :4] = torch.tensor([cap, 1023, 1024, 0])
+    _selected_both_ways(lens, cap, 900, lb_dtype, strategy)
 
 
 def _uneven(split, monkeypatch):

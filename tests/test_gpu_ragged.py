@@ -453,17 +453,17 @@ def test_decode_attention_dispatch_order_changes_nothing_but_scheduling():
 
 @pytest.mark.parametrize("nlayers,H", [(140, 8), (1, 1100), (3, 700)])
 def test_wide_selection_carries_ties_from_one_round_of_segments_to_the_next(nlayers, H):
-    """More than 1024 (layer, segment) pairs in a group, which the scan takes 1024 at a time, and one score for all rows: the earlier ones of the pairs in (layer, segment)
+    """More than 1024 (layer, segment) pairs in a group, which the scan takes 256 at a time, and one score for all rows: the earlier ones of the pairs in (layer, segment)
     order are kept, wherever the budget ends."""
     from trimkv_amd import _lib as L
     lib, rng, cap, D = L.load(), np.random.default_rng(nlayers), 24, 64
     lens = rng.integers(0, cap + 1, size=(nlayers, H)).astype(np.int32)
-    lens.reshape(-1)[[0, 1022, 1023, 1024, 1025]] = [0, 3, cap, 1, 2]
+    lens.reshape(-1)[[0, 255, 256, 1022, 1023, 1024, 1025]] = [0, 4, 5, 3, cap, 1, 2]
     lb, pos = torch.full((nlayers, H, cap), -0.5, device=DEV), torch.full((nlayers, H, cap), 3, dtype=torch.int64, device=DEV)
     ln = torch.from_numpy(lens).to(DEV)
     tables = [torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64, device=DEV) for ts in (lb, pos, ln)]
     before = np.concatenate([[0], np.cumsum(lens.reshape(-1))])
-    for budget in (int(before[1023]), int(before[1024]) - 1, int(before[1024]), int(before[1024]) + 1, int(before[1026]) - 1, int(before[-1]) - 5):
+    for budget in (int(before[256]), int(before[256]) + 2, int(before[1023]), int(before[1024]) - 1, int(before[1024]), int(before[1024]) + 1, int(before[1026]) - 1, int(before[-1]) - 5):
         outs = []
         for wide in (False, True):
             out = [torch.full(s, -1, dtype=torch.int32, device=DEV) for s in ((1,), (1,), (nlayers, H), (nlayers, H), (nlayers, H))]

@@ -782,9 +782,11 @@ __global__ __launch_bounds__(GT_THREADS) void group_threshold_kernel(GroupArgs a
 // scan of 256 bins) before it bins its own segment.  A count launch then classifies every segment's tokens against
 // the cut, and a scan launch (one workgroup per group) turns the per-segment counts into new_len / tie_base in
 // (layer, segment) order.  Kernel boundaries are the only synchronisation.  per_layer: a group per layer, its cut at layer * groups + group.
-// Four rows a thread in flight: with 256 threads a segment of 2900 rows took three round trips to memory for one (192 segments: a digit 10.7 -> 6.5 us, the count
-// 12.9 -> 9.1).
-constexpr int GW_THREADS = 1024;
+// Threads of a histogram's or count's workgroup, each with four rows in flight: 1024 while every segment has a compute unit of its own (192 segments of 2400 rows, the selection whole,
+// 256 -> 1024 threads: 41.0 -> 35.5 us, of 8200 75.5 -> 47.6), 256 of more (288 of 2400: 62.0 | 70.8, 1152: 85.0 | 133, 2304: 128 | 218) and of segments whose rows 256
+// threads have in flight at once (192 of 300: 31.0 | 31.4).  With norms of keys, a wavefront to four rows, 1024 whatever their length (64 of 300 114 -> 74, 192 of 2400 595 -> 207; 288
+// of 300 139 | 151, 1152 197 | 378).
+constexpr int GW_FEW = 256, GW_ROWS = 1024, GW_SCAN = 256;
 struct WideArgs {
     GroupArgs g;
     uint32_t* hist;   // [ngroups][4][256]
@@ -793,11 +795,12 @@ struct WideArgs {
 
 // Prefix (digits of passes 0..npass-1) and remaining rank for group g; *total = tokens in the group.  All threads call: thread t
 // looks at bin 255 - t, a scan walks the bins from the largest down (one thread alone took 8 us a pass for it).
+template <int THREADS>
 __device__ __forceinline__ void wide_prefix(const WideArgs& w, int g, int npass, unsigned long long* sh, uint32_t& prefix,
                                             uint64_t& remaining, uint64_t& total) {
-    static_assert(GW_THREADS >= 256, "a thread per bin");
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const bool bin = t < 256;
+    static_assert(THREADS >= 256, "a thread per bin");
+    const bool bin = THREADS == 256 || t < 256;
     uint32_t h[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) h[q] = q < npass && bin ? w.hist[((int64_t)g * 4 + q) * 256 + 255 - t] : 0u;
@@ -834,7 +837,8 @@ __device__ __forceinline__ void wide_prefix(const WideArgs& w, int g, int npass,
     __syncthreads();
 }
 
-__global__ __launch_bounds__(GW_THREADS) void group_hist_kernel(WideArgs w, int pass) {
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void group_hist_kernel(WideArgs w, int pass) {
     __shared__ uint32_t lh[256];
     __shared__ unsigned long long sh[6];
     const GroupArgs& a = w.g;
@@ -842,21 +846,22 @@ __global__ __launch_bounds__(GW_THREADS) void group_hist_kernel(WideArgs w, int 
     const int seg = g * a.segs_per_group + s, cut = a.per_layer ? l * (int)gridDim.z + g : g;
     uint32_t prefix;
     uint64_t remaining, total;
-    wide_prefix(w, cut, pass, sh, prefix, remaining, total);
+    wide_prefix<THREADS>(w, cut, pass, sh, prefix, remaining, total);
     const int shift = 24 - 8 * pass;
     const uint32_t hi_mask = pass == 0 ? 0u : (0xffffffffu << (shift + 8));
-    if (threadIdx.x < 256) lh[threadIdx.x] = 0;
+    if (THREADS == 256 || threadIdx.x < 256) lh[threadIdx.x] = 0;
     __syncthreads();
     const int n = max(0, min(a.seg_lens[l][seg], a.cap));
     const ScoreArgs sa = group_segment(a, l, seg);
-    for_each_key<GW_THREADS, 4>(sa, n, [&](int, uint32_t key) {
+    for_each_key<THREADS, 4>(sa, n, [&](int, uint32_t key) {
         if ((key & hi_mask) == prefix) atomicAdd(&lh[(key >> shift) & 255u], 1u);
     });
     __syncthreads();
-    if (threadIdx.x < 256 && lh[threadIdx.x]) atomicAdd(&w.hist[((int64_t)cut * 4 + pass) * 256 + threadIdx.x], lh[threadIdx.x]);
+    if ((THREADS == 256 || threadIdx.x < 256) && lh[threadIdx.x]) atomicAdd(&w.hist[((int64_t)cut * 4 + pass) * 256 + threadIdx.x], lh[threadIdx.x]);
 }
 
 // cut of group g: from the threshold, or from the four histograms (with the keep-all / keep-nothing cases)
+template <int THREADS>
 __device__ __forceinline__ void wide_cut(const WideArgs& w, int g, unsigned long long* sh, uint32_t& thr, int64_t& take) {
     const GroupArgs& a = w.g;
     if (a.use_threshold) {
@@ -866,27 +871,28 @@ __device__ __forceinline__ void wide_cut(const WideArgs& w, int g, unsigned long
     }
     uint32_t prefix;
     uint64_t remaining, total;
-    wide_prefix(w, g, 4, sh, prefix, remaining, total);
+    wide_prefix<THREADS>(w, g, 4, sh, prefix, remaining, total);
     const uint64_t budget = (uint64_t)max((int64_t)0, a.budget);
     if (budget >= total) { thr = 0u; take = INT32_MAX; }
     else if (budget == 0) { thr = 0xffffffffu; take = 0; }
     else { thr = prefix; take = (int64_t)remaining; }
 }
 
-__global__ __launch_bounds__(GW_THREADS) void group_count_kernel(WideArgs w) {
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void group_count_kernel(WideArgs w) {
     __shared__ unsigned long long sh[6];
-    __shared__ uint64_t red[GW_THREADS / 64];
+    __shared__ uint64_t red[THREADS / 64];
     const GroupArgs& a = w.g;
     const int s = blockIdx.x, l = blockIdx.y, g = blockIdx.z;
     const int seg = g * a.segs_per_group + s, cut = a.per_layer ? l * (int)gridDim.z + g : g;
     uint32_t thr;
     int64_t take;
-    wide_cut(w, cut, sh, thr, take);
+    wide_cut<THREADS>(w, cut, sh, thr, take);
     const int n = max(0, min(a.seg_lens[l][seg], a.cap));
     const ScoreArgs sa = group_segment(a, l, seg);
     uint64_t cnt = 0;  // low 32 bits: greater, high 32 bits: equal
     uint32_t row0 = 0;  // thread 0 owns row 0
-    for_each_key<GW_THREADS, 4>(sa, n, [&](int i, uint32_t key) {
+    for_each_key<THREADS, 4>(sa, n, [&](int i, uint32_t key) {
         cnt += (key > thr ? 1ull : 0ull) + (key == thr ? (1ull << 32) : 0ull);
         if (i == 0) row0 = (key > thr ? 1u : 0u) | (key == thr ? 2u : 0u);
     });
@@ -895,7 +901,7 @@ __global__ __launch_bounds__(GW_THREADS) void group_count_kernel(WideArgs w) {
     __syncthreads();
     if (threadIdx.x == 0) {
         uint64_t t = 0;
-        for (int i = 0; i < GW_THREADS / 64; ++i) t += red[i];
+        for (int i = 0; i < THREADS / 64; ++i) t += red[i];
         const int64_t e = ((int64_t)l * a.nseg + seg) * 3;
         w.cnt[e] = (uint32_t)(t & 0xffffffffull);
         w.cnt[e + 1] = (uint32_t)(t >> 32);
@@ -907,9 +913,9 @@ __global__ __launch_bounds__(GW_THREADS) void group_count_kernel(WideArgs w) {
     }
 }
 
-__global__ __launch_bounds__(GW_THREADS) void group_scan_kernel(WideArgs w) {
-    __shared__ uint32_t gt_l[GW_THREADS], eq_l[GW_THREADS];
-    __shared__ int32_t len_l[GW_THREADS], base_l[GW_THREADS];
+__global__ __launch_bounds__(GW_SCAN) void group_scan_kernel(WideArgs w) {
+    __shared__ uint32_t gt_l[GW_SCAN], eq_l[GW_SCAN];
+    __shared__ int32_t len_l[GW_SCAN], base_l[GW_SCAN];
     uint32_t row0 = 0;
     __shared__ long long carry;
     const GroupArgs& a = w.g;
@@ -917,7 +923,7 @@ __global__ __launch_bounds__(GW_THREADS) void group_scan_kernel(WideArgs w) {
     const int64_t take = a.tie_take[l0 * (int)gridDim.x + g];   // written by the count launch
     const int entries = (a.per_layer ? 1 : a.nlayers) * a.segs_per_group;   // (layer, segment) pairs of the group, in tie order
     if (threadIdx.x == 0) carry = 0;
-    for (int e0 = 0; e0 < entries; e0 += GW_THREADS) {
+    for (int e0 = 0; e0 < entries; e0 += GW_SCAN) {
         __syncthreads();
         const int e = e0 + threadIdx.x;
         int64_t idx = 0;
@@ -931,7 +937,7 @@ __global__ __launch_bounds__(GW_THREADS) void group_scan_kernel(WideArgs w) {
         __syncthreads();
         if (threadIdx.x == 0) {
             long long eq_seen = carry;
-            const int m = min(GW_THREADS, entries - e0);
+            const int m = min(GW_SCAN, entries - e0);
             for (int i = 0; i < m; ++i) {
                 const long long eq = eq_l[i];
                 const long long eq_kept = max(0ll, min(eq, (long long)take - eq_seen));
@@ -1376,10 +1382,16 @@ static int group_threshold_wide_common(const char* fn, int per_layer, const void
     if (!use_threshold) {
         const int64_t nh = (int64_t)cuts * 4 * 256;
         hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, w.hist, nh, 0u);
-        for (int pass = 0; pass < 4; ++pass) hipLaunchKernelGGL(group_hist_kernel, grid, dim3(GW_THREADS), 0, st, w, pass);
     }
-    hipLaunchKernelGGL(group_count_kernel, grid, dim3(GW_THREADS), 0, st, w);
-    hipLaunchKernelGGL(group_scan_kernel, dim3(ngroups, per_layer ? nlayers : 1), dim3(GW_THREADS), 0, st, w);
+    auto look = [&](auto threads) {
+        constexpr int T = decltype(threads)::value;
+        if (!use_threshold)
+            for (int pass = 0; pass < 4; ++pass) hipLaunchKernelGGL(group_hist_kernel<T>, grid, dim3(T), 0, st, w, pass);
+        hipLaunchKernelGGL(group_count_kernel<T>, grid, dim3(T), 0, st, w);
+    };
+    if ((int64_t)nlayers * nseg <= GW_FEW && (cap > GW_ROWS || a.k_slabs)) look(std::integral_constant<int, 1024>{});
+    else look(std::integral_constant<int, 256>{});
+    hipLaunchKernelGGL(group_scan_kernel, dim3(ngroups, per_layer ? nlayers : 1), dim3(GW_SCAN), 0, st, w);
     return launch_status(fn);
 }
 

@@ -89,7 +89,7 @@ __device__ __forceinline__ void lr_load_to_lds(const uint16_t* base, uint32_t of
 // adds the residual where it rounds and leaves sums of squares, a few KB that the product behind them (NORM) adds up while its first
 // operands are on their way; x becomes round(round(x / rms) * weight), as modules round, on its way from LDS to the matrix cores.
 // A layer's four products with adds and norms, 16 rows: 43.6 -> 40.2 us at 2048 features and 6144, 92.0 -> 83.5 at 4096 and 12288; 1 row
-// 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102 (all in blocks of 16).  With more rows the arithmetic on the way no longer hides.
+// 38.9 -> 35.9 and 84.7 -> 79.7; 32 rows 49.8 -> 48.0 and 107 -> 102 (both sides while tiles were blocks of 16).  With more rows the arithmetic on the way no longer hides.
 enum { LR_PLAIN = 0, LR_ADD = 1, LR_NORM = 2 };
 template <bool F16, bool SILU, int MODE, int XG, int NG, int W, int D>
 __global__ __launch_bounds__(64 * W) void linear_rows_kernel(LinearRowsArgs a) {
