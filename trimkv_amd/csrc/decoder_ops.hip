@@ -176,8 +176,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(RopeArgs a) {
 // of fewer than 128 features leave lanes idle).  Needs 16-byte aligned rows, head_dim % 8 == 0 and rotary_dim % 16 == 0, so
 // that a lane's eight features lie on one side of the rotation's halfway point and its partner features in ONE other lane.
 // At 8 x 4096 tokens of the Qwen3-8B shape: 351 us (2.3 TB/s) against 945 us with the 2-byte accesses of the kernel above.
-// A decode step's few rows are latency alone: the norm's weight, cosines and sines are requested with the row, and quotients are taken in 32 bits while
-// they fit (16 tokens of 16 + 8 + 8 heads with a gate in a graph of launches 3.9 -> 2.7 us, the rounding in one instruction and the sums without LDS included).
+// A decode step's few rows are latency alone: quotients are taken in 32 bits while they fit (16 tokens of 16 + 8 + 8 heads with a gate in a graph of launches 3.9 -> 2.7 us, the
+// rounding in one instruction and the sums without LDS included).  The norm's weight, cosines and sines are requested where they are used: together with the row no step
+// was faster (64 launches' sizes up to 100 tokens, alike within noise) and prompts slower, 8 x 4096 tokens of 32 + 8 + 8 heads with norms 218 -> 224 us, in fp16 198 -> 217.
 template <bool F16, typename I>        // I: holds the rows
 __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64_t total_rows, int64_t row_waves) {
     const int lane = threadIdx.x & 63;
@@ -206,15 +207,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64
     const int64_t b = (int64_t)((I)t / (I)a.seq), s = t - b * a.seq;
     uint16_t* dst = (kind == 0 ? a.q_out : kind == 1 ? a.k_out : a.v_out) + ((b * nh + head) * a.seq + s) * a.d;
     const int e0 = lr * 8;
-    const bool turned = live && e0 < rd;
-    Vec8 xv, wv, cv, sv;
-    xv.v = wv.v = cv.v = sv.v = make_uint4(0, 0, 0, 0);
+    Vec8 xv; xv.v = make_uint4(0, 0, 0, 0);
     if (live) xv.v = *(const uint4*)(src + e0);
-    if (live && w) wv.v = *(const uint4*)(w + e0);
-    if (turned) {
-        cv.v = *(const uint4*)(a.cos + b * a.cs_batch_stride + s * a.rd + e0);
-        sv.v = *(const uint4*)(a.sin + b * a.cs_batch_stride + s * a.rd + e0);
-    }
     float y[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) y[j] = dop_load<F16>(xv.h[j]);
@@ -224,6 +218,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64
         for (int j = 0; j < 8; ++j) ss += y[j] * y[j];
         ss = dop_sum16(ss);
         const float inv = rsqrtf(ss / (float)a.d + a.eps);
+        Vec8 wv; wv.v = make_uint4(0, 0, 0, 0);
+        if (live) wv.v = *(const uint4*)(w + e0);
 #pragma unroll
         for (int j = 0; j < 8; ++j) y[j] = dop_round<F16>(dop_load<F16>(wv.h[j]) * dop_round<F16>(y[j] * inv));
     }
@@ -235,7 +231,10 @@ __global__ __launch_bounds__(256) void qk_norm_rope_vec_kernel(RopeArgs a, int64
 #pragma unroll
     for (int j = 0; j < 8; ++j) r[j] = __shfl(y[j], partner, 64);
     Vec8 ov;
-    if (turned) {
+    if (live && e0 < rd) {
+        Vec8 cv, sv;
+        cv.v = *(const uint4*)(a.cos + b * a.cs_batch_stride + s * a.rd + e0);
+        sv.v = *(const uint4*)(a.sin + b * a.cs_batch_stride + s * a.rd + e0);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             ov.h[j] = dop_bits<F16>(dop_round<F16>(y[j] * dop_load<F16>(cv.h[j])) + dop_round<F16>((low ? -r[j] : r[j]) * dop_load<F16>(sv.h[j])));
