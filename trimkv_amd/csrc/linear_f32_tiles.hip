@@ -18,7 +18,7 @@
 // What bf16 terms do not hold is done by fp32 matrix instructions.  Infinities, NaN and numbers that round to infinity end as results that are not finite: blocks with such
 // results are done again.  Numbers below 2^-103 lose up to 2^-125 each.  That is nothing beside a result of 2^-97 k times the largest number and more; a tile with a smaller
 // result looks through its rows, and blocks with a row that has such a number are done again (rows 2^-118 times a normal distribution, against a matrix 2^100 times, without it:
-// error 8.8e-6, 2^-126 2.3e-3, 2^-134 0.6; now 4.1e-7).  Following the largest costs 3 - 5 % of a launch, a row of zeros in each tile 40 %: 811 x 6144 x 2048 117 -> 122 us, 160 with
+// error 8.8e-6, 2^-126 2.3e-3, 2^-134 0.6; now 4.1e-7).  Following the largest costs 3 - 5 % of a launch, 7 % in the smallest tiles, a row of zeros in each tile 40 %: 811 x 6144 x 2048 117 -> 122 us, 160 with
 // such rows (the vendor library's 205), 900 if all of x is below 2^-103.  With the smallest number followed instead, single zeros sent tiles to look.
 //
 // Measured (rows x n x k, us here | the vendor library's product): 811 x 6144 x 2048 122 | 205, 811 x 2048 x 2048 45 | 58, 811 x 1024 x 2048 27 | 35, 300 x 6144 x
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256, (MU + NU) * D <= 10 ? 2 : 1) void linear_f32_t
 struct F32Form { int mu, nu, d; bool pairs; float begin, period; };      // pairs: two workgroups to a compute unit
 
 // A form takes begin + period * periods of 128 k (us) for a round of a tile per compute unit; with two workgroups to each, the beginnings of later
-// rounds pass unseen.  Measured with 128 .. 1024 tiles of k = 512, 2048 and 4096, without the largest number followed: as it is 3 - 5 % more, of all forms alike.
+// rounds pass unseen.  Measured with 128 .. 1024 tiles of k = 512, 2048 and 4096, without the largest number followed: as it is 3 - 5 % more, of the first two 7 %.
 constexpr F32Form F32_FORMS[] = {{1, 4, 2, true, 4.2f, 0.69f}, {2, 3, 2, true, 3.6f, 0.80f}, {2, 6, 1, true, 3.8f, 1.34f}, {3, 4, 1, true, 3.9f, 1.20f}, {4, 4, 1, true, 4.8f, 1.43f},
                                  {3, 6, 1, true, 4.6f, 1.68f}, {4, 5, 1, true, 5.2f, 1.72f}, {4, 6, 1, true, 5.2f, 2.05f}, {5, 6, 1, false, 6.8f, 2.34f}, {3, 9, 1, false, 7.0f, 2.37f},
                                  {4, 8, 1, false, 7.4f, 2.50f}, {4, 10, 1, false, 8.0f, 3.10f}, {6, 8, 1, false, 9.0f, 3.50f}};
